@@ -1,75 +1,128 @@
-// Token-by-token gated delta rule with the state tile resident in registers.
-//
-// One workgroup of 256 threads owns the K x BV tile of one (sequence, head) state: columns
-// of the state evolve independently, so V is split over workgroups without any exchange.
-// Each thread holds RPT consecutive rows x 4 consecutive columns (fp32) of the tile; a wave's
-// loads are whole 16 B-per-lane rows of the tile.  Per token:
+// Token-by-token gated delta rule with the state in registers.  Per token and (sequence, head):
 //
 //     r  = beta (v - e^g S^T k)        S' = e^g S + k r^T        o = e^g S^T q + (k . q) r
 //
-// i.e. one read and one write of the state for T == 1 (the decode step); both are streaming
-// (non-temporal) accesses, since a state far larger than the caches is touched exactly once per step.  The two
-// K-reductions (S^T k, S^T q) are done in registers, then across the row groups of a wave
-// with shuffles and across the four waves through LDS.
+// The columns of a state evolve independently, so V is split over workgroups without any exchange.  Two kernels:
+// recurrent_step_kernel for a single token (the decode step), bound by the state's way from HBM and back, and
+// recurrent_tokens_kernel for more, bound by the chain from one token's state to the next.  They add up in the same order
+// (gdn_recurrent_common.h): decoding a token gives the bits that running over it in a longer call gives.
 //
 // Replaces fla.ops.gated_delta_rule.fused_recurrent_gated_delta_rule as called at
 // lm_engine/modeling_utils/sequence_mixer_blocks/gated_deltanet/module.py:210-222.
 
-#include "gdn_common.h"
-#include "gdn_launch.h"
+#include <type_traits>
+
+#include "gdn_recurrent_common.h"
 
 namespace gdn {
 
 constexpr int REC_THREADS = 256;
 constexpr int REC_WAVES = REC_THREADS / WAVE;
 
-struct RecurrentParams {
-    const void* q;
-    const void* k;
-    const void* v;
-    const void* beta;
-    const float* g;
-    const float* h0;
-    float* ht;
-    void* o;
-    const int32_t* cu_seqlens;
-    const int32_t* pad_lens;  // left-padded batch: prefix sums of the valid lengths
-    int64_t q_stride_b, q_stride_t, q_stride_h;
-    int64_t k_stride_b, k_stride_t, k_stride_h;
-    int64_t v_stride_b, v_stride_t, v_stride_h;
-    int64_t o_stride_b, o_stride_t, o_stride_h;
-    int T, H, V;
-    int qk_div;  // value heads per head of q and k
-    int beta_dtype;
-    int l2norm;
-    float scale;
-};
-
+// The decode step, and calls of a few tokens over many states: one read and one write of the state, everything else hidden
+// behind them.  A workgroup streams a K x BV tile through its registers.  A token's own operands are asked for ahead of the
+// state (loads return in order), so that their norms are formed while the state is on its way; every wave forms them for
+// itself.  Measured at 256 sequences x 32 heads, K = V = 128 (1.07 GB to and from HBM): 164 us = 6.6 TB/s, 186 us when the
+// norms waited behind the state in one wave and 256 threads held 16 rows each.
 template <typename T, int K, int BV>
-__global__ __launch_bounds__(REC_THREADS) void recurrent_kernel(const RecurrentParams p) {
-    constexpr int LANES_V = BV / 4;            // lanes along the value dim (4 columns each)
-    constexpr int ROWG = REC_THREADS / LANES_V;  // row groups in the workgroup
-    constexpr int RPT = K / ROWG;              // state rows per thread
-    constexpr int KPL = K / WAVE;  // q/k elements per lane when one wave loads a whole row
-    static_assert(K % ROWG == 0 && RPT >= 1, "tile does not divide over the workgroup");
-    static_assert(K % WAVE == 0, "K must be a multiple of the wave size");
+__global__ __launch_bounds__(4 * BV) void recurrent_step_kernel(const RecurrentParams p) {
+    typedef StepTile<K, BV> Tile;
+    constexpr int RPT = Tile::RPT, KPL = K / WAVE;
+    __shared__ __attribute__((aligned(16))) float s_red[Tile::WAVES][2][BV];
+    __shared__ __attribute__((aligned(16))) float s_kq[2][K];
+    const Tile tile(s_red);
+    const int v0 = blockIdx.x * BV;
+    const int h = blockIdx.y, n = blockIdx.z;
 
-    // k^ is read again after the second barrier of a token (the rank-1 update) while wave 0 may already be
-    // staging the next token: two buffers, alternating by token.  q^ and k^ . q^ are only read between the
-    // two barriers, where wave 0 cannot have moved on.
-    __shared__ __attribute__((aligned(16))) float s_k2[2][K];
-    __shared__ __attribute__((aligned(16))) float s_q[K];
-    __shared__ float s_kq[1];
-    __shared__ __attribute__((aligned(16))) float s_red[REC_WAVES][LANES_V][8];
+    int64_t b = n, t_begin = 0, t_end = p.T;
+    if (p.pad_lens != nullptr) t_begin = p.T - min(max(p.pad_lens[n + 1] - p.pad_lens[n], 0), p.T);  // the last tokens of row n
+    if (p.cu_seqlens != nullptr) {
+        int t0, len;
+        packed_bounds(p.cu_seqlens, n, p.T, t0, len);
+        b = 0, t_begin = t0, t_end = t0 + len;
+    }
+    const int64_t hqk = p.qk_div > 1 ? h / p.qk_div : h;
+    const T* qp = reinterpret_cast<const T*>(p.q) + b * p.q_stride_b + hqk * p.q_stride_h;
+    const T* kp = reinterpret_cast<const T*>(p.k) + b * p.k_stride_b + hqk * p.k_stride_h;
+    const T* vp = reinterpret_cast<const T*>(p.v) + b * p.v_stride_b + h * p.v_stride_h + v0 + 4 * tile.lv;
+    T* op = reinterpret_cast<T*>(p.o) + b * p.o_stride_b + h * p.o_stride_h + v0 + 4 * tile.lv;
 
-    const int tid = threadIdx.x;
-    const int lane = tid % WAVE;
-    const int wave = tid / WAVE;
-    const int lv = tid % LANES_V;   // which 4 columns
-    const int rg = tid / LANES_V;   // which row group
-    const int v0 = blockIdx.x * BV + lv * 4;
-    const int h = blockIdx.y;
-    const int n = blockIdx.z;
+    float kx[KPL], qx[KPL], gt = 0.f, beta = 1.f;
+    f32x4 vt;
+    auto fetch = [&](int64_t t) {
+        const int64_t sidx = (b * p.T + t) * p.H + h;
+        load_run<KPL>(kp + t * p.k_stride_t + tile.lane * KPL, kx);
+        load_run<KPL>(qp + t * p.q_stride_t + tile.lane * KPL, qx);
+        if (p.g != nullptr) gt = p.g[sidx];
+        beta = load_beta(p.beta, p.beta_dtype, sidx);
+        vt = load4<T>(vp + t * p.v_stride_t);
+    };
+    if (t_begin < t_end) fetch(t_begin);  // (an empty sequence keeps its state)
+
+    const int64_t state_off = ((int64_t)n * p.H + h) * K * p.V + v0;
+    f32x4 S[RPT];
+    tile.load(S, p.h0 == nullptr ? nullptr : p.h0 + state_off, p.V);
+
+    for (int64_t t = t_begin; t < t_end; t++) {
+        const float eg = (p.g != nullptr) ? expf(gt) : 1.0f;
+        const TokenNorms norms = token_norms<KPL>(kx, qx, p.l2norm, p.scale);
+        // (the waves have taken the previous token's k^ and q^ out of s_kq when they leave contract's barrier, and its
+        // sums out of s_red when they reach this one)
+        if (tile.wave < 2) {
+#pragma unroll
+            for (int e = 0; e < KPL; e++) s_kq[tile.wave][tile.lane * KPL + e] = tile.wave == 0 ? kx[e] * norms.kn : qx[e] * norms.qn;
+        }
+        __syncthreads();
+        f32x4 k[RPT / 4], q[RPT / 4];
+#pragma unroll
+        for (int j = 0; j < RPT / 4; j++) {
+            k[j] = *reinterpret_cast<const f32x4*>(&s_kq[0][tile.row(4 * j)]);
+            q[j] = *reinterpret_cast<const f32x4*>(&s_kq[1][tile.row(4 * j)]);
+        }
+        f32x4 sk, sq, o;
+        tile.contract(S, k, q, sk, sq);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const float r = token_residual(vt[c], sk[c], eg, beta);
+            o[c] = token_output(sq[c], eg, r, norms.kq);
+#pragma unroll
+            for (int i = 0; i < RPT; i++) S[i][c] = token_state(S[i][c], eg, r, k[i / 4][i % 4]);
+        }
+        if (tile.rg == 0) store4<T>(op + t * p.o_stride_t, o);
+        if (t + 1 < t_end) fetch(t + 1);
+    }
+    if (p.ht != nullptr) tile.store(S, p.ht + state_off, p.V);
+}
+
+// More than one token: the same recurrence, laid out for the latency of a token.
+//
+// A token's state depends on the one before it, so a sequence takes as long as its tokens' chain: S^T k (a reduction over
+// K), r, S'.  Here the whole reduction stays in one DPP row: 16 lanes hold the K rows of CPL columns (K / 16 rows each), the
+// sum over them is four row rotations, and no wave waits for another one inside a token.  The four waves of a workgroup
+// take 4 CPL columns each of the same chain and share the tokens' vectors, which are staged in LDS TB tokens at a time
+// (normalised, as fp32) while the global loads of the next TB tokens are in flight: one barrier per TB tokens.
+// Bound by that chain: 0.21 us per token at K = 64 (B = 1, T = 256, H = 2, V = 64, fp32: 56 us, against 305 us with two
+// barriers and a trip to the L2 in every token), 0.32 us at K = 128 with the chip full (B = 4, T = 1024, H = 16, V = 128, fp32:
+// 350 us against 1434).
+template <typename T, int K, int CPL>
+__global__ __launch_bounds__(REC_THREADS) void recurrent_tokens_kernel(const RecurrentParams p) {
+    constexpr int TB = 16;                   // tokens per staged block
+    constexpr int RPT = K / 16;              // state rows per lane, consecutive ones
+    constexpr int KPL = K / WAVE;            // q/k elements per lane when a wave loads a whole row
+    constexpr int BV = 16 * CPL;             // columns per workgroup
+    constexpr int TPW = TB / REC_WAVES;      // tokens a wave stages
+    constexpr int NV = TB * BV / REC_THREADS;  // values of v a thread stages
+    static_assert(TB * BV % REC_THREADS == 0 && TB % REC_WAVES == 0, "staging does not divide over the workgroup");
+
+    __shared__ __attribute__((aligned(16))) float s_k[2][TB][K], s_q[2][TB][K];
+    __shared__ __attribute__((aligned(16))) float s_v[2][TB][BV];
+    __shared__ __attribute__((aligned(16))) float s_sc[2][TB][4];  // e^g, beta, k^ . q^
+
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
+    const int rg = lane % 16, cg = lane / 16;
+    const int v_base = blockIdx.x * BV;
+    const int v0 = wave * (4 * CPL) + cg * CPL;  // this lane's first column, within the workgroup's
+    const int h = blockIdx.y, n = blockIdx.z;
 
     int64_t b = n, t_begin = 0, t_end = p.T;
     if (p.pad_lens != nullptr) t_begin = p.T - min(max(p.pad_lens[n + 1] - p.pad_lens[n], 0), p.T);  // the last tokens of row n
@@ -79,120 +132,155 @@ __global__ __launch_bounds__(REC_THREADS) void recurrent_kernel(const RecurrentP
         b = 0, t_begin = t0, t_end = t0 + len;
     }
 
-    const int64_t state_off = (((int64_t)n * p.H + h) * K + (int64_t)rg * RPT) * p.V + v0;
-
-    f32x4 S[RPT];
-    if (p.h0 != nullptr) {
-#pragma unroll
-        for (int i = 0; i < RPT; i++) S[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p.h0 + state_off + (int64_t)i * p.V));
-    } else {
-#pragma unroll
-        for (int i = 0; i < RPT; i++) S[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-
     const int64_t hqk = p.qk_div > 1 ? h / p.qk_div : h;
     const T* qp = reinterpret_cast<const T*>(p.q) + b * p.q_stride_b + hqk * p.q_stride_h;
     const T* kp = reinterpret_cast<const T*>(p.k) + b * p.k_stride_b + hqk * p.k_stride_h;
-    const T* vp = reinterpret_cast<const T*>(p.v) + b * p.v_stride_b + h * p.v_stride_h + v0;
-    T* op = reinterpret_cast<T*>(p.o) + b * p.o_stride_b + h * p.o_stride_h + v0;
+    const T* vp = reinterpret_cast<const T*>(p.v) + b * p.v_stride_b + h * p.v_stride_h + v_base;
+    T* op = reinterpret_cast<T*>(p.o) + b * p.o_stride_b + h * p.o_stride_h + v_base + v0;
 
-    for (int64_t t = t_begin; t < t_end; t++) {
-        float* const s_k = s_k2[(t - t_begin) & 1];
-        // ---- wave 0 stages k^ and q^ (normalised, q scaled) in LDS; others go straight on ----
-        if (wave == 0) {
-            float kx[KPL], qx[KPL];
-            float ssk = 0.f, ssq = 0.f;
+    // ---- the next block's values: asked for in fetch, put into LDS in stage ----
+    float kx[TPW][KPL], qx[TPW][KPL], vx[NV], gx = 0.f, bx = 1.f;
+    auto fetch = [&](int64_t t0) {  // tokens past the sequence's end are read from its last one and never used
+#pragma unroll
+        for (int i = 0; i < TPW; i++) {
+            const int64_t t = min(t0 + wave * TPW + i, t_end - 1);
+            load_run<KPL>(kp + t * p.k_stride_t + lane * KPL, kx[i]);
+            load_run<KPL>(qp + t * p.q_stride_t + lane * KPL, qx[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const int at = i * REC_THREADS + tid;
+            vx[i] = to_f32(vp[min(t0 + at / BV, t_end - 1) * p.v_stride_t + at % BV]);
+        }
+        if (tid < TB) {
+            const int64_t sidx = (b * p.T + min(t0 + tid, t_end - 1)) * p.H + h;
+            if (p.g != nullptr) gx = p.g[sidx];
+            bx = load_beta(p.beta, p.beta_dtype, sidx);
+        }
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < TPW; i++) {
+            const int tt = wave * TPW + i;
+            const TokenNorms norms = token_norms<KPL>(kx[i], qx[i], p.l2norm, p.scale);
 #pragma unroll
             for (int e = 0; e < KPL; e++) {
-                kx[e] = to_f32(kp[t * p.k_stride_t + lane * KPL + e]);
-                qx[e] = to_f32(qp[t * p.q_stride_t + lane * KPL + e]);
-                ssk += kx[e] * kx[e];
-                ssq += qx[e] * qx[e];
+                // row lane KPL + e is row `at` of row group lane / 4; the groups' pieces of 4 rows lie side by side
+                const int at = lane % 4 * KPL + e, pos = at / 4 * 64 + lane / 4 * 4 + at % 4;
+                s_k[buf][tt][pos] = kx[i][e] * norms.kn;
+                s_q[buf][tt][pos] = qx[i][e] * norms.qn;
             }
-            float kn = 1.f, qn = p.scale;
-            if (p.l2norm) {
-                kn = rsqrtf(wave_sum(ssk) + L2NORM_EPS);
-                qn = rsqrtf(wave_sum(ssq) + L2NORM_EPS) * p.scale;
-            }
-            float kq = 0.f;
-#pragma unroll
-            for (int e = 0; e < KPL; e++) {
-                kx[e] *= kn;
-                qx[e] *= qn;
-                kq += kx[e] * qx[e];
-                s_k[lane * KPL + e] = kx[e];
-                s_q[lane * KPL + e] = qx[e];
-            }
-            kq = wave_sum(kq);
-            if (lane == 0) s_kq[0] = kq;
+            if (lane == 0) s_sc[buf][tt][2] = norms.kq;
         }
-        const int64_t sidx = (b * p.T + t) * p.H + h;
-        const float eg = (p.g != nullptr) ? expf(p.g[sidx]) : 1.0f;
-        const float beta = load_beta(p.beta, p.beta_dtype, sidx);
-        const f32x4 vt = load4<T>(vp + t * p.v_stride_t);
-        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NV; i++) {
+            const int at = i * REC_THREADS + tid;
+            s_v[buf][at / BV][at % BV] = vx[i];
+        }
+        if (tid < TB) s_sc[buf][tid][0] = p.g != nullptr ? expf(gx) : 1.f, s_sc[buf][tid][1] = bx;
+    };
 
-        // ---- partial S^T k and S^T q over this thread's rows ----
-        f32x4 pk = {0.f, 0.f, 0.f, 0.f}, pq = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int i = 0; i < RPT; i++) {
-            const float kr = s_k[rg * RPT + i];
-            const float qr = s_q[rg * RPT + i];
-            pk += S[i] * kr;
-            pq += S[i] * qr;
-        }
-        const float kq = s_kq[0];
-        // row groups inside a wave
-#pragma unroll
-        for (int off = LANES_V; off < WAVE; off <<= 1) {
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                pk[c] += __shfl_xor(pk[c], off, WAVE);
-                pq[c] += __shfl_xor(pq[c], off, WAVE);
-            }
-        }
-        if (lane < LANES_V) {
-            *reinterpret_cast<f32x4*>(&s_red[wave][lane][0]) = pk;
-            *reinterpret_cast<f32x4*>(&s_red[wave][lane][4]) = pq;
-        }
-        __syncthreads();
-        f32x4 sk = {0.f, 0.f, 0.f, 0.f}, sq = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int w = 0; w < REC_WAVES; w++) {
-            sk += *reinterpret_cast<const f32x4*>(&s_red[w][lv][0]);
-            sq += *reinterpret_cast<const f32x4*>(&s_red[w][lv][4]);
-        }
+    if (t_begin < t_end) fetch(t_begin);
 
-        // ---- rank-1 update and output ----
-        const f32x4 r = (vt - sk * eg) * beta;
+    auto state_at = [&](int i) { return (((int64_t)n * p.H + h) * K + RPT * rg + i) * p.V + v_base + v0; };
+    float S[RPT][CPL];
 #pragma unroll
-        for (int i = 0; i < RPT; i++) S[i] = S[i] * eg + r * s_k[rg * RPT + i];  // k^ re-read: keeps 16 registers free
-        if (rg == 0) store4<T>(op + t * p.o_stride_t, sq * eg + r * kq);
+    for (int i = 0; i < RPT; i++)
+#pragma unroll
+        for (int c = 0; c < CPL; c++) S[i][c] = p.h0 != nullptr ? p.h0[state_at(i) + c] : 0.f;
+
+    // one token's operands of this lane
+    struct Operands {
+        f32x4 k[RPT / 4], q[RPT / 4], sc;
+        float v[CPL];
+    };
+    auto read = [&](Operands& x, int buf, int tt) {
+#pragma unroll
+        for (int j = 0; j < RPT / 4; j++) {
+            x.k[j] = *reinterpret_cast<const f32x4*>(&s_k[buf][tt][64 * j + 4 * rg]);
+            x.q[j] = *reinterpret_cast<const f32x4*>(&s_q[buf][tt][64 * j + 4 * rg]);
+        }
+        x.sc = *reinterpret_cast<const f32x4*>(&s_sc[buf][tt][0]);
+#pragma unroll
+        for (int c = 0; c < CPL; c++) x.v[c] = s_v[buf][tt][v0 + c];
+    };
+
+    if (t_begin < t_end) stage(0);
+    __syncthreads();
+    int buf = 0;
+    for (int64_t t0 = t_begin; t0 < t_end; t0 += TB, buf ^= 1) {
+        const bool more = t0 + TB < t_end;
+        if (more) fetch(t0 + TB);
+        const int count = (int)min((int64_t)TB, t_end - t0);
+        Operands x;
+        read(x, buf, 0);
+        for (int tt = 0; tt < count; tt++) {
+            Operands next;
+            read(next, buf, min(tt + 1, TB - 1));
+            float sk[CPL], sq[CPL];
+#pragma unroll
+            for (int c = 0; c < CPL; c++) {
+                float k0 = 0.f, k1 = 0.f, q0 = 0.f, q1 = 0.f;
+#pragma unroll
+                for (int i = 0; i < RPT; i += 2) {
+                    k0 = fmaf(S[i][c], x.k[i / 4][i % 4], k0), k1 = fmaf(S[i + 1][c], x.k[i / 4][i % 4 + 1], k1);
+                    q0 = fmaf(S[i][c], x.q[i / 4][i % 4], q0), q1 = fmaf(S[i + 1][c], x.q[i / 4][i % 4 + 1], q1);
+                }
+                sk[c] = row16_sum(k0 + k1), sq[c] = row16_sum(q0 + q1);
+            }
+            const float eg = x.sc[0], beta = x.sc[1], kq = x.sc[2];
+#pragma unroll
+            for (int c = 0; c < CPL; c++) {
+                const float r = token_residual(x.v[c], sk[c], eg, beta);
+#pragma unroll
+                for (int i = 0; i < RPT; i++) S[i][c] = token_state(S[i][c], eg, r, x.k[i / 4][i % 4]);
+                if (rg == c) op[(t0 + tt) * p.o_stride_t + c] = from_f32<T>(token_output(sq[c], eg, r, kq));
+            }
+            x = next;
+        }
+        if (more) stage(buf ^ 1);
+        __syncthreads();
     }
 
     if (p.ht != nullptr) {
 #pragma unroll
-        for (int i = 0; i < RPT; i++) __builtin_nontemporal_store(S[i], reinterpret_cast<f32x4*>(p.ht + state_off + (int64_t)i * p.V));
+        for (int i = 0; i < RPT; i++)
+#pragma unroll
+            for (int c = 0; c < CPL; c++) p.ht[state_at(i) + c] = S[i][c];
     }
 }
 
+template <typename T, int K, int CPL>
+static int launch_recurrent_tokens(const RecurrentParams& p, int N, hipStream_t stream) {
+    hipLaunchKernelGGL((recurrent_tokens_kernel<T, K, CPL>), dim3(p.V / (16 * CPL), p.H, N), dim3(REC_THREADS), 0, stream, p);
+    return (int)hipGetLastError();
+}
+
 template <typename T, int K, int BV>
-static int launch_recurrent_tile(const RecurrentParams& p, int N, hipStream_t stream) {
-    dim3 grid(p.V / BV, p.H, N);
-    hipLaunchKernelGGL((recurrent_kernel<T, K, BV>), grid, dim3(REC_THREADS), 0, stream, p);
+static int launch_recurrent_step(const RecurrentParams& p, int N, hipStream_t stream) {
+    hipLaunchKernelGGL((recurrent_step_kernel<T, K, BV>), dim3(p.V / BV, p.H, N), dim3(4 * BV), 0, stream, p);
     return (int)hipGetLastError();
 }
 
 template <typename T, int K>
 static int launch_recurrent_k(const RecurrentParams& p, int N, hipStream_t stream) {
-    // Wide tiles give the longest contiguous rows; narrow ones give more workgroups when
-    // there are few (sequence, head) pairs.
     const int64_t pairs = (int64_t)N * p.H;
-    if constexpr (K <= 128) {  // a K = 256 tile of 128 columns would not fit the register file
-        if (p.V % 128 == 0 && pairs * (p.V / 128) >= 1024) return launch_recurrent_tile<T, K, 128>(p, N, stream);
+    // The tokens kernel: as few columns per lane as leave at most 1024 workgroups (four per CU, what LDS and registers hold at
+    // a time).  Measured with 1 | 2 | 4: B = 5, T = 60, H = 16, K = V = 128 (640 workgroups at 1) 36 | 38 | 41 us, B = 5, T = 33,
+    // H = 32, V = 256 (2560) 60 | 55 | 58 us, B = 64, T = 16, H = 16, V = 128 (8192) 100 | 83 | 72 us.  Its lanes take the state
+    // in 16-byte pieces of many rows, which costs more than its shorter chain wins where a large batch meets a few tokens:
+    // there the step kernel walks over the tokens (B = 64, H = 16, V = 128: T = 2 28 against 44 us, T = 16 77 against 72 us).
+    if (p.T > 1 && !(p.T < 12 && pairs * p.V >= 256 * 256)) {
+        if (pairs * (p.V / 16) <= 1024) return launch_recurrent_tokens<T, K, 1>(p, N, stream);
+        if (pairs * (p.V / 32) <= 2048 || p.V % 64 != 0) return launch_recurrent_tokens<T, K, 2>(p, N, stream);
+        return launch_recurrent_tokens<T, K, 4>(p, N, stream);
     }
-    if (p.V % 64 == 0 && pairs * (p.V / 64) >= 512) return launch_recurrent_tile<T, K, 64>(p, N, stream);
-    return launch_recurrent_tile<T, K, 32>(p, N, stream);
+    // The step kernel: wide tiles give the longest contiguous rows (256 sequences x 32 heads, K = V = 128: 164 us with 128
+    // columns, 185 with 64, 202 with 32), narrow ones more workgroups when there are few (sequence, head) pairs (1 x 16:
+    // 4.3, 3.8, 3.6 us).
+    if (p.V % 128 == 0 && pairs * (p.V / 128) >= 256) return launch_recurrent_step<T, K, 128>(p, N, stream);
+    if (p.V % 64 == 0 && pairs * (p.V / 64) >= 512) return launch_recurrent_step<T, K, 64>(p, N, stream);
+    return launch_recurrent_step<T, K, 32>(p, N, stream);
 }
 
 template <typename T>

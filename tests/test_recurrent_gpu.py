@@ -147,6 +147,26 @@ def test_decode_equals_prefill_continuation():
     assert torch.equal(o_tail, o_all[:, 20:]) and torch.equal(h_tail, h_all)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize(
+    "B, H, T, K, V",
+    # block edges of the several-token kernel (16 tokens), one to four columns per lane (by the number of workgroups), the
+    # few-token walk of the one-token kernel (large batch, T < 12) and its three tile widths
+    [(1, 1, 2, 64, 32), (1, 2, 15, 128, 96), (1, 2, 16, 256, 64), (2, 3, 17, 64, 128), (1, 1, 49, 256, 32),
+     (40, 16, 13, 64, 64), (70, 16, 12, 128, 128), (66, 16, 3, 64, 64), (33, 8, 11, 128, 256), (20, 16, 2, 256, 512)],
+)  # fmt: skip
+def test_several_tokens_match_the_oracle_and_the_steps_they_consist_of(dtype, B, H, T, K, V):
+    inp = random_inputs(B=B, T=T, H=H, K=K, V=V, dtype=dtype, seed=60 + T, normalize=False)
+    o, ht = _check(inp, dtype, use_qk_l2norm_in_kernel=True)
+    gpu = _to_gpu(inp)
+    cut = T - 1  # the last token on its own: the same bits, whichever kernel and tile width either call runs on
+    part = lambda lo, hi: {n: (x[:, lo:hi] if n != "initial_state" else x) for n, x in gpu.items()}  # noqa: E731
+    run = lambda x: lm_engine_amd.fused_recurrent_gated_delta_rule(**x, output_final_state=True, use_qk_l2norm_in_kernel=True)  # noqa: E731
+    o_head, h_head = run(part(0, cut))
+    o_last, h_last = run(dict(part(cut, T), initial_state=h_head))
+    assert torch.equal(torch.cat([o_head, o_last], dim=1), o) and torch.equal(h_last, ht)
+
+
 def test_output_final_state_false_returns_none_and_runs_are_bitwise_repeatable():
     inp = _to_gpu(random_inputs(B=2, T=8, H=2, K=64, V=64, dtype=torch.bfloat16, seed=46))
     o1, none = lm_engine_amd.fused_recurrent_gated_delta_rule(**inp)
