@@ -521,6 +521,46 @@ typedef struct gdn_norm_bwd_args {
 } gdn_norm_bwd_args;
 int gdn_gated_rmsnorm_bwd(const gdn_norm_bwd_args *args, void *stream);
 
+/*
+ * One decode step of the layer between its projections, in one launch: the convolution's one-token update
+ * (depthwise_causal_convolution.py:199-231), the gates (module.py:179-183), the recurrence with l2-normalised q and k
+ * (module.py:210-222) and the gated norm (module.py:238-242).  Results are those of gdn_causal_conv1d_fwd,
+ * gdn_gates_fwd, gdn_recurrent_fwd (GDN_FLAG_L2NORM) and gdn_gated_rmsnorm_fwd one after the other, up to the order of
+ * fp32 sums.
+ *   qkv             [B, C] in dtype, C = 2 HK K + H V channels (q | k | v), rows qkv_stride_b elements apart
+ *   conv_weight     [C, kernel_size], conv_bias [C] or NULL, in conv_w_dtype;  activation: gdn_activation
+ *   conv_state      [B, C, kernel_size - 1] contiguous in dtype or NULL (zeros);  conv_state_out: the same, not the same memory
+ *   a, b            [B, H] in dtype, rows *_stride_b apart;  A_log, dt_bias [H] fp32;  beta_scale as in gdn_gate_args
+ *   h0 (or NULL: zeros), ht   [B, H, K, V] fp32 contiguous, 16-byte aligned; ht may be h0
+ *   gate            [B, H V] in dtype, rows gate_stride_b apart, or NULL;  norm_weight [V] in norm_w_dtype or NULL
+ *   out             [B, H, V] contiguous in dtype, 16-byte aligned
+ *   tickets, scratch   int32 [B H], zero before the first call that uses it and left zero by every call, and fp32 [B H V];
+ *                   needed when gdn_layer_step_tiles(B, H, V) > 1, NULL otherwise.  Calls that may overlap (several streams)
+ *                   need their own.
+ * K = 64, 128 or 256, V a multiple of 32 and at most 512, kernel_size 2..4.  Only out, h0 and ht need more than
+ * the alignment of their elements.
+ */
+typedef struct gdn_layer_step_args {
+    const void *qkv, *conv_weight, *conv_bias, *conv_state;
+    void *conv_state_out;
+    const void *a, *b;
+    const float *A_log, *dt_bias;
+    const float *h0;
+    float *ht;
+    const void *gate, *norm_weight;
+    void *out;
+    int32_t *tickets;
+    float *scratch;
+    int64_t qkv_stride_b, a_stride_b, b_stride_b, gate_stride_b;
+    int32_t B, HK, H, K, V, kernel_size;
+    int32_t dtype, conv_w_dtype, norm_w_dtype, activation;
+    float beta_scale, scale, eps;
+    int32_t reserved;
+} gdn_layer_step_args;
+int gdn_layer_step(const gdn_layer_step_args *args, void *stream);
+/* Workgroups that gdn_layer_step puts on one (sequence, head); above 1 it needs tickets and scratch. */
+int gdn_layer_step_tiles(int B, int H, int V);
+
 #ifdef __cplusplus
 }
 #endif

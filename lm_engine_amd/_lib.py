@@ -54,6 +54,8 @@ EXPORTED_SYMBOLS = (
     "gdn_gates_bwd",
     "gdn_gated_rmsnorm_fwd",
     "gdn_gated_rmsnorm_bwd",
+    "gdn_layer_step",
+    "gdn_layer_step_tiles",
 )
 
 GDN_CHUNK_KERNELS = 3
@@ -252,6 +254,9 @@ def load_library() -> ctypes.CDLL:
     lib.gdn_gates_bwd.restype = ctypes.c_int
     lib.gdn_gated_rmsnorm_fwd.argtypes = [ctypes.POINTER(GdnNormArgs), ctypes.c_void_p]
     lib.gdn_gated_rmsnorm_fwd.restype = ctypes.c_int
+
+    lib.gdn_layer_step_tiles.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int]
+    lib.gdn_layer_step_tiles.restype = ctypes.c_int
 
     version = lib.gdn_abi_version()
     if version != GDN_ABI_VERSION:

@@ -1,4 +1,5 @@
-"""Builds lm_engine_amd/libgdn_hip.so from the HIP sources in lm_engine_amd/csrc with hipcc.
+"""Builds lm_engine_amd/libgdn_hip.so from the HIP sources in lm_engine_amd/csrc with hipcc, and
+lm_engine_amd/gdn_host.so (host code only, against torch's headers) with g++.
 
 The library is a plain C-ABI shared object (see include/gdn_hip.h): it links only the HIP
 runtime, so it is independent of the ROCm version PyTorch was built against.  hipcc
@@ -20,8 +21,9 @@ PACKAGE_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC_DIR = os.path.join(PACKAGE_DIR, "csrc")
 INCLUDE_DIR = os.path.join(os.path.dirname(PACKAGE_DIR), "include")
 LIBRARY_PATH = os.path.join(PACKAGE_DIR, "libgdn_hip.so")
+HOST_MODULE_PATH = os.path.join(PACKAGE_DIR, "gdn_host.so")
 
-SOURCES = ("gdn_api.hip", "gdn_recurrent.hip", "gdn_chunk.hip", "gdn_chunk32.hip", "gdn_chunk_fused.hip", "gdn_chunk_bwd.hip", "gdn_conv1d.hip", "gdn_conv1d_bwd.hip", "gdn_elementwise.hip")
+SOURCES = ("gdn_api.hip", "gdn_recurrent.hip", "gdn_layer_step.hip", "gdn_chunk.hip", "gdn_chunk32.hip", "gdn_chunk_fused.hip", "gdn_chunk_bwd.hip", "gdn_conv1d.hip", "gdn_conv1d_bwd.hip", "gdn_elementwise.hip")
 
 HIPCC_FLAGS = (
     "--offload-arch=gfx950",
@@ -48,6 +50,25 @@ def _hipcc() -> str:
 
 CYCLE_BUDGET_LIBRARY_PATH = os.path.join(PACKAGE_DIR, "libgdn_hip_cycles.so")
 CYCLE_BUDGET_SOURCES = ("gdn_api.hip", "gdn_chunk.hip", "gdn_chunk32.hip", "gdn_chunk_bwd.hip")  # the sources that read GDN_CYCLE_BUDGET
+
+
+def build_host_module() -> str:
+    """Compiles csrc/gdn_host.cpp, the host path of the inference entry points; always rebuilds."""
+    import sysconfig
+
+    import torch
+
+    torch_dir = os.path.dirname(os.path.abspath(torch.__file__))
+    tmp = HOST_MODULE_PATH + ".tmp"
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{INCLUDE_DIR}", f"-I{torch_dir}/include", f"-I{torch_dir}/include/torch/csrc/api/include",
+           f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC_DIR, "gdn_host.cpp"), "-o", tmp,
+           f"-L{torch_dir}/lib", "-ltorch_python", "-ltorch_cpu", "-lc10"]  # fmt: skip
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"g++ failed on gdn_host.cpp:\n{proc.stdout}\n{proc.stderr}")
+    os.replace(tmp, HOST_MODULE_PATH)
+    return HOST_MODULE_PATH
 
 
 def build_library(verbose: bool = False, extra_flags: tuple[str, ...] = (), cycle_budget: bool = False) -> str:
@@ -78,8 +99,11 @@ def build_library(verbose: bool = False, extra_flags: tuple[str, ...] = (), cycl
             print(proc.stderr, file=sys.stderr)
         return obj
 
-    with ThreadPoolExecutor(max_workers=len(sources)) as pool:
+    with ThreadPoolExecutor(max_workers=len(sources) + 1) as pool:
+        host_module = None if cycle_budget else pool.submit(build_host_module)
         objects = list(pool.map(compile_one, sources))
+        if host_module is not None:
+            host_module.result()
     if cycle_budget:
         objects += [os.path.join(build_dir, src.replace(".hip", ".o")) for src in SOURCES if src not in CYCLE_BUDGET_SOURCES]
 

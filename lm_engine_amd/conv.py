@@ -25,6 +25,7 @@ import torch
 
 from . import _lib
 from ._autograd import kernel_with_formula_backward
+from ._host import host, raw_stream
 from .kernels import Kernel, is_kernel_allowed
 
 
@@ -72,6 +73,12 @@ def depthwise_causal_convolution(
         from . import _opaque
 
         return _opaque.depthwise_causal_convolution(x, weight, bias, input_state, attention_mask, output_state, activation)
+
+    if x.is_cuda and activation in _IN_KERNEL_ACTIVATIONS and is_kernel_allowed(Kernel.gated_delta_rule):
+        result = host().conv(raw_stream(x.get_device()), x, weight, bias, input_state, attention_mask, output_state,
+                             _IN_KERNEL_ACTIVATIONS[activation])  # fmt: skip
+        if result is not None:
+            return result
 
     def formula(x, weight, bias, input_state):
         return convolution_formula(x, weight, bias, input_state, attention_mask, output_state, activation)

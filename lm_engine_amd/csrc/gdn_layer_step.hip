@@ -1,0 +1,274 @@
+// One decode step of the whole layer, between its input and its output projection, in one launch:
+//
+//     q, k, v = silu(conv(qkv, conv_state))        beta = sigmoid(b) [* 2]      g = -exp(A_log) softplus(a + dt_bias)
+//     o, S = gated delta rule with l2-normalised q, k      out = rmsnorm(o * silu(gate)) * weight
+//
+// lm_engine/modeling_utils/sequence_mixer_blocks/gated_deltanet/module.py:168-242 for a sequence dimension of one.  As
+// separate launches (convolution, gates, recurrence, norm) a step of one sequence is four launches of 2 - 5 us that wait for
+// each other through memory, and four host calls; the state, which is all that a larger batch has to move, passes once either
+// way.  Same roundings as the separate kernels: the convolution's output, beta and o are rounded to the activation dtype.
+//
+// A workgroup owns a K x BV tile of one state (StepTile) and computes the convolution of the 2 K + BV channels it needs; the
+// tiles of a (sequence, head), and the value heads that share a head of q and k, repeat those of q and k (a few hundred
+// multiply-adds next to 128 KiB of state).  The norm needs all V columns.  With one tile per head it is formed on the
+// spot; else the tiles leave o silu(gate) in `scratch` and take a ticket, and the tile that draws the last one writes the
+// head's output: those stores are device-scope (the tiles sit on different XCDs) and complete before the ticket is drawn, and
+// the state's stores are issued behind it, so nobody waits for them.
+//
+// Bound by the launch and one trip through memory for small batches (one sequence x 16 heads, K = V = 128: 6 us on the GPU,
+// 11 us a step with the host's work, where the four launches took 86), by the state's bytes for large ones (200 sequences x 16
+// heads: 75 us for 422 MB = 5.6 TB/s).
+
+#include <type_traits>
+
+#include "gdn_recurrent_common.h"
+
+namespace gdn {
+
+struct LayerStepParams {
+    const void *qkv, *conv_weight, *conv_bias, *conv_state;
+    void* conv_state_out;
+    const void *a, *b;
+    const float *A_log, *dt_bias;
+    const float* h0;
+    float* ht;
+    const void *gate, *norm_weight;
+    void* out;
+    int32_t* tickets;  // [B H], zero before and after the launch
+    float* scratch;    // [B H][V]
+    int64_t qkv_stride_b, a_stride_b, b_stride_b, gate_stride_b;
+    int HK, H, V, group;  // group = H / HK
+    int conv_w_dtype, norm_w_dtype, silu;
+    float beta_scale, scale, eps;
+};
+
+__device__ __forceinline__ float load_scalar(const void* p, int dtype, int64_t i) {
+    return dtype == GDN_BF16 ? (float)reinterpret_cast<const bf16_t*>(p)[i] : reinterpret_cast<const float*>(p)[i];
+}
+
+__device__ __forceinline__ float silu_of(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
+
+template <typename T, int K, int BV, int KS>
+__global__ __launch_bounds__(4 * BV) void layer_step_kernel(const LayerStepParams p) {
+    typedef StepTile<K, BV> Tile;
+    constexpr int RPT = Tile::RPT, KPL = K / WAVE, THREADS = Tile::THREADS;
+    constexpr int CH = 2 * K + BV;                        // channels of the convolution: q | k | v
+    constexpr int PER = (CH + THREADS - 1) / THREADS;     // of them per thread
+    __shared__ __attribute__((aligned(16))) float s_red[Tile::WAVES][2][BV];
+    __shared__ __attribute__((aligned(16))) float s_x[CH];
+    const Tile tile(s_red);
+    const int tid = threadIdx.x;
+    const int v0 = blockIdx.x * BV, h = blockIdx.y, hk = h / p.group;
+    const int64_t b = blockIdx.z, C = 2 * (int64_t)p.HK * K + (int64_t)p.H * p.V;
+
+    // ---- everything this token needs is asked for ahead of the state ----
+    const T* x = reinterpret_cast<const T*>(p.qkv) + b * p.qkv_stride_b;
+    T cur[PER], hist[PER][KS - 1];
+    float w[PER][KS], bias[PER];
+    int64_t channel[PER];
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        const int c = min(tid + i * THREADS, CH - 1);  // (the last round's spare threads repeat the last channel)
+        channel[i] = c < K ? (int64_t)hk * K + c : c < 2 * K ? (int64_t)(p.HK + hk) * K + c - K : 2 * (int64_t)p.HK * K + (int64_t)h * p.V + v0 + c - 2 * K;
+        cur[i] = x[channel[i]];
+#pragma unroll
+        for (int j = 0; j < KS - 1; j++)
+            hist[i][j] = p.conv_state == nullptr ? (T)0.f : reinterpret_cast<const T*>(p.conv_state)[(b * C + channel[i]) * (KS - 1) + j];
+#pragma unroll
+        for (int j = 0; j < KS; j++) w[i][j] = load_scalar(p.conv_weight, p.conv_w_dtype, channel[i] * KS + j);
+        bias[i] = p.conv_bias == nullptr ? 0.f : load_scalar(p.conv_bias, p.conv_w_dtype, channel[i]);
+    }
+    const bool writes_out = tile.rg == 0;  // the lanes that end up with the tile's output: the first BV / 4 of wave 0
+    float gate[4], norm_w[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        gate[e] = 0.f, norm_w[e] = 1.f;
+        if (writes_out && p.gate != nullptr) gate[e] = (float)reinterpret_cast<const T*>(p.gate)[b * p.gate_stride_b + (int64_t)h * p.V + v0 + 4 * tile.lv + e];
+        if (writes_out && p.norm_weight != nullptr) norm_w[e] = load_scalar(p.norm_weight, p.norm_w_dtype, v0 + 4 * tile.lv + e);
+    }
+    const float a_in = (float)reinterpret_cast<const T*>(p.a)[b * p.a_stride_b + h];
+    const float b_in = (float)reinterpret_cast<const T*>(p.b)[b * p.b_stride_b + h];
+    const float A_log = p.A_log[h], dt_bias = p.dt_bias[h];
+
+    const int64_t state_off = (b * p.H + h) * K * p.V + v0;
+    f32x4 S[RPT];
+    tile.load(S, p.h0 == nullptr ? nullptr : p.h0 + state_off, p.V);
+
+    // ---- convolution and gates ----
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+        const int c = tid + i * THREADS;
+        float acc = bias[i] + w[i][KS - 1] * (float)cur[i];
+#pragma unroll
+        for (int j = 0; j < KS - 1; j++) acc += w[i][j] * (float)hist[i][j];
+        if (p.silu) acc = silu_of(acc);
+        // q and k are written by one of the workgroups that compute them
+        if (c < CH) {
+            s_x[c] = (float)(T)acc;
+            if (c >= 2 * K || (blockIdx.x == 0 && h % p.group == 0)) {
+                T* out = reinterpret_cast<T*>(p.conv_state_out) + (b * C + channel[i]) * (KS - 1);
+#pragma unroll
+                for (int j = 0; j + 1 < KS - 1; j++) out[j] = hist[i][j + 1];
+                out[KS - 2] = cur[i];
+            }
+        }
+    }
+    const float z = a_in + dt_bias;
+    const float eg = expf(-expf(A_log) * (z > 20.f ? z : log1pf(__expf(z))));
+    const float beta = (float)(T)((float)(T)(1.f / (1.f + expf(-b_in))) * p.beta_scale);
+    __syncthreads();
+
+    // ---- the recurrence ----
+    float kx[KPL], qx[KPL];
+#pragma unroll
+    for (int e = 0; e < KPL; e++) qx[e] = s_x[tile.lane * KPL + e], kx[e] = s_x[K + tile.lane * KPL + e];
+    const TokenNorms norms = token_norms<KPL>(kx, qx, true, p.scale);
+    f32x4 k[RPT / 4], q[RPT / 4];
+#pragma unroll
+    for (int j = 0; j < RPT / 4; j++) {
+        q[j] = *reinterpret_cast<const f32x4*>(&s_x[tile.row(4 * j)]) * norms.qn;
+        k[j] = *reinterpret_cast<const f32x4*>(&s_x[K + tile.row(4 * j)]) * norms.kn;
+    }
+    const f32x4 vt = *reinterpret_cast<const f32x4*>(&s_x[2 * K + 4 * tile.lv]);
+    f32x4 sk, sq, r, y;
+    tile.contract(S, k, q, sk, sq);
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        r[c] = token_residual(vt[c], sk[c], eg, beta);
+        y[c] = (float)(T)token_output(sq[c], eg, r[c], norms.kq);  // o as the operator hands it on
+        if (p.gate != nullptr) y[c] *= silu_of(gate[c]);
+    }
+
+    // ---- the norm over the head's V columns: wave 0 ----
+    T* const out = reinterpret_cast<T*>(p.out) + (b * p.H + h) * p.V;
+    if (tile.wave == 0) {
+        if (p.V == BV) {
+            float ss = 0.f;
+            if (writes_out) ss = y[0] * y[0] + y[1] * y[1] + y[2] * y[2] + y[3] * y[3];
+            const float scale = rsqrtf(wave_total(ss) / (float)BV + p.eps);
+            if (writes_out) store4<T>(out + 4 * tile.lv, f32x4{y[0] * scale * norm_w[0], y[1] * scale * norm_w[1], y[2] * scale * norm_w[2], y[3] * scale * norm_w[3]});
+        } else {
+            float* const row = p.scratch + (b * p.H + h) * p.V;
+            if (writes_out) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) __hip_atomic_store(row + v0 + 4 * tile.lv + e, y[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            int drawn = 0;
+            int32_t* const ticket = p.tickets + b * p.H + h;
+            if (tile.lane == 0) drawn = __hip_atomic_fetch_add(ticket, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            drawn = __builtin_amdgcn_readfirstlane(drawn);
+            if (drawn == (int)gridDim.x - 1) {  // all other tiles of this head have stored their part
+                float ss = 0.f, part[8];
+#pragma unroll
+                for (int i = 0; i < 8; i++) {  // V <= 512
+                    const int c = tile.lane + 64 * i;
+                    part[i] = c < p.V ? __hip_atomic_load(row + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
+                    ss += part[i] * part[i];
+                }
+                const float scale = rsqrtf(wave_total(ss) / (float)p.V + p.eps);
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    const int c = tile.lane + 64 * i;
+                    if (c < p.V) out[c] = (T)(part[i] * scale * (p.norm_weight == nullptr ? 1.f : load_scalar(p.norm_weight, p.norm_w_dtype, c)));
+                }
+                if (tile.lane == 0) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+            }
+        }
+    }
+
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int i = 0; i < RPT; i++) S[i][c] = token_state(S[i][c], eg, r[c], k[i / 4][i % 4]);
+    tile.store(S, p.ht + state_off, p.V);
+}
+
+namespace {
+
+// Columns per workgroup.  A head of at most 128 columns is one tile and needs no ticket (one sequence x 16 heads, K = V = 128:
+// 6.0 us a launch, 9.1 and 10.0 with 64 and 32 columns and tickets).  Wider ones: 128 columns while that leaves every CU a
+// workgroup, else 64 (K = 256, V = 512, 2 heads, 32 | 64 | 128 columns: 2 sequences 13.9 | 12.6 | 12.9 us, 53 sequences 36.2 | 32.0 |
+// 30.3 us; the narrower the tile, the more often the convolution of q and k is repeated).
+int step_tile_columns(int B, int H, int V) {
+    if (V == 32 || V == 64 || V == 128) return V;
+    if (V % 128 == 0 && (int64_t)B * H * (V / 128) >= 256) return 128;
+    return V % 64 == 0 ? 64 : 32;
+}
+
+template <typename T, int K, int BV>
+int launch_step_tile(const LayerStepParams& p, int B, int kernel_size, hipStream_t stream) {
+    const dim3 grid(p.V / BV, p.H, B);
+    if (kernel_size == 2) hipLaunchKernelGGL((layer_step_kernel<T, K, BV, 2>), grid, dim3(4 * BV), 0, stream, p);
+    else if (kernel_size == 3) hipLaunchKernelGGL((layer_step_kernel<T, K, BV, 3>), grid, dim3(4 * BV), 0, stream, p);
+    else hipLaunchKernelGGL((layer_step_kernel<T, K, BV, 4>), grid, dim3(4 * BV), 0, stream, p);
+    return (int)hipGetLastError();
+}
+
+template <typename T, int K>
+int launch_step_k(const LayerStepParams& p, int B, int kernel_size, hipStream_t stream) {
+    switch (step_tile_columns(B, p.H, p.V)) {
+        case 128: return launch_step_tile<T, K, 128>(p, B, kernel_size, stream);
+        case 64: return launch_step_tile<T, K, 64>(p, B, kernel_size, stream);
+        default: return launch_step_tile<T, K, 32>(p, B, kernel_size, stream);
+    }
+}
+
+template <typename T>
+int launch_step(const LayerStepParams& p, int B, int K, int kernel_size, hipStream_t stream) {
+    if (K == 64) return launch_step_k<T, 64>(p, B, kernel_size, stream);
+    if (K == 128) return launch_step_k<T, 128>(p, B, kernel_size, stream);
+    return launch_step_k<T, 256>(p, B, kernel_size, stream);
+}
+
+inline bool aligned_to(const void* p, uintptr_t n) { return (reinterpret_cast<uintptr_t>(p) % n) == 0; }
+
+}  // namespace
+}  // namespace gdn
+
+extern "C" int gdn_layer_step_tiles(int B, int H, int V) {
+    return B <= 0 || H <= 0 || V <= 0 || V % 32 != 0 ? 0 : V / gdn::step_tile_columns(B, H, V);
+}
+
+extern "C" int gdn_layer_step(const gdn_layer_step_args* a, void* stream) {
+    if (a == nullptr) return GDN_ERR_NULL;
+    const void* needed[] = {a->qkv, a->conv_weight, a->conv_state_out, a->a, a->b, a->A_log, a->dt_bias, a->ht, a->out};
+    for (const void* x : needed)
+        if (x == nullptr) return GDN_ERR_NULL;
+    if (a->B <= 0 || a->HK <= 0 || a->H <= 0 || a->V <= 0 || a->H % a->HK != 0) return GDN_ERR_SHAPE;
+    if (a->B > 65535 || a->H > 65535) return GDN_ERR_UNSUPPORTED;
+    if ((a->K != 64 && a->K != 128 && a->K != 256) || a->V % 32 != 0 || a->V > 512) return GDN_ERR_UNSUPPORTED;
+    if (a->kernel_size < 2 || a->kernel_size > 4) return GDN_ERR_UNSUPPORTED;
+    if (a->activation != GDN_ACT_NONE && a->activation != GDN_ACT_SILU) return GDN_ERR_UNSUPPORTED;
+    const int32_t dtypes[] = {a->dtype, a->conv_w_dtype, a->norm_w_dtype};
+    for (int32_t d : dtypes)
+        if (d != GDN_BF16 && d != GDN_F32) return GDN_ERR_UNSUPPORTED;
+    const int64_t C = 2 * (int64_t)a->HK * a->K + (int64_t)a->H * a->V;
+    if (a->qkv_stride_b < (a->B > 1 ? C : 0) || a->a_stride_b < 0 || a->b_stride_b < 0 || a->gate_stride_b < 0) return GDN_ERR_SHAPE;
+    if (a->conv_state_out == a->conv_state) return GDN_ERR_SHAPE;  // several workgroups read a channel's state
+    if ((a->h0 && !gdn::aligned_to(a->h0, 16)) || !gdn::aligned_to(a->ht, 16) || !gdn::aligned_to(a->out, 16)) return GDN_ERR_ALIGN;
+    const uintptr_t size = a->dtype == GDN_BF16 ? 2 : 4;
+    const void* elements[] = {a->qkv, a->conv_state, a->conv_state_out, a->a, a->b, a->gate};
+    for (const void* x : elements)
+        if (!gdn::aligned_to(x, size)) return GDN_ERR_ALIGN;
+    const void* words[] = {a->A_log, a->dt_bias, a->tickets, a->scratch};
+    for (const void* x : words)
+        if (!gdn::aligned_to(x, 4)) return GDN_ERR_ALIGN;
+    if (!gdn::aligned_to(a->conv_weight, a->conv_w_dtype == GDN_BF16 ? 2 : 4) || !gdn::aligned_to(a->conv_bias, a->conv_w_dtype == GDN_BF16 ? 2 : 4) ||
+        !gdn::aligned_to(a->norm_weight, a->norm_w_dtype == GDN_BF16 ? 2 : 4))
+        return GDN_ERR_ALIGN;
+    if (gdn_layer_step_tiles(a->B, a->H, a->V) > 1 && (a->tickets == nullptr || a->scratch == nullptr)) return GDN_ERR_WORKSPACE;
+
+    gdn::LayerStepParams p;
+    p.qkv = a->qkv, p.conv_weight = a->conv_weight, p.conv_bias = a->conv_bias, p.conv_state = a->conv_state;
+    p.conv_state_out = a->conv_state_out, p.a = a->a, p.b = a->b, p.A_log = a->A_log, p.dt_bias = a->dt_bias;
+    p.h0 = a->h0, p.ht = a->ht, p.gate = a->gate, p.norm_weight = a->norm_weight, p.out = a->out;
+    p.tickets = a->tickets, p.scratch = a->scratch;
+    p.qkv_stride_b = a->qkv_stride_b, p.a_stride_b = a->a_stride_b, p.b_stride_b = a->b_stride_b, p.gate_stride_b = a->gate_stride_b;
+    p.HK = a->HK, p.H = a->H, p.V = a->V, p.group = a->H / a->HK;
+    p.conv_w_dtype = a->conv_w_dtype, p.norm_w_dtype = a->norm_w_dtype, p.silu = a->activation == GDN_ACT_SILU ? 1 : 0;
+    p.beta_scale = a->beta_scale, p.scale = a->scale, p.eps = a->eps;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    return a->dtype == GDN_BF16 ? gdn::launch_step<gdn::bf16_t>(p, a->B, a->K, a->kernel_size, st)
+                                : gdn::launch_step<float>(p, a->B, a->K, a->kernel_size, st);
+}

@@ -8,6 +8,8 @@ Follows lm_engine/modeling_utils/sequence_mixer_blocks/gated_deltanet/module.py:
     o, h = chunk or fused_recurrent (T <= 64)             :193-222  -> gated_delta_rule kernels
     o = o_norm(o * silu(gate))                            :238-241  -> gated_rmsnorm
 
+For one token per sequence (decoding) all of it is one launch, ``gdn_layer_step``.
+
 With an attention mask the reference packs q, k, v, g, beta into one token stream and unpacks the output
 (:185-191, :226-227, sequence_packing.py:25-93; as written there the packed tensors lose the batch
 dimension the operator wants and the unpack shape is not the output's).  Here nothing is copied: the mask
@@ -19,9 +21,11 @@ from __future__ import annotations
 
 import torch
 
-from .conv import depthwise_causal_convolution
+from ._host import host, raw_stream
+from .conv import _IN_KERNEL_ACTIVATIONS, depthwise_causal_convolution
+from .kernels import Kernel, is_kernel_allowed
 from .layer_ops import delta_rule_gates, gated_rmsnorm
-from .ops import RECURRENT_MAX_TOKENS, chunk_gated_delta_rule, fused_recurrent_gated_delta_rule
+from .ops import RECURRENT_MAX_TOKENS, chunk_gated_delta_rule, fused_recurrent_gated_delta_rule, layer_step_workspace
 
 
 def gated_deltanet_mixing(
@@ -58,6 +62,20 @@ def gated_deltanet_mixing(
         raise ValueError("num_v_heads must be a multiple of num_k_heads")
     use_cache = cache is not None
     conv_state, h = cache if use_cache else (None, None)
+
+    if (S == 1 and use_cache and attention_mask is None and qkv.is_cuda and conv_activation in _IN_KERNEL_ACTIVATIONS
+            and is_kernel_allowed(Kernel.gated_delta_rule) and not torch.compiler.is_compiling()):  # fmt: skip
+        # decoding: one launch, where the operands are the usual ones (None: they are not, or a gradient is needed)
+        device_index = qkv.get_device()
+        stream = raw_stream(device_index)
+        step = host().layer_step(stream, qkv, a, b, gate, conv_weight, conv_bias, A_log, dt_bias, norm_weight,
+                                 torch.finfo(qkv.dtype).eps if norm_eps is None else norm_eps, num_k_heads, num_v_heads, k_head_dim,
+                                 v_head_dim, conv_state, h, 2.0 if allow_neg_eigval else 1.0, k_head_dim**-0.5 if scale is None else scale,
+                                 _IN_KERNEL_ACTIVATIONS[conv_activation],
+                                 lambda pairs, V: layer_step_workspace(device_index, stream, pairs, V))  # fmt: skip
+        if step is not None:
+            o, conv_state, h = step
+            return o, (conv_state, h)
 
     qkv, conv_state = depthwise_causal_convolution(qkv, conv_weight, conv_bias, conv_state, attention_mask, use_cache,
                                                    conv_activation)  # fmt: skip

@@ -19,6 +19,7 @@ import torch
 
 from . import _lib
 from ._autograd import kernel_with_formula_backward
+from ._host import host, raw_stream
 from .kernels import Kernel, is_kernel_allowed
 
 
@@ -65,6 +66,11 @@ def delta_rule_gates(
         from . import _opaque
 
         return _opaque.delta_rule_gates(a, b, A_log, dt_bias, allow_neg_eigval)
+
+    if a.is_cuda and is_kernel_allowed(Kernel.gated_delta_rule):
+        result = host().gates(raw_stream(a.get_device()), a, b, A_log, dt_bias, 2.0 if allow_neg_eigval else 1.0)
+        if result is not None:
+            return result
 
     def formula(a, b, A_log, dt_bias):
         return gates_formula(a, b, A_log, dt_bias, allow_neg_eigval)
@@ -175,6 +181,11 @@ def gated_rmsnorm(
         from . import _opaque
 
         return _opaque.gated_rmsnorm(o, gate, weight, eps)
+
+    if o.is_cuda and is_kernel_allowed(Kernel.gated_delta_rule):
+        result = host().norm(raw_stream(o.get_device()), o, gate, weight, eps_value)
+        if result is not None:
+            return result
 
     def formula(o, gate, weight):
         return gated_rmsnorm_formula(o, gate, weight, eps_value)

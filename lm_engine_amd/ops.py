@@ -31,6 +31,7 @@ from collections import OrderedDict
 import torch
 
 from . import _lib
+from ._host import host, raw_stream
 from .backward import gated_delta_rule_backward
 from .kernels import Kernel, is_kernel_allowed
 
@@ -150,6 +151,7 @@ _WORKSPACES_LOCK = threading.Lock()
 # (gdn_args::error_word).  The host reads it without synchronising, before every chunked forward on that device: a
 # failure of an earlier call surfaces at the next one, the way asynchronous device errors do.
 _ERROR_WORDS: dict[int, torch.Tensor] = {}
+_ERROR_PEEKS: dict[int, ctypes.c_int32] = {}  # the same words, for a look that costs no tensor operation
 
 
 def release_workspaces() -> None:
@@ -162,15 +164,21 @@ def _error_word(device) -> torch.Tensor:
     word = _ERROR_WORDS.get(device.index)
     if word is None:
         word = torch.zeros(1, dtype=torch.int32).pin_memory()
+        _ERROR_PEEKS[device.index] = ctypes.c_int32.from_address(word.data_ptr())
         _ERROR_WORDS[device.index] = word
     return word
+
+
+def _forward_failed(device_index) -> bool:
+    peek = _ERROR_PEEKS.get(device_index)
+    return peek is not None and peek.value != 0
 
 
 def _raise_if_forward_failed(device) -> torch.Tensor:
     """The error word of ``device``; raises when an earlier one-launch forward on it reported a time-out (the kept
     workspaces of that device are dropped: their ready flags are in no defined state)."""
     word = _error_word(device)
-    if int(word[0]) != 0:
+    if _forward_failed(device.index):
         word.zero_()
         with _WORKSPACES_LOCK:
             for key in [k for k in _WORKSPACES if k[0] == device.index]:
@@ -198,6 +206,22 @@ def _kept_workspace(device, stream_handle, dims, nbytes, header_bytes):
         ):
             _WORKSPACES.popitem(last=False)
     return key, workspace
+
+
+def layer_step_workspace(device_index, stream_handle, pairs, V):
+    """``(tensor, tickets, scratch)`` for one ``gdn_layer_step`` on that stream: the tensor and the addresses of its two
+    parts, the tickets zero.  Kept like the forward's workspaces (every step leaves the tickets zero), for the next power of two
+    of ``pairs`` = sequences x heads, so that a batch that grows and shrinks finds its workspace again."""
+    capacity = 1 << max(8, (pairs - 1).bit_length())
+    nbytes, header = capacity * 4 * (1 + V), capacity * 4
+    device = torch.device("cuda", device_index)
+    if torch.cuda.is_current_stream_capturing():  # memory of the graph's own
+        workspace = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        workspace[:header].zero_()
+    else:
+        _, workspace = _kept_workspace(device, stream_handle, ("layer step", capacity, V), nbytes, header)
+    address = workspace.data_ptr()
+    return workspace, address, address + header
 
 
 def _drop_workspace(key) -> None:
@@ -633,6 +657,15 @@ def _dispatch(mode, q, k, v, g, beta, scale, initial_state, output_final_state, 
 
         return _opaque.gated_delta_rule(mode, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens,
                                         l2norm, inplace_state, left_padded)  # fmt: skip
+    if q.is_cuda and is_kernel_allowed(Kernel.gated_delta_rule):
+        device_index = q.get_device()
+        if mode != "chunk" or not _forward_failed(device_index):
+            flags = ((_lib.GDN_FLAG_L2NORM if l2norm else 0) | (_lib.GDN_FLAG_LEFT_PADDED if left_padded else 0)
+                     | (_lib.GDN_FLAG_FUSED_LAUNCH if is_kernel_allowed(Kernel.gated_delta_rule_fused_launch) else 0))  # fmt: skip
+            result = host().delta_rule(raw_stream(device_index), mode == "chunk", q, k, v, g, beta, scale, initial_state,
+                                       output_final_state, cu_seqlens, flags, inplace_state)  # fmt: skip
+            if result is not None:
+                return result
     tensors = (q, k, v, g, beta, initial_state)
     if torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in tensors):
         return _GatedDeltaRule.apply(mode, scale, output_final_state, l2norm, inplace_state, left_padded, q, k, v, g,

@@ -123,3 +123,69 @@ def test_left_padded_batch_with_attention_mask_equals_unpadded_runs(S):
         assert rel_l2(out[b : b + 1, S - n :], o_b) <= 1e-2
         assert rel_l2(h[b : b + 1], h_b) <= 1e-2
         assert torch.equal(cs[b : b + 1], cs_b)
+
+
+def _step_operands(B, HK, HV, DK, DV, dtype, seed):
+    qkv, ab, params = _layer_inputs(B, 1, HK, HV, DK, DV, seed=seed)
+    g = torch.Generator().manual_seed(seed + 1)
+    C = qkv.size(-1)
+    cast = lambda x: x.to(dtype).cuda()  # noqa: E731
+    cache = (cast(torch.randn(B, C, 3, generator=g)), (0.1 * torch.randn(B, HV, DK, DV, generator=g)).cuda())
+    keep = ("A_log", "dt_bias")  # fp32 parameters
+    return cast(qkv), cast(ab), {n: (x.cuda() if n in keep else cast(x)) for n, x in params.items()}, cache
+
+
+def _mix_step(qkv, ab, p, HK, HV, DK, DV, cache, gate=True, neg=True):
+    a, b, z = ab[..., :HV], ab[..., HV : 2 * HV], ab[..., 2 * HV :]
+    return lm_engine_amd.gated_deltanet_mixing(
+        qkv, a, b, z if gate else None, p["conv_weight"], p["conv_bias"], p["A_log"], p["dt_bias"], p["norm_weight"] if gate else None,
+        1e-5, HK, HV, DK, DV, cache=cache, allow_neg_eigval=neg)  # fmt: skip
+
+
+# one tile per head (V = 32, 64, 128), tiles of 32, 64 and 128 columns that share a norm through tickets, shared heads of
+# q and k, a projection whose gate slice starts off every 16-byte boundary (HV = 1, 2, 3), first token (no state yet)
+@pytest.mark.parametrize("dtype", [BF16, torch.float32])
+@pytest.mark.parametrize("B, HK, HV, DK, DV", [(1, 4, 4, 64, 32), (3, 2, 4, 128, 64), (5, 1, 3, 256, 128), (2, 2, 2, 128, 96),
+                                               (2, 2, 2, 256, 512), (3, 1, 2, 64, 192), (70, 2, 2, 128, 256)])  # fmt: skip
+def test_one_launch_step_matches_the_chain_of_kernels(B, HK, HV, DK, DV, dtype, monkeypatch):
+    from lm_engine_amd import layer
+    from lm_engine_amd._host import host
+
+    qkv, ab, p, cache = _step_operands(B, HK, HV, DK, DV, dtype, seed=B + DV)
+    print(f"case: layer step B={B} heads {HK}/{HV} dims {DK}/{DV} {dtype}", flush=True)
+
+    class WithoutTheStep:
+        def __getattr__(self, name):
+            return (lambda *args: None) if name == "layer_step" else getattr(host(), name)
+
+    for gate, start in ((True, cache), (False, cache), (True, (None, None))):
+        chained = {}
+        for name in ("step", "chain"):
+            with monkeypatch.context() as m:
+                if name == "chain":
+                    m.setattr(layer, "host", lambda: WithoutTheStep())
+                out, c1 = _mix_step(qkv, ab, p, HK, HV, DK, DV, start, gate=gate)
+                out2, c2 = _mix_step(qkv, ab, p, HK, HV, DK, DV, c1, gate=gate)  # on the state the first one left
+                chained[name] = (out, *c1, out2, *c2)
+        for name, x, y in zip(("out", "conv", "h", "out2", "conv2", "h2"), chained["step"], chained["chain"]):
+            if name.startswith("out"):  # the norm adds its V squares up in another order: at most an ulp of the result
+                assert rel_l2(x, y) <= (1e-3 if dtype == BF16 else 1e-6), (name, rel_l2(x, y))
+            else:
+                assert torch.equal(x, y), name
+
+
+def test_one_launch_step_under_graph_capture():
+    HK, HV, DK, DV = 2, 2, 128, 256  # several workgroups per head: tickets in memory of the graph's own
+    qkv, ab, p, cache = _step_operands(5, HK, HV, DK, DV, BF16, seed=9)
+    with torch.no_grad():
+        _mix_step(qkv, ab, p, HK, HV, DK, DV, cache)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out, (conv, h) = _mix_step(qkv, ab, p, HK, HV, DK, DV, cache)
+        gen = torch.Generator().manual_seed(3)
+        for _ in range(4):
+            qkv.copy_(torch.randn(qkv.shape, generator=gen).to(BF16))
+            want, (conv_want, h_want) = _mix_step(qkv, ab, p, HK, HV, DK, DV, cache)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want) and torch.equal(conv, conv_want) and torch.equal(h, h_want)
