@@ -17,7 +17,8 @@
 namespace gdn {
 
 constexpr int CONV_THREADS = 256;
-constexpr int CONV_TOKENS = 16;  // tokens per thread (measured: 16 beats 32, 64, 128; more workgroups in flight)
+constexpr int CONV_TOKENS = 16;  // tokens per thread of a large batch (measured: 16 beats 32, 64, 128; more workgroups in flight)
+constexpr int CONV_TOKENS_SHORT = 4;  // and of one whose waves would leave compute units idle (launch_conv)
 
 struct ConvParams {
     const void* x;
@@ -59,19 +60,20 @@ __device__ __forceinline__ void load_contiguous(const void* base, int64_t first,
     }
 }
 
-template <typename T, typename WT, int KS, bool SILU>
+template <typename T, typename WT, int KS, bool SILU, int TOKENS>
 __global__ __launch_bounds__(CONV_THREADS) void causal_conv1d_kernel(const ConvParams p) {
     constexpr int VEC = ConvVec<T>::N;
     typedef typename ConvVec<T>::type vec_t;
 
-    // a workgroup covers 64 channel vectors x (4 waves x CONV_TOKENS tokens): the halo rows of a wave are the
+    // a workgroup covers 64 channel vectors x (4 waves x TOKENS tokens): the halo rows of a wave are the
     // last rows of the wave before it, read on the same CU at about the same time
     const int c0 = (blockIdx.x * WAVE + threadIdx.x % WAVE) * VEC;
     if (c0 >= p.C) return;
     const int b = blockIdx.z;
-    const int s_begin = (blockIdx.y * (CONV_THREADS / WAVE) + threadIdx.x / WAVE) * CONV_TOKENS;
+    // (the same token in every lane of a wave: the mask comes in with scalar loads)
+    const int s_begin = (blockIdx.y * (CONV_THREADS / WAVE) + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE)) * TOKENS;
     if (s_begin >= p.S) return;
-    const int s_end = min(s_begin + CONV_TOKENS, p.S);
+    const int s_end = min(s_begin + TOKENS, p.S);
 
     const T* xb = reinterpret_cast<const T*>(p.x) + (int64_t)b * p.x_stride_b + c0;
     T* yb = reinterpret_cast<T*>(p.y) + (int64_t)b * p.y_stride_b + c0;
@@ -122,7 +124,7 @@ __global__ __launch_bounds__(CONV_THREADS) void causal_conv1d_kernel(const ConvP
     // cache; walked the same way, the second reader comes a whole walk later and fetches them from memory
     // again (measured: 19 % more bytes fetched than the input holds, 5 % this way; the kernel time did not
     // change, it streams at the rate of a plain copy either way).
-    const bool downward = ((s_begin / CONV_TOKENS) & 1) == 0;
+    const bool downward = ((s_begin / TOKENS) & 1) == 0;
     float hist[KS - 1][VEC];
     if (!downward) {
 #pragma unroll
@@ -177,20 +179,31 @@ __global__ __launch_bounds__(CONV_THREADS) void causal_conv1d_kernel(const ConvP
     }
 }
 
-template <typename T, typename WT, int KS>
-static void launch_conv_ks(const ConvParams& p, bool silu, dim3 grid, hipStream_t stream) {
-    if (silu) hipLaunchKernelGGL((causal_conv1d_kernel<T, WT, KS, true>), grid, dim3(CONV_THREADS), 0, stream, p);
-    else hipLaunchKernelGGL((causal_conv1d_kernel<T, WT, KS, false>), grid, dim3(CONV_THREADS), 0, stream, p);
+template <typename T, typename WT, int KS, int TOKENS>
+static void launch_conv_ks(const ConvParams& p, bool silu, hipStream_t stream) {
+    constexpr int SPAN = (CONV_THREADS / WAVE) * TOKENS;  // tokens per workgroup
+    const dim3 grid((p.C / ConvVec<T>::N + WAVE - 1) / WAVE, (p.S + SPAN - 1) / SPAN, p.B);
+    if (silu) hipLaunchKernelGGL((causal_conv1d_kernel<T, WT, KS, true, TOKENS>), grid, dim3(CONV_THREADS), 0, stream, p);
+    else hipLaunchKernelGGL((causal_conv1d_kernel<T, WT, KS, false, TOKENS>), grid, dim3(CONV_THREADS), 0, stream, p);
 }
 
 template <typename T, typename WT>
 static int launch_conv(const ConvParams& p, int kernel_size, bool silu, hipStream_t stream) {
-    const int vecs = p.C / ConvVec<T>::N;
-    constexpr int SPAN = (CONV_THREADS / WAVE) * CONV_TOKENS;  // tokens per workgroup
-    const dim3 grid((vecs + WAVE - 1) / WAVE, (p.S + SPAN - 1) / SPAN, p.B);
-    if (kernel_size == 2) launch_conv_ks<T, WT, 2>(p, silu, grid, stream);
-    else if (kernel_size == 3) launch_conv_ks<T, WT, 3>(p, silu, grid, stream);
-    else launch_conv_ks<T, WT, 4>(p, silu, grid, stream);
+    const int64_t groups = (p.C / ConvVec<T>::N + WAVE - 1) / WAVE;
+    const int64_t waves = groups * ((p.S + CONV_TOKENS - 1) / CONV_TOKENS) * p.B;
+    // Under 2048 waves (8 per compute unit) a walk of 16 tokens is one latency after another with little beside it: a
+    // prompt of 777 tokens x 2048 channels has 196 such waves and the layer's prefill takes 56.7 us with 16 tokens a thread,
+    // 51.8 with 4.  Above, the halo of 3 rows per block counts: 8 x 4096 x 2048 has 8192 waves, its layer's training step
+    // 1354 us with 16 tokens, 1363 with 4.
+    if (waves < 2048) {
+        if (kernel_size == 2) launch_conv_ks<T, WT, 2, CONV_TOKENS_SHORT>(p, silu, stream);
+        else if (kernel_size == 3) launch_conv_ks<T, WT, 3, CONV_TOKENS_SHORT>(p, silu, stream);
+        else launch_conv_ks<T, WT, 4, CONV_TOKENS_SHORT>(p, silu, stream);
+    } else {
+        if (kernel_size == 2) launch_conv_ks<T, WT, 2, CONV_TOKENS>(p, silu, stream);
+        else if (kernel_size == 3) launch_conv_ks<T, WT, 3, CONV_TOKENS>(p, silu, stream);
+        else launch_conv_ks<T, WT, 4, CONV_TOKENS>(p, silu, stream);
+    }
     return (int)hipGetLastError();
 }
 

@@ -136,3 +136,16 @@ def test_rejected_arguments():
         lm_engine_amd.depthwise_causal_convolution(torch.randn(2, 8, 18, device="cuda"), torch.randn(18, 1, 4, device="cuda"))
     with pytest.raises(ValueError):
         lm_engine_amd.depthwise_causal_convolution(x.cpu(), w.cpu())
+
+
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("masked", [False, True])
+def test_long_walks_match_short_ones(dtype, masked):
+    """A batch that fills the device takes 16 tokens a thread, its rows one by one take 4: the same bits, the oracle's values."""
+    x, w, b, st, m = _inputs(8, 4099, 64, 4, dtype, seed=5, state=True, mask=masked)
+    y, s = _check(x, w, b, st, m, "silu", "long walks")
+    for row in (0, 7):
+        xr = x[row : row + 1] if m is None else x[row : row + 1] * m[row : row + 1, :, None]
+        y1, s1 = lm_engine_amd.depthwise_causal_convolution(xr.cuda(), w.cuda(), b.cuda(), st[row : row + 1].cuda(), None, output_state=True)
+        first = 0 if m is None else int((m[row] == 0).sum())
+        assert torch.equal(y1[0, first:].cpu().to(F64), y[row, first:]) and torch.equal(s1[0].cpu().to(F64), s[row])
