@@ -483,7 +483,7 @@ int gdn_gates_bwd(const gdn_gate_bwd_args *args, void *stream);
  * lm_engine/modeling_utils/normalization.py:69-124: x / sqrt(mean(x^2) + eps) * weight.
  * o, y: [tokens, H, V] with element strides *_stride_t between tokens; gate: same shape with
  * gate_stride_t (a slice of a projection), or NULL (no gating); weight: [V] in w_dtype or NULL.
- * V a multiple of 8, at most 512; 16-byte aligned rows.
+ * V a multiple of 8, at most 512; 16-byte aligned rows of o and y, 4-byte aligned rows of gate.
  */
 typedef struct gdn_norm_args {
     const void *o;

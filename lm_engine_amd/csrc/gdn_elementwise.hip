@@ -101,6 +101,20 @@ __device__ __forceinline__ void load8(const bf16_t* p, float (&x)[8]) {
 #pragma unroll
     for (int e = 0; e < 8; e++) x[e] = (float)v[e];
 }
+// the same from rows that only start on a 4-byte boundary: still one 16-byte load for bf16, which the hardware takes at
+// any multiple of 4
+__device__ __forceinline__ void load8_dwords(const bf16_t* p, float (&x)[8]) {
+    typedef bf16x8 __attribute__((aligned(4))) bf16x8_dwords;
+    const bf16x8 v = *reinterpret_cast<const bf16x8_dwords*>(p);
+#pragma unroll
+    for (int e = 0; e < 8; e++) x[e] = (float)v[e];
+}
+__device__ __forceinline__ void load8_dwords(const float* p, float (&x)[8]) {
+    typedef f32x4 __attribute__((aligned(4))) f32x4_dwords;
+    const f32x4 a = *reinterpret_cast<const f32x4_dwords*>(p), b = *reinterpret_cast<const f32x4_dwords*>(p + 4);
+#pragma unroll
+    for (int e = 0; e < 4; e++) x[e] = a[e], x[4 + e] = b[e];
+}
 __device__ __forceinline__ void load8(const float* p, float (&x)[8]) {
     const f32x4 a = *reinterpret_cast<const f32x4*>(p), b = *reinterpret_cast<const f32x4*>(p + 4);
 #pragma unroll
@@ -140,7 +154,9 @@ struct NormParams {
     float eps;
 };
 
-// LPR lanes per row, 8 consecutive columns per lane (16-byte accesses for bf16, 2 x 16 for fp32)
+// LPR lanes per row, 8 consecutive columns per lane (16-byte accesses for bf16, 2 x 16 for fp32).  The gate is a slice of a
+// projection that starts behind 2 H scalars per row, so its rows need only a 4-byte boundary (at 2 heads they start 8 bytes
+// past a 16-byte one; copying them first took 28 us at 8 x 4096 x 2 x 512, in the forward and again in the backward).
 template <typename T, typename WT, int LPR>
 __global__ __launch_bounds__(256) void gated_rmsnorm_kernel(const NormParams p) {
     constexpr int ROWS_PER_BLOCK = 256 / LPR;
@@ -158,7 +174,7 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_kernel(const NormParams p) 
         load8(reinterpret_cast<const T*>(p.o) + t * p.o_stride_t + (int64_t)h * p.V + c, x);
         if (p.gate != nullptr) {
             float g[8];
-            load8(reinterpret_cast<const T*>(p.gate) + t * p.gate_stride_t + (int64_t)h * p.V + c, g);
+            load8_dwords(reinterpret_cast<const T*>(p.gate) + t * p.gate_stride_t + (int64_t)h * p.V + c, g);
 #pragma unroll
             for (int e = 0; e < 8; e++) x[e] *= g[e] * __builtin_amdgcn_rcpf(1.f + __expf(-g[e]));
         }
@@ -233,7 +249,7 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_bwd_kernel(const NormBwdPar
         if (live) {
             load8(reinterpret_cast<const T*>(p.o) + t * p.o_stride_t + (int64_t)h * p.V + c, o);
             load8(reinterpret_cast<const T*>(p.dy) + row * p.V + c, dy);
-            if (p.gate != nullptr) load8(reinterpret_cast<const T*>(p.gate) + t * p.gate_stride_t + (int64_t)h * p.V + c, g);
+            if (p.gate != nullptr) load8_dwords(reinterpret_cast<const T*>(p.gate) + t * p.gate_stride_t + (int64_t)h * p.V + c, g);
         }
         float ss = 0.f, dot = 0.f;
 #pragma unroll
@@ -339,8 +355,8 @@ extern "C" int gdn_gated_rmsnorm_fwd(const gdn_norm_args* a, void* stream) {
     const int64_t row_elems = (int64_t)a->H * a->V;
     if (a->o_stride_t < row_elems || a->y_stride_t < row_elems || (a->gate && a->gate_stride_t < row_elems)) return GDN_ERR_SHAPE;
     const size_t esz = a->dtype == GDN_BF16 ? 2 : 4;
-    if (!aligned_to(a->o, 16) || !aligned_to(a->y, 16) || (a->gate && !aligned_to(a->gate, 16)) || (a->weight && !aligned_to(a->weight, 16))) return GDN_ERR_ALIGN;
-    if ((a->o_stride_t * esz) % 16 || (a->y_stride_t * esz) % 16 || (a->gate && (a->gate_stride_t * esz) % 16)) return GDN_ERR_ALIGN;
+    if (!aligned_to(a->o, 16) || !aligned_to(a->y, 16) || (a->gate && !aligned_to(a->gate, 4)) || (a->weight && !aligned_to(a->weight, 16))) return GDN_ERR_ALIGN;
+    if ((a->o_stride_t * esz) % 16 || (a->y_stride_t * esz) % 16 || (a->gate && (a->gate_stride_t * esz) % 4)) return GDN_ERR_ALIGN;
     const int64_t rows = a->tokens * (int64_t)a->H;
     if (rows / 4 > 0x7fffffff) return GDN_ERR_UNSUPPORTED;
     gdn::NormParams p;
@@ -363,10 +379,10 @@ extern "C" int gdn_gated_rmsnorm_bwd(const gdn_norm_bwd_args* a, void* stream) {
     const int64_t row_elems = (int64_t)a->H * a->V;
     if (a->o_stride_t < row_elems || (a->gate && a->gate_stride_t < row_elems)) return GDN_ERR_SHAPE;
     const size_t esz = a->dtype == GDN_BF16 ? 2 : 4;
-    const void* ptrs[] = {a->o, a->dy, a->d_o, a->gate, a->d_gate, a->weight};
+    const void* ptrs[] = {a->o, a->dy, a->d_o, a->d_gate, a->weight};
     for (const void* x : ptrs)
         if (x != nullptr && !aligned_to(x, 16)) return GDN_ERR_ALIGN;
-    if ((a->o_stride_t * esz) % 16 || (a->gate && (a->gate_stride_t * esz) % 16)) return GDN_ERR_ALIGN;
+    if ((a->o_stride_t * esz) % 16 || (a->gate && (!aligned_to(a->gate, 4) || (a->gate_stride_t * esz) % 4))) return GDN_ERR_ALIGN;
     gdn::NormBwdParams p;
     p.o = a->o, p.gate = a->gate, p.weight = a->weight, p.dy = a->dy, p.d_o = a->d_o, p.d_gate = a->d_gate;
     p.dw_part = a->dweight_partial;

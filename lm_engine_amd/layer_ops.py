@@ -257,8 +257,8 @@ def _norm_operands(o, gate):
         if gate.shape[-2:] == (H, V) and gate.dim() == o.dim():
             gate = gate.flatten(-2) if gate.stride(-2) == V and gate.stride(-1) == 1 else gate.contiguous().flatten(-2)
         g2, g_stride = _token_rows(gate, H * V, "gate")
-        if g2.data_ptr() % 16 != 0 or (g_stride * g2.element_size()) % 16 != 0:
-            # a slice that starts off a 16-byte boundary (e.g. behind 2 * H gate scalars with H = 2) is compacted
+        if g2.data_ptr() % 4 != 0 or (g_stride * g2.element_size()) % 4 != 0:
+            # the kernels read the gate's rows from any 4-byte boundary (a slice behind 2 * H scalars per row has one)
             g2 = g2.contiguous()
             g_stride = H * V
     return o2, o_stride, g2, g_stride, H, V

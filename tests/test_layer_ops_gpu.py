@@ -74,6 +74,28 @@ def test_gate_slice_off_a_16_byte_boundary():
     assert rel_l2(y, y_ref) <= 1e-2
 
 
+@pytest.mark.parametrize("dtype,offset", [(BF16, 2), (BF16, 4), (BF16, 6), (BF16, 7), (F32, 1), (F32, 2), (F32, 3)])
+@pytest.mark.parametrize("V", [64, 504])
+def test_gate_rows_from_any_boundary_match_a_compact_gate(dtype, offset, V):
+    """Gate rows that start 4, 8 or 12 bytes past a 16-byte boundary (read as they lie) or on an odd element (copied first):
+    the same bits as from a compact copy, forward and backward."""
+    B, T, H = 2, 19, 3
+    gen = torch.Generator().manual_seed(offset)
+    o = torch.randn(B, T, H, V, generator=gen).to(dtype).cuda().requires_grad_(True)
+    w = (1 + 0.1 * torch.randn(V, generator=gen)).to(dtype).cuda().requires_grad_(True)
+    proj = torch.randn(B, T, offset + H * V, generator=gen).to(dtype).cuda()
+    dy = torch.randn(B, T, H, V, generator=gen).to(dtype).cuda()
+    results = []
+    for gate in (proj[..., offset:], proj[..., offset:].contiguous()):
+        with torch.no_grad():
+            y = lm_engine_amd.gated_rmsnorm(o, gate, w, 1e-5)
+        gate = gate.detach().requires_grad_(True)
+        under_grad = lm_engine_amd.gated_rmsnorm(o, gate, w, 1e-5)
+        results.append((y, under_grad, *torch.autograd.grad(under_grad, (o, gate, w), dy)))
+    for got, want in zip(*results):
+        assert torch.equal(got, want)
+
+
 def test_rejected_arguments():
     o = torch.randn(2, 3, 4, 20, device="cuda")
     with pytest.raises(ValueError):
