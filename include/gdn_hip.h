@@ -483,8 +483,10 @@ int gdn_gates_bwd(const gdn_gate_bwd_args *args, void *stream);
  * lm_engine/modeling_utils/normalization.py:69-124: x / sqrt(mean(x^2) + eps) * weight.
  * o, y: [tokens, H, V] with element strides *_stride_t between tokens; gate: same shape with
  * gate_stride_t (a slice of a projection), or NULL (no gating); weight: [V] in w_dtype or NULL.
- * V a multiple of 8, at most 512; 16-byte aligned rows of o and y, 4-byte aligned rows of gate.
+ * V a multiple of 8, at most 512; 16-byte aligned rows, those of gate on any 4-byte boundary with GDN_NORM_GATE_DWORDS in
+ * w_dtype (a slice behind 2 H scalars per row of a projection).
  */
+#define GDN_NORM_GATE_DWORDS 0x100
 typedef struct gdn_norm_args {
     const void *o;
     const void *gate;
@@ -494,7 +496,7 @@ typedef struct gdn_norm_args {
     int64_t tokens;
     int32_t H, V;
     int32_t dtype;   /* gdn_dtype of o, gate, y */
-    int32_t w_dtype; /* gdn_dtype of weight */
+    int32_t w_dtype; /* gdn_dtype of weight, | GDN_NORM_GATE_DWORDS */
     float eps;
     int32_t reserved;
 } gdn_norm_args;
@@ -506,7 +508,7 @@ int gdn_gated_rmsnorm_fwd(const gdn_norm_args *args, void *stream);
  * module.py:238-242, when the layer trains): given dy [tokens, H, V] (contiguous) it writes d_o and, with a
  * gate, d_gate (both [tokens, H, V] contiguous, dtype of o), and the partial sums of the gradient of weight
  * left by each of its `partial_blocks` workgroups, dweight_partial [partial_blocks][V] fp32, which the
- * caller adds up (also when weight is NULL).
+ * caller adds up (also when weight is NULL).  w_dtype as in gdn_norm_args.
  */
 typedef struct gdn_norm_bwd_args {
     const void *o, *gate, *weight, *dy;

@@ -24,6 +24,8 @@ GDN_FLAG_RECORDS_16X16 = 32
 GDN_FLAG_DEBUG_NO_PRODUCERS = 64
 GDN_FLAG_SKIP_EMPTY_CHUNKS = 128
 
+GDN_NORM_GATE_DWORDS = 0x100
+
 GDN_ERR_TIMEOUT = -7
 
 GDN_NOALLOC_SCRATCH_BYTES = 64 << 20  # built-in workspace of gdn_chunk_fwd_noalloc

@@ -311,6 +311,11 @@ static int launch_norm_bwd(const NormBwdParams& p, int blocks, hipStream_t strea
 
 namespace {
 inline bool aligned_to(const void* p, size_t a) { return (reinterpret_cast<uintptr_t>(p) % a) == 0; }
+// gate rows: on 16-byte boundaries, or on 4-byte ones where the caller says so (GDN_NORM_GATE_DWORDS in w_dtype)
+inline bool gate_aligned(const void* gate, int64_t stride_bytes, int w_dtype) {
+    const int64_t a = (w_dtype & GDN_NORM_GATE_DWORDS) ? 4 : 16;
+    return gate == nullptr || (aligned_to(gate, (size_t)a) && stride_bytes % a == 0);
+}
 }  // namespace
 
 extern "C" int gdn_gates_fwd(const gdn_gate_args* a, void* stream) {
@@ -351,12 +356,13 @@ extern "C" int gdn_gated_rmsnorm_fwd(const gdn_norm_args* a, void* stream) {
     if (a->tokens <= 0 || a->H <= 0 || a->V <= 0) return GDN_ERR_SHAPE;
     if (a->V % 8 != 0 || a->V > 512) return GDN_ERR_UNSUPPORTED;
     if (a->dtype != GDN_BF16 && a->dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
-    if (a->weight && a->w_dtype != GDN_BF16 && a->w_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
+    const int w_dtype = a->w_dtype & ~GDN_NORM_GATE_DWORDS;
+    if (a->weight && w_dtype != GDN_BF16 && w_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
     const int64_t row_elems = (int64_t)a->H * a->V;
     if (a->o_stride_t < row_elems || a->y_stride_t < row_elems || (a->gate && a->gate_stride_t < row_elems)) return GDN_ERR_SHAPE;
     const size_t esz = a->dtype == GDN_BF16 ? 2 : 4;
-    if (!aligned_to(a->o, 16) || !aligned_to(a->y, 16) || (a->gate && !aligned_to(a->gate, 4)) || (a->weight && !aligned_to(a->weight, 16))) return GDN_ERR_ALIGN;
-    if ((a->o_stride_t * esz) % 16 || (a->y_stride_t * esz) % 16 || (a->gate && (a->gate_stride_t * esz) % 4)) return GDN_ERR_ALIGN;
+    if (!aligned_to(a->o, 16) || !aligned_to(a->y, 16) || (a->weight && !aligned_to(a->weight, 16))) return GDN_ERR_ALIGN;
+    if ((a->o_stride_t * esz) % 16 || (a->y_stride_t * esz) % 16 || !gate_aligned(a->gate, a->gate_stride_t * (int64_t)esz, a->w_dtype)) return GDN_ERR_ALIGN;
     const int64_t rows = a->tokens * (int64_t)a->H;
     if (rows / 4 > 0x7fffffff) return GDN_ERR_UNSUPPORTED;
     gdn::NormParams p;
@@ -364,7 +370,7 @@ extern "C" int gdn_gated_rmsnorm_fwd(const gdn_norm_args* a, void* stream) {
     p.o_stride_t = a->o_stride_t, p.gate_stride_t = a->gate_stride_t, p.y_stride_t = a->y_stride_t;
     p.rows = rows, p.H = a->H, p.V = a->V, p.eps = a->eps;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const bool wf32 = a->weight == nullptr || a->w_dtype == GDN_F32;
+    const bool wf32 = a->weight == nullptr || w_dtype == GDN_F32;
     if (a->dtype == GDN_BF16) return wf32 ? gdn::launch_norm<gdn::bf16_t, float>(p, st) : gdn::launch_norm<gdn::bf16_t, gdn::bf16_t>(p, st);
     return wf32 ? gdn::launch_norm<float, float>(p, st) : gdn::launch_norm<float, gdn::bf16_t>(p, st);
 }
@@ -375,21 +381,22 @@ extern "C" int gdn_gated_rmsnorm_bwd(const gdn_norm_bwd_args* a, void* stream) {
     if (a->tokens <= 0 || a->H <= 0 || a->V <= 0 || a->partial_blocks <= 0) return GDN_ERR_SHAPE;
     if (a->V % 8 != 0 || a->V > 512) return GDN_ERR_UNSUPPORTED;
     if (a->dtype != GDN_BF16 && a->dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
-    if (a->weight && a->w_dtype != GDN_BF16 && a->w_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
+    const int w_dtype = a->w_dtype & ~GDN_NORM_GATE_DWORDS;
+    if (a->weight && w_dtype != GDN_BF16 && w_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
     const int64_t row_elems = (int64_t)a->H * a->V;
     if (a->o_stride_t < row_elems || (a->gate && a->gate_stride_t < row_elems)) return GDN_ERR_SHAPE;
     const size_t esz = a->dtype == GDN_BF16 ? 2 : 4;
     const void* ptrs[] = {a->o, a->dy, a->d_o, a->d_gate, a->weight};
     for (const void* x : ptrs)
         if (x != nullptr && !aligned_to(x, 16)) return GDN_ERR_ALIGN;
-    if ((a->o_stride_t * esz) % 16 || (a->gate && (!aligned_to(a->gate, 4) || (a->gate_stride_t * esz) % 4))) return GDN_ERR_ALIGN;
+    if ((a->o_stride_t * esz) % 16 || !gate_aligned(a->gate, a->gate_stride_t * (int64_t)esz, a->w_dtype)) return GDN_ERR_ALIGN;
     gdn::NormBwdParams p;
     p.o = a->o, p.gate = a->gate, p.weight = a->weight, p.dy = a->dy, p.d_o = a->d_o, p.d_gate = a->d_gate;
     p.dw_part = a->dweight_partial;
     p.o_stride_t = a->o_stride_t, p.gate_stride_t = a->gate_stride_t;
     p.rows = a->tokens * (int64_t)a->H, p.H = a->H, p.V = a->V, p.eps = a->eps;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const bool wf32 = a->weight == nullptr || a->w_dtype == GDN_F32;
+    const bool wf32 = a->weight == nullptr || w_dtype == GDN_F32;
     if (a->dtype == GDN_BF16)
         return wf32 ? gdn::launch_norm_bwd<gdn::bf16_t, float>(p, a->partial_blocks, st)
                     : gdn::launch_norm_bwd<gdn::bf16_t, gdn::bf16_t>(p, a->partial_blocks, st);

@@ -274,6 +274,7 @@ PyObject* norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
             s.w_dtype = code_of(*weight);
             need(weight->dim() == 1 && weight->size(0) == V && weight->is_contiguous());
         }
+        s.w_dtype |= GDN_NORM_GATE_DWORDS;
         const at::Tensor y = fresh(o, o.sizes());
         s.o = ptr(o), s.gate = ptr(gate), s.weight = ptr(weight), s.y = ptr(y);
         s.o_stride_t = s.y_stride_t = H * V, s.H = size32(H), s.V = (int32_t)V, s.eps = (float)number(args[4]);

@@ -230,7 +230,7 @@ def _gated_rmsnorm_backward(o, gate, weight, eps, dy):
     args.weight = None if w is None else w.data_ptr()
     args.o_stride_t, args.gate_stride_t, args.tokens, args.H, args.V = o_stride, g_stride, tokens, H, V
     args.dtype = _dtype_code(o.dtype, "o")
-    args.w_dtype = _lib.GDN_F32 if w is None else _dtype_code(w.dtype, "weight")
+    args.w_dtype = (_lib.GDN_F32 if w is None else _dtype_code(w.dtype, "weight")) | _lib.GDN_NORM_GATE_DWORDS
     args.eps = float(torch.finfo(o.dtype).eps if eps is None else eps)
     args.partial_blocks = blocks
     lib = _lib.load_library()
@@ -278,7 +278,7 @@ def _gated_rmsnorm(o, gate, weight, eps):
     args.o_stride_t, args.gate_stride_t, args.y_stride_t = o_stride, g_stride, H * V
     args.tokens, args.H, args.V = o2.size(0), H, V
     args.dtype = _dtype_code(o.dtype, "o")
-    args.w_dtype = _lib.GDN_F32 if weight is None else _dtype_code(weight.dtype, "weight")
+    args.w_dtype = (_lib.GDN_F32 if weight is None else _dtype_code(weight.dtype, "weight")) | _lib.GDN_NORM_GATE_DWORDS
     args.eps = float(torch.finfo(o.dtype).eps if eps is None else eps)
     lib = _lib.load_library()
     with torch.cuda.device(o.device):
