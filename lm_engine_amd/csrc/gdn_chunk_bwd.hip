@@ -170,7 +170,12 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
     constexpr int NTW = NKT == 4 ? 2 : 1;
     static_assert(K == 64 || K == 128 || K == 256, "head dims");
     constexpr int SLAB = C * LDS64 * 2;        // bytes of a staged [64][64] matrix
-    constexpr int PHASE1 = 3 * SLAB + K * LDS64 * 2;        // dO | Y | V~ | states
+    // With two workgroups per CU and all saves bf16, dS1 has rows of its own beside S0 (the three phases then need the same
+    // LDS) and a slab is asked for in one go: what such a workgroup spends its time on is trips through memory, one
+    // after another - three per slab when dS1 waits for S0's place and V~'s rows for the store of dv, one this way
+    // (4 x 4096 tokens, 16 heads, K = V = 128, the whole backward and forward: 869 -> 800 us).
+    constexpr bool ONE_TRIP = SL && K <= 128;
+    constexpr int PHASE1 = 3 * SLAB + (ONE_TRIP ? 2 : 1) * K * LDS64 * 2;  // dO | Y | V~ | states (S0, then dS1) or S0 | dS1
     constexpr int PHASE2 = 3 * SLAB + 2 * C * LDK * 2;      // G | G^T | Hm + Hm^T | q | k
     // Phase 3 needs q^T and k^T as MFMA operands.  K = 256 (a CU to itself) reads them out of the row-major copies with
     // the transposing LDS load; with two workgroups per CU (K <= 128) that variant ran slower (more registers, spills)
@@ -184,6 +189,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
     bf16_t* const sY = sDO + C * LDS64;
     bf16_t* const sVN = sY + C * LDS64;
     bf16_t* const sST = sVN + C * LDS64;  // [K][LDS64]: S0, then dS1
+    bf16_t* const sS1 = ONE_TRIP ? sST + K * LDS64 : sST;
     bf16_t* const sG = reinterpret_cast<bf16_t*>(lds);
     bf16_t* const sGT = sG + C * LDS64;
     bf16_t* const sH = sGT + C * LDS64;
@@ -348,6 +354,51 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
             }
 #pragma unroll
             for (int i = 0; i < K / 32; i++) *reinterpret_cast<bf16x8*>(sST + (t / 8 + 32 * i) * LDS64 + 8 * p8) = nx_s0[i];
+        } else if constexpr (ONE_TRIP) {
+            const int p8 = t % 8;
+            const bf16_t* const vnew = reinterpret_cast<const bf16_t*>(vnb);
+            const bf16_t* const s0 = reinterpret_cast<const bf16_t*>(s0b);
+            bf16x8 vr[2], dr[2], yr[2], nr[2], sr[K / 32], er[K / 32];
+            float b[2];
+#pragma unroll
+            for (int it = 0; it < 2; it++) {
+                const int row = t / 8 + 32 * it;
+                dr[it] = *reinterpret_cast<const bf16x8*>(row_of(p.d_raw, p.d_stride_b, p.d_stride_t, p.d_stride_h, row) + v0 + 8 * p8);
+                yr[it] = *reinterpret_cast<const bf16x8*>(p.y_chunks + chunk * C * V + sliced_at(C - 1 - row, v0 + 8 * p8, C));
+                vr[it] = *reinterpret_cast<const bf16x8*>(row_of(p.v_raw, p.v_stride_b, p.v_stride_t, p.v_stride_h, row) + v0 + 8 * p8);
+                nr[it] = *reinterpret_cast<const bf16x8*>(vnew + sliced_at(row, v0 + 8 * p8, C));
+                b[it] = p.beta[chunk * C + row];
+            }
+#pragma unroll
+            for (int i = 0; i < K / 32; i++) sr[i] = *reinterpret_cast<const bf16x8*>(s0 + sliced_at(t / 8 + 32 * i, v0 + 8 * p8, K));
+#pragma unroll
+            for (int i = 0; i < K / 32; i++) er[i] = *reinterpret_cast<const bf16x8*>(ds1h + sliced_at(t / 8 + 32 * i, v0 + 8 * p8, K));
+            __builtin_amdgcn_sched_barrier(0);  // everything is on its way
+#pragma unroll
+            for (int it = 0; it < 2; it++) {
+                const int row = t / 8 + 32 * it;
+                const bool live = row < valid;
+                bf16x8 dv;
+                float acc = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    dv[e] = (bf16_t)((float)yr[it][e] * b[it]);
+                    acc += (float)yr[it][e] * (live ? (float)vr[it][e] : 0.f);
+                }
+                *reinterpret_cast<bf16x8*>(sDO + row * LDS64 + 8 * p8) = live ? dr[it] : zero8;
+                *reinterpret_cast<bf16x8*>(sY + row * LDS64 + 8 * p8) = yr[it];
+                *reinterpret_cast<bf16x8*>(sVN + row * LDS64 + 8 * p8) = live ? nr[it] : zero8;
+                if (live) *reinterpret_cast<bf16x8*>(p.dv_out + ((tok0 + row) * p.H + h) * V + v0 + 8 * p8) = dv;
+                yv[it] = acc;
+            }
+#pragma unroll
+            for (int i = 0; i < K / 32; i++) {
+                const int at = (t / 8 + 32 * i) * LDS64 + 8 * p8;
+                *reinterpret_cast<bf16x8*>(sST + at) = sr[i];
+                *reinterpret_cast<bf16x8*>(sS1 + at) = er[i];
+#pragma unroll
+                for (int e = 0; e < 8; e++) dot += (float)er[i][e] * (float)sr[i][e];
+            }
         } else {
             // v, dO and Y (token `row` is token 63 - row of mirror chunk A); dV = beta Y goes out right away
             const int p8 = t % 8;
@@ -461,13 +512,14 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
             }
         DP = mma_nt(sDO + 32 * (wave / 2) * LDS64, LDS64, sVN + 32 * (wave % 2) * LDS64, LDS64, VW, DP, l32, lh);
         DA = mma_nt(sY + 32 * (wave / 2) * LDS64, LDS64, sVN + 32 * (wave % 2) * LDS64, LDS64, VW, DA, l32, lh);
-        if constexpr (!PREFETCH) ask_ds1();
+        if constexpr (!PREFETCH && !ONE_TRIP) ask_ds1();
         LTICK(5);
-        __syncthreads();  // S0 has been read by every wave
+        if constexpr (!ONE_TRIP) __syncthreads();  // S0 has been read by every wave
         LTICK(6);
 
         // dS1 takes the place of S0; <dS1, S0> on the way (S0 as the bf16 the products used)
-        if constexpr (DS1H) {
+        if constexpr (ONE_TRIP) {  // (it lies beside it)
+        } else if constexpr (DS1H) {
 #pragma unroll
             for (int i = 0; i < K / 32; i++) {
                 bf16_t* const at = sST + (t / 8 + 32 * i) * LDS64 + 8 * (t % 8);
@@ -487,13 +539,13 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
             }
         }
         LTICK(7);
-        __syncthreads();
+        if constexpr (!ONE_TRIP) __syncthreads();
         LTICK(8);
 #pragma unroll
         for (int kh = 0; kh < KH; kh++)
 #pragma unroll
             for (int m = 0; m < NTW; m++)
-                dKdT[kh][m] = mma_nt(sST + 32 * (ktl + NKT * kh) * LDS64, LDS64, sVN + 32 * tt_of(m) * LDS64, LDS64, VW, dKdT[kh][m], l32, lh);
+                dKdT[kh][m] = mma_nt(sS1 + 32 * (ktl + NKT * kh) * LDS64, LDS64, sVN + 32 * tt_of(m) * LDS64, LDS64, VW, dKdT[kh][m], l32, lh);
         LTICK(9);
         __syncthreads();  // the staged slab is free
         LTICK(10);
