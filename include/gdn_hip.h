@@ -524,6 +524,21 @@ typedef struct gdn_norm_bwd_args {
 int gdn_gated_rmsnorm_bwd(const gdn_norm_bwd_args *args, void *stream);
 
 /*
+ * The sums over the first dim of the partial arrays that the backward kernels above leave, one launch for up to two of
+ * them: out[j][c] = sum over rows of partial[j][row][c], accumulated in fp32 in a fixed order, in out_dtype[j]
+ * (gdn_dtype).  partial[j] is [rows][cols[j]] fp32 contiguous.
+ */
+typedef struct gdn_column_sums_args {
+    const float *partial[2];
+    void *out[2];
+    int64_t cols[2];
+    int32_t out_dtype[2];
+    int32_t rows;
+    int32_t arrays; /* 1 or 2 */
+} gdn_column_sums_args;
+int gdn_column_sums(const gdn_column_sums_args *args, void *stream);
+
+/*
  * One decode step of the layer between its projections, in one launch: the convolution's one-token update
  * (depthwise_causal_convolution.py:199-231), the gates (module.py:179-183), the recurrence with l2-normalised q and k
  * (module.py:210-222) and the gated norm (module.py:238-242).  Results are those of gdn_causal_conv1d_fwd,

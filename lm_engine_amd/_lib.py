@@ -56,6 +56,7 @@ EXPORTED_SYMBOLS = (
     "gdn_gates_bwd",
     "gdn_gated_rmsnorm_fwd",
     "gdn_gated_rmsnorm_bwd",
+    "gdn_column_sums",
     "gdn_layer_step",
     "gdn_layer_step_tiles",
 )
@@ -134,6 +135,17 @@ class GdnNormBwdArgs(ctypes.Structure):
         + [(name, ctypes.c_int32) for name in ("H", "V", "dtype", "w_dtype")]
         + [("eps", ctypes.c_float), ("partial_blocks", ctypes.c_int32)]
     )  # fmt: skip
+
+
+class GdnColumnSumsArgs(ctypes.Structure):
+    _fields_ = [
+        ("partial", ctypes.c_void_p * 2),
+        ("out", ctypes.c_void_p * 2),
+        ("cols", ctypes.c_int64 * 2),
+        ("out_dtype", ctypes.c_int32 * 2),
+        ("rows", ctypes.c_int32),
+        ("arrays", ctypes.c_int32),
+    ]
 
 
 class GdnArgs(ctypes.Structure):
@@ -254,6 +266,8 @@ def load_library() -> ctypes.CDLL:
     lib.gdn_gates_fwd.restype = ctypes.c_int
     lib.gdn_gates_bwd.argtypes = [ctypes.POINTER(GdnGateBwdArgs), ctypes.c_void_p]
     lib.gdn_gates_bwd.restype = ctypes.c_int
+    lib.gdn_column_sums.argtypes = [ctypes.POINTER(GdnColumnSumsArgs), ctypes.c_void_p]
+    lib.gdn_column_sums.restype = ctypes.c_int
     lib.gdn_gated_rmsnorm_fwd.argtypes = [ctypes.POINTER(GdnNormArgs), ctypes.c_void_p]
     lib.gdn_gated_rmsnorm_fwd.restype = ctypes.c_int
 

@@ -27,6 +27,7 @@ from . import _lib
 from ._autograd import kernel_with_formula_backward
 from ._host import host, raw_stream
 from .kernels import Kernel, is_kernel_allowed
+from .layer_ops import column_sums
 
 
 _IN_KERNEL_ACTIVATIONS = {None: _lib.GDN_ACT_NONE, "silu": _lib.GDN_ACT_SILU, "swish": _lib.GDN_ACT_SILU}
@@ -173,8 +174,9 @@ def _convolution_backward(x, weight, bias, input_state, attention_mask, dy, acti
     with torch.cuda.device(x.device):
         stream = ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
         _lib.check_status(lib.gdn_causal_conv1d_bwd(ctypes.byref(a), stream), "gdn_causal_conv1d_bwd")
-    dweight = dw_part.sum(dim=0).to(weight.dtype).reshape(weight.shape)
-    dbias = None if bias is None else db_part.sum(dim=0).to(bias.dtype)
+        wanted = [(dw_part, weight.dtype)] + ([] if bias is None else [(db_part, bias.dtype)])
+        dweight, dbias = (*column_sums(lib, stream, *wanted), None)[:2]
+    dweight = dweight.reshape(weight.shape)
     dstate = None if dstate is None else dstate.to(input_state.dtype)
     return dx, dweight, dbias, dstate
 

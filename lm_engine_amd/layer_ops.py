@@ -50,6 +50,23 @@ def _token_rows(x: torch.Tensor, width: int, what: str) -> tuple[torch.Tensor, i
     return rows, rows.stride(0) if rows.size(0) > 1 else width
 
 
+def column_sums(lib, stream, *wanted):
+    """``gdn_column_sums``: for every ``(partial [rows, ...] fp32 contiguous, dtype)`` (one or two, the same ``rows``) the sum
+    over the first dim in that dtype.  Runs on the caller's current device and stream."""
+    if any(dtype not in (torch.bfloat16, torch.float32) for _, dtype in wanted):  # parameters of another type
+        return [partial.sum(dim=0).to(dtype) for partial, dtype in wanted]
+    args = _lib.GdnColumnSumsArgs()
+    results = []
+    for j, (partial, dtype) in enumerate(wanted):
+        result = torch.empty(partial.shape[1:], dtype=dtype, device=partial.device)
+        args.partial[j], args.out[j], args.cols[j] = partial.data_ptr(), result.data_ptr(), result.numel()
+        args.out_dtype[j] = _dtype_code(dtype, "gradient")
+        results.append(result)
+    args.rows, args.arrays = wanted[0][0].size(0), len(wanted)
+    _lib.check_status(lib.gdn_column_sums(ctypes.byref(args), stream), "gdn_column_sums")
+    return results
+
+
 def gates_formula(a, b, A_log, dt_bias, allow_neg_eigval):
     """The gates in torch operations: what their backward differentiates."""
     g = -torch.exp(A_log.float()) * torch.nn.functional.softplus(a.float() + dt_bias.float())
@@ -127,8 +144,9 @@ def _delta_rule_gates_backward(a, b, A_log, dt_bias, dg, dbeta, allow_neg_eigval
     with torch.cuda.device(dev):
         stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
         _lib.check_status(lib.gdn_gates_bwd(ctypes.byref(args), stream), "gdn_gates_bwd")
-    # two results that share no storage (an operator's outputs must not alias each other)
-    return da, db, parts[0].sum(dim=0).to(A_log.dtype), parts[1].sum(dim=0).to(dt_bias.dtype)
+        # two results that share no storage (an operator's outputs must not alias each other)
+        dA_log, ddt_bias = column_sums(lib, stream, (parts[0], A_log.dtype), (parts[1], dt_bias.dtype))
+    return da, db, dA_log, ddt_bias
 
 
 def _delta_rule_gates(a, b, A_log, dt_bias, allow_neg_eigval):
@@ -237,7 +255,7 @@ def _gated_rmsnorm_backward(o, gate, weight, eps, dy):
     with torch.cuda.device(o.device):
         stream = ctypes.c_void_p(torch.cuda.current_stream(o.device).cuda_stream)
         _lib.check_status(lib.gdn_gated_rmsnorm_bwd(ctypes.byref(args), stream), "gdn_gated_rmsnorm_bwd")
-    d_weight = None if weight is None else dw_part.sum(dim=0).to(weight.dtype)
+        d_weight = None if weight is None else column_sums(lib, stream, (dw_part, weight.dtype))[0]
     return d_o, (None if gate is None else d_gate.reshape(gate.shape)), d_weight
 
 

@@ -105,3 +105,21 @@ def test_rejected_arguments():
     a = torch.randn(2, 5, 4, device="cuda")
     with pytest.raises(ValueError):
         lm_engine_amd.delta_rule_gates(a, a, torch.zeros(3), torch.zeros(4))
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (63, 15), (64, 16), (65, 17), (2048, 512)])
+def test_column_sums(rows, cols):
+    """Two partial arrays of different widths in one launch, fp32 and bf16 results.  Each element is at most rows / 64 + 6
+    rounded additions deep; bf16 adds half a unit in its eighth bit."""
+    from lm_engine_amd import _lib
+    from lm_engine_amd.layer_ops import column_sums
+
+    gen = torch.Generator().manual_seed(rows + cols)
+    parts = [torch.randn(rows, n, generator=gen) for n in (cols, 3 * cols + 1)]
+    lib, stream = _lib.load_library(), torch.cuda.current_stream().cuda_stream
+    got = column_sums(lib, stream, (parts[0].cuda(), F32), (parts[1].cuda(), BF16))
+    for part, sums, unit in zip(parts, got, (0.0, 2.0**-8)):
+        want = part.double().sum(dim=0)
+        bound = part.abs().double().sum(dim=0) * (rows / 64 + 7) * 2.0**-24
+        assert sums.shape == want.shape
+        assert ((sums.double().cpu() - want).abs() <= bound + (want.abs() + bound) * unit).all()
