@@ -225,6 +225,8 @@ int gdn_recurrent_fwd(const gdn_args *args, void *stream);
  * of ITS entries whatever the row's length.  row_order (then only; NULL = as they lie): the rows in the order in which
  * their chains are dealt out to the XCDs and started, best longest first - a ragged batch takes as long as the XCD with
  * the most chunks.
+ * packed_records != 0 (records_given, packed cu_seqlens; GDN_ERR_VARLEN without it): args->workspace has the full layout of
+ * gdn_workspace_bytes for these sequences, its last part holds the records (gdn_chunk_bwd_prepare with records_fwd_slots).
  * mirror_reads: T / 64 must be even.  The twelve operand fragments of every odd chunk are read from the record of chunk 1 of the chain
  * (in the mirror problem they are the same for all odd chunks: T' = I, P = 0); an odd chunk's own record supplies its
  * row scales and e^{gamma_C} only.
@@ -241,7 +243,7 @@ typedef struct gdn_chunk_saves {
     int32_t no_output;
     int32_t mirror_reads;
     int32_t sliced;
-    int32_t reserved;
+    int32_t packed_records;
     const void *k_odd, *v_odd;
     int64_t k_odd_stride_b, k_odd_stride_t, k_odd_stride_h;
     int64_t v_odd_stride_b, v_odd_stride_t, v_odd_stride_h;
@@ -341,11 +343,14 @@ typedef struct gdn_chunk_bwd_prepare_args {
      * (>= ceil(max seq_len / 64)); T / 64 is read as NC when seq_start is NULL */
     const int32_t *seq_start, *seq_len;
     int32_t NC;
-    int32_t reserved;
-    /* optional (whole-chunk batches only: seq_start NULL): the records of the forward pass itself, [H][N * T/64] as
+    /* packed sequences (seq_start given) with records_fwd: its record slots per head, T/64 + N; 0 otherwise */
+    int32_t records_fwd_slots;
+    /* optional (whole-chunk batches, seq_start NULL, and packed sequences): the records of the forward pass itself, [H][N * T/64] as
      * gdn_chunk_fwd's prepare step writes them (fragment order as chosen by GDN_FLAG_RECORDS_16X16), for a forward
      * sweep through gdn_chunk_fwd_saving with records_given (q, k, v are then the caller's own tensors);
-     * records_fwd_bytes >= H * N * T/64 * 13312 */
+     * records_fwd_bytes >= H * N * T/64 * 13312.  For packed sequences they are [H][records_fwd_slots], a sequence's chunks
+     * behind those of the sequences before it: the last part of a gdn_chunk_fwd workspace of those sequences, for
+     * gdn_chunk_fwd_saving with packed_records. */
     void *records_fwd;
     uint64_t records_fwd_bytes;
 } gdn_chunk_bwd_prepare_args;

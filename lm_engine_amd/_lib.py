@@ -78,7 +78,7 @@ class GdnChunkSaves(ctypes.Structure):
         ("no_output", ctypes.c_int32),
         ("mirror_reads", ctypes.c_int32),
         ("sliced", ctypes.c_int32),
-        ("reserved", ctypes.c_int32),
+        ("packed_records", ctypes.c_int32),
         ("k_odd", ctypes.c_void_p),
         ("v_odd", ctypes.c_void_p),
         ("k_odd_stride_b", ctypes.c_int64),
@@ -113,7 +113,7 @@ class GdnChunkBwdPrepareArgs(ctypes.Structure):
         + [("scale", ctypes.c_float)]
         + [(name, ctypes.c_void_p) for name in ("gamma", "beta_packed", "rq", "rk", "k_mirror", "v_mirror", "records")]
         + [("records_bytes", ctypes.c_uint64), ("seq_start", ctypes.c_void_p), ("seq_len", ctypes.c_void_p),
-           ("NC", ctypes.c_int32), ("reserved", ctypes.c_int32), ("records_fwd", ctypes.c_void_p),
+           ("NC", ctypes.c_int32), ("records_fwd_slots", ctypes.c_int32), ("records_fwd", ctypes.c_void_p),
            ("records_fwd_bytes", ctypes.c_uint64)]
     )  # fmt: skip
 

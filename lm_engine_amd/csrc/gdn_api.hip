@@ -189,9 +189,11 @@ int gdn_chunk_fwd_saving(const gdn_args* a, const gdn_chunk_saves* saves, void* 
     if (saves->records_given == 1 && a->K > 128) return GDN_ERR_UNSUPPORTED;  // K = 256 scans on half-slice waves only
     if (saves->records_given) {
         // records are given for batches of rows: fixed-length, or left-padded with whole chunks per row
-        if (a->cu_seqlens != nullptr && (!(a->flags & GDN_FLAG_LEFT_PADDED) || saves->mirror_reads)) return GDN_ERR_VARLEN;
+        // (or, in a workspace of the full layout, for packed sequences)
+        const bool packed = a->cu_seqlens != nullptr && !(a->flags & GDN_FLAG_LEFT_PADDED);
+        if (a->cu_seqlens != nullptr && ((packed && !saves->packed_records) || saves->mirror_reads)) return GDN_ERR_VARLEN;
         if (saves->row_order != nullptr && !aligned(saves->row_order, 4)) return GDN_ERR_ALIGN;
-        need = gdn::chunk_record_bytes(*a);
+        if (!packed) need = gdn::chunk_record_bytes(*a);
     }
     if (a->workspace == nullptr || a->workspace_bytes < need || !aligned(a->workspace, 256)) return GDN_ERR_WORKSPACE;
     if ((saves->states_dtype != GDN_F32 && saves->states_dtype != GDN_BF16) || (saves->v_new_dtype != GDN_F32 && saves->v_new_dtype != GDN_BF16))
@@ -265,8 +267,10 @@ int gdn_chunk_bwd_prepare(const gdn_chunk_bwd_prepare_args* a, void* stream) {
     if ((int64_t)a->N * a->H * (a->seq_start != nullptr ? a->NC : a->T / 64) > 0x7fffffff) return GDN_ERR_UNSUPPORTED;
     if (!aligned(a->records, 256) || a->records_bytes < gdn::chunk_bwd_record_bytes(*a)) return GDN_ERR_WORKSPACE;
     if (a->records_fwd != nullptr) {
-        if (a->seq_start != nullptr) return GDN_ERR_VARLEN;  // the forward's records are laid out for whole-chunk batches
-        if (!aligned(a->records_fwd, 256) || a->records_fwd_bytes < gdn::chunk_bwd_record_bytes(*a) / 2) return GDN_ERR_WORKSPACE;
+        if (a->seq_start != nullptr && a->records_fwd_slots <= 0) return GDN_ERR_VARLEN;  // batches of rows that are not whole chunks
+        const uint64_t fwd_bytes = a->seq_start == nullptr ? gdn::chunk_bwd_record_bytes(*a) / 2
+                                                           : gdn::chunk_bwd_record_bytes(*a) / (2 * (uint64_t)a->N * a->NC) * a->records_fwd_slots;
+        if (!aligned(a->records_fwd, 256) || a->records_fwd_bytes < fwd_bytes) return GDN_ERR_WORKSPACE;
     }
     return gdn::launch_chunk_bwd_prepare(*a, static_cast<hipStream_t>(stream));
 }

@@ -201,7 +201,9 @@ int launch_chunk_fwd(const gdn_args& a, hipStream_t stream, hipEvent_t* events, 
         p.no_output = saves->no_output ? 1 : 0;
         p.save_every = saves->save_every > 0 ? saves->save_every : 1, p.save_reverse = saves->save_reverse ? 1 : 0;
         p.records_given = saves->records_given;
-        if (p.records_given) p.chunk_off = nullptr, p.seq_order = nullptr, p.ready = nullptr, p.err = nullptr, p.rec = static_cast<uint8_t*>(a.workspace);
+        // (given records of packed sequences: a workspace of the full layout, the chunk offsets are formed in it below)
+        if (p.records_given && p.cu_seqlens == nullptr) p.chunk_off = nullptr, p.seq_order = nullptr, p.rec = static_cast<uint8_t*>(a.workspace);
+        if (p.records_given) p.ready = nullptr, p.err = nullptr;
     }
     p.q_stride_b = a.q_stride_b, p.q_stride_t = a.q_stride_t, p.q_stride_h = a.q_stride_h;
     p.k_stride_b = a.k_stride_b, p.k_stride_t = a.k_stride_t, p.k_stride_h = a.k_stride_h;

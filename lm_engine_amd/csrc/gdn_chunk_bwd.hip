@@ -839,7 +839,8 @@ struct BwdPrepareParams {
     bf16_t* k_m;
     bf16_t* v_m;
     uint8_t* rec;
-    uint8_t* rec_fwd;  // the forward sweep's own records, [H][N NC] (whole-chunk batches), or NULL
+    uint8_t* rec_fwd;  // the forward sweep's own records, [H][N NC] (whole-chunk batches) or [H][fwd_slots] (packed), or NULL
+    int fwd_slots;     // packed batches: record slots per head; sequence n's begin behind the chunks of the sequences before it
     uint32_t rec_bytes, off_p, off_qs, off_ks, off_cs, off_eg;
 };
 
@@ -1214,10 +1215,32 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 64 ? 3 : 2)) void chunk_bwd_prep
             reinterpret_cast<bf16x8*>(recB + p.off_p)[fl] = zz;
         }
     }
+    if (t < C) {
+        const int src = C - 1 - t;
+        reinterpret_cast<float*>(recA + p.off_qs)[t] = 0.f;
+        reinterpret_cast<float*>(recA + p.off_ks)[t] = -(s_beta[src] * s_e[src] * s_rk[src]);
+        reinterpret_cast<float*>(recA + p.off_cs)[t] = -(s_tail[src] * s_rk[src]);
+        reinterpret_cast<float*>(recB + p.off_qs)[t] = 0.f;
+        reinterpret_cast<float*>(recB + p.off_ks)[t] = s_e[src] * s_rq[src] * p.scale;
+        reinterpret_cast<float*>(recB + p.off_cs)[t] = 0.f;
+        if (t == 0) {
+            *reinterpret_cast<float*>(recA + p.off_eg) = s_e[C - 1];
+            *reinterpret_cast<float*>(recB + p.off_eg) = 1.f;
+        }
+    }
     if (p.rec_fwd != nullptr) {
         // The record the forward's prepare step would write for this chunk (T diag(beta), P, the three row scales,
         // e^{gamma_C}), so that the forward sweep of the backward pass needs no prepare launch of its own.
-        uint8_t* const recF = p.rec_fwd + ((int64_t)h * ((int64_t)p.N * p.NC) + (int64_t)n * p.NC + ci) * p.rec_bytes;
+        int64_t slot = (int64_t)h * ((int64_t)p.N * p.NC) + (int64_t)n * p.NC + ci;
+        if (p.fwd_slots > 0) {  // the offsets chunk_offsets_kernel gives the scan (every wave adds them up for itself)
+            int before = 0;
+            for (int m = lane; m < n; m += WAVE) before += (max(p.seq_len[m], 0) + C - 1) / C;
+#pragma unroll
+            for (int off = WAVE / 2; off >= 1; off >>= 1) before += __shfl_xor(before, off, WAVE);
+            if (valid == 0 || before + ci >= p.fwd_slots) return;  // the empty first slot of an empty sequence has no record
+            slot = (int64_t)h * p.fwd_slots + before + ci;
+        }
+        uint8_t* const recF = p.rec_fwd + slot * p.rec_bytes;
         for (int fl = t; fl < 6 * WAVE; fl += BWD_THREADS) {
             const int f = fl / WAVE, L = fl % WAVE;
             const int row = p.rec16 ? 16 * (f < 2 ? f : 2 + (f - 2) / 2) + L % 16 : 32 * (f < 2 ? 0 : 1) + L % 32;
@@ -1239,19 +1262,6 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 64 ? 3 : 2)) void chunk_bwd_prep
             reinterpret_cast<float*>(recF + p.off_ks)[t] = live ? s_tail[t] * s_rk[t] : 0.f;
             reinterpret_cast<float*>(recF + p.off_cs)[t] = live ? s_e[t] * s_rk[t] : 0.f;
             if (t == 0) *reinterpret_cast<float*>(recF + p.off_eg) = s_e[C - 1];
-        }
-    }
-    if (t < C) {
-        const int src = C - 1 - t;
-        reinterpret_cast<float*>(recA + p.off_qs)[t] = 0.f;
-        reinterpret_cast<float*>(recA + p.off_ks)[t] = -(s_beta[src] * s_e[src] * s_rk[src]);
-        reinterpret_cast<float*>(recA + p.off_cs)[t] = -(s_tail[src] * s_rk[src]);
-        reinterpret_cast<float*>(recB + p.off_qs)[t] = 0.f;
-        reinterpret_cast<float*>(recB + p.off_ks)[t] = s_e[src] * s_rq[src] * p.scale;
-        reinterpret_cast<float*>(recB + p.off_cs)[t] = 0.f;
-        if (t == 0) {
-            *reinterpret_cast<float*>(recA + p.off_eg) = s_e[C - 1];
-            *reinterpret_cast<float*>(recB + p.off_eg) = 1.f;
         }
     }
 }
@@ -1326,7 +1336,8 @@ int launch_chunk_bwd_prepare(const gdn_chunk_bwd_prepare_args& a, hipStream_t st
     p.rq = a.rq, p.rk = a.rk;
     p.k_m = static_cast<bf16_t*>(a.k_mirror), p.v_m = static_cast<bf16_t*>(a.v_mirror);
     p.rec = static_cast<uint8_t*>(a.records);
-    p.rec_fwd = a.seq_start == nullptr ? static_cast<uint8_t*>(a.records_fwd) : nullptr;
+    p.rec_fwd = static_cast<uint8_t*>(a.records_fwd);
+    p.fwd_slots = a.seq_start != nullptr ? a.records_fwd_slots : 0;
     p.rec_bytes = r.bytes, p.off_p = r.off_p, p.off_qs = r.off_qs, p.off_ks = r.off_ks, p.off_cs = r.off_cs, p.off_eg = r.off_eg;
     const int64_t chunks = (int64_t)a.N * a.H * p.NC;
     const dim3 grid((unsigned)chunks), block(BWD_THREADS);

@@ -364,11 +364,12 @@ def saving_scan_is_staged(N, T, H, K, V, cu_seqlens=None, left_padded=False, rec
 
 
 def chunk_forward_saving(q, k, v, g, beta, scale, initial_state, cu_seqlens, l2norm, left_padded, states, v_new,
-                         chunks_per_chain, no_output=False, sliced=False):  # fmt: skip
+                         chunks_per_chain, no_output=False, sliced=False, workspace=None):  # fmt: skip
     """The chunked forward once more, for the backward pass: through ``gdn_chunk_fwd_saving`` it writes the
     state every chunk starts from into ``states`` ``[N * H, chunks_per_chain, K, V]`` and V~ into ``v_new``
     ``[N * H, chunks_per_chain, 64, V]`` (contiguous; fp32, or bf16 where ``saving_scan_is_staged``).  The output
-    itself is discarded (``no_output``: the library skips forming it where it has a scan without output)."""
+    itself is discarded (``no_output``: the library skips forming it where it has a scan without output).  ``workspace``
+    (packed sequences): what ``chunk_bwd_prepare`` returned as ``workspace_fwd``, whose records are used as they are."""
     _require_hip_path()
     lib = _lib.load_library()
     dims = _check_inputs(q, k, v, g, beta, initial_state, cu_seqlens, left_padded)
@@ -385,9 +386,12 @@ def chunk_forward_saving(q, k, v, g, beta, scale, initial_state, cu_seqlens, l2n
     args = _fill_args(q, k, v, g, beta, h0, None, o, cu_seqlens, scale, l2norm, False, dims, left_padded)
     saves = _lib.GdnChunkSaves(states.data_ptr(), v_new.data_ptr(), chunks_per_chain, 0, 1, 0, states_code, v_new_code,
                                1 if no_output else 0, 0, 1 if sliced else 0)  # fmt: skip
+    if workspace is not None:
+        saves.records_given, saves.packed_records = 2, 1
     with torch.cuda.device(q.device):
-        nbytes = lib.gdn_workspace_bytes(ctypes.byref(args))
-        workspace = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=q.device)
+        if workspace is None:
+            nbytes = lib.gdn_workspace_bytes(ctypes.byref(args))
+            workspace = torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=q.device)
         args.workspace, args.workspace_bytes = workspace.data_ptr(), workspace.numel()
         stream = ctypes.c_void_p(torch.cuda.current_stream(q.device).cuda_stream)
         _lib.check_status(lib.gdn_chunk_fwd_saving(ctypes.byref(args), ctypes.byref(saves), stream),
@@ -401,17 +405,33 @@ def half_slice_records_pay(chains: int, V: int, device) -> bool:
     return chains * (V // 32) <= torch.cuda.get_device_properties(device).multi_processor_count
 
 
-def left_padded_rows(valid_lengths, T: int, device):
-    """Device tensors for ``chunk_scan_given_records(..., valid_lengths=...)`` from the rows' valid lengths (host integers,
-    positive multiples of 64, at most ``T``): the int32 prefix sums ``[B + 1]`` and the rows longest first ``[B]``.  Making
-    them is two small host-to-device copies; a caller that scans several times, or wants the copies out of the way of
-    its launches, makes them once and passes the pair."""
+def left_padded_row_lists(valid_lengths, T: int):
+    """The prefix sums of the rows' valid lengths and the rows longest first, as host lists (see ``left_padded_rows``)."""
     if any(int(n) <= 0 or int(n) % 64 != 0 or int(n) > T for n in valid_lengths):
         raise ValueError(f"valid_lengths must be positive multiples of 64 of at most T = {T}")
     sums = [0]
     for length in valid_lengths:
         sums.append(sums[-1] + int(length))
-    longest_first = sorted(range(len(valid_lengths)), key=lambda n: (-int(valid_lengths[n]), n))
+    return sums, sorted(range(len(valid_lengths)), key=lambda n: (-int(valid_lengths[n]), n))
+
+
+def upload_int32(lists, device):
+    """Host lists of integers as int32 device tensors, in one copy out of pinned memory that the host does not wait for (a
+    copy out of pageable memory waits until the stream has come to it; under graph capture it is the pageable one, which
+    is refused there)."""
+    flat = torch.tensor([x for values in lists for x in values], dtype=torch.int32)
+    if not torch.cuda.is_current_stream_capturing():
+        flat = flat.pin_memory()
+    with torch.cuda.device(device):
+        return flat.to(device, non_blocking=flat.is_pinned()).split([len(values) for values in lists])
+
+
+def left_padded_rows(valid_lengths, T: int, device):
+    """Device tensors for ``chunk_scan_given_records(..., valid_lengths=...)`` from the rows' valid lengths (host integers,
+    positive multiples of 64, at most ``T``): the int32 prefix sums ``[B + 1]`` and the rows longest first ``[B]``.  Making
+    them is two small host-to-device copies; a caller that scans several times, or wants the copies out of the way of
+    its launches, makes them once and passes the pair."""
+    sums, longest_first = left_padded_row_lists(valid_lengths, T)
     return (torch.tensor(sums, dtype=torch.int32, device=device), torch.tensor(longest_first, dtype=torch.int32, device=device))
 
 
@@ -485,7 +505,8 @@ def backward_kernels_apply(K: int, V: int) -> bool:
     return K in _SUPPORTED_K and V % 64 == 0
 
 
-def chunk_local_grads(q, k, v, dout, prep, y_mirror, v_new, states, dstates, scale, l2norm, sequences=None, sliced=False):
+def chunk_local_grads(q, k, v, dout, prep, y_mirror, v_new, states, dstates, scale, l2norm, sequences=None, sliced=False,
+                      covers=False):
     """``gdn_chunk_bwd_local``: q, k, v, dout are the caller's bf16 ``[B, T, H, D]`` tensors (last dim contiguous),
     ``prep`` what ``chunk_bwd_prepare`` returned (same ``sequences``), ``y_mirror`` the output of the scan over its
     mirror problem (bf16 ``[N, 2 NC 64, H, V]``) or, as a 4-D tensor, the V~ that scan saved at its even chunks (bf16
@@ -512,7 +533,8 @@ def chunk_local_grads(q, k, v, dout, prep, y_mirror, v_new, states, dstates, sca
                                   ("dstates", dstates, (Bt, NC, K, V), dstates.dtype)):  # fmt: skip
         if tuple(x.shape) != shape or x.dtype != dtype or not x.is_contiguous():
             raise ValueError(f"{name} must be contiguous {dtype} {shape}")
-    alloc = torch.empty if sequences is None else torch.zeros  # tokens outside every sequence are not written
+    # tokens outside every sequence are not written (`covers`: there are none)
+    alloc = torch.empty if sequences is None or covers else torch.zeros
     out = dict(
         dq_out=alloc(B, T, H, K, dtype=torch.bfloat16, device=dev),
         dk_out=alloc(B, T, H, K, dtype=torch.bfloat16, device=dev),
@@ -554,7 +576,7 @@ RECORD_BYTES = 13312  # a chunk record: 12 operand fragments, 3 x 64 row scales,
 
 
 def chunk_bwd_prepare(q, k, dout, g, beta, scale, l2norm, V, sequences=None, half_slice_records=False,
-                      forward_records=False, reversed_copies=True, skip_empty_chunks=False):
+                      forward_records=False, reversed_copies=True, skip_empty_chunks=False, packed=False):
     """``gdn_chunk_bwd_prepare``.  ``q, k, dout`` are the caller's bf16 ``[B, T, H, D]`` tensors; without
     ``sequences`` every row is one sequence of whole chunks, else ``sequences = (seq_start, seq_len, NC)``: int32
     device tensors ``[N]`` (first token as a flat index over the rows, length) and the chunks per sequence to lay
@@ -562,8 +584,9 @@ def chunk_bwd_prepare(q, k, dout, g, beta, scale, l2norm, V, sequences=None, hal
     the chunks, beta, inverse norms of the rows of q and k) and the mirror problem ``k_mirror, v_mirror``
     ``[N, 2 NC 64, H, D]`` bf16, ``records`` uint8 ``[H, N * 2 NC, RECORD_BYTES]`` (their fragments in the lane order
     of the 16x16x32 MFMA with ``half_slice_records``, see ``chunk_scan_given_records``).  ``forward_records``
-    (whole-chunk batches only): also ``records_fwd`` ``[H, N * NC, RECORD_BYTES]``, the records of the forward pass
-    itself in the same fragment order, for a forward sweep without a prepare launch of its own.  Without
+    (whole-chunk batches): also ``records_fwd`` ``[H, N * NC, RECORD_BYTES]``, the records of the forward pass
+    itself in the same fragment order, for a forward sweep without a prepare launch of its own; with ``packed``
+    (``sequences`` are those of one packed row) instead ``workspace_fwd``, for ``chunk_forward_saving``.  Without
     ``reversed_copies`` (whole-chunk batches only) ``k_mirror`` is None and ``v_mirror`` is ``[N, T, H, V]``: P^T dO in
     the caller's token order, for a scan with ``mirror_odd`` that reads the caller's q, k and dout backwards itself.
     ``skip_empty_chunks`` (with ``sequences``): chunk slots past the end of their sequence get no records and no mirror
@@ -612,10 +635,19 @@ def chunk_bwd_prepare(q, k, dout, g, beta, scale, l2norm, V, sequences=None, hal
     a.v_mirror, a.records = out["v_mirror"].data_ptr(), out["records"].data_ptr()
     a.records_bytes = out["records"].numel()
     if forward_records:
-        if sequences is not None:
-            raise ValueError("forward records are written for whole-chunk batches only")
-        out["records_fwd"] = torch.empty(H, N * NC, RECORD_BYTES, dtype=torch.uint8, device=dev)
-        a.records_fwd, a.records_fwd_bytes = out["records_fwd"].data_ptr(), out["records_fwd"].numel()
+        if sequences is None:
+            out["records_fwd"] = torch.empty(H, N * NC, RECORD_BYTES, dtype=torch.uint8, device=dev)
+            a.records_fwd, a.records_fwd_bytes = out["records_fwd"].data_ptr(), out["records_fwd"].numel()
+        elif packed:
+            f = _lib.GdnArgs()  # shape fields and "packed" are all that the size depends on
+            f.B, f.T, f.H, f.K, f.V, f.N, f.chunk, f.dtype = 1, T, H, K, V, N, 64, _lib.GDN_BF16
+            f.cu_seqlens = seq_start.data_ptr()
+            out["workspace_fwd"] = torch.empty(int(lib.gdn_workspace_bytes(ctypes.byref(f))), dtype=torch.uint8, device=dev)
+            a.records_fwd_slots = T // 64 + N
+            a.records_fwd_bytes = H * a.records_fwd_slots * RECORD_BYTES  # the workspace's last part
+            a.records_fwd = out["workspace_fwd"].data_ptr() + out["workspace_fwd"].numel() - a.records_fwd_bytes
+        else:
+            raise ValueError("forward records are written for whole-chunk batches and packed sequences only")
     if sequences is not None:
         a.seq_start, a.seq_len, a.NC = seq_start.data_ptr(), seq_len.data_ptr(), NC
     with torch.cuda.device(dev):

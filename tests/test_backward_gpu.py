@@ -535,3 +535,32 @@ def test_sliced_saves_hold_the_same_values(K, V, no_output):
     assert out[0][0].abs().max() > 0 and out[0][1].abs().max() > 0
     assert torch.equal(out[0][0], _unslice(out[1][0], K)), "states"
     assert torch.equal(out[0][1], _unslice(out[1][1], 64)), "V~"
+
+
+@pytest.mark.parametrize("lens, tail", [([1, 63, 64, 65, 128], 0), ([0, 5, 0, 130, 0], 3), ([0] * 4 + [70] + [3] * 150, 0)])
+@pytest.mark.parametrize("K", [64, 128])
+def test_packed_gradients_match_those_of_single_sequences(lens, tail, K):
+    """The forward sweep of packed sequences on records placed by the backward's prepare kernel (empty sequences, tails, more
+    sequences than lanes, tokens behind the last sequence) against every sequence on its own, within the bf16 gates."""
+    T = sum(lens) + tail
+    inp = random_inputs(B=1, T=T, H=2, K=K, V=64, dtype=torch.bfloat16, seed=21, normalize=False)
+    inp.pop("initial_state", None)
+    names = ("q", "k", "v", "g", "beta")
+    leaves = {n: inp[n].cuda().requires_grad_(True) for n in names}
+    do = torch.randn(inp["v"].shape, generator=torch.Generator().manual_seed(4)).to(torch.bfloat16).cuda()
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+    o, _ = lm_engine_amd.chunk_gated_delta_rule(**leaves, cu_seqlens=cu, use_qk_l2norm_in_kernel=True)
+    covered = T - tail
+    got = torch.autograd.grad(o, list(leaves.values()), do)
+    want = [torch.zeros_like(g) for g in got]
+    begin = 0
+    for length in lens:
+        if length > 0:
+            one = {n: x.detach()[:, begin : begin + length].contiguous().requires_grad_(True) for n, x in leaves.items()}
+            o, _ = lm_engine_amd.chunk_gated_delta_rule(**one, use_qk_l2norm_in_kernel=True)
+            for total, part in zip(want, torch.autograd.grad(o, list(one.values()), do[:, begin : begin + length])):
+                total[:, begin : begin + length] = part
+        begin += length
+    for g in got:
+        assert not g[:, covered:].any(), "tokens that belong to no sequence"
+    _assert_grads([g.cpu() for g in got], [g.cpu() for g in want], torch.bfloat16)
