@@ -302,7 +302,8 @@ typedef struct gdn_chunk_local_args {
     int32_t dstates_dtype; /* gdn_dtype of dstates */
     int32_t saves_sliced;  /* v_new, states, dstates and y_chunks are laid out by 32-column slice, [chunks][V / 32][rows][32]
                               (gdn_chunk_saves.sliced); all of them bf16 then */
-    int32_t reserved;
+    int32_t out_stride_t;  /* elements between the tokens of dq_out, dk_out and dv_out, a multiple of 8: they are column blocks
+                              of one array of token rows; 0: each contiguous */
 } gdn_chunk_local_args;
 int gdn_chunk_bwd_local(const gdn_chunk_local_args *args, void *stream);
 

@@ -101,7 +101,7 @@ class GdnChunkLocalArgs(ctypes.Structure):
         + [(name, ctypes.c_void_p) for name in ("q_raw", "k_raw", "v_raw", "dout_raw")]
         + [(f"{x}_stride_{d}", ctypes.c_int64) for x in ("q", "k", "v", "dout") for d in ("b", "t", "h")]
         + [("seq_start", ctypes.c_void_p), ("seq_len", ctypes.c_void_p), ("T_rows", ctypes.c_int32), ("dstates_dtype", ctypes.c_int32),
-           ("saves_sliced", ctypes.c_int32), ("reserved", ctypes.c_int32)]
+           ("saves_sliced", ctypes.c_int32), ("out_stride_t", ctypes.c_int32)]
     )  # fmt: skip
 
 

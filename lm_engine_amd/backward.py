@@ -336,7 +336,7 @@ def _chunk_local_grads(qs, kn, vc, doc, Y, Vn, S0, dS1, gam, bc):
     return dqs, dkn, dbc, dgam
 
 
-def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm, cu_seqlens, left_padded):
+def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm, cu_seqlens, left_padded, joined):
     """The whole backward on four kernel launches (bf16; K = 64, 128 or 256; V a multiple of 64): ``gdn_chunk_bwd_prepare``
     (per-chunk scalars, the mirror problem, and for whole-chunk batches the forward sweep's records), the saving
     forward sweep, the saving scan over the mirror problem (reverse sweep), ``gdn_chunk_bwd_local`` writing the
@@ -406,7 +406,7 @@ def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm
                                            mirror_odd=(q, do) if mirror_reads else None, sliced=sliced,
                                            valid_lengths=None if mirror_lengths is None else tuple(mirror_lengths))  # fmt: skip
     dq, dk, dv, dg, dbeta = ops.chunk_local_grads(q, k, v, do, prep, Y if staged_m else o_m, Vn, S0, dS1, scale, l2norm,
-                                                  sequences, sliced=sliced, covers=covers)  # fmt: skip
+                                                  sequences, sliced=sliced, covers=covers, joined=joined)  # fmt: skip
     return (
         dq,
         dk,
@@ -419,14 +419,14 @@ def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm
 
 def gated_delta_rule_backward(
     q, k, v, g, beta, do, dht=None, scale=None, initial_state=None, cu_seqlens=None,
-    use_qk_l2norm_in_kernel=False, left_padded=False,
+    use_qk_l2norm_in_kernel=False, left_padded=False, joined=False,
 ):  # fmt: skip
     """Gradients of ``sum(o * do) + sum(final_state * dht)``.
 
     Arguments as for the forward (``g`` or ``beta`` may be None: ungated / beta = 1); ``do`` has the
     shape of ``o``, ``dht`` that of the final state or is None.  Returns
     ``dq, dk, dv, dg, dbeta, dh0`` in the dtypes of the corresponding inputs (fp32 for dh0); entries for
-    absent inputs are None."""
+    absent inputs are None.  ``joined``: dq, dk and dv may be column blocks of one tensor (they are on the kernels)."""
     if q.size(2) != v.size(2):
         # Grouped value attention: the backward runs on the expanded heads (what the reference's repeat_interleave hands
         # its operator, gated_deltanet/module.py:175-177) and adds the gradients of a group's copies up.
@@ -442,7 +442,7 @@ def gated_delta_rule_backward(
     scale = K**-0.5 if scale is None else scale
     if q.is_cuda and q.dtype == torch.bfloat16 and _kernels_apply(K, V):
         return _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, use_qk_l2norm_in_kernel,
-                                    cu_seqlens, left_padded)  # fmt: skip
+                                    cu_seqlens, left_padded, joined)  # fmt: skip
     pk = _Packing(B, T, H, cu_seqlens, left_padded, dev)
     N, NC, Bt = pk.N, pk.NC, pk.N * H
 

@@ -233,6 +233,8 @@ int gdn_chunk_bwd_local(const gdn_chunk_local_args* a, void* stream) {
     if (a->saves_dtype != GDN_BF16 && a->saves_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
     if (a->dstates_dtype != GDN_BF16 && a->dstates_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
     if (a->saves_sliced && (a->saves_dtype != GDN_BF16 || a->dstates_dtype != GDN_BF16 || a->y_chunks == nullptr)) return GDN_ERR_UNSUPPORTED;
+    if (a->out_stride_t != 0 && (a->out_stride_t < (int64_t)a->H * a->K || a->out_stride_t < (int64_t)a->H * a->V)) return GDN_ERR_SHAPE;
+    if (a->out_stride_t % 8 != 0) return GDN_ERR_ALIGN;
     if (a->H <= 0 || a->NC <= 0 || a->chunks % ((int64_t)a->H * a->NC) != 0) return GDN_ERR_SHAPE;
     if (a->seq_start != nullptr && (a->seq_len == nullptr || a->T_rows <= 0)) return GDN_ERR_SHAPE;
     const int64_t raw_strides[] = {a->q_stride_b, a->q_stride_t, a->q_stride_h, a->k_stride_b, a->k_stride_t, a->k_stride_h,

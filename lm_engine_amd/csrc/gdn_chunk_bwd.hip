@@ -80,6 +80,7 @@ struct ChunkLocalParams {
     bf16_t* dv_out;
     float* dg_out;
     float* dbeta_out;
+    int64_t dqk_stride_t, dv_stride_t;  // elements between the tokens of dq_out and dk_out, and of dv_out
     int H, NC, V;
     // sequences that are not whole rows of whole chunks (packed or left-padded batches): first token (flat index
     // over the rows of the caller's tensors) and length of every sequence; NULL = sequence n is row n
@@ -349,7 +350,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                 *reinterpret_cast<bf16x8*>(sDO + row * LDS64 + 8 * p8) = dr;
                 *reinterpret_cast<bf16x8*>(sY + row * LDS64 + 8 * p8) = yr;
                 *reinterpret_cast<bf16x8*>(sVN + row * LDS64 + 8 * p8) = live ? nx_vn[it] : zero8;
-                if (live) *reinterpret_cast<bf16x8*>(p.dv_out + ((tok0 + row) * p.H + h) * V + v0 + 8 * p8) = dv;
+                if (live) *reinterpret_cast<bf16x8*>(p.dv_out + (tok0 + row) * p.dv_stride_t + (int64_t)h * V + v0 + 8 * p8) = dv;
                 yv[it] = acc;
             }
 #pragma unroll
@@ -388,7 +389,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                 *reinterpret_cast<bf16x8*>(sDO + row * LDS64 + 8 * p8) = live ? dr[it] : zero8;
                 *reinterpret_cast<bf16x8*>(sY + row * LDS64 + 8 * p8) = yr[it];
                 *reinterpret_cast<bf16x8*>(sVN + row * LDS64 + 8 * p8) = live ? nr[it] : zero8;
-                if (live) *reinterpret_cast<bf16x8*>(p.dv_out + ((tok0 + row) * p.H + h) * V + v0 + 8 * p8) = dv;
+                if (live) *reinterpret_cast<bf16x8*>(p.dv_out + (tok0 + row) * p.dv_stride_t + (int64_t)h * V + v0 + 8 * p8) = dv;
                 yv[it] = acc;
             }
 #pragma unroll
@@ -424,7 +425,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                 }
                 *reinterpret_cast<bf16x8*>(sDO + row * LDS64 + 8 * p8) = dr;
                 *reinterpret_cast<bf16x8*>(sY + row * LDS64 + 8 * p8) = yr;
-                if (live) *reinterpret_cast<bf16x8*>(p.dv_out + ((tok0 + row) * p.H + h) * V + v0 + 8 * p8) = dv;
+                if (live) *reinterpret_cast<bf16x8*>(p.dv_out + (tok0 + row) * p.dv_stride_t + (int64_t)h * V + v0 + 8 * p8) = dv;
                 yv[it] = acc;
             }
             if (p.saves_bf16) {
@@ -749,7 +750,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 #pragma unroll
         for (int m = 0; m < NTW; m++) {
             const int i = 32 * tt_of(m) + l32;
-            const int64_t at = ((tok0 + i) * p.H + h) * K + KW * kh + 32 * ktl + 4 * lh;
+            const int64_t at = (tok0 + i) * p.dqk_stride_t + (int64_t)h * K + KW * kh + 32 * ktl + 4 * lh;
             const bool norm = p.rq != nullptr;
             const float rq = norm ? p.rq[chunk * C + i] : 1.f, rk = norm ? p.rk[chunk * C + i] : 1.f;
             const float cq = norm ? s_dotq[i] / p.scale : 0.f, ck = norm ? s_dotk[i] : 0.f;
@@ -1284,6 +1285,8 @@ int launch_chunk_bwd_local(const gdn_chunk_local_args& a, hipStream_t stream) {
     p.y_mirror = static_cast<const bf16_t*>(a.y_mirror), p.y_chunks = static_cast<const bf16_t*>(a.y_chunks);
     p.dq_out = static_cast<bf16_t*>(a.dq_out), p.dk_out = static_cast<bf16_t*>(a.dk_out), p.dv_out = static_cast<bf16_t*>(a.dv_out);
     p.dg_out = a.dg_out, p.dbeta_out = a.dbeta_out;
+    p.dqk_stride_t = a.out_stride_t > 0 ? a.out_stride_t : (int64_t)a.H * a.K;
+    p.dv_stride_t = a.out_stride_t > 0 ? a.out_stride_t : (int64_t)a.H * a.V;
     p.H = a.H, p.NC = a.NC, p.V = a.V;
     p.q_raw = static_cast<const bf16_t*>(a.q_raw), p.k_raw = static_cast<const bf16_t*>(a.k_raw);
     p.v_raw = static_cast<const bf16_t*>(a.v_raw), p.d_raw = static_cast<const bf16_t*>(a.dout_raw);

@@ -25,7 +25,34 @@ from ._host import host, raw_stream
 from .conv import _IN_KERNEL_ACTIVATIONS, depthwise_causal_convolution
 from .kernels import Kernel, is_kernel_allowed
 from .layer_ops import delta_rule_gates, gated_rmsnorm
-from .ops import RECURRENT_MAX_TOKENS, chunk_gated_delta_rule, fused_recurrent_gated_delta_rule, layer_step_workspace
+from .ops import RECURRENT_MAX_TOKENS, chunk_gated_delta_rule, column_blocks, fused_recurrent_gated_delta_rule, layer_step_workspace
+
+
+class _SplitChannels(torch.autograd.Function):
+    """``qkv.split`` whose backward hands the three gradients on without a copy when they are the column blocks of one tensor
+    already (what the operator's backward writes for q, k and v that are); else it concatenates them as split's does."""
+
+    @staticmethod
+    def forward(ctx, qkv, num_k_heads, num_v_heads, k_head_dim, v_head_dim):
+        B, S, _ = qkv.shape
+        ctx.set_materialize_grads(False)
+        ctx.shapes = ((B, S, num_k_heads, k_head_dim), (B, S, num_k_heads, k_head_dim), (B, S, num_v_heads, v_head_dim))
+        ctx.options = dict(dtype=qkv.dtype, device=qkv.device)
+        key_dim = num_k_heads * k_head_dim
+        return tuple(x.view(shape) for x, shape in zip(qkv.split((key_dim, key_dim, num_v_heads * v_head_dim), dim=-1), ctx.shapes))
+
+    @staticmethod
+    def backward(ctx, *grads):
+        if all(d is None for d in grads):
+            return None, None, None, None, None
+        grads = [torch.zeros(shape, **ctx.options) if d is None else d for d, shape in zip(grads, ctx.shapes)]
+        if column_blocks(*grads):
+            B, S = grads[0].shape[:2]
+            row = sum(d.size(2) * d.size(3) for d in grads)
+            joined = grads[0].as_strided((B, S, row), (S * row, row, 1))
+        else:
+            joined = torch.cat([d.flatten(-2) for d in grads], dim=-1)
+        return joined, None, None, None, None
 
 
 def gated_deltanet_mixing(
@@ -79,10 +106,13 @@ def gated_deltanet_mixing(
 
     qkv, conv_state = depthwise_causal_convolution(qkv, conv_weight, conv_bias, conv_state, attention_mask, use_cache,
                                                    conv_activation)  # fmt: skip
-    q, k, v = qkv.split((key_dim, key_dim, value_dim), dim=-1)
-    q = q.view(B, S, num_k_heads, k_head_dim)
-    k = k.view(B, S, num_k_heads, k_head_dim)
-    v = v.view(B, S, num_v_heads, v_head_dim)
+    if torch.is_grad_enabled() and qkv.requires_grad and not torch.compiler.is_compiling():
+        q, k, v = _SplitChannels.apply(qkv, num_k_heads, num_v_heads, k_head_dim, v_head_dim)
+    else:
+        q, k, v = qkv.split((key_dim, key_dim, value_dim), dim=-1)
+        q = q.view(B, S, num_k_heads, k_head_dim)
+        k = k.view(B, S, num_k_heads, k_head_dim)
+        v = v.view(B, S, num_v_heads, v_head_dim)
     # grouped value attention (num_v_heads > num_k_heads): the operator reads head h / (num_v_heads / num_k_heads) of q
     # and k for value head h, so the reference's repeat_interleave copies (module.py:175-177) are not made
 

@@ -505,14 +505,26 @@ def backward_kernels_apply(K: int, V: int) -> bool:
     return K in _SUPPORTED_K and V % 64 == 0
 
 
+def column_blocks(q, k, v) -> bool:
+    """Whether q, k and v ``[B, T, H, D]`` are the three column blocks, in this order, of the rows of one ``[B, T, C]`` tensor."""
+    width = q.size(2) * q.size(3)
+    row = 2 * width + v.size(2) * v.size(3)
+    return (
+        k.shape == q.shape and q.dtype == k.dtype == v.dtype
+        and all(x.stride() == (x.size(1) * row, row, x.size(3), 1) for x in (q, k, v))
+        and q.untyped_storage().data_ptr() == k.untyped_storage().data_ptr() == v.untyped_storage().data_ptr()
+        and k.storage_offset() == q.storage_offset() + width and v.storage_offset() == k.storage_offset() + width
+    )
+
+
 def chunk_local_grads(q, k, v, dout, prep, y_mirror, v_new, states, dstates, scale, l2norm, sequences=None, sliced=False,
-                      covers=False):
+                      covers=False, joined=False):
     """``gdn_chunk_bwd_local``: q, k, v, dout are the caller's bf16 ``[B, T, H, D]`` tensors (last dim contiguous),
     ``prep`` what ``chunk_bwd_prepare`` returned (same ``sequences``), ``y_mirror`` the output of the scan over its
     mirror problem (bf16 ``[N, 2 NC 64, H, V]``) or, as a 4-D tensor, the V~ that scan saved at its even chunks (bf16
     ``[N H, NC, 64, V]``), ``v_new`` and ``states`` what the saving forward sweep wrote (both fp32 or both bf16),
-    ``dstates`` the states the mirror scan saved (fp32 or bf16).  Returns ``dq, dk, dv`` bf16 ``[B, T, H, D]`` and ``dg, dbeta`` fp32
-    ``[B, T, H]`` (zero where no sequence lives)."""
+    ``dstates`` the states the mirror scan saved (fp32 or bf16).  Returns ``dq, dk, dv`` bf16 ``[B, T, H, D]`` (with ``joined``
+    the column blocks of one ``[B, T, H (2 K + V)]`` tensor) and ``dg, dbeta`` fp32 ``[B, T, H]`` (zero where no sequence lives)."""
     _require_hip_path()
     lib = _lib.load_library()
     B, T, H, K = q.shape
@@ -535,10 +547,13 @@ def chunk_local_grads(q, k, v, dout, prep, y_mirror, v_new, states, dstates, sca
             raise ValueError(f"{name} must be contiguous {dtype} {shape}")
     # tokens outside every sequence are not written (`covers`: there are none)
     alloc = torch.empty if sequences is None or covers else torch.zeros
+    if joined:  # column blocks of one array
+        rows = alloc(B, T, H * (2 * K + V), dtype=torch.bfloat16, device=dev)
+        dq, dk, dv = (x.view(B, T, H, -1) for x in rows.split((H * K, H * K, H * V), dim=-1))
+    else:
+        dq, dk, dv = (alloc(B, T, H, D, dtype=torch.bfloat16, device=dev) for D in (K, K, V))
     out = dict(
-        dq_out=alloc(B, T, H, K, dtype=torch.bfloat16, device=dev),
-        dk_out=alloc(B, T, H, K, dtype=torch.bfloat16, device=dev),
-        dv_out=alloc(B, T, H, V, dtype=torch.bfloat16, device=dev),
+        dq_out=dq, dk_out=dk, dv_out=dv,
         dg_out=alloc(B, T, H, dtype=torch.float32, device=dev),
         dbeta_out=alloc(B, T, H, dtype=torch.float32, device=dev),
     )
@@ -564,6 +579,7 @@ def chunk_local_grads(q, k, v, dout, prep, y_mirror, v_new, states, dstates, sca
     for name, x in out.items():
         setattr(a, name, x.data_ptr())
     a.chunks, a.K, a.V, a.scale, a.H, a.NC = Bt * NC, K, V, float(scale), H, NC
+    a.out_stride_t = H * (2 * K + V) if joined else 0
     if sequences is not None:
         a.seq_start, a.seq_len, a.T_rows = sequences[0].data_ptr(), sequences[1].data_ptr(), T
     with torch.cuda.device(dev):
@@ -675,9 +691,10 @@ class _GatedDeltaRule(torch.autograd.Function):
     def backward(ctx, do, dht):
         q, k, v, g, beta, initial_state, cu_seqlens = ctx.saved_tensors
         scale, l2norm, left_padded = ctx.options
+        # where q, k and v are column blocks of one tensor their gradients are too (the layer's split hands them on as one)
         dq, dk, dv, dg, dbeta, dh0 = gated_delta_rule_backward(
             q, k, v, g, beta, do, dht, scale=scale, initial_state=initial_state, cu_seqlens=cu_seqlens,
-            use_qk_l2norm_in_kernel=l2norm, left_padded=left_padded,
+            use_qk_l2norm_in_kernel=l2norm, left_padded=left_padded, joined=column_blocks(q, k, v),
         )  # fmt: skip
         return None, None, None, None, None, None, dq, dk, dv, dg, dbeta, dh0, None
 

@@ -214,3 +214,36 @@ def test_layer_chain_gradients():
     got = _grads(kernels, [t.cuda() for t in tensors], [c.cuda()])
     assert [g.dtype for g in got] == [t.dtype for t in tensors]
     _compare(got, want, 3e-2, ("dqkv", "dab", "dconv_weight", "dconv_bias", "dA_log", "ddt_bias", "dnorm_weight"))
+
+
+@pytest.mark.parametrize("B, S, HK, H, K, V", [(2, 192, 2, 2, 128, 64), (1, 130, 3, 3, 64, 64), (2, 128, 2, 4, 64, 64), (1, 64, 2, 2, 256, 512)])
+def test_gradients_of_column_blocks_are_those_of_separate_tensors(B, S, HK, H, K, V):
+    """q, k and v as column blocks of one tensor get gradients that are column blocks of one (written with its token stride);
+    the values are those of three separate tensors, and the layer's split hands them on without a copy.  Bound: the kernel adds
+    some fp32 sums up with LDS atomics, whose order varies from run to run, so a result may round to the neighbouring bf16
+    value: a relative difference of at most 2^-7 where it happens, and it happens to few."""
+    from lm_engine_amd.layer import _SplitChannels
+    from lm_engine_amd.ops import column_blocks
+
+    gen = torch.Generator().manual_seed(S)
+    qkv = torch.randn(B, S, 2 * HK * K + H * V, generator=gen).to(torch.bfloat16).cuda().requires_grad_(True)
+    g = -torch.rand(B, S, H, generator=gen).cuda()
+    beta = torch.rand(B, S, H, generator=gen).to(torch.bfloat16).cuda()
+    d_o = torch.randn(B, S, H, V, generator=gen).to(torch.bfloat16).cuda()
+    blocks = _SplitChannels.apply(qkv, HK, H, K, V)
+    separate = [x.detach().contiguous().requires_grad_(True) for x in blocks]
+    assert column_blocks(*blocks) and not column_blocks(*separate) and not column_blocks(blocks[1], blocks[0], blocks[2])
+
+    def grads(q, k, v, wrt):
+        o, _ = lm_engine_amd.chunk_gated_delta_rule(q, k, v, g, beta, use_qk_l2norm_in_kernel=True)
+        return torch.autograd.grad(o, wrt, d_o, retain_graph=True)
+
+    joined, apart = grads(*blocks, blocks), grads(*separate, separate)
+    assert column_blocks(*joined) == (HK == H)
+    for a, b in zip(joined, apart):
+        assert rel_l2(a, b.cpu()) <= 2.0**-8
+    (whole,) = grads(*blocks, (qkv,))
+    assert rel_l2(whole, torch.cat([x.flatten(-2) for x in apart], dim=-1).cpu()) <= 2.0**-8
+    # one of the three does not get a gradient, or gets a larger one
+    (part,) = torch.autograd.grad((2 * blocks[2].float()).sum(), (qkv,), retain_graph=True)
+    assert (part[..., 2 * HK * K :] == 2).all() and not part[..., : 2 * HK * K].any()
