@@ -312,9 +312,9 @@ def bench_decode(steps, warmup):
         "ms_per_step": round(wall_ms, 4),
         "kernel_ms": round(kernel_ms, 4),
         "seq_tokens_per_s": round(w.B / (wall_ms * 1e-3), 1),
-        "roofline": {"kernel": "recurrent_kernel", "bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
+        "roofline": {"kernel": "recurrent_step_kernel", "bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(gbs / HBM_PEAK_GBS, 4),
-                     "traffic": measured_traffic("cfg3_decode_bf16", "recurrent_kernel")},
+                     "traffic": measured_traffic("cfg3_decode_bf16", "recurrent_step_kernel")},
     }  # fmt: skip
 
 
@@ -624,8 +624,8 @@ def bench_backward(w, inp, steps, warmup):
         "steps": steps,
         "ms_per_backward": round(ms, 3),
         "tokens_per_s": round(inp["q"].size(0) * inp["q"].size(1) / (ms * 1e-3), 1),
-        "composition": ("5 kernel launches (and the 7 us chunk-offsets helper): backward prepare, forward prepare + saving scan (forward sweep), saving scan "
-                        "over the mirror problem with every row scanned over its own chunks (reverse sweep), chunk-local "
+        "composition": ("4 kernel launches (and small helpers): backward prepare (also writes the forward sweep's records), saving "
+                        "scan on those records (forward sweep), saving scan over the mirror problem with every row scanned over its own chunks (reverse sweep), chunk-local "
                         "gradients; chunk states, V~ and Y pass between them as bf16"
                         if backward_kernels_apply(w.K, w.V) and inp["cu_seqlens"] is not None else
                         "4 kernel launches: backward prepare (also writes the forward sweep's records), saving scan "
