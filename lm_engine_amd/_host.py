@@ -33,6 +33,6 @@ def host():
         if not os.path.exists(MODULE_PATH):
             raise _lib.GdnLibraryError(f"{MODULE_PATH} is missing: run `python -m lm_engine_amd.build`")
         module = importlib.import_module(".gdn_host", __package__)
-        module.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _BOUND))
+        module.bind(_lib.check_status, *(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _BOUND))
         _module = module
     return _module

@@ -12,9 +12,11 @@
 #include <c10/core/GradMode.h>
 #include <c10/core/impl/VirtualGuardImpl.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/utils/object_ptr.h>
 
 #include <cmath>
 #include <initializer_list>
+#include <utility>
 
 #include "gdn_hip.h"
 
@@ -29,16 +31,20 @@ decltype(&gdn_recurrent_fwd) recurrent_fn = nullptr;
 decltype(&gdn_chunk_fwd) chunk_fn = nullptr;
 decltype(&gdn_workspace_bytes) workspace_bytes_fn = nullptr;
 decltype(&gdn_chunk_fwd_is_one_launch) one_launch_fn = nullptr;
+PyObject* check_status = nullptr;  // _lib.check_status: raises what a status stands for
 
+// bind(check_status, addresses...)
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
     void** slots[] = {(void**)&layer_step_fn, (void**)&layer_step_tiles_fn, (void**)&conv_fn, (void**)&gates_fn, (void**)&norm_fn,
                       (void**)&recurrent_fn, (void**)&chunk_fn, (void**)&workspace_bytes_fn, (void**)&one_launch_fn};
     constexpr Py_ssize_t count = sizeof(slots) / sizeof(slots[0]);
-    if (n != count) return PyErr_Format(PyExc_TypeError, "bind takes %zd addresses, got %zd", count, n);
+    if (n != count + 1) return PyErr_Format(PyExc_TypeError, "bind takes a function and %zd addresses, got %zd arguments", count, n);
     for (Py_ssize_t i = 0; i < count; i++) {
-        *slots[i] = PyLong_AsVoidPtr(args[i]);
+        *slots[i] = PyLong_AsVoidPtr(args[i + 1]);
         if (PyErr_Occurred()) return nullptr;
     }
+    Py_XDECREF(check_status);
+    check_status = Py_NewRef(args[0]);
     Py_RETURN_NONE;
 }
 
@@ -133,6 +139,18 @@ PyObject* pack_results(std::initializer_list<at::Tensor> tensors) {
     return out;
 }
 
+// The last step of a call: launches and hands `results` on.  They are made before the launch, so that nothing can fail behind
+// it.  A refused argument (a negative status: nothing was launched) ends the fast path.  A HIP error (positive) may be that
+// of an earlier call beside a launch that did go through: it is raised, the call is never tried again.
+template <typename F>
+PyObject* launch(const char* what, THPObjectPtr results, F&& entry) {
+    if (!results) return nullptr;
+    const int status = entry();
+    if (status == GDN_OK) return results.release();
+    need(status > 0);
+    return PyObject_CallFunction(check_status, "is", status, what);
+}
+
 at::Tensor fresh(const at::Tensor& like, at::IntArrayRef sizes) { return at::empty(sizes, like.options()); }
 
 // layer_step(stream, qkv, a, b, gate, conv_weight, conv_bias, A_log, dt_bias, norm_weight, eps, HK, H, K, V, conv_state, h,
@@ -189,10 +207,9 @@ PyObject* layer_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
         s.qkv_stride_b = qkv.stride(0), s.a_stride_b = a.stride(0), s.b_stride_b = b.stride(0);
         s.beta_scale = (float)number(args[17]), s.scale = (float)number(args[18]), s.eps = (float)number(args[10]);
         s.activation = (int32_t)integer(args[19]);
-        const int status = layer_step_fn(&s, stream_of(args[0]));
+        PyObject* const result = launch("gdn_layer_step", pack_results({out, state_out, ht}), [&] { return layer_step_fn(&s, stream_of(args[0])); });
         Py_XDECREF(workspace);
-        need(status == 0);
-        return pack_results({out, state_out, ht});
+        return result;
     });
 }
 
@@ -222,8 +239,7 @@ PyObject* conv(PyObject*, PyObject* const* args, Py_ssize_t n) {
         s.x_stride_b = x.stride(0), s.x_stride_s = S > 1 ? x.stride(1) : C, s.y_stride_b = S * C, s.y_stride_s = C;
         s.B = size32(B), s.S = size32(S), s.C = size32(C), s.kernel_size = (int32_t)ks;
         s.activation = (int32_t)integer(args[7]);
-        need(conv_fn(&s, stream_of(args[0])) == 0);
-        return pack_results({y, final_state});
+        return launch("gdn_causal_conv1d_fwd", pack_results({y, final_state}), [&] { return conv_fn(&s, stream_of(args[0])); });
     });
 }
 
@@ -243,8 +259,7 @@ PyObject* gates(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const at::Tensor g = at::empty(a.sizes(), a.options().dtype(at::kFloat)), beta = fresh(a, a.sizes());
         s.a = ptr(a), s.b = ptr(b), s.A_log = static_cast<const float*>(ptr(A_log)), s.dt_bias = static_cast<const float*>(ptr(dt_bias));
         s.g = static_cast<float*>(ptr(g)), s.beta = ptr(beta), s.beta_scale = (float)number(args[5]);
-        need(gates_fn(&s, stream_of(args[0])) == 0);
-        return pack_results({g, beta});
+        return launch("gdn_gates_fwd", pack_results({g, beta}), [&] { return gates_fn(&s, stream_of(args[0])); });
     });
 }
 
@@ -278,8 +293,7 @@ PyObject* norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const at::Tensor y = fresh(o, o.sizes());
         s.o = ptr(o), s.gate = ptr(gate), s.weight = ptr(weight), s.y = ptr(y);
         s.o_stride_t = s.y_stride_t = H * V, s.H = size32(H), s.V = (int32_t)V, s.eps = (float)number(args[4]);
-        need(norm_fn(&s, stream_of(args[0])) == 0);
-        return THPVariable_Wrap(y);
+        return launch("gdn_gated_rmsnorm_fwd", THPVariable_Wrap(y), [&] { return norm_fn(&s, stream_of(args[0])); });
     });
 }
 
@@ -338,15 +352,10 @@ PyObject* delta_rule(PyObject*, PyObject* const* args, Py_ssize_t n) {
         s.v_stride_b = v.stride(0), s.v_stride_t = v.stride(1), s.v_stride_h = v.stride(2);
         s.o_stride_b = o.stride(0), s.o_stride_t = o.stride(1), s.o_stride_h = o.stride(2);
         s.scale = args[7] == Py_None ? (float)std::pow((double)K, -0.5) : (float)number(args[7]);
-        need((chunked ? chunk_fn : recurrent_fn)(&s, stream_of(args[0])) == 0);
-        if (output_final && inplace) {  // the caller's own tensor object
-            PyObject* out = PyTuple_New(2);
-            if (out == nullptr) return nullptr;
-            PyTuple_SET_ITEM(out, 0, THPVariable_Wrap(o));
-            PyTuple_SET_ITEM(out, 1, Py_NewRef(args[8]));
-            return out;
-        }
-        return pack_results({o, ht});
+        THPObjectPtr results(pack_results({o, ht}));
+        if (results && output_final && inplace) PyTuple_SetItem(results.get(), 1, Py_NewRef(args[8]));  // the caller's own tensor object
+        return launch(chunked ? "gdn_chunk_fwd" : "gdn_recurrent_fwd", std::move(results),
+                      [&] { return (chunked ? chunk_fn : recurrent_fn)(&s, stream_of(args[0])); });
     });
 }
 

@@ -1,0 +1,82 @@
+"""The native host path of the inference entry points (csrc/gdn_host.cpp): what it hands on to the Python code, what it raises,
+and what it leaves behind.  The library's entry points are replaced by small stand-ins where a test needs a status or a look
+at the thread's state: nothing is launched then."""
+
+import contextlib
+import ctypes
+
+import pytest
+import torch
+
+import lm_engine_amd
+from lm_engine_amd import _host, _lib
+
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+@contextlib.contextmanager
+def _entry_points_replaced(**stand_ins):
+    """Binds ``name=address`` in place of the library's own entry points."""
+    module, lib = _host.host(), _lib.load_library()
+    own = {name: ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in _host._BOUND}
+    module.bind(_lib.check_status, *({**own, **stand_ins}[name] for name in _host._BOUND))
+    try:
+        yield
+    finally:
+        module.bind(_lib.check_status, *own.values())
+
+
+def _layer_operands(B, S, H=2, K=64, V=64, seed=1):
+    gen = torch.Generator().manual_seed(seed)
+    r = lambda *shape: torch.randn(*shape, generator=gen).to(BF16).cuda()  # noqa: E731
+    C = H * (2 * K + V)
+    return dict(qkv=r(B, S, C), a=r(B, S, H), b=r(B, S, H), gate=r(B, S, H * V), conv_weight=0.3 * r(C, 1, 4), conv_bias=0.1 * r(C),
+                A_log=torch.zeros(H).cuda(), dt_bias=torch.zeros(H).cuda(), norm_weight=r(V), norm_eps=1e-5,
+                num_k_heads=H, num_v_heads=H, k_head_dim=K, v_head_dim=V)  # fmt: skip
+
+
+def _calls():
+    """``name of the C entry -> a call that ends in it``."""
+    x = _layer_operands(2, 1)
+    gen = torch.Generator().manual_seed(2)
+    r = lambda *shape: torch.randn(*shape, generator=gen).to(BF16).cuda()  # noqa: E731
+    q, k, v, long = r(2, 1, 2, 64), r(2, 1, 2, 64), r(2, 1, 2, 64), r(1, 130, 2, 64)
+    h = torch.zeros(2, 2, 64, 64).cuda()
+    return {
+        "gdn_layer_step": lambda: lm_engine_amd.gated_deltanet_mixing(**x, cache=(None, None)),
+        "gdn_causal_conv1d_fwd": lambda: lm_engine_amd.depthwise_causal_convolution(x["qkv"], x["conv_weight"], x["conv_bias"]),
+        "gdn_gates_fwd": lambda: lm_engine_amd.delta_rule_gates(x["a"], x["b"], x["A_log"], x["dt_bias"]),
+        "gdn_gated_rmsnorm_fwd": lambda: lm_engine_amd.gated_rmsnorm(v, None, x["norm_weight"], 1e-5),
+        "gdn_recurrent_fwd": lambda: lm_engine_amd.fused_recurrent_gated_delta_rule(q, k, v, initial_state=h, output_final_state=True,
+                                                                                      inplace_state=True),
+        "gdn_chunk_fwd": lambda: lm_engine_amd.chunk_gated_delta_rule(long, long, long),
+    }  # fmt: skip
+
+
+@pytest.mark.parametrize("entry", ["gdn_layer_step", "gdn_causal_conv1d_fwd", "gdn_gates_fwd", "gdn_gated_rmsnorm_fwd", "gdn_recurrent_fwd",
+                                   "gdn_chunk_fwd"])  # fmt: skip
+def test_a_hip_error_is_raised_and_the_call_not_made_again(entry):
+    """A positive status can come with a launch that is in the stream (the error was pending on the thread): a second launch
+    of an in-place step would advance its state twice.  A negative one (nothing launched) goes to the Python path."""
+    made = []
+
+    def stand_in(status):
+        @ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p)
+        def fn(args, stream):
+            made.append(status)
+            return status
+
+        return fn
+
+    call = _calls()[entry]
+    call()
+    failing, refusing = stand_in(1), stand_in(-3)
+    with _entry_points_replaced(**{entry: ctypes.cast(failing, ctypes.c_void_p).value}):
+        with pytest.raises(RuntimeError, match=f"{entry}.*status 1"):
+            call()
+    with _entry_points_replaced(**{entry: ctypes.cast(refusing, ctypes.c_void_p).value}):
+        call()
+    assert made == [1, -3]
+    torch.cuda.synchronize()
