@@ -16,7 +16,6 @@
 
 #include <cmath>
 #include <initializer_list>
-#include <utility>
 
 #include "gdn_hip.h"
 
@@ -139,11 +138,12 @@ PyObject* pack_results(std::initializer_list<at::Tensor> tensors) {
     return out;
 }
 
-// The last step of a call: launches and hands `results` on.  They are made before the launch, so that nothing can fail behind
+// The last step of a call: launches and hands the results on, which it takes over.  They are made before the launch, so that nothing can fail behind
 // it.  A refused argument (a negative status: nothing was launched) ends the fast path.  A HIP error (positive) may be that
 // of an earlier call beside a launch that did go through: it is raised, the call is never tried again.
 template <typename F>
-PyObject* launch(const char* what, THPObjectPtr results, F&& entry) {
+PyObject* launch(const char* what, PyObject* made, F&& entry) {
+    THPObjectPtr results(made);
     if (!results) return nullptr;
     const int status = entry();
     if (status == GDN_OK) return results.release();
@@ -354,7 +354,7 @@ PyObject* delta_rule(PyObject*, PyObject* const* args, Py_ssize_t n) {
         s.scale = args[7] == Py_None ? (float)std::pow((double)K, -0.5) : (float)number(args[7]);
         THPObjectPtr results(pack_results({o, ht}));
         if (results && output_final && inplace) PyTuple_SetItem(results.get(), 1, Py_NewRef(args[8]));  // the caller's own tensor object
-        return launch(chunked ? "gdn_chunk_fwd" : "gdn_recurrent_fwd", std::move(results),
+        return launch(chunked ? "gdn_chunk_fwd" : "gdn_recurrent_fwd", results.release(),
                       [&] { return (chunked ? chunk_fn : recurrent_fn)(&s, stream_of(args[0])); });
     });
 }
