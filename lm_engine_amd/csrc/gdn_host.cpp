@@ -183,7 +183,7 @@ PyObject* layer_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (conv_state != nullptr) need(conv_state->scalar_type() == qkv.scalar_type() && conv_state->sizes() == at::IntArrayRef({B, C, ks - 1}) && conv_state->is_contiguous());
         if (h0 != nullptr) need(h0->scalar_type() == at::kFloat && h0->sizes() == at::IntArrayRef({B, H, K, V}) && h0->is_contiguous() && aligned(ptr(h0), 16));
         if (gate != nullptr) {
-            need(gate->scalar_type() == qkv.scalar_type() && gate->dim() == 3 && gate->size(0) == B && gate->size(2) == H * V && gate->stride(2) == 1);
+            need(gate->scalar_type() == qkv.scalar_type() && gate->dim() == 3 && gate->size(0) == B && gate->size(1) == 1 && gate->size(2) == H * V && gate->stride(2) == 1);
             s.gate_stride_b = gate->stride(0);
         }
         s.norm_w_dtype = s.dtype;

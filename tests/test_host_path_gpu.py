@@ -80,3 +80,11 @@ def test_a_hip_error_is_raised_and_the_call_not_made_again(entry):
         call()
     assert made == [1, -3]
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("tokens", [2, 3])
+def test_a_gate_of_several_tokens_beside_one_token_is_refused(tokens):
+    x = _layer_operands(2, 1)
+    gate = torch.randn(2, tokens, 128, generator=torch.Generator().manual_seed(3)).to(BF16).cuda()
+    with pytest.raises(ValueError, match="gate must have"):
+        lm_engine_amd.gated_deltanet_mixing(**{**x, "gate": gate}, cache=(None, None))
