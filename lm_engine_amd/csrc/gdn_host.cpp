@@ -227,7 +227,8 @@ PyObject* conv(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (bias != nullptr) need(bias->scalar_type() == weight.scalar_type() && bias->dim() == 1 && bias->size(0) == C && bias->is_contiguous());
         if (state != nullptr) need(state->scalar_type() == x.scalar_type() && state->sizes() == at::IntArrayRef({B, C, ks - 1}) && state->is_contiguous());
         at::Tensor kept_mask;
-        if (mask != nullptr && mask->dim() == 2 && mask->size(0) > 1 && mask->size(1) > 1) {
+        if (mask != nullptr) need(mask->dim() == 2);
+        if (mask != nullptr && mask->size(0) > 1 && mask->size(1) > 1) {
             need(mask->size(0) == B && mask->size(1) == S);
             kept_mask = mask->to(x.scalar_type()).contiguous();
             s.mask = ptr(kept_mask);

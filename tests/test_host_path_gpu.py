@@ -88,3 +88,10 @@ def test_a_gate_of_several_tokens_beside_one_token_is_refused(tokens):
     gate = torch.randn(2, tokens, 128, generator=torch.Generator().manual_seed(3)).to(BF16).cuda()
     with pytest.raises(ValueError, match="gate must have"):
         lm_engine_amd.gated_deltanet_mixing(**{**x, "gate": gate}, cache=(None, None))
+
+
+@pytest.mark.parametrize("shape", [(2, 5, 1), (2, 5, 384), (2, 4), (3, 5)])
+def test_an_attention_mask_that_is_not_one_value_per_token_is_refused(shape):
+    x = _layer_operands(2, 5)
+    with pytest.raises(ValueError, match="attention_mask must be"):
+        lm_engine_amd.depthwise_causal_convolution(x["qkv"], x["conv_weight"], attention_mask=torch.zeros(shape).cuda())
