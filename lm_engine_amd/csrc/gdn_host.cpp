@@ -112,6 +112,15 @@ int64_t row_stride(const at::Tensor& t, int64_t width) {
     return count > 1 ? stride : width;
 }
 
+// taps per channel of a convolution weight [C, 1, taps] or [C, taps]
+int64_t taps_of(const at::Tensor& weight, int64_t C) {
+    const int64_t d = weight.dim();
+    need((d == 2 || (d == 3 && weight.size(1) == 1)) && weight.size(0) == C && weight.is_contiguous());
+    const int64_t taps = weight.size(d - 1);
+    need(taps >= 2 && taps <= 4);
+    return taps;
+}
+
 template <typename F>
 PyObject* fast_path(Py_ssize_t n, Py_ssize_t wanted, F&& body) {
     if (n != wanted) return PyErr_Format(PyExc_TypeError, "takes %zd arguments, got %zd", wanted, n);
@@ -176,9 +185,9 @@ PyObject* layer_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
             need(t->scalar_type() == qkv.scalar_type() && t->dim() == 3 && t->size(0) == B && t->size(1) == 1 && t->size(2) == H && (t->stride(2) == 1 || H == 1));
         const at::Tensor* decay[] = {&A_log, &dt_bias};
         for (const at::Tensor* t : decay) need(t->scalar_type() == at::kFloat && t->dim() == 1 && t->size(0) == H && t->is_contiguous());
-        const int64_t ks = weight.dim() > 0 ? weight.size(-1) : 0;
+        const int64_t ks = taps_of(weight, C);
         s.conv_w_dtype = code_of(weight);
-        need(weight.is_contiguous() && ks >= 2 && ks <= 4 && weight.size(0) == C && weight.numel() == C * ks && (s.dtype == GDN_BF16 || s.conv_w_dtype == GDN_F32));
+        need(s.dtype == GDN_BF16 || s.conv_w_dtype == GDN_F32);
         if (bias != nullptr) need(bias->scalar_type() == weight.scalar_type() && bias->dim() == 1 && bias->size(0) == C && bias->is_contiguous());
         if (conv_state != nullptr) need(conv_state->scalar_type() == qkv.scalar_type() && conv_state->sizes() == at::IntArrayRef({B, C, ks - 1}) && conv_state->is_contiguous());
         if (h0 != nullptr) need(h0->scalar_type() == at::kFloat && h0->sizes() == at::IntArrayRef({B, H, K, V}) && h0->is_contiguous() && aligned(ptr(h0), 16));
@@ -222,8 +231,8 @@ PyObject* conv(PyObject*, PyObject* const* args, Py_ssize_t n) {
         gdn_conv_args s{};
         s.dtype = code_of(x), s.w_dtype = code_of(weight);
         need(x.dim() == 3 && x.stride(2) == 1 && (s.dtype == GDN_BF16 || s.w_dtype == GDN_F32));
-        const int64_t B = x.size(0), S = x.size(1), C = x.size(2), ks = weight.dim() > 1 ? weight.size(-1) : 0;
-        need(B > 0 && S > 0 && ks >= 2 && ks <= 4 && weight.size(0) == C && weight.numel() == C * ks && weight.is_contiguous());
+        const int64_t B = x.size(0), S = x.size(1), C = x.size(2), ks = taps_of(weight, C);
+        need(B > 0 && S > 0);
         if (bias != nullptr) need(bias->scalar_type() == weight.scalar_type() && bias->dim() == 1 && bias->size(0) == C && bias->is_contiguous());
         if (state != nullptr) need(state->scalar_type() == x.scalar_type() && state->sizes() == at::IntArrayRef({B, C, ks - 1}) && state->is_contiguous());
         at::Tensor kept_mask;

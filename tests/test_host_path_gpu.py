@@ -95,3 +95,17 @@ def test_an_attention_mask_that_is_not_one_value_per_token_is_refused(shape):
     x = _layer_operands(2, 5)
     with pytest.raises(ValueError, match="attention_mask must be"):
         lm_engine_amd.depthwise_causal_convolution(x["qkv"], x["conv_weight"], attention_mask=torch.zeros(shape).cuda())
+
+
+def test_a_convolution_weight_of_another_layout_is_refused():
+    """``[C, 1, ks]`` and ``[C, ks]`` are what is taken, on one token (the layer's step) and on several."""
+    x = _layer_operands(2, 1)
+    for shape in ((384, 1, 1, 4), (384, 2, 2), (384, 4, 1)):
+        weight = x["conv_weight"].reshape(shape)
+        with pytest.raises(ValueError, match="weight must be|kernel_size"):
+            lm_engine_amd.depthwise_causal_convolution(x["qkv"], weight)
+        with pytest.raises(ValueError, match="weight must be|kernel_size"):
+            lm_engine_amd.gated_deltanet_mixing(**{**x, "conv_weight": weight}, cache=(None, None))
+    taken = [lm_engine_amd.gated_deltanet_mixing(**{**x, "conv_weight": x["conv_weight"].reshape(shape)}, cache=(None, None))[0]
+             for shape in ((384, 1, 4), (384, 4))]  # fmt: skip
+    assert torch.equal(*taken)
