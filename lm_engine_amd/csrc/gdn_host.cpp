@@ -201,12 +201,12 @@ PyObject* layer_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
             need(norm_w->dim() == 1 && norm_w->size(0) == V && norm_w->is_contiguous());
         }
         s.B = (int32_t)B, s.HK = size32(HK), s.H = (int32_t)H, s.K = (int32_t)K, s.V = (int32_t)V, s.kernel_size = (int32_t)ks;
-        PyObject* workspace = nullptr;  // keeps it alive until the launch is in the stream
+        THPObjectPtr workspace;  // keeps it alive until the launch is in the stream
         if (layer_step_tiles_fn(s.B, s.H, s.V) > 1) {
             workspace = PyObject_CallFunction(args[20], "LL", (long long)(B * H), (long long)V);
-            if (workspace == nullptr) return nullptr;
-            s.tickets = static_cast<int32_t*>(PyLong_AsVoidPtr(PyTuple_GetItem(workspace, 1)));
-            s.scratch = static_cast<float*>(PyLong_AsVoidPtr(PyTuple_GetItem(workspace, 2)));
+            if (!workspace) return nullptr;
+            s.tickets = static_cast<int32_t*>(PyLong_AsVoidPtr(PyTuple_GetItem(workspace.get(), 1)));
+            s.scratch = static_cast<float*>(PyLong_AsVoidPtr(PyTuple_GetItem(workspace.get(), 2)));
         }
         const at::Tensor out = fresh(qkv, {B, 1, H * V}), state_out = fresh(qkv, {B, C, ks - 1});
         const at::Tensor ht = at::empty({B, H, K, V}, qkv.options().dtype(at::kFloat));
@@ -216,9 +216,7 @@ PyObject* layer_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
         s.qkv_stride_b = qkv.stride(0), s.a_stride_b = a.stride(0), s.b_stride_b = b.stride(0);
         s.beta_scale = (float)number(args[17]), s.scale = (float)number(args[18]), s.eps = (float)number(args[10]);
         s.activation = (int32_t)integer(args[19]);
-        PyObject* const result = launch("gdn_layer_step", pack_results({out, state_out, ht}), [&] { return layer_step_fn(&s, stream_of(args[0])); });
-        Py_XDECREF(workspace);
-        return result;
+        return launch("gdn_layer_step", pack_results({out, state_out, ht}), [&] { return layer_step_fn(&s, stream_of(args[0])); });
     });
 }
 

@@ -4,6 +4,7 @@ at the thread's state: nothing is launched then."""
 
 import contextlib
 import ctypes
+import sys
 
 import pytest
 import torch
@@ -109,3 +110,15 @@ def test_a_convolution_weight_of_another_layout_is_refused():
     taken = [lm_engine_amd.gated_deltanet_mixing(**{**x, "conv_weight": x["conv_weight"].reshape(shape)}, cache=(None, None))[0]
              for shape in ((384, 1, 4), (384, 4))]  # fmt: skip
     assert torch.equal(*taken)
+
+
+def test_a_step_that_ends_early_gives_its_workspace_back():
+    """Several workgroups per head: the tickets' memory is asked for, then an operand turns out not to be a number."""
+    x = _layer_operands(2, 1, K=128, V=256)
+    owner = torch.zeros(1 << 16, dtype=torch.int32).cuda()
+    before = sys.getrefcount(owner)
+    result = _host.host().layer_step(
+        _host.raw_stream(0), x["qkv"], x["a"], x["b"], x["gate"], x["conv_weight"], x["conv_bias"], x["A_log"], x["dt_bias"],
+        x["norm_weight"], 1e-5, 2, 2, 128, 256, None, None, "not a number", 1.0, 1,
+        lambda pairs, V: (owner, owner.data_ptr(), owner.data_ptr() + 4 * pairs))  # fmt: skip
+    assert result is None and sys.getrefcount(owner) == before
