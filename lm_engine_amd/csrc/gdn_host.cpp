@@ -78,6 +78,17 @@ int32_t code_of(const at::Tensor& t) {
     need(t.scalar_type() == at::kFloat);
     return GDN_F32;
 }
+// Runs `body`, which touches no Python object, while other Python threads may run: around the allocations of a call, which
+// may wait for the device, and around the library's entry point.
+template <typename F>
+auto without_interpreter_lock(F&& body) {
+    struct Released {
+        PyThreadState* const state = PyEval_SaveThread();
+        ~Released() { PyEval_RestoreThread(state); }
+    } released;
+    return body();
+}
+
 void* ptr(const at::Tensor& t) { return t.data_ptr(); }
 void* ptr(const at::Tensor* t) { return t == nullptr ? nullptr : t->data_ptr(); }
 bool aligned(const void* p, size_t n) { return reinterpret_cast<uintptr_t>(p) % n == 0; }
@@ -147,20 +158,21 @@ PyObject* pack_results(std::initializer_list<at::Tensor> tensors) {
     return out;
 }
 
-// The last step of a call: launches and hands the results on, which it takes over.  They are made before the launch, so that nothing can fail behind
-// it.  A refused argument (a negative status: nothing was launched) ends the fast path.  A HIP error (positive) may be that
-// of an earlier call beside a launch that did go through: it is raised, the call is never tried again.
+// The last step of a call: launches and hands the results on, which it takes over.  They are made before the launch, so that
+// nothing can fail behind it.  A refused argument (a negative status: nothing was launched) ends the fast path.  A HIP error
+// (positive) may be that of an earlier call beside a launch that did go through: it is raised, the call is never tried again.
 template <typename F>
 PyObject* launch(const char* what, PyObject* made, F&& entry) {
     THPObjectPtr results(made);
     if (!results) return nullptr;
-    const int status = entry();
+    const int status = without_interpreter_lock(entry);
     if (status == GDN_OK) return results.release();
     need(status > 0);
     return PyObject_CallFunction(check_status, "is", status, what);
 }
 
 at::Tensor fresh(const at::Tensor& like, at::IntArrayRef sizes) { return at::empty(sizes, like.options()); }
+at::Tensor fresh_f32(const at::Tensor& like, at::IntArrayRef sizes) { return at::empty(sizes, like.options().dtype(at::kFloat)); }
 
 // layer_step(stream, qkv, a, b, gate, conv_weight, conv_bias, A_log, dt_bias, norm_weight, eps, HK, H, K, V, conv_state, h,
 //            beta_scale, scale, activation, workspace) -> (o [B, 1, H V], conv_state, h)
@@ -168,6 +180,7 @@ at::Tensor fresh(const at::Tensor& like, at::IntArrayRef sizes) { return at::emp
 PyObject* layer_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return fast_path(n, 21, [&]() -> PyObject* {
         Operands operand;
+        void* const stream = stream_of(args[0]);
         const at::Tensor &qkv = operand(args[1]), &a = operand(args[2]), &b = operand(args[3]), &weight = operand(args[5]);
         const at::Tensor &A_log = operand(args[7]), &dt_bias = operand(args[8]);
         const at::Tensor *gate = operand.optional(args[4]), *bias = operand.optional(args[6]), *norm_w = operand.optional(args[9]);
@@ -208,15 +221,15 @@ PyObject* layer_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
             s.tickets = static_cast<int32_t*>(PyLong_AsVoidPtr(PyTuple_GetItem(workspace.get(), 1)));
             s.scratch = static_cast<float*>(PyLong_AsVoidPtr(PyTuple_GetItem(workspace.get(), 2)));
         }
-        const at::Tensor out = fresh(qkv, {B, 1, H * V}), state_out = fresh(qkv, {B, C, ks - 1});
-        const at::Tensor ht = at::empty({B, H, K, V}, qkv.options().dtype(at::kFloat));
+        at::Tensor out, state_out, ht;
+        without_interpreter_lock([&] { out = fresh(qkv, {B, 1, H * V}), state_out = fresh(qkv, {B, C, ks - 1}), ht = fresh_f32(qkv, {B, H, K, V}); });
         s.qkv = ptr(qkv), s.conv_weight = ptr(weight), s.conv_bias = ptr(bias), s.conv_state = ptr(conv_state), s.conv_state_out = ptr(state_out);
         s.a = ptr(a), s.b = ptr(b), s.A_log = static_cast<const float*>(ptr(A_log)), s.dt_bias = static_cast<const float*>(ptr(dt_bias));
         s.h0 = static_cast<const float*>(ptr(h0)), s.ht = static_cast<float*>(ptr(ht)), s.gate = ptr(gate), s.norm_weight = ptr(norm_w), s.out = ptr(out);
         s.qkv_stride_b = qkv.stride(0), s.a_stride_b = a.stride(0), s.b_stride_b = b.stride(0);
         s.beta_scale = (float)number(args[17]), s.scale = (float)number(args[18]), s.eps = (float)number(args[10]);
         s.activation = (int32_t)integer(args[19]);
-        return launch("gdn_layer_step", pack_results({out, state_out, ht}), [&] { return layer_step_fn(&s, stream_of(args[0])); });
+        return launch("gdn_layer_step", pack_results({out, state_out, ht}), [&] { return layer_step_fn(&s, stream); });
     });
 }
 
@@ -224,6 +237,7 @@ PyObject* layer_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyObject* conv(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return fast_path(n, 8, [&]() -> PyObject* {
         Operands operand;
+        void* const stream = stream_of(args[0]);
         const at::Tensor &x = operand(args[1]), &weight = operand(args[2]);
         const at::Tensor *bias = operand.optional(args[3]), *state = operand.optional(args[4]), *mask = operand.optional(args[5]);
         gdn_conv_args s{};
@@ -234,20 +248,24 @@ PyObject* conv(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (bias != nullptr) need(bias->scalar_type() == weight.scalar_type() && bias->dim() == 1 && bias->size(0) == C && bias->is_contiguous());
         if (state != nullptr) need(state->scalar_type() == x.scalar_type() && state->sizes() == at::IntArrayRef({B, C, ks - 1}) && state->is_contiguous());
         at::Tensor kept_mask;
+        bool masked = false;
         if (mask != nullptr) need(mask->dim() == 2);
         if (mask != nullptr && mask->size(0) > 1 && mask->size(1) > 1) {
             need(mask->size(0) == B && mask->size(1) == S);
-            kept_mask = mask->to(x.scalar_type()).contiguous();
-            s.mask = ptr(kept_mask);
+            masked = true;
         }
-        const at::Tensor y = fresh(x, {B, S, C});
-        at::Tensor final_state;
-        if (truth(args[6])) final_state = fresh(x, {B, C, ks - 1}), s.final_state = ptr(final_state);
+        const bool output_state = truth(args[6]);
+        at::Tensor y, final_state;
+        without_interpreter_lock([&] {
+            if (masked) kept_mask = mask->to(x.scalar_type()).contiguous(), s.mask = ptr(kept_mask);
+            y = fresh(x, {B, S, C});
+            if (output_state) final_state = fresh(x, {B, C, ks - 1}), s.final_state = ptr(final_state);
+        });
         s.x = ptr(x), s.weight = ptr(weight), s.bias = ptr(bias), s.input_state = ptr(state), s.y = ptr(y);
         s.x_stride_b = x.stride(0), s.x_stride_s = S > 1 ? x.stride(1) : C, s.y_stride_b = S * C, s.y_stride_s = C;
         s.B = size32(B), s.S = size32(S), s.C = size32(C), s.kernel_size = (int32_t)ks;
         s.activation = (int32_t)integer(args[7]);
-        return launch("gdn_causal_conv1d_fwd", pack_results({y, final_state}), [&] { return conv_fn(&s, stream_of(args[0])); });
+        return launch("gdn_causal_conv1d_fwd", pack_results({y, final_state}), [&] { return conv_fn(&s, stream); });
     });
 }
 
@@ -255,6 +273,7 @@ PyObject* conv(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyObject* gates(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return fast_path(n, 6, [&]() -> PyObject* {
         Operands operand;
+        void* const stream = stream_of(args[0]);
         const at::Tensor &a = operand(args[1]), &b = operand(args[2]), &A_log = operand(args[3]), &dt_bias = operand(args[4]);
         gdn_gate_args s{};
         s.dtype = code_of(a);
@@ -264,10 +283,11 @@ PyObject* gates(PyObject*, PyObject* const* args, Py_ssize_t n) {
         for (const at::Tensor* t : decay) need(t->scalar_type() == at::kFloat && t->dim() == 1 && t->size(0) == H && t->is_contiguous());
         s.a_stride = row_stride(a, H), s.b_stride = row_stride(b, H);
         s.tokens = a.numel() / H, s.H = size32(H);
-        const at::Tensor g = at::empty(a.sizes(), a.options().dtype(at::kFloat)), beta = fresh(a, a.sizes());
+        at::Tensor g, beta;
+        without_interpreter_lock([&] { g = fresh_f32(a, a.sizes()), beta = fresh(a, a.sizes()); });
         s.a = ptr(a), s.b = ptr(b), s.A_log = static_cast<const float*>(ptr(A_log)), s.dt_bias = static_cast<const float*>(ptr(dt_bias));
         s.g = static_cast<float*>(ptr(g)), s.beta = ptr(beta), s.beta_scale = (float)number(args[5]);
-        return launch("gdn_gates_fwd", pack_results({g, beta}), [&] { return gates_fn(&s, stream_of(args[0])); });
+        return launch("gdn_gates_fwd", pack_results({g, beta}), [&] { return gates_fn(&s, stream); });
     });
 }
 
@@ -275,6 +295,7 @@ PyObject* gates(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyObject* norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return fast_path(n, 5, [&]() -> PyObject* {
         Operands operand;
+        void* const stream = stream_of(args[0]);
         const at::Tensor& o = operand(args[1]);
         const at::Tensor *gate = operand.optional(args[2]), *weight = operand.optional(args[3]);
         gdn_norm_args s{};
@@ -298,10 +319,10 @@ PyObject* norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
             need(weight->dim() == 1 && weight->size(0) == V && weight->is_contiguous());
         }
         s.w_dtype |= GDN_NORM_GATE_DWORDS;
-        const at::Tensor y = fresh(o, o.sizes());
+        const at::Tensor y = without_interpreter_lock([&] { return fresh(o, o.sizes()); });
         s.o = ptr(o), s.gate = ptr(gate), s.weight = ptr(weight), s.y = ptr(y);
         s.o_stride_t = s.y_stride_t = H * V, s.H = size32(H), s.V = (int32_t)V, s.eps = (float)number(args[4]);
-        return launch("gdn_gated_rmsnorm_fwd", THPVariable_Wrap(y), [&] { return norm_fn(&s, stream_of(args[0])); });
+        return launch("gdn_gated_rmsnorm_fwd", THPVariable_Wrap(y), [&] { return norm_fn(&s, stream); });
     });
 }
 
@@ -311,6 +332,7 @@ PyObject* norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
 PyObject* delta_rule(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return fast_path(n, 13, [&]() -> PyObject* {
         Operands operand;
+        void* const stream = stream_of(args[0]);
         const bool chunked = truth(args[1]), output_final = truth(args[9]), inplace = truth(args[12]);
         const at::Tensor &q = operand(args[2]), &k = operand(args[3]), &v = operand(args[4]);
         const at::Tensor *g = operand.optional(args[5]), *beta = operand.optional(args[6]), *h0 = operand.optional(args[8]), *cu = operand.optional(args[10]);
@@ -337,22 +359,21 @@ PyObject* delta_rule(PyObject*, PyObject* const* args, Py_ssize_t n) {
         s.B = size32(B), s.T = size32(T), s.H = size32(H), s.K = size32(K), s.V = size32(V), s.N = size32(N), s.chunk = 64;
         s.qk_heads = HK == H ? 0 : (int32_t)HK;
         s.cu_seqlens = static_cast<const int32_t*>(ptr(cu));
-        at::Tensor workspace;
+        uint64_t workspace_bytes = 0;
         if (chunked) {
             need(s.dtype == GDN_BF16 && one_launch_fn(&s) == 0);
-            const uint64_t bytes = workspace_bytes_fn(&s);
-            need(bytes > 0);
-            workspace = at::empty({(int64_t)bytes}, q.options().dtype(at::kByte));
-            s.workspace = ptr(workspace), s.workspace_bytes = bytes;
+            workspace_bytes = workspace_bytes_fn(&s);
+            need(workspace_bytes > 0);
         }
-        // (padding positions of a left-padded batch are not written by the kernels: they read as zeros)
-        const at::Tensor o = padded ? at::zeros({B, T, H, V}, v.options()) : fresh(v, {B, T, H, V});
-        at::Tensor ht;
-        if (output_final) {
-            if (inplace) need(h0 != nullptr), ht = *h0, s.flags |= GDN_FLAG_STATE_INPLACE;
-            else ht = at::empty({N, H, K, V}, v.options().dtype(at::kFloat));
-            s.ht = static_cast<float*>(ptr(ht));
-        }
+        at::Tensor workspace, o, ht;
+        if (output_final && inplace) need(h0 != nullptr), ht = *h0, s.flags |= GDN_FLAG_STATE_INPLACE;
+        without_interpreter_lock([&] {
+            if (chunked) workspace = at::empty({(int64_t)workspace_bytes}, q.options().dtype(at::kByte)), s.workspace = ptr(workspace), s.workspace_bytes = workspace_bytes;
+            // (padding positions of a left-padded batch are not written by the kernels: they read as zeros)
+            o = padded ? at::zeros({B, T, H, V}, v.options()) : fresh(v, {B, T, H, V});
+            if (output_final && !inplace) ht = fresh_f32(v, {N, H, K, V});
+        });
+        if (output_final) s.ht = static_cast<float*>(ptr(ht));
         s.q = ptr(q), s.k = ptr(k), s.v = ptr(v), s.beta = ptr(beta), s.o = ptr(o);
         s.g = static_cast<const float*>(ptr(g)), s.h0 = static_cast<const float*>(ptr(h0));
         s.q_stride_b = q.stride(0), s.q_stride_t = q.stride(1), s.q_stride_h = q.stride(2);
@@ -363,7 +384,7 @@ PyObject* delta_rule(PyObject*, PyObject* const* args, Py_ssize_t n) {
         THPObjectPtr results(pack_results({o, ht}));
         if (results && output_final && inplace) PyTuple_SetItem(results.get(), 1, Py_NewRef(args[8]));  // the caller's own tensor object
         return launch(chunked ? "gdn_chunk_fwd" : "gdn_recurrent_fwd", results.release(),
-                      [&] { return (chunked ? chunk_fn : recurrent_fn)(&s, stream_of(args[0])); });
+                      [&] { return (chunked ? chunk_fn : recurrent_fn)(&s, stream); });
     });
 }
 

@@ -122,3 +122,15 @@ def test_a_step_that_ends_early_gives_its_workspace_back():
         x["norm_weight"], 1e-5, 2, 2, 128, 256, None, None, "not a number", 1.0, 1,
         lambda pairs, V: (owner, owner.data_ptr(), owner.data_ptr() + 4 * pairs))  # fmt: skip
     assert result is None and sys.getrefcount(owner) == before
+
+
+@pytest.mark.parametrize("entry", ["gdn_layer_step", "gdn_causal_conv1d_fwd", "gdn_gates_fwd", "gdn_gated_rmsnorm_fwd", "gdn_recurrent_fwd",
+                                   "gdn_chunk_fwd"])  # fmt: skip
+def test_other_threads_run_while_a_call_launches(entry):
+    """The interpreter lock is free inside the library: its own question "does this thread hold it" stands in for the entry
+    point, and answers with the status 0."""
+    call = _calls()[entry]
+    call()
+    with _entry_points_replaced(**{entry: ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value}):
+        call()
+    torch.cuda.synchronize()
