@@ -187,6 +187,15 @@ def test_missing_library_fails_loudly(monkeypatch):
         _lib.load_library()
 
 
+def test_package_imports_on_a_torch_build_without_gpu_support():
+    code = ("import torch; del torch._C._cuda_getCurrentRawStream\n"
+            "import lm_engine_amd, oracle; x = torch.zeros(1, 8, 2, 64, dtype=torch.bfloat16)\n"
+            "try: lm_engine_amd.chunk_gated_delta_rule(x, x, x)\n"
+            "except ValueError as e: print(e)")  # fmt: skip
+    run = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert run.returncode == 0 and "GPU only" in run.stdout, run.stderr
+
+
 def test_kernel_flag_registry_follows_the_reference_convention():
     assert is_kernel_allowed(Kernel.gated_delta_rule)
     with enable_kernels([], reset=True):
