@@ -24,7 +24,9 @@
 extern "C" {
 #endif
 
-#define GDN_ABI_VERSION 2
+/* 3: gdn_chunk_saves.packed_records, gdn_chunk_local_args.out_stride_t and gdn_chunk_bwd_prepare_args.records_fwd_slots are read
+ * (fields named `reserved` before).  Zero a struct before filling it: a later version may read what is reserved in this one. */
+#define GDN_ABI_VERSION 3
 
 typedef enum gdn_dtype { GDN_BF16 = 0, GDN_F32 = 1 } gdn_dtype;
 

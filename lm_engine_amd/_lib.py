@@ -10,7 +10,7 @@ import ctypes
 import os
 
 
-GDN_ABI_VERSION = 2
+GDN_ABI_VERSION = 3
 
 GDN_BF16 = 0
 GDN_F32 = 1

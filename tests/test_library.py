@@ -3,6 +3,7 @@ declares, agrees with the ctypes mirror of the argument struct, and rejects bad 
 before anything is launched."""
 
 import ctypes
+import hashlib
 import os
 import re
 import subprocess
@@ -62,6 +63,20 @@ def test_struct_layout_matches_the_header():
                       A.B.offset, A.flags.offset, A.scale.offset, A.spin_limit.offset, A.error_word.offset,
                       ctypes.sizeof(Cv), Cv.final_state.offset, Cv.x_stride_b.offset, Cv.B.offset,
                       Cv.activation.offset]  # fmt: skip
+
+
+# sha256 (16 digits) of the header's structs without comments, by the version that they had
+STRUCTS_OF_VERSION = {2: "7652088ae5119dd4", 3: "19be2afcc6940cb1"}
+
+
+def test_a_change_of_the_structs_comes_with_a_new_version():
+    """A caller built against an older header is told so by the version: also where a reserved field became one that is read
+    (callers were not asked to clear it)."""
+    text = re.sub(r"/\*.*?\*/", "", open(HEADER).read(), flags=re.S)
+    structs = re.findall(r"typedef struct \w+ \{.*?\} \w+;", text, flags=re.S)
+    digest = hashlib.sha256(" ".join(" ".join(structs).split()).encode()).hexdigest()[:16]
+    version = int(re.search(r"#define GDN_ABI_VERSION (\d+)", text).group(1))
+    assert STRUCTS_OF_VERSION.get(version) == digest, f"version {version}: structs {digest}"
 
 
 def test_layer_ops_reject_bad_arguments_before_any_launch():
