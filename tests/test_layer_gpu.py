@@ -142,31 +142,47 @@ def _mix_step(qkv, ab, p, HK, HV, DK, DV, cache, gate=True, neg=True):
         1e-5, HK, HV, DK, DV, cache=cache, allow_neg_eigval=neg)  # fmt: skip
 
 
+def _watched_host(monkeypatch, step):
+    """Puts a recorder in front of the native host path of the layer; ``step`` False: without its one-launch step.  Returns
+    the list of what the step answered (None: it left the call to the chain of kernels)."""
+    from lm_engine_amd import layer
+    from lm_engine_amd._host import host
+
+    answers = []
+
+    class Watched:
+        def __getattr__(self, name):
+            if name != "layer_step":
+                return getattr(host(), name)
+
+            def layer_step(*args):
+                answers.append(host().layer_step(*args) if step else None)
+                return answers[-1]
+
+            return layer_step
+
+    monkeypatch.setattr(layer, "host", lambda: Watched())
+    return answers
+
+
 # one tile per head (V = 32, 64, 128), tiles of 32, 64 and 128 columns that share a norm through tickets, shared heads of
 # q and k, a projection whose gate slice starts off every 16-byte boundary (HV = 1, 2, 3), first token (no state yet)
 @pytest.mark.parametrize("dtype", [BF16, torch.float32])
 @pytest.mark.parametrize("B, HK, HV, DK, DV", [(1, 4, 4, 64, 32), (3, 2, 4, 128, 64), (5, 1, 3, 256, 128), (2, 2, 2, 128, 96),
                                                (2, 2, 2, 256, 512), (3, 1, 2, 64, 192), (70, 2, 2, 128, 256)])  # fmt: skip
 def test_one_launch_step_matches_the_chain_of_kernels(B, HK, HV, DK, DV, dtype, monkeypatch):
-    from lm_engine_amd import layer
-    from lm_engine_amd._host import host
-
     qkv, ab, p, cache = _step_operands(B, HK, HV, DK, DV, dtype, seed=B + DV)
     print(f"case: layer step B={B} heads {HK}/{HV} dims {DK}/{DV} {dtype}", flush=True)
-
-    class WithoutTheStep:
-        def __getattr__(self, name):
-            return (lambda *args: None) if name == "layer_step" else getattr(host(), name)
 
     for gate, start in ((True, cache), (False, cache), (True, (None, None))):
         chained = {}
         for name in ("step", "chain"):
             with monkeypatch.context() as m:
-                if name == "chain":
-                    m.setattr(layer, "host", lambda: WithoutTheStep())
+                answers = _watched_host(m, step=name == "step")
                 out, c1 = _mix_step(qkv, ab, p, HK, HV, DK, DV, start, gate=gate)
                 out2, c2 = _mix_step(qkv, ab, p, HK, HV, DK, DV, c1, gate=gate)  # on the state the first one left
                 chained[name] = (out, *c1, out2, *c2)
+            assert [x is not None for x in answers] == [name == "step"] * 2, "the kernel under test did not run"
         for name, x, y in zip(("out", "conv", "h", "out2", "conv2", "h2"), chained["step"], chained["chain"]):
             if name.startswith("out"):  # the norm adds its V squares up in another order: at most an ulp of the result
                 assert rel_l2(x, y) <= (1e-3 if dtype == BF16 else 1e-6), (name, rel_l2(x, y))
@@ -174,7 +190,8 @@ def test_one_launch_step_matches_the_chain_of_kernels(B, HK, HV, DK, DV, dtype, 
                 assert torch.equal(x, y), name
 
 
-def test_one_launch_step_under_graph_capture():
+def test_one_launch_step_under_graph_capture(monkeypatch):
+    answers = _watched_host(monkeypatch, step=True)
     HK, HV, DK, DV = 2, 2, 128, 256  # several workgroups per head: tickets in memory of the graph's own
     qkv, ab, p, cache = _step_operands(5, HK, HV, DK, DV, BF16, seed=9)
     with torch.no_grad():
@@ -189,3 +206,4 @@ def test_one_launch_step_under_graph_capture():
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, want) and torch.equal(conv, conv_want) and torch.equal(h, h_want)
+    assert len(answers) == 6 and all(x is not None for x in answers), "the kernel under test did not run"
