@@ -91,20 +91,24 @@ struct TokenNorms {
 };
 template <int KPL>
 __device__ __forceinline__ TokenNorms token_norms(const float (&kx)[KPL], const float (&qx)[KPL], bool l2norm, float scale) {
+    const float q_scale = l2norm ? 1.f : scale;  // of the product below, so that without norms it overflows where k^ . q^ does
     float ssk = 0.f, ssq = 0.f, dot = 0.f;
 #pragma unroll
     for (int e = 0; e < KPL; e++) {
         ssk = fmaf(kx[e], kx[e], ssk);
         ssq = fmaf(qx[e], qx[e], ssq);
-        dot = fmaf(kx[e], qx[e], dot);
+        dot = fmaf(kx[e], qx[e] * q_scale, dot);
     }
     TokenNorms r;
     r.kn = 1.f, r.qn = scale;
+    r.kq = wave_total(dot);
     if (l2norm) {
         r.kn = rsqrtf(wave_total(ssk) + L2NORM_EPS);
         r.qn = rsqrtf(wave_total(ssq) + L2NORM_EPS) * scale;
+        // k . q of finite rows overflows only if a sum of squares does; that row's k^ or q^ is 0 then, and so is k^ . q^
+        // (0 times the overflowed product would be a NaN)
+        r.kq = r.kn == 0.f || r.qn == 0.f ? 0.f : r.kq * r.kn * r.qn;
     }
-    r.kq = wave_total(dot) * r.kn * r.qn;
     return r;
 }
 

@@ -207,3 +207,19 @@ def test_one_launch_step_under_graph_capture(monkeypatch):
             torch.cuda.synchronize()
             assert torch.equal(out, want) and torch.equal(conv, conv_want) and torch.equal(h, h_want)
     assert len(answers) == 6 and all(x is not None for x in answers), "the kernel under test did not run"
+
+
+def test_step_of_rows_whose_norm_overflows_is_that_of_zero_rows(monkeypatch):
+    """Finite rows of q and k whose sum of squares is infinite have k^ = q^ = 0: no NaN from k . q."""
+    HK, HV, DK, DV = 2, 2, 128, 64
+    qkv, ab, p, (_, h) = _step_operands(3, HK, HV, DK, DV, BF16, seed=12)
+    p["conv_weight"], p["conv_bias"] = p["conv_weight"].abs(), None
+    answers = _watched_host(monkeypatch, step=True)
+    outs = []
+    for value in (1e25, 0.0):
+        x = qkv.clone()
+        x[..., : 2 * HK * DK] = value
+        out, (_, h_new) = _mix_step(x, ab, p, HK, HV, DK, DV, (None, h))
+        outs.append((out, h_new))
+    assert len(answers) == 2 and all(x is not None for x in answers)
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1]) and torch.isfinite(outs[0][1]).all()

@@ -180,3 +180,27 @@ def test_inplace_state_is_refused_when_gradients_are_needed():
     inp["v"].requires_grad_(True)
     with pytest.raises(ValueError, match="inplace_state"):
         lm_engine_amd.fused_recurrent_gated_delta_rule(**inp, output_final_state=True, inplace_state=True)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("T, magnitude", [(1, 1e25), (1, 3e19), (40, 1e25)])
+def test_rows_whose_norm_overflows_count_as_zero_rows(dtype, T, magnitude):
+    """x / sqrt(sum x^2 + eps) of a finite row whose sum of squares is infinite is 0 in fp32: such rows of q and k give the
+    bits that rows of zeros give, one token or several, and no NaN."""
+    inp = _to_gpu(random_inputs(B=2, T=T, H=2, K=128, V=64, dtype=dtype, seed=71, normalize=False))
+    huge, zero = dict(inp), dict(inp)
+    for n in ("q", "k"):
+        huge[n], zero[n] = inp[n].clone(), inp[n].clone()
+        huge[n][:, T // 2] = inp[n][:, T // 2].sign() * magnitude
+        zero[n][:, T // 2] = 0
+    run = lambda x: lm_engine_amd.fused_recurrent_gated_delta_rule(**x, output_final_state=True, use_qk_l2norm_in_kernel=True)  # noqa: E731
+    (o, h), (o_zero, h_zero) = run(huge), run(zero)
+    assert torch.equal(o, o_zero) and torch.equal(h, h_zero) and torch.isfinite(h).all()
+
+
+def test_products_of_unnormalised_rows_overflow_only_where_the_result_does():
+    """Without l2norm the scale is applied to q before k . q is formed: 2e38 and not infinity times a tenth."""
+    z = torch.zeros(1, 1, 1, 64).cuda()
+    k, q, v = z + 2e19, z + 2e19, z + 1e-30  # k . q = 64 * 4e38
+    o, _ = lm_engine_amd.fused_recurrent_gated_delta_rule(q, k, v, scale=1e-3)
+    assert torch.isfinite(o).all() and abs(o.mean().item() / (64 * 4e38 * 1e-3 * 1e-30) - 1) <= 1e-5
