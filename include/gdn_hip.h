@@ -188,6 +188,16 @@ int gdn_chunk_fwd_noalloc(const gdn_args *args, void *stream);
 int gdn_recurrent_fwd(const gdn_args *args, void *stream);
 
 /*
+ * The kernels that gdn_recurrent_fwd would run these arguments on, GDN_RECURRENT_* or both (every packed sequence then runs on
+ * the one for its length).  Reads the shape fields, the flags and whether cu_seqlens is NULL; no pointer is followed.
+ */
+enum {
+    GDN_RECURRENT_STEP = 1,   /* streams every state through registers once: decoding, a few tokens over many states */
+    GDN_RECURRENT_TOKENS = 2, /* for longer sequences: the shortest chain from a token's state to the next */
+};
+int gdn_recurrent_fwd_kernels(const gdn_args *args);
+
+/*
  * Training support.  The reference differentiates through chunk_gated_delta_rule (chunk mode is asserted
  * while training, gated_deltanet/module.py:194-209); a backward pass needs the state every chunk starts
  * from and the chunk's V~ (the values written into the state), which gdn_chunk_fwd does not keep.

@@ -45,6 +45,7 @@ EXPORTED_SYMBOLS = (
     "gdn_chunk_fwd_is_one_launch",
     "gdn_chunk_fwd_noalloc",
     "gdn_recurrent_fwd",
+    "gdn_recurrent_fwd_kernels",
     "gdn_chunk_fwd_profile",
     "gdn_chunk_fwd_saving",
     "gdn_chunk_fwd_saving_is_staged",
@@ -238,6 +239,8 @@ def load_library() -> ctypes.CDLL:
     lib.gdn_workspace_header_bytes.restype = ctypes.c_uint64
     lib.gdn_chunk_fwd.argtypes = [ctypes.POINTER(GdnArgs), ctypes.c_void_p]
     lib.gdn_chunk_fwd.restype = ctypes.c_int
+    lib.gdn_recurrent_fwd_kernels.argtypes = [ctypes.POINTER(GdnArgs)]
+    lib.gdn_recurrent_fwd_kernels.restype = ctypes.c_int
     lib.gdn_chunk_fwd_is_one_launch.argtypes = [ctypes.POINTER(GdnArgs)]
     lib.gdn_chunk_fwd_is_one_launch.restype = ctypes.c_int
     lib.gdn_chunk_fwd_status.argtypes = [ctypes.POINTER(GdnArgs), ctypes.c_void_p]

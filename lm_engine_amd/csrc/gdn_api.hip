@@ -129,6 +129,8 @@ int gdn_recurrent_fwd(const gdn_args* a, void* stream) {
     return gdn::launch_recurrent(*a, static_cast<hipStream_t>(stream));
 }
 
+int gdn_recurrent_fwd_kernels(const gdn_args* a) { return a == nullptr ? 0 : gdn::recurrent_kernels(*a); }
+
 static int validate_chunk(const gdn_args* a) {
     const int rc = validate_common(a);
     if (rc != GDN_OK) return rc;

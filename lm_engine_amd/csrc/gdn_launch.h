@@ -22,6 +22,7 @@ inline int compute_units() {
 
 // Arguments are validated by the caller (gdn_api.hip); these only pick an instantiation and launch.
 int launch_recurrent(const gdn_args& a, hipStream_t stream);
+int recurrent_kernels(const gdn_args& a);  // gdn_recurrent_fwd_kernels: shape fields, the left-padded flag and whether cu_seqlens is NULL
 // `events`, when not null, holds GDN_CHUNK_KERNELS + 1 events recorded around the kernels.
 // `saves`, when not null, selects the state-saving scan (see gdn_chunk_fwd_saving).
 int launch_chunk_fwd(const gdn_args& a, hipStream_t stream, hipEvent_t* events = nullptr, const gdn_chunk_saves* saves = nullptr);

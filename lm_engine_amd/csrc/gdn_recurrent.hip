@@ -39,6 +39,7 @@ __global__ __launch_bounds__(4 * BV) void recurrent_step_kernel(const RecurrentP
     if (p.cu_seqlens != nullptr) {
         int t0, len;
         packed_bounds(p.cu_seqlens, n, p.T, t0, len);
+        if (len < p.len_min || len > p.len_max) return;  // the other kernel's (the whole workgroup)
         b = 0, t_begin = t0, t_end = t0 + len;
     }
     const int64_t hqk = p.qk_div > 1 ? h / p.qk_div : h;
@@ -129,6 +130,7 @@ __global__ __launch_bounds__(REC_THREADS) void recurrent_tokens_kernel(const Rec
     if (p.cu_seqlens != nullptr) {
         int t0, len;
         packed_bounds(p.cu_seqlens, n, p.T, t0, len);
+        if (len < p.len_min || len > p.len_max) return;  // the other kernel's (the whole workgroup)
         b = 0, t_begin = t0, t_end = t0 + len;
     }
 
@@ -262,33 +264,66 @@ static int launch_recurrent_step(const RecurrentParams& p, int N, hipStream_t st
     return (int)hipGetLastError();
 }
 
+// Which kernels a call runs on.  One token per sequence, or a few over many states: the step kernel.  The tokens kernel's
+// lanes take the state in 16-byte pieces of many rows, which costs more than its shorter chain wins there (B = 64, H = 16,
+// V = 128: T = 2 28 against 44 us, T = 16 77 against 72 us).
+// Packed sequences differ in length, and T is the tokens of all of them.  No more tokens than sequences is decoding: the step
+// kernel (32 heads, K = V = 128, 256 x 1 token: 163 us, 328 on the tokens kernel).  Else, where there are many states and the
+// sequences are short on average, each kernel takes the sequences of its lengths, in a launch of its own.  Split | tokens
+// kernel alone: 32 heads, 256 x 4 tokens 210 | 332 us, 255 x 1 and 1 x 256 tokens 325 | 489 us (490 on the step kernel alone);
+// 16 heads, 64 x 16 tokens 71 | 68 us, 63 x 1 and 1 x 200 tokens 145 | 154 us (256).  With few states the second launch is no
+// longer small next to the work (16 heads, 4 x 3 tokens: 9 us on the tokens kernel).
+constexpr int STEP_TOKENS = 12;                    // fixed-length calls of fewer run on the step kernel where there are many states
+constexpr int SPLIT_TOKENS = 17;                   // so do the sequences of a split call: at 16 the kernels are still nearly even
+constexpr int64_t SPLIT_STATE = (int64_t)1 << 23;  // elements of all states together
+constexpr int SPLIT_MEAN = 48;                     // mean length from which the short sequences are few
+
+int recurrent_kernels(const gdn_args& a) {
+    const bool few_tokens = a.T < STEP_TOKENS && (int64_t)a.N * a.H * a.V >= 256 * 256;
+    if (a.T <= 1 || few_tokens) return GDN_RECURRENT_STEP;
+    if (a.cu_seqlens == nullptr || (a.flags & GDN_FLAG_LEFT_PADDED)) return GDN_RECURRENT_TOKENS;
+    if (a.T <= a.N) return GDN_RECURRENT_STEP;
+    if ((int64_t)a.N * a.H * a.K * a.V >= SPLIT_STATE && a.T < (int64_t)SPLIT_MEAN * a.N) return GDN_RECURRENT_STEP | GDN_RECURRENT_TOKENS;
+    return GDN_RECURRENT_TOKENS;
+}
+
 template <typename T, int K>
-static int launch_recurrent_k(const RecurrentParams& p, int N, hipStream_t stream) {
+static int launch_recurrent_tokens_k(const RecurrentParams& p, int N, hipStream_t stream) {
     const int64_t pairs = (int64_t)N * p.H;
-    // The tokens kernel: as few columns per lane as leave at most 1024 workgroups (four per CU, what LDS and registers hold at
-    // a time).  Measured with 1 | 2 | 4: B = 5, T = 60, H = 16, K = V = 128 (640 workgroups at 1) 36 | 38 | 41 us, B = 5, T = 33,
-    // H = 32, V = 256 (2560) 60 | 55 | 58 us, B = 64, T = 16, H = 16, V = 128 (8192) 100 | 83 | 72 us.  Its lanes take the state
-    // in 16-byte pieces of many rows, which costs more than its shorter chain wins where a large batch meets a few tokens:
-    // there the step kernel walks over the tokens (B = 64, H = 16, V = 128: T = 2 28 against 44 us, T = 16 77 against 72 us).
-    if (p.T > 1 && !(p.T < 12 && pairs * p.V >= 256 * 256)) {
-        if (pairs * (p.V / 16) <= 1024) return launch_recurrent_tokens<T, K, 1>(p, N, stream);
-        if (pairs * (p.V / 32) <= 2048 || p.V % 64 != 0) return launch_recurrent_tokens<T, K, 2>(p, N, stream);
-        return launch_recurrent_tokens<T, K, 4>(p, N, stream);
-    }
-    // The step kernel: wide tiles give the longest contiguous rows (256 sequences x 32 heads, K = V = 128: 164 us with 128
-    // columns, 185 with 64, 202 with 32), narrow ones more workgroups when there are few (sequence, head) pairs (1 x 16:
-    // 4.3, 3.8, 3.6 us).
+    // As few columns per lane as leave at most 1024 workgroups (at K <= 128 four per CU, what LDS and registers hold at a
+    // time).  Measured with 1 | 2 | 4: B = 5, T = 60, H = 16, K = V = 128 (640 workgroups at 1) 36 | 38 | 41 us, B = 5, T = 33,
+    // H = 32, V = 256 (2560) 60 | 55 | 58 us, B = 64, T = 16, H = 16, V = 128 (8192) 100 | 83 | 72 us.
+    if (pairs * (p.V / 16) <= 1024) return launch_recurrent_tokens<T, K, 1>(p, N, stream);
+    if (pairs * (p.V / 32) <= 2048 || p.V % 64 != 0) return launch_recurrent_tokens<T, K, 2>(p, N, stream);
+    return launch_recurrent_tokens<T, K, 4>(p, N, stream);
+}
+
+template <typename T, int K>
+static int launch_recurrent_step_k(const RecurrentParams& p, int N, hipStream_t stream) {
+    const int64_t pairs = (int64_t)N * p.H;
+    // Wide tiles give the longest contiguous rows (256 sequences x 32 heads, K = V = 128: 164 us with 128 columns, 185 with
+    // 64, 202 with 32), narrow ones more workgroups when there are few (sequence, head) pairs (1 x 16: 4.3, 3.8, 3.6 us).
     if (p.V % 128 == 0 && pairs * (p.V / 128) >= 256) return launch_recurrent_step<T, K, 128>(p, N, stream);
     if (p.V % 64 == 0 && pairs * (p.V / 64) >= 512) return launch_recurrent_step<T, K, 64>(p, N, stream);
     return launch_recurrent_step<T, K, 32>(p, N, stream);
 }
 
+template <typename T, int K>
+static int launch_recurrent_k(RecurrentParams p, int N, int kernels, hipStream_t stream) {
+    if (kernels == GDN_RECURRENT_TOKENS) return launch_recurrent_tokens_k<T, K>(p, N, stream);
+    if (kernels == GDN_RECURRENT_STEP) return launch_recurrent_step_k<T, K>(p, N, stream);
+    p.len_max = SPLIT_TOKENS - 1;
+    if (const int status = launch_recurrent_step_k<T, K>(p, N, stream); status != 0) return status;
+    p.len_min = SPLIT_TOKENS, p.len_max = INT32_MAX;
+    return launch_recurrent_tokens_k<T, K>(p, N, stream);
+}
+
 template <typename T>
-static int launch_recurrent_t(const RecurrentParams& p, int K, int N, hipStream_t stream) {
+static int launch_recurrent_t(const RecurrentParams& p, int K, int N, int kernels, hipStream_t stream) {
     switch (K) {
-        case 64: return launch_recurrent_k<T, 64>(p, N, stream);
-        case 128: return launch_recurrent_k<T, 128>(p, N, stream);
-        case 256: return launch_recurrent_k<T, 256>(p, N, stream);
+        case 64: return launch_recurrent_k<T, 64>(p, N, kernels, stream);
+        case 128: return launch_recurrent_k<T, 128>(p, N, kernels, stream);
+        case 256: return launch_recurrent_k<T, 256>(p, N, kernels, stream);
         default: return GDN_ERR_UNSUPPORTED;
     }
 }
@@ -314,8 +349,9 @@ int launch_recurrent(const gdn_args& a, hipStream_t stream) {
     p.beta_dtype = a.beta_dtype;
     p.l2norm = (a.flags & GDN_FLAG_L2NORM) ? 1 : 0;
     p.scale = a.scale;
-    if (a.dtype == GDN_BF16) return launch_recurrent_t<bf16_t>(p, a.K, a.N, stream);
-    if (a.dtype == GDN_F32) return launch_recurrent_t<float>(p, a.K, a.N, stream);
+    const int kernels = recurrent_kernels(a);
+    if (a.dtype == GDN_BF16) return launch_recurrent_t<bf16_t>(p, a.K, a.N, kernels, stream);
+    if (a.dtype == GDN_F32) return launch_recurrent_t<float>(p, a.K, a.N, kernels, stream);
     return GDN_ERR_UNSUPPORTED;
 }
 

@@ -25,6 +25,7 @@ struct RecurrentParams {
     int64_t v_stride_b, v_stride_t, v_stride_h;
     int64_t o_stride_b, o_stride_t, o_stride_h;
     int T, H, V;
+    int len_min = 0, len_max = INT32_MAX;  // packed sequences: the lengths that this launch takes
     int qk_div;  // value heads per head of q and k
     int beta_dtype;
     int l2norm;

@@ -170,6 +170,28 @@ def test_bad_arguments_are_rejected_before_launch(over, status):
     assert _lib.strerror(status) != "unknown gdn status"
 
 
+STEP, TOKENS = 1, 2
+
+
+@pytest.mark.parametrize(
+    "over, kernels",
+    [
+        # fixed-length batches and rows of a left-padded one: T tokens each
+        (dict(T=1), STEP), (dict(T=2), TOKENS), (dict(T=11, B=256, N=256, H=32, V=128), STEP), (dict(T=12, B=256, N=256, H=32, V=128), TOKENS),
+        (dict(T=40, B=40, N=40, cu_seqlens=0x2000, flags=_lib.GDN_FLAG_LEFT_PADDED), TOKENS),
+        # packed: T is the tokens of all sequences
+        (dict(T=256, N=256, cu_seqlens=0x2000), STEP), (dict(T=12, N=12, cu_seqlens=0x2000), STEP), (dict(T=12, N=20, cu_seqlens=0x2000), STEP),
+        (dict(T=257, N=256, H=32, K=128, V=128, cu_seqlens=0x2000), STEP | TOKENS),
+        (dict(T=256 * 48 - 1, N=256, H=32, K=128, V=128, cu_seqlens=0x2000), STEP | TOKENS),
+        (dict(T=256 * 48, N=256, H=32, K=128, V=128, cu_seqlens=0x2000), TOKENS),
+        (dict(T=12, N=4, H=16, K=128, V=128, cu_seqlens=0x2000), TOKENS),  # few states
+        (dict(T=5000, N=4, H=16, K=128, V=128, cu_seqlens=0x2000), TOKENS),
+    ],
+)  # fmt: skip
+def test_kernels_of_the_recurrent_forward_by_tokens_per_sequence(over, kernels):
+    assert _lib.load_library().gdn_recurrent_fwd_kernels(ctypes.byref(_args(**over))) == kernels
+
+
 def test_chunk_fwd_needs_a_workspace():
     lib = _lib.load_library()
     a = _args(T=128, K=128, V=128, q_stride_h=128, k_stride_h=128, v_stride_h=128, o_stride_h=128,

@@ -204,3 +204,28 @@ def test_products_of_unnormalised_rows_overflow_only_where_the_result_does():
     k, q, v = z + 2e19, z + 2e19, z + 1e-30  # k . q = 64 * 4e38
     o, _ = lm_engine_amd.fused_recurrent_gated_delta_rule(q, k, v, scale=1e-3)
     assert torch.isfinite(o).all() and abs(o.mean().item() / (64 * 4e38 * 1e-3 * 1e-30) - 1) <= 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("inplace", [False, True])
+@pytest.mark.parametrize("lens", [[1] * 70, [1] * 30 + [0, 1, 2, 12, 15, 16, 0, 17, 18, 40] + [3] * 25, [0] * 40 + [64] * 24])
+def test_packed_sequences_get_the_bits_of_single_ones_on_either_kernel(lens, inplace, dtype):
+    """Decoding (one token each), lengths on both sides of the border between the kernels of one call, empty sequences."""
+    H, K, V = 32, 64, 64
+    N, T = len(lens), sum(lens)
+    gpu = _to_gpu(random_inputs(B=1, T=T, H=H, K=K, V=V, dtype=dtype, seed=83, normalize=False, N=N))
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+    h0 = gpu.pop("initial_state")
+    own = h0.clone()
+    run = lambda x, h, **kw: lm_engine_amd.fused_recurrent_gated_delta_rule(  # noqa: E731
+        **x, initial_state=h, output_final_state=True, use_qk_l2norm_in_kernel=True, **kw)
+    o, ht = run(gpu, own, cu_seqlens=cu, inplace_state=inplace)
+    assert (ht is own) == inplace and (inplace or torch.equal(own, h0))
+    begin = 0
+    for n, length in enumerate(lens):
+        want_h = h0[n : n + 1]
+        if length > 0:
+            want_o, want_h = run({name: x[:, begin : begin + length] for name, x in gpu.items()}, want_h)
+            assert torch.equal(o[:, begin : begin + length], want_o), n
+        assert torch.equal(ht[n : n + 1], want_h), n
+        begin += length
