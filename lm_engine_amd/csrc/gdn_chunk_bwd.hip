@@ -962,7 +962,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 64 ? 3 : 2)) void chunk_bwd_prep
     __shared__ __attribute__((aligned(16))) bf16_t sQK[QK_ELEMS];   // rows of q, of k; then slabs of dO; then the scratch of the inverse
     __shared__ __attribute__((aligned(16))) bf16_t sPT[C * LDS64];     // P^T
     __shared__ __attribute__((aligned(16))) float sA[C * LDA];         // A, then T in its place
-    __shared__ float s_gam[C], s_beta[C], s_e[C], s_tail[C], s_rq[C], s_rk[C];
+    __shared__ __attribute__((aligned(16))) float s_gam[C], s_beta[C], s_e[C], s_tail[C], s_rq[C], s_rk[C];
     bf16_t* const sQ = sQK;
     bf16_t* const sK = sQK + C * LDQ;
     bf16_t* const sDO = sQK;  // [64][VS + 8]
@@ -1079,19 +1079,14 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 64 ? 3 : 2)) void chunk_bwd_prep
                     s_rq[row] = rq, s_rk[row] = rk;
                     p.rq[chunk * C + row] = rq, p.rk[chunk * C + row] = rk;
                 }
-                bf16x8 qb, kb;
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    qb[e] = (bf16_t)((float)qr[e] * rq * p.scale);
-                    kb[e] = (bf16_t)((float)kr[e] * rk);
-                }
+                // the rows as they are: norms and scale go onto the fp32 sums below, as in the forward's prepare step
                 if constexpr (QH) {
-                    qn[it] = qb;  // scaled; the pieces of the second half are written after the first half's products
-                    if (p8 < CPR / 2) *reinterpret_cast<bf16x8*>(sQ + row * LDQ + 8 * p8) = qb;
+                    qn[it] = qr;  // (the pieces of the second half are written after the first half's products)
+                    if (p8 < CPR / 2) *reinterpret_cast<bf16x8*>(sQ + row * LDQ + 8 * p8) = qr;
                 } else {
-                    *reinterpret_cast<bf16x8*>(sQ + row * LDQ + 8 * p8) = qb;
+                    *reinterpret_cast<bf16x8*>(sQ + row * LDQ + 8 * p8) = qr;
                 }
-                *reinterpret_cast<bf16x8*>(sK + row * LDK + 8 * p8) = kb;
+                *reinterpret_cast<bf16x8*>(sK + row * LDK + 8 * p8) = kr;
                 // mirror rows: k of chunk A is k, k of chunk B is q
                 if (copies) {
                     const int64_t tokA = tok_a(row), tokB = tokA + (int64_t)C * p.H;
@@ -1122,13 +1117,19 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 64 ? 3 : 2)) void chunk_bwd_prep
                 QK = mma_nt(sQ + 32 * ti * LDQ, LDQ, sK + 32 * tj * LDK + K / 2, LDK, K / 2, QK, l32, lh);
             }
             const int j = 32 * tj + l32;
-            const float gj = s_gam[j];
+            const float gj = s_gam[j], rkj = s_rk[j];
 #pragma unroll
-            for (int r = 0; r < 16; r++) {
-                const int i = 32 * ti + 8 * (r / 4) + 4 * lh + r % 4;
-                const float E = i >= j ? __expf(s_gam[i] - gj) : 0.f;
-                sA[i * LDA + j] = i > j ? s_beta[i] * E * KK[r] : 0.f;
-                sPT[j * LDS64 + i] = (bf16_t)(E * QK[r]);
+            for (int r4 = 0; r4 < 4; r4++) {
+                const int i0 = 32 * ti + 8 * r4 + 4 * lh;  // rows i0 .. i0 + 3: their per-token values in one read each
+                const f32x4 gi = *reinterpret_cast<const f32x4*>(&s_gam[i0]), bi = *reinterpret_cast<const f32x4*>(&s_beta[i0]);
+                const f32x4 rki = *reinterpret_cast<const f32x4*>(&s_rk[i0]), rqi = *reinterpret_cast<const f32x4*>(&s_rq[i0]);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int i = i0 + e;
+                    const float E = i >= j ? __expf(gi[e] - gj) : 0.f;
+                    sA[i * LDA + j] = i > j ? bi[e] * rki[e] * E * (rkj * KK[4 * r4 + e]) : 0.f;
+                    sPT[j * LDS64 + i] = (bf16_t)(p.scale * rqi[e] * E * (rkj * QK[4 * r4 + e]));
+                }
             }
         }
         __syncthreads();  // the rows of q and k are dead

@@ -564,3 +564,53 @@ def test_packed_gradients_match_those_of_single_sequences(lens, tail, K):
     for g in got:
         assert not g[:, covered:].any(), "tokens that belong to no sequence"
     _assert_grads([g.cpu() for g in got], [g.cpu() for g in want], torch.bfloat16)
+
+
+@pytest.mark.parametrize("lens", [None, [130, 0, 64, 7]])
+@pytest.mark.parametrize("K", [64, 128, 256])
+@pytest.mark.parametrize("l2norm", [True, False])
+def test_forward_records_are_exact_up_to_their_own_rounding(lens, K, l2norm):
+    """T diag(beta) and P that the backward's prepare kernel writes for the forward sweep, against the same matrices in fp64
+    from the same bf16 rows: as far off as their rounding to bf16 alone, within 5 % (fp32 sums, a thousandth of a bf16 unit
+    each).  Rows that are rounded once more after their norm was applied are 1.7 times as far off."""
+    from lm_engine_amd import ops
+
+    H, V = 2, 64
+    T = 256 if lens is None else sum(lens)
+    inp = random_inputs(B=1, T=T, H=H, K=K, V=V, dtype=torch.bfloat16, seed=K, normalize=not l2norm, beta_max=2.0)
+    q, k, v, g, beta = (inp[n].cuda() for n in ("q", "k", "v", "g", "beta"))
+    scale = K**-0.5
+    if lens is None:
+        chains, sequences, packed = [(64 * c, 64) for c in range(4)], None, False
+    else:
+        starts = [sum(lens[:n]) for n in range(len(lens))]
+        sequences, packed = (*ops.upload_int32((starts, lens), q.device), -(-max(lens) // 64)), True
+        chains = [(s + c, min(64, n - c)) for s, n in zip(starts, lens) for c in range(0, n, 64)]
+    prep = ops.chunk_bwd_prepare(q, k, v, g, beta, scale, l2norm, V, sequences, half_slice_records=True, forward_records=True, packed=packed)
+    slots = T // 64 + (len(lens) if packed else 0)
+    records = (prep["workspace_fwd"][-H * slots * ops.RECORD_BYTES :] if packed else prep["records_fwd"]).view(H, slots, -1).cpu()
+
+    # fragment f, lane L, element e of the 16x16x32 order -> row, column
+    f, lane, e = torch.meshgrid(torch.arange(6), torch.arange(64), torch.arange(8), indexing="ij")
+    row = 16 * torch.where(f < 2, f, 2 + (f - 2) // 2) + lane % 16
+    col = 32 * torch.where(f < 2, 0, f % 2) + 4 * (lane // 16) + torch.where(e < 4, e, e + 12)
+    lower = (row > col).double()
+    rounded, error = {"T": 0.0, "P": 0.0}, {"T": 0.0, "P": 0.0}
+    for slot, (first, count) in enumerate(chains):
+        for h in range(H):
+            rows = lambda x: torch.nn.functional.pad(x[0, first : first + count, h].double().cpu(), (0, 0, 0, 64 - count))  # noqa: E731
+            one = lambda x: torch.nn.functional.pad(x[0, first : first + count, h].double().cpu(), (0, 64 - count))  # noqa: E731
+            norm = lambda x: x * torch.rsqrt((x * x).sum(-1, keepdim=True) + 1e-6) if l2norm else x  # noqa: E731
+            qn, kn, gam, b = norm(rows(q)) * scale, norm(rows(k)), one(g).cumsum(0), one(beta)
+            decay = (gam[:, None] - gam[None, :]).exp()
+            A = (b[:, None] * decay * (kn @ kn.T)).tril(-1)
+            exact = {"T": torch.linalg.inv(torch.eye(64).double() + A) * b[None, :], "P": (decay * (qn @ kn.T)).tril()}
+            fragments = records[h, slot, : 2 * 6144].view(torch.bfloat16).view(2, 6, 64, 8).double()
+            for part, name in enumerate(("T", "P")):
+                want = exact[name][row, col] * lower
+                error[name] += (fragments[part] * lower - want).square().sum().item()
+                rounded[name] += (want.to(torch.bfloat16).double() - want).square().sum().item()
+    for name in ("T", "P"):
+        ratio = (error[name] / rounded[name]) ** 0.5
+        print(f"   {name}: error / rounding {ratio:.3f}", flush=True)
+        assert ratio <= 1.05, name
