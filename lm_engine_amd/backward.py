@@ -338,11 +338,11 @@ def _chunk_local_grads(qs, kn, vc, doc, Y, Vn, S0, dS1, gam, bc):
 
 def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm, cu_seqlens, left_padded, joined):
     """The whole backward on four kernel launches (bf16; K = 64, 128 or 256; V a multiple of 64): ``gdn_chunk_bwd_prepare``
-    (per-chunk scalars, the mirror problem, and for whole-chunk batches the forward sweep's records), the saving
-    forward sweep, the saving scan over the mirror problem (reverse sweep), ``gdn_chunk_bwd_local`` writing the
+    (per-chunk scalars, the mirror problem, and for whole-chunk batches and packed sequences the forward sweep's records),
+    the saving forward sweep, the saving scan over the mirror problem (reverse sweep), ``gdn_chunk_bwd_local`` writing the
     gradients in the caller's layout.  Chunk states, V~ and Y pass between them as bf16 where the saving scan stages
     its saves through LDS.  Packed and left-padded batches are laid out with the chunk count of their longest
-    sequence and run one more launch (their forward sweep prepares its own records)."""
+    sequence; batches of rows that are not whole chunks run one more launch (their forward sweep prepares its own records)."""
     from . import ops  # late: ops imports this module
 
     B, T, H, K = q.shape

@@ -400,7 +400,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 #pragma unroll
                 for (int e = 0; e < 8; e++) dot += (float)er[i][e] * (float)sr[i][e];
             }
-        } else {
+        } else {  // (saves that are not sliced)
             // v, dO and Y (token `row` is token 63 - row of mirror chunk A); dV = beta Y goes out right away
             const int p8 = t % 8;
 #pragma unroll
@@ -410,10 +410,8 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                 bf16x8 vr = *reinterpret_cast<const bf16x8*>(row_of(p.v_raw, p.v_stride_b, p.v_stride_t, p.v_stride_h, row) + v0 + 8 * p8);
                 bf16x8 dr = *reinterpret_cast<const bf16x8*>(row_of(p.d_raw, p.d_stride_b, p.d_stride_t, p.d_stride_h, row) + v0 + 8 * p8);
                 if (!live) vr = zero8, dr = zero8;
-                const bf16_t* yrow;
-                if constexpr (SL) yrow = p.y_chunks + chunk * C * V + sliced_at(C - 1 - row, v0 + 8 * p8, C);
-                else yrow = p.y_mirror != nullptr ? p.y_mirror + ((mirA + (C - 1 - row)) * p.H + h) * V + v0 + 8 * p8
-                                                  : p.y_chunks + (chunk * C + (C - 1 - row)) * V + v0 + 8 * p8;
+                const bf16_t* const yrow = p.y_mirror != nullptr ? p.y_mirror + ((mirA + (C - 1 - row)) * p.H + h) * V + v0 + 8 * p8
+                                                                 : p.y_chunks + (chunk * C + (C - 1 - row)) * V + v0 + 8 * p8;
                 const bf16x8 yr = *reinterpret_cast<const bf16x8*>(yrow);
                 const float b = p.beta[chunk * C + row];
                 bf16x8 dv;
@@ -433,16 +431,14 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 #pragma unroll
                 for (int it = 0; it < 2; it++) {  // rows of V~ past the end of the sequence hold whatever the scan left
                     const int row = t / 8 + 32 * it;
-                    const bf16x8 x = *reinterpret_cast<const bf16x8*>(SL ? vnew + sliced_at(row, v0 + 8 * p8, C)
-                                                                                : vnew + row * V + v0 + 8 * p8);
+                    const bf16x8 x = *reinterpret_cast<const bf16x8*>(vnew + row * V + v0 + 8 * p8);
                     *reinterpret_cast<bf16x8*>(sVN + row * LDS64 + 8 * p8) = row < valid ? x : zero8;
                 }
                 const bf16_t* s0 = reinterpret_cast<const bf16_t*>(s0b);
 #pragma unroll
                 for (int i = 0; i < K / 32; i++) {  // S0[:, v0 .. v0 + 63]: row = 32 i + t / 8
                     const int row = t / 8 + 32 * i;
-                    *reinterpret_cast<bf16x8*>(sST + row * LDS64 + 8 * p8) =
-                        *reinterpret_cast<const bf16x8*>(SL ? s0 + sliced_at(row, v0 + 8 * p8, K) : s0 + row * V + v0 + 8 * p8);
+                    *reinterpret_cast<bf16x8*>(sST + row * LDS64 + 8 * p8) = *reinterpret_cast<const bf16x8*>(s0 + row * V + v0 + 8 * p8);
                 }
             } else {
                 const float* vnew = reinterpret_cast<const float*>(vnb);

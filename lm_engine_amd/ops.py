@@ -133,10 +133,11 @@ def _fill_args(q, k, v, g, beta, h0, ht, o, cu_seqlens, scale, l2norm, inplace, 
     return a
 
 
-# Workspaces of the one-launch chunked forward, kept between calls: one per (device, stream, shape), its header
+# Workspaces of the one-launch chunked forward and of the layer's decode step (layer_step_workspace: tickets and a row of
+# scratch per head), kept between calls: one per (device, stream, shape), its header
 # (chunk offsets, error latch, ready flags) zero-filled when it is made.  The library then need not clear the ready flags
 # before every call (it leaves them clear itself, GDN_FLAG_READY_FLAGS_CLEAR), and a step of that shape no longer asks
-# the allocator for tens of megabytes.  Only shapes that run as one launch keep a workspace: every other call (packed
+# the allocator for tens of megabytes.  Of the forwards, only shapes that run as one launch keep a workspace: every other call (packed
 # or left-padded batches, K = 256, shapes outside the window) reads no flag and takes a fresh torch.empty workspace
 # from the caching allocator, whatever T it comes with.  Calls on one stream run in order, so they can share a
 # workspace; another stream gets its own.  The least recently used entries go when there are more than
