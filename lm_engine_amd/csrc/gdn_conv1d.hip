@@ -191,10 +191,11 @@ template <typename T, typename WT>
 static int launch_conv(const ConvParams& p, int kernel_size, bool silu, hipStream_t stream) {
     const int64_t groups = (p.C / ConvVec<T>::N + WAVE - 1) / WAVE;
     const int64_t waves = groups * ((p.S + CONV_TOKENS - 1) / CONV_TOKENS) * p.B;
-    // Under 2048 waves (8 per compute unit) a walk of 16 tokens is one latency after another with little beside it: a
-    // prompt of 777 tokens x 2048 channels has 196 such waves and the layer's prefill takes 56.7 us with 16 tokens a thread,
-    // 51.8 with 4.  Above, the halo of 3 rows per block counts: 8 x 4096 x 2048 has 8192 waves, its layer's training step
-    // 1354 us with 16 tokens, 1363 with 4.
+    // Under 2048 waves (8 per compute unit) a walk of 16 tokens is one latency after another with little beside it; above, the
+    // halo of 3 rows per block counts.  4 | 16 tokens a thread, bf16, inputs from memory: C = 2048, 200 waves 5.9 | 12.1 us,
+    // 1024 11.5 | 18.1, 2000 19.9 | 22.3, 2100 21.9 | 23.4, 3072 28.4 | 27.5, 8192 71.5 | 59.7; C = 6144, 2000 waves
+    // 20.2 | 21.2, 2100 22.4 | 22.4, 3072 28.9 | 25.0.  fp32 crosses at about the same place: C = 2048, 2100 17.9 | 19.8,
+    // 4096 28.1 | 26.3.
     if (waves < 2048) {
         if (kernel_size == 2) launch_conv_ks<T, WT, 2, CONV_TOKENS_SHORT>(p, silu, stream);
         else if (kernel_size == 3) launch_conv_ks<T, WT, 3, CONV_TOKENS_SHORT>(p, silu, stream);
