@@ -164,9 +164,12 @@ def release_workspaces() -> None:
 def _error_word(device) -> torch.Tensor:
     word = _ERROR_WORDS.get(device.index)
     if word is None:
-        word = torch.zeros(1, dtype=torch.int32).pin_memory()
-        _ERROR_PEEKS[device.index] = ctypes.c_int32.from_address(word.data_ptr())
-        _ERROR_WORDS[device.index] = word
+        with _WORKSPACES_LOCK:  # one word per device, whoever asks first
+            word = _ERROR_WORDS.get(device.index)
+            if word is None:
+                word = torch.zeros(1, dtype=torch.int32).pin_memory()
+                _ERROR_PEEKS[device.index] = ctypes.c_int32.from_address(word.data_ptr())
+                _ERROR_WORDS[device.index] = word
     return word
 
 

@@ -9,6 +9,8 @@ import re
 import subprocess
 import sys
 import tempfile
+import threading
+import time
 
 import pytest
 import torch
@@ -231,6 +233,33 @@ def test_package_imports_on_a_torch_build_without_gpu_support():
             "except ValueError as e: print(e)")  # fmt: skip
     run = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
     assert run.returncode == 0 and "GPU only" in run.stdout, run.stderr
+
+
+def test_threads_that_ask_first_share_one_error_word(monkeypatch):
+    """The look at a device's error word goes to the address of the word that the library is given, also when several threads
+    make their first call at once (the slow allocation lets both in; no device is touched)."""
+    from lm_engine_amd import ops
+
+    zeros = torch.zeros
+
+    def slow_zeros(*args, **kwargs):
+        word = zeros(*args, **kwargs)
+        time.sleep(0.05 * (1 + len(made)))
+        made.append(word)
+        return word
+
+    made, got = [], []
+    monkeypatch.setattr(ops, "_ERROR_WORDS", {})
+    monkeypatch.setattr(ops, "_ERROR_PEEKS", {})
+    monkeypatch.setattr(torch, "zeros", slow_zeros)
+    monkeypatch.setattr(torch.Tensor, "pin_memory", lambda self: self)
+    threads = [threading.Thread(target=lambda: got.append(ops._error_word(torch.device("cuda", 3)))) for _ in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert len(got) == 3 and all(word is ops._ERROR_WORDS[3] for word in got)
+    assert ctypes.addressof(ops._ERROR_PEEKS[3]) == ops._ERROR_WORDS[3].data_ptr()
 
 
 def test_kernel_flag_registry_follows_the_reference_convention():
