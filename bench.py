@@ -114,10 +114,12 @@ def device_warmup(call, ms: float = DEVICE_WARMUP_MS):
     some 20 ms of sustained work to reach the clocks it then holds: a leg that starts timing after a handful of warm-up
     steps measures the ramp (configuration 1: 0.132 ms per step over the first 7 ms, 0.114 over the next 6, then 0.107
     for as long as the loop runs).  Every leg therefore first brings the device to that state with its own step; the
-    W warm-up steps and the K timed steps follow immediately."""
+    W warm-up steps and the K timed steps follow immediately.  The first call is made before the clock starts: in a fresh
+    process it loads libraries and code objects, which takes longer than all of the ``ms``."""
     import torch
 
     takes_index = call.__code__.co_argcount == 1  # the decode leg rotates its state buffers
+    call(0) if takes_index else call()
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     n = 0

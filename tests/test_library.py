@@ -235,6 +235,16 @@ def test_package_imports_on_a_torch_build_without_gpu_support():
     assert run.returncode == 0 and "GPU only" in run.stdout, run.stderr
 
 
+def test_warmup_of_the_benchmark_is_not_spent_on_loading(monkeypatch):
+    """The first call of a process loads libraries and code objects for longer than the warm-up lasts: it comes before the clock."""
+    import bench
+
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda: None)
+    made = []
+    bench.device_warmup(lambda: time.sleep(0.002 if made else 0.2) or made.append(1), ms=40.0)
+    assert len(made) >= 12
+
+
 def test_threads_that_ask_first_share_one_error_word(monkeypatch):
     """The look at a device's error word goes to the address of the word that the library is given, also when several threads
     make their first call at once (the slow allocation lets both in; no device is touched)."""
