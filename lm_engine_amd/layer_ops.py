@@ -38,6 +38,13 @@ def _require(x: torch.Tensor, what: str) -> None:
         raise ValueError(f"{what} must be a device tensor: these kernels run on the GPU only")
 
 
+def _require_same_device(x: torch.Tensor, what: str, **others) -> None:
+    """Ahead of every launch: a tensor elsewhere (on the host, say) would be read through an address that faults the GPU."""
+    for name, t in others.items():
+        if t is not None and t.device != x.device:
+            raise ValueError(f"{name} is on {t.device}, {what} is on {x.device}")
+
+
 def _token_rows(x: torch.Tensor, width: int, what: str) -> tuple[torch.Tensor, int]:
     """[..., width] view whose leading dims collapse to one token axis with a single stride."""
     if x.size(-1) != width:
@@ -156,6 +163,7 @@ def _delta_rule_gates(a, b, A_log, dt_bias, allow_neg_eigval):
         raise ValueError("a and b must share shape and dtype")
     if tuple(A_log.shape) != (H,) or tuple(dt_bias.shape) != (H,):
         raise ValueError(f"A_log and dt_bias must be [H] = {(H,)}")
+    _require_same_device(a, "a", b=b)
     a2, a_stride = _token_rows(a, H, "a")
     b2, b_stride = _token_rows(b, H, "b")
     A_log = A_log.to(device=a.device, dtype=torch.float32).contiguous()
@@ -272,6 +280,7 @@ def _norm_operands(o, gate):
     if gate is not None:
         if gate.dtype != o.dtype or gate.numel() != o.numel():
             raise ValueError("gate must have the dtype and number of elements of o")
+        _require_same_device(o, "o", gate=gate)
         if gate.shape[-2:] == (H, V) and gate.dim() == o.dim():
             gate = gate.flatten(-2) if gate.stride(-2) == V and gate.stride(-1) == 1 else gate.contiguous().flatten(-2)
         g2, g_stride = _token_rows(gate, H * V, "gate")
@@ -286,6 +295,7 @@ def _gated_rmsnorm(o, gate, weight, eps):
     o2, o_stride, g2, g_stride, H, V = _norm_operands(o, gate)
     if weight is not None and tuple(weight.shape) != (V,):
         raise ValueError(f"weight must be [V] = {(V,)}")
+    _require_same_device(o, "o", weight=weight)
     weight = None if weight is None else weight.contiguous()
     y = torch.empty(o.shape, dtype=o.dtype, device=o.device)
 

@@ -123,3 +123,17 @@ def test_column_sums(rows, cols):
         bound = part.abs().double().sum(dim=0) * (rows / 64 + 7) * 2.0**-24
         assert sums.shape == want.shape
         assert ((sums.double().cpu() - want).abs() <= bound + (want.abs() + bound) * unit).all()
+
+
+def test_operands_on_the_host_are_refused_before_any_launch():
+    """A host tensor beside device tensors raises; its address never reaches a kernel."""
+    H, V = 2, 64
+    a, A = torch.zeros(2, 5, H, dtype=BF16).cuda(), torch.zeros(H).cuda()
+    o, z, w = torch.zeros(2, 5, H, V, dtype=BF16).cuda(), torch.zeros(2, 5, H * V, dtype=BF16), torch.ones(V, dtype=BF16)
+    with pytest.raises(ValueError, match="b is on cpu"):
+        lm_engine_amd.delta_rule_gates(a, a.cpu(), A, A)
+    for gate, weight, name in ((z, None, "gate"), (z.view(2, 5, H, V), w.cuda(), "gate"), (z.cuda(), w, "weight"), (None, w, "weight")):
+        with pytest.raises(ValueError, match=f"{name} is on cpu"):
+            lm_engine_amd.gated_rmsnorm(o, gate, weight, 1e-5)
+        with pytest.raises(ValueError, match=f"{name} is on cpu"):
+            lm_engine_amd.gated_rmsnorm(o.clone().requires_grad_(True), gate, weight, 1e-5)
