@@ -201,6 +201,10 @@ PyObject* layer_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const int64_t ks = taps_of(weight, C);
         s.conv_w_dtype = code_of(weight);
         need(s.dtype == GDN_BF16 || s.conv_w_dtype == GDN_F32);
+        // (the kernel reads by elements; what the convolution and the norm on their own refuse for its place in memory goes to them)
+        const int64_t vec = s.dtype == GDN_BF16 ? 8 : 4;
+        need(aligned(ptr(qkv), 16) && qkv.stride(0) % vec == 0 && qkv.stride(1) % vec == 0 && qkv.stride(1) >= C && aligned(ptr(weight), 16));
+        need(aligned(ptr(bias), 16) && aligned(ptr(norm_w), 16));
         if (bias != nullptr) need(bias->scalar_type() == weight.scalar_type() && bias->dim() == 1 && bias->size(0) == C && bias->is_contiguous());
         if (conv_state != nullptr) need(conv_state->scalar_type() == qkv.scalar_type() && conv_state->sizes() == at::IntArrayRef({B, C, ks - 1}) && conv_state->is_contiguous());
         if (h0 != nullptr) need(h0->scalar_type() == at::kFloat && h0->sizes() == at::IntArrayRef({B, H, K, V}) && h0->is_contiguous() && aligned(ptr(h0), 16));
@@ -262,7 +266,7 @@ PyObject* conv(PyObject*, PyObject* const* args, Py_ssize_t n) {
             if (output_state) final_state = fresh(x, {B, C, ks - 1}), s.final_state = ptr(final_state);
         });
         s.x = ptr(x), s.weight = ptr(weight), s.bias = ptr(bias), s.input_state = ptr(state), s.y = ptr(y);
-        s.x_stride_b = x.stride(0), s.x_stride_s = S > 1 ? x.stride(1) : C, s.y_stride_b = S * C, s.y_stride_s = C;
+        s.x_stride_b = x.stride(0), s.x_stride_s = x.stride(1), s.y_stride_b = S * C, s.y_stride_s = C;
         s.B = size32(B), s.S = size32(S), s.C = size32(C), s.kernel_size = (int32_t)ks;
         s.activation = (int32_t)integer(args[7]);
         return launch("gdn_causal_conv1d_fwd", pack_results({y, final_state}), [&] { return conv_fn(&s, stream); });

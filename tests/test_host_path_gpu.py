@@ -134,3 +134,23 @@ def test_other_threads_run_while_a_call_launches(entry):
     with _entry_points_replaced(**{entry: ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value}):
         call()
     torch.cuda.synchronize()
+
+
+def test_layouts_that_the_convolution_refuses_are_refused_on_one_token_too():
+    """Rows off 16-byte boundaries or on top of each other: the convolution raises for them, alone and as part of the layer's step."""
+    x = _layer_operands(2, 1)
+    r = lambda *shape: torch.randn(*shape, generator=torch.Generator().manual_seed(5)).to(BF16).cuda()  # noqa: E731
+    wide, flat = r(2, 1, 400), r(384 * 4 + 1)
+    for over in (dict(qkv=wide[..., 1:385]), dict(qkv=r(2, 1, 388)[..., :384]), dict(qkv=r(384).as_strided((2, 1, 384), (0, 8, 1))), dict(conv_weight=flat[1:].view(384, 1, 4)),
+                 dict(conv_bias=flat[1:385])):  # fmt: skip
+        operands = {**x, **over}
+        with pytest.raises(ValueError, match="gdn_causal_conv1d_fwd"):
+            lm_engine_amd.depthwise_causal_convolution(operands["qkv"], operands["conv_weight"], operands["conv_bias"])
+        with pytest.raises(ValueError, match="gdn_causal_conv1d_fwd"):
+            lm_engine_amd.gated_deltanet_mixing(**operands, cache=(None, None))
+    with pytest.raises(ValueError, match="gdn_gated_rmsnorm_fwd"):
+        lm_engine_amd.gated_deltanet_mixing(**{**x, "norm_weight": flat[1:65]}, cache=(None, None))
+    taken = dict(qkv=wide[..., 8:392], a=wide[..., 1:3], b=wide[..., 3:5], gate=wide[..., 7:135])  # scalars and gate lie anywhere
+    out, _ = lm_engine_amd.gated_deltanet_mixing(**{**x, **taken}, cache=(None, None))
+    want, _ = lm_engine_amd.gated_deltanet_mixing(**{**x, **{n: t.contiguous() for n, t in taken.items()}}, cache=(None, None))
+    assert torch.equal(out, want)
