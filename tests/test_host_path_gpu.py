@@ -12,6 +12,8 @@ import torch
 import lm_engine_amd
 from lm_engine_amd import _host, _lib
 
+from .helpers import rel_l2
+
 
 pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
@@ -154,3 +156,149 @@ def test_layouts_that_the_convolution_refuses_are_refused_on_one_token_too():
     out, _ = lm_engine_amd.gated_deltanet_mixing(**{**x, **taken}, cache=(None, None))
     want, _ = lm_engine_amd.gated_deltanet_mixing(**{**x, **{n: t.contiguous() for n, t in taken.items()}}, cache=(None, None))
     assert torch.equal(out, want)
+
+
+class _NativePath:
+    """The native host path with a record of which calls it took on; ``on`` False: it takes none."""
+
+    def __init__(self, on):
+        self.on, self.took = on, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            result = getattr(_host.host(), name)(*args) if self.on else None
+            self.took.append(result is not None)
+            return result
+
+        return call
+
+
+def _outcome(call):
+    """What a call gives: its tensors, or the type and text of what it raises."""
+    try:
+        with torch.no_grad():
+            result = call()
+    except (ValueError, RuntimeError, TypeError, IndexError, AttributeError) as error:
+        return type(error), str(error)
+    flat = []
+    for x in result if isinstance(result, tuple) else (result,):
+        flat += x if isinstance(x, tuple) else (x,)
+    return flat
+
+
+def _operand_forms():
+    """Calls in forms that a caller may use or get wrong: layouts, types, shapes, options."""
+    gen = torch.Generator().manual_seed(7)
+    r = lambda *shape: torch.randn(*shape, generator=gen).to(BF16).cuda()  # noqa: E731
+    x3, w, bias, state = r(2, 5, 384), 0.3 * r(384, 1, 4), 0.1 * r(384), r(2, 384, 3)
+    mask = (torch.rand(2, 5, generator=gen) > 0.3).cuda()
+    conv = lambda *args, **kw: lambda: lm_engine_amd.depthwise_causal_convolution(*args, output_state=True, **kw)  # noqa: E731
+    wide = r(2, 5, 400)
+    yield "conv", {
+        "plain": conv(x3, w, bias, state), "no state": conv(x3, w, bias), "no bias": conv(x3, w), "one token": conv(x3[:, :1], w, bias, state),
+        "slice": conv(wide[..., 8:392], w, bias, state), "slice off its boundary": conv(wide[..., 1:385], w, bias, state),
+        "tokens first": conv(r(5, 2, 384).transpose(0, 1), w, bias, state), "channels strided": conv(r(2, 384, 5).transpose(1, 2), w, bias, state),
+        "fp32 weight": conv(x3, w.float(), bias.float(), state), "fp32 x": conv(x3.float(), w, bias, state), "mixed bias": conv(x3, w, bias.float()),
+        "fp16": conv(x3.half(), w.half()), "state fp32": conv(x3, w, bias, state.float()), "state of another size": conv(x3, w, bias, state[..., :2]),
+        "state strided": conv(x3, w, bias, r(2, 3, 384).transpose(1, 2)), "weight strided": conv(x3, r(4, 384).t(), bias), "weight 2-D": conv(x3, w[:, 0], bias),
+        "weight of other channels": conv(x3, w[:383], bias), "five taps": conv(x3, r(384, 1, 5)), "one tap": conv(x3, r(384, 1, 1)), "bias 2-D": conv(x3, w, bias[None]),
+        "2-D x": conv(x3[0], w), "no tokens": conv(x3[:, :0], w), "odd channels": conv(r(2, 5, 381), r(381, 1, 4)), "mask bool": conv(x3, w, bias, state, mask),
+        "mask int": conv(x3, w, bias, state, mask.long()), "mask fp32": conv(x3, w, bias, state, mask.float()), "mask of one row": conv(x3, w, bias, state, mask[:1]),
+        "mask of one token": conv(x3, w, bias, state, mask[:, :1]), "mask 1-D": conv(x3, w, bias, state, mask[0]), "mask 3-D of one row": conv(x3, w, bias, state, mask[:1, :, None]),
+        "mask of other tokens": conv(x3, w, bias, state, mask[:, :4]), "mask on the host": conv(x3, w, bias, state, mask.cpu()), "swish": conv(x3, w, activation="swish"),
+        "no activation": conv(x3, w, activation=None), "gelu": conv(x3, w, activation="gelu"), "weight on the host": conv(x3, w.cpu()),
+    }  # fmt: skip
+    a, b, A, dt = r(2, 5, 3), r(2, 5, 3), torch.rand(3, generator=gen).cuda(), torch.rand(3, generator=gen).cuda()
+    gates = lambda *args, **kw: lambda: lm_engine_amd.delta_rule_gates(*args, **kw)  # noqa: E731
+    ab = r(2, 5, 8)
+    yield "gates", {
+        "plain": gates(a, b, A, dt), "negative eigenvalues": gates(a, b, A, dt, allow_neg_eigval=True), "slices": gates(ab[..., :3], ab[..., 3:6], A, dt),
+        "slices of one token": gates(ab[:, :1, :3], ab[:, :1, 3:6], A, dt), "every second row": gates(ab[:, ::2, :3], ab[:, ::2, 3:6], A, dt),
+        "heads strided": gates(ab[..., ::3], ab[..., 1::3][..., :3], A, dt), "transposed": gates(r(5, 2, 3).transpose(0, 1), b, A, dt), "2-D": gates(a[0], b[0], A, dt),
+        "1-D": gates(a[0, 0], b[0, 0], A, dt), "bf16 parameters": gates(a, b, A.to(BF16), dt.to(BF16)), "parameters 2-D": gates(a, b, A[None], dt[None]),
+        "fp32": gates(a.float(), b.float(), A, dt), "mixed": gates(a, b.float(), A, dt), "other shape": gates(a, b[:, :4], A, dt), "other heads": gates(a, b, A[:2], dt),
+        "no tokens": gates(a[:, :0], b[:, :0], A, dt), "parameters on the host": gates(a, b, A.cpu(), dt.cpu()), "parameters strided": gates(a, b, torch.rand(6).cuda()[::2], dt),
+        "one head": gates(r(2, 5, 1), r(2, 5, 1), A[:1], dt[:1]), "b on the host": gates(a, b.cpu(), A, dt),
+    }  # fmt: skip
+    o, z, nw = r(2, 5, 2, 64), r(2, 5, 128), r(64)
+    norm = lambda *args: lambda: lm_engine_amd.gated_rmsnorm(*args)  # noqa: E731
+    zw = r(2, 5, 140)
+    yield "norm", {
+        "plain": norm(o, z, nw, 1e-5), "no gate": norm(o, None, nw, 1e-5), "no weight": norm(o, z, None, 1e-5), "default eps": norm(o, z, nw), "gate by heads": norm(o, z.view(2, 5, 2, 64), nw, 1e-5),
+        "gate slice": norm(o, zw[..., 4:132], nw, 1e-5), "gate slice off its boundary": norm(o, zw[..., 3:131], nw, 1e-5), "gate heads strided": norm(o, r(2, 5, 64, 2).transpose(2, 3), nw, 1e-5),
+        "gate of other leading dims": norm(o, z.view(10, 128), nw, 1e-5), "gate tokens first": norm(o, r(5, 2, 128).transpose(0, 1), nw, 1e-5), "gate of one token": norm(o, z[:, :1], nw, 1e-5),
+        "gate fp32": norm(o, z.float(), nw, 1e-5), "o strided": norm(r(2, 2, 5, 64).transpose(1, 2), z, nw, 1e-5), "o 2-D": norm(o[0, 0], z[0, 0], nw, 1e-5), "o 2-D, gate 2-D": norm(o[0, 0], z[0, 0].view(2, 64), nw, 1e-5),
+        "o 1-D": norm(o[0, 0, 0], None, nw, 1e-5), "weight fp32": norm(o, z, nw.float(), 1e-5), "weight of another size": norm(o, z, nw[:32], 1e-5), "weight 2-D": norm(o, z, nw[None], 1e-5),
+        "weight strided": norm(o, z, r(128)[::2], 1e-5), "fp32": norm(o.float(), z.float(), nw.float(), 1e-5), "fp16": norm(o.half(), None, None, 1e-5), "no tokens": norm(o[:, :0], z[:, :0], nw, 1e-5),
+        "odd V": norm(r(2, 5, 2, 20), None, None, 1e-5), "wide V": norm(r(2, 5, 2, 520), None, None, 1e-5), "one head": norm(r(2, 5, 1, 64), r(2, 5, 64), nw, 1e-5), "gate on the host": norm(o, z.cpu(), nw, 1e-5),
+    }  # fmt: skip
+    for T, op in ((5, lm_engine_amd.fused_recurrent_gated_delta_rule), (130, lm_engine_amd.chunk_gated_delta_rule)):
+        q, k, v = r(2, T, 2, 64), r(2, T, 2, 64), r(2, T, 4, 64)
+        g, beta, h = -torch.rand(2, T, 4, generator=gen).cuda(), torch.rand(2, T, 4, generator=gen).to(BF16).cuda(), torch.randn(2, 4, 64, 64, generator=gen).cuda()
+        row = lambda *xs: [x[:1] for x in xs]  # noqa: E731
+        prefix = lambda *ends, dtype=torch.int32: torch.tensor(ends, dtype=dtype).cuda()  # noqa: E731
+        base = dict(q=q, k=k, v=v, g=g, beta=beta, initial_state=h, output_final_state=True, use_qk_l2norm_in_kernel=True)
+        packed = {**base, **dict(zip(("q", "k", "v", "g", "beta"), row(q, k, v, g, beta))), "cu_seqlens": prefix(0, 3, T)}
+        padded = {**base, "left_padded": True, "cu_seqlens": prefix(0, 2, T + 2)}
+        qkv = r(2, T, 2 * 64 + 2 * 64 + 4 * 64 + 8)
+        views = dict(q=qkv[..., :128].view(2, T, 2, 64), k=qkv[..., 128:256].view(2, T, 2, 64), v=qkv[..., 256:512].view(2, T, 4, 64))
+        off = dict(q=qkv[..., 4:132].unflatten(-1, (2, 64)))
+        call = lambda over, base=base, op=op: lambda: op(**{**base, **over})  # noqa: E731
+        forms = {
+            "plain": call({}), "no state": call(dict(initial_state=None)), "no final state": call(dict(output_final_state=False)), "ungated": call(dict(g=None, beta=None)),
+            "scale": call(dict(scale=0.3)), "scale as tensor": call(dict(scale=torch.tensor(0.3))), "no l2norm": call(dict(use_qk_l2norm_in_kernel=False)), "slices": call(views),
+            "slice off its boundary": call(off), "tokens first": call(dict(q=r(T, 2, 2, 64).transpose(0, 1))), "last dim strided": call(dict(v=r(2, T, 64, 4).transpose(2, 3))),
+            "equal heads": call(dict(q=r(2, T, 4, 64), k=r(2, T, 4, 64))), "heads that do not divide": call(dict(q=r(2, T, 3, 64), k=r(2, T, 3, 64))), "k of other heads": call(dict(k=r(2, T, 4, 64))),
+            "g bf16": call(dict(g=g.to(BF16))), "g strided": call(dict(g=-torch.rand(2, 4, T, generator=gen).cuda().transpose(1, 2))), "g of other heads": call(dict(g=g[..., :2])), "beta fp32": call(dict(beta=beta.float())),
+            "beta fp16": call(dict(beta=beta.half())), "beta 4-D": call(dict(beta=beta[..., None])), "state bf16": call(dict(initial_state=h.to(BF16))), "state of another batch": call(dict(initial_state=h[:1])),
+            "state strided": call(dict(initial_state=h.transpose(2, 3))), "mixed types": call(dict(k=k.float())), "fp32": call(dict(q=q.float(), k=k.float(), v=v.float())), "fp16": call(dict(q=q.half(), k=k.half(), v=v.half())),
+            "K = 96": call(dict(q=r(2, T, 2, 96), k=r(2, T, 2, 96), initial_state=None)), "V = 40": call(dict(v=r(2, T, 4, 40), initial_state=None)), "other tokens": call(dict(v=v[:, 1:])), "k on the host": call(dict(k=k.cpu())),
+            "packed": call(packed), "packed, int64 prefix": call({**packed, "cu_seqlens": prefix(0, 3, T, dtype=torch.int64)}), "packed, strided prefix": call({**packed, "cu_seqlens": prefix(0, 0, 3, 0, T)[::2]}),
+            "packed with an empty sequence": call({**packed, "cu_seqlens": prefix(0, 0, T)}), "packed, state of another count": call({**packed, "cu_seqlens": prefix(0, 1, 2, T)}),
+            "prefix beside a batch": call(dict(cu_seqlens=prefix(0, 3, T))), "prefix of one": call({**packed, "cu_seqlens": prefix(0)}), "prefix 2-D": call({**packed, "cu_seqlens": prefix(0, 3, T)[None]}), "padded": call(padded),
+            "padded, prefix too short": call({**padded, "cu_seqlens": prefix(0, T)}), "padded without prefix": call({**padded, "cu_seqlens": None}), "no tokens": call({n: base[n][:, :0] for n in ("q", "k", "v", "g", "beta")}),
+        }  # fmt: skip
+        if T == 5:  # in place on a copy that the outcome shows
+            own = lambda h0=h, **over: lambda: (lambda s: (*op(**{**base, **over, "initial_state": s, "inplace_state": True}), s))(None if h0 is None else h0.clone())  # noqa: E731
+            forms.update({"in place": own(), "in place without a state": own(None), "in place, strided": own(h.transpose(2, 3)), "in place, no final state": own(output_final_state=False)})
+        yield ("recurrent", "chunk")[T > 64], forms
+    x = _layer_operands(2, 1)
+    zc, hc = r(2, 384, 3), torch.randn(2, 2, 64, 64, generator=gen).cuda()
+    abz = r(2, 1, 2 + 2 + 128)
+    step = lambda cache=(zc, hc), **over: lambda: lm_engine_amd.gated_deltanet_mixing(**{**x, **over}, cache=cache)  # noqa: E731
+    yield "layer_step", {
+        "plain": step(), "no cache yet": step((None, None)), "no convolution state": step((None, hc)), "no gate": step(gate=None), "no norm weight": step(norm_weight=None), "no bias": step(conv_bias=None),
+        "slices": step(a=abz[..., :2], b=abz[..., 2:4], gate=abz[..., 4:]), "gate by heads": step(gate=r(2, 1, 2, 64)), "gate 2-D": step(gate=r(2, 128)), "gate of another batch": step(gate=r(1, 1, 128)), "gate fp32": step(gate=r(2, 1, 128).float()),
+        "a of another batch": step(a=r(1, 1, 2)), "a fp32": step(a=r(2, 1, 2).float()), "bf16 decay": step(A_log=x["A_log"].to(BF16), dt_bias=x["dt_bias"].to(BF16)), "fp32 convolution weight": step(conv_weight=x["conv_weight"].float(), conv_bias=x["conv_bias"].float()),
+        "fp32 norm weight": step(norm_weight=x["norm_weight"].float()), "norm weight of another size": step(norm_weight=r(32)), "state bf16": step((zc, hc.to(BF16))), "convolution state fp32": step((zc.float(), hc)), "convolution state strided": step((r(2, 3, 384).transpose(1, 2), hc)),
+        "convolution state of another size": step((zc[..., :2], hc)), "state of another batch": step((zc, hc[:1])), "no activation": step(conv_activation=None), "gelu": step(conv_activation="gelu"), "negative eigenvalues": step(allow_neg_eigval=True), "scale": step(scale=0.2),
+        "default eps": step(norm_eps=None), "qkv slice": step(qkv=r(2, 1, 400)[..., 8:392]), "qkv slice off its boundary": step(qkv=r(2, 1, 400)[..., 1:385]), "qkv of other channels": step(qkv=r(2, 1, 392)), "fp32": step((zc.float(), hc), **{n: y.float() for n, y in x.items() if isinstance(y, torch.Tensor)}),
+        "mask": step(attention_mask=torch.ones(2, 1).cuda()), "state on the host": step((zc, hc.cpu())), "gate on the host": step(gate=r(2, 1, 128).cpu()),
+    }  # fmt: skip
+
+
+def test_calls_end_as_they_do_without_the_native_path(monkeypatch):
+    """Every form of a call gives the same bits, or raises the same error, with the native host path and without it.  The layer's
+    one-launch step adds the norm's squares up in another order (its output: an ulp; its states: the same bits)."""
+    from lm_engine_amd import conv, layer, layer_ops, ops
+
+    differ = []
+    for name, forms in _operand_forms():
+        for form, call in forms.items():
+            print(f"case: {name}, {form}", flush=True)
+            outcomes = []
+            for path in (_NativePath(True), _NativePath(False)):
+                with monkeypatch.context() as m:
+                    for module in (conv, layer, layer_ops, ops):
+                        m.setattr(module, "host", lambda path=path: path)
+                    outcomes.append(_outcome(call))
+                assert form != "plain" or path.took[0] == path.on, "the path under test was not the one taken"
+            native, python = outcomes
+            same = native == python if isinstance(native, tuple) or isinstance(python, tuple) else len(native) == len(python) and all(
+                (x is None and y is None) or (x.dtype == y.dtype and x.shape == y.shape and x.stride() == y.stride()
+                                              and (torch.equal(x, y) or (name == "layer_step" and i == 0 and rel_l2(x, y) <= 1e-3)))
+                for i, (x, y) in enumerate(zip(native, python)))  # fmt: skip
+            if not same:
+                differ.append((name, form, *(z if isinstance(z, tuple) else "tensors" for z in (native, python))))
+    torch.cuda.synchronize()
+    assert not differ, "\n".join(map(str, differ))
