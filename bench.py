@@ -626,13 +626,8 @@ def bench_backward(w, inp, steps, warmup):
         "steps": steps,
         "ms_per_backward": round(ms, 3),
         "tokens_per_s": round(inp["q"].size(0) * inp["q"].size(1) / (ms * 1e-3), 1),
-        "composition": ("4 kernel launches (and small helpers): backward prepare (also writes the forward sweep's records), saving "
-                        "scan on those records (forward sweep), saving scan over the mirror problem with every row scanned over its own chunks (reverse sweep), chunk-local "
-                        "gradients; chunk states, V~ and Y pass between them as bf16"
-                        if backward_kernels_apply(w.K, w.V) and inp["cu_seqlens"] is not None else
-                        "4 kernel launches: backward prepare (also writes the forward sweep's records), saving scan "
-                        "on those records (forward sweep), saving scan over the mirror problem (reverse sweep), "
-                        "chunk-local gradients; chunk states, V~ and Y pass between them as bf16"
+        "composition": ("4 kernel launches (packed sequences: and their chunk offsets): per-chunk records, forward sweep, reverse "
+                        "sweep, chunk-local gradients; chunk states, V~ and Y pass between them as bf16"
                         if backward_kernels_apply(w.K, w.V) else
                         "2 saving scans + rocBLAS batched GEMMs + elementwise torch ops"),
     }

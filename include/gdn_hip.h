@@ -370,6 +370,23 @@ typedef struct gdn_chunk_bwd_prepare_args {
 int gdn_chunk_bwd_prepare(const gdn_chunk_bwd_prepare_args *args, void *stream);
 
 /*
+ * Training support, fourth part: everything gdn_chunk_bwd_local needs from the states, in one call of three kernels - per-chunk
+ * records, the forward sweep (the states the chunks start from, V~) and the reverse sweep (the gradients of the states they end
+ * with, Y).  What gdn_chunk_bwd_prepare and two calls of gdn_chunk_fwd_saving arrive at through a mirror problem, in one step per
+ * chunk, for every batch that gdn_chunk_fwd takes (fixed-length rows of any length, packed, left-padded; qk_heads as there):
+ * bf16, K = 64, 128 or 256, V a multiple of 64 (GDN_ERR_UNSUPPORTED otherwise).
+ *   args   as for gdn_chunk_fwd; h0, g, beta may be NULL; ht is not used and o not written (it must be a valid pointer and strides);
+ *          workspace of gdn_chunk_bwd_sweeps_workspace_bytes, 256-byte aligned, nothing in it has to be cleared
+ *   local  the arrays that gdn_chunk_bwd_local will read are written here: v_new, states, dstates, y_chunks (bf16, saves_sliced),
+ *          gamma, beta, rq, rk (all four; rq and rk are 1 without GDN_FLAG_L2NORM); H, K, V, NC, chunks = N H NC describe them, with
+ *          NC at least the chunks of the longest sequence.  dout_raw and its strides are read.  The rest is not looked at.
+ *          Entries of chunks past the end of their sequence are not written (nor read by gdn_chunk_bwd_local).
+ *   dht    fp32 [N, H, K, V], the gradient of the final state, or NULL (zeros);  dh0: that of the initial state is written, or NULL
+ */
+int gdn_chunk_bwd_sweeps(const gdn_args *args, const gdn_chunk_local_args *local, const float *dht, float *dh0, void *stream);
+uint64_t gdn_chunk_bwd_sweeps_workspace_bytes(const gdn_args *args);
+
+/*
  * Measurement aid, no counterpart in the reference: runs exactly what gdn_chunk_fwd runs, with a
  * HIP event recorded on `stream` before and after every kernel, waits for the last one and
  * returns each kernel's duration in milliseconds in kernel_ms[GDN_CHUNK_KERNELS], in launch

@@ -51,6 +51,8 @@ EXPORTED_SYMBOLS = (
     "gdn_chunk_fwd_saving_is_staged",
     "gdn_chunk_bwd_local",
     "gdn_chunk_bwd_prepare",
+    "gdn_chunk_bwd_sweeps",
+    "gdn_chunk_bwd_sweeps_workspace_bytes",
     "gdn_causal_conv1d_fwd",
     "gdn_causal_conv1d_bwd",
     "gdn_gates_fwd",
@@ -259,6 +261,10 @@ def load_library() -> ctypes.CDLL:
     lib.gdn_chunk_bwd_local.restype = ctypes.c_int
     lib.gdn_chunk_bwd_prepare.argtypes = [ctypes.POINTER(GdnChunkBwdPrepareArgs), ctypes.c_void_p]
     lib.gdn_chunk_bwd_prepare.restype = ctypes.c_int
+    lib.gdn_chunk_bwd_sweeps.argtypes = [ctypes.POINTER(GdnArgs), ctypes.POINTER(GdnChunkLocalArgs), ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
+    lib.gdn_chunk_bwd_sweeps.restype = ctypes.c_int
+    lib.gdn_chunk_bwd_sweeps_workspace_bytes.argtypes = [ctypes.POINTER(GdnArgs)]
+    lib.gdn_chunk_bwd_sweeps_workspace_bytes.restype = ctypes.c_uint64
     lib.gdn_causal_conv1d_fwd.argtypes = [ctypes.POINTER(GdnConvArgs), ctypes.c_void_p]
     lib.gdn_causal_conv1d_fwd.restype = ctypes.c_int
     lib.gdn_gated_rmsnorm_bwd.argtypes = [ctypes.POINTER(GdnNormBwdArgs), ctypes.c_void_p]

@@ -7,24 +7,22 @@ the gradients of ``(o, final_state)`` with respect to ``(q, k, v, g, beta, initi
 Three ways through, same formulas:
 
 * bf16, K = 64, 128 or 256, V a multiple of 64 (whole rows, packed or left-padded batches): four kernel launches
-  (``_backward_on_kernels``) - ``gdn_chunk_bwd_prepare``, ``gdn_chunk_fwd_saving`` for the forward sweep and
-  again over the mirror problem for the reverse sweep, ``gdn_chunk_bwd_local``;
+  (``_backward_on_kernels``) - ``gdn_chunk_bwd_sweeps`` (records, forward sweep, reverse sweep) and ``gdn_chunk_bwd_local``;
 * other bf16 shapes (V a multiple of 32 only): the two sweeps over the chunks of a chain on the scan kernel
   (``gdn_chunk_fwd_saving``: the forward's scan in a variant that also writes the chunk states and V~),
   everything chunk-local as batched library GEMMs (fp32, ``torch.bmm``) and elementwise torch operations on
   sequences padded to whole chunks;
 * fp32 inputs, CPU tensors: the sweeps as loops of batched GEMMs as well.
 
-The reverse sweep is the same recurrence as the forward one on other data, which is how it gets onto
-that kernel: with the tokens of a chain in reverse order (a transposed lower-triangular matrix is
-lower-triangular again), chunk c becomes two chunks of a "mirror" problem,
+On the second way the reverse sweep gets onto the forward's scan as the same recurrence on other data: with the tokens of
+a chain in reverse order (a transposed lower-triangular matrix is lower-triangular again), chunk c becomes two chunks of a
+"mirror" problem,
 
     A:  v := P^T dO,  k := k,  T' := T^T,  row scales -(Kd's) and -(Kb's)       =>  V~ = Y = T^T dV~,
         state: exp(gamma_C) dS1 - Kb^T Y
     B:  v := dO,      k := q,  T' := I,    row scale Qe's, no decay             =>  state += Qe^T dO
 
-whose rows and records ``gdn_chunk_bwd_prepare`` writes (``_mirror_problem`` on the second way); the states
-the scan saves at the A chunks are dS1, its output there is Y.
+whose rows and records ``_mirror_problem`` forms; the states the scan saves at the A chunks are dS1, its output there is Y.
 
 Chunk-local quantities (C = 64 tokens, gamma = prefix sum of g inside the chunk, e = exp(gamma),
 E_ij = exp(gamma_i - gamma_j) for j <= i):
@@ -337,83 +335,33 @@ def _chunk_local_grads(qs, kn, vc, doc, Y, Vn, S0, dS1, gam, bc):
 
 
 def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm, cu_seqlens, left_padded, joined):
-    """The whole backward on four kernel launches (bf16; K = 64, 128 or 256; V a multiple of 64): ``gdn_chunk_bwd_prepare``
-    (per-chunk scalars, the mirror problem, and for whole-chunk batches and packed sequences the forward sweep's records),
-    the saving forward sweep, the saving scan over the mirror problem (reverse sweep), ``gdn_chunk_bwd_local`` writing the
-    gradients in the caller's layout.  Chunk states, V~ and Y pass between them as bf16 where the saving scan stages
-    its saves through LDS.  Packed and left-padded batches are laid out with the chunk count of their longest
-    sequence; batches of rows that are not whole chunks run one more launch (their forward sweep prepares its own records)."""
+    """The whole backward on four kernel launches (bf16; K = 64, 128 or 256; V a multiple of 64): ``gdn_chunk_bwd_sweeps``
+    (per-chunk records and scalars, the forward sweep, the reverse sweep; one more launch for the chunk offsets of packed
+    sequences) and ``gdn_chunk_bwd_local`` writing the gradients in the caller's layout.  Chunk states, V~ and Y pass between
+    them as bf16, what the chunk-local products round them to anyway.  Batches that are not whole rows of whole chunks are laid
+    out with the chunk count of their longest sequence."""
     from . import ops  # late: ops imports this module
 
-    B, T, H, K = q.shape
-    V = v.size(-1)
-    dev = q.device
-    packed = cu_seqlens is not None and not left_padded
+    B, T = q.shape[:2]
     covers = True  # every token belongs to a sequence
     if cu_seqlens is None and T % CHUNK == 0:
-        N, NC, sequences, mirror_lengths = B, T // CHUNK, None, None
+        NC, sequences = T // CHUNK, None
     else:
         starts, lens = _chains(B, T, cu_seqlens, left_padded)
-        N, NC = len(lens), max(1, -(-max(lens + [1]) // CHUNK))
+        NC = max(1, -(-max(lens + [1]) // CHUNK))
         covers = sum(lens) == B * T
-        # (a row of the mirror problem is scanned over the two chunks per chunk of ITS sequence, which lie at the row's end, not
-        # over those of the longest one)
-        mirror_chunks = [2 * CHUNK * max(1, -(-length // CHUNK)) for length in lens]
-        *mirror_lengths, seq_start, seq_len = ops.upload_int32((*ops.left_padded_row_lists(mirror_chunks, 2 * NC * CHUNK), starts, lens), dev)
-        sequences = (seq_start, seq_len, NC)
-    Bt = N * H
+        sequences = (*ops.upload_int32((starts, lens), q.device), NC)
     q, k, v, do = (x if x.stride(-1) == 1 else x.contiguous() for x in (q, k, v, do.to(torch.bfloat16)))
-    # The sweeps run on the half-slice scan, one 32-column slice per workgroup, whatever the number of chains: it is the
-    # variant that stages its saves through LDS (bf16, whole lines) and scans without output, which outweighs the records
-    # that four slices per workgroup would share (measured with 2 to 6 workgroups per CU: 1.35 against 2.17 ms at twice
-    # configuration 1's batch, 3.17 against 4.29 ms at B = 12, V = 256).
-    half_slices = True
-    # Where the mirror scan stages its saves through LDS, Y and the gradients of the chunks' final states leave as bf16
-    # (the chunk-local products round them to that anyway; their part in dg, <dS1, S0>, moved by less than its third
-    # digit in every test), and where it is the scan without output it reads the caller's q, k and dO backwards itself
-    # instead of reversed copies of them (whole-chunk batches).
-    staged_m = ops.saving_scan_is_staged(N, 2 * NC * CHUNK, H, K, V, None, False, 2 if half_slices else 1, dev,
-                                         states_dtype=torch.bfloat16, save_every=2)  # fmt: skip
-    mirror_reads = staged_m and K >= 128 and sequences is None
-    # a batch of whole chunks and packed sequences get the forward sweep's records from the same kernel: no prepare launch of
-    # its own (eleven packed documents of 32768 tokens, 16 heads, K = V = 128: 1945 -> 1708 us per training step together with
-    # the single upload above and gradients that are not cleared where sequences cover every token)
-    prep = ops.chunk_bwd_prepare(q, k, do, g, beta, scale, l2norm, V, sequences, half_slice_records=half_slices,
-                                 forward_records=sequences is None or packed, reversed_copies=not mirror_reads,
-                                 skip_empty_chunks=True, packed=packed)  # fmt: skip
-    # Where the saving scan stages its saves through LDS, the sweeps write S0, V~ and Y as bf16 (what the chunk-local
-    # products round them to anyway) and form no output; elsewhere fp32 saves and Y from the mirror scan's output.
-    given = 0 if sequences is not None and not packed else 2 if half_slices else 1
-    staged = ops.saving_scan_is_staged(N, T, H, K, V, cu_seqlens, left_padded, given, dev)
-    # where both sweeps stage their saves, what a scan workgroup saves of a chunk lies in one piece (by 32-column slice)
-    sliced = staged and staged_m
-    saves = dict(dtype=torch.bfloat16 if staged else torch.float32, device=dev)
-    S0 = torch.empty(Bt, NC, K, V, **saves)
-    Vn = torch.empty(Bt, NC, CHUNK, V, **saves)
-    if sequences is None:
-        h0 = None if initial_state is None else initial_state.to(torch.float32).contiguous()
-        ops.chunk_scan_given_records(k, v, prep["records_fwd"], h0, S0, NC, half_slice_records=half_slices, v_new=Vn,
-                                     no_output=True, q=q, sliced=sliced)  # fmt: skip
-    else:
-        ops.chunk_forward_saving(q, k, v, g, beta, scale, initial_state, cu_seqlens, l2norm, left_padded, S0, Vn, NC,
-                                 no_output=True, sliced=sliced, workspace=prep.get("workspace_fwd"))  # fmt: skip
-    dht32 = None if dht is None else dht.to(torch.float32).contiguous()
-    dS1 = torch.empty(Bt, NC, K, V, device=dev, dtype=torch.bfloat16 if staged_m else torch.float32)
-    Y = torch.empty(Bt, NC, CHUNK, V, dtype=torch.bfloat16, device=dev) if staged_m else None
-    o_m, dS = ops.chunk_scan_given_records(k if mirror_reads else prep["k_mirror"], prep["v_mirror"], prep["records"],
-                                           dht32, dS1, NC, save_every=2, save_reverse=True,
-                                           half_slice_records=half_slices, v_new=Y, no_output=staged_m,
-                                           mirror_odd=(q, do) if mirror_reads else None, sliced=sliced,
-                                           valid_lengths=None if mirror_lengths is None else tuple(mirror_lengths))  # fmt: skip
-    dq, dk, dv, dg, dbeta = ops.chunk_local_grads(q, k, v, do, prep, Y if staged_m else o_m, Vn, S0, dS1, scale, l2norm,
-                                                  sequences, sliced=sliced, covers=covers, joined=joined)  # fmt: skip
+    prep, S0, Vn, dS1, Y, dh0 = ops.chunk_bwd_sweeps(q, k, v, do, g, beta, scale, l2norm, initial_state, cu_seqlens, left_padded, dht, NC)
+    dq, dk, dv, dg, dbeta = ops.chunk_local_grads(q, k, v, do, prep, Y, Vn, S0, dS1, scale, l2norm, sequences, sliced=True,
+                                                  covers=covers, joined=joined)  # fmt: skip
     return (
         dq,
         dk,
         dv,
         dg.to(g.dtype) if g is not None else None,
         dbeta.to(beta.dtype) if beta is not None else None,
-        dS if initial_state is not None else None,
+        dh0,
     )
 
 

@@ -279,6 +279,32 @@ int gdn_chunk_bwd_prepare(const gdn_chunk_bwd_prepare_args* a, void* stream) {
     return gdn::launch_chunk_bwd_prepare(*a, static_cast<hipStream_t>(stream));
 }
 
+uint64_t gdn_chunk_bwd_sweeps_workspace_bytes(const gdn_args* a) {
+    if (a == nullptr || !gdn::chunk_shape_supported(*a)) return 0;
+    return gdn::chunk_sweeps_workspace_bytes(*a);
+}
+
+int gdn_chunk_bwd_sweeps(const gdn_args* a, const gdn_chunk_local_args* l, const float* dht, float* dh0, void* stream) {
+    if (l == nullptr) return GDN_ERR_NULL;
+    const int rc = validate_common(a);
+    if (rc != GDN_OK) return rc;
+    if (!gdn::chunk_shape_supported(*a) || a->V % 64 != 0) return GDN_ERR_UNSUPPORTED;
+    const void* needed[] = {l->v_new, l->states, l->dstates, l->gamma, l->beta, l->rq, l->rk, l->y_chunks, l->dout_raw};
+    for (const void* x : needed)
+        if (x == nullptr) return GDN_ERR_NULL;
+        else if (!aligned(x, 16)) return GDN_ERR_ALIGN;
+    if ((dht && !aligned(dht, 16)) || (dh0 && !aligned(dh0, 16))) return GDN_ERR_ALIGN;
+    if (l->saves_dtype != GDN_BF16 || l->dstates_dtype != GDN_BF16 || !l->saves_sliced) return GDN_ERR_UNSUPPORTED;
+    if (l->K != a->K || l->V != a->V || l->H != a->H || l->NC <= 0 || l->chunks != (int64_t)a->N * a->H * l->NC) return GDN_ERR_SHAPE;
+    const int64_t strides[] = {l->dout_stride_b, l->dout_stride_t, l->dout_stride_h};
+    for (int64_t s : strides)
+        if (s < 0 || s % 8 != 0) return GDN_ERR_ALIGN;
+    if (l->dout_stride_t > ((int64_t)1 << 24)) return GDN_ERR_UNSUPPORTED;
+    if (!(a->scale > 0.f)) return GDN_ERR_SHAPE;
+    if (a->workspace == nullptr || a->workspace_bytes < gdn::chunk_sweeps_workspace_bytes(*a) || !aligned(a->workspace, 256)) return GDN_ERR_WORKSPACE;
+    return gdn::launch_chunk_bwd_sweeps(*a, *l, dht, dh0, static_cast<hipStream_t>(stream));
+}
+
 int gdn_causal_conv1d_bwd(const gdn_conv_bwd_args* a, void* stream) {
     if (a == nullptr) return GDN_ERR_NULL;
     if (!a->x || !a->dy || !a->weight || !a->dx || !a->dweight_partial || !a->dbias_partial) return GDN_ERR_NULL;

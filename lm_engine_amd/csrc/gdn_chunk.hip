@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "gdn_chunk_common.h"
+#include "gdn_chunk_sweep.h"
 #include "gdn_launch.h"
 
 namespace gdn {
@@ -157,14 +158,11 @@ int cycle_budget_read(uint64_t* host, int slots) {
 }
 #endif
 
-int launch_chunk_fwd(const gdn_args& a, hipStream_t stream, hipEvent_t* events, const gdn_chunk_saves* saves) {
+// the kernels' parameter block of a call: everything but what a saving call adds
+static ChunkParams chunk_params(const gdn_args& a) {
     const RecordLayout r = record_layout(a.K, a.V);
     ChunkParams p;
     p.cycle_out = nullptr;
-#ifdef GDN_CYCLE_BUDGET
-    p.cycle_out = cycle_buffer();
-    if (p.cycle_out != nullptr) (void)hipMemsetAsync(p.cycle_out, 0, GDN_CYCLE_BUDGET_SLOTS * 8 * sizeof(uint64_t), stream);
-#endif
     p.q = static_cast<const bf16_t*>(a.q);
     p.k = static_cast<const bf16_t*>(a.k);
     p.v = static_cast<const bf16_t*>(a.v);
@@ -187,24 +185,8 @@ int launch_chunk_fwd(const gdn_args& a, hipStream_t stream, hipEvent_t* events, 
     p.save_state = nullptr, p.save_vnew = nullptr, p.save_nc = 0, p.records_given = 0, p.save_every = 1, p.save_reverse = 0;
     p.save_state_bf16 = 0, p.save_vnew_bf16 = 0, p.no_output = 0;
     p.mirror = 0, p.k2 = nullptr, p.v2 = nullptr;
-    p.row_order = saves != nullptr && saves->records_given && left_padded ? saves->row_order : nullptr;
-    p.save_sliced = saves != nullptr && saves->sliced ? 1 : 0;
+    p.row_order = nullptr, p.save_sliced = 0;
     p.k2_stride_b = p.k2_stride_t = p.k2_stride_h = p.v2_stride_b = p.v2_stride_t = p.v2_stride_h = 0;
-    if (saves != nullptr && saves->mirror_reads) {
-        p.mirror = 1, p.k2 = static_cast<const bf16_t*>(saves->k_odd), p.v2 = static_cast<const bf16_t*>(saves->v_odd);
-        p.k2_stride_b = saves->k_odd_stride_b, p.k2_stride_t = saves->k_odd_stride_t, p.k2_stride_h = saves->k_odd_stride_h;
-        p.v2_stride_b = saves->v_odd_stride_b, p.v2_stride_t = saves->v_odd_stride_t, p.v2_stride_h = saves->v_odd_stride_h;
-    }
-    if (saves != nullptr) {
-        p.save_state = static_cast<float*>(saves->states), p.save_vnew = static_cast<float*>(saves->v_new), p.save_nc = saves->chunks_per_chain;
-        p.save_state_bf16 = saves->states_dtype == GDN_BF16 ? 1 : 0, p.save_vnew_bf16 = saves->v_new_dtype == GDN_BF16 ? 1 : 0;
-        p.no_output = saves->no_output ? 1 : 0;
-        p.save_every = saves->save_every > 0 ? saves->save_every : 1, p.save_reverse = saves->save_reverse ? 1 : 0;
-        p.records_given = saves->records_given;
-        // (given records of packed sequences: a workspace of the full layout, the chunk offsets are formed in it below)
-        if (p.records_given && p.cu_seqlens == nullptr) p.chunk_off = nullptr, p.seq_order = nullptr, p.rec = static_cast<uint8_t*>(a.workspace);
-        if (p.records_given) p.ready = nullptr, p.err = nullptr;
-    }
     p.q_stride_b = a.q_stride_b, p.q_stride_t = a.q_stride_t, p.q_stride_h = a.q_stride_h;
     p.k_stride_b = a.k_stride_b, p.k_stride_t = a.k_stride_t, p.k_stride_h = a.k_stride_h;
     p.v_stride_b = a.v_stride_b, p.v_stride_t = a.v_stride_t, p.v_stride_h = a.v_stride_h;
@@ -221,6 +203,32 @@ int launch_chunk_fwd(const gdn_args& a, hipStream_t stream, hipEvent_t* events, 
     p.scan_groups = 1;
     p.fused = (a.flags & GDN_FLAG_FUSED_LAUNCH) ? 1 : 0;
     p.ready_clear = (a.flags & GDN_FLAG_READY_FLAGS_CLEAR) ? 1 : 0;
+    return p;
+}
+
+int launch_chunk_fwd(const gdn_args& a, hipStream_t stream, hipEvent_t* events, const gdn_chunk_saves* saves) {
+    ChunkParams p = chunk_params(a);
+#ifdef GDN_CYCLE_BUDGET
+    p.cycle_out = cycle_buffer();
+    if (p.cycle_out != nullptr) (void)hipMemsetAsync(p.cycle_out, 0, GDN_CYCLE_BUDGET_SLOTS * 8 * sizeof(uint64_t), stream);
+#endif
+    p.row_order = saves != nullptr && saves->records_given && p.pad_lens != nullptr ? saves->row_order : nullptr;
+    p.save_sliced = saves != nullptr && saves->sliced ? 1 : 0;
+    if (saves != nullptr && saves->mirror_reads) {
+        p.mirror = 1, p.k2 = static_cast<const bf16_t*>(saves->k_odd), p.v2 = static_cast<const bf16_t*>(saves->v_odd);
+        p.k2_stride_b = saves->k_odd_stride_b, p.k2_stride_t = saves->k_odd_stride_t, p.k2_stride_h = saves->k_odd_stride_h;
+        p.v2_stride_b = saves->v_odd_stride_b, p.v2_stride_t = saves->v_odd_stride_t, p.v2_stride_h = saves->v_odd_stride_h;
+    }
+    if (saves != nullptr) {
+        p.save_state = static_cast<float*>(saves->states), p.save_vnew = static_cast<float*>(saves->v_new), p.save_nc = saves->chunks_per_chain;
+        p.save_state_bf16 = saves->states_dtype == GDN_BF16 ? 1 : 0, p.save_vnew_bf16 = saves->v_new_dtype == GDN_BF16 ? 1 : 0;
+        p.no_output = saves->no_output ? 1 : 0;
+        p.save_every = saves->save_every > 0 ? saves->save_every : 1, p.save_reverse = saves->save_reverse ? 1 : 0;
+        p.records_given = saves->records_given;
+        // (given records of packed sequences: a workspace of the full layout, the chunk offsets are formed in it below)
+        if (p.records_given && p.cu_seqlens == nullptr) p.chunk_off = nullptr, p.seq_order = nullptr, p.rec = static_cast<uint8_t*>(a.workspace);
+        if (p.records_given) p.ready = nullptr, p.err = nullptr;
+    }
 
     auto mark = [&](int i) {
         if (events != nullptr) (void)hipEventRecord(events[i], stream);
@@ -234,6 +242,48 @@ int launch_chunk_fwd(const gdn_args& a, hipStream_t stream, hipEvent_t* events, 
     const int rc = launch_chunk32(p, a.K, stream, events, compute_units());
     mark(3);
     return rc;
+}
+
+// ------------------------------------------------------------------------------------------
+// the backward's two sweeps: prepare (records of both), forward sweep, reverse sweep
+// ------------------------------------------------------------------------------------------
+int launch_prepare_sweeps(ChunkParams& p, const SweepScalars& sw, int K, hipStream_t stream, int num_cus);  // gdn_chunk_prepare.hip
+int launch_chunk_sweeps(const SweepParams& fwd, const SweepParams& rev, int K, hipStream_t stream);          // gdn_chunk_sweep.hip
+
+uint64_t chunk_sweeps_workspace_bytes(const gdn_args& a) {
+    return chunk_off_bytes(a) + (uint64_t)a.H * chunk_slots(a) * SWEEP_RECORD_BYTES;
+}
+
+int launch_chunk_bwd_sweeps(const gdn_args& a, const gdn_chunk_local_args& l, const float* dht, float* dh0, hipStream_t stream) {
+    ChunkParams p = chunk_params(a);
+    p.rec = static_cast<uint8_t*>(a.workspace) + chunk_off_bytes(a);
+    p.rec_bytes = SWEEP_RECORD_BYTES;
+    p.ready = nullptr, p.err = nullptr;
+    SweepScalars sw;
+    sw.gamma = const_cast<float*>(l.gamma), sw.beta = const_cast<float*>(l.beta), sw.rq = const_cast<float*>(l.rq), sw.rk = const_cast<float*>(l.rk);
+    sw.nc = l.NC;
+    SweepParams f;
+    f.q = p.q, f.k = p.k, f.v = p.v;
+    f.q_stride_b = a.q_stride_b, f.q_stride_t = a.q_stride_t, f.q_stride_h = a.q_stride_h;
+    f.k_stride_b = a.k_stride_b, f.k_stride_t = a.k_stride_t, f.k_stride_h = a.k_stride_h;
+    f.v_stride_b = a.v_stride_b, f.v_stride_t = a.v_stride_t, f.v_stride_h = a.v_stride_h;
+    f.rec = p.rec, f.rec_bytes = p.rec_bytes;
+    f.s_in = a.h0, f.s_out = nullptr;
+    f.save_state = static_cast<bf16_t*>(const_cast<void*>(l.states)), f.save_v = static_cast<bf16_t*>(const_cast<void*>(l.v_new));
+    f.save_nc = l.NC;
+    f.cu_seqlens = p.cu_seqlens, f.pad_lens = p.pad_lens, f.chunk_off = p.chunk_off, f.seq_order = p.seq_order;
+    f.T = p.T, f.H = p.H, f.V = p.V, f.N = p.N, f.NT = p.NT, f.TC = p.TC, f.qk_div = p.qk_div;
+    SweepParams r = f;
+    r.v = static_cast<const bf16_t*>(l.dout_raw);
+    r.v_stride_b = l.dout_stride_b, r.v_stride_t = l.dout_stride_t, r.v_stride_h = l.dout_stride_h;
+    r.s_in = dht, r.s_out = dh0;
+    r.save_state = static_cast<bf16_t*>(const_cast<void*>(l.dstates)), r.save_v = static_cast<bf16_t*>(const_cast<void*>(l.y_chunks));
+    if (p.cu_seqlens != nullptr) {
+        hipLaunchKernelGGL(chunk_offsets_kernel, dim3(1), dim3(256), 0, stream, p.cu_seqlens, p.chunk_off, p.seq_order, p.N, p.T, p.TC);
+        if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
+    }
+    if (const int rc = launch_prepare_sweeps(p, sw, a.K, stream, compute_units()); rc != GDN_OK) return rc;
+    return launch_chunk_sweeps(f, r, a.K, stream);
 }
 
 }  // namespace gdn

@@ -43,33 +43,9 @@
 #include <type_traits>
 
 #include "gdn_chunk32_common.h"
-#include "gdn_chunk_prepare32.h"
 #include "gdn_launch.h"
 
 namespace gdn {
-
-// ------------------------------------------------------------------------------------------
-// prepare as a kernel of its own: persistent workgroups of four waves, three per CU
-// ------------------------------------------------------------------------------------------
-template <int K>
-__global__ __launch_bounds__(PREP_THREADS, (K > 128 ? 1 : 3)) void chunk_prepare32_kernel(const ChunkParams p) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[prepare32_lds_bytes<K>()];
-    // Work items: (chunk slot, head), the slots rounded up to a multiple of 8.  Workgroup i runs on XCD i % 8 and
-    // takes items i, i + grid, ... with the grid a multiple of 8, so w % 8 names the XCD.  That digit goes into
-    // the slot number and the heads rotate with the rest: every XCD works on all heads.  The rows of one head
-    // lie a whole token row (a multiple of 2 KiB) apart, so they fall on few channels of an XCD's L2; an XCD
-    // that only ever sees one or two heads would send all its q, k, v traffic there.
-    const uint32_t items = (uint32_t)((p.TC + 7) / 8) * 8u * (uint32_t)p.H;  // the launcher rejects more than 2^31
-    if (blockIdx.x >= items) return;
-    const uint32_t H = (uint32_t)p.H;
-    auto item_of = [H](uint32_t w, int& h, int& slot) {
-        const uint32_t j = w / 8u, jh = j / H;
-        h = (int)(j - jh * H);
-        slot = (int)(jh * 8u + w % 8u);
-    };
-    const uint32_t rounds = (items - blockIdx.x + gridDim.x - 1) / gridDim.x;
-    chunk_prepare32_body<K, 1, false>(p, lds, item_of, items, blockIdx.x, gridDim.x, rounds, nullptr, 0);
-}
 
 // ------------------------------------------------------------------------------------------
 // scan
@@ -1349,7 +1325,8 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
 // ------------------------------------------------------------------------------------------
 // launch
 // ------------------------------------------------------------------------------------------
-int launch_chunk_fused(ChunkParams& p, int K, hipStream_t stream, int num_cus);  // gdn_chunk_fused.hip
+int launch_chunk_fused(ChunkParams& p, int K, hipStream_t stream, int num_cus);        // gdn_chunk_fused.hip
+int launch_prepare32(const ChunkParams& p, int K, hipStream_t stream, int num_cus);  // gdn_chunk_prepare.hip
 
 // Which scan kernel a launch gets: compute waves (32-column slices) per workgroup, and whether a slice is split over
 // two half-slice waves.
@@ -1388,10 +1365,6 @@ ScanPlan plan_scan(int K, int64_t chains, int V, bool packed, bool save, int rec
 
 template <int K>
 static int launch32(ChunkParams& p, hipStream_t stream, hipEvent_t* events, int num_cus) {
-    const int64_t items = (int64_t)((p.TC + 7) / 8) * 8 * p.H;  // a multiple of 8, see the kernel
-    const int64_t cap = (int64_t)(3 * num_cus + 7) / 8 * 8;      // three workgroups per CU (LDS and registers allow it)
-    if (items >= ((int64_t)1 << 31)) return GDN_ERR_UNSUPPORTED;  // the kernel counts items in 32 bits
-    const int grid_prep = (int)(items < cap ? items : cap);
     p.rec16 = 0;
     if (p.fused) {  // prepare and scan in one launch, when the shape qualifies
         if (events != nullptr) (void)hipEventRecord(events[2], stream);
@@ -1411,8 +1384,7 @@ static int launch32(ChunkParams& p, hipStream_t stream, hipEvent_t* events, int 
     if ((p.save_state_bf16 || p.save_vnew_bf16) && !plan.staged_saves) return GDN_ERR_UNSUPPORTED;  // (the C entry asks plan_scan first)
     p.rec16 = half ? 1 : 0;
     if (!p.records_given) {
-        hipLaunchKernelGGL((chunk_prepare32_kernel<K>), dim3(grid_prep), dim3(PREP_THREADS), 0, stream, p);
-        if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
+        if (const int rc = launch_prepare32(p, K, stream, num_cus); rc != GDN_OK) return rc;
     }
     if (events != nullptr) (void)hipEventRecord(events[2], stream);
     p.scan_groups = vtiles / nw;

@@ -120,9 +120,9 @@ inline RecordLayout record_layout(int K, int V) {
     return r;
 }
 
-// Where chunk slot `slot` of the grid lives: sequence, first token, valid length (0 = unused slot).
+// Where chunk slot `slot` of the grid lives: sequence, chunk of it, first token, valid length (0 = unused slot).
 struct ChunkCoord {
-    int n;
+    int n, c;
     int64_t b, t0;
     int len;
 };
@@ -130,13 +130,13 @@ struct ChunkCoord {
 __device__ __forceinline__ ChunkCoord locate_chunk(const ChunkParams& p, int slot) {
     ChunkCoord cc;
     if (slot >= p.TC) {  // past the last slot (the item grid of prepare is rounded up): nothing there
-        cc.n = 0, cc.b = 0, cc.t0 = 0, cc.len = 0;
+        cc.n = 0, cc.c = 0, cc.b = 0, cc.t0 = 0, cc.len = 0;
         return cc;
     }
     if (p.cu_seqlens == nullptr) {
         cc.n = slot / p.NT;
         const int c = slot - cc.n * p.NT;
-        cc.b = cc.n;
+        cc.b = cc.n, cc.c = c;
         // the last `len` tokens of the row (clamped: a malformed prefix must not send a load out of the row)
         const int len = p.pad_lens == nullptr ? p.T : min(max(p.pad_lens[cc.n + 1] - p.pad_lens[cc.n], 0), p.T);
         cc.t0 = (int64_t)(p.T - len) + (int64_t)c * C;
@@ -145,7 +145,7 @@ __device__ __forceinline__ ChunkCoord locate_chunk(const ChunkParams& p, int slo
     }
     cc.b = 0;
     if (slot >= p.chunk_off[p.N]) {
-        cc.n = 0, cc.t0 = 0, cc.len = 0;
+        cc.n = 0, cc.c = 0, cc.t0 = 0, cc.len = 0;
         return cc;
     }
     int lo = 0, hi = p.N;  // largest n with chunk_off[n] <= slot
@@ -156,6 +156,7 @@ __device__ __forceinline__ ChunkCoord locate_chunk(const ChunkParams& p, int slo
     }
     cc.n = lo;
     const int c = slot - p.chunk_off[lo];
+    cc.c = c;
     int t0, len;
     packed_bounds(p.cu_seqlens, lo, p.T, t0, len);
     cc.t0 = (int64_t)t0 + (int64_t)c * C;

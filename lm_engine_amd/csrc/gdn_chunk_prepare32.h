@@ -4,6 +4,7 @@
 #pragma once
 
 #include "gdn_chunk32_common.h"
+#include "gdn_chunk_sweep.h"
 
 namespace gdn {
 
@@ -59,15 +60,18 @@ constexpr int prepare32_lds_bytes() {
 //                    of the workgroup (a group whose item index runs past `items` only keeps the barriers company)
 //   FLAGS, ready     ready[h * TC + slot] is set to `epoch` once the record is complete and visible to the whole
 //                    device (the scan of the same launch waits for it)
-template <int K, int GROUPS, bool FLAGS, typename ItemOf>
+//   SWEEP, sw        the records are those of the backward's sweeps (gdn_chunk_sweep.h), and gamma, beta and the inverse norms
+//                    go out per token as well
+template <int K, int GROUPS, bool FLAGS, bool SWEEP, typename ItemOf>
 __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8_t* lds_base, ItemOf item_of, uint32_t items,
-                                                     uint32_t first, uint32_t step, uint32_t rounds, int32_t* ready, int32_t epoch) {
+                                                     uint32_t first, uint32_t step, uint32_t rounds, int32_t* ready, int32_t epoch,
+                                                     const SweepScalars& sw) {
+    static_assert(!SWEEP || !FLAGS, "the sweeps have a prepare launch of their own");
     constexpr int LDK = K + 8;  // bf16 elements per LDS row of K / Q
     constexpr int LDA = C + 4;  // fp32 elements per LDS row of A / T
     constexpr int LDT = 36;     // fp32 elements per row of the 32 x 32 transposed blocks
     constexpr int LDM = 20;     // fp32 elements per row of a 16 x 16 scratch block
     constexpr int KS16 = K / 16;
-    constexpr int KD = K / 32;  // 32-row tiles of the key dim
     constexpr int CPR = K / 8;  // 16 B pieces per row of K / Q
     constexpr int RPP = PREP_THREADS / CPR;  // rows per pass of the K / Q copy
     constexpr int NPASS = C / RPP;
@@ -105,7 +109,7 @@ __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8
             item_of(w, nh, nslot);
             ncc = locate_chunk(p, nslot);
         } else {
-            nh = 0, nslot = 0, ncc.n = 0, ncc.b = 0, ncc.t0 = 0, ncc.len = 0;
+            nh = 0, nslot = 0, ncc.n = 0, ncc.c = 0, ncc.b = 0, ncc.t0 = 0, ncc.len = 0;
         }
     };
     // Loads are written as (workgroup-uniform base pointer) + (32-bit per-lane element offset) so that the
@@ -152,7 +156,6 @@ __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8
         asm volatile("" : "+v"(lane));
         const int l16 = lane % 16, lq = lane / 16;  // 16 x 16 MFMA coordinates
         const int l32 = lane % 32, lh = lane / 32;  // 32 x 32 MFMA coordinates
-        const int g16 = l32 / 16;                   // which 16-lane group of the 32-row operand
         const ChunkCoord cc = ncc;
         const int h = nh;
         const int len = cc.len;  // <= 0 for an unused slot (packed batch, rounded-up grid): nothing to do
@@ -225,16 +228,27 @@ __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8
             // row scales the scan applies: to q S0, to the rows of V~ in the state update, to k S0 (none for
             // the rows past the end of a short chunk: the scan reads some other token's k and v there)
             const bool valid = tid < len;
-            record_store<FLAGS>(rec, p.rec_bytes, p.off_qs + 4 * tid, __expf(gam) * p.scale * rq);
-            record_store<FLAGS>(rec, p.rec_bytes, p.off_ks + 4 * tid, valid ? __expf(gl - gam) * rk : 0.f);
-            record_store<FLAGS>(rec, p.rec_bytes, p.off_cs + 4 * tid, valid ? __expf(gam) * rk : 0.f);
-            if (tid == 0) record_store<FLAGS>(rec, p.rec_bytes, p.off_eg, __expf(gl));
+            if constexpr (SWEEP) {
+                const float e = __expf(gam), ks = valid ? __expf(gl - gam) * rk : 0.f, cs = valid ? e * rk : 0.f, eg = __expf(gl);
+                float* const f = reinterpret_cast<float*>(rec + SWEEP_REC_FWD_SCALES) + tid;
+                float* const r = reinterpret_cast<float*>(rec + SWEEP_REC_REV_SCALES) + tid;
+                f[0] = ks, f[C] = cs, f[2 * C] = eg;
+                r[0] = valid ? e * p.scale * rq : 0.f, r[C] = ks, r[2 * C] = -(s_beta[tid] * cs), r[3 * C] = eg;
+                const int64_t at = (((int64_t)cc.n * p.H + h) * sw.nc + cc.c) * C + tid;
+                if (cc.c < sw.nc) sw.gamma[at] = gam, sw.beta[at] = s_beta[tid], sw.rq[at] = rq, sw.rk[at] = rk;
+            } else {
+                record_store<FLAGS>(rec, p.rec_bytes, p.off_qs + 4 * tid, __expf(gam) * p.scale * rq);
+                record_store<FLAGS>(rec, p.rec_bytes, p.off_ks + 4 * tid, valid ? __expf(gl - gam) * rk : 0.f);
+                record_store<FLAGS>(rec, p.rec_bytes, p.off_cs + 4 * tid, valid ? __expf(gam) * rk : 0.f);
+                if (tid == 0) record_store<FLAGS>(rec, p.rec_bytes, p.off_eg, __expf(gl));
+            }
         }
         __syncthreads();  // #2
 
         // ---- A = strict-lower(beta_i e^{gamma_i - gamma_j} k^_i . k^_j) -> sA;  P -> record ----
         {
-            // 32 x 32 tile jobs: G(Ti, Tj) = K_Ti K_Tj^T (rows i, column j), Pt(Tj, Ti) = K_Tj Q_Ti^T (rows j, column i)
+            // 32 x 32 tile jobs: G(Ti, Tj) = K_Ti K_Tj^T (rows i, column j), Pt(Tj, Ti) = K_Tj Q_Ti^T (rows j, column i; SWEEP: its
+            // transpose, so that a lane holds consecutive rows i of P^T's reduction)
             auto tile_job = [&](bool is_p, int trow, int tcol) {
                 f32x16 acc;
 #pragma unroll
@@ -244,7 +258,7 @@ __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8
                 for (int s = 0; s < KS16; s++) {
                     const bf16x8 a = *reinterpret_cast<const bf16x8*>(&sK[(32 * trow + l32) * LDK + 16 * s + 8 * lh]);
                     const bf16x8 b = *reinterpret_cast<const bf16x8*>(&bsrc[(32 * tcol + l32) * LDK + 16 * s + 8 * lh]);
-                    acc = mfma32_bf16(a, b, acc);
+                    acc = SWEEP && is_p ? mfma32_bf16(b, a, acc) : mfma32_bf16(a, b, acc);
                     if (s % 2 == 1) __builtin_amdgcn_sched_barrier(0);  // keeps the operand reads from piling up in registers
                 }
                 // register quad q of the tile holds rows 32 trow + 8 q + 4 h + 0..3: their per-token values in one read
@@ -261,6 +275,29 @@ __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8
                             const float val = bi[e] * __builtin_amdgcn_exp2f(gi[e] - gj) * (rkj * acc[4 * q + e]);
                             sA[(i0 + e) * LDA + j] = (trow > tcol || i0 + e > j) ? val : 0.f;
                         }
+                    }
+                } else if constexpr (SWEEP) {
+                    // P^T: tokens i = 32 tcol + 8 q + 4 h + 0..3 of this lane's key token j.  16x16x32 fragment of the rows
+                    // 16 (j / 16) .. and the 32 reduction tokens 32 tcol ..: lane (j % 16, g) holds the tokens 4 g + 0..3 and
+                    // 16 + 4 g + 0..3 of the slab, here a half of g = 2 (q % 2) + h.  The fragments are numbered as those of the
+                    // lower triangle that P^T is with rows and columns in reverse order.
+                    const int j = 32 * trow + l32;
+                    const float gj = s_g2[j], rkj = s_rk[j];
+                    const int lt = 3 - (2 * trow + l32 / 16), ls = 1 - tcol;
+                    const int frag = lt < 2 ? lt : 2 * lt - 2 + ls;
+#pragma unroll
+                    for (int q = 0; q < 4; q++) {
+                        const int i0 = 32 * tcol + 8 * q + 4 * lh;
+                        const f32x4 ri = *reinterpret_cast<const f32x4*>(&s_rq[i0]);
+                        const f32x4 gi = *reinterpret_cast<const f32x4*>(&s_g2[i0]);
+                        bf16x4 piece;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const float val = rkj * __builtin_amdgcn_exp2f(gi[e] - gj) * (p.scale * ri[e] * acc[4 * q + e]);
+                            piece[e] = (bf16_t)((tcol > trow || i0 + e >= j) ? val : 0.f);
+                        }
+                        const int g = 2 * (q % 2) + lh;
+                        *reinterpret_cast<bf16x4*>(rec + SWEEP_REC_REV_P + (frag * WAVE + 16 * g + l32 % 16) * 16 + 8 * (q / 2)) = piece;
                     }
                 } else {
                     const int i = 32 * tcol + l32;
@@ -425,6 +462,17 @@ __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8
                 r[4 + e] = (bf16_t)(t1[e] * c1[e]);
             }
             record_store<FLAGS>(rec, p.rec_bytes, (f * WAVE + lane) * 16, r);
+            if constexpr (SWEEP) {
+                // T^T, fragments numbered like P^T's: lane (row i of the 16-row tile, g) holds T[32 s + 4 g + 0..3, + 16][i]
+                const int row = 16 * (3 - tt16) + l16, c0 = 32 * (1 - s16) + 4 * lq;
+                bf16x8 tr;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    tr[e] = (bf16_t)sT[(c0 + e) * LDA + row];
+                    tr[4 + e] = (bf16_t)sT[(c0 + 16 + e) * LDA + row];
+                }
+                *reinterpret_cast<bf16x8*>(rec + SWEEP_REC_REV + (f * WAVE + lane) * 16) = tr;
+            }
         }
         if constexpr (FLAGS) __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's part of the record has reached memory
         __syncthreads();  // #8: LDS is reused by the next item

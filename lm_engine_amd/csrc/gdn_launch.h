@@ -38,6 +38,9 @@ bool chunk_bwd_local_supported(const gdn_chunk_local_args& a);
 int launch_chunk_bwd_prepare(const gdn_chunk_bwd_prepare_args& a, hipStream_t stream);
 bool chunk_bwd_prepare_supported(const gdn_chunk_bwd_prepare_args& a);
 uint64_t chunk_bwd_record_bytes(const gdn_chunk_bwd_prepare_args& a);
+// prepare, forward sweep and reverse sweep of the backward (gdn_chunk_bwd_sweeps)
+int launch_chunk_bwd_sweeps(const gdn_args& a, const gdn_chunk_local_args& l, const float* dht, float* dh0, hipStream_t stream);
+uint64_t chunk_sweeps_workspace_bytes(const gdn_args& a);
 int launch_conv_bwd(const gdn_conv_bwd_args& a, hipStream_t stream);  // gdn_conv1d_bwd.hip
 #ifdef GDN_CYCLE_BUDGET
 uint64_t* cycle_buffer();  // gdn_chunk.hip, measurement build only: the device buffer sampled waves report their cycles into

@@ -592,6 +592,45 @@ def chunk_local_grads(q, k, v, dout, prep, y_mirror, v_new, states, dstates, sca
     return out["dq_out"], out["dk_out"], out["dv_out"], out["dg_out"], out["dbeta_out"]
 
 
+def chunk_bwd_sweeps(q, k, v, dout, g, beta, scale, l2norm, initial_state, cu_seqlens, left_padded, dht, chunks_per_chain):
+    """``gdn_chunk_bwd_sweeps``: q, k, v, dout are the caller's bf16 ``[B, T, H, D]`` tensors (last dim contiguous), ``dht`` the
+    gradient of the final state or None, ``chunks_per_chain`` (NC) at least the chunks of the longest sequence.  Returns
+    ``prep`` (``gamma, beta, rq, rk`` fp32 ``[N H, NC, 64]``) and, bf16 by 32-column slice, the states the chunks start from, V~, the
+    gradients of the states they end with and Y with its tokens reversed - ``chunk_local_grads(..., sliced=True)`` takes them all -
+    and the gradient of the initial state (None without one).  Chunks past the end of their sequence have no entries."""
+    _require_hip_path()
+    lib = _lib.load_library()
+    dims = _check_inputs(q, k, v, g, beta, initial_state, cu_seqlens, left_padded)
+    B, T, H, K, V, N = dims
+    NC, dev = chunks_per_chain, q.device
+    g = None if g is None else g.to(torch.float32).contiguous()
+    if beta is not None:
+        beta = beta.contiguous() if beta.dtype in (torch.bfloat16, torch.float32) else beta.float().contiguous()
+    cu_seqlens = None if cu_seqlens is None else cu_seqlens.to(torch.int32).contiguous()
+    h0 = None if initial_state is None else initial_state.contiguous()
+    dht = None if dht is None else dht.to(torch.float32).contiguous()
+    prep = {name: torch.empty(N * H, NC, 64, dtype=torch.float32, device=dev) for name in ("gamma", "beta", "rq", "rk")}
+    states, dstates = (torch.empty(N * H, NC, K, V, dtype=torch.bfloat16, device=dev) for _ in range(2))
+    v_new, y = (torch.empty(N * H, NC, 64, V, dtype=torch.bfloat16, device=dev) for _ in range(2))
+    dh0 = None if h0 is None else torch.empty(N, H, K, V, dtype=torch.float32, device=dev)
+    args = _fill_args(q, k, v, g, beta, h0, None, v, cu_seqlens, scale, l2norm, False, dims, left_padded)  # (no output is written)
+    workspace = torch.empty(int(lib.gdn_chunk_bwd_sweeps_workspace_bytes(ctypes.byref(args))), dtype=torch.uint8, device=dev)
+    args.workspace, args.workspace_bytes = workspace.data_ptr(), workspace.numel()
+    a = _lib.GdnChunkLocalArgs()
+    a.gamma, a.beta, a.rq, a.rk = (prep[name].data_ptr() for name in ("gamma", "beta", "rq", "rk"))
+    a.v_new, a.states, a.dstates, a.y_chunks = v_new.data_ptr(), states.data_ptr(), dstates.data_ptr(), y.data_ptr()
+    a.saves_dtype = a.dstates_dtype = _lib.GDN_BF16
+    a.saves_sliced = 1
+    a.chunks, a.K, a.V, a.H, a.NC = N * H * NC, K, V, H, NC
+    a.dout_raw = dout.data_ptr()
+    a.dout_stride_b, a.dout_stride_t, a.dout_stride_h = dout.stride(0), dout.stride(1), dout.stride(2)
+    with torch.cuda.device(dev):
+        stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+        _lib.check_status(lib.gdn_chunk_bwd_sweeps(ctypes.byref(args), ctypes.byref(a), None if dht is None else dht.data_ptr(),
+                                                   None if dh0 is None else dh0.data_ptr(), stream), "gdn_chunk_bwd_sweeps")  # fmt: skip
+    return prep, states, v_new, dstates, y, dh0
+
+
 RECORD_BYTES = 13312  # a chunk record: 12 operand fragments, 3 x 64 row scales, e^{gamma_C}
 
 

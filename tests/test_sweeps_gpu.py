@@ -1,0 +1,97 @@
+"""``gdn_chunk_bwd_sweeps`` against both sweeps in fp64 (the formulas of lm_engine_amd/backward.py): what the forward and the reverse
+sweep save per chunk, and the gradient of the initial state."""
+
+import pytest
+import torch
+
+from tests.helpers import rel_l2
+
+
+C = 64
+
+
+def _reference(q, k, v, do, g, beta, scale, h0, dht, spans):
+    """Per sequence ``(row, start, length)``: S0, V~, dS1, Y of every chunk and dS0, fp64, from the rounded inputs."""
+    H, group = v.size(2), v.size(2) // q.size(2)
+    out = []
+    for n, (row, start, length) in enumerate(spans):
+        NC = -(-length // C)
+        pad = lambda x: torch.nn.functional.pad(x[row, start : start + length].double().movedim(1, 0), (0, 0, 0, NC * C - length))  # noqa: E731
+        qs, ks = (pad(x).repeat_interleave(group, dim=0) for x in (q, k))
+        qs, ks = (x * torch.rsqrt(x.square().sum(-1, keepdim=True) + 1e-6) for x in (qs, ks))
+        qs = qs * scale
+        vs, ds = pad(v), pad(do)
+        gs, bs = (pad(x[..., None])[..., 0] for x in (g, beta))
+        chunks = lambda x: x.reshape(H, NC, C, *x.shape[2:])  # noqa: E731
+        qs, ks, vs, ds, gs, bs = (chunks(x) for x in (qs, ks, vs, ds, gs, bs))
+        gam = gs.cumsum(-1)
+        e, tail, egl = gam.exp(), (gam[..., -1:] - gam).exp(), gam[..., -1].exp()
+        E = (gam[..., :, None] - gam[..., None, :]).exp().tril()
+        A = (bs[..., None] * E * (ks @ ks.transpose(-1, -2))).tril(-1)
+        T = torch.linalg.inv(torch.eye(C, dtype=torch.float64) + A)
+        P = E * (qs @ ks.transpose(-1, -2))
+        S = h0[n].double() if h0 is not None else torch.zeros(H, q.size(-1), v.size(-1), dtype=torch.float64)
+        dS = dht[n].double() if dht is not None else torch.zeros_like(S)
+        S0, Vn, dS1, Y = [], [], [None] * NC, [None] * NC
+        for c in range(NC):
+            S0.append(S)
+            Vn.append(T[:, c] @ (bs[:, c, :, None] * (vs[:, c] - e[:, c, :, None] * (ks[:, c] @ S))))
+            S = egl[:, c, None, None] * S + (tail[:, c, :, None] * ks[:, c]).transpose(-1, -2) @ Vn[c]
+        for c in reversed(range(NC)):
+            dS1[c] = dS
+            Y[c] = T[:, c].transpose(-1, -2) @ (P[:, c].transpose(-1, -2) @ ds[:, c] + tail[:, c, :, None] * (ks[:, c] @ dS))
+            dS = (egl[:, c, None, None] * dS + (e[:, c, :, None] * qs[:, c]).transpose(-1, -2) @ ds[:, c]
+                  - (bs[:, c, :, None] * e[:, c, :, None] * ks[:, c]).transpose(-1, -2) @ Y[c])  # fmt: skip
+        out.append((S0, Vn, dS1, Y, dS))
+    return out
+
+
+def _rows(sliced, rows, V):  # [.., V / 32, rows, 32] in the memory of [.., rows, V]
+    return sliced.reshape(*sliced.shape[:-2], V // 32, rows, 32).transpose(-3, -2).reshape(*sliced.shape[:-2], rows, V).double().cpu()
+
+
+# one to six chunks (the loaders' ring fills and drains differently up to five), first and last token of a chunk, empty sequences,
+# shared heads of q and k, one and several column slices
+CASES = [
+    *(("rows", [T], K, 64, 2, 2) for K in (64, 128, 256) for T in (1, 63, 64, 65, 128, 192, 257, 384)),
+    *(("packed", [100, 0, 64, 1, 333], K, V, 1, 2) for K, V in ((64, 64), (128, 128), (256, 64), (256, 512))),
+    *(("padded", [200, 70, 0, 1], K, 128, 3, 3) for K in (64, 128, 256)),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout, lens, K, V, HK, H", CASES)
+def test_sweeps_match_the_formulas(layout, lens, K, V, HK, H):
+    from lm_engine_amd import ops
+
+    gen = torch.Generator().manual_seed(sum(lens) + K + V)
+    N = len(lens)
+    B, T = (1, sum(lens)) if layout == "packed" else (N, max(lens))
+    normal = lambda *shape: torch.randn(*shape, generator=gen)  # noqa: E731
+    q, k, v, do = (normal(B, T, *s).bfloat16() for s in ((HK, K), (HK, K), (H, V), (H, V)))
+    g, beta = torch.nn.functional.logsigmoid(3 + normal(B, T, H)), normal(B, T, H).sigmoid().bfloat16()
+    h0, dht = 0.1 * normal(N, H, K, V), 0.1 * normal(N, H, K, V)
+    starts = [sum(lens[:n]) for n in range(N)]
+    spans = [(0, starts[n], lens[n]) if layout == "packed" else (n, T - lens[n], lens[n]) for n in range(N)]
+    cu = None if layout == "rows" else torch.tensor([*starts, sum(lens)], dtype=torch.int32).cuda()
+    scale, NC = K**-0.5, max(1, -(-max(lens) // C))
+    want = _reference(q, k, v, do, g, beta, scale, h0, dht, spans)
+    prep, S0, Vn, dS1, Y, dh0 = ops.chunk_bwd_sweeps(*(x.cuda() for x in (q, k, v, do, g, beta)), scale, True, h0.cuda(), cu,
+                                                     layout == "padded", dht.cuda(), NC)  # fmt: skip
+    S0, dS1 = (_rows(x.view(N, H, NC, K, V), K, V) for x in (S0, dS1))
+    Vn, Y = (_rows(x.view(N, H, NC, C, V), C, V) for x in (Vn, Y))
+    for n, (s0, vn, ds1, y, ds0) in enumerate(want):
+        # operands rounded to bf16 on the way (2^-9 each) and results saved as bf16: the operator's own gate, 1e-2 in the 2-norm
+        assert rel_l2(dh0[n].cpu(), ds0) < 1e-2, f"dh0 of sequence {n}"
+        for c in range(len(s0)):
+            live = min(C, lens[n] - C * c)
+            assert rel_l2(S0[n, :, c], s0[c]) < 1e-2, f"state of sequence {n}, chunk {c}"
+            assert rel_l2(dS1[n, :, c], ds1[c]) < 1e-2, f"gradient of the state of sequence {n}, chunk {c}"
+            assert rel_l2(Vn[n, :, c, :live], vn[c][:, :live]) < 1e-2, f"V~ of sequence {n}, chunk {c}"
+            assert rel_l2(Y[n, :, c].flip(-2)[:, :live], y[c][:, :live]) < 1e-2, f"Y of sequence {n}, chunk {c}"
+            assert Y[n, :, c].flip(-2)[:, live:].abs().sum() == 0, "rows past the end"  # the chunk-local kernel reads them
+        gamma = torch.cat([prep["gamma"].view(N, H, NC * C)[n, :, C * c : C * c + 1] for c in range(len(s0))], dim=1) if s0 else None
+        if s0:
+            row, start, _ = spans[n]
+            first = torch.stack([g[row, start + C * c] for c in range(len(s0))], dim=1)
+            assert torch.equal(gamma.cpu(), first), "prefix sums start at the chunk's first token"
