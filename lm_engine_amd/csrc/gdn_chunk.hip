@@ -11,7 +11,7 @@
 //     O  = diag(e^gamma scale) Q^ S0 + P V~,   P_ij = scale e^{gamma_i - gamma_j} (q^_i . k^_j)  (i >= j)
 //     S_C = e^{gamma_C} S0 + K~^T V~,          K~_j = e^{gamma_C - gamma_j} k^_j
 //
-// Two steps, both in gdn_chunk32.hip (one launch each, or one launch for both: gdn_chunk_fused.hip):
+// Two steps, gdn_chunk_prepare32.h and gdn_chunk_scan32.h (one launch each, or one launch for both: gdn_chunk_fused.hip):
 //   prepare (parallel over every chunk and head): everything that does not depend on the state - K K^T, the
 //       triangular inverse, P and the row scales - written to a workspace record per (head, chunk) as bf16 MFMA
 //       operand fragments, in the register order the scan consumes them;

@@ -1,4 +1,4 @@
-// Device helpers shared by the kernels built on v_mfma_f32_32x32x16_bf16 (gdn_chunk32.hip, gdn_chunk_fused.hip).
+// Device helpers shared by the kernels built on v_mfma_f32_32x32x16_bf16 (gdn_chunk_scan32.h, gdn_chunk_fused.hip).
 #pragma once
 
 #include <type_traits>

@@ -1,7 +1,7 @@
 // The chunked forward as ONE launch (K <= 128, fixed-length batches whose scan fills about half of the CUs):
 // producer workgroups run the prepare step and scan workgroups consume its records as they appear.
 //
-// Scan workgroups.  gdn_chunk32.hip's scan gives one wave a whole 32-column slice of the state, and a slice a CU.
+// Scan workgroups.  gdn_chunk_scan32.h's scan gives one wave a whole 32-column slice of the state, and a slice a CU.
 // Here a workgroup holds two slices of a chain (64 columns: whole 128-byte lines of the output) and each slice is
 // shared by a PAIR of compute waves on two SIMDs, so the scan of a batch needs half as many CUs and leaves the
 // others to the producers.  Wave tt (0 or 1) of a pair owns
@@ -10,7 +10,7 @@
 //   * key half tt (state rows K/2 tt .. K/2 tt + K/2 - 1) of the state, as MFMA accumulators, in the update
 //     S = e^{gamma_C} S + K^T diag(ks) V~.
 // So each product is split by its OUTPUT rows: no partial sums are ever added across waves, every
-// accumulator keeps the register layout of gdn_chunk32.hip (so an accumulator tile still turns into the
+// accumulator keeps the register layout of gdn_chunk_scan32.h (so an accumulator tile still turns into the
 // next MFMA's operand without leaving registers), and what a wave lacks are operands only, all bf16:
 //   1. the partner's half of S0 as B / A operand of K S0 and (Q S0)^T      (K/32 fragments each way)
 //   2. X of token tile 0, which V~ of token tile 1 needs (T' is lower triangular: one way, 2 fragments)
@@ -24,7 +24,7 @@
 // The exchange buffers overlap: a wave's tile of V~ is written over the partner's half of S0, which that
 // wave alone reads and has finished with by then; the partner overwrites it with its next half of S0 only
 // after it has read V~ from it.
-// Loaders (4 waves) and the LDS double buffer are those of gdn_chunk32.hip; the loaders also write the output
+// Loaders (4 waves) and the LDS double buffer are those of gdn_chunk_scan32.h; the loaders also write the output
 // (a compute wave leaves its bf16 output tile in LDS at the start of the next chunk).  One workgroup barrier
 // per chunk hands the stage halves over.  Waves of a scan workgroup with two slices: 0..3 compute (pairs 0-1,
 // 2-3), 4..7 loaders.  (With one slice: 0 1 compute | 2 3 6 7 loaders | 4 output store | 5 exits at once.)

@@ -17,7 +17,7 @@
 // K = V = 128: 148 + 106 + 160 | 53 + 95 + 122 us; 11 packed sequences of 32768 tokens together: 339 + 225 + 330 | 108 + 190 +
 // 243 us; 8 x 4096 tokens, 2 heads, K = 256, V = 512: 82 + 136 + 205 | 50 + 133 + 163 us.
 //
-// The workgroup is that of the half-slice scan (gdn_chunk32.hip): one (sequence, head) chain and one slice of 32 columns of V;
+// The workgroup is that of the half-slice scan (gdn_chunk_scan32.h): one (sequence, head) chain and one slice of 32 columns of V;
 // two compute waves with 16 columns of the state each in 16x16x32 accumulators, four loader waves that bring the next chunks
 // global -> registers -> LDS, a store wave that takes what is saved out of LDS.  What bounds it: the instruction stream of a
 // compute wave (K = 128: 38 and 60 MFMAs per chunk) and, with 256 workgroups, the memory (4 x 4096 tokens, 16 heads: 370 and 460 MB
@@ -37,7 +37,7 @@ constexpr int SWEEP_WAVES = 8;  // 0 1 compute | 2 3 loaders | 4 store | 5 exits
 constexpr int SWEEP_LOADERS = 4;
 
 // Order of the MFMAs of one chunk in a compute wave ("ops"), and where its side work goes; placement is the earliest-deadline
-// walk of Scan16Rules (gdn_chunk32.hip), at compile time.  Groups:
+// walk of Scan16Rules (gdn_chunk_scan32.h), at compile time.  Groups:
 //     reverse only: U = P^T dO (6) | K S (4 K/32) | reverse only: S += Q^T dO' (part A) | T X (6) | part B | S += K^T Y' (2 K/16)
 // Part A runs while X is formed and part B while Y is: neither depends on them.  The token tiles and slabs of the
 // triangular products are numbered in the order in which they become known: forwards in a forward sweep, backwards in a
@@ -414,7 +414,7 @@ __global__ __launch_bounds__(SWEEP_WAVES* WAVE) void chunk_sweep_kernel(const Sw
     // ------------------------------ compute ------------------------------
     // Lane (j, g) = (lane % 16, lane / 16); operands A[j][8 g + 0..7], B[8 g + 0..7][j], accumulator D[4 g + r][j] of the 16x16x32
     // MFMA.  State tile t, register r: key 32 (t / 2) + 8 g + 4 (t % 2) + r of column c0 + j; token tile t, register r: token
-    // 16 t + 4 g + r.  (The orders in which operands enumerate their reduction index: gdn_chunk32.hip.)
+    // 16 t + 4 g + r.  (The orders in which operands enumerate their reduction index: gdn_chunk_scan32.h.)
     constexpr int NOPS = SCH::NOPS, OP_S = SCH::OP_S, OP_QA = SCH::OP_QA, OP_T = SCH::OP_T, OP_QB = SCH::OP_QB, OP_K = SCH::OP_K, OP_BAR = SCH::OP_BAR;
     constexpr int LA = SCH::LA;
     const int j16 = lane % 16, g = lane / 16;
