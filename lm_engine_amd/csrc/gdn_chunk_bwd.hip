@@ -27,10 +27,9 @@
 // to itself by its register count):
 //   1. over the value dim in slabs of 64 columns: dO, Y, V~ and the slab of S0, then of dS1, staged; the products
 //      with the states and the two 64 x 64 products that contract over the value dim accumulate;
-//   2. the rows of q and k (128 keys at a time) for Q K^T and K K^T, then the 64 x 64 stage: G, G^T and Hm + Hm^T
-//      are left in LDS;
-//   3. per 128 keys: the transposes of q and k (K <= 128: staged from the rows phase 2 left in LDS; K = 256: read out
-//      of those rows with the transposing LDS load), the per-token sums over the key dim, dQ^T and dK^T.
+//   2. the rows of q and k (128 keys at a time) for Q K^T and K K^T, then the 64 x 64 stage: G^T and Hm^T are left in LDS;
+//   3. per 128 keys: the per-token sums over the key dim, dQ^T and dK^T; q^T, k^T, G and Hm come out of those rows with the
+//      transposing LDS load.
 // K = 256 on the sliced saves of the staging scans has one wave per SIMD and so 512 registers per lane: it asks for the
 // rows of the next slab, and of the next half of q and k, while the products of the current one run, and keeps them
 // in registers until their turn (PIPE below).
@@ -99,51 +98,60 @@ __device__ __forceinline__ f32x16 mma_nt(const bf16_t* A, int lda, const bf16_t*
     return acc;
 }
 
-// acc[r] += sum_t M[t][col0 + 8 (r/4) + 4 h + r%4] B[l32][t] over t < kd: the A operand is the transpose of 32 columns of
-// the row-major matrix M, read through the transposing LDS load (4 tokens x 16 columns per instruction)
-__device__ __forceinline__ f32x16 mma_tn(const bf16_t* M, int ldm, int col0, const bf16_t* B, int ldb, int kd, f32x16 acc, int l32, int lh) {
+// 8 consecutive rows t0 + 8 h .. of column col0 + l32 of the row-major matrix M, as an operand whose reduction runs over the rows:
+// two transposing LDS loads (4 rows x 16 columns each)
+__device__ __forceinline__ bf16x8 column_operand(const bf16_t* M, int ldm, int t0, int col0, int l32, int lh) {
     const int l16 = l32 % 16, g16 = l32 / 16;
-    for (int kk = 0; kk < kd; kk += 16) {
-        const bf16x4 lo = lds_read_tr4x16<false>(M, ldm, kk + 8 * lh, col0 + 16 * g16, l16);
-        const bf16x4 hi = lds_read_tr4x16<false>(M, ldm, kk + 8 * lh + 4, col0 + 16 * g16, l16);
-        bf16x8 a;
+    const bf16x4 lo = lds_read_tr4x16<false>(M, ldm, t0 + 8 * lh, col0 + 16 * g16, l16);
+    const bf16x4 hi = lds_read_tr4x16<false>(M, ldm, t0 + 8 * lh + 4, col0 + 16 * g16, l16);
+    bf16x8 r;
 #pragma unroll
-        for (int e = 0; e < 4; e++) a[e] = lo[e], a[4 + e] = hi[e];
-        const bf16x8 b = *reinterpret_cast<const bf16x8*>(B + l32 * ldb + kk + 8 * lh);
-        acc = mfma32_bf16(a, b, acc);
-    }
-    return acc;
+    for (int e = 0; e < 4; e++) r[e] = lo[e], r[4 + e] = hi[e];
+    return r;
 }
 
 // acc[r] += sum_t A[8 (r/4) + 4 h + r%4][t] M[t][col0 + l32] over t < kd: the B operand is the transpose of 32 columns of the
-// row-major matrix M (same transposing loads as mma_tn, on the other operand)
+// row-major matrix M
 __device__ __forceinline__ f32x16 mma_nn(const bf16_t* A, int lda, const bf16_t* M, int ldm, int col0, int kd, f32x16 acc, int l32, int lh) {
-    const int l16 = l32 % 16, g16 = l32 / 16;
     for (int kk = 0; kk < kd; kk += 16) {
         const bf16x8 a = *reinterpret_cast<const bf16x8*>(A + l32 * lda + kk + 8 * lh);
-        const bf16x4 lo = lds_read_tr4x16<false>(M, ldm, kk + 8 * lh, col0 + 16 * g16, l16);
-        const bf16x4 hi = lds_read_tr4x16<false>(M, ldm, kk + 8 * lh + 4, col0 + 16 * g16, l16);
-        bf16x8 b;
-#pragma unroll
-        for (int e = 0; e < 4; e++) b[e] = lo[e], b[4 + e] = hi[e];
-        acc = mfma32_bf16(a, b, acc);
+        acc = mfma32_bf16(a, column_operand(M, ldm, kk, col0, l32, lh), acc);
     }
     return acc;
 }
 
-// Sixteen sums over the 32 lanes of a wave half at once: on return every lane holds the sum of x[l32 / 2].  Each
-// exchange halves the number of values a lane carries (16 shuffles instead of 80).
+// x of another lane of the same 16 as a DPP control word names it: lane l ^ 1, l ^ 2 (quad_perm), l ^ 7 (row_half_mirror), l ^ 8 (row_ror:8)
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_XOR7 = 0x141, DPP_XOR8 = 0x128;
+template <int CTRL>
+__device__ __forceinline__ float dpp_lane(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+
+// Sixteen sums over the 32 lanes of a wave half at once: on return every lane holds the sum of x[l32 / 2].  Each exchange
+// halves the number of values a lane carries; all of them are register moves (a shuffle through the LDS crossbar each took 7 cycles
+// of its pipe, 32 of them per chunk and wave).
 __device__ __forceinline__ float half_sums16(const float (&x)[16], int l32) {
     float y[8], z[4], w[2];
-    const bool b4 = l32 & 16, b3 = l32 & 8, b2 = l32 & 4, b1 = l32 & 2;
+    const bool b3 = l32 & 8, b2 = l32 & 4, b1 = l32 & 2;
 #pragma unroll
-    for (int e = 0; e < 8; e++) y[e] = (b4 ? x[8 + e] : x[e]) + __shfl_xor(b4 ? x[e] : x[8 + e], 16, WAVE);
+    for (int e = 0; e < 8; e++) {  // lanes l and l ^ 16: with bit 4 clear they go on with x[e], else with x[8 + e]
+        const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, x[e]), __builtin_bit_cast(unsigned, x[8 + e]), false, false);
+        const unsigned lo = r[0], hi = r[1];
+        y[e] = __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+    }
 #pragma unroll
-    for (int e = 0; e < 4; e++) z[e] = (b3 ? y[4 + e] : y[e]) + __shfl_xor(b3 ? y[e] : y[4 + e], 8, WAVE);
+    for (int e = 0; e < 4; e++) z[e] = (b3 ? y[4 + e] : y[e]) + dpp_lane<DPP_XOR8>(b3 ? y[e] : y[4 + e]);
 #pragma unroll
-    for (int e = 0; e < 2; e++) w[e] = (b2 ? z[2 + e] : z[e]) + __shfl_xor(b2 ? z[e] : z[2 + e], 4, WAVE);
-    float u = (b1 ? w[1] : w[0]) + __shfl_xor(b1 ? w[0] : w[1], 2, WAVE);
-    return u + __shfl_xor(u, 1, WAVE);
+    for (int e = 0; e < 2; e++) w[e] = (b2 ? z[2 + e] : z[e]) + dpp_lane<DPP_XOR7>(b2 ? z[e] : z[2 + e]);  // (l ^ 7 has the other bit 2; the rest of the eight lanes follows)
+    const float u = (b1 ? w[1] : w[0]) + dpp_lane<DPP_XOR2>(b1 ? w[0] : w[1]);
+    return u + dpp_lane<DPP_XOR1>(u);
+}
+
+// Sum over 8 neighbouring lanes, in each of them.
+__device__ __forceinline__ float sum8(float x) {
+    x += dpp_lane<DPP_XOR7>(x);
+    x += dpp_lane<DPP_XOR2>(x);
+    return x + dpp_lane<DPP_XOR1>(x);
 }
 
 __device__ __forceinline__ void put4(bf16_t* dst, f32x4 x) {
@@ -177,13 +185,8 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
     // (4 x 4096 tokens, 16 heads, K = V = 128, the whole backward and forward: 869 -> 800 us).
     constexpr bool ONE_TRIP = SL && K <= 128;
     constexpr int PHASE1 = 3 * SLAB + (ONE_TRIP ? 2 : 1) * K * LDS64 * 2;  // dO | Y | V~ | states (S0, then dS1) or S0 | dS1
-    constexpr int PHASE2 = 3 * SLAB + 2 * C * LDK * 2;      // G | G^T | Hm + Hm^T | q | k
-    // Phase 3 needs q^T and k^T as MFMA operands.  K = 256 (a CU to itself) reads them out of the row-major copies with
-    // the transposing LDS load; with two workgroups per CU (K <= 128) that variant ran slower (more registers, spills)
-    // than staging the transposes once more, 2 bytes at a time.
-    constexpr bool TR = K > 128;
-    constexpr int PHASE3 = TR ? PHASE2 : 3 * SLAB + 2 * KW * LDS64 * 2;  // G | G^T | Hm + Hm^T | q^T | k^T
-    constexpr int LDS_BYTES = cmax(PHASE1, cmax(PHASE2, PHASE3));
+    constexpr int PHASE2 = 2 * SLAB + 2 * C * LDK * 2;      // G^T | Hm^T | q | k (and phase 3)
+    constexpr int LDS_BYTES = cmax(PHASE1, PHASE2);
     __shared__ __attribute__((aligned(16))) uint8_t lds[LDS_BYTES];
     __shared__ float s_gam[C], s_beta[C], s_e[C], s_tail[C], s_dgam[C], s_dbeta[C], s_dotq[C], s_dotk[C], s_fq[C], s_fk[C], s_red[4];
     bf16_t* const sDO = reinterpret_cast<bf16_t*>(lds);
@@ -191,13 +194,10 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
     bf16_t* const sVN = sY + C * LDS64;
     bf16_t* const sST = sVN + C * LDS64;  // [K][LDS64]: S0, then dS1
     bf16_t* const sS1 = ONE_TRIP ? sST + K * LDS64 : sST;
-    bf16_t* const sG = reinterpret_cast<bf16_t*>(lds);
-    bf16_t* const sGT = sG + C * LDS64;
-    bf16_t* const sH = sGT + C * LDS64;
-    bf16_t* const sQ = sH + C * LDS64;    // phase 2 (and 3 with TR): [64][LDK]
+    bf16_t* const sGT = reinterpret_cast<bf16_t*>(lds);
+    bf16_t* const sHT = sGT + C * LDS64;
+    bf16_t* const sQ = sHT + C * LDS64;   // [64][LDK]
     bf16_t* const sK = sQ + C * LDK;
-    bf16_t* const sQT = sH + C * LDS64;   // phase 3 without TR: [KW][LDS64]
-    bf16_t* const sKT = sQT + KW * LDS64;
 
     const int t = threadIdx.x;
     const int lane = t % WAVE, wave = t / WAVE;
@@ -280,7 +280,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
     // slab are asked for while the products of this one run and wait in registers, so that no trip through memory
     // stands between a slab's barriers.
     constexpr bool PIPE = SL && K > 128;
-    bf16x8 nx_v[PIPE ? 2 : 1], nx_d[PIPE ? 2 : 1], nx_y[PIPE ? 2 : 1], nx_vn[PIPE ? 2 : 1], nx_s0[TR ? K / 32 : 1];  // nx_s0: also q and k on their way into LDS
+    bf16x8 nx_v[PIPE ? 2 : 1], nx_d[PIPE ? 2 : 1], nx_y[PIPE ? 2 : 1], nx_vn[PIPE ? 2 : 1], nx_s0[K > 128 ? K / 32 : 1];  // nx_s0: also q and k on their way into LDS
     auto ask_slab = [&](int v0) {
         const int p8 = t % 8;
         const bf16_t* vnew = reinterpret_cast<const bf16_t*>(vnb);
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 #pragma unroll
         for (int i = 0; i < K / 32; i++) nx_s0[i] = *reinterpret_cast<const bf16x8*>(s0 + sliced_at(t / 8 + 32 * i, v0 + 8 * p8, K));
     };
-    // rows of q and k (keys KW kh ..) into registers, and from there, scaled, row-major into sQ and sK (TR only)
+    // rows of q and k (keys KW kh ..) into registers, and from there, scaled, row-major into sQ and sK (K = 256 only)
     auto ask_qk = [&](int kh) {
         constexpr int CPR = KW / 8, RPP = BWD_THREADS / CPR;  // 16-byte pieces per staged row, rows per pass
         int tl = t;
@@ -461,9 +461,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
         LTICK(1);
 #pragma unroll
         for (int it = 0; it < 2; it++) {  // 8 lanes hold one row
-            float x = yv[it];
-#pragma unroll
-            for (int off = 4; off >= 1; off >>= 1) x += __shfl_xor(x, off, WAVE);
+            const float x = sum8(yv[it]);
             if (t % 8 == 0) atomicAdd(&s_dbeta[t / 8 + 32 * it], x);
         }
 
@@ -507,8 +505,10 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                 dQeT[kh][m] = mma_nt(srows, LDS64, sDO + 32 * tt_of(m) * LDS64, LDS64, VW, dQeT[kh][m], l32, lh);
                 ZT[kh][m] = mma_nt(srows, LDS64, sY + 32 * tt_of(m) * LDS64, LDS64, VW, ZT[kh][m], l32, lh);
             }
-        DP = mma_nt(sDO + 32 * (wave / 2) * LDS64, LDS64, sVN + 32 * (wave % 2) * LDS64, LDS64, VW, DP, l32, lh);
-        DA = mma_nt(sY + 32 * (wave / 2) * LDS64, LDS64, sVN + 32 * (wave % 2) * LDS64, LDS64, VW, DA, l32, lh);
+        if (wave != 1) {  // (the tile above the diagonal is not needed)
+            DP = mma_nt(sDO + 32 * (wave / 2) * LDS64, LDS64, sVN + 32 * (wave % 2) * LDS64, LDS64, VW, DP, l32, lh);
+            DA = mma_nt(sY + 32 * (wave / 2) * LDS64, LDS64, sVN + 32 * (wave % 2) * LDS64, LDS64, VW, DA, l32, lh);
+        }
         if constexpr (!PREFETCH && !ONE_TRIP) ask_ds1();
         LTICK(5);
         if constexpr (!ONE_TRIP) __syncthreads();  // S0 has been read by every wave
@@ -559,7 +559,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 #pragma unroll
         for (int kh = 0; kh < KH; kh++) {
             if (kh > 0) __syncthreads();  // the products of the previous half have read q and k
-            if constexpr (TR) {
+            if constexpr (K > 128) {
                 if constexpr (!PIPE) {
                     if (kh == 0) ask_qk(0);
                 }
@@ -585,42 +585,48 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                 }
             }
             __syncthreads();
-            if constexpr (TR) {  // the rows staged next travel while these products run: the other half, then half 0 again for phase 3
+            if constexpr (K > 128) {  // the rows staged next travel while these products run: the other half, then half 0 again for phase 3
                 ask_qk(kh + 1 < KH ? kh + 1 : 0);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            QK = mma_nt(sQ + 32 * ti * LDK, LDK, sK + 32 * tj * LDK, LDK, KW, QK, l32, lh);
-            KK = mma_nt(sK + 32 * ti * LDK, LDK, sK + 32 * tj * LDK, LDK, KW, KK, l32, lh);
-        }
-        const int j = 32 * tj + l32;
-        const float gj = s_gam[j];
-        float colsum = 0.f;
-        float rowm[16], rowb[16];  // this lane's terms of the row sums for dgamma and dbeta
-#pragma unroll
-        for (int r = 0; r < 16; r++) {
-            const int i = 32 * ti + 8 * (r / 4) + 4 * lh + r % 4;
-            const float bi = s_beta[i];
-            const float E = i >= j ? __expf(s_gam[i] - gj) : 0.f;
-            const float dP = i >= j ? DP[r] : 0.f;
-            const float dA = i > j ? -DA[r] : 0.f;
-            const float Pm = E * QK[r];
-            const float Am = i > j ? bi * E * KK[r] : 0.f;
-            const float G = dP * E;
-            const float Hm = dA * bi * E;
-            const float m = dP * Pm + dA * Am;
-            colsum += m;
-            rowm[r] = m;
-            rowb[r] = dA * E * KK[r];
-            sG[i * LDS64 + j] = (bf16_t)G;
-            sGT[j * LDS64 + i] = (bf16_t)G;
-            if (i > j) {
-                sH[i * LDS64 + j] = (bf16_t)Hm;
-                sH[j * LDS64 + i] = (bf16_t)Hm;
-            } else if (i == j) {
-                sH[i * LDS64 + i] = (bf16_t)0.f;
+            if (wave != 1) {
+                QK = mma_nt(sQ + 32 * ti * LDK, LDK, sK + 32 * tj * LDK, LDK, KW, QK, l32, lh);
+                KK = mma_nt(sK + 32 * ti * LDK, LDK, sK + 32 * tj * LDK, LDK, KW, KK, l32, lh);
             }
         }
-        {
+        // The three tiles on and below the diagonal.  G^T and Hm^T are stored: a lane holds four consecutive rows i of column j,
+        // which is one 8-byte write of each; their zero tile is neither written nor read.  (As G, G^T and Hm + Hm^T with 64 2-byte
+        // writes behind 32 branches, and with q^T and k^T staged 2 bytes at a time at K <= 128: 257 us for 4 x 4096 tokens, 16 heads,
+        // K = V = 128, and 291 us for 8 x 4096 tokens, 2 heads, K = 256, V = 512; 243 and 278 us this way.)
+        if (wave != 1) {
+            const int j = 32 * tj + l32;
+            const float gj = s_gam[j];
+            float colsum = 0.f;
+            float rowm[16], rowb[16];  // this lane's terms of the row sums for dgamma and dbeta
+#pragma unroll
+            for (int r4 = 0; r4 < 4; r4++) {
+                const int i0 = 32 * ti + 8 * r4 + 4 * lh;
+                const f32x4 gi = *reinterpret_cast<const f32x4*>(&s_gam[i0]), bi = *reinterpret_cast<const f32x4*>(&s_beta[i0]);
+                f32x4 G, Hm;
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int r = 4 * r4 + e, i = i0 + e;
+                    const float E = i >= j ? __expf(gi[e] - gj) : 0.f;
+                    const float dP = i >= j ? DP[r] : 0.f;
+                    const float dA = i > j ? -DA[r] : 0.f;
+                    const float Pm = E * QK[r];
+                    const float EK = E * KK[r];
+                    const float Am = i > j ? bi[e] * EK : 0.f;
+                    const float m = dP * Pm + dA * Am;
+                    colsum += m;
+                    rowm[r] = m;
+                    rowb[r] = dA * EK;
+                    G[e] = dP * E;
+                    Hm[e] = dA * bi[e] * E;
+                }
+                put4(sGT + j * LDS64 + i0, G);
+                put4(sHT + j * LDS64 + i0, Hm);
+            }
             const float sm = half_sums16(rowm, l32), sb = half_sums16(rowb, l32);
             const int r = l32 / 2;
             const int i = 32 * ti + 8 * (r / 4) + 4 * lh + r % 4;
@@ -628,22 +634,10 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                 atomicAdd(&s_dgam[i], sm);
                 atomicAdd(&s_dbeta[i], sb);
             }
+            atomicAdd(&s_dgam[j], -colsum);
         }
-        atomicAdd(&s_dgam[j], -colsum);
     }
     LTICK(12);
-    // K <= 128: the transposes of phase 3 take the place of the rows of q and k in LDS; every thread picks its pieces of
-    // the rows up here, before the barrier that ends their use
-    bf16x8 tq[TR ? 1 : KW / 32], tk[TR ? 1 : KW / 32];
-    if constexpr (!TR) {
-        static_assert(TR || KH == 1, "one staging of q and k");
-#pragma unroll
-        for (int it = 0; it < KW / 32; it++) {
-            const int row = t % C, p8 = t / C + 4 * it;
-            tq[it] = *reinterpret_cast<const bf16x8*>(sQ + row * LDK + 8 * p8);
-            tk[it] = *reinterpret_cast<const bf16x8*>(sK + row * LDK + 8 * p8);
-        }
-    }
     // ---------------- phase 3: per-token sums over the key dim, dQ^T and dK^T, 128 keys at a time ----------------
     // (dQ^T and dK^T are built in the registers of dQe^T and dKd^T)
     float nkd = 0.f;
@@ -652,29 +646,20 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
     bf16x8 qv[KH][NTW][2], kv[KH][NTW][2];  // this lane's entries of q and k, kept for the backward of the normalisation
 #pragma unroll
     for (int kx = 0; kx < KH; kx++) {
-        const int kh = TR ? KH - 1 - kx : kx;  // TR: the half that phase 2 staged last is still there
-        __syncthreads();  // G, G^T, Hm + Hm^T are complete (or: the previous half's reads are over)
-        if constexpr (TR) {
+        const int kh = KH - 1 - kx;  // the half that phase 2 staged last is still there
+        __syncthreads();  // G^T and Hm^T are complete (or: the previous half's reads are over)
+        if constexpr (K > 128) {
             if (kx > 0) {
                 put_qk();
                 __syncthreads();
             }
-        } else {
-            // a wave takes 16 bytes of all 64 rows at a time: its 2-byte writes of one key then cover 64 consecutive
-            // tokens of a transposed row (no bank conflicts; the rows themselves come out of the cache)
-            // (the values are the scaled rows that phase 2 staged, taken out of LDS before the barrier above)
-            constexpr int CPR = KW / 8;
-            const int row = t % C;
+        }
+        // q^T and k^T: this wave's 32 keys, 16 tokens each, the same for its token tiles
+        bf16x8 qT[C / 16], kT[C / 16];
 #pragma unroll
-            for (int it = 0; it < CPR / 4; it++) {
-                const int p8 = t / C + 4 * it;
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    sQT[(8 * p8 + e) * LDS64 + row] = tq[it][e];
-                    sKT[(8 * p8 + e) * LDS64 + row] = tk[it][e];
-                }
-            }
-            __syncthreads();
+        for (int s = 0; s < C / 16; s++) {
+            qT[s] = column_operand(sQ, LDK, 16 * s, 32 * ktl, l32, lh);
+            kT[s] = column_operand(sK, LDK, 16 * s, 32 * ktl, l32, lh);
         }
 #pragma unroll
         for (int m = 0; m < NTW; m++) {
@@ -682,20 +667,12 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
             const int i = 32 * tt + l32;
             const float ei = s_e[i], tl = s_tail[i], bi = s_beta[i];
             float s_qe = 0.f, s_kd = 0.f, s_zk = 0.f;
-            if constexpr (TR) {
 #pragma unroll
-                for (int r4 = 0; r4 < 4; r4++) {  // keys 32 ktl + 8 r4 + 4 h + 0..3 of token i
-                    const bf16x4 q4 = *reinterpret_cast<const bf16x4*>(sQ + i * LDK + 32 * ktl + 8 * r4 + 4 * lh);
-                    const bf16x4 k4 = *reinterpret_cast<const bf16x4*>(sK + i * LDK + 32 * ktl + 8 * r4 + 4 * lh);
+            for (int r4 = 0; r4 < 4; r4++) {  // keys 32 ktl + 8 r4 + 4 h + 0..3 of token i
+                const bf16x4 q4 = *reinterpret_cast<const bf16x4*>(sQ + i * LDK + 32 * ktl + 8 * r4 + 4 * lh);
+                const bf16x4 k4 = *reinterpret_cast<const bf16x4*>(sK + i * LDK + 32 * ktl + 8 * r4 + 4 * lh);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) qv[kh][m][r4 / 2][4 * (r4 % 2) + e] = q4[e], kv[kh][m][r4 / 2][4 * (r4 % 2) + e] = k4[e];
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < 16; r++) {
-                    const int d = 32 * ktl + 8 * (r / 4) + 4 * lh + r % 4;
-                    qv[kh][m][r / 8][r % 8] = sQT[d * LDS64 + i], kv[kh][m][r / 8][r % 8] = sKT[d * LDS64 + i];
-                }
+                for (int e = 0; e < 4; e++) qv[kh][m][r4 / 2][4 * (r4 % 2) + e] = q4[e], kv[kh][m][r4 / 2][4 * (r4 % 2) + e] = k4[e];
             }
 #pragma unroll
             for (int r = 0; r < 16; r++) {
@@ -713,14 +690,17 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                 accq[kh][m][r] *= ei;
                 acck[kh][m][r] = acck[kh][m][r] * tl - ZT[kh][m][r] * (bi * ei);
             }
-            if constexpr (TR) {
-                accq[kh][m] = mma_tn(sK, LDK, 32 * ktl, sG + 32 * tt * LDS64, LDS64, C, accq[kh][m], l32, lh);
-                acck[kh][m] = mma_tn(sQ, LDK, 32 * ktl, sGT + 32 * tt * LDS64, LDS64, C, acck[kh][m], l32, lh);
-                acck[kh][m] = mma_tn(sK, LDK, 32 * ktl, sH + 32 * tt * LDS64, LDS64, C, acck[kh][m], l32, lh);
-            } else {
-                accq[kh][m] = mma_nt(sKT + 32 * ktl * LDS64, LDS64, sG + 32 * tt * LDS64, LDS64, C, accq[kh][m], l32, lh);
-                acck[kh][m] = mma_nt(sQT + 32 * ktl * LDS64, LDS64, sGT + 32 * tt * LDS64, LDS64, C, acck[kh][m], l32, lh);
-                acck[kh][m] = mma_nt(sKT + 32 * ktl * LDS64, LDS64, sH + 32 * tt * LDS64, LDS64, C, acck[kh][m], l32, lh);
+            // dQ^T += K^T G^T (tokens j <= i), dK^T += Q^T G (tokens i >= j), K^T (Hm + Hm^T)^T
+#pragma unroll
+            for (int s = 0; s < C / 16; s++) {
+                if (s < 2 || tt == 1) {
+                    accq[kh][m] = mfma32_bf16(kT[s], column_operand(sGT, LDS64, 16 * s, 32 * tt, l32, lh), accq[kh][m]);
+                    acck[kh][m] = mfma32_bf16(kT[s], column_operand(sHT, LDS64, 16 * s, 32 * tt, l32, lh), acck[kh][m]);
+                }
+                if (s >= 2 || tt == 0) {
+                    acck[kh][m] = mfma32_bf16(qT[s], *reinterpret_cast<const bf16x8*>(sGT + i * LDS64 + 16 * s + 8 * lh), acck[kh][m]);
+                    acck[kh][m] = mfma32_bf16(kT[s], *reinterpret_cast<const bf16x8*>(sHT + i * LDS64 + 16 * s + 8 * lh), acck[kh][m]);
+                }
             }
             if (p.rq != nullptr) {  // <dQs_i, Qs_i> and <dK_i, K_i> for the backward of the normalisation
                 float dq_q = 0.f, dk_k = 0.f;
