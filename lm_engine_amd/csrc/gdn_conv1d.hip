@@ -12,6 +12,8 @@
 // vectors: every load and store of a wave is one contiguous row segment; the four waves of a
 // workgroup take consecutive token blocks of the same channels.
 
+#include <type_traits>
+
 #include "gdn_common.h"
 
 namespace gdn {
@@ -60,24 +62,40 @@ __device__ __forceinline__ void load_contiguous(const void* base, int64_t first,
     }
 }
 
-template <typename T, typename WT, int KS, bool SILU, int TOKENS>
+// MASK: the rows are multiplied by the padding mask on the way in and out.  A wave's TOKENS + KS - 1 mask values are one load, a
+// value per lane, read out per row: as a load for every row and every output row they stood between the loads of x (6 x 1500
+// tokens, 4096 channels, bf16: 33.7 -> 28.3 us a call, 29.3 without a mask; 8 x 4096 tokens, 2048 channels: 58.0 -> 54.3, 51.3).
+template <typename T, typename WT, int KS, bool SILU, int TOKENS, bool MASK>
 __global__ __launch_bounds__(CONV_THREADS) void causal_conv1d_kernel(const ConvParams p) {
     constexpr int VEC = ConvVec<T>::N;
     typedef typename ConvVec<T>::type vec_t;
 
     // a workgroup covers 64 channel vectors x (4 waves x TOKENS tokens): the halo rows of a wave are the
     // last rows of the wave before it, read on the same CU at about the same time
-    const int c0 = (blockIdx.x * WAVE + threadIdx.x % WAVE) * VEC;
-    if (c0 >= p.C) return;
+    int c0 = (blockIdx.x * WAVE + threadIdx.x % WAVE) * VEC;
+    if constexpr (MASK) {
+        c0 = min(c0, p.C - VEC);  // every lane stays, as a holder of mask values: spare ones repeat the last channels, with the same results
+    } else {
+        if (c0 >= p.C) return;
+    }
     const int b = blockIdx.z;
-    // (the same token in every lane of a wave: the mask comes in with scalar loads)
+    // (the same token in every lane of a wave)
     const int s_begin = (blockIdx.y * (CONV_THREADS / WAVE) + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE)) * TOKENS;
     if (s_begin >= p.S) return;
     const int s_end = min(s_begin + TOKENS, p.S);
 
     const T* xb = reinterpret_cast<const T*>(p.x) + (int64_t)b * p.x_stride_b + c0;
     T* yb = reinterpret_cast<T*>(p.y) + (int64_t)b * p.y_stride_b + c0;
-    const T* mb = p.mask == nullptr ? nullptr : reinterpret_cast<const T*>(p.mask) + (int64_t)b * p.S;
+    // lane l: mask of token s_begin - (KS - 1) + l (the halo's and this walk's; others are not asked for)
+    static_assert(TOKENS + KS - 1 <= WAVE, "a lane per mask value");
+    float mask_of_lane = 0.f;
+    if constexpr (MASK) {
+        const int s = s_begin - (KS - 1) + (int)(threadIdx.x % WAVE);
+        if (s >= 0 && s < s_end) mask_of_lane = (float)(reinterpret_cast<const T*>(p.mask) + (int64_t)b * p.S)[s];
+    }
+    auto mask_at = [&](int s) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mask_of_lane), s - s_begin + (KS - 1)));
+    };
 
     float wflat[VEC * KS], bias[VEC];  // wflat[e * KS + j]: tap j of channel c0 + e
     load_contiguous<WT, VEC * KS>(p.weight, (int64_t)c0 * KS, wflat);
@@ -87,9 +105,13 @@ __global__ __launch_bounds__(CONV_THREADS) void causal_conv1d_kernel(const ConvP
 
     auto load_row = [&](int s, float (&row)[VEC]) {
         const vec_t v = *reinterpret_cast<const vec_t*>(xb + (int64_t)s * p.x_stride_s);
-        const float m = mb == nullptr ? 1.f : (float)mb[s];
 #pragma unroll
-        for (int e = 0; e < VEC; e++) row[e] = (float)v[e] * m;
+        for (int e = 0; e < VEC; e++) row[e] = (float)v[e];
+        if constexpr (MASK) {
+            const float m = mask_at(s);
+#pragma unroll
+            for (int e = 0; e < VEC; e++) row[e] *= m;
+        }
     };
 
     // row s of the (masked) input for s >= 0, the carried state or zeros for the kernel_size - 1 rows before the sequence
@@ -105,7 +127,7 @@ __global__ __launch_bounds__(CONV_THREADS) void causal_conv1d_kernel(const ConvP
         }
     };
     auto emit = [&](int s, const float (&cur)[VEC], const float (&hist)[KS - 1][VEC]) {  // hist[j] = row s - (KS - 1) + j
-        const float m = mb == nullptr ? 1.f : (float)mb[s];
+        const float m = MASK ? mask_at(s) : 1.f;
         vec_t out;
 #pragma unroll
         for (int e = 0; e < VEC; e++) {
@@ -113,7 +135,7 @@ __global__ __launch_bounds__(CONV_THREADS) void causal_conv1d_kernel(const ConvP
 #pragma unroll
             for (int j = 0; j < KS - 1; j++) acc += wflat[e * KS + j] * hist[j][e];
             if (SILU) acc = acc * __builtin_amdgcn_rcpf(1.f + __expf(-acc));  // x * sigmoid(x)
-            out[e] = (T)(acc * m);
+            out[e] = (T)(MASK ? acc * m : acc);
         }
         *reinterpret_cast<vec_t*>(yb + (int64_t)s * p.y_stride_s) = out;
     };
@@ -183,8 +205,13 @@ template <typename T, typename WT, int KS, int TOKENS>
 static void launch_conv_ks(const ConvParams& p, bool silu, hipStream_t stream) {
     constexpr int SPAN = (CONV_THREADS / WAVE) * TOKENS;  // tokens per workgroup
     const dim3 grid((p.C / ConvVec<T>::N + WAVE - 1) / WAVE, (p.S + SPAN - 1) / SPAN, p.B);
-    if (silu) hipLaunchKernelGGL((causal_conv1d_kernel<T, WT, KS, true, TOKENS>), grid, dim3(CONV_THREADS), 0, stream, p);
-    else hipLaunchKernelGGL((causal_conv1d_kernel<T, WT, KS, false, TOKENS>), grid, dim3(CONV_THREADS), 0, stream, p);
+    auto launch = [&](auto silu_tag, auto mask_tag) {
+        hipLaunchKernelGGL((causal_conv1d_kernel<T, WT, KS, decltype(silu_tag)::value, TOKENS, decltype(mask_tag)::value>), grid, dim3(CONV_THREADS), 0, stream, p);
+    };
+    if (silu && p.mask != nullptr) launch(std::true_type{}, std::true_type{});
+    else if (silu) launch(std::true_type{}, std::false_type{});
+    else if (p.mask != nullptr) launch(std::false_type{}, std::true_type{});
+    else launch(std::false_type{}, std::false_type{});
 }
 
 template <typename T, typename WT>

@@ -149,3 +149,15 @@ def test_long_walks_match_short_ones(dtype, masked):
         y1, s1 = lm_engine_amd.depthwise_causal_convolution(xr.cuda(), w.cuda(), b.cuda(), st[row : row + 1].cuda(), None, output_state=True)
         first = 0 if m is None else int((m[row] == 0).sum())
         assert torch.equal(y1[0, first:].cpu().to(F64), y[row, first:]) and torch.equal(s1[0].cpu().to(F64), s[row])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("C", [8, 144, 152, 512, 520])
+@pytest.mark.parametrize("S", [1, 15, 16, 17, 61])
+def test_mask_values_reach_every_row_of_a_partly_filled_wave(C, S):
+    """A wave keeps its rows' mask values one per lane: fewer channel vectors than values (C = 8: 1 of 64 lanes, 144 and 152: 18 and 19
+    for 16 + 3 values, 520: a last wave of one), mask values other than 0 and 1, both walk lengths."""
+    for B in (2, 40 * 2048 // max(S, 16) if S > 16 and C <= 152 else 3):
+        x, w, b, st, m = _inputs(B, S, C, 4, BF16, seed=C + S, state=True, mask=True)
+        m = m * 2.0 ** (torch.arange(S) % 3 - 1)[None, :].to(m.dtype)  # (powers of two: the state is compared bit for bit)
+        _check(x, w, b, st, m, "silu", f"C={C} S={S}")
