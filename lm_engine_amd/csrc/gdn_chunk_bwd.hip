@@ -188,7 +188,10 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
     constexpr int PHASE2 = 2 * SLAB + 2 * C * LDK * 2;      // G^T | Hm^T | q | k (and phase 3)
     constexpr int LDS_BYTES = cmax(PHASE1, PHASE2);
     __shared__ __attribute__((aligned(16))) uint8_t lds[LDS_BYTES];
-    __shared__ float s_gam[C], s_beta[C], s_e[C], s_tail[C], s_dgam[C], s_dbeta[C], s_dotq[C], s_dotk[C], s_fq[C], s_fk[C], s_red[4];
+    __shared__ float s_gam[C], s_beta[C], s_e[C], s_tail[C], s_dgam[C], s_dbeta[C], s_fq[C], s_fk[C], s_red[4];
+    // <dQs_i, Qs_i> and <dK_i, K_i> by 32 keys, added up in one order: as sums in whatever order the waves arrive they moved the rounding
+    // of a few of the gradients from run to run
+    __shared__ float s_dotq[K / 32][C], s_dotk[K / 32][C];
     bf16_t* const sDO = reinterpret_cast<bf16_t*>(lds);
     bf16_t* const sY = sDO + C * LDS64;
     bf16_t* const sVN = sY + C * LDS64;
@@ -240,8 +243,6 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
         s_tail[t] = __expf(p.gam[chunk * C + C - 1] - g);
         s_dgam[t] = 0.f;
         s_dbeta[t] = 0.f;
-        s_dotq[t] = 0.f;
-        s_dotk[t] = 0.f;
         s_fq[t] = (p.rq != nullptr ? p.rq[chunk * C + t] : 1.f) * p.scale;  // q and k rows are scaled on their way into LDS
         s_fk[t] = p.rk != nullptr ? p.rk[chunk * C + t] : 1.f;
     }
@@ -709,8 +710,8 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                     dq_q += accq[kh][m][r] * (float)qv[kh][m][r / 8][r % 8];
                     dk_k += acck[kh][m][r] * (float)kv[kh][m][r / 8][r % 8];
                 }
-                atomicAdd(&s_dotq[i], dq_q);
-                atomicAdd(&s_dotk[i], dk_k);
+                dq_q += __shfl_xor(dq_q, 32, WAVE), dk_k += __shfl_xor(dk_k, 32, WAVE);
+                if (lh == 0) s_dotq[ktl + NKT * kh][i] = dq_q, s_dotk[ktl + NKT * kh][i] = dk_k;
             }
         }
     }
@@ -729,7 +730,12 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
             const int64_t at = (tok0 + i) * p.dqk_stride_t + (int64_t)h * K + KW * kh + 32 * ktl + 4 * lh;
             const bool norm = p.rq != nullptr;
             const float rq = norm ? p.rq[chunk * C + i] : 1.f, rk = norm ? p.rk[chunk * C + i] : 1.f;
-            const float cq = norm ? s_dotq[i] / p.scale : 0.f, ck = norm ? s_dotk[i] : 0.f;
+            float cq = 0.f, ck = 0.f;
+            if (norm) {
+#pragma unroll
+                for (int x = 0; x < K / 32; x++) cq += s_dotq[x][i], ck += s_dotk[x][i];
+                cq /= p.scale;
+            }
 #pragma unroll
             for (int r4 = 0; r4 < 4; r4++) {
                 f32x4 oq, ok;
