@@ -80,7 +80,8 @@ enum {
  *               equal B, and cu_seqlens holds the prefix sums of the valid lengths: sequence b is the
  *               last cu_seqlens[b+1] - cu_seqlens[b] tokens of row b (what the reference gets from
  *               compute_cu_seqlens_and_max_seqlen_from_attention_mask, sequence_packing.py:18-22, and
- *               then packs and unpacks around the operator, :25-93); o is written at valid tokens only.
+ *               then packs and unpacks around the operator, :25-93); gdn_chunk_fwd writes zeros at the padding
+ *               of o, gdn_recurrent_fwd writes o at valid tokens only.
  *
  * Replaces the argument list of both fla calls at gated_deltanet/module.py:198-222.
  */

@@ -756,6 +756,19 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
         return;
     }
 
+    // The padding rows of a left-padded batch read as zeros: a compute wave writes those of its columns (16 bytes a lane, 4 lanes a
+    // row; two half-slice waves take turns) while the first chunk is on its way.  As a fill of the whole output by the caller they
+    // took a launch and a pass of their own (6 x 1500 tokens, 16 heads, V = 128: 7.5 us).
+    if (p.pad_lens != nullptr && !p.records_given && !NOOUT) {
+        const int w = HALF ? 0 : wave, step = HALF ? 32 : 16;
+        bf16_t* const og = p.o + b * p.o_stride_b + (int64_t)h * p.o_stride_h + 32 * (vgroup * NW + w) + 8 * (lane % 4);
+        bf16x8 zero8;
+#pragma unroll
+        for (int e = 0; e < 8; e++) zero8[e] = (bf16_t)0.f;
+        for (int row = lane / 4 + (HALF ? 16 * wave : 0); row < (int)seq_t0; row += step)
+            __builtin_nontemporal_store(zero8, reinterpret_cast<bf16x8*>(og + (int64_t)row * p.o_stride_t));
+    }
+
     if constexpr (HALF) {
         // ------------------------------ compute (HALF) ------------------------------
         // Lane (j, g) = (lane % 16, lane / 16).  Operands of the 16x16x32 MFMA: A[j][8 g + 0..7], B[8 g + 0..7][j]; its

@@ -266,8 +266,8 @@ def _run(mode, q, k, v, g, beta, scale, initial_state, output_final_state, cu_se
         cu_seqlens = cu_seqlens.to(torch.int32).contiguous()
     h0 = None if initial_state is None else initial_state.contiguous()
 
-    # padding positions of a left-padded batch are not written by the kernels: they read as zeros
-    o = (torch.zeros if left_padded else torch.empty)(B, T, H, V, dtype=v.dtype, device=v.device)
+    # padding positions of a left-padded batch read as zeros: gdn_chunk_fwd writes them, the token kernels do not
+    o = (torch.zeros if left_padded and mode != "chunk" else torch.empty)(B, T, H, V, dtype=v.dtype, device=v.device)
     ht = None
     if output_final_state:
         if inplace_state:
