@@ -188,10 +188,14 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
     constexpr int PHASE2 = 2 * SLAB + 2 * C * LDK * 2;      // G^T | Hm^T | q | k (and phase 3)
     constexpr int LDS_BYTES = cmax(PHASE1, PHASE2);
     __shared__ __attribute__((aligned(16))) uint8_t lds[LDS_BYTES];
-    __shared__ float s_gam[C], s_beta[C], s_e[C], s_tail[C], s_dgam[C], s_dbeta[C], s_fq[C], s_fk[C], s_red[4];
-    // <dQs_i, Qs_i> and <dK_i, K_i> by 32 keys, added up in one order: as sums in whatever order the waves arrive they moved the rounding
-    // of a few of the gradients from run to run
-    __shared__ float s_dotq[K / 32][C], s_dotk[K / 32][C];
+    __shared__ float s_gam[C], s_beta[C], s_e[C], s_tail[C], s_fq[C], s_fk[C];
+    // Sums over waves: every wave leaves its part in a place of its own and they are added up in one order at the end (as LDS atomics
+    // they stood in the waves' way - 653 -> 617 us per training step of 4 x 4096 tokens, 16 heads, K = V = 128 - and moved the
+    // rounding of a few gradients from run to run).  Per token: <Y, V>; by 32 keys <dQs, Qs>, <dK, K> and the terms of dgamma and dbeta
+    // from the 64 x K products; by tile the row sums for dgamma and dbeta and the column sums for dgamma.  Per wave: <dS1, S0> and
+    // sum_i tail_i <dKd_i, K_i>.
+    __shared__ float s_yv[C], s_dotq[K / 32][C], s_dotk[K / 32][C], s_keyg[K / 32][C], s_keyb[K / 32][C];
+    __shared__ float s_rowg[2][C], s_rowb[2][C], s_colg[2][C], s_red[2][BWD_THREADS / WAVE];
     bf16_t* const sDO = reinterpret_cast<bf16_t*>(lds);
     bf16_t* const sY = sDO + C * LDS64;
     bf16_t* const sVN = sY + C * LDS64;
@@ -241,12 +245,9 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
         s_beta[t] = p.beta[chunk * C + t];
         s_e[t] = __expf(g);
         s_tail[t] = __expf(p.gam[chunk * C + C - 1] - g);
-        s_dgam[t] = 0.f;
-        s_dbeta[t] = 0.f;
         s_fq[t] = (p.rq != nullptr ? p.rq[chunk * C + t] : 1.f) * p.scale;  // q and k rows are scaled on their way into LDS
         s_fk[t] = p.rk != nullptr ? p.rk[chunk * C + t] : 1.f;
     }
-    if (t < 4) s_red[t] = 0.f;
 #ifdef GDN_CYCLE_BUDGET
     // Measurement build (python -m lm_engine_amd.build --cycle-budget): wave 0 reads the shader clock between the steps
     // of the kernel and adds the cycles of each up; sampled workgroups report at the end (the steps are named in bench.py's LOCAL_GROUPS).
@@ -328,11 +329,11 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
             *reinterpret_cast<bf16x8*>(sK + row * LDK + 8 * p8) = kb;
         }
     };
+    float yv[2] = {0.f, 0.f};  // this thread's part of <Y_i, V_i>, rows t / 8 and t / 8 + 32
     if constexpr (PIPE) ask_slab(0);
 #pragma unroll 1
     for (int hv = 0; hv < V / VW; hv++) {
         const int v0 = VW * hv;
-        float yv[2];  // <Y_i, V_i> pieces, reduced after the barrier (s_dbeta is cleared before the first one)
         if constexpr (PIPE) {
             const int p8 = t % 8;
 #pragma unroll
@@ -352,7 +353,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                 *reinterpret_cast<bf16x8*>(sY + row * LDS64 + 8 * p8) = yr;
                 *reinterpret_cast<bf16x8*>(sVN + row * LDS64 + 8 * p8) = live ? nx_vn[it] : zero8;
                 if (live) *reinterpret_cast<bf16x8*>(p.dv_out + (tok0 + row) * p.dv_stride_t + (int64_t)h * V + v0 + 8 * p8) = dv;
-                yv[it] = acc;
+                yv[it] += acc;
             }
 #pragma unroll
             for (int i = 0; i < K / 32; i++) *reinterpret_cast<bf16x8*>(sST + (t / 8 + 32 * i) * LDS64 + 8 * p8) = nx_s0[i];
@@ -391,7 +392,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                 *reinterpret_cast<bf16x8*>(sY + row * LDS64 + 8 * p8) = yr[it];
                 *reinterpret_cast<bf16x8*>(sVN + row * LDS64 + 8 * p8) = live ? nr[it] : zero8;
                 if (live) *reinterpret_cast<bf16x8*>(p.dv_out + (tok0 + row) * p.dv_stride_t + (int64_t)h * V + v0 + 8 * p8) = dv;
-                yv[it] = acc;
+                yv[it] += acc;
             }
 #pragma unroll
             for (int i = 0; i < K / 32; i++) {
@@ -425,7 +426,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                 *reinterpret_cast<bf16x8*>(sDO + row * LDS64 + 8 * p8) = dr;
                 *reinterpret_cast<bf16x8*>(sY + row * LDS64 + 8 * p8) = yr;
                 if (live) *reinterpret_cast<bf16x8*>(p.dv_out + (tok0 + row) * p.dv_stride_t + (int64_t)h * V + v0 + 8 * p8) = dv;
-                yv[it] = acc;
+                yv[it] += acc;
             }
             if (p.saves_bf16) {
                 const bf16_t* vnew = reinterpret_cast<const bf16_t*>(vnb);
@@ -460,12 +461,6 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
         LTICK(0);
         __syncthreads();
         LTICK(1);
-#pragma unroll
-        for (int it = 0; it < 2; it++) {  // 8 lanes hold one row
-            const float x = sum8(yv[it]);
-            if (t % 8 == 0) atomicAdd(&s_dbeta[t / 8 + 32 * it], x);
-        }
-
         // K = 256 (a CU to itself, registers to spare): dS1 of this slab is asked for now and stays in registers while the
         // products with S0 run, so that its trip through memory is behind them instead of in front of the barrier below.
         // With two workgroups per CU the other one's products fill that wait, and the registers are needed.
@@ -549,7 +544,12 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
         LTICK(10);
     }
     dot = wave_sum(dot);
-    if (lane == 0) atomicAdd(&s_red[0], dot);
+    if (lane == 0) s_red[0][wave] = dot;
+#pragma unroll
+    for (int it = 0; it < 2; it++) {  // 8 lanes hold one row
+        const float x = sum8(yv[it]);
+        if (t % 8 == 0) s_yv[t / 8 + 32 * it] = x;
+    }
 
     LTICK(11);
     // ---------------- phase 2: Q K^T, K K^T and the 64 x 64 stage ----------------
@@ -631,11 +631,9 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
             const float sm = half_sums16(rowm, l32), sb = half_sums16(rowb, l32);
             const int r = l32 / 2;
             const int i = 32 * ti + 8 * (r / 4) + 4 * lh + r % 4;
-            if (l32 % 2 == 0) {
-                atomicAdd(&s_dgam[i], sm);
-                atomicAdd(&s_dbeta[i], sb);
-            }
-            atomicAdd(&s_dgam[j], -colsum);
+            if (l32 % 2 == 0) s_rowg[tj][i] = sm, s_rowb[tj][i] = sb;
+            colsum += __shfl_xor(colsum, 32, WAVE);
+            if (lh == 0) s_colg[ti][j] = colsum;
         }
     }
     LTICK(12);
@@ -682,9 +680,9 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                 s_kd += dKdT[kh][m][r] * (float)ke;
                 s_zk += ZT[kh][m][r] * (float)ke;
             }
-            atomicAdd(&s_dgam[i], ei * s_qe - tl * s_kd - bi * ei * s_zk);
-            atomicAdd(&s_dbeta[i], -ei * s_zk);
             nkd += tl * s_kd;
+            s_qe += __shfl_xor(s_qe, 32, WAVE), s_kd += __shfl_xor(s_kd, 32, WAVE), s_zk += __shfl_xor(s_zk, 32, WAVE);
+            if (lh == 0) s_keyg[ktl + NKT * kh][i] = ei * s_qe - tl * s_kd - bi * ei * s_zk, s_keyb[ktl + NKT * kh][i] = -ei * s_zk;
 
 #pragma unroll
             for (int r = 0; r < 16; r++) {
@@ -717,7 +715,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
     }
     LTICK(13);
     nkd = wave_sum(nkd);
-    if (lane == 0) atomicAdd(&s_red[1], nkd);
+    if (lane == 0) s_red[1][wave] = nkd;
     __syncthreads();
 
     // With x = y / r the normalised row (y: input, r = |y|^-1 incl. epsilon): dy = r (dx - x <x, dx>); the scale of
@@ -753,8 +751,13 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
         }
 
     if (t < C) {  // wave 0
-        float dg = s_dgam[t];
-        if (t == C - 1) dg += s_e[C - 1] * s_red[0] + s_red[1];
+        // (the tile above the diagonal has no sums)
+        float dg = s_rowg[0][t] - s_colg[1][t], dbeta = s_yv[t] + s_rowb[0][t];
+        if (t >= C / 2) dg += s_rowg[1][t], dbeta += s_rowb[1][t];
+        else dg -= s_colg[0][t];
+#pragma unroll
+        for (int x = 0; x < K / 32; x++) dg += s_keyg[x][t], dbeta += s_keyb[x][t];
+        if (t == C - 1) dg += s_e[C - 1] * ((s_red[0][0] + s_red[0][1]) + (s_red[0][2] + s_red[0][3])) + ((s_red[1][0] + s_red[1][1]) + (s_red[1][2] + s_red[1][3]));
         // dg_t = sum of dgamma over the tokens t .. 63 of the chunk
 #pragma unroll
         for (int off = 1; off < WAVE; off <<= 1) {
@@ -763,7 +766,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
         }
         if (t < valid) {
             p.dg_out[(tok0 + t) * p.H + h] = dg;
-            p.dbeta_out[(tok0 + t) * p.H + h] = s_dbeta[t];
+            p.dbeta_out[(tok0 + t) * p.H + h] = dbeta;
         }
     }
 #ifdef GDN_CYCLE_BUDGET
