@@ -160,6 +160,16 @@ __device__ __forceinline__ void put4(bf16_t* dst, f32x4 x) {
     *reinterpret_cast<bf16x4*>(dst) = r;
 }
 
+// Lane halves h = 0, 1 hold keys 4 h + 0..3 (a) and 8 + 4 h + 0..3 (b) of 16: keys 8 h + 0..7 in each lane, for 16-byte stores.
+__device__ __forceinline__ bf16x8 eight_keys(bf16x4 a, bf16x4 b) {
+    typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
+    typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
+    const u32x2 ua = __builtin_bit_cast(u32x2, a), ub = __builtin_bit_cast(u32x2, b);
+    const auto lo = __builtin_amdgcn_permlane32_swap(ua.x, ub.x, false, false), hi = __builtin_amdgcn_permlane32_swap(ua.y, ub.y, false, false);
+    const u32x4 r = {lo[0], hi[0], lo[1], hi[1]};
+    return __builtin_bit_cast(bf16x8, r);
+}
+
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
 // element (row, column c) of a [rows][V] array laid out by groups of 8 rows and, within a group, by 32-column slice
@@ -725,27 +735,32 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 #pragma unroll
         for (int m = 0; m < NTW; m++) {
             const int i = 32 * tt_of(m) + l32;
-            const int64_t at = (tok0 + i) * p.dqk_stride_t + (int64_t)h * K + KW * kh + 32 * ktl + 4 * lh;
             const bool norm = p.rq != nullptr;
             const float rq = norm ? p.rq[chunk * C + i] : 1.f, rk = norm ? p.rk[chunk * C + i] : 1.f;
             float cq = 0.f, ck = 0.f;
             if (norm) {
 #pragma unroll
                 for (int x = 0; x < K / 32; x++) cq += s_dotq[x][i], ck += s_dotk[x][i];
-                cq /= p.scale;
+                cq *= rq / p.scale, ck *= rk;
             }
+            const float rqs = rq * p.scale;
+            bf16_t* const dq = p.dq_out + (tok0 + i) * p.dqk_stride_t + (int64_t)h * K + KW * kh + 32 * ktl + 8 * lh;
+            bf16_t* const dk = p.dk_out + (tok0 + i) * p.dqk_stride_t + (int64_t)h * K + KW * kh + 32 * ktl + 8 * lh;
 #pragma unroll
-            for (int r4 = 0; r4 < 4; r4++) {
-                f32x4 oq, ok;
+            for (int r8 = 0; r8 < 2; r8++) {  // registers 8 r8 + 4 x + e: keys 16 r8 + 8 x + 4 h + e
+                bf16x4 oq[2], ok[2];
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int r = 4 * r4 + e;
-                    oq[e] = rq * (accq[kh][m][r] * p.scale - cq * (float)qv[kh][m][r / 8][r % 8]);
-                    ok[e] = rk * (acck[kh][m][r] - ck * (float)kv[kh][m][r / 8][r % 8]);
-                }
+                for (int x = 0; x < 2; x++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int r = 8 * r8 + 4 * x + e;
+                        oq[x][e] = (bf16_t)(accq[kh][m][r] * rqs - cq * (float)qv[kh][m][r8][r % 8]);
+                        ok[x][e] = (bf16_t)(acck[kh][m][r] * rk - ck * (float)kv[kh][m][r8][r % 8]);
+                    }
+                const bf16x8 q8 = eight_keys(oq[0], oq[1]), k8 = eight_keys(ok[0], ok[1]);
                 if (i < valid) {
-                    store4<bf16_t>(p.dq_out + at + 8 * r4, oq);
-                    store4<bf16_t>(p.dk_out + at + 8 * r4, ok);
+                    *reinterpret_cast<bf16x8*>(dq + 16 * r8) = q8;
+                    *reinterpret_cast<bf16x8*>(dk + 16 * r8) = k8;
                 }
             }
         }
