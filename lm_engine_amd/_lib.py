@@ -60,6 +60,7 @@ EXPORTED_SYMBOLS = (
     "gdn_gated_rmsnorm_fwd",
     "gdn_gated_rmsnorm_bwd",
     "gdn_column_sums",
+    "gdn_padding_mask",
     "gdn_layer_step",
     "gdn_layer_step_tiles",
 )
@@ -275,6 +276,9 @@ def load_library() -> ctypes.CDLL:
     lib.gdn_gates_fwd.restype = ctypes.c_int
     lib.gdn_gates_bwd.argtypes = [ctypes.POINTER(GdnGateBwdArgs), ctypes.c_void_p]
     lib.gdn_gates_bwd.restype = ctypes.c_int
+    lib.gdn_padding_mask.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_void_p,
+                                     ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]  # fmt: skip
+    lib.gdn_padding_mask.restype = ctypes.c_int
     lib.gdn_column_sums.argtypes = [ctypes.POINTER(GdnColumnSumsArgs), ctypes.c_void_p]
     lib.gdn_column_sums.restype = ctypes.c_int
     lib.gdn_gated_rmsnorm_fwd.argtypes = [ctypes.POINTER(GdnNormArgs), ctypes.c_void_p]

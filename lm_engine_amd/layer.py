@@ -24,7 +24,7 @@ import torch
 from ._host import host, raw_stream
 from .conv import _IN_KERNEL_ACTIVATIONS, depthwise_causal_convolution
 from .kernels import Kernel, is_kernel_allowed
-from .layer_ops import delta_rule_gates, gated_rmsnorm
+from .layer_ops import delta_rule_gates, gated_rmsnorm, padding_mask
 from .ops import RECURRENT_MAX_TOKENS, chunk_gated_delta_rule, column_blocks, fused_recurrent_gated_delta_rule, layer_step_workspace
 
 
@@ -104,6 +104,11 @@ def gated_deltanet_mixing(
             o, conv_state, h = step
             return o, (conv_state, h)
 
+    cu_seqlens = None
+    if (attention_mask is not None and attention_mask.dim() == 2 and attention_mask.shape == (B, S) and attention_mask.device == qkv.device
+            and is_kernel_allowed(Kernel.gated_delta_rule) and not torch.compiler.is_compiling()):  # fmt: skip
+        attention_mask, cu_seqlens = padding_mask(attention_mask, qkv.dtype)
+
     qkv, conv_state = depthwise_causal_convolution(qkv, conv_weight, conv_bias, conv_state, attention_mask, use_cache,
                                                    conv_activation)  # fmt: skip
     if torch.is_grad_enabled() and qkv.requires_grad and not torch.compiler.is_compiling():
@@ -118,9 +123,8 @@ def gated_deltanet_mixing(
 
     g, beta = delta_rule_gates(a, b, A_log, dt_bias, allow_neg_eigval)
 
-    cu_seqlens = None
-    if attention_mask is not None:  # sequence_packing.py:18-22
-        seqlens = attention_mask.sum(dim=-1, dtype=torch.int32)
+    if attention_mask is not None and cu_seqlens is None:  # (a captured graph; what is no mask of this batch the convolution has refused)
+        seqlens = attention_mask.sum(dim=-1, dtype=torch.int32)  # sequence_packing.py:18-22
         cu_seqlens = torch.nn.functional.pad(torch.cumsum(seqlens, dim=0, dtype=torch.int32), (1, 0))
 
     op = fused_recurrent_gated_delta_rule if S <= RECURRENT_MAX_TOKENS else chunk_gated_delta_rule

@@ -57,6 +57,29 @@ def _token_rows(x: torch.Tensor, width: int, what: str) -> tuple[torch.Tensor, i
     return rows, rows.stride(0) if rows.size(0) > 1 else width
 
 
+_MASK_BYTES = {torch.int64: 8, torch.int32: 4, torch.uint8: 1, torch.bool: 1}
+_MASK_ROWS, _MASK_ELEMENTS = 1024, 1 << 16  # one workgroup's work: a few microseconds
+
+
+def padding_mask(attention_mask: torch.Tensor, dtype: torch.dtype):
+    """The integer ``attention_mask`` ``[B, S]`` in ``dtype`` (contiguous) and the prefix sums of its rows' sums, int32 ``[B + 1]``, in
+    one launch (``gdn_padding_mask``); the same through torch where the mask is large or of another type."""
+    B, S = attention_mask.shape
+    element_bytes = _MASK_BYTES.get(attention_mask.dtype)
+    if element_bytes is None or not attention_mask.is_cuda or B > _MASK_ROWS or not 0 < B * S <= _MASK_ELEMENTS or dtype not in (torch.bfloat16, torch.float32):
+        seqlens = attention_mask.sum(dim=-1, dtype=torch.int32)  # sequence_packing.py:18-22
+        return attention_mask, torch.nn.functional.pad(torch.cumsum(seqlens, dim=0, dtype=torch.int32), (1, 0))
+    mask = torch.empty(B, S, dtype=dtype, device=attention_mask.device)
+    prefix = torch.empty(B + 1, dtype=torch.int32, device=attention_mask.device)
+    lib = _lib.load_library()
+    with torch.cuda.device(attention_mask.device):
+        stream = ctypes.c_void_p(torch.cuda.current_stream(attention_mask.device).cuda_stream)
+        _lib.check_status(
+            lib.gdn_padding_mask(attention_mask.data_ptr(), element_bytes, attention_mask.stride(0), attention_mask.stride(1), B, S,
+                                 mask.data_ptr(), _dtype_code(dtype, "mask"), prefix.data_ptr(), stream), "gdn_padding_mask")  # fmt: skip
+    return mask, prefix
+
+
 def column_sums(lib, stream, *wanted):
     """``gdn_column_sums``: for every ``(partial [rows, ...] fp32 contiguous, dtype)`` (one or two, the same ``rows``) the sum
     over the first dim in that dtype.  Runs on the caller's current device and stream."""

@@ -137,3 +137,22 @@ def test_operands_on_the_host_are_refused_before_any_launch():
             lm_engine_amd.gated_rmsnorm(o, gate, weight, 1e-5)
         with pytest.raises(ValueError, match=f"{name} is on cpu"):
             lm_engine_amd.gated_rmsnorm(o.clone().requires_grad_(True), gate, weight, 1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32, torch.uint8, torch.bool, torch.float32])
+@pytest.mark.parametrize("B, S", [(1, 1), (1, 64), (2, 65), (6, 1500), (15, 63), (16, 64), (17, 129), (300, 7), (1024, 64), (1025, 3), (8, 8193)])
+def test_padding_mask_matches_torch(dtype, B, S):
+    """One launch against sum, cumsum and conversion: whole numbers, so the same values.  Rows shared by several waves, a row per wave, more
+    rows than waves and than lanes, sizes that go through torch; also a mask that is not contiguous."""
+    from lm_engine_amd.layer_ops import padding_mask
+
+    lengths = torch.randint(0, S + 1, (B,), generator=torch.Generator().manual_seed(B + S))
+    mask = (torch.arange(S)[None, :] >= S - lengths[:, None]).to(dtype).cuda()
+    strided = torch.stack((mask, torch.zeros_like(mask)), dim=-1)[..., 0]
+    for x in (mask, strided, mask[:1].expand(B, S)):
+        for out_dtype in (torch.bfloat16, torch.float32):
+            got, prefix = padding_mask(x, out_dtype)
+            assert torch.equal(got.to(out_dtype), x.to(out_dtype))
+            assert prefix.dtype == torch.int32
+            assert torch.equal(prefix.cpu(), torch.nn.functional.pad(x.cpu().long().sum(-1).cumsum(0), (1, 0)).int())
