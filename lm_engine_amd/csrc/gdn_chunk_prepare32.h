@@ -15,6 +15,23 @@ __device__ __forceinline__ float dpp_move(float x) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, ROW_MASK, 0xF, false));
 }
 
+// Sum over LANES (8, 16 or 32) neighbouring lanes, in each of them, in register moves: as shuffles through the LDS crossbar the row sums of
+// squares were a quarter of an item's LDS instructions.
+template <int LANES>
+__device__ __forceinline__ float lanes_sum(float x) {
+    static_assert(LANES == 8 || LANES == 16 || LANES == 32, "a row of q or k");
+    x += dpp_move<0xB1, 0xF>(x);   // quad_perm: lane l ^ 1
+    x += dpp_move<0x4E, 0xF>(x);   // l ^ 2
+    x += dpp_move<0x141, 0xF>(x);  // row_half_mirror: the other four of eight
+    if constexpr (LANES >= 16) x += dpp_move<0x128, 0xF>(x);  // row_ror:8
+    if constexpr (LANES == 32) {
+        const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, x), __builtin_bit_cast(unsigned, x), false, false);
+        const unsigned a = r[0], b = r[1];
+        x = __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+    }
+    return x;
+}
+
 // Stores into a record, `offset` bytes from its start.  DEVICE_SCOPE: written through to memory (scope bit sc1), so that
 // a workgroup on another XCD, whose L2 is a different one, reads what was written once the flag of the record says so.
 // (The alternative, a release fence at device scope, writes back every dirty line of the XCD's L2: 13 us per record.
@@ -178,11 +195,7 @@ __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8
                         a += (float)kx[it][e] * (float)kx[it][e];
                         b += (float)qx[it][e] * (float)qx[it][e];
                     }
-#pragma unroll
-                    for (int off = 1; off < CPR; off <<= 1) {
-                        a += __shfl_xor(a, off, WAVE);
-                        b += __shfl_xor(b, off, WAVE);
-                    }
+                    a = lanes_sum<CPR>(a), b = lanes_sum<CPR>(b);
                     if (piece == 0) s_ssk[row] = a, s_ssq[row] = b;
                 }
             }
@@ -215,41 +228,11 @@ __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8
         }
         __syncthreads();  // #1
 
-        if (tid < C) {
-            const float gam = s_gam[tid], gl = s_gam[C - 1];
-            const float rk = p.l2norm ? rsqrtf(s_ssk[tid] + L2NORM_EPS) : 1.f;
-            const float rq = p.l2norm ? rsqrtf(s_ssq[tid] + L2NORM_EPS) : 1.f;
-            s_rk[tid] = rk;
-            s_rq[tid] = rq;
-            // what the tile epilogues below multiply with, once per token instead of once per matrix entry (the sums of
-            // squares are not needed any more): beta_i / |k_i| and gamma_i in units of log 2
-            s_ssk[tid] = s_beta[tid] * rk;
-            s_ssq[tid] = gam * 1.44269504088896341f;
-            // row scales the scan applies: to q S0, to the rows of V~ in the state update, to k S0 (none for
-            // the rows past the end of a short chunk: the scan reads some other token's k and v there)
-            const bool valid = tid < len;
-            if constexpr (SWEEP) {
-                const float e = __expf(gam), ks = valid ? __expf(gl - gam) * rk : 0.f, cs = valid ? e * rk : 0.f, eg = __expf(gl);
-                float* const f = reinterpret_cast<float*>(rec + SWEEP_REC_FWD_SCALES) + tid;
-                float* const r = reinterpret_cast<float*>(rec + SWEEP_REC_REV_SCALES) + tid;
-                f[0] = ks, f[C] = cs, f[2 * C] = eg;
-                r[0] = valid ? e * p.scale * rq : 0.f, r[C] = ks, r[2 * C] = -(s_beta[tid] * cs), r[3 * C] = eg;
-                const int64_t at = (((int64_t)cc.n * p.H + h) * sw.nc + cc.c) * C + tid;
-                if (cc.c < sw.nc) sw.gamma[at] = gam, sw.beta[at] = s_beta[tid], sw.rq[at] = rq, sw.rk[at] = rk;
-            } else {
-                record_store<FLAGS>(rec, p.rec_bytes, p.off_qs + 4 * tid, __expf(gam) * p.scale * rq);
-                record_store<FLAGS>(rec, p.rec_bytes, p.off_ks + 4 * tid, valid ? __expf(gl - gam) * rk : 0.f);
-                record_store<FLAGS>(rec, p.rec_bytes, p.off_cs + 4 * tid, valid ? __expf(gam) * rk : 0.f);
-                if (tid == 0) record_store<FLAGS>(rec, p.rec_bytes, p.off_eg, __expf(gl));
-            }
-        }
-        __syncthreads();  // #2
-
         // ---- A = strict-lower(beta_i e^{gamma_i - gamma_j} k^_i . k^_j) -> sA;  P -> record ----
         {
             // 32 x 32 tile jobs: G(Ti, Tj) = K_Ti K_Tj^T (rows i, column j), Pt(Tj, Ti) = K_Tj Q_Ti^T (rows j, column i; SWEEP: its
             // transpose, so that a lane holds consecutive rows i of P^T's reduction)
-            auto tile_job = [&](bool is_p, int trow, int tcol) {
+            auto tile_products = [&](bool is_p, int trow, int tcol) -> f32x16 {
                 f32x16 acc;
 #pragma unroll
                 for (int r = 0; r < 16; r++) acc[r] = 0.f;
@@ -261,6 +244,9 @@ __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8
                     acc = SWEEP && is_p ? mfma32_bf16(b, a, acc) : mfma32_bf16(a, b, acc);
                     if (s % 2 == 1) __builtin_amdgcn_sched_barrier(0);  // keeps the operand reads from piling up in registers
                 }
+                return acc;
+            };
+            auto tile_finish = [&](bool is_p, int trow, int tcol, const f32x16& acc) {
                 // register quad q of the tile holds rows 32 trow + 8 q + 4 h + 0..3: their per-token values in one read
                 if (!is_p) {
                     const int j = 32 * tcol + l32;
@@ -338,15 +324,46 @@ __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8
                 }
             };
             // first the two diagonal tiles of A, which the inverse starts from, and two of the three tiles of P
-            if (wave == 0) tile_job(false, 0, 0);
-            else if (wave == 1) tile_job(true, 0, 0);
-            else if (wave == 2) tile_job(false, 1, 1);
-            else tile_job(true, 1, 1);  // P[i < 32][j >= 32] = 0 is not stored
+            // (P[i < 32][j >= 32] = 0 is not stored); their products need the rows only and run beside the first wave's scales
+            // (with the row sums in registers: one-launch forward of 4 x 4096 tokens, 16 heads, K = V = 128 110.0 -> 107.3 us)
+            const bool is_p = wave % 2 == 1;
+            const int diag = wave / 2;
+            if (tid < C) {
+                const float gam = s_gam[tid], gl = s_gam[C - 1];
+                const float rk = p.l2norm ? rsqrtf(s_ssk[tid] + L2NORM_EPS) : 1.f;
+                const float rq = p.l2norm ? rsqrtf(s_ssq[tid] + L2NORM_EPS) : 1.f;
+                s_rk[tid] = rk;
+                s_rq[tid] = rq;
+                // what the tile epilogues below multiply with, once per token instead of once per matrix entry (the sums of
+                // squares are not needed any more): beta_i / |k_i| and gamma_i in units of log 2
+                s_ssk[tid] = s_beta[tid] * rk;
+                s_ssq[tid] = gam * 1.44269504088896341f;
+                // row scales the scan applies: to q S0, to the rows of V~ in the state update, to k S0 (none for
+                // the rows past the end of a short chunk: the scan reads some other token's k and v there)
+                const bool valid = tid < len;
+                if constexpr (SWEEP) {
+                    const float e = __expf(gam), ks = valid ? __expf(gl - gam) * rk : 0.f, cs = valid ? e * rk : 0.f, eg = __expf(gl);
+                    float* const f = reinterpret_cast<float*>(rec + SWEEP_REC_FWD_SCALES) + tid;
+                    float* const r = reinterpret_cast<float*>(rec + SWEEP_REC_REV_SCALES) + tid;
+                    f[0] = ks, f[C] = cs, f[2 * C] = eg;
+                    r[0] = valid ? e * p.scale * rq : 0.f, r[C] = ks, r[2 * C] = -(s_beta[tid] * cs), r[3 * C] = eg;
+                    const int64_t at = (((int64_t)cc.n * p.H + h) * sw.nc + cc.c) * C + tid;
+                    if (cc.c < sw.nc) sw.gamma[at] = gam, sw.beta[at] = s_beta[tid], sw.rq[at] = rq, sw.rk[at] = rk;
+                } else {
+                    record_store<FLAGS>(rec, p.rec_bytes, p.off_qs + 4 * tid, __expf(gam) * p.scale * rq);
+                    record_store<FLAGS>(rec, p.rec_bytes, p.off_ks + 4 * tid, valid ? __expf(gl - gam) * rk : 0.f);
+                    record_store<FLAGS>(rec, p.rec_bytes, p.off_cs + 4 * tid, valid ? __expf(gam) * rk : 0.f);
+                    if (tid == 0) record_store<FLAGS>(rec, p.rec_bytes, p.off_eg, __expf(gl));
+                }
+            }
+            const f32x16 acc = tile_products(is_p, diag, diag);
+            __syncthreads();  // #2
+            tile_finish(is_p, diag, diag, acc);
             __syncthreads();  // #3: the diagonal tiles of A are complete
             // then wave 0 inverts the diagonal blocks (a long dependent chain on one wave) while two others
             // finish the tiles: K and Q stay in place until barrier #4
-            if (wave == 1) tile_job(false, 1, 0);
-            else if (wave == 2) tile_job(true, 0, 1);
+            if (wave == 1) tile_finish(false, 1, 0, tile_products(false, 1, 0));
+            else if (wave == 2) tile_finish(true, 0, 1, tile_products(true, 0, 1));
         }
 
         // ---- wave 0: inverses of the four 16 x 16 diagonal blocks, written over the blocks of A ----
