@@ -352,6 +352,8 @@ def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm
         covers = sum(lens) == B * T
         sequences = (*ops.upload_int32((starts, lens), q.device), NC)
     q, k, v, do = (x if x.stride(-1) == 1 else x.contiguous() for x in (q, k, v, do.to(torch.bfloat16)))
+    if do.stride(1) > 1 << 24:  # the kernels count a chunk's rows in 32 bits; q, k and v were held to that by the forward
+        do = do.contiguous()
     prep, S0, Vn, dS1, Y, dh0 = ops.chunk_bwd_sweeps(q, k, v, do, g, beta, scale, l2norm, initial_state, cu_seqlens, left_padded, dht, NC)
     dq, dk, dv, dg, dbeta = ops.chunk_local_grads(q, k, v, do, prep, Y, Vn, S0, dS1, scale, l2norm, sequences, sliced=True,
                                                   covers=covers, joined=joined)  # fmt: skip

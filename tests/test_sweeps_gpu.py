@@ -95,3 +95,18 @@ def test_sweeps_match_the_formulas(layout, lens, K, V, HK, H):
             row, start, _ = spans[n]
             first = torch.stack([g[row, start + C * c] for c in range(len(s0))], dim=1)
             assert torch.equal(gamma.cpu(), first), "prefix sums start at the chunk's first token"
+
+
+@pytest.mark.gpu
+def test_output_gradient_with_rows_far_apart():
+    # rows of dO further apart than the kernels' 32-bit row arithmetic takes: the same gradients as from a dense dO
+    from lm_engine_amd.backward import gated_delta_rule_backward
+
+    T, K, V, apart = 3, 64, 64, (1 << 24) + 64
+    gen = torch.Generator().manual_seed(5)
+    q, k, v, dense = (torch.randn(1, T, 1, n, generator=gen).to(torch.bfloat16).cuda() for n in (K, K, V, V))
+    do = torch.zeros((T - 1) * apart + V, dtype=torch.bfloat16, device="cuda").as_strided((1, T, 1, V), (T * apart, apart, V, 1))
+    do.copy_(dense)
+    print(f"case: dO rows {apart} apart", flush=True)
+    for far, near in zip(*(gated_delta_rule_backward(q, k, v, None, None, d)[:3] for d in (do, dense))):
+        assert torch.equal(far, near)
