@@ -77,8 +77,8 @@ uint64_t chunk_workspace_bytes(const gdn_args& a) {
 constexpr int ORDER_MAX = 1024;
 __global__ __launch_bounds__(256) void chunk_offsets_kernel(const int32_t* __restrict__ cu, int32_t* __restrict__ off,
                                                             int32_t* __restrict__ order, int N, int total, int slots) {
-    __shared__ int s_part[256];
-    const int tid = threadIdx.x;
+    __shared__ int s_wave[4];
+    const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
     const int per = (N + 255) / 256;
     const int begin = min(tid * per, N), end = min(begin + per, N);
     auto chunks_of = [&](int n) {
@@ -88,19 +88,23 @@ __global__ __launch_bounds__(256) void chunk_offsets_kernel(const int32_t* __res
     };
     int sum = 0;
     for (int n = begin; n < end; n++) sum = min(sum + chunks_of(n), slots);
-    s_part[tid] = sum;
-    __syncthreads();
-    if (tid == 0) {
-        int run = 0;
-        for (int i = 0; i < 256; i++) {
-            const int x = s_part[i];
-            s_part[i] = run;
-            run = min(run + x, slots);
-        }
-        off[N] = run;
+    // Prefix sums over the threads, capped at every addition (which is associative for what is not negative).  The launch is one
+    // serial chain in front of everything else, and one thread adding up 256 parts out of LDS was the longest piece of it:
+    // 8.1 -> 5.1 us at 11 sequences.
+    int upto = sum;
+#pragma unroll
+    for (int d = 1; d < WAVE; d <<= 1) {
+        const int y = __shfl_up(upto, d, WAVE);
+        if (lane >= d) upto = min(upto + y, slots);
     }
+    if (lane == WAVE - 1) s_wave[wave] = upto;
     __syncthreads();
-    int run = s_part[tid];
+    int before = 0;  // of this thread
+    for (int w = 0; w < wave; w++) before = min(before + s_wave[w], slots);
+    if (tid == 255) off[N] = min(before + upto, slots);
+    const int left = __shfl_up(upto, 1, WAVE);
+    if (lane > 0) before = min(before + left, slots);
+    int run = before;
     for (int n = begin; n < end; n++) {
         off[n] = run;
         run = min(run + chunks_of(n), slots);
