@@ -92,7 +92,19 @@ def depthwise_causal_convolution(
     return kernel_with_formula_backward(kernel, formula, x, weight, bias, input_state)
 
 
-_BWD_TOKENS_PER_BLOCK = 256  # tokens a thread of the backward kernel walks over (64: 0.196 ms, 128: 0.171, 256: 0.163 at 4 x 4096 x 6144)
+# Tokens a thread of the backward kernel walks over: 256 (a block's first and last rows are read twice, and its partial sums are written
+# and added up), halved down to 64 while the launch has fewer than two workgroups per CU.  B x S x C, microseconds with the sums, at
+# 64 / 128 / 256 tokens: 8 x 4096 x 2048 100 / 96 / 83, 4 x 4096 x 6144 143 / 138 / 137, 4 x 4096 x 2048 55 / 46 / 53,
+# 1 x 32768 x 1024 50 / 44 / 52, 1 x 8192 x 2048 32 / 33 / 52, 2 x 2048 x 2048 29 / 31 / 52 (32 and 16: no less).
+_BWD_TOKENS_PER_BLOCK, _BWD_TOKENS_LEAST = 256, 64
+_BWD_WORKGROUPS, _BWD_CHANNELS_PER_WORKGROUP = 512, 512
+
+
+def _backward_tokens_per_block(B, S, C) -> int:
+    tokens, columns = _BWD_TOKENS_PER_BLOCK, -(-C // _BWD_CHANNELS_PER_WORKGROUP)
+    while tokens > _BWD_TOKENS_LEAST and columns * B * -(-S // tokens) < _BWD_WORKGROUPS:
+        tokens //= 2
+    return tokens
 
 
 def _backward_kernel_applies(x, weight, activation) -> bool:
@@ -154,7 +166,8 @@ def _convolution_backward(x, weight, bias, input_state, attention_mask, dy, acti
     mask = None
     if attention_mask is not None and attention_mask.shape[1] > 1 and attention_mask.shape[0] > 1:
         mask = attention_mask.to(x.dtype).contiguous()
-    blocks = B * (-(-S // _BWD_TOKENS_PER_BLOCK))
+    tokens = _backward_tokens_per_block(B, S, C)
+    blocks = B * (-(-S // tokens))
     dx = torch.empty(B, S, C, dtype=x.dtype, device=x.device)
     dstate = None if state is None else torch.empty(B, C, ks - 1, dtype=x.dtype, device=x.device)
     dw_part = torch.empty(blocks, C, ks, dtype=torch.float32, device=x.device)
@@ -167,7 +180,7 @@ def _convolution_backward(x, weight, bias, input_state, attention_mask, dy, acti
     a.dstate = None if dstate is None else dstate.data_ptr()
     a.dweight_partial, a.dbias_partial = dw_part.data_ptr(), db_part.data_ptr()
     a.x_stride_b, a.x_stride_s, a.dy_stride_b, a.dy_stride_s = x.stride(0), x.stride(1), dy.stride(0), dy.stride(1)
-    a.B, a.S, a.C, a.kernel_size, a.tokens_per_block = B, S, C, ks, _BWD_TOKENS_PER_BLOCK
+    a.B, a.S, a.C, a.kernel_size, a.tokens_per_block = B, S, C, ks, tokens
     a.w_dtype = _dtype_code(w2.dtype, "weight")
     a.dtype = _dtype_code(x.dtype, "x")
     a.activation = _IN_KERNEL_ACTIVATIONS[activation]

@@ -12,6 +12,8 @@
 // for dx only.  The per-block partial sums of dw and dbias go to a [blocks][C] array each that the caller adds up.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "gdn_common.h"
 #include "gdn_launch.h"
 
@@ -20,10 +22,10 @@ namespace gdn {
 namespace {
 
 constexpr int CB_THREADS = 256;
-// Channels per thread.  The kernel is bound by its arithmetic (about 35 vector instructions per token and channel against
-// 6 bytes), so narrow accesses that put more waves on a CU beat 16-byte ones: at B = 4, S = 4096, C = 6144 bf16, kernel plus
-// the two sums of the partial results, 8 channels 189 us, 4 channels 173 us, 2 channels (8 rows in flight, 256 tokens
-// per block) 163 us.
+// Channels per thread.  The kernel is bound by its arithmetic nearly as much as by memory (24 vector instructions per token and
+// channel against 6 bytes), so narrow accesses that put more waves on a CU beat 16-byte ones: at B = 4, S = 4096, C = 6144 bf16,
+// kernel plus the two sums of the partial results, when rows were not yet requested a step ahead, 8 channels 189 us, 4 channels
+// 173 us, 2 channels (8 rows in flight, 256 tokens per block) 163 us.
 constexpr int CB_VEC = 2;
 
 struct ConvBwdParams {
@@ -51,18 +53,22 @@ __device__ __forceinline__ float load_w(const void* w, int is_bf16, int64_t i) {
 template <typename T, int KS, bool SILU, int VEC, bool MASK>
 __global__ __launch_bounds__(CB_THREADS) void causal_conv1d_bwd_kernel(const ConvBwdParams p) {
     typedef T vec_t __attribute__((ext_vector_type(VEC)));
-    const int c0 = (blockIdx.x * CB_THREADS + threadIdx.x) * VEC;
-    if (c0 >= p.C) return;
+    const uint32_t c0 = (blockIdx.x * CB_THREADS + threadIdx.x) * VEC;
+    if (c0 >= (uint32_t)p.C) return;
     const int blocks_per_row = (p.S + p.tokens_per_block - 1) / p.tokens_per_block;
     const int b = blockIdx.y / blocks_per_row, blk = blockIdx.y % blocks_per_row;
     const int s_begin = blk * p.tokens_per_block;
     const int s_own = min(s_begin + p.tokens_per_block, p.S);      // dz of [s_begin, s_own) belongs to this block
     const int s_end = min(s_own + KS - 1, p.S);           // dz up to here feeds dx of this block
 
-    const T* xb = static_cast<const T*>(p.x) + (int64_t)b * p.x_stride_b + c0;
-    const T* dyb = static_cast<const T*>(p.dy) + (int64_t)b * p.dy_stride_b + c0;
+    // Rows start at addresses that are the same for the whole wave and stay in scalar registers; the lane's own part of an address is
+    // its channel, in bytes.
+    const uint32_t c_bytes = c0 * (uint32_t)sizeof(T);
+    auto at = [&](const T* row) { return *reinterpret_cast<const vec_t*>(reinterpret_cast<const uint8_t*>(row) + c_bytes); };
+    const T* xb = static_cast<const T*>(p.x) + (int64_t)b * p.x_stride_b;
+    const T* dyb = static_cast<const T*>(p.dy) + (int64_t)b * p.dy_stride_b;
     const T* mb = MASK ? static_cast<const T*>(p.mask) + (int64_t)b * p.S : nullptr;  // MASK is false when there is none
-    T* dxb = static_cast<T*>(p.dx) + ((int64_t)b * p.S) * p.C + c0;
+    T* dxb = static_cast<T*>(p.dx) + ((int64_t)b * p.S) * p.C;
     const T* const state_in = static_cast<const T*>(p.input_state);
     T* const state_out = static_cast<T*>(p.dstate);
 
@@ -77,7 +83,7 @@ __global__ __launch_bounds__(CB_THREADS) void causal_conv1d_bwd_kernel(const Con
     // row s of xx in x's index (s < 0: carried state or zeros)
     auto load_xx = [&](int s, float (&row)[VEC]) {
         if (s >= 0) {
-            const vec_t v = *reinterpret_cast<const vec_t*>(xb + (int64_t)s * p.x_stride_s);
+            const vec_t v = at(xb + (int64_t)s * p.x_stride_s);
             const float m = MASK ? (float)mb[s] : 1.f;
 #pragma unroll
             for (int e = 0; e < VEC; e++) row[e] = (float)v[e] * m;
@@ -100,65 +106,84 @@ __global__ __launch_bounds__(CB_THREADS) void causal_conv1d_bwd_kernel(const Con
 #pragma unroll
     for (int j = 0; j < KS - 1; j++) load_xx(s_begin - (KS - 1) + j, win[j + 1]);  // shifted into place by the first step
 
-    // The walk goes in steps of UNROLL tokens whose rows of x and dy are all requested before the first is used: a
-    // thread then has 2 UNROLL loads in flight instead of two, which is what a streaming kernel with this few waves
-    // per CU needs to keep the memory system busy.  (Rows past s_end are read again from row s_end - 1 and not used.)
+    // One token of the walk: dz of row s, and dx of row s - (KS - 1), which is complete then.  INNER: dz and dx both are rows of
+    // this block.
+    auto token = [&](auto inner, int s, const vec_t xv, const vec_t g) {
+        constexpr bool INNER = decltype(inner)::value;
+        // slide: win[j] <- win[j + 1], pend likewise (pend[0] of the last step was emitted below)
+#pragma unroll
+        for (int e = 0; e < VEC; e++) {
+#pragma unroll
+            for (int j = 0; j + 1 < KS; j++) win[j][e] = win[j + 1][e], pend[j][e] = pend[j + 1][e];
+            pend[KS - 1][e] = 0.f;
+        }
+        const float m = MASK ? (float)mb[s] : 1.f;
+#pragma unroll
+        for (int e = 0; e < VEC; e++) win[KS - 1][e] = (float)xv[e] * m;
+        const bool own = INNER || s < s_own;
+#pragma unroll
+        for (int e = 0; e < VEC; e++) {
+            float z = bias[e];
+#pragma unroll
+            for (int j = 0; j < KS; j++) z += w[e][j] * win[j][e];
+            float dz = (float)g[e] * m;
+            if (SILU) {
+                const float sg = __builtin_amdgcn_rcpf(1.f + __expf(-z));
+                dz *= sg * (1.f + z * (1.f - sg));
+            }
+#pragma unroll
+            for (int j = 0; j < KS; j++) pend[j][e] += w[e][j] * dz;  // x index s - (KS - 1) + j
+            if (own) {
+                db[e] += dz;
+#pragma unroll
+                for (int j = 0; j < KS; j++) dw[e][j] += dz * win[j][e];
+            }
+        }
+        // x index t = s - (KS - 1) is complete now
+        const int t = s - (KS - 1);
+        if (INNER || t >= s_begin) {
+            const float mt = MASK ? (float)mb[t] : 1.f;
+            vec_t out;
+#pragma unroll
+            for (int e = 0; e < VEC; e++) out[e] = (T)(pend[0][e] * mt);
+            __builtin_nontemporal_store(out, reinterpret_cast<vec_t*>(reinterpret_cast<uint8_t*>(dxb + (int64_t)t * p.C) + c_bytes));  // (nobody reads dx back soon)
+        } else if (t < 0 && state_out != nullptr) {  // only in the first block of a row
+#pragma unroll
+            for (int e = 0; e < VEC; e++) state_out[((int64_t)b * p.C + c0 + e) * (KS - 1) + (KS - 1) + t] = (T)pend[0][e];
+        }
+    };
+    // The walk goes in steps of UNROLL tokens whose rows of x and dy are all requested before the step in front of them is
+    // computed: a thread then has 2 UNROLL loads in flight under its arithmetic, which is what a streaming kernel with this few
+    // waves per CU needs to keep the memory system busy, and the tokens of a whole step are one piece of code without branches.
+    // Requested at the head of their own step, with a check per token, and with addresses in vector registers:
+    // 8 x 4096 x 2048 103.5 -> 82.8 us with the sums (403 MB), 4 x 4096 x 2048 79.8 -> 52.9, 4 x 4096 x 6144 136.8 as before.
+    // (139 registers, three waves per SIMD; held to 128 it spills, and 82.8 becomes 111.8.)  Rows past s_end are read again from
+    // row s_end - 1 and not used.
     constexpr int UNROLL = 8;
-    for (int s0 = s_begin; s0 < s_end; s0 += UNROLL) {
-        vec_t xr[UNROLL], gr[UNROLL];
+    vec_t xr[UNROLL], gr[UNROLL], xn[UNROLL], gn[UNROLL];
+    auto request = [&](int s0, vec_t (&xs)[UNROLL], vec_t (&gs)[UNROLL]) {
 #pragma unroll
         for (int u = 0; u < UNROLL; u++) {
             const int su = min(s0 + u, s_end - 1);
-            xr[u] = *reinterpret_cast<const vec_t*>(xb + (int64_t)su * p.x_stride_s);
-            gr[u] = *reinterpret_cast<const vec_t*>(dyb + (int64_t)su * p.dy_stride_s);
+            xs[u] = at(xb + (int64_t)su * p.x_stride_s);
+            gs[u] = at(dyb + (int64_t)su * p.dy_stride_s);
+        }
+    };
+    request(s_begin, xr, gr);
+    for (int s0 = s_begin; s0 < s_end; s0 += UNROLL) {
+        request(s0 + UNROLL, xn, gn);
+        if (s0 >= s_begin + KS - 1 && s0 + UNROLL <= s_own) {
+#pragma unroll
+            for (int u = 0; u < UNROLL; u++) token(std::true_type{}, s0 + u, xr[u], gr[u]);
+        } else {
+#pragma unroll
+            for (int u = 0; u < UNROLL; u++) {
+                if (s0 + u >= s_end) break;
+                token(std::false_type{}, s0 + u, xr[u], gr[u]);
+            }
         }
 #pragma unroll
-        for (int u = 0; u < UNROLL; u++) {
-            const int s = s0 + u;
-            if (s >= s_end) break;
-            // slide: win[j] <- win[j + 1], pend likewise (pend[0] of the last step was emitted below)
-#pragma unroll
-            for (int e = 0; e < VEC; e++) {
-#pragma unroll
-                for (int j = 0; j + 1 < KS; j++) win[j][e] = win[j + 1][e], pend[j][e] = pend[j + 1][e];
-                pend[KS - 1][e] = 0.f;
-            }
-            const float m = MASK ? (float)mb[s] : 1.f;
-#pragma unroll
-            for (int e = 0; e < VEC; e++) win[KS - 1][e] = (float)xr[u][e] * m;
-            const vec_t g = gr[u];
-            const bool own = s < s_own;
-#pragma unroll
-            for (int e = 0; e < VEC; e++) {
-                float z = bias[e];
-#pragma unroll
-                for (int j = 0; j < KS; j++) z += w[e][j] * win[j][e];
-                float dz = (float)g[e] * m;
-                if (SILU) {
-                    const float sg = __builtin_amdgcn_rcpf(1.f + __expf(-z));
-                    dz *= sg * (1.f + z * (1.f - sg));
-                }
-#pragma unroll
-                for (int j = 0; j < KS; j++) pend[j][e] += w[e][j] * dz;  // x index s - (KS - 1) + j
-                if (own) {
-                    db[e] += dz;
-#pragma unroll
-                    for (int j = 0; j < KS; j++) dw[e][j] += dz * win[j][e];
-                }
-            }
-            // x index t = s - (KS - 1) is complete now
-            const int t = s - (KS - 1);
-            if (t >= s_begin) {
-                const float mt = MASK ? (float)mb[t] : 1.f;
-                vec_t out;
-#pragma unroll
-                for (int e = 0; e < VEC; e++) out[e] = (T)(pend[0][e] * mt);
-                __builtin_nontemporal_store(out, reinterpret_cast<vec_t*>(dxb + (int64_t)t * p.C));  // (nobody reads dx back soon)
-            } else if (t < 0 && state_out != nullptr) {  // only in the first block of a row
-#pragma unroll
-                for (int e = 0; e < VEC; e++) state_out[((int64_t)b * p.C + c0 + e) * (KS - 1) + (KS - 1) + t] = (T)pend[0][e];
-            }
-        }
+        for (int u = 0; u < UNROLL; u++) xr[u] = xn[u], gr[u] = gn[u];
     }
     // the rows still in flight: x indices s_end - (KS - 1) + 1 .. s_end - 1 (complete only at the end of the sequence;
     // inside it they belong to the next block, which recomputes them)
@@ -171,7 +196,7 @@ __global__ __launch_bounds__(CB_THREADS) void causal_conv1d_bwd_kernel(const Con
                 vec_t out;
 #pragma unroll
                 for (int e = 0; e < VEC; e++) out[e] = (T)(pend[j][e] * mt);
-                __builtin_nontemporal_store(out, reinterpret_cast<vec_t*>(dxb + (int64_t)t * p.C));  // (nobody reads dx back soon)
+                __builtin_nontemporal_store(out, reinterpret_cast<vec_t*>(reinterpret_cast<uint8_t*>(dxb + (int64_t)t * p.C) + c_bytes));  // (nobody reads dx back soon)
             } else if (t < 0 && t >= -(KS - 1) && s_begin == 0 && state_out != nullptr) {
 #pragma unroll
                 for (int e = 0; e < VEC; e++) state_out[((int64_t)b * p.C + c0 + e) * (KS - 1) + (KS - 1) + t] = (T)pend[j][e];

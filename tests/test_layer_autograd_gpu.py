@@ -179,6 +179,23 @@ def test_convolution_gradients(with_state, masked, S, ks):
         _compare(got, want, 1e-5, ("dx", "dweight", "dbias"))
 
 
+@pytest.mark.parametrize("B, S, C", [(2, 193, 516), (16, 4097, 8), (32, 4097, 8), (1, 257, 1028)])
+def test_convolution_gradients_in_every_block_length(B, S, C):
+    """The walk of ``gdn_causal_conv1d_bwd`` in blocks of 64, 128 and 256 tokens (the launch picks by the workgroups it gives), the last
+    block of a row one token long, channels in one workgroup and a few past it.  fp32: sums of up to 256 terms in a block and of the
+    blocks, 2^-24 per addition and a growth with the root of their number, stay under 2e-6 of the result; 1e-5 as above."""
+    from lm_engine_amd.conv import _backward_tokens_per_block
+
+    assert _backward_tokens_per_block(B, S, C) == {16: 128, 32: 256}.get(B, 64)
+    gen = torch.Generator().manual_seed(S + C)
+    x, w, bias = torch.randn(B, S, C, generator=gen), 0.5 * torch.randn(C, 1, 4, generator=gen), torch.randn(C, generator=gen)
+    cy = torch.randn(B, S, C, generator=gen)
+    want = _grads(lambda x, w, b: depthwise_causal_convolution_ref(x, w, b, None, None, False, "silu")[:1], [t.to(F64) for t in (x, w, bias)], [cy.to(F64)])
+    got = _grads(lambda x, w, b: lm_engine_amd.depthwise_causal_convolution(x, w, b, None, None, True, "silu")[:1],
+                 [t.cuda() for t in (x, w, bias)], [cy.cuda()])  # fmt: skip
+    _compare(got, want, 1e-5, ("dx", "dweight", "dbias"))
+
+
 def test_layer_chain_gradients():
     B, S, HK, HV, DK, DV = 2, 130, 2, 4, 128, 128
     key_dim, value_dim = HK * DK, HV * DV
