@@ -62,6 +62,12 @@ def test_gates_gradients(dtype, tol, shape, H):
     _compare([got[0][..., keep], *got[1:]], [want[0][..., keep], *want[1:]], tol, ("da|db", "dA_log", "ddt_bias"))
 
 
+@pytest.mark.parametrize("H", [1, 2, 3, 5, 16, 17, 64, 65, 128, 255, 257, 300])
+def test_gates_gradients_of_any_number_of_heads(H):
+    # a head's sums in a workgroup are added up by 8, 4, 2 threads or one, from 256 sums down to none; tolerance as above
+    test_gates_gradients(torch.float32, 1e-5, (2, 1 + 1100 // H), H)
+
+
 def test_gates_gradient_of_one_output_only():
     gen = torch.Generator().manual_seed(4)
     H = 16
