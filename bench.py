@@ -673,7 +673,7 @@ def main():
             shipped = replace(get_workload(1, B=8, H=2, K=256, V=512), name="shipped_head_shape_k256_v512_bf16")
             backward["other"] = [bench_backward(shipped, make_inputs(shipped, device="cuda"), args.steps, args.warmup)]
             torch.cuda.empty_cache()
-            # and on the packed, ragged batch of configuration 2 (the rows of its mirror problem are scanned over their own lengths)
+            # and on the packed, ragged batch of configuration 2 (every sequence is swept over its own chunks)
             ragged = get_workload(2)
             backward["other"].append(bench_backward(ragged, make_inputs(ragged, device="cuda"), args.steps, args.warmup))
             torch.cuda.empty_cache()
