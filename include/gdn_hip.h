@@ -61,6 +61,8 @@ enum {
                                        * sequence (other than a sequence's first slot) get no records and no rows of the
                                        * mirror problem - for a mirror scan that walks every row over its own length
                                        * (gdn_chunk_fwd_saving with records_given on a left-padded batch) */
+    GDN_FLAG_ZERO_PADDING = 256, /* gdn_chunk_fwd with GDN_FLAG_LEFT_PADDED: zeros are written at the padding of o as well (what the
+                                   reference's unpack leaves there); without the flag nothing is written there */
     GDN_FLAG_DEBUG_NO_PRODUCERS = 64, /* test aid for the one-launch forward: its prepare workgroups return at once, so that
                                    the scan's bounded wait runs out (with a small args->spin_limit) and the error path can be
                                    exercised while every kernel still ends normally; outputs are invalid */
@@ -80,8 +82,8 @@ enum {
  *               equal B, and cu_seqlens holds the prefix sums of the valid lengths: sequence b is the
  *               last cu_seqlens[b+1] - cu_seqlens[b] tokens of row b (what the reference gets from
  *               compute_cu_seqlens_and_max_seqlen_from_attention_mask, sequence_packing.py:18-22, and
- *               then packs and unpacks around the operator, :25-93); gdn_chunk_fwd writes zeros at the padding
- *               of o, gdn_recurrent_fwd writes o at valid tokens only.
+ *               then packs and unpacks around the operator, :25-93); o is written at valid tokens only, unless
+ *               GDN_FLAG_ZERO_PADDING asks gdn_chunk_fwd for zeros at the padding.
  *
  * Replaces the argument list of both fla calls at gated_deltanet/module.py:198-222.
  */

@@ -23,6 +23,7 @@ GDN_FLAG_READY_FLAGS_CLEAR = 16
 GDN_FLAG_RECORDS_16X16 = 32
 GDN_FLAG_DEBUG_NO_PRODUCERS = 64
 GDN_FLAG_SKIP_EMPTY_CHUNKS = 128
+GDN_FLAG_ZERO_PADDING = 256
 
 GDN_NORM_GATE_DWORDS = 0x100
 

@@ -178,6 +178,7 @@ static ChunkParams chunk_params(const gdn_args& a) {
     const bool left_padded = (a.flags & GDN_FLAG_LEFT_PADDED) != 0;
     p.cu_seqlens = left_padded ? nullptr : a.cu_seqlens;
     p.pad_lens = left_padded ? a.cu_seqlens : nullptr;
+    p.zero_padding = left_padded && (a.flags & GDN_FLAG_ZERO_PADDING) ? 1 : 0;
     p.chunk_off = static_cast<int32_t*>(a.workspace);
     p.seq_order = p.chunk_off + a.N + 1;
     p.ready = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(a.workspace) + chunk_off_bytes(a));

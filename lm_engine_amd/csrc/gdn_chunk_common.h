@@ -25,6 +25,7 @@ struct ChunkParams {
     bf16_t* o;
     const int32_t* cu_seqlens;  // packed sequences (B == 1), else NULL
     const int32_t* pad_lens;    // left-padded batch: prefix sums of the valid lengths, else NULL
+    int zero_padding;           // left-padded batch: zeros at the padding of o (GDN_FLAG_ZERO_PADDING)
     int32_t* chunk_off;  // [N + 1] prefix of chunks per sequence (packed input only)
     int32_t* seq_order;  // [N] the sequences by decreasing number of chunks (packed input only)
     uint8_t* rec;        // workspace records, [H][TC]

@@ -756,10 +756,10 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
         return;
     }
 
-    // The padding rows of a left-padded batch read as zeros: a compute wave writes those of its columns (16 bytes a lane, 4 lanes a
-    // row; two half-slice waves take turns) while the first chunk is on its way.  As a fill of the whole output by the caller they
-    // took a launch and a pass of their own (6 x 1500 tokens, 16 heads, V = 128: 7.5 us).
-    if (p.pad_lens != nullptr && !p.records_given && !NOOUT) {
+    // Zeros at the padding rows of a left-padded batch, for a caller that asks for them: a compute wave writes those of its columns (16
+    // bytes a lane, 4 lanes a row; two half-slice waves take turns) while the first chunk is on its way.  As a fill of the whole output
+    // by the caller they took a launch and a pass of their own (6 x 1500 tokens, 16 heads, V = 128: 7.5 us).
+    if (p.zero_padding && !NOOUT) {
         const int w = HALF ? 0 : wave, step = HALF ? 32 : 16;
         bf16_t* const og = p.o + b * p.o_stride_b + (int64_t)h * p.o_stride_h + 32 * (vgroup * NW + w) + 8 * (lane % 4);
         bf16x8 zero8;

@@ -373,7 +373,8 @@ PyObject* delta_rule(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (output_final && inplace) need(h0 != nullptr), ht = *h0, s.flags |= GDN_FLAG_STATE_INPLACE;
         without_interpreter_lock([&] {
             if (chunked) workspace = at::empty({(int64_t)workspace_bytes}, q.options().dtype(at::kByte)), s.workspace = ptr(workspace), s.workspace_bytes = workspace_bytes;
-            // (padding positions of a left-padded batch read as zeros: gdn_chunk_fwd writes them, the token kernels do not)
+            // (padding positions of a left-padded batch read as zeros: gdn_chunk_fwd writes them on request, the token kernels do not)
+            if (padded && chunked) s.flags |= GDN_FLAG_ZERO_PADDING;
             o = padded && !chunked ? at::zeros({B, T, H, V}, v.options()) : fresh(v, {B, T, H, V});
             if (output_final && !inplace) ht = fresh_f32(v, {N, H, K, V});
         });

@@ -266,7 +266,7 @@ def _run(mode, q, k, v, g, beta, scale, initial_state, output_final_state, cu_se
         cu_seqlens = cu_seqlens.to(torch.int32).contiguous()
     h0 = None if initial_state is None else initial_state.contiguous()
 
-    # padding positions of a left-padded batch read as zeros: gdn_chunk_fwd writes them, the token kernels do not
+    # padding positions of a left-padded batch read as zeros: gdn_chunk_fwd writes them on request, the token kernels do not
     o = (torch.zeros if left_padded and mode != "chunk" else torch.empty)(B, T, H, V, dtype=v.dtype, device=v.device)
     ht = None
     if output_final_state:
@@ -283,6 +283,8 @@ def _run(mode, q, k, v, g, beta, scale, initial_state, output_final_state, cu_se
 
     with torch.cuda.device(q.device):
         if mode == "chunk":
+            if left_padded:
+                args.flags |= _lib.GDN_FLAG_ZERO_PADDING
             args.error_word = _raise_if_forward_failed(q.device).data_ptr()
             key, workspace = _chunk_workspace(lib, args, q, dims, stream.value)
             try:

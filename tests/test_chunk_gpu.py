@@ -4,12 +4,14 @@ Every case feeds the GPU and the oracle the same bf16-rounded tensors; the gate 
 the benchmark contract for bf16 inputs: max-abs <= 2e-2 and relative-L2 <= 1e-2 on both the
 output and the final state."""
 
+import ctypes
 import os
 
 import pytest
 import torch
 
 import lm_engine_amd
+from lm_engine_amd import _lib, ops
 from lm_engine_amd.workloads import get_workload, make_inputs
 from oracle.c_oracle import recurrent_gated_delta_rule_c
 from tests.helpers import assert_parity, max_abs, random_inputs, rel_l2
@@ -189,6 +191,45 @@ def test_left_padded_batch_equals_separate_runs(K, V):
         o_ref, h_ref = recurrent_gated_delta_rule_c(**cpu, initial_state=inp["initial_state"][b : b + 1], output_final_state=True)
         assert_parity(o_b.float(), o_ref, BF16, "o")
         assert_parity(h_b, h_ref, BF16, "final_state")
+
+
+@pytest.mark.parametrize("B, H, K, V, slices", [(4, 2, 64, 64, 1), (4, 2, 128, 96, 1), (4, 2, 256, 64, 1), (8, 32, 64, 64, 2), (4, 32, 128, 128, 2),
+                                                (8, 32, 64, 128, 4), (8, 32, 128, 128, 4), (4, 32, 128, 256, 4)])  # fmt: skip
+def test_padding_of_the_output_is_written_on_request_only(B, H, K, V, slices):
+    """gdn_chunk_fwd on a left-padded batch, into an output full of NaN: with GDN_FLAG_ZERO_PADDING the padding is zero, without
+    it nothing is written there, and the tokens are the same.  Every scan that writes an output: half-slice waves, two and four
+    slices per workgroup (one workgroup per chain and several)."""
+    cus, chains, tiles = torch.cuda.get_device_properties(0).multi_processor_count, B * H, V // 32
+    nw = 1  # as plan_scan counts them
+    while K <= 128 and nw < 4 and tiles % (2 * nw) == 0 and chains * (tiles // nw) > cus:
+        nw *= 2
+    if cus == 256:
+        assert nw == slices
+    T = 130
+    lengths = [T, 0, 1, T - 1, 64, 66, 129, 65][:B]
+    gpu = _to_gpu(random_inputs(B=B, T=T, H=H, K=K, V=V, dtype=BF16, seed=79))
+    q, k, v, g, beta, h0 = (gpu[n] for n in ("q", "k", "v", "g", "beta", "initial_state"))
+    cu = torch.tensor([0] + lengths).cumsum(0).to(torch.int32).cuda()
+    dims = ops._check_inputs(q, k, v, g, beta, h0, cu, True)
+    lib, stream = _lib.load_library(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    print(f"case: padding of the output B={B} H={H} K={K} V={V}", flush=True)
+    out = {}
+    for flag in (0, _lib.GDN_FLAG_ZERO_PADDING):
+        o = torch.full((B, T, H, V), float("nan"), dtype=BF16, device="cuda")
+        args = ops._fill_args(q, k, v, g, beta, h0, None, o, cu, None, True, False, dims, True)
+        args.flags |= flag
+        workspace = torch.empty(int(lib.gdn_workspace_bytes(ctypes.byref(args))), dtype=torch.uint8, device="cuda")
+        args.workspace, args.workspace_bytes = workspace.data_ptr(), workspace.numel()
+        _lib.check_status(lib.gdn_chunk_fwd(ctypes.byref(args), stream), "gdn_chunk_fwd")
+        torch.cuda.synchronize()
+        out[flag] = o
+    for b, n in enumerate(lengths):
+        assert out[0][b, : T - n].isnan().all(), f"row {b}: written at the padding"
+        assert (out[_lib.GDN_FLAG_ZERO_PADDING][b, : T - n] == 0).all(), f"row {b}: not zero at the padding"
+        tokens = [o[b, T - n :] for o in out.values()]
+        assert torch.isfinite(tokens[0].float()).all() and torch.equal(*tokens)
+    o, _ = lm_engine_amd.chunk_gated_delta_rule(q, k, v, g, beta, initial_state=h0, cu_seqlens=cu, use_qk_l2norm_in_kernel=True, left_padded=True)
+    assert torch.equal(o, out[_lib.GDN_FLAG_ZERO_PADDING])
 
 
 def test_strided_views_of_a_fused_projection():
