@@ -756,17 +756,23 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
         return;
     }
 
-    // Zeros at the padding rows of a left-padded batch, for a caller that asks for them: a compute wave writes those of its columns (16
-    // bytes a lane, 4 lanes a row; two half-slice waves take turns) while the first chunk is on its way.  As a fill of the whole output
-    // by the caller they took a launch and a pass of their own (6 x 1500 tokens, 16 heads, V = 128: 7.5 us).
+    // Zeros at the padding rows of a left-padded batch, for a caller that asks for them, by the compute waves while the first chunk is
+    // on its way.  As a fill of the whole output by the caller they took a launch and a pass of their own (6 x 1500 tokens, two thirds
+    // of them valid, 16 heads, K = V = 128: 67.9 | 61.3 us).  The workgroups of a chain write whole rows of a head together, 16 bytes a
+    // lane, 16 rows a step (32 with two waves per slice) whatever V and NW; a workgroup writing the 64 bytes per row of its own slices
+    // left half lines to the memory (8 x 4096 tokens, 64 valid in each row, 16 heads, K = V = 128: a fill in front 50.1, slices 64.6,
+    // whole rows 46.5 us).  Only where no row holds more than a few chunks and there are few workgroups is a fill the faster one
+    // (2 x 16384 tokens, 65 valid in each row, 4 heads, K = V = 128: 23.2 | 26.0 us).
     if (p.zero_padding && !NOOUT) {
-        const int w = HALF ? 0 : wave, step = HALF ? 32 : 16;
-        bf16_t* const og = p.o + b * p.o_stride_b + (int64_t)h * p.o_stride_h + 32 * (vgroup * NW + w) + 8 * (lane % 4);
+        constexpr int LANES = (HALF ? 2 : NW) * WAVE, STEP = HALF ? 32 : 16;
+        const int per_row = p.V / 8, first = vgroup * LANES + (int)threadIdx.x;
         bf16x8 zero8;
 #pragma unroll
         for (int e = 0; e < 8; e++) zero8[e] = (bf16_t)0.f;
-        for (int row = lane / 4 + (HALF ? 16 * wave : 0); row < (int)seq_t0; row += step)
-            __builtin_nontemporal_store(zero8, reinterpret_cast<bf16x8*>(og + (int64_t)row * p.o_stride_t));
+        int row = first / per_row;
+        bf16_t* at = p.o + b * p.o_stride_b + (int64_t)h * p.o_stride_h + 8 * (first % per_row) + (int64_t)row * p.o_stride_t;
+#pragma unroll 4
+        for (; row < (int)seq_t0; row += STEP, at += STEP * p.o_stride_t) *reinterpret_cast<bf16x8*>(at) = zero8;
     }
 
     if constexpr (HALF) {

@@ -215,13 +215,15 @@ def test_padding_of_the_output_is_written_on_request_only(B, H, K, V, slices):
     print(f"case: padding of the output B={B} H={H} K={K} V={V}", flush=True)
     out = {}
     for flag in (0, _lib.GDN_FLAG_ZERO_PADDING):
-        o = torch.full((B, T, H, V), float("nan"), dtype=BF16, device="cuda")
+        rows = torch.full((B, T, H, V + 8), float("nan"), dtype=BF16, device="cuda")  # (heads with something between them)
+        o = rows[..., :V]
         args = ops._fill_args(q, k, v, g, beta, h0, None, o, cu, None, True, False, dims, True)
         args.flags |= flag
         workspace = torch.empty(int(lib.gdn_workspace_bytes(ctypes.byref(args))), dtype=torch.uint8, device="cuda")
         args.workspace, args.workspace_bytes = workspace.data_ptr(), workspace.numel()
         _lib.check_status(lib.gdn_chunk_fwd(ctypes.byref(args), stream), "gdn_chunk_fwd")
         torch.cuda.synchronize()
+        assert rows[..., V:].isnan().all()
         out[flag] = o
     for b, n in enumerate(lengths):
         assert out[0][b, : T - n].isnan().all(), f"row {b}: written at the padding"
