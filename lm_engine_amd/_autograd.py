@@ -9,6 +9,15 @@ from __future__ import annotations
 import torch
 
 
+def kernel_rows(grad: torch.Tensor, stride_elements: int = 8, address_bytes: int = 16) -> torch.Tensor:
+    """``grad``, or a dense copy of it where a kernel could not read it as it lies: last dim contiguous, the other strides multiples of
+    ``stride_elements``, the first element at a multiple of ``address_bytes``.  For gradients that flow in: their layout is the choice of
+    whatever consumed the output (a column block of a wider gradient, a view at an odd offset), not of the caller."""
+    if grad.stride(-1) == 1 and grad.data_ptr() % address_bytes == 0 and all(s % stride_elements == 0 for s in grad.stride()[:-1]):
+        return grad
+    return grad.clone(memory_format=torch.contiguous_format)  # (contiguous() returns a dense tensor at an odd offset as it is)
+
+
 class _KernelWithFormulaBackward(torch.autograd.Function):
     @staticmethod
     def forward(ctx, kernel, formula, *inputs):

@@ -45,6 +45,8 @@ import weakref
 
 import torch
 
+from ._autograd import kernel_rows
+
 
 CHUNK = 64
 L2NORM_EPS = 1e-6  # the epsilon of the forward kernels' q/k normalisation
@@ -275,7 +277,7 @@ def _sweeps_on_scan_kernel(q, k, v, do, g, beta, scale, initial_state, cu_seqlen
     k_m, v_m, rec = _mirror_problem(N, H, kraw, qraw, doc, Tm, P, egl, cs_a, ks_a, ks_b,
                                     aligned_inputs=(q, k, do) if pk.aligned else None, half_slices=half_slices)  # fmt: skip
     dS1 = torch.empty(Bt, NC, K, V, device=dev)
-    dht32 = None if dht is None else dht.to(torch.float32).contiguous()
+    dht32 = None if dht is None else kernel_rows(dht.to(torch.float32).contiguous())
     # the A chunks are the even ones; mirror chunk 2 r is chunk NC - 1 - r of the forward order
     o_m, dS = ops.chunk_scan_given_records(k_m, v_m, rec, dht32, dS1, NC, save_every=2, save_reverse=True,
                                            half_slice_records=half_slices)  # fmt: skip
@@ -351,7 +353,8 @@ def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm
         NC = max(1, -(-max(lens + [1]) // CHUNK))
         covers = sum(lens) == B * T
         sequences = (*ops.upload_int32((starts, lens), q.device), NC)
-    q, k, v, do = (x if x.stride(-1) == 1 else x.contiguous() for x in (q, k, v, do.to(torch.bfloat16)))
+    q, k, v = (x if x.stride(-1) == 1 else x.contiguous() for x in (q, k, v))
+    do = kernel_rows(do.to(torch.bfloat16))
     if do.stride(1) > 1 << 24:  # the kernels count a chunk's rows in 32 bits; q, k and v were held to that by the forward
         do = do.contiguous()
     prep, S0, Vn, dS1, Y, dh0 = ops.chunk_bwd_sweeps(q, k, v, do, g, beta, scale, l2norm, initial_state, cu_seqlens, left_padded, dht, NC)

@@ -24,7 +24,7 @@ import ctypes
 import torch
 
 from . import _lib
-from ._autograd import kernel_with_formula_backward
+from ._autograd import kernel_rows, kernel_with_formula_backward
 from ._host import host, raw_stream
 from .kernels import Kernel, is_kernel_allowed
 from .layer_ops import column_sums
@@ -158,9 +158,7 @@ def _convolution_backward(x, weight, bias, input_state, attention_mask, dy, acti
     ks = w2.size(1)
     if x.stride(-1) != 1:
         x = x.contiguous()
-    dy = dy.to(x.dtype)
-    if dy.stride(-1) != 1:
-        dy = dy.contiguous()
+    dy = kernel_rows(dy.to(x.dtype), stride_elements=2, address_bytes=8)
     b2 = None if bias is None else bias.to(w2.dtype).contiguous()
     state = None if input_state is None else input_state.to(x.dtype).contiguous()
     mask = None

@@ -18,7 +18,7 @@ import ctypes
 import torch
 
 from . import _lib
-from ._autograd import kernel_with_formula_backward
+from ._autograd import kernel_rows, kernel_with_formula_backward
 from ._host import host, raw_stream
 from .kernels import Kernel, is_kernel_allowed
 
@@ -266,7 +266,7 @@ def _gated_rmsnorm_backward(o, gate, weight, eps, dy):
     """``gdn_gated_rmsnorm_bwd``: gradients with respect to o, gate (shaped like gate) and weight."""
     o2, o_stride, g2, g_stride, H, V = _norm_operands(o, gate)
     tokens = o2.size(0)
-    dy = dy.to(o.dtype).contiguous()
+    dy = kernel_rows(dy.to(o.dtype).contiguous())
     d_o = torch.empty(o.shape, dtype=o.dtype, device=o.device)
     d_gate = None if gate is None else torch.empty(o.shape, dtype=o.dtype, device=o.device)
     blocks = min(2048, max(1, (tokens * H * max(V // 8, 8) + 255) // 256))

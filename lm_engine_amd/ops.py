@@ -31,6 +31,7 @@ from collections import OrderedDict
 import torch
 
 from . import _lib
+from ._autograd import kernel_rows
 from ._host import host, raw_stream
 from .backward import gated_delta_rule_backward
 from .kernels import Kernel, is_kernel_allowed
@@ -610,7 +611,7 @@ def chunk_bwd_sweeps(q, k, v, dout, g, beta, scale, l2norm, initial_state, cu_se
         beta = beta.contiguous() if beta.dtype in (torch.bfloat16, torch.float32) else beta.float().contiguous()
     cu_seqlens = None if cu_seqlens is None else cu_seqlens.to(torch.int32).contiguous()
     h0 = None if initial_state is None else initial_state.contiguous()
-    dht = None if dht is None else dht.to(torch.float32).contiguous()
+    dht = None if dht is None else kernel_rows(dht.to(torch.float32).contiguous())
     prep = {name: torch.empty(N * H, NC, 64, dtype=torch.float32, device=dev) for name in ("gamma", "beta", "rq", "rk")}
     states, dstates = (torch.empty(N * H, NC, K, V, dtype=torch.bfloat16, device=dev) for _ in range(2))
     v_new, y = (torch.empty(N * H, NC, 64, V, dtype=torch.bfloat16, device=dev) for _ in range(2))

@@ -270,3 +270,45 @@ def test_gradients_of_column_blocks_are_those_of_separate_tensors(B, S, HK, H, K
     # one of the three does not get a gradient, or gets a larger one
     (part,) = torch.autograd.grad((2 * blocks[2].float()).sum(), (qkv,), retain_graph=True)
     assert (part[..., 2 * HK * K :] == 2).all() and not part[..., : 2 * HK * K].any()
+
+
+def _layouts(dense):
+    """``dense`` as backward functions of other operations hand gradients on: a column block of a wider tensor (strides that are no
+    multiple of 8, then odd ones) and a view that starts at an odd element."""
+    for extra in (4, 1):
+        wide = torch.cat([dense, torch.full((*dense.shape[:-1], extra), float("nan"), dtype=dense.dtype, device="cuda")], dim=-1)
+        yield f"{extra} columns wider", wide[..., : dense.size(-1)]
+    flat = torch.full((dense.numel() + 1,), float("nan"), dtype=dense.dtype, device="cuda")
+    shifted = flat[1:].view(dense.shape)
+    yield "at an odd element", shifted.copy_(dense)
+
+
+@pytest.mark.parametrize("step", ["operator, V = 64", "operator, V = 32", "operator, fp32", "convolution", "norm", "gates"])
+def test_gradients_flow_in_whatever_their_layout(step):
+    """The layout of an incoming gradient is chosen by whatever consumed the output: every layout gives the gradients of the dense one,
+    in the same bits (the same kernels on the same values)."""
+    gen = torch.Generator().manual_seed(7)
+    dtype = F32 if step.endswith("fp32") else BF16
+    leaf = lambda *shape: torch.randn(*shape, generator=gen).to(dtype).cuda().requires_grad_(True)  # noqa: E731
+    B, T, H, K = 2, 130, 2, 64
+    V = 32 if step.endswith("32") else 64
+    if step.startswith("operator"):
+        q, k, v, h0 = leaf(B, T, H, K), leaf(B, T, H, K), leaf(B, T, H, V), leaf(B, H, K, V).detach().float().requires_grad_(True)
+        leaves = [q, k, v, h0]
+        outputs = lm_engine_amd.chunk_gated_delta_rule(q, k, v, initial_state=h0, output_final_state=True, use_qk_l2norm_in_kernel=True)
+    elif step == "convolution":
+        leaves = [leaf(B, T, 64), leaf(64, 4), leaf(64)]
+        outputs = lm_engine_amd.depthwise_causal_convolution(*leaves)[:1]
+    elif step == "norm":
+        leaves = [leaf(B, T, H, V), leaf(B, T, H, V), leaf(V)]
+        outputs = (lm_engine_amd.gated_rmsnorm(*leaves, 1e-5),)
+    else:
+        leaves = [leaf(B, T, H), leaf(B, T, H), leaf(H).detach().float().requires_grad_(True), leaf(H).detach().float().requires_grad_(True)]
+        outputs = lm_engine_amd.delta_rule_gates(*leaves)
+    dense = [torch.randn(o.shape, generator=gen).to(o.dtype).cuda() for o in outputs]
+    want = torch.autograd.grad(outputs, leaves, dense, retain_graph=True)
+    for j, d in enumerate(dense):
+        for name, x in _layouts(d):
+            print(f"case: {step}, gradient of output {j} {name}", flush=True)
+            got = torch.autograd.grad(outputs, leaves, [*dense[:j], x, *dense[j + 1 :]], retain_graph=True)
+            assert all(torch.equal(a, b) for a, b in zip(got, want)), name
