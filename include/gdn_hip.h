@@ -580,7 +580,8 @@ int gdn_column_sums(const gdn_column_sums_args *args, void *stream);
  * A padding mask [B, S] (1 for tokens, 0 for the padding; integers of element_bytes 1 (unsigned), 4 or 8, element strides, B at most
  * GDN_MASK_MAX_ROWS) in the two forms that the layer's calls take: out [B, S] contiguous in out_dtype (gdn_conv_args.mask) and prefix
  * int32 [B + 1], a leading 0 and the prefix sums of the rows' sums (gdn_args.cu_seqlens with GDN_FLAG_LEFT_PADDED;
- * compute_cu_seqlens_and_max_seqlen_from_attention_mask, sequence_packing.py:18-22).  One workgroup: meant for up to some 64 K elements.
+ * compute_cu_seqlens_and_max_seqlen_from_attention_mask, sequence_packing.py:18-22).  One workgroup: meant for up to some 64 rows and
+ * 64 K elements.
  */
 #define GDN_MASK_MAX_ROWS 1024
 int gdn_padding_mask(const void *mask, int element_bytes, int64_t stride_b, int64_t stride_s, int B, int S, void *out, int out_dtype,

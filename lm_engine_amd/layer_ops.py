@@ -58,24 +58,36 @@ def _token_rows(x: torch.Tensor, width: int, what: str) -> tuple[torch.Tensor, i
 
 
 _MASK_BYTES = {torch.int64: 8, torch.int32: 4, torch.uint8: 1, torch.bool: 1}
-_MASK_ROWS, _MASK_ELEMENTS = 1024, 1 << 16  # one workgroup's work: a few microseconds
+# The masks that go through one launch.  It is one workgroup of 16 waves, which take a row each and so wait for memory once per 16
+# rows; torch's six launches spread them over the chip.  One launch | torch, microseconds on the device (the host asks for 11 | 31),
+# int64: 1 x 1024 3.3 | 14, 6 x 1500 4.9 | 15, 64 x 140 6.7 | 14, 17 x 1927 8.6 | 19, 64 x 512 9.4 | 15, 6 x 10922 13 | 20,
+# 64 x 1024 14.0 | 15.4; with more rows 96 x 682 17 | 15.5, 128 x 512 16.6 | 14.8, 256 x 35 13.9 | 13.9, 256 x 256 22 | 14, 1024 x 8 49 | 14.
+_MASK_ROWS, _MASK_ELEMENTS = 64, 1 << 16
+
+
+def _one_launch_mask(B: int, S: int, mask_dtype: torch.dtype, dtype: torch.dtype) -> bool:
+    return mask_dtype in _MASK_BYTES and dtype in (torch.bfloat16, torch.float32) and 0 < B <= _MASK_ROWS and 0 < B * S <= _MASK_ELEMENTS
 
 
 def padding_mask(attention_mask: torch.Tensor, dtype: torch.dtype):
     """The integer ``attention_mask`` ``[B, S]`` in ``dtype`` (contiguous) and the prefix sums of its rows' sums, int32 ``[B + 1]``, in
-    one launch (``gdn_padding_mask``); the same through torch where the mask is large or of another type."""
+    one launch (``gdn_padding_mask``); the same through torch where that is the faster way or the mask of another type."""
     B, S = attention_mask.shape
-    element_bytes = _MASK_BYTES.get(attention_mask.dtype)
-    if element_bytes is None or not attention_mask.is_cuda or B > _MASK_ROWS or not 0 < B * S <= _MASK_ELEMENTS or dtype not in (torch.bfloat16, torch.float32):
+    if not attention_mask.is_cuda or not _one_launch_mask(B, S, attention_mask.dtype, dtype):
         seqlens = attention_mask.sum(dim=-1, dtype=torch.int32)  # sequence_packing.py:18-22
         return attention_mask, torch.nn.functional.pad(torch.cumsum(seqlens, dim=0, dtype=torch.int32), (1, 0))
+    return _padding_mask_kernel(attention_mask, dtype)
+
+
+def _padding_mask_kernel(attention_mask, dtype):
+    B, S = attention_mask.shape
     mask = torch.empty(B, S, dtype=dtype, device=attention_mask.device)
     prefix = torch.empty(B + 1, dtype=torch.int32, device=attention_mask.device)
     lib = _lib.load_library()
     with torch.cuda.device(attention_mask.device):
         stream = ctypes.c_void_p(torch.cuda.current_stream(attention_mask.device).cuda_stream)
         _lib.check_status(
-            lib.gdn_padding_mask(attention_mask.data_ptr(), element_bytes, attention_mask.stride(0), attention_mask.stride(1), B, S,
+            lib.gdn_padding_mask(attention_mask.data_ptr(), _MASK_BYTES[attention_mask.dtype], attention_mask.stride(0), attention_mask.stride(1), B, S,
                                  mask.data_ptr(), _dtype_code(dtype, "mask"), prefix.data_ptr(), stream), "gdn_padding_mask")  # fmt: skip
     return mask, prefix
 

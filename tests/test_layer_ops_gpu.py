@@ -144,15 +144,16 @@ def test_operands_on_the_host_are_refused_before_any_launch():
 @pytest.mark.parametrize("B, S", [(1, 1), (1, 64), (2, 65), (6, 1500), (15, 63), (16, 64), (17, 129), (300, 7), (1024, 64), (1025, 3), (8, 8193)])
 def test_padding_mask_matches_torch(dtype, B, S):
     """One launch against sum, cumsum and conversion: whole numbers, so the same values.  Rows shared by several waves, a row per wave, more
-    rows than waves and than lanes, sizes that go through torch; also a mask that is not contiguous."""
-    from lm_engine_amd.layer_ops import padding_mask
+    rows than waves and than lanes, sizes that go through torch (the launch by itself there as well); also a mask that is not contiguous."""
+    from lm_engine_amd.layer_ops import _MASK_BYTES, _padding_mask_kernel, padding_mask
 
+    ways = [padding_mask] + ([_padding_mask_kernel] if dtype in _MASK_BYTES and B <= 1024 else [])
     lengths = torch.randint(0, S + 1, (B,), generator=torch.Generator().manual_seed(B + S))
     mask = (torch.arange(S)[None, :] >= S - lengths[:, None]).to(dtype).cuda()
     strided = torch.stack((mask, torch.zeros_like(mask)), dim=-1)[..., 0]
     for x in (mask, strided, mask[:1].expand(B, S)):
-        for out_dtype in (torch.bfloat16, torch.float32):
-            got, prefix = padding_mask(x, out_dtype)
+        for out_dtype, way in [(o, w) for o in (torch.bfloat16, torch.float32) for w in ways]:
+            got, prefix = way(x, out_dtype)
             assert torch.equal(got.to(out_dtype), x.to(out_dtype))
             assert prefix.dtype == torch.int32
             assert torch.equal(prefix.cpu(), torch.nn.functional.pad(x.cpu().long().sum(-1).cumsum(0), (1, 0)).int())
