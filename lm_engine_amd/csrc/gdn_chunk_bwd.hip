@@ -198,7 +198,8 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
     constexpr int PHASE2 = 2 * SLAB + 2 * C * LDK * 2;      // G^T | Hm^T | q | k (and phase 3)
     constexpr int LDS_BYTES = cmax(PHASE1, PHASE2);
     __shared__ __attribute__((aligned(16))) uint8_t lds[LDS_BYTES];
-    __shared__ float s_gam[C], s_beta[C], s_e[C], s_tail[C], s_fq[C], s_fk[C];
+    __shared__ __attribute__((aligned(16))) float s_gam[C], s_beta[C];  // (read 16 bytes at a time)
+    __shared__ float s_e[C], s_tail[C], s_fq[C], s_fk[C];
     // Sums over waves: every wave leaves its part in a place of its own and they are added up in one order at the end (as LDS atomics
     // they stood in the waves' way - 653 -> 617 us per training step of 4 x 4096 tokens, 16 heads, K = V = 128 - and moved the
     // rounding of a few gradients from run to run).  Per token: <Y, V>; by 32 keys <dQs, Qs>, <dK, K> and the terms of dgamma and dbeta
@@ -617,6 +618,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 #pragma unroll
             for (int r4 = 0; r4 < 4; r4++) {
                 const int i0 = 32 * ti + 8 * r4 + 4 * lh;
+                static_assert(__alignof__(s_gam) % 16 == 0 && __alignof__(s_beta) % 16 == 0, "16-byte reads");
                 const f32x4 gi = *reinterpret_cast<const f32x4*>(&s_gam[i0]), bi = *reinterpret_cast<const f32x4*>(&s_beta[i0]);
                 f32x4 G, Hm;
 #pragma unroll
