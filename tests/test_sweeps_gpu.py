@@ -110,3 +110,29 @@ def test_output_gradient_with_rows_far_apart():
     print(f"case: dO rows {apart} apart", flush=True)
     for far, near in zip(*(gated_delta_rule_backward(q, k, v, None, None, d)[:3] for d in (do, dense))):
         assert torch.equal(far, near)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout, lens", [("rows", [256, 256]), ("rows", [130]), ("packed", [100, 0, 64, 1, 333]), ("padded", [200, 70, 0, 1])])
+@pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (256, 512)])
+def test_every_run_of_the_backward_gives_the_same_bits(layout, lens, K, V):
+    """Every sum of the sweeps and of the chunk-local kernel has one order.  Enough heads that several workgroups share a CU, ten runs
+    (sums through LDS atomics differed in a few entries from one run to the next)."""
+    from lm_engine_amd.backward import gated_delta_rule_backward
+
+    gen = torch.Generator().manual_seed(sum(lens) + K)
+    N, H = len(lens), 64
+    B, T = (1, sum(lens)) if layout == "packed" else (N, max(lens))
+    normal = lambda *shape: torch.randn(*shape, generator=gen)  # noqa: E731
+    q, k, v, do = (normal(B, T, H, n).bfloat16().cuda() for n in (K, K, V, V))
+    g, beta = torch.nn.functional.logsigmoid(3 + normal(B, T, H)).cuda(), normal(B, T, H).sigmoid().bfloat16().cuda()
+    h0, dht = (0.1 * normal(N, H, K, V).cuda() for _ in range(2))
+    cu = None if layout == "rows" else torch.tensor([0, *lens]).cumsum(0).to(torch.int32).cuda()
+    print(f"case: ten runs, {layout} {lens} K={K} V={V}", flush=True)
+    first = None
+    for _ in range(10):
+        grads = gated_delta_rule_backward(q, k, v, g, beta, do, dht, initial_state=h0, cu_seqlens=cu, use_qk_l2norm_in_kernel=True,
+                                          left_padded=layout == "padded")  # fmt: skip
+        first = grads if first is None else first
+        for name, a, b in zip(("dq", "dk", "dv", "dg", "dbeta", "dh0"), grads, first):
+            assert torch.isfinite(a.float()).all() and torch.equal(a, b), name
