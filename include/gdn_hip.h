@@ -217,7 +217,13 @@ int gdn_recurrent_fwd_kernels(const gdn_args *args);
  * whole-slice waves, 1 or 4 slices per workgroup).  records_given = 2: they are in the lane order of the
  * 16x16x32 MFMA (any K, required for K = 256); the scan then runs one slice per workgroup on two half-slice
  * waves, which is the faster kernel as long as N * H * V / 32 does not exceed the number of compute units.
- * The backward pass of this package runs its reverse sweep over the chunks that way.
+ *
+ * What the backward pass of this package calls: gdn_chunk_bwd_sweeps and gdn_chunk_bwd_local where V is a multiple of 64, and
+ * for other V this entry point with fp32 saves, once as it is and once with records_given, save_every and save_reverse.
+ * Everything else in this struct (bf16 saves, no_output, mirror_reads, sliced, row_order, packed_records), and all of
+ * gdn_chunk_bwd_prepare, is the two-scan form that gdn_chunk_bwd_sweeps took the place of: it stays, and is tested, for callers
+ * of this interface.
+ *
  * states_dtype, v_new_dtype: GDN_F32, or GDN_BF16 (the pointer is then a bf16 array of the same shape).  bf16 saves
  * need the variant of the scan that stages its saves through LDS, which gdn_chunk_fwd_saving_is_staged reports for
  * the same arguments and saves (one column slice per workgroup, and K <= 128; or K = 256 with no_output, bf16 or no
@@ -272,19 +278,20 @@ int gdn_chunk_fwd_saving_is_staged(const gdn_args *args, const gdn_chunk_saves *
 
 /*
  * Training support, second part: the chunk-local gradients, one workgroup per (sequence, head, chunk), once
- * the two sweeps over the chunks (gdn_chunk_fwd_saving, forward and mirrored) have delivered per chunk the
- * state it starts from, the gradient of the state it ends with, V~ and Y = T^T dV~.  Chunk index
+ * the two sweeps over the chunks (gdn_chunk_bwd_sweeps; or gdn_chunk_fwd_saving, forward and mirrored) have delivered per chunk
+ * the state it starts from, the gradient of the state it ends with, V~ and Y = T^T dV~.  Chunk index
  * = (n * H + h) * NC + c; per-chunk arrays are contiguous and chunk-major:
  *     v_new         [chunks][64][V]   V~, in saves_dtype (what gdn_chunk_fwd_saving wrote)
  *     states        [chunks][K][V]    the state a chunk starts from, in saves_dtype
  *     dstates       [chunks][K][V]    the gradient of the state it ends with, in dstates_dtype (fp32 or bf16)
- *     gamma, beta   [chunks][64]      prefix sum of g inside the chunk, beta (fp32; from gdn_chunk_bwd_prepare)
+ *     gamma, beta   [chunks][64]      prefix sum of g inside the chunk, beta (fp32; from gdn_chunk_bwd_sweeps or
+ *                                     gdn_chunk_bwd_prepare)
  *     rq, rk        [chunks][64]      1 / sqrt(|q|^2 + 1e-6), likewise for k, when q and k were normalised
  *                                     (the l2norm flag of the forward); both NULL otherwise
  *     y_mirror      bf16 [N, 2 * NC * 64, H, V]: the output of the scan over the mirror problem of
  *                   gdn_chunk_bwd_prepare (Y at its even chunks, tokens reversed); or NULL and
- *     y_chunks      bf16 [chunks][64][V]: the V~ that scan saved at its even chunks (save_every = 2, save_reverse,
- *                   bf16 saves, no output): Y of chunk (n, h, c) with its tokens in reverse order
+ *     y_chunks      bf16 [chunks][64][V]: Y of chunk (n, h, c) with its tokens in reverse order, from gdn_chunk_bwd_sweeps, or as
+ *                   the V~ that the mirror scan saved at its even chunks (save_every = 2, save_reverse, bf16 saves, no output)
  *     q_raw, k_raw, v_raw, dout_raw   the caller's bf16 q, k, v, dO, [N, NC * 64, H, D] with element strides
  * Outputs, in the caller's layout, contiguous: dq_out, dk_out [N, NC * 64, H, K] and dv_out [N, NC * 64, H, V]
  * (bf16; the gradients with respect to q and k themselves, through the scale and the normalisation), dg_out and
@@ -323,7 +330,7 @@ typedef struct gdn_chunk_local_args {
 int gdn_chunk_bwd_local(const gdn_chunk_local_args *args, void *stream);
 
 /*
- * Training support, third part: everything the backward needs per chunk before its two sweeps (batches of
+ * Training support, third part: everything the backward needs per chunk before two sweeps through gdn_chunk_fwd_saving (batches of
  * whole chunks: T a multiple of 64, one sequence per row; other batches through seq_start / seq_len below;
  * bf16 q, k, dout as [N, T, H, D] with element
  * strides; K = 64, 128 or 256 and V a multiple of 64, GDN_ERR_UNSUPPORTED otherwise).  One workgroup per (sequence, head, chunk) writes

@@ -30,7 +30,7 @@
 //   2. the rows of q and k (128 keys at a time) for Q K^T and K K^T, then the 64 x 64 stage: G^T and Hm^T are left in LDS;
 //   3. per 128 keys: the per-token sums over the key dim, dQ^T and dK^T; q^T, k^T, G and Hm come out of those rows with the
 //      transposing LDS load.
-// K = 256 on the sliced saves of the staging scans has one wave per SIMD and so 512 registers per lane: it asks for the
+// K = 256 on sliced saves has one wave per SIMD and so 512 registers per lane: it asks for the
 // rows of the next slab, and of the next half of q and k, while the products of the current one run, and keeps them
 // in registers until their turn (PIPE below).
 // K = 64, 128, 256; V a multiple of 64.
@@ -61,10 +61,9 @@ struct ChunkLocalParams {
     const float* rq;  // 1 / |q|, 1 / |k| per token when q and k were normalised, else NULL
     const float* rk;
     float scale;
-    // chunk = (n H + h) NC + c.  Y is read from the output of the scan over the mirror problem; q, k, v, dO are the
-    // caller's tensors (bf16, element strides); the gradients go out in the caller's layout, [N, NC 64, H, .] bf16
+    // chunk = (n H + h) NC + c.  q, k, v, dO are the caller's tensors (bf16, element strides); the gradients go out in the caller's layout, [N, NC 64, H, .] bf16
     // for q, k, v and fp32 [N, NC 64, H] for g (reverse prefix sum of dgamma done here) and beta
-    const bf16_t* y_mirror;  // [N][2 NC 64][H][V], or NULL and
+    const bf16_t* y_mirror;  // the output of a scan over the mirror problem, [N][2 NC 64][H][V], or NULL and
     const bf16_t* y_chunks;  // [chunk][64][V]: Y of the chunk, tokens reversed
     const bf16_t* q_raw;
     const bf16_t* k_raw;
@@ -802,8 +801,8 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 
 
 // ------------------------------------------------------------------------------------------
-// Everything the backward needs per chunk before its two sweeps, one workgroup per (sequence, head, chunk),
-// for batches of whole chunks (one sequence per row, T a multiple of 64):
+// gdn_chunk_bwd_prepare, for callers that run the two sweeps as scans (the package's backward runs gdn_chunk_sweep.hip):
+// everything needed per chunk before them, one workgroup per (sequence, head, chunk), for batches of whole chunks (one sequence per row, T a multiple of 64):
 //   * gamma, beta (fp32) and the inverse norms of the rows of q and k, packed per chunk, for
 //     chunk_local_grads_kernel;
 //   * the "mirror" problem that turns the reverse sweep into a forward scan (tokens in reverse order; chunk c

@@ -35,7 +35,7 @@ struct ChunkParams {
     int64_t o_stride_b, o_stride_t, o_stride_h;
     int B, T, H, V, N;
     int qk_div;  // value heads per head of q and k (grouped value attention): head h reads q and k of head h / qk_div
-    // Mirror reads (the reverse sweep of the backward pass on the scan without output): the sequence the scan walks is
+    // Mirror reads (gdn_chunk_saves.mirror_reads, the scan without output): the sequence the scan walks is
     // the caller's sequence backwards, every chunk twice - chunk 2 r takes its rows of k from k and of v from v, chunk
     // 2 r + 1 from k2 and v2, both as tokens 64 (NT / 2 - 1 - r) + 63 - row of those tensors ([N, T / 2, H, .]).
     int mirror;
@@ -60,7 +60,7 @@ struct ChunkParams {
     int save_reverse;  // ... or, when set, as entry save_nc - 1 - c / save_every
     const int32_t* row_order;  // left-padded rows of given records: the order in which the rows' chains are dealt out (or NULL)
     int save_state_bf16, save_vnew_bf16;  // that array is bf16 (the pointer then points at bf16 data); staged saves only
-    int no_output;     // the scan writes no output (a sweep of the backward pass); staged saves only
+    int no_output;     // the scan writes no output (gdn_chunk_saves.no_output); staged saves only
     int records_given;  // the records are already in place: prepare is not run
     int32_t* ready;     // [H][TC] one flag per record, for the launch that runs prepare and scan together
     int fused;          // that launch was asked for (GDN_FLAG_FUSED_LAUNCH)

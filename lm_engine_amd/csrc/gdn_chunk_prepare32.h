@@ -325,7 +325,9 @@ __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8
             };
             // first the two diagonal tiles of A, which the inverse starts from, and two of the three tiles of P
             // (P[i < 32][j >= 32] = 0 is not stored); their products need the rows only and run beside the first wave's scales
-            // (with the row sums in registers: one-launch forward of 4 x 4096 tokens, 16 heads, K = V = 128 110.0 -> 107.3 us)
+            // (with the row sums in registers, at steady clocks: one-launch forward of 4 x 4096 tokens, 16 heads, K = V = 128 109.5 ->
+            // 107.2 us, training step of the same batch 594 -> 584; no change in the one-launch forward of a device that has not come to
+            // its clocks, 122.5, and in a packed forward, 244)
             const bool is_p = wave % 2 == 1;
             const int diag = wave / 2;
             if (tid < C) {

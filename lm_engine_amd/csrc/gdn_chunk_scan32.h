@@ -201,7 +201,7 @@ struct ScanSchedule : ScanScheduleRules<K> {
 // The pieces are half as large as in the whole-slice schedule; placement is the same earliest-deadline walk.  With
 // MFMAs this short an op can be over in 16 cycles, so results are taken DIST ops after their MFMA and LDS data
 // LA ops (operand fragments) or AHEAD ops (scales, rows of v) after the read was issued.
-// NOOUT: a scan that only carries the state and V~ (the sweeps of the backward pass): the two groups that form the output
+// NOOUT: a scan that only carries the state and V~ (gdn_chunk_saves.no_output): the two groups that form the output
 // and the pieces that serve them are left out.
 template <int K, bool NOOUT = false>
 struct Scan16Rules {

@@ -372,7 +372,7 @@ def saving_scan_is_staged(N, T, H, K, V, cu_seqlens=None, left_padded=False, rec
 
 def chunk_forward_saving(q, k, v, g, beta, scale, initial_state, cu_seqlens, l2norm, left_padded, states, v_new,
                          chunks_per_chain, no_output=False, sliced=False, workspace=None):  # fmt: skip
-    """The chunked forward once more, for the backward pass: through ``gdn_chunk_fwd_saving`` it writes the
+    """The chunked forward once more, for the backward pass where V is not a multiple of 64: through ``gdn_chunk_fwd_saving`` it writes the
     state every chunk starts from into ``states`` ``[N * H, chunks_per_chain, K, V]`` and V~ into ``v_new``
     ``[N * H, chunks_per_chain, 64, V]`` (contiguous; fp32, or bf16 where ``saving_scan_is_staged``).  The output
     itself is discarded (``no_output``: the library skips forming it where it has a scan without output).  ``workspace``
@@ -508,7 +508,7 @@ def chunk_scan_given_records(k, v, records, initial_state, states, chunks_per_ch
 
 
 def backward_kernels_apply(K: int, V: int) -> bool:
-    """Head dims ``gdn_chunk_bwd_prepare`` and ``gdn_chunk_bwd_local`` are built for."""
+    """Head dims ``gdn_chunk_bwd_sweeps`` and ``gdn_chunk_bwd_local`` (and ``gdn_chunk_bwd_prepare``) are built for."""
     return K in _SUPPORTED_K and V % 64 == 0
 
 
@@ -527,10 +527,10 @@ def column_blocks(q, k, v) -> bool:
 def chunk_local_grads(q, k, v, dout, prep, y_mirror, v_new, states, dstates, scale, l2norm, sequences=None, sliced=False,
                       covers=False, joined=False):
     """``gdn_chunk_bwd_local``: q, k, v, dout are the caller's bf16 ``[B, T, H, D]`` tensors (last dim contiguous),
-    ``prep`` what ``chunk_bwd_prepare`` returned (same ``sequences``), ``y_mirror`` the output of the scan over its
-    mirror problem (bf16 ``[N, 2 NC 64, H, V]``) or, as a 4-D tensor, the V~ that scan saved at its even chunks (bf16
-    ``[N H, NC, 64, V]``), ``v_new`` and ``states`` what the saving forward sweep wrote (both fp32 or both bf16),
-    ``dstates`` the states the mirror scan saved (fp32 or bf16).  Returns ``dq, dk, dv`` bf16 ``[B, T, H, D]`` (with ``joined``
+    the other arrays what ``chunk_bwd_sweeps`` returned (``sliced``; ``y_mirror``: its Y, bf16 ``[N H, NC, 64, V]``).  Also for sweeps as
+    scans: ``prep`` from ``chunk_bwd_prepare`` (same ``sequences``), ``y_mirror`` the output of the scan over its mirror problem (bf16
+    ``[N, 2 NC 64, H, V]``) or the V~ that scan saved at its even chunks, ``v_new`` and ``states`` from the saving forward sweep (both
+    fp32 or both bf16), ``dstates`` the states the mirror scan saved (fp32 or bf16).  Returns ``dq, dk, dv`` bf16 ``[B, T, H, D]`` (with ``joined``
     the column blocks of one ``[B, T, H (2 K + V)]`` tensor) and ``dg, dbeta`` fp32 ``[B, T, H]`` (zero where no sequence lives)."""
     _require_hip_path()
     lib = _lib.load_library()
@@ -639,7 +639,7 @@ RECORD_BYTES = 13312  # a chunk record: 12 operand fragments, 3 x 64 row scales,
 
 def chunk_bwd_prepare(q, k, dout, g, beta, scale, l2norm, V, sequences=None, half_slice_records=False,
                       forward_records=False, reversed_copies=True, skip_empty_chunks=False, packed=False):
-    """``gdn_chunk_bwd_prepare``.  ``q, k, dout`` are the caller's bf16 ``[B, T, H, D]`` tensors; without
+    """``gdn_chunk_bwd_prepare``, what sweeps as scans need (the package's backward calls ``chunk_bwd_sweeps``).  ``q, k, dout`` are the caller's bf16 ``[B, T, H, D]`` tensors; without
     ``sequences`` every row is one sequence of whole chunks, else ``sequences = (seq_start, seq_len, NC)``: int32
     device tensors ``[N]`` (first token as a flat index over the rows, length) and the chunks per sequence to lay
     the results out with.  Returns a dict: ``gamma, beta, rq, rk`` (fp32 ``[N H, NC, 64]``: prefix sums of g inside
