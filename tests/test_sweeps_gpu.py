@@ -136,3 +136,45 @@ def test_every_run_of_the_backward_gives_the_same_bits(layout, lens, K, V):
         first = grads if first is None else first
         for name, a, b in zip(("dq", "dk", "dv", "dg", "dbeta", "dh0"), grads, first):
             assert torch.isfinite(a.float()).all() and torch.equal(a, b), name
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout, lens, bad", [("packed", [100, 64, 0, 1, 133, 70], 1), ("packed", [100, 64, 0, 1, 133, 70], 4), ("padded", [200, 70, 1, 129], 1)])
+@pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (256, 512)])
+def test_nan_stays_in_its_sequence(layout, lens, bad, K, V):
+    """NaN in every token, state and gradient of one sequence, and at the padding: the other sequences' results keep their bits."""
+    import lm_engine_amd
+    from lm_engine_amd.backward import gated_delta_rule_backward
+
+    gen = torch.Generator().manual_seed(3)
+    N, H, padded = len(lens), 3, layout == "padded"
+    B, T = (N, max(lens)) if padded else (1, sum(lens))
+    normal = lambda *shape: torch.randn(*shape, generator=gen)  # noqa: E731
+    q, k, v, do = (normal(B, T, H, n).bfloat16().cuda() for n in (K, K, V, V))
+    g, beta = torch.nn.functional.logsigmoid(3 + normal(B, T, H)).cuda(), normal(B, T, H).sigmoid().bfloat16().cuda()
+    h0, dht = (0.1 * normal(N, H, K, V).cuda() for _ in range(2))
+    cu = torch.tensor([0, *lens]).cumsum(0).to(torch.int32).cuda()
+    spans = [(n, slice(T - lens[n], T)) if padded else (0, slice(sum(lens[:n]), sum(lens[: n + 1]))) for n in range(N)]
+    print(f"case: NaN in sequence {bad} of {layout} {lens} K={K} V={V}", flush=True)
+
+    def results(q, k, v, do, g, beta, h0, dht):
+        options = dict(initial_state=h0, cu_seqlens=cu, use_qk_l2norm_in_kernel=True, left_padded=padded)
+        o, ht = lm_engine_amd.chunk_gated_delta_rule(q, k, v, g, beta, output_final_state=True, **options)
+        dq, dk, dv, dg, dbeta, dh0 = gated_delta_rule_backward(q, k, v, g, beta, do, dht, **options)
+        return (o, dq, dk, dv, dg, dbeta), (ht, dh0)
+
+    def poisoned(x):  # everything but the tokens of the good sequences
+        y = torch.full_like(x, float("nan"))
+        for n, span in enumerate(spans):
+            if n != bad:
+                y[span] = x[span]
+        return y
+
+    states = [x.clone() for x in (h0, dht)]
+    for x in states:
+        x[bad] = float("nan")
+    want, got = results(q, k, v, do, g, beta, h0, dht), results(*map(poisoned, (q, k, v, do, g, beta)), *states)
+    for n, span in enumerate(spans):
+        if n != bad:
+            assert all(torch.equal(a[span], b[span]) and torch.isfinite(a[span].float()).all() for a, b in zip(got[0], want[0]))
+            assert all(torch.equal(a[n], b[n]) for a, b in zip(got[1], want[1]))
