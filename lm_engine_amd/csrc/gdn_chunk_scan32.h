@@ -464,8 +464,34 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
     const bool is_store = OS && wave == 4;
     constexpr bool EIGHT = NW == 2 || HALF;  // the wave layout of two compute waves
     const bool is_loader = NW == 4 ? wave >= 4 : EIGHT ? (wave == 2 || wave == 3 || wave >= 6) : (wave >= 1 && wave != 4);
-    if (EIGHT && wave == 5) return;
+    // Zeros at the padding rows of a left-padded batch, for a caller that asks for them, while the first chunk is on its way: by two
+    // waves that have nothing else to do at that time, the store wave and the one whose place is empty, or by the four compute waves.
+    // As a fill of the whole output by the caller they took a launch and a pass of their own (6 x 1500 tokens, two thirds of them
+    // valid, 16 heads, K = V = 128: 67.9 | 61.2 us).  The workgroups of a chain write whole rows of a head together, 16 bytes a lane,
+    // 16 rows a step (32 with half slices) whatever V and NW; a workgroup writing the 64 bytes per row of its own slices left half
+    // lines to the memory (8 x 4096 tokens, 64 valid in each row, 16 heads, K = V = 128: a fill in front 50.1, slices 64.6, whole
+    // rows 46.7 us).  Only where no row holds more than a few chunks and there are few workgroups is a fill the faster one
+    // (2 x 16384 tokens, 65 valid in each row, 4 heads, K = V = 128: 23.2 | 25.5 us).
+    constexpr bool ZEROS = !SAVE;
+    static_assert(!ZEROS || EIGHT || NW == 4, "the waves that write them");
+    auto zero_rows = [&](int w) {  // wave w of them
+        if (!p.zero_padding) return;
+        constexpr int LANES = (EIGHT ? 2 : 4) * WAVE, STEP = LANES / (4 * NW);
+        const int per_row = p.V / 8, first = vgroup * LANES + w * WAVE + lane;
+        bf16x8 zero8;
+#pragma unroll
+        for (int e = 0; e < 8; e++) zero8[e] = (bf16_t)0.f;
+        int row = first / per_row;
+        bf16_t* at = p.o + b * p.o_stride_b + (int64_t)h * p.o_stride_h + 8 * (first % per_row) + (int64_t)row * p.o_stride_t;
+#pragma unroll 4
+        for (; row < (int)seq_t0; row += STEP, at += STEP * p.o_stride_t) *reinterpret_cast<bf16x8*>(at) = zero8;
+    };
+    if (EIGHT && wave == 5) {
+        if constexpr (ZEROS) zero_rows(1);
+        return;
+    }
     if (is_store) {
+        if constexpr (ZEROS && EIGHT) zero_rows(0);
         // ------------------------------ output store ------------------------------
         // The compute waves leave the bf16 output tile of chunk c in LDS while they work on chunk c + 1; this
         // wave writes it out after the next barrier.  A store that waits for queue space then stalls here and
@@ -756,24 +782,7 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
         return;
     }
 
-    // Zeros at the padding rows of a left-padded batch, for a caller that asks for them, by the compute waves while the first chunk is
-    // on its way.  As a fill of the whole output by the caller they took a launch and a pass of their own (6 x 1500 tokens, two thirds
-    // of them valid, 16 heads, K = V = 128: 67.9 | 61.3 us).  The workgroups of a chain write whole rows of a head together, 16 bytes a
-    // lane, 16 rows a step (32 with two waves per slice) whatever V and NW; a workgroup writing the 64 bytes per row of its own slices
-    // left half lines to the memory (8 x 4096 tokens, 64 valid in each row, 16 heads, K = V = 128: a fill in front 50.1, slices 64.6,
-    // whole rows 46.5 us).  Only where no row holds more than a few chunks and there are few workgroups is a fill the faster one
-    // (2 x 16384 tokens, 65 valid in each row, 4 heads, K = V = 128: 23.2 | 26.0 us).
-    if (p.zero_padding && !NOOUT) {
-        constexpr int LANES = (HALF ? 2 : NW) * WAVE, STEP = HALF ? 32 : 16;
-        const int per_row = p.V / 8, first = vgroup * LANES + (int)threadIdx.x;
-        bf16x8 zero8;
-#pragma unroll
-        for (int e = 0; e < 8; e++) zero8[e] = (bf16_t)0.f;
-        int row = first / per_row;
-        bf16_t* at = p.o + b * p.o_stride_b + (int64_t)h * p.o_stride_h + 8 * (first % per_row) + (int64_t)row * p.o_stride_t;
-#pragma unroll 4
-        for (; row < (int)seq_t0; row += STEP, at += STEP * p.o_stride_t) *reinterpret_cast<bf16x8*>(at) = zero8;
-    }
+    if constexpr (ZEROS && !EIGHT) zero_rows(wave);
 
     if constexpr (HALF) {
         // ------------------------------ compute (HALF) ------------------------------
