@@ -18,6 +18,7 @@ namespace gdn {
 
 constexpr int REC_THREADS = 256;
 constexpr int REC_WAVES = REC_THREADS / WAVE;
+constexpr int CHAIN_COLUMNS = 4;  // columns of a workgroup of recurrent_chain_kernel
 
 // The decode step, and calls of a few tokens over many states: one read and one write of the state, everything else hidden
 // behind them.  A workgroup streams a K x BV tile through its registers.  A token's own operands are asked for ahead of the
@@ -252,6 +253,215 @@ __global__ __launch_bounds__(REC_THREADS) void recurrent_tokens_kernel(const Rec
     }
 }
 
+// More than one token over few states: the same chain, with everything that is not the chain taken out of its wave.
+//
+// One wave's instructions issue one after another, so a token of recurrent_tokens_kernel costs the sum of its products with k
+// and with q, of its output, of its staging and of the copies between them, though only S^T k -> r -> S' depends on the token
+// before (487 cycles a token at K = 64, of which the chain is under 160).  Here a workgroup holds four columns and its four waves, each on a SIMD of its own, have a part each: one runs the
+// chain and leaves the residuals r of 16 tokens in LDS, one follows a block behind it, takes the same state through the same
+// steps with those residuals and forms the outputs, and two stage the block ahead.  The state's update is done twice, and k
+// and q are staged by four times as many workgroups: worth it only while the chip has SIMDs to spare (launch_recurrent_tokens_k).
+// Bound by the chain.  B = 1, T = 256, H = 2, K = V = 64, fp32: 57.0 -> 21.3 us, with norms 64.1 -> 26.5; T = 200, H = 16, K = V =
+// 128 67 -> 33.  Norms one token after the other (their sums over a wave are ten dependent steps) made the staging waves the
+// slowest: 33.9 us with norms; four tokens' sums in the four rows of a wave: 26.5.
+template <typename T, int K>
+__global__ __launch_bounds__(REC_THREADS) void recurrent_chain_kernel(const RecurrentParams p) {
+    constexpr int TB = 16;                // tokens per block: one per lane of a DPP row
+    constexpr int RPT = K / 16;           // state rows per lane, consecutive ones
+    constexpr int KPL = K / WAVE;         // q/k elements per lane when a wave loads a whole row
+    constexpr int BV = CHAIN_COLUMNS;     // columns per workgroup: one per DPP row
+    constexpr int TPW = TB / 2;           // tokens a staging wave takes
+    constexpr int AHEAD = K == 256 ? 2 : 4;  // tokens whose operands are on their way out of LDS
+
+    __shared__ __attribute__((aligned(16))) float s_k[3][TB][K], s_q[3][TB][K];
+    __shared__ __attribute__((aligned(16))) float s_tok[3][TB][BV][4];  // v, beta, e^g, k^ . q^
+    __shared__ float s_r[2][TB][BV];
+
+    const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int rg = lane % 16, cg = lane / 16;
+    const int v_base = blockIdx.x * BV;
+    const int h = blockIdx.y, n = blockIdx.z;
+
+    int64_t b = n, t_begin = 0, t_end = p.T;
+    if (p.pad_lens != nullptr) t_begin = p.T - min(max(p.pad_lens[n + 1] - p.pad_lens[n], 0), p.T);  // the last tokens of row n
+    if (p.cu_seqlens != nullptr) {
+        int t0, len;
+        packed_bounds(p.cu_seqlens, n, p.T, t0, len);
+        if (len < p.len_min || len > p.len_max) return;  // the other kernel's (the whole workgroup)
+        b = 0, t_begin = t0, t_end = t0 + len;
+    }
+    const int blocks = (int)((t_end - t_begin + TB - 1) / TB);
+    // Every wave passes blocks + 2 barriers: one behind the first block's staging, one behind each of blocks + 1 steps.  In
+    // step i the chain is at block i, the outputs at block i - 1, the staging at block i + 1.
+
+    if (wave >= 2) {
+        const int64_t hqk = p.qk_div > 1 ? h / p.qk_div : h;
+        const T* qp = reinterpret_cast<const T*>(p.q) + b * p.q_stride_b + hqk * p.q_stride_h;
+        const T* kp = reinterpret_cast<const T*>(p.k) + b * p.k_stride_b + hqk * p.k_stride_h;
+        const T* vp = reinterpret_cast<const T*>(p.v) + b * p.v_stride_b + h * p.v_stride_h + v_base;
+        const int first = (wave - 2) * TPW;
+        const int tl = lane / BV % TPW, cl = lane % BV;  // the token and the column whose s_tok this lane forms
+        struct Staged {
+            float k[TPW][KPL], q[TPW][KPL], v, g, beta;
+        };
+        auto fetch = [&](Staged& x, int i) {  // tokens past the sequence's end are read from its last one and never used
+            const int64_t t0 = t_begin + (int64_t)min(i, blocks - 1) * TB + first;
+#pragma unroll
+            for (int j = 0; j < TPW; j++) {
+                const int64_t t = min(t0 + j, t_end - 1);
+                load_run<KPL>(kp + t * p.k_stride_t + lane * KPL, x.k[j]);
+                load_run<KPL>(qp + t * p.q_stride_t + lane * KPL, x.q[j]);
+            }
+            const int64_t t = min(t0 + tl, t_end - 1), sidx = (b * p.T + t) * p.H + h;
+            x.v = to_f32(vp[t * p.v_stride_t + cl]);
+            x.g = p.g != nullptr ? p.g[sidx] : 0.f;
+            x.beta = load_beta(p.beta, p.beta_dtype, sidx);
+        };
+        auto stage = [&](const Staged& x, int buf) {
+            if (lane < TPW * BV) *reinterpret_cast<f32x3*>(&s_tok[buf][first + tl][cl][0]) = f32x3{x.v, x.beta, p.g != nullptr ? expf(x.g) : 1.f};
+#pragma unroll
+            for (int j = 0; j < TPW; j += 4) {
+                const TokenNorms norms = token_norms4<KPL>(x.k + j, x.q + j, p.l2norm, p.scale);
+                if (rg < BV) s_tok[buf][first + j + cg][rg][3] = norms.kq;
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    const float kn = lane_value(norms.kn, 16 * t), qn = lane_value(norms.qn, 16 * t);
+#pragma unroll
+                    for (int e = 0; e < KPL; e++) {
+                        // row lane KPL + e is row `at` of row group lane / 4; the groups' pieces of 4 rows lie side by side
+                        const int at = lane % 4 * KPL + e, pos = at / 4 * 64 + lane / 4 * 4 + at % 4;
+                        s_k[buf][first + j + t][pos] = x.k[j + t][e] * kn;
+                        s_q[buf][first + j + t][pos] = x.q[j + t][e] * qn;
+                    }
+                }
+            }
+        };
+        Staged x, y;
+        if (blocks > 0) {
+            fetch(x, 0);
+            fetch(y, 1);
+            stage(x, 0);
+        }
+        __syncthreads();
+        int buf = 1;
+        for (int i = 0; i <= blocks; i++) {
+            if (i + 1 < blocks) {
+                x = y;
+                fetch(y, i + 2);
+                stage(x, buf);
+            }
+            buf = buf == 2 ? 0 : buf + 1;
+            __syncthreads();
+        }
+        return;
+    }
+
+    const int64_t state_off = (((int64_t)n * p.H + h) * K + RPT * rg) * p.V + v_base + cg;
+    float S[RPT];
+#pragma unroll
+    for (int i = 0; i < RPT; i++) S[i] = p.h0 != nullptr ? p.h0[state_off + (int64_t)i * p.V] : 0.f;
+
+    auto walk = [&](auto&& token, auto&& read, auto& x, int count) {  // one block, operands read AHEAD tokens before their use
+#pragma unroll
+        for (int j = 0; j < AHEAD; j++) read(x[j], j);
+        if (count == TB) {
+#pragma unroll
+            for (int tt = 0; tt < TB; tt++) {
+                token(x[tt % AHEAD], tt);
+                if (tt + AHEAD < TB) read(x[tt % AHEAD], tt + AHEAD);
+                __builtin_amdgcn_sched_barrier(0);  // else the reads sink to their use
+            }
+        } else {
+            for (int tt = 0; tt < count; tt++) {
+                read(x[0], tt);
+                token(x[0], tt);
+            }
+        }
+    };
+
+    if (wave == 0) {
+        struct Operands {
+            f32x4 k[RPT / 4];
+            f32x3 tok;
+        } x[AHEAD];
+        __syncthreads();
+        int buf = 0;
+        for (int i = 0; i <= blocks; i++) {
+            if (i < blocks) {
+                float kept = 0.f;  // r of token rg
+                walk(
+                    [&](const Operands& x, int tt) {
+                        float k0 = 0.f, k1 = 0.f;
+#pragma unroll
+                        for (int e = 0; e < RPT; e += 2) {
+                            k0 = fmaf(S[e], x.k[e / 4][e % 4], k0), k1 = fmaf(S[e + 1], x.k[e / 4][e % 4 + 1], k1);
+                        }
+                        const float r = token_residual(x.tok[0], row16_sum(k0 + k1), x.tok[2], x.tok[1]);
+#pragma unroll
+                        for (int e = 0; e < RPT; e++) S[e] = token_state(S[e], x.tok[2], r, x.k[e / 4][e % 4]);
+                        kept = rg == tt ? r : kept;
+                    },
+                    [&](Operands& x, int tt) {
+#pragma unroll
+                        for (int j = 0; j < RPT / 4; j++) x.k[j] = *reinterpret_cast<const f32x4*>(&s_k[buf][tt][64 * j + 4 * rg]);
+                        x.tok = *reinterpret_cast<const f32x3*>(&s_tok[buf][tt][cg][0]);
+                    },
+                    x, (int)min((int64_t)TB, t_end - t_begin - (int64_t)i * TB));
+                s_r[i % 2][rg][cg] = kept;
+            }
+            buf = buf == 2 ? 0 : buf + 1;
+            __syncthreads();
+        }
+        return;
+    }
+
+    struct Operands {
+        f32x4 k[RPT / 4], q[RPT / 4];
+        f32x2 tok;
+        float r;
+    } x[AHEAD];
+    T* op = reinterpret_cast<T*>(p.o) + b * p.o_stride_b + h * p.o_stride_h + v_base + cg;
+    __syncthreads();
+    int buf = 2;
+    for (int i = 0; i <= blocks; i++) {
+        if (i > 0) {
+            const int64_t t0 = t_begin + (int64_t)(i - 1) * TB;
+            const int count = (int)min((int64_t)TB, t_end - t0);
+            float kept = 0.f;  // o of token rg
+            walk(
+                [&](const Operands& x, int tt) {
+                    float q0 = 0.f, q1 = 0.f;
+#pragma unroll
+                    for (int e = 0; e < RPT; e += 2) {
+                        q0 = fmaf(S[e], x.q[e / 4][e % 4], q0), q1 = fmaf(S[e + 1], x.q[e / 4][e % 4 + 1], q1);
+                    }
+                    const float o = token_output(row16_sum(q0 + q1), x.tok[0], x.r, x.tok[1]);
+#pragma unroll
+                    for (int e = 0; e < RPT; e++) S[e] = token_state(S[e], x.tok[0], x.r, x.k[e / 4][e % 4]);
+                    kept = rg == tt ? o : kept;
+                },
+                [&](Operands& x, int tt) {
+#pragma unroll
+                    for (int j = 0; j < RPT / 4; j++) {
+                        x.k[j] = *reinterpret_cast<const f32x4*>(&s_k[buf][tt][64 * j + 4 * rg]);
+                        x.q[j] = *reinterpret_cast<const f32x4*>(&s_q[buf][tt][64 * j + 4 * rg]);
+                    }
+                    x.tok = *reinterpret_cast<const f32x2*>(&s_tok[buf][tt][cg][2]);
+                    x.r = s_r[(i - 1) % 2][tt][cg];
+                },
+                x, count);
+            if (rg < count) op[(t0 + rg) * p.o_stride_t] = from_f32<T>(kept);
+        }
+        buf = buf == 2 ? 0 : buf + 1;
+        __syncthreads();
+    }
+    // (the chain's wave took its copy of the state in before the first step ended, so a state updated in place is safe here)
+    if (p.ht != nullptr) {
+#pragma unroll
+        for (int i = 0; i < RPT; i++) p.ht[state_off + (int64_t)i * p.V] = S[i];
+    }
+}
+
 template <typename T, int K, int CPL>
 static int launch_recurrent_tokens(const RecurrentParams& p, int N, hipStream_t stream) {
     hipLaunchKernelGGL((recurrent_tokens_kernel<T, K, CPL>), dim3(p.V / (16 * CPL), p.H, N), dim3(REC_THREADS), 0, stream, p);
@@ -287,9 +497,22 @@ int recurrent_kernels(const gdn_args& a) {
     return GDN_RECURRENT_TOKENS;
 }
 
+// recurrent_chain_kernel's workgroups hold four columns; as many as are worth their doubled work.  tokens kernel | chain kernel:
+// K = 64, T = 64, 512 workgroups 19.2 | 12.9 us, 1024 18.0 | 16.4, 2048 20.3 | 37; K = 128, T = 60, 512 24.1 | 16.9, 1024 25.1 |
+// 28.5; K = 256 (100 KB of LDS, one workgroup per CU) T = 60, 256 27.3 | 18.1, T = 40, 512 20.9 | 27.7.  A block is 16 tokens; with
+// fewer there is nothing to run side by side (K = 128, 512 workgroups: T = 3 6.5 | 7.4, T = 20 11.2 | 10.7).
+constexpr int CHAIN_TOKENS = 16;
+template <int K>
+constexpr int64_t CHAIN_WORKGROUPS = K == 64 ? 1024 : K == 128 ? 512 : 256;
+
 template <typename T, int K>
 static int launch_recurrent_tokens_k(const RecurrentParams& p, int N, hipStream_t stream) {
     const int64_t pairs = (int64_t)N * p.H;
+    const int64_t tokens = p.cu_seqlens != nullptr ? p.T / N : p.T;  // of a sequence, on average
+    if (tokens >= CHAIN_TOKENS && pairs * (p.V / CHAIN_COLUMNS) <= CHAIN_WORKGROUPS<K>) {
+        hipLaunchKernelGGL((recurrent_chain_kernel<T, K>), dim3(p.V / CHAIN_COLUMNS, p.H, N), dim3(REC_THREADS), 0, stream, p);
+        return (int)hipGetLastError();
+    }
     // As few columns per lane as leave at most 1024 workgroups (at K <= 128 four per CU, what LDS and registers hold at a
     // time).  Measured with 1 | 2 | 4: B = 5, T = 60, H = 16, K = V = 128 (640 workgroups at 1) 36 | 38 | 41 us, B = 5, T = 33,
     // H = 32, V = 256 (2560) 60 | 55 | 58 us, B = 64, T = 16, H = 16, V = 128 (8192) 100 | 83 | 72 us.

@@ -70,6 +70,12 @@ __device__ __forceinline__ float wave_total(float x) {
     return swap_add<32>(x, x);
 }
 
+// Four such sums at once: the 16 lanes of row r get that of x[r].
+__device__ __forceinline__ float wave_totals4(float x0, float x1, float x2, float x3) {
+    x0 = row16_sum(x0), x1 = row16_sum(x1), x2 = row16_sum(x2), x3 = row16_sum(x3);
+    return swap_add<32>(swap_add<16>(x0, x1), swap_add<16>(x2, x3));
+}
+
 // N consecutive elements as fp32, in one access
 template <int N>
 __device__ __forceinline__ void load_run(const bf16_t* p, float (&x)[N]) {
@@ -108,6 +114,31 @@ __device__ __forceinline__ TokenNorms token_norms(const float (&kx)[KPL], const 
         r.qn = rsqrtf(wave_total(ssq) + L2NORM_EPS) * scale;
         // k . q of finite rows overflows only if a sum of squares does; that row's k^ or q^ is 0 then, and so is k^ . q^
         // (0 times the overflowed product would be a NaN)
+        r.kq = r.kn == 0.f || r.qn == 0.f ? 0.f : r.kq * r.kn * r.qn;
+    }
+    return r;
+}
+// The same for four tokens: row r of the wave gets the norms of token r, bit for bit those of token_norms.
+template <int KPL>
+__device__ __forceinline__ TokenNorms token_norms4(const float (*kx)[KPL], const float (*qx)[KPL], bool l2norm, float scale) {
+    const float q_scale = l2norm ? 1.f : scale;
+    float ssk[4], ssq[4], dot[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        ssk[j] = 0.f, ssq[j] = 0.f, dot[j] = 0.f;
+#pragma unroll
+        for (int e = 0; e < KPL; e++) {
+            ssk[j] = fmaf(kx[j][e], kx[j][e], ssk[j]);
+            ssq[j] = fmaf(qx[j][e], qx[j][e], ssq[j]);
+            dot[j] = fmaf(kx[j][e], qx[j][e] * q_scale, dot[j]);
+        }
+    }
+    TokenNorms r;
+    r.kn = 1.f, r.qn = scale;
+    r.kq = wave_totals4(dot[0], dot[1], dot[2], dot[3]);
+    if (l2norm) {
+        r.kn = rsqrtf(wave_totals4(ssk[0], ssk[1], ssk[2], ssk[3]) + L2NORM_EPS);
+        r.qn = rsqrtf(wave_totals4(ssq[0], ssq[1], ssq[2], ssq[3]) + L2NORM_EPS) * scale;
         r.kq = r.kn == 0.f || r.qn == 0.f ? 0.f : r.kq * r.kn * r.qn;
     }
     return r;

@@ -167,6 +167,31 @@ def test_several_tokens_match_the_oracle_and_the_steps_they_consist_of(dtype, B,
     assert torch.equal(torch.cat([o_head, o_last], dim=1), o) and torch.equal(h_last, ht)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("l2norm", [False, True])
+@pytest.mark.parametrize(
+    "lens, H, K, V",
+    # V / 4 workgroups per (sequence, head) up to 1024, 512, 256 at K = 64, 128, 256 run as chain, outputs and staging side by
+    # side, from 16 tokens on: both sides of these limits, whole and cut blocks, empty and short sequences among longer ones
+    [([15], 2, 64, 64), ([16], 2, 64, 64), ([17] * 2, 32, 64, 64), ([17] * 2, 33, 64, 64), ([33], 16, 128, 128),
+     ([33], 17, 128, 128), ([48], 2, 256, 512), ([31], 3, 256, 512), ([0, 1, 63, 16, 0, 32, 5], 3, 128, 64)],
+)  # fmt: skip
+def test_a_few_chains_give_the_bits_of_single_steps(lens, H, K, V, l2norm, dtype):
+    N, T = len(lens), sum(lens)
+    gpu = _to_gpu(random_inputs(B=1, T=T, H=H, K=K, V=V, dtype=dtype, seed=90 + T, normalize=not l2norm, N=N))
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+    h0 = gpu.pop("initial_state")
+    state, steps = h0.clone(), h0.clone()
+    run = lambda x, h, **kw: lm_engine_amd.fused_recurrent_gated_delta_rule(  # noqa: E731
+        **x, initial_state=h, output_final_state=True, use_qk_l2norm_in_kernel=l2norm, **kw)  # fmt: skip
+    o, _ = run(gpu, state, cu_seqlens=cu, inplace_state=True)
+    for n, begin in enumerate(cu.tolist()[:-1]):
+        for t in range(begin, begin + lens[n]):
+            want, _ = run({name: x[:, t : t + 1] for name, x in gpu.items()}, steps[n : n + 1], inplace_state=True)
+            assert torch.equal(o[:, t : t + 1], want), (n, t)
+    assert torch.equal(state, steps)
+
+
 def test_output_final_state_false_returns_none_and_runs_are_bitwise_repeatable():
     inp = _to_gpu(random_inputs(B=2, T=8, H=2, K=64, V=64, dtype=torch.bfloat16, seed=46))
     o1, none = lm_engine_amd.fused_recurrent_gated_delta_rule(**inp)
