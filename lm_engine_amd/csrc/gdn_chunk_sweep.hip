@@ -167,52 +167,60 @@ struct SweepSchedule : SweepRules<K, REV> {
     static constexpr int op_of(int pc) { return TABLE.op[pc]; }
 };
 
+// One workgroup of a sweep.
 template <int K, bool REV>
-__global__ __launch_bounds__(SWEEP_WAVES* WAVE) void chunk_sweep_kernel(const SweepParams p) {
+struct Sweep {
     typedef SweepSchedule<K, REV> SCH;
     // K = 256, reverse: two stage halves with the rows of q and of k do not fit the LDS.  The rows of q, which a chunk needs for
     // one group of MFMAs only, then get a single buffer and a second workgroup barrier per chunk ("barrier Q"), and so do
     // the staged saves: they are written between that barrier and the chunk's own and taken out between the latter and
     // the next barrier Q.
-    constexpr bool QS = SCH::QS;
-    constexpr int NL = SWEEP_LOADERS;
-    constexpr int KS = SCH::KS, KT = SCH::KT;
+    static constexpr bool QS = SCH::QS;
+    static constexpr int NL = SWEEP_LOADERS;
+    static constexpr int KS = SCH::KS, KT = SCH::KT;
     // One half of the stage: fragments T' (forward: 6) or T^T | P^T (reverse: 12) | this workgroup's 32 columns of 64 rows of v or
     // dO | rows of q (reverse) | of k | four vectors of 64 scales: ks | cs | e^{gamma_C} | - (forward), qs | ks | beta cs | e^{gamma_C}
-    constexpr int FRAGS = REV ? 12 : 6;
-    constexpr int VLD = 64;                          // bytes per staged row of v / dO
-    constexpr int V_UNITS = C * VLD / FRAG_BYTES;    // 1 KiB pieces: 16 rows each
-    constexpr int QLD = 2 * K + 16;                  // bytes per staged row of q / k (16 bytes of padding against bank conflicts)
-    constexpr int Q_UNITS = C * 2 * K / FRAG_BYTES;  // 1 KiB pieces of the rows of k; as many of q
-    constexpr int V_OFF = FRAGS * FRAG_BYTES;
-    constexpr int Q_OFF = V_OFF + C * VLD;  // not part of the stage halves when QS
-    constexpr int K_OFF = (REV && !QS) ? Q_OFF + C * QLD : Q_OFF;
-    constexpr int SC_OFF = K_OFF + C * QLD;
-    constexpr int STAGE_BYTES = SC_OFF + 4 * C * 4;
-    constexpr int XS_OFF = SC_OFF + C * 4;  // scale of K S's rows: cs, ks
-    constexpr int YS_OFF = SC_OFF + (REV ? 2 : 0) * C * 4;  // scale of V~'s or Y's rows in the state update: ks, beta cs
-    constexpr int EG_OFF = SC_OFF + (REV ? 3 : 2) * C * 4;
-    constexpr int NF = (FRAGS + NL - 1) / NL;  // fragment slots per loader wave (forward: 8 slots for 6 fragments, two of them twice)
-    constexpr int NV = V_UNITS / NL;
-    constexpr int NKR = Q_UNITS / NL;          // slots of rows of k; as many of q
-    constexpr int NQR = REV ? NKR : 0;
-    constexpr int NLOAD = NF + NV + NKR + NQR;
+    static constexpr int FRAGS = REV ? 12 : 6;
+    static constexpr int VLD = 64;                          // bytes per staged row of v / dO
+    static constexpr int V_UNITS = C * VLD / FRAG_BYTES;    // 1 KiB pieces: 16 rows each
+    static constexpr int QLD = 2 * K + 16;                  // bytes per staged row of q / k (16 bytes of padding against bank conflicts)
+    static constexpr int Q_UNITS = C * 2 * K / FRAG_BYTES;  // 1 KiB pieces of the rows of k; as many of q
+    static constexpr int V_OFF = FRAGS * FRAG_BYTES;
+    static constexpr int Q_OFF = V_OFF + C * VLD;  // not part of the stage halves when QS
+    static constexpr int K_OFF = (REV && !QS) ? Q_OFF + C * QLD : Q_OFF;
+    static constexpr int SC_OFF = K_OFF + C * QLD;
+    static constexpr int STAGE_BYTES = SC_OFF + 4 * C * 4;
+    static constexpr int XS_OFF = SC_OFF + C * 4;  // scale of K S's rows: cs, ks
+    static constexpr int YS_OFF = SC_OFF + (REV ? 2 : 0) * C * 4;  // scale of V~'s or Y's rows in the state update: ks, beta cs
+    static constexpr int EG_OFF = SC_OFF + (REV ? 3 : 2) * C * 4;
+    static constexpr int NF = (FRAGS + NL - 1) / NL;  // fragment slots per loader wave (forward: 8 slots for 6 fragments, two of them twice)
+    static constexpr int NV = V_UNITS / NL;
+    static constexpr int NKR = Q_UNITS / NL;          // slots of rows of k; as many of q
+    static constexpr int NQR = REV ? NKR : 0;
+    static constexpr int NLOAD = NF + NV + NKR + NQR;
     static_assert(V_UNITS % NL == 0 && Q_UNITS % NL == 0, "the pieces must divide over the loader waves");
     // the staged saves, transposed: [32 columns][K + 8 keys], [32 columns][64 + 8 tokens]; a compute-wave lane writes 8 consecutive
     // keys (its operand register as it is) or 4 consecutive tokens of one column, the store wave turns them back into rows
-    constexpr int SCOL = (K + 8) * 2, VCOL = (C + 8) * 2, SBUFS = QS ? 1 : 2;
-    __shared__ __attribute__((aligned(16))) uint8_t stage[2][STAGE_BYTES];
-    __shared__ __attribute__((aligned(16))) uint8_t qstage[QS ? C * QLD : 16];
-    __shared__ __attribute__((aligned(16))) uint8_t sstage[SBUFS][32 * SCOL];
-    __shared__ __attribute__((aligned(16))) uint8_t vstage[SBUFS][32 * VCOL];
-    static_assert(2 * STAGE_BYTES + (QS ? C * QLD : 16) + SBUFS * 32 * (SCOL + VCOL) <= 160 * 1024, "stage exceeds LDS");
+    static constexpr int SCOL = (K + 8) * 2, VCOL = (C + 8) * 2, SBUFS = QS ? 1 : 2;
+    // LDS: the stage halves | qstage | sstage | vstage
+    static constexpr int QSTAGE_OFF = 2 * STAGE_BYTES, SSTAGE_OFF = QSTAGE_OFF + (QS ? C * QLD : 0), VSTAGE_OFF = SSTAGE_OFF + SBUFS * 32 * SCOL;
+    static constexpr int LDS_BYTES = VSTAGE_OFF + SBUFS * 32 * VCOL;
+    static_assert(LDS_BYTES <= 160 * 1024 && STAGE_BYTES % 16 == 0, "stage exceeds LDS");
 
+    static __device__ __forceinline__ void run(const SweepParams& p, int id, uint8_t* lds);
+};
+
+template <int K, bool REV>
+__device__ __forceinline__ void Sweep<K, REV>::run(const SweepParams& p, int id, uint8_t* const lds) {
+    uint8_t* const qstage = lds + QSTAGE_OFF;
+    auto stage = [&](int i) { return lds + (i & 1) * STAGE_BYTES; };
+    auto sstage = [&](int i) { return lds + SSTAGE_OFF + (QS ? 0 : i & 1) * 32 * SCOL; };
+    auto vstage = [&](int i) { return lds + VSTAGE_OFF + (QS ? 0 : i & 1) * 32 * VCOL; };
     const int lane = threadIdx.x % WAVE;
     const int wave = threadIdx.x / WAVE;
 
     // workgroup -> (sequence-head chain, column slice), as in the scan of the forward: the slices of a chain on one XCD, the
     // chains of a packed batch dealt out longest first
-    const int id = blockIdx.x;
     const int xcd = id % 8, rest = id / 8;
     const int groups = p.V / 32;
     const int vgroup = rest % groups;
@@ -281,11 +289,11 @@ __global__ __launch_bounds__(SWEEP_WAVES* WAVE) void chunk_sweep_kernel(const Sw
         };
         auto flush_state = [&](int i) {
             const int64_t at = ((int64_t)chain * p.save_nc + chunk_of(i)) * K * p.V + K * 32 * vgroup;
-            flush(sstage[QS ? 0 : i & 1], SCOL / 2, p.save_state + at, std::integral_constant<int, K>{}, std::false_type{});
+            flush(sstage(i), SCOL / 2, p.save_state + at, std::integral_constant<int, K>{}, std::false_type{});
         };
         auto flush_v = [&](int i) {
             const int64_t at = ((int64_t)chain * p.save_nc + chunk_of(i)) * C * p.V + C * 32 * vgroup;
-            flush(vstage[QS ? 0 : i & 1], VCOL / 2, p.save_v + at, std::integral_constant<int, C>{}, std::integral_constant<bool, REV>{});
+            flush(vstage(i), VCOL / 2, p.save_v + at, std::integral_constant<int, C>{}, std::integral_constant<bool, REV>{});
         };
         __syncthreads();
         for (int i = 0; i < nchunks; i++) {
@@ -354,7 +362,7 @@ __global__ __launch_bounds__(SWEEP_WAVES* WAVE) void chunk_sweep_kernel(const Sw
         auto store_and_reload = [&](bf16x8(&buf)[NLOAD], float& sc, int i, int i2, auto reload_tag, auto barrier_q_tag) {
             constexpr bool reload = decltype(reload_tag)::value;
             constexpr bool barrier_q = decltype(barrier_q_tag)::value;
-            uint8_t* const dst = stage[i & 1];
+            uint8_t* const dst = stage(i);
             const int c2 = chunk_of(i2);
             reinterpret_cast<float*>(dst + SC_OFF)[lw * C + lane] = sc;
 #pragma unroll
@@ -482,17 +490,17 @@ __global__ __launch_bounds__(SWEEP_WAVES* WAVE) void chunk_sweep_kernel(const Sw
     };
 
     __syncthreads();  // stage[0] holds step 0
-    egc = lds_eg(stage[0]);
-    if constexpr (REV) dobn[0] = load_do(stage[0], 0), dobn[1] = load_do(stage[0], 1);
-    static_for<0, LA>([&](auto i) { fnext[decltype(i)::value] = lds_frag(stage[0], i); });
+    egc = lds_eg(stage(0));
+    if constexpr (REV) dobn[0] = load_do(stage(0), 0), dobn[1] = load_do(stage(0), 1);
+    static_for<0, LA>([&](auto i) { fnext[decltype(i)::value] = lds_frag(stage(0), i); });
 #pragma unroll
     for (int s = 0; s < KS; s++) sb[s] = pack4x2(S[2 * s], S[2 * s + 1]);
 
     for (int i = 0; i < nchunks; i++) {
-        const uint8_t* const st = stage[i & 1];
-        const uint8_t* const stn = stage[(i + 1) & 1];
-        uint8_t* const s_at = sstage[QS ? 0 : i & 1] + (16 * half + j16) * SCOL + (8 * g) * 2;
-        uint8_t* const v_at = vstage[QS ? 0 : i & 1] + (16 * half + j16) * VCOL + (4 * g) * 2;
+        const uint8_t* const st = stage(i);
+        const uint8_t* const stn = stage(i + 1);
+        uint8_t* const s_at = sstage(i) + (16 * half + j16) * SCOL + (8 * g) * 2;
+        uint8_t* const v_at = vstage(i) + (16 * half + j16) * VCOL + (4 * g) * 2;
         bf16x8 fr[NOPS];
 #pragma unroll
         for (int f = 0; f < LA; f++) fr[f] = fnext[f];
@@ -611,14 +619,50 @@ __global__ __launch_bounds__(SWEEP_WAVES* WAVE) void chunk_sweep_kernel(const Sw
     }
 }
 
+// Both sweeps in one launch: neither needs anything of the other, so with fewer workgroups than compute units they run side by
+// side, and with more the forward sweep's first workgroups start on the units that the reverse sweep's last ones leave idle.  The
+// reverse sweep comes first, its chunks are the longer ones.  `first`: the number of the launch's first workgroup.  Kernel times, two
+// launches | one: 4 x 4096 tokens, 16 heads, K = V = 128 (256 workgroups a sweep) 220 | 208 us, 2 x 4096 142 | 107, 2184 tokens 77 | 45;
+// 11 packed sequences, 32768 tokens 428 | 397; 9000 tokens, 3 heads, K = 256, V = 512 467 | 289.  Slower only where one launch takes
+// forward workgroups their place, see launch_sweeps, and by 3 % at 2 x 2048 tokens, 32 heads, V = 256 (196 | 202; the gap between
+// two launches is not in these figures).
+template <int K>
+__global__ __launch_bounds__(SWEEP_WAVES* WAVE) void chunk_sweeps_kernel(const SweepParams fwd, const SweepParams rev, unsigned groups, unsigned first) {
+    constexpr int LDS = Sweep<K, true>::LDS_BYTES > Sweep<K, false>::LDS_BYTES ? Sweep<K, true>::LDS_BYTES : Sweep<K, false>::LDS_BYTES;
+    __shared__ __attribute__((aligned(16))) uint8_t lds[LDS];
+    const unsigned id = blockIdx.x + first;
+    if (id < groups) Sweep<K, true>::run(rev, id, lds);
+    else Sweep<K, false>::run(fwd, id - groups, lds);
+}
+
+template <int K, bool REV>
+__global__ __launch_bounds__(SWEEP_WAVES* WAVE) void chunk_sweep_kernel(const SweepParams p) {
+    __shared__ __attribute__((aligned(16))) uint8_t lds[Sweep<K, REV>::LDS_BYTES];
+    Sweep<K, REV>::run(p, blockIdx.x, lds);
+}
+
 template <int K>
 int launch_sweeps(const SweepParams& fwd, const SweepParams& rev, hipStream_t stream) {
     const int64_t chains8 = ((int64_t)fwd.N * fwd.H + 7) / 8 * 8;
-    const dim3 grid((unsigned)(chains8 * (fwd.V / 32))), block(SWEEP_WAVES * WAVE);
-    hipLaunchKernelGGL((chunk_sweep_kernel<K, false>), grid, block, 0, stream, fwd);
-    if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL((chunk_sweep_kernel<K, true>), grid, block, 0, stream, rev);
-    return (int)hipGetLastError();
+    const unsigned groups = (unsigned)(chains8 * (fwd.V / 32));
+    const dim3 block(SWEEP_WAVES * WAVE);
+    if constexpr (K == 64) {
+        // Here two forward workgroups fit a compute unit (59 KB of LDS) and only one of both sweeps' (90 KB).  64 x 1024 tokens, 4
+        // heads, two launches | one: 82 | 89 us; a packed batch, of uneven chains, gains all the same (30000 tokens, 16 heads 178 | 153).
+        if (fwd.cu_seqlens == nullptr && groups > (unsigned)compute_units()) {
+            hipLaunchKernelGGL((chunk_sweep_kernel<K, false>), dim3(groups), block, 0, stream, fwd);
+            if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
+            hipLaunchKernelGGL((chunk_sweep_kernel<K, true>), dim3(groups), block, 0, stream, rev);
+            return (int)hipGetLastError();
+        }
+    }
+    // (a launch holds at most 2^32 - 1 threads)
+    const int launches = (uint64_t)2 * groups * block.x >> 32 ? 2 : 1;
+    for (int i = 0; i < launches; i++) {
+        hipLaunchKernelGGL((chunk_sweeps_kernel<K>), dim3(2 / launches * groups), block, 0, stream, fwd, rev, groups, i * groups);
+        if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
+    }
+    return GDN_OK;
 }
 
 }  // namespace

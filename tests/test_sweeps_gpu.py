@@ -139,6 +139,26 @@ def test_every_run_of_the_backward_gives_the_same_bits(layout, lens, K, V):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K, V, B, T", [(64, 128, 65, 65), (64, 128, 64, 130), (128, 128, 65, 65), (256, 64, 129, 64)])
+def test_sweeps_in_one_launch_give_the_bits_of_smaller_batches(K, V, B, T):
+    """One launch or two (K = 64, more workgroups than compute units), side by side or one after the other."""
+    from lm_engine_amd import ops
+
+    gen = torch.Generator().manual_seed(B + T)
+    q, k, v, do = (torch.randn(B, T, 1, n, generator=gen).bfloat16().cuda() for n in (K, K, V, V))
+    g, beta = torch.nn.functional.logsigmoid(3 + torch.randn(B, T, 1, generator=gen)).cuda(), torch.rand(B, T, 1, generator=gen).bfloat16().cuda()
+    h0, dht = (0.1 * torch.randn(B, 1, K, V, generator=gen).cuda() for _ in range(2))
+    print(f"case: sweeps of {B} x {T} tokens, K={K} V={V}", flush=True)
+
+    def sweeps(rows):
+        return ops.chunk_bwd_sweeps(*(x[rows] for x in (q, k, v, do, g, beta)), K**-0.5, True, h0[rows], None, False, dht[rows], (T + 63) // 64)[1:]
+
+    whole, parts = sweeps(slice(0, B)), [sweeps(slice(b, b + 1)) for b in range(B)]
+    for i, (name, x) in enumerate(zip(("S0", "V~", "dS1", "Y", "dh0"), whole)):
+        assert torch.equal(x, torch.cat([p[i] for p in parts])), name
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("layout, lens, bad", [("packed", [100, 64, 0, 1, 133, 70], 1), ("packed", [100, 64, 0, 1, 133, 70], 4), ("padded", [200, 70, 1, 129], 1)])
 @pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (256, 512)])
 def test_nan_stays_in_its_sequence(layout, lens, bad, K, V):
