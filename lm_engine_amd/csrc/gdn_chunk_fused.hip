@@ -665,7 +665,7 @@ __global__ __launch_bounds__(PAIR_THREADS) void chunk_fused_kernel(const ChunkPa
     const uint32_t rounds = (items + step - 1) / step;
     const uint32_t group = threadIdx.x / PREP_THREADS;
     if (group >= (uint32_t)FUSED_GROUPS) return;
-    chunk_prepare32_body<K, FUSED_GROUPS, true, false>(p, lds, item_of, items, (uint32_t)rank * FUSED_GROUPS + group, step, rounds, p.ready, 1, SweepScalars{});
+    chunk_prepare32_body<K, FUSED_GROUPS, true, false, FindInRows>(p, lds, item_of, items, (uint32_t)rank * FUSED_GROUPS + group, step, rounds, p.ready, 1, SweepScalars{});
 }
 
 __global__ void fill_zero_kernel(int32_t* x, int64_t n) {

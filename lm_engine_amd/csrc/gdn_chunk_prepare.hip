@@ -10,7 +10,7 @@ namespace gdn {
 // persistent workgroups of four waves, three per CU
 // ------------------------------------------------------------------------------------------
 // SWEEP: the records of the backward's sweeps, and gamma, beta and the inverse norms per token (sw)
-template <int K, bool SWEEP>
+template <int K, bool SWEEP, typename Find>
 __global__ __launch_bounds__(PREP_THREADS, (K > 128 ? 1 : 3)) void chunk_prepare32_kernel(const ChunkParams p, const SweepScalars sw) {
     __shared__ __attribute__((aligned(16))) uint8_t lds[prepare32_lds_bytes<K>()];
     // Work items: (chunk slot, head), the slots rounded up to a multiple of 8.  Workgroup i runs on XCD i % 8 and
@@ -27,7 +27,7 @@ __global__ __launch_bounds__(PREP_THREADS, (K > 128 ? 1 : 3)) void chunk_prepare
         slot = (int)(jh * 8u + w % 8u);
     };
     const uint32_t rounds = (items - blockIdx.x + gridDim.x - 1) / gridDim.x;
-    chunk_prepare32_body<K, 1, false, SWEEP>(p, lds, item_of, items, blockIdx.x, gridDim.x, rounds, nullptr, 0, sw);
+    chunk_prepare32_body<K, 1, false, SWEEP, Find>(p, lds, item_of, items, blockIdx.x, gridDim.x, rounds, nullptr, 0, sw);
 }
 
 // workgroups of the prepare kernel: three per CU (LDS and registers allow it), a multiple of 8, see the kernel
@@ -37,27 +37,26 @@ static int prepare_grid(const ChunkParams& p, int num_cus) {
     return items >= ((int64_t)1 << 31) ? 0 : (int)(items < cap ? items : cap);  // (the kernel counts items in 32 bits)
 }
 
-int launch_prepare32(const ChunkParams& p, int K, hipStream_t stream, int num_cus) {
+template <bool SWEEP, typename Find>
+static int launch_prepare(const ChunkParams& p, const SweepScalars& sw, int K, hipStream_t stream, int num_cus) {
     const int grid = prepare_grid(p, num_cus);
     if (grid == 0) return GDN_ERR_UNSUPPORTED;
-    const SweepScalars none = {};
-    if (K == 64) hipLaunchKernelGGL((chunk_prepare32_kernel<64, false>), dim3(grid), dim3(PREP_THREADS), 0, stream, p, none);
-    else if (K == 128) hipLaunchKernelGGL((chunk_prepare32_kernel<128, false>), dim3(grid), dim3(PREP_THREADS), 0, stream, p, none);
-    else if (K == 256) hipLaunchKernelGGL((chunk_prepare32_kernel<256, false>), dim3(grid), dim3(PREP_THREADS), 0, stream, p, none);
+    if (K == 64) hipLaunchKernelGGL((chunk_prepare32_kernel<64, SWEEP, Find>), dim3(grid), dim3(PREP_THREADS), 0, stream, p, sw);
+    else if (K == 128) hipLaunchKernelGGL((chunk_prepare32_kernel<128, SWEEP, Find>), dim3(grid), dim3(PREP_THREADS), 0, stream, p, sw);
+    else if (K == 256) hipLaunchKernelGGL((chunk_prepare32_kernel<256, SWEEP, Find>), dim3(grid), dim3(PREP_THREADS), 0, stream, p, sw);
     else return GDN_ERR_UNSUPPORTED;
     return (int)hipGetLastError();
 }
 
+int launch_prepare32(const ChunkParams& p, int K, hipStream_t stream, int num_cus) {
+    const SweepScalars none = {};
+    return p.cu_seqlens != nullptr ? launch_prepare<false, FindPacked>(p, none, K, stream, num_cus) : launch_prepare<false, FindInRows>(p, none, K, stream, num_cus);
+}
+
 // the prepare step of the backward's sweeps
 int launch_prepare_sweeps(ChunkParams& p, const SweepScalars& sw, int K, hipStream_t stream, int num_cus) {
-    const int grid = prepare_grid(p, num_cus);
-    if (grid == 0) return GDN_ERR_UNSUPPORTED;
     p.rec16 = 1;
-    if (K == 64) hipLaunchKernelGGL((chunk_prepare32_kernel<64, true>), dim3(grid), dim3(PREP_THREADS), 0, stream, p, sw);
-    else if (K == 128) hipLaunchKernelGGL((chunk_prepare32_kernel<128, true>), dim3(grid), dim3(PREP_THREADS), 0, stream, p, sw);
-    else if (K == 256) hipLaunchKernelGGL((chunk_prepare32_kernel<256, true>), dim3(grid), dim3(PREP_THREADS), 0, stream, p, sw);
-    else return GDN_ERR_UNSUPPORTED;
-    return (int)hipGetLastError();
+    return p.cu_seqlens != nullptr ? launch_prepare<true, FindPacked>(p, sw, K, stream, num_cus) : launch_prepare<true, FindInRows>(p, sw, K, stream, num_cus);
 }
 
 }  // namespace gdn

@@ -77,9 +77,10 @@ constexpr int prepare32_lds_bytes() {
 //                    of the workgroup (a group whose item index runs past `items` only keeps the barriers company)
 //   FLAGS, ready     ready[h * TC + slot] is set to `epoch` once the record is complete and visible to the whole
 //                    device (the scan of the same launch waits for it)
+//   Find             names the chunk of a slot: FindInRows or FindPacked
 //   SWEEP, sw        the records are those of the backward's sweeps (gdn_chunk_sweep.h), and gamma, beta and the inverse norms
 //                    go out per token as well
-template <int K, int GROUPS, bool FLAGS, bool SWEEP, typename ItemOf>
+template <int K, int GROUPS, bool FLAGS, bool SWEEP, typename Find, typename ItemOf>
 __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8_t* lds_base, ItemOf item_of, uint32_t items,
                                                      uint32_t first, uint32_t step, uint32_t rounds, int32_t* ready, int32_t epoch,
                                                      const SweepScalars& sw) {
@@ -121,10 +122,11 @@ __device__ __forceinline__ void chunk_prepare32_body(const ChunkParams& p, uint8
     uint32_t bx_raw = 0;  // beta of the prefetched item, raw bits: any arithmetic on it here would wait for every load in flight
     ChunkCoord ncc;  // coordinates of the prefetched item
     int nh = 0, nslot = 0;
+    const Find find_chunk(p, tid % WAVE);
     auto locate = [&](uint32_t w) {  // wave-uniform 32-bit arithmetic
         if (w < items) {
             item_of(w, nh, nslot);
-            ncc = locate_chunk(p, nslot);
+            ncc = find_chunk(p, nslot);
         } else {
             nh = 0, nslot = 0, ncc.n = 0, ncc.c = 0, ncc.b = 0, ncc.t0 = 0, ncc.len = 0;
         }

@@ -157,6 +157,19 @@ def test_varlen_many_sequences_start_longest_first(count, H, V):
     _check(dict(inp, cu_seqlens=cu), f"varlen, {count} sequences")
 
 
+@pytest.mark.parametrize("count", [1, 2, 63, 64, 65])
+def test_varlen_chunks_are_found_for_any_number_of_sequences(count):
+    # the prepare step holds up to 63 prefixes in registers and searches more: empty sequences at the ends and in a row, cut chunks
+    gen = torch.Generator().manual_seed(count)
+    lengths = torch.randint(0, 200, (count,), generator=gen)
+    lengths[torch.rand(count, generator=gen) < 0.3] = 0
+    lengths[count // 2] = 129
+    inp = random_inputs(B=1, T=int(lengths.sum()), H=2, K=64, V=64, dtype=BF16, seed=79, N=count)
+    cu = torch.nn.functional.pad(lengths.cumsum(0), (1, 0)).to(torch.int32)
+    _, ht = _check(dict(inp, cu_seqlens=cu), f"varlen, {count} sequences")
+    assert torch.equal(ht[lengths == 0].cpu(), inp["initial_state"][lengths == 0])
+
+
 @pytest.mark.parametrize("K, V", [(128, 128), (64, 64), (256, 128)])
 def test_varlen_with_an_empty_sequence(K, V):
     # a sequence of length 0 has no chunk: its final state is its initial state, and its neighbours are untouched
