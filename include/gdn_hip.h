@@ -300,10 +300,11 @@ int gdn_chunk_fwd_saving_is_staged(const gdn_args *args, const gdn_chunk_saves *
  * K = 64, 128 or 256 and V a multiple of 64 (GDN_ERR_UNSUPPORTED otherwise).  Counterpart upstream: the chunk-local
  * kernels of fla's backward of chunk_gated_delta_rule, reached from gated_deltanet/module.py:197-209 under autograd.
  */
+#define GDN_LOCAL_DBETA_BF16 0x100 /* in saves_dtype: dbeta_out is bf16 */
 typedef struct gdn_chunk_local_args {
     const void *v_new, *states, *dstates;
     const float *gamma, *beta, *rq, *rk;
-    int32_t saves_dtype; /* gdn_dtype of v_new and states */
+    int32_t saves_dtype; /* gdn_dtype of v_new and states, | GDN_LOCAL_DBETA_BF16 */
     float scale;
     int64_t chunks;
     int32_t K, V;
@@ -318,7 +319,8 @@ typedef struct gdn_chunk_local_args {
     int64_t dout_stride_b, dout_stride_t, dout_stride_h;
     /* packed or left-padded batches: sequence n starts at token seq_start[n] (a flat index over the
      * rows of the caller's tensors, T_rows tokens per row) and has seq_len[n] tokens; its chunks c * 64 >= seq_len[n]
-     * are skipped, tokens past its end are not written.  NULL: sequence n is row n, NC * 64 tokens. */
+     * are skipped, tokens past its end are not written.  NULL: sequence n is row n, of T_rows tokens where
+     * (NC - 1) * 64 < T_rows < NC * 64, else of NC * 64. */
     const int32_t *seq_start, *seq_len;
     int32_t T_rows;
     int32_t dstates_dtype; /* gdn_dtype of dstates */

@@ -45,7 +45,9 @@ import weakref
 
 import torch
 
+from . import _lib
 from ._autograd import kernel_rows
+from ._host import host, raw_stream
 
 
 CHUNK = 64
@@ -346,13 +348,21 @@ def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm
 
     B, T = q.shape[:2]
     covers = True  # every token belongs to a sequence
-    if cu_seqlens is None and T % CHUNK == 0:
-        NC, sequences = T // CHUNK, None
-    else:
+    sequences = None
+    if cu_seqlens is not None:
         starts, lens = _chains(B, T, cu_seqlens, left_padded)
         NC = max(1, -(-max(lens + [1]) // CHUNK))
         covers = sum(lens) == B * T
         sequences = (*ops.upload_int32((starts, lens), q.device), NC)
+    flags = (_lib.GDN_FLAG_L2NORM if l2norm else 0) | (_lib.GDN_FLAG_LEFT_PADDED if left_padded else 0)
+    grads = host().delta_rule_bwd(raw_stream(q.get_device()), q, k, v, g, beta, initial_state, cu_seqlens, do, dht, scale, flags,
+                                  *(sequences or (None, None, 0)), covers, joined)  # fmt: skip
+    if grads is not None:
+        return grads
+    if cu_seqlens is None:
+        NC = -(-T // CHUNK)
+        if T % CHUNK != 0:
+            sequences = (*ops.upload_int32(_chains(B, T, None, False), q.device), NC)
     q, k, v = (x if x.stride(-1) == 1 else x.contiguous() for x in (q, k, v))
     do = kernel_rows(do.to(torch.bfloat16))
     if do.stride(1) > 1 << 24:  # the kernels count a chunk's rows in 32 bits; q, k and v were held to that by the forward

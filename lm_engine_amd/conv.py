@@ -120,8 +120,13 @@ class _ConvolutionOnKernels(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, weight, bias, input_state, attention_mask, output_state, activation):
-        y, final_state = _depthwise_causal_convolution(x, weight, bias, input_state, attention_mask, output_state,
-                                                       activation)  # fmt: skip
+        result = None
+        if is_kernel_allowed(Kernel.gated_delta_rule):
+            result = host().conv(raw_stream(x.get_device()), x, weight, bias, input_state, attention_mask, output_state,
+                                 _IN_KERNEL_ACTIVATIONS[activation])  # fmt: skip
+        if result is None:
+            result = _depthwise_causal_convolution(x, weight, bias, input_state, attention_mask, output_state, activation)
+        y, final_state = result
         ctx.save_for_backward(x, weight, bias, input_state, attention_mask)
         ctx.activation = activation
         ctx.set_materialize_grads(False)
@@ -152,8 +157,13 @@ class _ConvolutionOnKernels(torch.autograd.Function):
 
 def _convolution_backward(x, weight, bias, input_state, attention_mask, dy, activation):
     """``gdn_causal_conv1d_bwd``: dx, dweight, dbias, dinput_state for bf16 or fp32 x (see include/gdn_hip.h)."""
-    lib = _lib.load_library()
     B, S, C = x.shape
+    if input_state is None:
+        grads = host().conv_bwd(raw_stream(x.get_device()), x, weight, bias, attention_mask, dy, _IN_KERNEL_ACTIVATIONS[activation],
+                                _backward_tokens_per_block(B, S, C))  # fmt: skip
+        if grads is not None:
+            return (*grads, None)
+    lib = _lib.load_library()
     w2 = (weight.squeeze(1) if weight.dim() == 3 else weight).contiguous()
     ks = w2.size(1)
     if x.stride(-1) != 1:

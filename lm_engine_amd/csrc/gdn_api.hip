@@ -232,9 +232,10 @@ int gdn_chunk_bwd_local(const gdn_chunk_local_args* a, void* stream) {
     for (const void* x : needed)
         if (x == nullptr) return GDN_ERR_NULL;
         else if (!aligned(x, 16)) return GDN_ERR_ALIGN;
-    if (a->saves_dtype != GDN_BF16 && a->saves_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
+    const int saves_dtype = a->saves_dtype & ~GDN_LOCAL_DBETA_BF16;
+    if (saves_dtype != GDN_BF16 && saves_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
     if (a->dstates_dtype != GDN_BF16 && a->dstates_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
-    if (a->saves_sliced && (a->saves_dtype != GDN_BF16 || a->dstates_dtype != GDN_BF16 || a->y_chunks == nullptr)) return GDN_ERR_UNSUPPORTED;
+    if (a->saves_sliced && (saves_dtype != GDN_BF16 || a->dstates_dtype != GDN_BF16 || a->y_chunks == nullptr)) return GDN_ERR_UNSUPPORTED;
     if (a->out_stride_t != 0 && (a->out_stride_t < (int64_t)a->H * a->K || a->out_stride_t < (int64_t)a->H * a->V)) return GDN_ERR_SHAPE;
     if (a->out_stride_t % 8 != 0) return GDN_ERR_ALIGN;
     if (a->H <= 0 || a->NC <= 0 || a->chunks % ((int64_t)a->H * a->NC) != 0) return GDN_ERR_SHAPE;

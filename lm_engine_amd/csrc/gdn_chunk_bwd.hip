@@ -78,6 +78,7 @@ struct ChunkLocalParams {
     bf16_t* dv_out;
     float* dg_out;
     float* dbeta_out;
+    int dbeta_bf16;
     int64_t dqk_stride_t, dv_stride_t;  // elements between the tokens of dq_out and dk_out, and of dv_out
     int H, NC, V;
     // sequences that are not whole rows of whole chunks (packed or left-padded batches): first token (flat index
@@ -232,6 +233,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
         valid = min(max(p.seq_len[n] - ci * C, 0), C);
         tok0 = (int64_t)p.seq_start[n] + (int64_t)ci * C;
     } else {
+        valid = min(C, p.T_rows - ci * C);
         tok0 = (int64_t)n * p.T_rows + (int64_t)ci * C;
     }
     if (valid == 0) return;  // a chunk past the end of its sequence (whole workgroup)
@@ -782,7 +784,9 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
         }
         if (t < valid) {
             p.dg_out[(tok0 + t) * p.H + h] = dg;
-            p.dbeta_out[(tok0 + t) * p.H + h] = dbeta;
+            const int64_t at = (tok0 + t) * p.H + h;
+            if (p.dbeta_bf16) reinterpret_cast<bf16_t*>(p.dbeta_out)[at] = (bf16_t)dbeta;
+            else p.dbeta_out[at] = dbeta;
         }
     }
 #ifdef GDN_CYCLE_BUDGET
@@ -1279,7 +1283,8 @@ int launch_chunk_bwd_local(const gdn_chunk_local_args& a, hipStream_t stream) {
     p.cycle_out = cycle_buffer();
     if (p.cycle_out != nullptr) (void)hipMemsetAsync(p.cycle_out, 0, GDN_LOCAL_CYCLE_SLOTS * 16 * sizeof(uint64_t), stream);
 #endif
-    p.vnew = a.v_new, p.s0 = a.states, p.ds1 = a.dstates, p.saves_bf16 = a.saves_dtype == GDN_BF16 ? 1 : 0;
+    p.vnew = a.v_new, p.s0 = a.states, p.ds1 = a.dstates, p.saves_bf16 = (a.saves_dtype & ~GDN_LOCAL_DBETA_BF16) == GDN_BF16 ? 1 : 0;
+    p.dbeta_bf16 = (a.saves_dtype & GDN_LOCAL_DBETA_BF16) != 0 ? 1 : 0;
     const bool h = a.dstates_dtype == GDN_BF16;
     const bool sl = a.saves_sliced != 0;
     p.gam = a.gamma, p.beta = a.beta;
@@ -1296,7 +1301,8 @@ int launch_chunk_bwd_local(const gdn_chunk_local_args& a, hipStream_t stream) {
     p.k_stride_b = a.k_stride_b, p.k_stride_t = a.k_stride_t, p.k_stride_h = a.k_stride_h;
     p.v_stride_b = a.v_stride_b, p.v_stride_t = a.v_stride_t, p.v_stride_h = a.v_stride_h;
     p.d_stride_b = a.dout_stride_b, p.d_stride_t = a.dout_stride_t, p.d_stride_h = a.dout_stride_h;
-    p.seq_start = a.seq_start, p.seq_len = a.seq_len, p.T_rows = a.seq_start != nullptr ? a.T_rows : a.NC * C;
+    p.seq_start = a.seq_start, p.seq_len = a.seq_len;
+    p.T_rows = a.seq_start != nullptr || (a.T_rows > (a.NC - 1) * C && a.T_rows < a.NC * C) ? a.T_rows : a.NC * C;
     const dim3 grid((unsigned)a.chunks), block(BWD_THREADS);
     auto launch = [&](auto kc) {
         constexpr int KK = decltype(kc)::value;

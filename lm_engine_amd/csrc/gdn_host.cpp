@@ -1,8 +1,8 @@
-// The host path of the inference entry points: from torch tensors to one call of the C ABI (include/gdn_hip.h).
+// The host path of the entry points and of their backward passes: from torch tensors to the calls of the C ABI (include/gdn_hip.h).
 //
-// On a decode step or a short prompt the GPU needs a few microseconds per kernel, and reading shapes, strides and
-// pointers out of tensors, allocating the results and filling the argument struct takes 10 to 20 in Python per call.  Here
-// it takes 1 to 4.  Every function is a fast path only: it takes well-formed operands that need no conversion and no
+// On a decode step, a short prompt or a short training sequence the GPU needs a few microseconds per kernel, and reading shapes,
+// strides and pointers out of tensors, allocating the results and filling the argument structs takes 10 to 60 in Python per call.
+// Here it takes 1 to 6.  Every function is a fast path only: it takes well-formed operands that need no conversion and no
 // gradient, and returns None for everything else, so that the Python code behind it converts, differentiates or reports.
 // The library itself stays independent of torch: its entry points come in as addresses (bind), from the one loaded copy.
 
@@ -14,6 +14,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/utils/object_ptr.h>
 
+#include <algorithm>
 #include <cmath>
 #include <initializer_list>
 
@@ -30,12 +31,21 @@ decltype(&gdn_recurrent_fwd) recurrent_fn = nullptr;
 decltype(&gdn_chunk_fwd) chunk_fn = nullptr;
 decltype(&gdn_workspace_bytes) workspace_bytes_fn = nullptr;
 decltype(&gdn_chunk_fwd_is_one_launch) one_launch_fn = nullptr;
+decltype(&gdn_chunk_bwd_sweeps) sweeps_fn = nullptr;
+decltype(&gdn_chunk_bwd_sweeps_workspace_bytes) sweeps_workspace_fn = nullptr;
+decltype(&gdn_chunk_bwd_local) local_fn = nullptr;
+decltype(&gdn_causal_conv1d_bwd) conv_bwd_fn = nullptr;
+decltype(&gdn_gates_bwd) gates_bwd_fn = nullptr;
+decltype(&gdn_gated_rmsnorm_bwd) norm_bwd_fn = nullptr;
+decltype(&gdn_column_sums) column_sums_fn = nullptr;
 PyObject* check_status = nullptr;  // _lib.check_status: raises what a status stands for
 
 // bind(check_status, addresses...)
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
     void** slots[] = {(void**)&layer_step_fn, (void**)&layer_step_tiles_fn, (void**)&conv_fn, (void**)&gates_fn, (void**)&norm_fn,
-                      (void**)&recurrent_fn, (void**)&chunk_fn, (void**)&workspace_bytes_fn, (void**)&one_launch_fn};
+                      (void**)&recurrent_fn, (void**)&chunk_fn, (void**)&workspace_bytes_fn, (void**)&one_launch_fn,
+                      (void**)&sweeps_fn, (void**)&sweeps_workspace_fn, (void**)&local_fn, (void**)&conv_bwd_fn, (void**)&gates_bwd_fn,
+                      (void**)&norm_bwd_fn, (void**)&column_sums_fn};
     constexpr Py_ssize_t count = sizeof(slots) / sizeof(slots[0]);
     if (n != count + 1) return PyErr_Format(PyExc_TypeError, "bind takes a function and %zd addresses, got %zd arguments", count, n);
     for (Py_ssize_t i = 0; i < count; i++) {
@@ -295,6 +305,24 @@ PyObject* gates(PyObject*, PyObject* const* args, Py_ssize_t n) {
     });
 }
 
+// o and gate of the gated norm, forward and backward: (heads, columns, elements between the gate's tokens)
+struct NormOperands {
+    int64_t H, V, gate_stride = 0;
+    NormOperands(const at::Tensor& o, const at::Tensor* gate) {
+        need(o.dim() >= 2 && o.is_contiguous() && o.numel() > 0);
+        H = o.size(-2), V = o.size(-1);
+        need(V % 8 == 0 && V <= 512);
+        if (gate == nullptr) return;
+        need(gate->scalar_type() == o.scalar_type() && gate->numel() == o.numel() && gate->dim() >= 2);
+        if (gate->size(-1) == H * V && gate->dim() == o.dim() - 1) {
+            gate_stride = row_stride(*gate, H * V);
+        } else {
+            need(gate->sizes() == o.sizes() && gate->is_contiguous());
+            gate_stride = H * V;
+        }
+    }
+};
+
 // norm(stream, o, gate, weight, eps) -> y
 PyObject* norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return fast_path(n, 5, [&]() -> PyObject* {
@@ -304,19 +332,9 @@ PyObject* norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const at::Tensor *gate = operand.optional(args[2]), *weight = operand.optional(args[3]);
         gdn_norm_args s{};
         s.dtype = code_of(o);
-        need(o.dim() >= 2 && o.is_contiguous() && o.numel() > 0);
-        const int64_t H = o.size(-2), V = o.size(-1);
-        need(V % 8 == 0 && V <= 512);
-        s.tokens = o.numel() / (H * V);
-        if (gate != nullptr) {
-            need(gate->scalar_type() == o.scalar_type() && gate->numel() == o.numel() && gate->dim() >= 2);
-            if (gate->size(-1) == H * V && gate->dim() == o.dim() - 1) {
-                s.gate_stride_t = row_stride(*gate, H * V);
-            } else {
-                need(gate->sizes() == o.sizes() && gate->is_contiguous());
-                s.gate_stride_t = H * V;
-            }
-        }
+        const NormOperands x(o, gate);
+        const int64_t H = x.H, V = x.V;
+        s.tokens = o.numel() / (H * V), s.gate_stride_t = x.gate_stride;
         s.w_dtype = GDN_F32;
         if (weight != nullptr) {
             s.w_dtype = code_of(*weight);
@@ -393,6 +411,247 @@ PyObject* delta_rule(PyObject*, PyObject* const* args, Py_ssize_t n) {
     });
 }
 
+// ---- backward passes.  Like the forward: what needs a conversion or a copy, and what is itself differentiated, is not here. ----
+
+// the sums over the first dim of one or two partial arrays, in the dtypes of the parameters they are the gradients of
+struct ColumnSums {
+    gdn_column_sums_args s{};
+    void add(const at::Tensor& partial, const at::Tensor& out) {
+        const int j = s.arrays++;
+        s.partial[j] = static_cast<const float*>(ptr(partial)), s.out[j] = ptr(out), s.cols[j] = out.numel(), s.out_dtype[j] = code_of(out);
+        s.rows = (int32_t)partial.size(0);
+    }
+};
+
+// a gradient that a kernel reads as it lies: what kernel_rows (_autograd.py) would not copy
+void need_rows(const at::Tensor& t, int64_t stride_elements, size_t address_bytes) {
+    need(t.stride(-1) == 1 && aligned(ptr(t), address_bytes));
+    for (int64_t i = 0; i + 1 < t.dim(); i++) need(t.stride(i) % stride_elements == 0);
+}
+
+// delta_rule_bwd(stream, q, k, v, g, beta, initial_state, cu_seqlens, do, dht, scale, flags, seq_start, seq_len, NC, covers, joined)
+//   -> (dq, dk, dv, dg, dbeta, dh0)
+// Rows of a batch: without seq_start and seq_len.  Else NC chunks for the longest sequence; covers: every token belongs to one.
+// joined: dq, dk and dv as column blocks of one tensor.
+PyObject* delta_rule_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    return fast_path(n, 17, [&]() -> PyObject* {
+        Operands operand;
+        void* const stream = stream_of(args[0]);
+        const at::Tensor &q = operand(args[1]), &k = operand(args[2]), &v = operand(args[3]), &d = operand(args[8]);
+        const at::Tensor *g = operand.optional(args[4]), *beta = operand.optional(args[5]), *h0 = operand.optional(args[6]), *cu = operand.optional(args[7]);
+        const at::Tensor *dht = operand.optional(args[9]), *seq_start = operand.optional(args[12]), *seq_len = operand.optional(args[13]);
+        const bool covers = truth(args[15]), joined = truth(args[16]);
+        gdn_args s{};
+        gdn_chunk_local_args l{};
+        s.dtype = code_of(q), s.flags = (int32_t)integer(args[11]);
+        const bool padded = (s.flags & GDN_FLAG_LEFT_PADDED) != 0;
+        need(s.dtype == GDN_BF16 && q.dim() == 4 && k.sizes() == q.sizes() && v.dim() == 4 && k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type());
+        const int64_t B = q.size(0), T = q.size(1), H = q.size(2), K = q.size(3), V = v.size(3);
+        need(v.size(0) == B && v.size(1) == T && v.size(2) == H && B > 0 && T > 0 && H > 0 && q.stride(3) == 1 && k.stride(3) == 1 && v.stride(3) == 1);
+        need((K == 64 || K == 128 || K == 256) && V % 64 == 0);
+        need(d.scalar_type() == at::kBFloat16 && d.sizes() == v.sizes() && d.stride(1) <= (int64_t)1 << 24);
+        need_rows(d, 8, 16);
+        int64_t N = B, NC = (T + 63) / 64;
+        need((cu == nullptr) == (seq_start == nullptr) && (cu == nullptr) == (seq_len == nullptr));
+        if (cu != nullptr) {
+            need(cu->scalar_type() == at::kInt && cu->dim() == 1 && cu->is_contiguous() && cu->numel() >= 2);
+            if (padded) need(cu->numel() == B + 1);
+            else need(B == 1), N = cu->numel() - 1;
+            NC = integer(args[14]);
+            const at::Tensor* places[] = {seq_start, seq_len};
+            for (const at::Tensor* t : places) need(t->scalar_type() == at::kInt && t->dim() == 1 && t->numel() == N && t->is_contiguous());
+            l.seq_start = static_cast<const int32_t*>(ptr(seq_start)), l.seq_len = static_cast<const int32_t*>(ptr(seq_len));
+        } else {
+            need(!padded);
+        }
+        need(NC > 0);
+        l.T_rows = size32(T);
+        if (g != nullptr) need(g->scalar_type() == at::kFloat && g->sizes() == at::IntArrayRef({B, T, H}) && g->is_contiguous());
+        s.beta_dtype = GDN_F32;
+        if (beta != nullptr) {
+            s.beta_dtype = code_of(*beta);
+            need(beta->sizes() == at::IntArrayRef({B, T, H}) && beta->is_contiguous());
+        }
+        const at::Tensor* states[] = {h0, dht};
+        for (const at::Tensor* t : states)
+            if (t != nullptr) need(t->scalar_type() == at::kFloat && t->sizes() == at::IntArrayRef({N, H, K, V}) && t->is_contiguous() && aligned(ptr(t), 16));
+        s.B = size32(B), s.T = size32(T), s.H = size32(H), s.K = (int32_t)K, s.V = size32(V), s.N = size32(N), s.chunk = 64;
+        s.cu_seqlens = static_cast<const int32_t*>(ptr(cu));
+        s.scale = (float)number(args[10]);
+        s.q = ptr(q), s.k = ptr(k), s.v = ptr(v), s.o = ptr(v), s.beta = ptr(beta);  // (no output is written)
+        s.g = static_cast<const float*>(ptr(g)), s.h0 = static_cast<const float*>(ptr(h0));
+        s.q_stride_b = l.q_stride_b = q.stride(0), s.q_stride_t = l.q_stride_t = q.stride(1), s.q_stride_h = l.q_stride_h = q.stride(2);
+        s.k_stride_b = l.k_stride_b = k.stride(0), s.k_stride_t = l.k_stride_t = k.stride(1), s.k_stride_h = l.k_stride_h = k.stride(2);
+        s.v_stride_b = l.v_stride_b = v.stride(0), s.v_stride_t = l.v_stride_t = v.stride(1), s.v_stride_h = l.v_stride_h = v.stride(2);
+        s.o_stride_b = s.v_stride_b, s.o_stride_t = s.v_stride_t, s.o_stride_h = s.v_stride_h;
+        s.workspace_bytes = sweeps_workspace_fn(&s);
+        need(s.workspace_bytes > 0);
+
+        at::Tensor workspace, scalars, S0, dS1, Vn, Y, dq, dk, dv, dg, dbeta, dh0;
+        without_interpreter_lock([&] {
+            scalars = fresh_f32(q, {4, N * H, NC, 64});
+            S0 = fresh(q, {N * H, NC, K, V}), dS1 = fresh(q, {N * H, NC, K, V}), Vn = fresh(q, {N * H, NC, 64, V}), Y = fresh(q, {N * H, NC, 64, V});
+            if (h0 != nullptr) dh0 = fresh_f32(q, {N, H, K, V});
+            workspace = at::empty({(int64_t)s.workspace_bytes}, q.options().dtype(at::kByte));
+        });
+        s.workspace = ptr(workspace);
+        float* const f = static_cast<float*>(ptr(scalars));
+        const int64_t each = N * H * NC * 64;
+        l.gamma = f, l.beta = f + each, l.rq = f + 2 * each, l.rk = f + 3 * each;
+        l.states = ptr(S0), l.dstates = ptr(dS1), l.v_new = ptr(Vn), l.y_chunks = ptr(Y);
+        l.saves_dtype = l.dstates_dtype = GDN_BF16, l.saves_sliced = 1;
+        l.chunks = N * H * NC, l.K = (int32_t)K, l.V = (int32_t)V, l.H = (int32_t)H, l.NC = size32(NC), l.scale = s.scale;
+        l.q_raw = s.q, l.k_raw = s.k, l.v_raw = s.v, l.dout_raw = ptr(d);
+        l.dout_stride_b = d.stride(0), l.dout_stride_t = d.stride(1), l.dout_stride_h = d.stride(2);
+        const int status = without_interpreter_lock([&] {
+            return sweeps_fn(&s, &l, static_cast<const float*>(ptr(dht)), dh0.defined() ? static_cast<float*>(ptr(dh0)) : nullptr, stream);
+        });
+        need(status >= 0);
+        if (status != GDN_OK) return PyObject_CallFunction(check_status, "is", status, "gdn_chunk_bwd_sweeps");
+
+        // The results are allocated behind the sweeps' launch, where the workspace can go: they then take its place, in memory and
+        // in the caches (4 x 4096 tokens, 16 heads, K = V = 128: the chunk-local kernel 208 us, 216 beside the workspace).  Should an
+        // allocation fail here, the Python path starts over: nothing so far has changed an operand.
+        without_interpreter_lock([&] {
+            workspace.reset();
+            // tokens outside every sequence are not written
+            auto made = [&](at::IntArrayRef sizes, at::ScalarType dtype) {
+                return covers || cu == nullptr ? at::empty(sizes, q.options().dtype(dtype)) : at::zeros(sizes, q.options().dtype(dtype));
+            };
+            if (joined) {
+                const int64_t row = H * (2 * K + V);
+                const at::Tensor rows = made({B, T, row}, at::kBFloat16);
+                dq = rows.as_strided({B, T, H, K}, {T * row, row, K, 1}, 0);
+                dk = rows.as_strided({B, T, H, K}, {T * row, row, K, 1}, H * K);
+                dv = rows.as_strided({B, T, H, V}, {T * row, row, V, 1}, 2 * H * K);
+                l.out_stride_t = size32(row);
+            } else {
+                dq = made({B, T, H, K}, at::kBFloat16), dk = made({B, T, H, K}, at::kBFloat16), dv = made({B, T, H, V}, at::kBFloat16);
+            }
+            dg = made({B, T, H}, at::kFloat), dbeta = made({B, T, H}, beta == nullptr ? at::kFloat : beta->scalar_type());
+        });
+        l.dq_out = ptr(dq), l.dk_out = ptr(dk), l.dv_out = ptr(dv), l.dg_out = static_cast<float*>(ptr(dg)), l.dbeta_out = static_cast<float*>(ptr(dbeta));
+        if (!(s.flags & GDN_FLAG_L2NORM)) l.rq = l.rk = nullptr;
+        if (dbeta.scalar_type() == at::kBFloat16) l.saves_dtype |= GDN_LOCAL_DBETA_BF16;
+        return launch("gdn_chunk_bwd_local", pack_results({dq, dk, dv, g == nullptr ? at::Tensor() : dg, beta == nullptr ? at::Tensor() : dbeta, dh0}),
+                      [&] { return local_fn(&l, stream); });
+    });
+}
+
+// conv_bwd(stream, x, weight, bias, mask, dy, activation, tokens_per_block) -> (dx, dweight, dbias or None)
+PyObject* conv_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    return fast_path(n, 8, [&]() -> PyObject* {
+        Operands operand;
+        void* const stream = stream_of(args[0]);
+        const at::Tensor &x = operand(args[1]), &weight = operand(args[2]), &dy = operand(args[5]);
+        const at::Tensor *bias = operand.optional(args[3]), *mask = operand.optional(args[4]);
+        gdn_conv_bwd_args s{};
+        s.dtype = code_of(x), s.w_dtype = code_of(weight);
+        need(x.dim() == 3 && x.stride(2) == 1 && dy.scalar_type() == x.scalar_type() && dy.sizes() == x.sizes());
+        need_rows(dy, 2, 8);
+        const int64_t B = x.size(0), S = x.size(1), C = x.size(2), ks = taps_of(weight, C), tokens = integer(args[7]);
+        need(B > 0 && S > 0 && tokens > 0);
+        if (bias != nullptr) need(bias->scalar_type() == weight.scalar_type() && bias->dim() == 1 && bias->size(0) == C && bias->is_contiguous());
+        const int64_t blocks = B * ((S + tokens - 1) / tokens);
+        at::Tensor kept_mask, dx, dw_part, db_part, dweight, dbias;
+        const bool masked = mask != nullptr && mask->dim() == 2 && mask->size(0) > 1 && mask->size(1) > 1;
+        need(mask == nullptr || mask->dim() == 2);
+        if (masked) need(mask->size(0) == B && mask->size(1) == S);
+        without_interpreter_lock([&] {
+            if (masked) kept_mask = mask->to(x.scalar_type()).contiguous(), s.mask = ptr(kept_mask);
+            dx = fresh(x, {B, S, C}), dw_part = fresh_f32(x, {blocks, C, ks}), db_part = fresh_f32(x, {blocks, C});
+            dweight = at::empty(weight.sizes(), weight.options());
+            if (bias != nullptr) dbias = at::empty({C}, bias->options());
+        });
+        s.x = ptr(x), s.dy = ptr(dy), s.weight = ptr(weight), s.bias = ptr(bias), s.dx = ptr(dx);
+        s.dweight_partial = static_cast<float*>(ptr(dw_part)), s.dbias_partial = static_cast<float*>(ptr(db_part));
+        s.x_stride_b = x.stride(0), s.x_stride_s = x.stride(1), s.dy_stride_b = dy.stride(0), s.dy_stride_s = dy.stride(1);
+        s.B = size32(B), s.S = size32(S), s.C = size32(C), s.kernel_size = (int32_t)ks, s.tokens_per_block = size32(tokens);
+        s.activation = (int32_t)integer(args[6]);
+        ColumnSums sums;
+        sums.add(dw_part, dweight);
+        if (dbias.defined()) sums.add(db_part, dbias);
+        return launch("gdn_causal_conv1d_bwd, gdn_column_sums", pack_results({dx, dweight, dbias}), [&] {
+            const int status = conv_bwd_fn(&s, stream);
+            return status == GDN_OK ? column_sums_fn(&sums.s, stream) : status;
+        });
+    });
+}
+
+// gates_bwd(stream, a, b, A_log, dt_bias, dg, dbeta, beta_scale) -> (da, db, dA_log, ddt_bias)
+PyObject* gates_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    return fast_path(n, 8, [&]() -> PyObject* {
+        Operands operand;
+        void* const stream = stream_of(args[0]);
+        const at::Tensor &a = operand(args[1]), &b = operand(args[2]), &A_log = operand(args[3]), &dt_bias = operand(args[4]), &dg = operand(args[5]), &dbeta = operand(args[6]);
+        gdn_gate_bwd_args s{};
+        s.dtype = code_of(a);
+        need(a.dim() >= 2 && b.scalar_type() == a.scalar_type() && b.sizes() == a.sizes() && a.numel() > 0);
+        const int64_t H = a.size(-1);
+        const at::Tensor* decay[] = {&A_log, &dt_bias};
+        for (const at::Tensor* t : decay) need(t->scalar_type() == at::kFloat && t->dim() == 1 && t->size(0) == H && t->is_contiguous());
+        need(dg.scalar_type() == at::kFloat && dg.sizes() == a.sizes() && dg.is_contiguous());
+        need(dbeta.scalar_type() == a.scalar_type() && dbeta.sizes() == a.sizes() && dbeta.is_contiguous());
+        s.a_stride = row_stride(a, H), s.b_stride = row_stride(b, H);
+        s.tokens = a.numel() / H, s.H = size32(H);
+        s.partial_blocks = (int32_t)std::min<int64_t>(1024, (a.numel() + 255) / 256);
+        at::Tensor da, db, dA_part, ddt_part, dA_log, ddt_bias;
+        without_interpreter_lock([&] {
+            da = fresh(a, a.sizes()), db = fresh(a, a.sizes());
+            dA_part = fresh_f32(a, {s.partial_blocks, H}), ddt_part = fresh_f32(a, {s.partial_blocks, H});
+            dA_log = fresh_f32(a, {H}), ddt_bias = fresh_f32(a, {H});
+        });
+        s.a = ptr(a), s.b = ptr(b), s.A_log = static_cast<const float*>(ptr(A_log)), s.dt_bias = static_cast<const float*>(ptr(dt_bias));
+        s.dg = static_cast<const float*>(ptr(dg)), s.dbeta = ptr(dbeta), s.da = ptr(da), s.db = ptr(db);
+        s.dA_log_partial = static_cast<float*>(ptr(dA_part)), s.ddt_bias_partial = static_cast<float*>(ptr(ddt_part));
+        s.beta_scale = (float)number(args[7]);
+        ColumnSums sums;
+        sums.add(dA_part, dA_log), sums.add(ddt_part, ddt_bias);
+        return launch("gdn_gates_bwd, gdn_column_sums", pack_results({da, db, dA_log, ddt_bias}), [&] {
+            const int status = gates_bwd_fn(&s, stream);
+            return status == GDN_OK ? column_sums_fn(&sums.s, stream) : status;
+        });
+    });
+}
+
+// norm_bwd(stream, o, gate, weight, eps, dy) -> (d_o, d_gate or None, d_weight or None)
+PyObject* norm_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    return fast_path(n, 6, [&]() -> PyObject* {
+        Operands operand;
+        void* const stream = stream_of(args[0]);
+        const at::Tensor &o = operand(args[1]), &dy = operand(args[5]);
+        const at::Tensor *gate = operand.optional(args[2]), *weight = operand.optional(args[3]);
+        gdn_norm_bwd_args s{};
+        s.dtype = code_of(o);
+        const NormOperands x(o, gate);
+        need(dy.scalar_type() == o.scalar_type() && dy.sizes() == o.sizes() && dy.is_contiguous());
+        need_rows(dy, 8, 16);
+        s.tokens = o.numel() / (x.H * x.V), s.gate_stride_t = x.gate_stride;
+        s.w_dtype = GDN_F32;
+        if (weight != nullptr) {
+            s.w_dtype = code_of(*weight);
+            need(weight->dim() == 1 && weight->size(0) == x.V && weight->is_contiguous());
+        }
+        s.w_dtype |= GDN_NORM_GATE_DWORDS;
+        s.partial_blocks = (int32_t)std::min<int64_t>(2048, std::max<int64_t>(1, (s.tokens * x.H * std::max<int64_t>(x.V / 8, 8) + 255) / 256));
+        at::Tensor d_o, d_gate, part, d_weight;
+        without_interpreter_lock([&] {
+            d_o = fresh(o, o.sizes()), part = fresh_f32(o, {s.partial_blocks, x.V});
+            if (gate != nullptr) d_gate = fresh(o, gate->sizes());
+            if (weight != nullptr) d_weight = at::empty({x.V}, weight->options());
+        });
+        s.o = ptr(o), s.gate = ptr(gate), s.weight = ptr(weight), s.dy = ptr(dy), s.d_o = ptr(d_o), s.d_gate = d_gate.defined() ? ptr(d_gate) : nullptr;
+        s.dweight_partial = static_cast<float*>(ptr(part));
+        s.o_stride_t = x.H * x.V, s.H = size32(x.H), s.V = (int32_t)x.V, s.eps = (float)number(args[4]);
+        ColumnSums sums;
+        if (d_weight.defined()) sums.add(part, d_weight);
+        return launch("gdn_gated_rmsnorm_bwd, gdn_column_sums", pack_results({d_o, d_gate, d_weight}), [&] {
+            const int status = norm_bwd_fn(&s, stream);
+            return status == GDN_OK && sums.s.arrays > 0 ? column_sums_fn(&sums.s, stream) : status;
+        });
+    });
+}
+
 PyMethodDef methods[] = {
     {"bind", (PyCFunction)(void (*)())bind, METH_FASTCALL, "takes the addresses of the library's entry points"},
     {"layer_step", (PyCFunction)(void (*)())layer_step, METH_FASTCALL, "gdn_layer_step"},
@@ -400,9 +659,13 @@ PyMethodDef methods[] = {
     {"gates", (PyCFunction)(void (*)())gates, METH_FASTCALL, "gdn_gates_fwd"},
     {"norm", (PyCFunction)(void (*)())norm, METH_FASTCALL, "gdn_gated_rmsnorm_fwd"},
     {"delta_rule", (PyCFunction)(void (*)())delta_rule, METH_FASTCALL, "gdn_chunk_fwd or gdn_recurrent_fwd"},
+    {"delta_rule_bwd", (PyCFunction)(void (*)())delta_rule_bwd, METH_FASTCALL, "gdn_chunk_bwd_sweeps, gdn_chunk_bwd_local"},
+    {"conv_bwd", (PyCFunction)(void (*)())conv_bwd, METH_FASTCALL, "gdn_causal_conv1d_bwd, gdn_column_sums"},
+    {"gates_bwd", (PyCFunction)(void (*)())gates_bwd, METH_FASTCALL, "gdn_gates_bwd, gdn_column_sums"},
+    {"norm_bwd", (PyCFunction)(void (*)())norm_bwd, METH_FASTCALL, "gdn_gated_rmsnorm_bwd, gdn_column_sums"},
     {nullptr, nullptr, 0, nullptr},
 };
-PyModuleDef module = {PyModuleDef_HEAD_INIT, "gdn_host", "host path of the inference entry points", -1, methods, nullptr, nullptr, nullptr, nullptr};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "gdn_host", "host path of the entry points and their backward passes", -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
 

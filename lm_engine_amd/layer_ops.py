@@ -148,7 +148,10 @@ class _GatesOnKernels(torch.autograd.Function):
     def forward(ctx, a, b, A_log, dt_bias, allow_neg_eigval):
         ctx.save_for_backward(a, b, A_log, dt_bias)
         ctx.allow_neg_eigval = allow_neg_eigval
-        return _delta_rule_gates(a, b, A_log, dt_bias, allow_neg_eigval)
+        result = None
+        if is_kernel_allowed(Kernel.gated_delta_rule):
+            result = host().gates(raw_stream(a.get_device()), a, b, A_log, dt_bias, 2.0 if allow_neg_eigval else 1.0)
+        return _delta_rule_gates(a, b, A_log, dt_bias, allow_neg_eigval) if result is None else result
 
     @staticmethod
     def backward(ctx, dg, dbeta):
@@ -159,6 +162,10 @@ class _GatesOnKernels(torch.autograd.Function):
 def _delta_rule_gates_backward(a, b, A_log, dt_bias, dg, dbeta, allow_neg_eigval):
     """``gdn_gates_bwd``: gradients with respect to a, b (contiguous, their dtype), A_log and dt_bias."""
     _require(a, "a")
+    if dg is not None and dbeta is not None:
+        grads = host().gates_bwd(raw_stream(a.get_device()), a, b, A_log, dt_bias, dg, dbeta, 2.0 if allow_neg_eigval else 1.0)
+        if grads is not None:
+            return grads
     H = a.size(-1)
     a2, a_stride = _token_rows(a, H, "a")
     b2, b_stride = _token_rows(b, H, "b")
@@ -265,7 +272,10 @@ class _GatedRMSNormOnKernels(torch.autograd.Function):
     def forward(ctx, o, gate, weight, eps):
         ctx.save_for_backward(o, gate, weight)
         ctx.eps = eps
-        return _gated_rmsnorm(o, gate, weight, eps)
+        y = None
+        if is_kernel_allowed(Kernel.gated_delta_rule):
+            y = host().norm(raw_stream(o.get_device()), o, gate, weight, float(torch.finfo(o.dtype).eps if eps is None else eps))
+        return _gated_rmsnorm(o, gate, weight, eps) if y is None else y
 
     @staticmethod
     def backward(ctx, dy):
@@ -276,6 +286,10 @@ class _GatedRMSNormOnKernels(torch.autograd.Function):
 
 def _gated_rmsnorm_backward(o, gate, weight, eps, dy):
     """``gdn_gated_rmsnorm_bwd``: gradients with respect to o, gate (shaped like gate) and weight."""
+    _require(o, "o")
+    grads = host().norm_bwd(raw_stream(o.get_device()), o, gate, weight, float(torch.finfo(o.dtype).eps if eps is None else eps), dy)
+    if grads is not None:
+        return grads
     o2, o_stride, g2, g_stride, H, V = _norm_operands(o, gate)
     tokens = o2.size(0)
     dy = kernel_rows(dy.to(o.dtype).contiguous())

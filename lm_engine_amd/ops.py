@@ -718,6 +718,19 @@ def chunk_bwd_prepare(q, k, dout, g, beta, scale, l2norm, V, sequences=None, hal
     return out
 
 
+def _on_host_path(mode, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm, inplace_state, left_padded):
+    """``(o, final_state)``, or None where the operands need a conversion, a gradient or a workspace that is kept."""
+    if not q.is_cuda or not is_kernel_allowed(Kernel.gated_delta_rule):
+        return None
+    device_index = q.get_device()
+    if mode == "chunk" and _forward_failed(device_index):
+        return None
+    flags = ((_lib.GDN_FLAG_L2NORM if l2norm else 0) | (_lib.GDN_FLAG_LEFT_PADDED if left_padded else 0)
+             | (_lib.GDN_FLAG_FUSED_LAUNCH if is_kernel_allowed(Kernel.gated_delta_rule_fused_launch) else 0))  # fmt: skip
+    return host().delta_rule(raw_stream(device_index), mode == "chunk", q, k, v, g, beta, scale, initial_state,
+                             output_final_state, cu_seqlens, flags, inplace_state)  # fmt: skip
+
+
 class _GatedDeltaRule(torch.autograd.Function):
     """Forward on the HIP kernels; backward by ``backward.gated_delta_rule_backward`` from the saved
     inputs (the forward keeps no intermediate results)."""
@@ -727,8 +740,9 @@ class _GatedDeltaRule(torch.autograd.Function):
                 initial_state, cu_seqlens):  # fmt: skip
         if inplace_state:
             raise ValueError("inplace_state overwrites the initial state the backward needs; it is for inference")
-        o, ht = _run(mode, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm,
-                     inplace_state, left_padded)  # fmt: skip
+        operands = (q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm, inplace_state, left_padded)
+        result = _on_host_path(mode, *operands)
+        o, ht = _run(mode, *operands) if result is None else result
         ctx.save_for_backward(q, k, v, g, beta, initial_state, cu_seqlens)
         ctx.options = (scale, l2norm, left_padded)
         return o, ht
@@ -752,15 +766,10 @@ def _dispatch(mode, q, k, v, g, beta, scale, initial_state, output_final_state, 
 
         return _opaque.gated_delta_rule(mode, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens,
                                         l2norm, inplace_state, left_padded)  # fmt: skip
-    if q.is_cuda and is_kernel_allowed(Kernel.gated_delta_rule):
-        device_index = q.get_device()
-        if mode != "chunk" or not _forward_failed(device_index):
-            flags = ((_lib.GDN_FLAG_L2NORM if l2norm else 0) | (_lib.GDN_FLAG_LEFT_PADDED if left_padded else 0)
-                     | (_lib.GDN_FLAG_FUSED_LAUNCH if is_kernel_allowed(Kernel.gated_delta_rule_fused_launch) else 0))  # fmt: skip
-            result = host().delta_rule(raw_stream(device_index), mode == "chunk", q, k, v, g, beta, scale, initial_state,
-                                       output_final_state, cu_seqlens, flags, inplace_state)  # fmt: skip
-            if result is not None:
-                return result
+    result = _on_host_path(mode, q, k, v, g, beta, scale, initial_state, output_final_state, cu_seqlens, l2norm, inplace_state,
+                           left_padded)  # fmt: skip
+    if result is not None:
+        return result
     tensors = (q, k, v, g, beta, initial_state)
     if torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in tensors):
         return _GatedDeltaRule.apply(mode, scale, output_final_state, l2norm, inplace_state, left_padded, q, k, v, g,

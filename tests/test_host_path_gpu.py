@@ -302,3 +302,84 @@ def test_calls_end_as_they_do_without_the_native_path(monkeypatch):
                 differ.append((name, form, *(z if isinstance(z, tuple) else "tensors" for z in (native, python))))
     torch.cuda.synchronize()
     assert not differ, "\n".join(map(str, differ))
+
+
+def _training_forms():
+    """``(name of the native backward, {form: (function, operands that want a gradient)})``"""
+    gen = torch.Generator().manual_seed(21)
+    r = lambda *shape: torch.randn(*shape, generator=gen).to(BF16).cuda()  # noqa: E731
+    x, w, bias, mask = r(2, 70, 384), 0.3 * r(384, 1, 4), 0.1 * r(384), (torch.rand(2, 70, generator=gen) > 0.3).to(BF16).cuda()
+    conv = lambda **kw: lambda *t: lm_engine_amd.depthwise_causal_convolution(*t, **kw)[0]  # noqa: E731
+    yield "conv_bwd", {
+        "plain": (conv(), (x, w, bias)), "no bias": (conv(), (x, w)), "2-D weight": (conv(), (x, w[:, 0])), "mask": (conv(attention_mask=mask), (x, w, bias)),
+        "mask int": (conv(attention_mask=mask.long()), (x, w, bias)), "mask of one row": (conv(attention_mask=mask[:1]), (x, w, bias)), "no activation": (conv(activation=None), (x, w, bias)),
+        "fp32": (conv(), (x.float(), w.float(), bias.float())), "fp32 weight": (conv(), (x, w.float(), bias.float())), "slice": (conv(), (r(2, 70, 400)[..., 8:392], w, bias)),
+        "state": (lambda x, w, s: lm_engine_amd.depthwise_causal_convolution(x, w, None, s)[0], (x, w, r(2, 384, 3))), "one token": (conv(), (x[:, :1], w, bias)),
+    }  # fmt: skip
+    a, b, A, dt, ab = r(2, 70, 3), r(2, 70, 3), torch.rand(3, generator=gen).cuda(), torch.rand(3, generator=gen).cuda(), r(2, 70, 8)
+    gates = lambda *t, **kw: torch.cat([y.float().flatten() for y in lm_engine_amd.delta_rule_gates(*t, **kw)])  # noqa: E731
+    yield "gates_bwd", {
+        "plain": (gates, (a, b, A, dt)), "slices": (gates, (ab[..., :3], ab[..., 3:6], A, dt)), "negative eigenvalues": (lambda *t: gates(*t, allow_neg_eigval=True), (a, b, A, dt)),
+        "bf16 decay": (gates, (a, b, A.to(BF16), dt.to(BF16))), "fp32": (gates, (a.float(), b.float(), A, dt)), "one of two": (lambda *t: lm_engine_amd.delta_rule_gates(*t)[0], (a, b, A, dt)),
+    }  # fmt: skip
+    o, z, nw = r(2, 70, 2, 64), r(2, 70, 128), r(64)
+    norm = lambda o, z, w=None: lm_engine_amd.gated_rmsnorm(o, z, w, 1e-5)  # noqa: E731
+    yield "norm_bwd", {
+        "plain": (norm, (o, z, nw)), "no weight": (norm, (o, z)), "no gate": (lambda o, w: norm(o, None, w), (o, nw)), "gate by heads": (norm, (o, z.view(2, 70, 2, 64), nw)),
+        "gate slice": (norm, (o, r(2, 70, 140)[..., 4:132], nw)), "gate slice off its boundary": (norm, (o, r(2, 70, 140)[..., 3:131], nw)), "o strided": (norm, (r(2, 2, 70, 64).transpose(1, 2), z, nw)),
+        "fp32": (norm, (o.float(), z.float(), nw.float())), "fp32 weight": (norm, (o, z, nw.float())),
+    }  # fmt: skip
+    for T in (128, 130):
+        unit = lambda x: torch.nn.functional.normalize(x, dim=-1)  # noqa: E731
+        q, k, v = unit(r(2, T, 2, 64)), unit(r(2, T, 2, 64)), r(2, T, 2, 64)
+        g, beta, h = -torch.rand(2, T, 2, generator=gen).cuda(), torch.rand(2, T, 2, generator=gen).to(BF16).cuda(), torch.randn(2, 2, 64, 64, generator=gen).cuda()
+        qkv = 0.1 * r(2, T, 3 * 128)
+        blocks = [x.view(2, T, 2, 64) for x in qkv.split(128, dim=-1)]
+
+        def op(**kw):
+            def run(q, k, v, g=None, beta=None, h=None):
+                o, ht = lm_engine_amd.chunk_gated_delta_rule(q, k, v, g, beta, initial_state=h, **kw)
+                return o if ht is None else torch.cat([o.flatten().float(), ht.flatten()])
+
+            return run
+
+        cu = lambda *ends: torch.tensor(ends, dtype=torch.int32).cuda()  # noqa: E731
+        one = tuple(t[:1] for t in (q, k, v, g, beta))
+        yield "delta_rule_bwd", {
+            "plain": (op(use_qk_l2norm_in_kernel=True), (q, k, v, g, beta)), "no l2norm": (op(), (q, k, v, g, beta)), "ungated": (op(), (q, k, v)), "beta fp32": (op(), (q, k, v, g, beta.float())),
+            "states": (op(output_final_state=True, use_qk_l2norm_in_kernel=True), (q, k, v, g, beta, h)), "scale": (op(scale=0.3), (q, k, v, g, beta)), "blocks of one tensor": (op(), (*blocks, g, beta)),
+            "strided q": (op(), (unit(r(2, 2, T, 64)).transpose(1, 2), k, v, g, beta)), "shared heads": (op(use_qk_l2norm_in_kernel=True), (q[:, :, :1], k[:, :, :1], v, g, beta)),
+            "packed": (op(cu_seqlens=cu(0, 3, T), output_final_state=True), (*one, h)), "packed, empty ones": (op(cu_seqlens=cu(0, 0, 70, 70, T)), one), "packed, tokens left over": (op(cu_seqlens=cu(0, 70, T - 9)), one),
+            "packed, int64 prefix": (op(cu_seqlens=cu(0, 3, T).long()), one), "padded": (op(cu_seqlens=cu(0, 70, 70 + T), left_padded=True), (q, k, v, g, beta)), "fp32": (op(), tuple(t.float() for t in (q, k, v, g, beta))),
+            "V = 96": (op(), (q, k, r(2, T, 2, 96), g, beta)),
+        }  # fmt: skip
+
+
+def test_backward_passes_end_as_they_do_without_the_native_path(monkeypatch):
+    """The gradients of every form are the same bits with the native host path and without it, for a gradient that lies as
+    the output does, a column block of a wider one, and one value for all elements."""
+    from lm_engine_amd import backward, conv, layer_ops, ops
+
+    differ = []
+    for name, forms in _training_forms():
+        for form, (function, operands) in forms.items():
+            outcomes = []
+            print(f"case: {name}, {form}", flush=True)
+            for on in (True, False):
+                path = _NativePath(on)
+                with monkeypatch.context() as m:
+                    for module in (backward, conv, layer_ops, ops):
+                        m.setattr(module, "host", lambda path=path: path)
+                    leaves = [x.detach().requires_grad_(True) for x in operands]
+                    out = function(*leaves)
+                    path.took.clear()
+                    wide = torch.randn(*out.shape[:-1], 2 * out.size(-1) + 8, generator=torch.Generator().manual_seed(4)).to(out.dtype).cuda()
+                    results = []
+                    for d in (wide[..., : out.size(-1)].contiguous(), wide[..., 8 : 8 + out.size(-1)], torch.ones((), dtype=out.dtype).cuda().expand(out.shape)):
+                        results += [x.clone() for x in torch.autograd.grad(out, leaves, d, retain_graph=True, allow_unused=True) if x is not None]
+                outcomes.append(results)
+                assert form != "plain" or path.took[0] == on, "the path under test was not the one taken"
+            if not all(x.dtype == y.dtype and x.shape == y.shape and torch.equal(x, y) for x, y in zip(*outcomes)) or len(outcomes[0]) != len(outcomes[1]):
+                differ.append((name, form))
+    torch.cuda.synchronize()
+    assert not differ, differ
