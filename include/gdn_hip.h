@@ -301,10 +301,13 @@ int gdn_chunk_fwd_saving_is_staged(const gdn_args *args, const gdn_chunk_saves *
  * kernels of fla's backward of chunk_gated_delta_rule, reached from gated_deltanet/module.py:197-209 under autograd.
  */
 #define GDN_LOCAL_DBETA_BF16 0x100 /* in saves_dtype: dbeta_out is bf16 */
+/* in saves_dtype: n heads of v share a head of q and k (n divides H): q_raw and k_raw have H / n heads; dq_out and dk_out keep a
+ * gradient per head of v, [N, T, H, K] contiguous whatever out_stride_t, for gdn_fold_heads */
+#define GDN_LOCAL_SHARED_HEADS(n) ((n) << 16)
 typedef struct gdn_chunk_local_args {
     const void *v_new, *states, *dstates;
     const float *gamma, *beta, *rq, *rk;
-    int32_t saves_dtype; /* gdn_dtype of v_new and states, | GDN_LOCAL_DBETA_BF16 */
+    int32_t saves_dtype; /* gdn_dtype of v_new and states, | GDN_LOCAL_DBETA_BF16 | GDN_LOCAL_SHARED_HEADS(n) */
     float scale;
     int64_t chunks;
     int32_t K, V;
@@ -330,6 +333,14 @@ typedef struct gdn_chunk_local_args {
                               of one array of token rows; 0: each contiguous */
 } gdn_chunk_local_args;
 int gdn_chunk_bwd_local(const gdn_chunk_local_args *args, void *stream);
+/*
+ * The gradients of heads of q and k that `group` value heads share: out_a[t][h][:] = sum over j < group of a[t][h group + j][:], the
+ * same for b, bf16 summed up in fp32.  a, b [tokens][heads group][D] contiguous; out_stride_t elements between the tokens of out_a
+ * and out_b, which must not overlap a and b.  D and out_stride_t multiples of 8, 16-byte aligned.  What autograd does behind the
+ * reference's repeat_interleave (gated_deltanet/module.py:175-177).
+ */
+int gdn_fold_heads(const void *a, const void *b, void *out_a, void *out_b, int64_t tokens, int heads, int group, int D,
+                   int64_t out_stride_t, void *stream);
 
 /*
  * Training support, third part: everything the backward needs per chunk before two sweeps through gdn_chunk_fwd_saving (batches of

@@ -61,6 +61,7 @@ EXPORTED_SYMBOLS = (
     "gdn_gated_rmsnorm_fwd",
     "gdn_gated_rmsnorm_bwd",
     "gdn_column_sums",
+    "gdn_fold_heads",
     "gdn_padding_mask",
     "gdn_layer_step",
     "gdn_layer_step_tiles",
@@ -282,6 +283,8 @@ def load_library() -> ctypes.CDLL:
     lib.gdn_padding_mask.restype = ctypes.c_int
     lib.gdn_column_sums.argtypes = [ctypes.POINTER(GdnColumnSumsArgs), ctypes.c_void_p]
     lib.gdn_column_sums.restype = ctypes.c_int
+    lib.gdn_fold_heads.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_void_p]
+    lib.gdn_fold_heads.restype = ctypes.c_int
     lib.gdn_gated_rmsnorm_fwd.argtypes = [ctypes.POINTER(GdnNormArgs), ctypes.c_void_p]
     lib.gdn_gated_rmsnorm_fwd.restype = ctypes.c_int
 

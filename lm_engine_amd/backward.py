@@ -340,8 +340,9 @@ def _chunk_local_grads(qs, kn, vc, doc, Y, Vn, S0, dS1, gam, bc):
 
 def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm, cu_seqlens, left_padded, joined):
     """The whole backward on three kernel launches (bf16; K = 64, 128 or 256; V a multiple of 64): ``gdn_chunk_bwd_sweeps``
-    (per-chunk records and scalars, the forward sweep, the reverse sweep; one more launch for the chunk offsets of packed
-    sequences) and ``gdn_chunk_bwd_local`` writing the gradients in the caller's layout.  Chunk states, V~ and Y pass between
+    (per-chunk records and scalars, both sweeps; one more launch for the chunk offsets of packed
+    sequences) and ``gdn_chunk_bwd_local`` writing the gradients in the caller's layout (one more launch, ``gdn_fold_heads``, where
+    value heads share those of q and k).  Chunk states, V~ and Y pass between
     them as bf16, what the chunk-local products round them to anyway.  Batches that are not whole rows of whole chunks are laid
     out with the chunk count of their longest sequence."""
     from . import ops  # late: ops imports this module
@@ -363,6 +364,11 @@ def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm
         NC = -(-T // CHUNK)
         if T % CHUNK != 0:
             sequences = (*ops.upload_int32(_chains(B, T, None, False), q.device), NC)
+    heads, group = q.size(2), v.size(2) // q.size(2)
+    if group > 1:
+        # Grouped value attention: on the expanded heads (what the reference's repeat_interleave hands its operator,
+        # gated_deltanet/module.py:175-177), a group's gradients added up.
+        q, k, joined = q.repeat_interleave(group, dim=2), k.repeat_interleave(group, dim=2), False
     q, k, v = (x if x.stride(-1) == 1 else x.contiguous() for x in (q, k, v))
     do = kernel_rows(do.to(torch.bfloat16))
     if do.stride(1) > 1 << 24:  # the kernels count a chunk's rows in 32 bits; q, k and v were held to that by the forward
@@ -370,6 +376,8 @@ def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm
     prep, S0, Vn, dS1, Y, dh0 = ops.chunk_bwd_sweeps(q, k, v, do, g, beta, scale, l2norm, initial_state, cu_seqlens, left_padded, dht, NC)
     dq, dk, dv, dg, dbeta = ops.chunk_local_grads(q, k, v, do, prep, Y, Vn, S0, dS1, scale, l2norm, sequences, sliced=True,
                                                   covers=covers, joined=joined)  # fmt: skip
+    if group > 1:
+        dq, dk = (_fold(d, heads, group) for d in (dq, dk))
     return (
         dq,
         dk,
@@ -378,6 +386,10 @@ def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm
         dbeta.to(beta.dtype) if beta is not None else None,
         dh0,
     )
+
+
+def _fold(d, heads, group):
+    return d.view(*d.shape[:2], heads, group, d.size(3)).sum(dim=3, dtype=torch.float32).to(d.dtype)
 
 
 def gated_delta_rule_backward(
@@ -390,22 +402,19 @@ def gated_delta_rule_backward(
     shape of ``o``, ``dht`` that of the final state or is None.  Returns
     ``dq, dk, dv, dg, dbeta, dh0`` in the dtypes of the corresponding inputs (fp32 for dh0); entries for
     absent inputs are None.  ``joined``: dq, dk and dv may be column blocks of one tensor (they are on the kernels)."""
-    if q.size(2) != v.size(2):
-        # Grouped value attention: the backward runs on the expanded heads (what the reference's repeat_interleave hands
-        # its operator, gated_deltanet/module.py:175-177) and adds the gradients of a group's copies up.
-        group = v.size(2) // q.size(2)
-        dq, dk, *rest = gated_delta_rule_backward(
-            q.repeat_interleave(group, dim=2), k.repeat_interleave(group, dim=2), v, g, beta, do, dht, scale, initial_state,
-            cu_seqlens, use_qk_l2norm_in_kernel, left_padded)  # fmt: skip
-        fold = lambda d: d.view(*q.shape[:2], q.size(2), group, q.size(3)).sum(dim=3, dtype=torch.float32).to(d.dtype)  # noqa: E731
-        return (fold(dq), fold(dk), *rest)
-    B, T, H, K = q.shape
-    V = v.size(-1)
-    dev = q.device
+    K, V = q.size(-1), v.size(-1)
     scale = K**-0.5 if scale is None else scale
     if q.is_cuda and q.dtype == torch.bfloat16 and _kernels_apply(K, V):
         return _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, use_qk_l2norm_in_kernel,
                                     cu_seqlens, left_padded, joined)  # fmt: skip
+    if q.size(2) != v.size(2):  # grouped value attention, as on the kernels
+        group = v.size(2) // q.size(2)
+        dq, dk, *rest = gated_delta_rule_backward(
+            q.repeat_interleave(group, dim=2), k.repeat_interleave(group, dim=2), v, g, beta, do, dht, scale, initial_state,
+            cu_seqlens, use_qk_l2norm_in_kernel, left_padded)  # fmt: skip
+        return (_fold(dq, q.size(2), group), _fold(dk, q.size(2), group), *rest)
+    B, T, H, K = q.shape
+    dev = q.device
     pk = _Packing(B, T, H, cu_seqlens, left_padded, dev)
     N, NC, Bt = pk.N, pk.NC, pk.N * H
 

@@ -232,11 +232,13 @@ int gdn_chunk_bwd_local(const gdn_chunk_local_args* a, void* stream) {
     for (const void* x : needed)
         if (x == nullptr) return GDN_ERR_NULL;
         else if (!aligned(x, 16)) return GDN_ERR_ALIGN;
-    const int saves_dtype = a->saves_dtype & ~GDN_LOCAL_DBETA_BF16;
+    const int saves_dtype = a->saves_dtype & 0xff, group = a->saves_dtype >> 16;
+    if ((a->saves_dtype & 0xff00) != 0 && (a->saves_dtype & 0xff00) != GDN_LOCAL_DBETA_BF16) return GDN_ERR_UNSUPPORTED;
+    if (group < 0 || (group > 0 && a->H % group != 0)) return GDN_ERR_SHAPE;
     if (saves_dtype != GDN_BF16 && saves_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
     if (a->dstates_dtype != GDN_BF16 && a->dstates_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
     if (a->saves_sliced && (saves_dtype != GDN_BF16 || a->dstates_dtype != GDN_BF16 || a->y_chunks == nullptr)) return GDN_ERR_UNSUPPORTED;
-    if (a->out_stride_t != 0 && (a->out_stride_t < (int64_t)a->H * a->K || a->out_stride_t < (int64_t)a->H * a->V)) return GDN_ERR_SHAPE;
+    if (a->out_stride_t != 0 && ((group <= 1 && a->out_stride_t < (int64_t)a->H * a->K) || a->out_stride_t < (int64_t)a->H * a->V)) return GDN_ERR_SHAPE;
     if (a->out_stride_t % 8 != 0) return GDN_ERR_ALIGN;
     if (a->H <= 0 || a->NC <= 0 || a->chunks % ((int64_t)a->H * a->NC) != 0) return GDN_ERR_SHAPE;
     if (a->seq_start != nullptr && (a->seq_len == nullptr || a->T_rows <= 0)) return GDN_ERR_SHAPE;

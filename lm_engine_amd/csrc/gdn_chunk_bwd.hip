@@ -81,6 +81,7 @@ struct ChunkLocalParams {
     int dbeta_bf16;
     int64_t dqk_stride_t, dv_stride_t;  // elements between the tokens of dq_out and dk_out, and of dv_out
     int H, NC, V;
+    int qk_div;  // value heads per head of q and k
     // sequences that are not whole rows of whole chunks (packed or left-padded batches): first token (flat index
     // over the rows of the caller's tensors) and length of every sequence; NULL = sequence n is row n
     const int32_t* seq_start;
@@ -241,8 +242,12 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
     // row `row` of the chunk in one of the caller's tensors (a chunk lies within one row of the batch); rows past the
     // end of the sequence read its last token and are zeroed
     const int64_t row_b = tok0 / p.T_rows, row_t = tok0 % p.T_rows;
+    const int hqk = qk_head_of(h, p.qk_div);
     auto row_of = [&](const bf16_t* base, int64_t sb, int64_t st, int64_t sh, int row) -> const bf16_t* {
         return base + row_b * sb + (row_t + min(row, valid - 1)) * st + (int64_t)h * sh;
+    };
+    auto qk_row_of = [&](const bf16_t* base, int64_t sb, int64_t st, int64_t sh, int row) -> const bf16_t* {
+        return base + row_b * sb + (row_t + min(row, valid - 1)) * st + (int64_t)hqk * sh;
     };
     bf16x8 zero8;
 #pragma unroll
@@ -319,8 +324,8 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 #pragma unroll
         for (int it = 0; it < C / RPP; it++) {
             const int row = tl / CPR + RPP * it;
-            nx_s0[2 * it] = *reinterpret_cast<const bf16x8*>(row_of(p.q_raw, p.q_stride_b, p.q_stride_t, p.q_stride_h, row) + KW * kh + 8 * p8);
-            nx_s0[2 * it + 1] = *reinterpret_cast<const bf16x8*>(row_of(p.k_raw, p.k_stride_b, p.k_stride_t, p.k_stride_h, row) + KW * kh + 8 * p8);
+            nx_s0[2 * it] = *reinterpret_cast<const bf16x8*>(qk_row_of(p.q_raw, p.q_stride_b, p.q_stride_t, p.q_stride_h, row) + KW * kh + 8 * p8);
+            nx_s0[2 * it + 1] = *reinterpret_cast<const bf16x8*>(qk_row_of(p.k_raw, p.k_stride_b, p.k_stride_t, p.k_stride_h, row) + KW * kh + 8 * p8);
         }
     };
     auto put_qk = [&]() {
@@ -583,8 +588,8 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 #pragma unroll
                 for (int it = 0; it < C / RPP; it++) {
                     const int row = t / CPR + RPP * it;
-                    bf16x8 qr = *reinterpret_cast<const bf16x8*>(row_of(p.q_raw, p.q_stride_b, p.q_stride_t, p.q_stride_h, row) + KW * kh + 8 * p8);
-                    bf16x8 kr = *reinterpret_cast<const bf16x8*>(row_of(p.k_raw, p.k_stride_b, p.k_stride_t, p.k_stride_h, row) + KW * kh + 8 * p8);
+                    bf16x8 qr = *reinterpret_cast<const bf16x8*>(qk_row_of(p.q_raw, p.q_stride_b, p.q_stride_t, p.q_stride_h, row) + KW * kh + 8 * p8);
+                    bf16x8 kr = *reinterpret_cast<const bf16x8*>(qk_row_of(p.k_raw, p.k_stride_b, p.k_stride_t, p.k_stride_h, row) + KW * kh + 8 * p8);
                     if (row >= valid) qr = zero8, kr = zero8;
                     const float fq = s_fq[row], fk = s_fk[row];
                     bf16x8 qb, kb;
@@ -1283,7 +1288,7 @@ int launch_chunk_bwd_local(const gdn_chunk_local_args& a, hipStream_t stream) {
     p.cycle_out = cycle_buffer();
     if (p.cycle_out != nullptr) (void)hipMemsetAsync(p.cycle_out, 0, GDN_LOCAL_CYCLE_SLOTS * 16 * sizeof(uint64_t), stream);
 #endif
-    p.vnew = a.v_new, p.s0 = a.states, p.ds1 = a.dstates, p.saves_bf16 = (a.saves_dtype & ~GDN_LOCAL_DBETA_BF16) == GDN_BF16 ? 1 : 0;
+    p.vnew = a.v_new, p.s0 = a.states, p.ds1 = a.dstates, p.saves_bf16 = (a.saves_dtype & 0xff) == GDN_BF16 ? 1 : 0;
     p.dbeta_bf16 = (a.saves_dtype & GDN_LOCAL_DBETA_BF16) != 0 ? 1 : 0;
     const bool h = a.dstates_dtype == GDN_BF16;
     const bool sl = a.saves_sliced != 0;
@@ -1292,7 +1297,8 @@ int launch_chunk_bwd_local(const gdn_chunk_local_args& a, hipStream_t stream) {
     p.y_mirror = static_cast<const bf16_t*>(a.y_mirror), p.y_chunks = static_cast<const bf16_t*>(a.y_chunks);
     p.dq_out = static_cast<bf16_t*>(a.dq_out), p.dk_out = static_cast<bf16_t*>(a.dk_out), p.dv_out = static_cast<bf16_t*>(a.dv_out);
     p.dg_out = a.dg_out, p.dbeta_out = a.dbeta_out;
-    p.dqk_stride_t = a.out_stride_t > 0 ? a.out_stride_t : (int64_t)a.H * a.K;
+    p.qk_div = a.saves_dtype >> 16;
+    p.dqk_stride_t = a.out_stride_t > 0 && p.qk_div <= 1 ? a.out_stride_t : (int64_t)a.H * a.K;
     p.dv_stride_t = a.out_stride_t > 0 ? a.out_stride_t : (int64_t)a.H * a.V;
     p.H = a.H, p.NC = a.NC, p.V = a.V;
     p.q_raw = static_cast<const bf16_t*>(a.q_raw), p.k_raw = static_cast<const bf16_t*>(a.k_raw);

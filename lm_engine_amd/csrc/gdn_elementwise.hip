@@ -365,6 +365,37 @@ __global__ __launch_bounds__(SUM_COLS * SUM_ROWS) void column_sums_kernel(const 
     }
 }
 
+// dq and dk of value heads that share a head of q and k, added up (blockIdx.y names which of the two).  A thread has 8 columns of one
+// head and reads the group's rows of them, 16 bytes each.  Bound by memory: (group + 1) rows per row written;
+// 4 x 4096 tokens, 16 heads on 8, D = 128: 34 us for both, 6.0 TB/s (as torch's sums and copies of q and k in front 196).
+struct FoldParams {
+    const bf16_t* in[2];
+    bf16_t* out[2];
+    int64_t pieces;  // of 8 columns, over all tokens
+    int64_t out_stride_t;
+    int group, D, heads;
+};
+
+__global__ __launch_bounds__(256) void fold_heads_kernel(const FoldParams p) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= p.pieces) return;
+    const int per_head = p.D / 8;
+    const int64_t row = i / per_head;  // token and head
+    const int c = (int)(i - row * per_head) * 8;
+    const int64_t token = row / p.heads;
+    const bf16_t* in = p.in[blockIdx.y] + row * p.group * p.D + c;
+    float sum[8] = {};
+    for (int j = 0; j < p.group; j++) {
+        const bf16x8 x = *reinterpret_cast<const bf16x8*>(in + (int64_t)j * p.D);
+#pragma unroll
+        for (int e = 0; e < 8; e++) sum[e] += (float)x[e];
+    }
+    bf16x8 y;
+#pragma unroll
+    for (int e = 0; e < 8; e++) y[e] = (bf16_t)sum[e];
+    *reinterpret_cast<bf16x8*>(p.out[blockIdx.y] + token * p.out_stride_t + (row - token * p.heads) * p.D + c) = y;
+}
+
 // A padding mask [B, S] of integers in the two forms the layer works with: the mask in the activation dtype (rows contiguous) and the
 // int32 prefix sums of its rows' sums [B + 1].  One workgroup, whose waves share the rows between them: bound by the launch and
 // one trip through memory.  As conversion, row sums, prefix sum, pad and copies it was six launches (6 x 1500 tokens, 8 / 16 heads,
@@ -540,6 +571,25 @@ extern "C" int gdn_column_sums(const gdn_column_sums_args* a, void* stream) {
     if (blocks > 0x7fffffff) return GDN_ERR_UNSUPPORTED;
     hipLaunchKernelGGL(gdn::column_sums_kernel, dim3((unsigned)blocks, (unsigned)a->arrays), dim3(gdn::SUM_COLS * gdn::SUM_ROWS), 0,
                        static_cast<hipStream_t>(stream), p);
+    return (int)hipGetLastError();
+}
+
+extern "C" int gdn_fold_heads(const void* a, const void* b, void* out_a, void* out_b, int64_t tokens, int heads, int group, int D,
+                              int64_t out_stride_t, void* stream) {
+    const void* ptrs[] = {a, b, out_a, out_b};
+    for (const void* x : ptrs)
+        if (x == nullptr) return GDN_ERR_NULL;
+        else if (!aligned_to(x, 16)) return GDN_ERR_ALIGN;
+    if (tokens <= 0 || heads <= 0 || group <= 0 || D <= 0 || out_stride_t < (int64_t)heads * D) return GDN_ERR_SHAPE;
+    if (D % 8 != 0 || out_stride_t % 8 != 0) return GDN_ERR_ALIGN;
+    gdn::FoldParams p;
+    p.in[0] = static_cast<const gdn::bf16_t*>(a), p.in[1] = static_cast<const gdn::bf16_t*>(b);
+    p.out[0] = static_cast<gdn::bf16_t*>(out_a), p.out[1] = static_cast<gdn::bf16_t*>(out_b);
+    p.pieces = tokens * heads * (D / 8), p.out_stride_t = out_stride_t;
+    p.group = group, p.D = D, p.heads = heads;
+    const int64_t blocks = (p.pieces + 255) / 256;
+    if (blocks > (int64_t)0xffffffff / 256) return GDN_ERR_UNSUPPORTED;  // (a launch holds at most 2^32 - 1 threads)
+    hipLaunchKernelGGL(gdn::fold_heads_kernel, dim3((unsigned)blocks, 2), dim3(256), 0, static_cast<hipStream_t>(stream), p);
     return (int)hipGetLastError();
 }
 

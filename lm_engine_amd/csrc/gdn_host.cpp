@@ -38,6 +38,7 @@ decltype(&gdn_causal_conv1d_bwd) conv_bwd_fn = nullptr;
 decltype(&gdn_gates_bwd) gates_bwd_fn = nullptr;
 decltype(&gdn_gated_rmsnorm_bwd) norm_bwd_fn = nullptr;
 decltype(&gdn_column_sums) column_sums_fn = nullptr;
+decltype(&gdn_fold_heads) fold_heads_fn = nullptr;
 PyObject* check_status = nullptr;  // _lib.check_status: raises what a status stands for
 
 // bind(check_status, addresses...)
@@ -45,7 +46,7 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
     void** slots[] = {(void**)&layer_step_fn, (void**)&layer_step_tiles_fn, (void**)&conv_fn, (void**)&gates_fn, (void**)&norm_fn,
                       (void**)&recurrent_fn, (void**)&chunk_fn, (void**)&workspace_bytes_fn, (void**)&one_launch_fn,
                       (void**)&sweeps_fn, (void**)&sweeps_workspace_fn, (void**)&local_fn, (void**)&conv_bwd_fn, (void**)&gates_bwd_fn,
-                      (void**)&norm_bwd_fn, (void**)&column_sums_fn};
+                      (void**)&norm_bwd_fn, (void**)&column_sums_fn, (void**)&fold_heads_fn};
     constexpr Py_ssize_t count = sizeof(slots) / sizeof(slots[0]);
     if (n != count + 1) return PyErr_Format(PyExc_TypeError, "bind takes a function and %zd addresses, got %zd arguments", count, n);
     for (Py_ssize_t i = 0; i < count; i++) {
@@ -432,7 +433,7 @@ void need_rows(const at::Tensor& t, int64_t stride_elements, size_t address_byte
 // delta_rule_bwd(stream, q, k, v, g, beta, initial_state, cu_seqlens, do, dht, scale, flags, seq_start, seq_len, NC, covers, joined)
 //   -> (dq, dk, dv, dg, dbeta, dh0)
 // Rows of a batch: without seq_start and seq_len.  Else NC chunks for the longest sequence; covers: every token belongs to one.
-// joined: dq, dk and dv as column blocks of one tensor.
+// joined: dq, dk and dv as column blocks of one tensor, where v has no more heads than q and k.
 PyObject* delta_rule_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return fast_path(n, 17, [&]() -> PyObject* {
         Operands operand;
@@ -446,8 +447,8 @@ PyObject* delta_rule_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
         s.dtype = code_of(q), s.flags = (int32_t)integer(args[11]);
         const bool padded = (s.flags & GDN_FLAG_LEFT_PADDED) != 0;
         need(s.dtype == GDN_BF16 && q.dim() == 4 && k.sizes() == q.sizes() && v.dim() == 4 && k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type());
-        const int64_t B = q.size(0), T = q.size(1), H = q.size(2), K = q.size(3), V = v.size(3);
-        need(v.size(0) == B && v.size(1) == T && v.size(2) == H && B > 0 && T > 0 && H > 0 && q.stride(3) == 1 && k.stride(3) == 1 && v.stride(3) == 1);
+        const int64_t B = q.size(0), T = q.size(1), HK = q.size(2), K = q.size(3), H = v.size(2), V = v.size(3);
+        need(v.size(0) == B && v.size(1) == T && B > 0 && T > 0 && HK > 0 && H > 0 && H % HK == 0 && H / HK < 0x8000 && q.stride(3) == 1 && k.stride(3) == 1 && v.stride(3) == 1);
         need((K == 64 || K == 128 || K == 256) && V % 64 == 0);
         need(d.scalar_type() == at::kBFloat16 && d.sizes() == v.sizes() && d.stride(1) <= (int64_t)1 << 24);
         need_rows(d, 8, 16);
@@ -476,6 +477,7 @@ PyObject* delta_rule_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
         for (const at::Tensor* t : states)
             if (t != nullptr) need(t->scalar_type() == at::kFloat && t->sizes() == at::IntArrayRef({N, H, K, V}) && t->is_contiguous() && aligned(ptr(t), 16));
         s.B = size32(B), s.T = size32(T), s.H = size32(H), s.K = (int32_t)K, s.V = size32(V), s.N = size32(N), s.chunk = 64;
+        s.qk_heads = HK == H ? 0 : (int32_t)HK;
         s.cu_seqlens = static_cast<const int32_t*>(ptr(cu));
         s.scale = (float)number(args[10]);
         s.q = ptr(q), s.k = ptr(k), s.v = ptr(v), s.o = ptr(v), s.beta = ptr(beta);  // (no output is written)
@@ -488,6 +490,7 @@ PyObject* delta_rule_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
         need(s.workspace_bytes > 0);
 
         at::Tensor workspace, scalars, S0, dS1, Vn, Y, dq, dk, dv, dg, dbeta, dh0;
+        at::Tensor dq_each, dk_each;  // per value head, where value heads share those of q and k
         without_interpreter_lock([&] {
             scalars = fresh_f32(q, {4, N * H, NC, 64});
             S0 = fresh(q, {N * H, NC, K, V}), dS1 = fresh(q, {N * H, NC, K, V}), Vn = fresh(q, {N * H, NC, 64, V}), Y = fresh(q, {N * H, NC, 64, V});
@@ -518,7 +521,8 @@ PyObject* delta_rule_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
             auto made = [&](at::IntArrayRef sizes, at::ScalarType dtype) {
                 return covers || cu == nullptr ? at::empty(sizes, q.options().dtype(dtype)) : at::zeros(sizes, q.options().dtype(dtype));
             };
-            if (joined) {
+            if (HK != H) dq_each = made({B, T, H, K}, at::kBFloat16), dk_each = made({B, T, H, K}, at::kBFloat16);
+            if (joined && HK == H) {
                 const int64_t row = H * (2 * K + V);
                 const at::Tensor rows = made({B, T, row}, at::kBFloat16);
                 dq = rows.as_strided({B, T, H, K}, {T * row, row, K, 1}, 0);
@@ -526,15 +530,19 @@ PyObject* delta_rule_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
                 dv = rows.as_strided({B, T, H, V}, {T * row, row, V, 1}, 2 * H * K);
                 l.out_stride_t = size32(row);
             } else {
-                dq = made({B, T, H, K}, at::kBFloat16), dk = made({B, T, H, K}, at::kBFloat16), dv = made({B, T, H, V}, at::kBFloat16);
+                dq = made({B, T, HK, K}, at::kBFloat16), dk = made({B, T, HK, K}, at::kBFloat16), dv = made({B, T, H, V}, at::kBFloat16);
             }
             dg = made({B, T, H}, at::kFloat), dbeta = made({B, T, H}, beta == nullptr ? at::kFloat : beta->scalar_type());
         });
         l.dq_out = ptr(dq), l.dk_out = ptr(dk), l.dv_out = ptr(dv), l.dg_out = static_cast<float*>(ptr(dg)), l.dbeta_out = static_cast<float*>(ptr(dbeta));
         if (!(s.flags & GDN_FLAG_L2NORM)) l.rq = l.rk = nullptr;
         if (dbeta.scalar_type() == at::kBFloat16) l.saves_dtype |= GDN_LOCAL_DBETA_BF16;
-        return launch("gdn_chunk_bwd_local", pack_results({dq, dk, dv, g == nullptr ? at::Tensor() : dg, beta == nullptr ? at::Tensor() : dbeta, dh0}),
-                      [&] { return local_fn(&l, stream); });
+        if (HK != H) l.saves_dtype |= GDN_LOCAL_SHARED_HEADS((int32_t)(H / HK)), l.dq_out = ptr(dq_each), l.dk_out = ptr(dk_each);
+        return launch("gdn_chunk_bwd_local", pack_results({dq, dk, dv, g == nullptr ? at::Tensor() : dg, beta == nullptr ? at::Tensor() : dbeta, dh0}), [&] {
+            const int status = local_fn(&l, stream);
+            if (status != GDN_OK || HK == H) return status;
+            return fold_heads_fn(l.dq_out, l.dk_out, ptr(dq), ptr(dk), B * T, (int)HK, (int)(H / HK), (int)K, dq.stride(1), stream);
+        });
     });
 }
 

@@ -114,3 +114,25 @@ def test_gradients_are_the_sums_over_a_group(K, V):
         err = rel_l2(a, b)
         print(f"   K={K} V={V} d{name}: rel-L2 {err:.3e}", flush=True)
         assert err <= 4e-3, f"d{name}: rel-L2 {err:.3e}"  # the group's sum is rounded once here, per copy and then summed there
+
+
+@pytest.mark.parametrize("HK, group, K, V, T, packed", [(1, 2, 64, 64, 1, False), (3, 2, 128, 128, 130, False), (2, 4, 256, 64, 64, False), (1, 5, 64, 128, 200, True)])
+def test_gradients_of_shared_heads_are_those_of_copies_added_up(HK, group, K, V, T, packed):
+    """The kernels' gradients of q and k copied per value head, added up in fp32 and rounded once (2^-9; the order of the sum: 2^-22 per term)."""
+    from lm_engine_amd.backward import gated_delta_rule_backward
+
+    gen = torch.Generator().manual_seed(T + K)
+    B, H = 1 if packed else 2, HK * group
+    rows = torch.randn(B, T, 2 * HK * K + H * V, generator=gen).bfloat16().cuda()
+    q, k, v = (x.unflatten(-1, (-1, d)) for x, d in zip(rows.split((HK * K, HK * K, H * V), dim=-1), (K, K, V)))
+    g, beta = -torch.rand(B, T, H, generator=gen).cuda(), torch.rand(B, T, H, generator=gen).bfloat16().cuda()
+    do = torch.randn(B, T, H, V, generator=gen).bfloat16().cuda()
+    cu = torch.tensor([0, T // 3, T - 5], dtype=torch.int32).cuda() if packed else None  # the last tokens belong to no sequence
+    print(f"case: gradients of shared heads HK={HK} group={group} K={K} V={V} T={T}", flush=True)
+    run = lambda q, k: gated_delta_rule_backward(q, k, v, g, beta, do, cu_seqlens=cu, use_qk_l2norm_in_kernel=True)  # noqa: E731
+    shared, copies = run(q, k), run(q.repeat_interleave(group, dim=2), k.repeat_interleave(group, dim=2))
+    for got, each in zip(shared[:2], copies[:2]):
+        want = each.double().unflatten(2, (HK, group)).sum(dim=3)
+        assert got.shape == want.shape and ((got.double() - want).abs() <= 2.0**-8 * want.abs() + 2.0**-20 * each.double().abs().amax()).all()
+    for got, want in zip(shared[2:5], copies[2:5]):
+        assert torch.equal(got, want)

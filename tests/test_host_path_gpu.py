@@ -347,7 +347,7 @@ def _training_forms():
         one = tuple(t[:1] for t in (q, k, v, g, beta))
         yield "delta_rule_bwd", {
             "plain": (op(use_qk_l2norm_in_kernel=True), (q, k, v, g, beta)), "no l2norm": (op(), (q, k, v, g, beta)), "ungated": (op(), (q, k, v)), "beta fp32": (op(), (q, k, v, g, beta.float())),
-            "states": (op(output_final_state=True, use_qk_l2norm_in_kernel=True), (q, k, v, g, beta, h)), "scale": (op(scale=0.3), (q, k, v, g, beta)), "blocks of one tensor": (op(), (*blocks, g, beta)),
+            "states": (op(output_final_state=True, use_qk_l2norm_in_kernel=True), (q, k, v, g, beta, h)), "scale": (op(scale=0.3), (q, k, v, g, beta)), "blocks of one tensor": (op(), (*blocks, g, beta)), "blocks, shared heads": (op(), (blocks[0][:, :, :1], blocks[1][:, :, :1], blocks[2], g, beta)),
             "strided q": (op(), (unit(r(2, 2, T, 64)).transpose(1, 2), k, v, g, beta)), "shared heads": (op(use_qk_l2norm_in_kernel=True), (q[:, :, :1], k[:, :, :1], v, g, beta)),
             "packed": (op(cu_seqlens=cu(0, 3, T), output_final_state=True), (*one, h)), "packed, empty ones": (op(cu_seqlens=cu(0, 0, 70, 70, T)), one), "packed, tokens left over": (op(cu_seqlens=cu(0, 70, T - 9)), one),
             "packed, int64 prefix": (op(cu_seqlens=cu(0, 3, T).long()), one), "padded": (op(cu_seqlens=cu(0, 70, 70 + T), left_padded=True), (q, k, v, g, beta)), "fp32": (op(), tuple(t.float() for t in (q, k, v, g, beta))),
