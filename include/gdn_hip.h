@@ -535,6 +535,14 @@ typedef struct gdn_gate_bwd_args {
 int gdn_gates_bwd(const gdn_gate_bwd_args *args, void *stream);
 
 /*
+ * gdn_causal_conv1d_fwd and gdn_gates_fwd (of the same dtype) in one launch: what the layer does in front of the operator,
+ * module.py:168-183.  mask (or NULL): a padding mask [B, S] of integers as in gdn_padding_mask, of at most 64 rows and with conv->mask NULL; the
+ * convolution is masked with it (where B > 1 and S > 1, depthwise_causal_convolution.py:28-37) and prefix becomes the prefix sums of its rows' sums.
+ */
+int gdn_layer_front(const gdn_conv_args *conv, const gdn_gate_args *gates, const void *mask, int element_bytes, int64_t stride_b,
+                    int64_t stride_s, int32_t *prefix, void *stream);
+
+/*
  * What the layer does to the operator's output before the output projection, one pass:
  *   y = rmsnorm(o * silu(gate)) * weight   over the V columns of every (token, head)
  * gated_deltanet/module.py:238-242 (`o = o * silu(g)`, `o = self.o_norm(o)`), RMSNorm of

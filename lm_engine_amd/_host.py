@@ -21,7 +21,7 @@ MODULE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "gdn_host
 _BOUND = ("gdn_layer_step", "gdn_layer_step_tiles", "gdn_causal_conv1d_fwd", "gdn_gates_fwd", "gdn_gated_rmsnorm_fwd",
           "gdn_recurrent_fwd", "gdn_chunk_fwd", "gdn_workspace_bytes", "gdn_chunk_fwd_is_one_launch", "gdn_chunk_bwd_sweeps",
           "gdn_chunk_bwd_sweeps_workspace_bytes", "gdn_chunk_bwd_local", "gdn_causal_conv1d_bwd", "gdn_gates_bwd",
-          "gdn_gated_rmsnorm_bwd", "gdn_column_sums", "gdn_fold_heads")  # fmt: skip
+          "gdn_gated_rmsnorm_bwd", "gdn_column_sums", "gdn_fold_heads", "gdn_layer_front")  # fmt: skip
 
 # device index -> hipStream_t of the calling thread's current stream (a torch build without GPU support has no such function,
 # nor a device tensor that would lead here)

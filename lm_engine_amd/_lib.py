@@ -62,6 +62,7 @@ EXPORTED_SYMBOLS = (
     "gdn_gated_rmsnorm_bwd",
     "gdn_column_sums",
     "gdn_fold_heads",
+    "gdn_layer_front",
     "gdn_padding_mask",
     "gdn_layer_step",
     "gdn_layer_step_tiles",
@@ -285,6 +286,9 @@ def load_library() -> ctypes.CDLL:
     lib.gdn_column_sums.restype = ctypes.c_int
     lib.gdn_fold_heads.argtypes = [ctypes.c_void_p] * 4 + [ctypes.c_int64, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_void_p]
     lib.gdn_fold_heads.restype = ctypes.c_int
+    lib.gdn_layer_front.argtypes = [ctypes.POINTER(GdnConvArgs), ctypes.POINTER(GdnGateArgs), ctypes.c_void_p, ctypes.c_int, ctypes.c_int64,
+                                    ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p]  # fmt: skip
+    lib.gdn_layer_front.restype = ctypes.c_int
     lib.gdn_gated_rmsnorm_fwd.argtypes = [ctypes.POINTER(GdnNormArgs), ctypes.c_void_p]
     lib.gdn_gated_rmsnorm_fwd.restype = ctypes.c_int
 

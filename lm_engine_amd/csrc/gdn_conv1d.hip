@@ -15,11 +15,13 @@
 #include <type_traits>
 
 #include "gdn_common.h"
+#include "gdn_elementwise.h"
 
 namespace gdn {
 
 constexpr int CONV_THREADS = 256;
 constexpr int CONV_TOKENS = 16;  // tokens per thread of a large batch (measured: 16 beats 32, 64, 128; more workgroups in flight)
+constexpr int FRONT_MASK_ROWS = 64;  // of an integer mask in the layer's front
 constexpr int CONV_TOKENS_SHORT = 4;  // and of one whose waves would leave compute units idle (launch_conv)
 
 struct ConvParams {
@@ -32,6 +34,14 @@ struct ConvParams {
     void* final_state;
     int64_t x_stride_b, x_stride_s, y_stride_b, y_stride_s;
     int B, S, C;
+    // The layer's front (gdn_layer_front): the launch's first plane of workgroups forms the gates, and its first workgroup the
+    // prefix sums of an integer mask, which the convolution then reads itself.  As launches of their own, mask, convolution and
+    // gates waited for each other: a padded prefill of 6 x 1500 tokens, 8 / 16 heads, K = V = 128 125.5 -> 116.8 us (6.5 + 33.4 + 4.2 |
+    // 35.4 us of kernels), a prompt of 777 tokens, 2 heads, K = 256, V = 512 50.3 -> 47.9 (7.1 + 4.1 | 6.5).
+    int front = 0;         // 1: there is such a plane
+    int mask_bytes = 0;    // element size of the integer mask; 0: `mask`, in the activations' type, if any
+    GateParams gates = {};
+    MaskParams ints = {};
 };
 
 template <typename T>
@@ -65,10 +75,22 @@ __device__ __forceinline__ void load_contiguous(const void* base, int64_t first,
 // MASK: the rows are multiplied by the padding mask on the way in and out.  A wave's TOKENS + KS - 1 mask values are one load, a
 // value per lane, read out per row: as a load for every row and every output row they stood between the loads of x (6 x 1500
 // tokens, 4096 channels, bf16: 33.7 -> 28.3 us a call, 29.3 without a mask; 8 x 4096 tokens, 2048 channels: 58.0 -> 54.3, 51.3).
+// Five waves per SIMD: at the 98 registers that the compiler takes unasked it is four (the masked convolution above 39.7 us).
 template <typename T, typename WT, int KS, bool SILU, int TOKENS, bool MASK>
-__global__ __launch_bounds__(CONV_THREADS) void causal_conv1d_kernel(const ConvParams p) {
+__global__ __launch_bounds__(CONV_THREADS, 5) void causal_conv1d_kernel(const ConvParams p) {
     constexpr int VEC = ConvVec<T>::N;
     typedef typename ConvVec<T>::type vec_t;
+    if ((int)blockIdx.z < p.front) {
+        __shared__ int32_t s_sum[FRONT_MASK_ROWS];
+        const int64_t group = (int64_t)blockIdx.y * gridDim.x + blockIdx.x, groups = (int64_t)gridDim.x * gridDim.y;
+        if (group == 0 && p.mask_bytes != 0) {
+            if (p.mask_bytes == 8) padding_mask<CONV_THREADS, int64_t, void>(p.ints, s_sum);
+            else if (p.mask_bytes == 4) padding_mask<CONV_THREADS, int32_t, void>(p.ints, s_sum);
+            else padding_mask<CONV_THREADS, uint8_t, void>(p.ints, s_sum);
+        }
+        for (int64_t i = group * CONV_THREADS + threadIdx.x; i < p.gates.tokens * p.gates.H; i += groups * CONV_THREADS) gates_at<T>(p.gates, i);
+        return;
+    }
 
     // a workgroup covers 64 channel vectors x (4 waves x TOKENS tokens): the halo rows of a wave are the
     // last rows of the wave before it, read on the same CU at about the same time
@@ -78,7 +100,7 @@ __global__ __launch_bounds__(CONV_THREADS) void causal_conv1d_kernel(const ConvP
     } else {
         if (c0 >= p.C) return;
     }
-    const int b = blockIdx.z;
+    const int b = (int)blockIdx.z - p.front;
     // (the same token in every lane of a wave)
     const int s_begin = (blockIdx.y * (CONV_THREADS / WAVE) + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE)) * TOKENS;
     if (s_begin >= p.S) return;
@@ -91,7 +113,13 @@ __global__ __launch_bounds__(CONV_THREADS) void causal_conv1d_kernel(const ConvP
     float mask_of_lane = 0.f;
     if constexpr (MASK) {
         const int s = s_begin - (KS - 1) + (int)(threadIdx.x % WAVE);
-        if (s >= 0 && s < s_end) mask_of_lane = (float)(reinterpret_cast<const T*>(p.mask) + (int64_t)b * p.S)[s];
+        if (s >= 0 && s < s_end) {
+            const int64_t at = b * p.ints.stride_b + s * p.ints.stride_s;
+            if (p.mask_bytes == 0) mask_of_lane = (float)(reinterpret_cast<const T*>(p.mask) + (int64_t)b * p.S)[s];
+            else if (p.mask_bytes == 8) mask_of_lane = (float)(T)(float)reinterpret_cast<const int64_t*>(p.ints.mask)[at];
+            else if (p.mask_bytes == 4) mask_of_lane = (float)(T)(float)reinterpret_cast<const int32_t*>(p.ints.mask)[at];
+            else mask_of_lane = (float)(T)(float)reinterpret_cast<const uint8_t*>(p.ints.mask)[at];
+        }
     }
     auto mask_at = [&](int s) {
         return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mask_of_lane), s - s_begin + (KS - 1)));
@@ -204,13 +232,15 @@ __global__ __launch_bounds__(CONV_THREADS) void causal_conv1d_kernel(const ConvP
 template <typename T, typename WT, int KS, int TOKENS>
 static void launch_conv_ks(const ConvParams& p, bool silu, hipStream_t stream) {
     constexpr int SPAN = (CONV_THREADS / WAVE) * TOKENS;  // tokens per workgroup
-    const dim3 grid((p.C / ConvVec<T>::N + WAVE - 1) / WAVE, (p.S + SPAN - 1) / SPAN, p.B);
+    const dim3 grid((p.C / ConvVec<T>::N + WAVE - 1) / WAVE, (p.S + SPAN - 1) / SPAN, p.B + p.front);
+    // the integer mask of a single row, or of single tokens, is for the prefix sums alone, as in the convolution by itself
+    const bool masked = p.mask != nullptr || (p.mask_bytes != 0 && p.B > 1 && p.S > 1);
     auto launch = [&](auto silu_tag, auto mask_tag) {
         hipLaunchKernelGGL((causal_conv1d_kernel<T, WT, KS, decltype(silu_tag)::value, TOKENS, decltype(mask_tag)::value>), grid, dim3(CONV_THREADS), 0, stream, p);
     };
-    if (silu && p.mask != nullptr) launch(std::true_type{}, std::true_type{});
+    if (silu && masked) launch(std::true_type{}, std::true_type{});
     else if (silu) launch(std::true_type{}, std::false_type{});
-    else if (p.mask != nullptr) launch(std::false_type{}, std::true_type{});
+    else if (masked) launch(std::false_type{}, std::true_type{});
     else launch(std::false_type{}, std::false_type{});
 }
 
@@ -239,9 +269,7 @@ static int launch_conv(const ConvParams& p, int kernel_size, bool silu, hipStrea
 
 namespace {
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) % 16) == 0; }
-}  // namespace
-
-extern "C" int gdn_causal_conv1d_fwd(const gdn_conv_args* a, void* stream) {
+int conv_args_status(const gdn_conv_args* a) {
     if (a == nullptr || a->x == nullptr || a->y == nullptr || a->weight == nullptr) return GDN_ERR_NULL;
     if (a->B <= 0 || a->S <= 0 || a->C <= 0) return GDN_ERR_SHAPE;
     if (a->kernel_size < 2 || a->kernel_size > 4) return GDN_ERR_UNSUPPORTED;
@@ -258,16 +286,50 @@ extern "C" int gdn_causal_conv1d_fwd(const gdn_conv_args* a, void* stream) {
     if (a->x_stride_s < a->C || a->y_stride_s < a->C) return GDN_ERR_SHAPE;
     if (!aligned16(a->x) || !aligned16(a->y) || !aligned16(a->weight) || (a->bias && !aligned16(a->bias))) return GDN_ERR_ALIGN;
     if (a->x == a->y) return GDN_ERR_SHAPE;  // neighbouring token blocks re-read rows of x
+    return GDN_OK;
+}
 
+gdn::ConvParams conv_params(const gdn_conv_args* a) {
     gdn::ConvParams p;
     p.x = a->x, p.weight = a->weight, p.bias = a->bias, p.input_state = a->input_state, p.mask = a->mask;
     p.y = a->y, p.final_state = a->final_state;
     p.x_stride_b = a->x_stride_b, p.x_stride_s = a->x_stride_s;
     p.y_stride_b = a->y_stride_b, p.y_stride_s = a->y_stride_s;
     p.B = a->B, p.S = a->S, p.C = a->C;
+    return p;
+}
+
+int launch(const gdn_conv_args* a, const gdn::ConvParams& p, void* stream) {
     const bool silu = a->activation == GDN_ACT_SILU;
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (a->dtype == GDN_BF16 && a->w_dtype == GDN_BF16) return gdn::launch_conv<gdn::bf16_t, gdn::bf16_t>(p, a->kernel_size, silu, st);
     if (a->dtype == GDN_BF16) return gdn::launch_conv<gdn::bf16_t, float>(p, a->kernel_size, silu, st);
     return gdn::launch_conv<float, float>(p, a->kernel_size, silu, st);
+}
+}  // namespace
+
+extern "C" int gdn_causal_conv1d_fwd(const gdn_conv_args* a, void* stream) {
+    const int status = conv_args_status(a);
+    return status != GDN_OK ? status : launch(a, conv_params(a), stream);
+}
+
+extern "C" int gdn_layer_front(const gdn_conv_args* a, const gdn_gate_args* gates, const void* mask, int element_bytes, int64_t stride_b,
+                               int64_t stride_s, int32_t* prefix, void* stream) {
+    if (const int status = conv_args_status(a); status != GDN_OK) return status;
+    if (gates == nullptr || !gates->a || !gates->b || !gates->A_log || !gates->dt_bias || !gates->g || !gates->beta) return GDN_ERR_NULL;
+    if (gates->tokens <= 0 || gates->H <= 0 || gates->a_stride < gates->H || gates->b_stride < gates->H) return GDN_ERR_SHAPE;
+    if (gates->dtype != a->dtype || a->B >= 65535) return GDN_ERR_UNSUPPORTED;
+    gdn::ConvParams p = conv_params(a);
+    p.front = 1;
+    p.gates.a = gates->a, p.gates.b = gates->b, p.gates.A_log = gates->A_log, p.gates.dt_bias = gates->dt_bias, p.gates.g = gates->g, p.gates.beta = gates->beta;
+    p.gates.a_stride = gates->a_stride, p.gates.b_stride = gates->b_stride, p.gates.tokens = gates->tokens, p.gates.H = gates->H, p.gates.beta_scale = gates->beta_scale;
+    if (mask != nullptr) {
+        if (prefix == nullptr || a->mask != nullptr) return GDN_ERR_NULL;
+        if (element_bytes != 1 && element_bytes != 4 && element_bytes != 8) return GDN_ERR_UNSUPPORTED;
+        if (a->B > gdn::FRONT_MASK_ROWS || stride_b < 0 || stride_s < 0) return GDN_ERR_SHAPE;
+        if (reinterpret_cast<uintptr_t>(mask) % element_bytes != 0 || reinterpret_cast<uintptr_t>(prefix) % 4 != 0) return GDN_ERR_ALIGN;
+        p.mask_bytes = element_bytes;
+        p.ints.mask = mask, p.ints.stride_b = stride_b, p.ints.stride_s = stride_s, p.ints.prefix = prefix, p.ints.B = a->B, p.ints.S = a->S;
+    }
+    return launch(a, p, stream);
 }

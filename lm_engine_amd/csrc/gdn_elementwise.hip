@@ -8,37 +8,14 @@
 // activations; epilogue 3 elements (o and gate in, y out) per (token, head, column).
 
 #include "gdn_common.h"
+#include "gdn_elementwise.h"
 
 namespace gdn {
-
-struct GateParams {
-    const void* a;
-    const void* b;
-    const float* A_log;
-    const float* dt_bias;
-    float* g;
-    void* beta;
-    int64_t a_stride, b_stride;
-    int64_t tokens;
-    int H;
-    float beta_scale;
-};
-
-// F.softplus with its default threshold: x for x > 20, log1p(exp(x)) otherwise
-__device__ __forceinline__ float softplus(float x) { return x > 20.f ? x : log1pf(__expf(x)); }
 
 template <typename T>
 __global__ __launch_bounds__(256) void gates_kernel(const GateParams p) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= p.tokens * p.H) return;
-    const int64_t t = idx / p.H;
-    const int h = (int)(idx % p.H);
-    const float a = (float)reinterpret_cast<const T*>(p.a)[t * p.a_stride + h];
-    const float b = (float)reinterpret_cast<const T*>(p.b)[t * p.b_stride + h];
-    p.g[idx] = -expf(p.A_log[h]) * softplus(a + p.dt_bias[h]);
-    // sigmoid in fp32, rounded to the activation dtype, then scaled in that dtype like `b.sigmoid() * 2`
-    const T s = (T)(1.f / (1.f + expf(-b)));
-    reinterpret_cast<T*>(p.beta)[idx] = (T)((float)s * p.beta_scale);
+    if (idx < p.tokens * p.H) gates_at<T>(p, idx);
 }
 
 // Backward of the gates: with z = a + dt_bias, rate = -exp(A_log), s = sigmoid(b)
@@ -400,55 +377,12 @@ __global__ __launch_bounds__(256) void fold_heads_kernel(const FoldParams p) {
 // int32 prefix sums of its rows' sums [B + 1].  One workgroup, whose waves share the rows between them: bound by the launch and
 // one trip through memory.  As conversion, row sums, prefix sum, pad and copies it was six launches (6 x 1500 tokens, 8 / 16 heads,
 // K = V = 128: 145 -> 127 us for the layer's prefill); torch's kernels are the better ones where a workgroup would read for long.
-constexpr int MASK_THREADS = 1024, MASK_WAVES = MASK_THREADS / WAVE;
-
-struct MaskParams {
-    const void* mask;
-    int64_t stride_b, stride_s;
-    void* out;
-    int32_t* prefix;
-    int B, S;
-};
+constexpr int MASK_THREADS = 1024;
 
 template <typename I, typename T>
 __global__ __launch_bounds__(MASK_THREADS) void padding_mask_kernel(const MaskParams p) {
     __shared__ int32_t s_sum[GDN_MASK_MAX_ROWS];
-    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
-    for (int b = threadIdx.x; b < p.B; b += MASK_THREADS) s_sum[b] = 0;
-    __syncthreads();
-    const int parts = p.B < MASK_WAVES ? MASK_WAVES / p.B : 1;  // waves per row
-    const int per = ((p.S + parts - 1) / parts + WAVE - 1) / WAVE * WAVE;
-    for (int unit = wave; unit < p.B * parts; unit += MASK_WAVES) {
-        const int b = unit / parts, begin = (unit % parts) * per, end = min(begin + per, p.S);
-        const I* const row = reinterpret_cast<const I*>(p.mask) + b * p.stride_b;
-        T* const out = reinterpret_cast<T*>(p.out) + (int64_t)b * p.S;
-        int32_t sum = 0;
-#pragma unroll 4
-        for (int s = begin + lane; s < end; s += WAVE) {
-            const I x = row[s * p.stride_s];
-            out[s] = (T)(float)x;
-            sum = (int32_t)((uint32_t)sum + (uint32_t)x);
-        }
-#pragma unroll
-        for (int off = WAVE / 2; off >= 1; off >>= 1) sum = (int32_t)((uint32_t)sum + (uint32_t)__shfl_xor(sum, off, WAVE));
-        if (lane == 0) atomicAdd(&s_sum[b], sum);
-    }
-    __syncthreads();
-    if (wave == 0) {  // prefix sums, 64 rows at a time
-        int32_t before = 0;
-        for (int b0 = 0; b0 < p.B; b0 += WAVE) {
-            int32_t x = b0 + lane < p.B ? s_sum[b0 + lane] : 0;
-#pragma unroll
-            for (int off = 1; off < WAVE; off <<= 1) {
-                const int32_t y = __shfl_up(x, off, WAVE);
-                if (lane >= off) x = (int32_t)((uint32_t)x + (uint32_t)y);
-            }
-            x = (int32_t)((uint32_t)x + (uint32_t)before);
-            if (b0 + lane < p.B) p.prefix[b0 + lane + 1] = x;
-            before = __shfl(x, WAVE - 1, WAVE);
-        }
-        if (lane == 0) p.prefix[0] = 0;
-    }
+    padding_mask<MASK_THREADS, I, T>(p, s_sum);
 }
 
 template <typename I>

@@ -39,6 +39,7 @@ decltype(&gdn_gates_bwd) gates_bwd_fn = nullptr;
 decltype(&gdn_gated_rmsnorm_bwd) norm_bwd_fn = nullptr;
 decltype(&gdn_column_sums) column_sums_fn = nullptr;
 decltype(&gdn_fold_heads) fold_heads_fn = nullptr;
+decltype(&gdn_layer_front) layer_front_fn = nullptr;
 PyObject* check_status = nullptr;  // _lib.check_status: raises what a status stands for
 
 // bind(check_status, addresses...)
@@ -46,7 +47,7 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n) {
     void** slots[] = {(void**)&layer_step_fn, (void**)&layer_step_tiles_fn, (void**)&conv_fn, (void**)&gates_fn, (void**)&norm_fn,
                       (void**)&recurrent_fn, (void**)&chunk_fn, (void**)&workspace_bytes_fn, (void**)&one_launch_fn,
                       (void**)&sweeps_fn, (void**)&sweeps_workspace_fn, (void**)&local_fn, (void**)&conv_bwd_fn, (void**)&gates_bwd_fn,
-                      (void**)&norm_bwd_fn, (void**)&column_sums_fn, (void**)&fold_heads_fn};
+                      (void**)&norm_bwd_fn, (void**)&column_sums_fn, (void**)&fold_heads_fn, (void**)&layer_front_fn};
     constexpr Py_ssize_t count = sizeof(slots) / sizeof(slots[0]);
     if (n != count + 1) return PyErr_Format(PyExc_TypeError, "bind takes a function and %zd addresses, got %zd arguments", count, n);
     for (Py_ssize_t i = 0; i < count; i++) {
@@ -248,6 +249,28 @@ PyObject* layer_step(PyObject*, PyObject* const* args, Py_ssize_t n) {
     });
 }
 
+// the convolution's arguments, but for its mask and results: (batch, tokens, channels, taps)
+struct ConvOperands {
+    gdn_conv_args s{};
+    int64_t B, S, C, ks;
+    ConvOperands(const at::Tensor& x, const at::Tensor& weight, const at::Tensor* bias, const at::Tensor* state, PyObject* activation) {
+        s.dtype = code_of(x), s.w_dtype = code_of(weight);
+        need(x.dim() == 3 && x.stride(2) == 1 && (s.dtype == GDN_BF16 || s.w_dtype == GDN_F32));
+        B = x.size(0), S = x.size(1), C = x.size(2), ks = taps_of(weight, C);
+        need(B > 0 && S > 0);
+        if (bias != nullptr) need(bias->scalar_type() == weight.scalar_type() && bias->dim() == 1 && bias->size(0) == C && bias->is_contiguous());
+        if (state != nullptr) need(state->scalar_type() == x.scalar_type() && state->sizes() == at::IntArrayRef({B, C, ks - 1}) && state->is_contiguous());
+        s.x = ptr(x), s.weight = ptr(weight), s.bias = ptr(bias), s.input_state = ptr(state);
+        s.x_stride_b = x.stride(0), s.x_stride_s = x.stride(1), s.y_stride_b = S * C, s.y_stride_s = C;
+        s.B = size32(B), s.S = size32(S), s.C = size32(C), s.kernel_size = (int32_t)ks;
+        s.activation = (int32_t)integer(activation);
+    }
+    void results(const at::Tensor& x, bool output_state, at::Tensor& y, at::Tensor& final_state) {
+        y = fresh(x, {B, S, C}), s.y = ptr(y);
+        if (output_state) final_state = fresh(x, {B, C, ks - 1}), s.final_state = ptr(final_state);
+    }
+};
+
 // conv(stream, x, weight, bias, input_state, mask, output_state, activation) -> (y, final_state or None)
 PyObject* conv(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return fast_path(n, 8, [&]() -> PyObject* {
@@ -255,33 +278,37 @@ PyObject* conv(PyObject*, PyObject* const* args, Py_ssize_t n) {
         void* const stream = stream_of(args[0]);
         const at::Tensor &x = operand(args[1]), &weight = operand(args[2]);
         const at::Tensor *bias = operand.optional(args[3]), *state = operand.optional(args[4]), *mask = operand.optional(args[5]);
-        gdn_conv_args s{};
-        s.dtype = code_of(x), s.w_dtype = code_of(weight);
-        need(x.dim() == 3 && x.stride(2) == 1 && (s.dtype == GDN_BF16 || s.w_dtype == GDN_F32));
-        const int64_t B = x.size(0), S = x.size(1), C = x.size(2), ks = taps_of(weight, C);
-        need(B > 0 && S > 0);
-        if (bias != nullptr) need(bias->scalar_type() == weight.scalar_type() && bias->dim() == 1 && bias->size(0) == C && bias->is_contiguous());
-        if (state != nullptr) need(state->scalar_type() == x.scalar_type() && state->sizes() == at::IntArrayRef({B, C, ks - 1}) && state->is_contiguous());
+        ConvOperands c(x, weight, bias, state, args[7]);
         at::Tensor kept_mask;
         bool masked = false;
         if (mask != nullptr) need(mask->dim() == 2);
         if (mask != nullptr && mask->size(0) > 1 && mask->size(1) > 1) {
-            need(mask->size(0) == B && mask->size(1) == S);
+            need(mask->size(0) == c.B && mask->size(1) == c.S);
             masked = true;
         }
         const bool output_state = truth(args[6]);
         at::Tensor y, final_state;
         without_interpreter_lock([&] {
-            if (masked) kept_mask = mask->to(x.scalar_type()).contiguous(), s.mask = ptr(kept_mask);
-            y = fresh(x, {B, S, C});
-            if (output_state) final_state = fresh(x, {B, C, ks - 1}), s.final_state = ptr(final_state);
+            if (masked) kept_mask = mask->to(x.scalar_type()).contiguous(), c.s.mask = ptr(kept_mask);
+            c.results(x, output_state, y, final_state);
         });
-        s.x = ptr(x), s.weight = ptr(weight), s.bias = ptr(bias), s.input_state = ptr(state), s.y = ptr(y);
-        s.x_stride_b = x.stride(0), s.x_stride_s = x.stride(1), s.y_stride_b = S * C, s.y_stride_s = C;
-        s.B = size32(B), s.S = size32(S), s.C = size32(C), s.kernel_size = (int32_t)ks;
-        s.activation = (int32_t)integer(args[7]);
-        return launch("gdn_causal_conv1d_fwd", pack_results({y, final_state}), [&] { return conv_fn(&s, stream); });
+        return launch("gdn_causal_conv1d_fwd", pack_results({y, final_state}), [&] { return conv_fn(&c.s, stream); });
     });
+}
+
+// the gates' arguments, but for their results
+gdn_gate_args gate_args(const at::Tensor& a, const at::Tensor& b, const at::Tensor& A_log, const at::Tensor& dt_bias, PyObject* beta_scale) {
+    gdn_gate_args s{};
+    s.dtype = code_of(a);
+    need(a.dim() >= 2 && b.scalar_type() == a.scalar_type() && b.sizes() == a.sizes() && a.numel() > 0);
+    const int64_t H = a.size(-1);
+    const at::Tensor* decay[] = {&A_log, &dt_bias};
+    for (const at::Tensor* t : decay) need(t->scalar_type() == at::kFloat && t->dim() == 1 && t->size(0) == H && t->is_contiguous());
+    s.a_stride = row_stride(a, H), s.b_stride = row_stride(b, H);
+    s.tokens = a.numel() / H, s.H = size32(H);
+    s.a = ptr(a), s.b = ptr(b), s.A_log = static_cast<const float*>(ptr(A_log)), s.dt_bias = static_cast<const float*>(ptr(dt_bias));
+    s.beta_scale = (float)number(beta_scale);
+    return s;
 }
 
 // gates(stream, a, b, A_log, dt_bias, beta_scale) -> (g, beta)
@@ -290,19 +317,46 @@ PyObject* gates(PyObject*, PyObject* const* args, Py_ssize_t n) {
         Operands operand;
         void* const stream = stream_of(args[0]);
         const at::Tensor &a = operand(args[1]), &b = operand(args[2]), &A_log = operand(args[3]), &dt_bias = operand(args[4]);
-        gdn_gate_args s{};
-        s.dtype = code_of(a);
-        need(a.dim() >= 2 && b.scalar_type() == a.scalar_type() && b.sizes() == a.sizes() && a.numel() > 0);
-        const int64_t H = a.size(-1);
-        const at::Tensor* decay[] = {&A_log, &dt_bias};
-        for (const at::Tensor* t : decay) need(t->scalar_type() == at::kFloat && t->dim() == 1 && t->size(0) == H && t->is_contiguous());
-        s.a_stride = row_stride(a, H), s.b_stride = row_stride(b, H);
-        s.tokens = a.numel() / H, s.H = size32(H);
+        gdn_gate_args s = gate_args(a, b, A_log, dt_bias, args[5]);
         at::Tensor g, beta;
         without_interpreter_lock([&] { g = fresh_f32(a, a.sizes()), beta = fresh(a, a.sizes()); });
-        s.a = ptr(a), s.b = ptr(b), s.A_log = static_cast<const float*>(ptr(A_log)), s.dt_bias = static_cast<const float*>(ptr(dt_bias));
-        s.g = static_cast<float*>(ptr(g)), s.beta = ptr(beta), s.beta_scale = (float)number(args[5]);
+        s.g = static_cast<float*>(ptr(g)), s.beta = ptr(beta);
         return launch("gdn_gates_fwd", pack_results({g, beta}), [&] { return gates_fn(&s, stream); });
+    });
+}
+
+// layer_front(stream, qkv, weight, bias, input_state, mask, output_state, activation, a, b, A_log, dt_bias, beta_scale)
+//   -> (y, final_state or None, g, beta, prefix sums of the mask's rows or None)
+// The convolution and the gates in one launch.  mask: [B, S] of integers or None.
+PyObject* layer_front(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    return fast_path(n, 13, [&]() -> PyObject* {
+        Operands operand;
+        void* const stream = stream_of(args[0]);
+        const at::Tensor &x = operand(args[1]), &weight = operand(args[2]), &a = operand(args[8]), &b = operand(args[9]), &A_log = operand(args[10]), &dt_bias = operand(args[11]);
+        const at::Tensor *bias = operand.optional(args[3]), *state = operand.optional(args[4]), *mask = operand.optional(args[5]);
+        ConvOperands c(x, weight, bias, state, args[7]);
+        gdn_gate_args s = gate_args(a, b, A_log, dt_bias, args[12]);
+        need(s.dtype == c.s.dtype);
+        int element_bytes = 0;
+        if (mask != nullptr) {
+            // (the masks that _one_launch_mask takes, layer_ops.py)
+            need(mask->dim() == 2 && mask->size(0) == c.B && mask->size(1) == c.S && c.B <= 64 && c.B * c.S <= 1 << 16);
+            const at::ScalarType type = mask->scalar_type();
+            need(type == at::kLong || type == at::kInt || type == at::kByte || type == at::kBool);
+            element_bytes = (int)mask->element_size();
+        }
+        const bool output_state = truth(args[6]);
+        at::Tensor y, final_state, g, beta, prefix;
+        without_interpreter_lock([&] {
+            c.results(x, output_state, y, final_state);
+            g = fresh_f32(a, a.sizes()), beta = fresh(a, a.sizes());
+            if (mask != nullptr) prefix = at::empty({c.B + 1}, x.options().dtype(at::kInt));
+        });
+        s.g = static_cast<float*>(ptr(g)), s.beta = ptr(beta);
+        return launch("gdn_layer_front", pack_results({y, final_state, g, beta, prefix}), [&] {
+            return layer_front_fn(&c.s, &s, ptr(mask), element_bytes, mask == nullptr ? 0 : mask->stride(0), mask == nullptr ? 0 : mask->stride(1),
+                                  prefix.defined() ? static_cast<int32_t*>(ptr(prefix)) : nullptr, stream);
+        });
     });
 }
 
@@ -665,6 +719,7 @@ PyMethodDef methods[] = {
     {"layer_step", (PyCFunction)(void (*)())layer_step, METH_FASTCALL, "gdn_layer_step"},
     {"conv", (PyCFunction)(void (*)())conv, METH_FASTCALL, "gdn_causal_conv1d_fwd"},
     {"gates", (PyCFunction)(void (*)())gates, METH_FASTCALL, "gdn_gates_fwd"},
+    {"layer_front", (PyCFunction)(void (*)())layer_front, METH_FASTCALL, "gdn_layer_front"},
     {"norm", (PyCFunction)(void (*)())norm, METH_FASTCALL, "gdn_gated_rmsnorm_fwd"},
     {"delta_rule", (PyCFunction)(void (*)())delta_rule, METH_FASTCALL, "gdn_chunk_fwd or gdn_recurrent_fwd"},
     {"delta_rule_bwd", (PyCFunction)(void (*)())delta_rule_bwd, METH_FASTCALL, "gdn_chunk_bwd_sweeps, gdn_chunk_bwd_local"},

@@ -104,13 +104,20 @@ def gated_deltanet_mixing(
             o, conv_state, h = step
             return o, (conv_state, h)
 
-    cu_seqlens = None
-    if (attention_mask is not None and attention_mask.dim() == 2 and attention_mask.shape == (B, S) and attention_mask.device == qkv.device
-            and is_kernel_allowed(Kernel.gated_delta_rule) and not torch.compiler.is_compiling()):  # fmt: skip
-        attention_mask, cu_seqlens = padding_mask(attention_mask, qkv.dtype)
-
-    qkv, conv_state = depthwise_causal_convolution(qkv, conv_weight, conv_bias, conv_state, attention_mask, use_cache,
-                                                   conv_activation)  # fmt: skip
+    front = cu_seqlens = None
+    if (qkv.is_cuda and conv_activation in _IN_KERNEL_ACTIVATIONS and is_kernel_allowed(Kernel.gated_delta_rule)
+            and not torch.compiler.is_compiling()):  # fmt: skip
+        # convolution, gates and the mask's prefix sums in one launch, where the operands are the usual ones
+        front = host().layer_front(raw_stream(qkv.get_device()), qkv, conv_weight, conv_bias, conv_state, attention_mask, use_cache,
+                                   _IN_KERNEL_ACTIVATIONS[conv_activation], a, b, A_log, dt_bias, 2.0 if allow_neg_eigval else 1.0)  # fmt: skip
+    if front is not None:
+        qkv, conv_state, g, beta, cu_seqlens = front
+    else:
+        if (attention_mask is not None and attention_mask.dim() == 2 and attention_mask.shape == (B, S) and attention_mask.device == qkv.device
+                and is_kernel_allowed(Kernel.gated_delta_rule) and not torch.compiler.is_compiling()):  # fmt: skip
+            attention_mask, cu_seqlens = padding_mask(attention_mask, qkv.dtype)
+        qkv, conv_state = depthwise_causal_convolution(qkv, conv_weight, conv_bias, conv_state, attention_mask, use_cache,
+                                                       conv_activation)  # fmt: skip
     if torch.is_grad_enabled() and qkv.requires_grad and not torch.compiler.is_compiling():
         q, k, v = _SplitChannels.apply(qkv, num_k_heads, num_v_heads, k_head_dim, v_head_dim)
     else:
@@ -121,7 +128,8 @@ def gated_deltanet_mixing(
     # grouped value attention (num_v_heads > num_k_heads): the operator reads head h / (num_v_heads / num_k_heads) of q
     # and k for value head h, so the reference's repeat_interleave copies (module.py:175-177) are not made
 
-    g, beta = delta_rule_gates(a, b, A_log, dt_bias, allow_neg_eigval)
+    if front is None:
+        g, beta = delta_rule_gates(a, b, A_log, dt_bias, allow_neg_eigval)
 
     if attention_mask is not None and cu_seqlens is None:  # (a captured graph; what is no mask of this batch the convolution has refused)
         seqlens = attention_mask.sum(dim=-1, dtype=torch.int32)  # sequence_packing.py:18-22

@@ -383,3 +383,48 @@ def test_backward_passes_end_as_they_do_without_the_native_path(monkeypatch):
                 differ.append((name, form))
     torch.cuda.synchronize()
     assert not differ, differ
+
+
+@pytest.mark.parametrize("S, dtype", [(2, BF16), (70, BF16), (130, torch.float32), (1100, BF16)])
+@pytest.mark.parametrize("B", [1, 3])
+def test_the_layers_front_in_one_launch_gives_the_bits_of_its_steps(B, S, dtype, monkeypatch):
+    """Convolution, gates and the mask's prefix sums: short and long walks over the tokens, integer masks of every type and layout, a
+    single row (whose mask the convolution does not apply), rows without a token, and what is refused."""
+    from lm_engine_amd import layer
+
+    x = _layer_operands(B, S)
+    x = {n: t.to(dtype) if isinstance(t, torch.Tensor) and t.dtype == BF16 else t for n, t in x.items()}
+    wide = torch.randn(B, S, 2 + 2 + 128, generator=torch.Generator().manual_seed(5)).to(dtype).cuda()
+    state = torch.randn(B, 384, 3, generator=torch.Generator().manual_seed(6)).to(dtype).cuda()
+    lengths = torch.tensor([S, 0, S // 2][:B])
+    mask = (torch.arange(S)[None] >= S - lengths[:, None]).cuda()
+    forms = {
+        "no mask": {}, "cache": dict(cache=(None, None)), "carried": dict(cache=(state, None)), "slices": dict(a=wide[..., :2], b=wide[..., 2:4], gate=wide[..., 4:]),
+        "int64": dict(attention_mask=mask.long()), "int32": dict(attention_mask=mask.int()), "uint8": dict(attention_mask=mask.byte()), "bool": dict(attention_mask=mask),
+        "transposed mask": dict(attention_mask=mask.long().t().contiguous().t(), cache=(None, None)), "expanded mask": dict(attention_mask=torch.ones(B, 1, dtype=torch.int32).cuda().expand(B, S)),
+        "mask in fp32": dict(attention_mask=mask.float()), "mask of another shape": dict(attention_mask=mask[:, 1:].long()), "a of fewer tokens": dict(a=x["a"][:, 1:], b=x["b"][:, 1:]),
+        "2-D weight": dict(conv_weight=x["conv_weight"][:, 0]), "3 taps": dict(conv_weight=x["conv_weight"][..., 1:].contiguous()), "no activation": dict(conv_activation=None), "negative eigenvalues": dict(allow_neg_eigval=True),
+    }  # fmt: skip
+    for form, over in forms.items():
+        print(f"case: layer's front, {B} x {S}, {form}", flush=True)
+        outcomes = []
+        for on in (True, False):
+            took = []
+
+            class Path:
+                def __getattr__(self, name):
+                    return getattr(_host.host(), name)
+
+                def layer_front(self, *args, on=on, took=took):
+                    result = _host.host().layer_front(*args) if on else None
+                    took.append(result is not None)
+                    return result
+
+            with monkeypatch.context() as m:
+                m.setattr(layer, "host", Path)
+                outcomes.append(_outcome(lambda: lm_engine_amd.gated_deltanet_mixing(**{**x, **over})))
+            assert form == "a of fewer tokens" or took == [on and form not in ("mask in fp32", "mask of another shape")]
+        (one, steps), refused = outcomes, isinstance(outcomes[0], tuple)
+        assert refused == isinstance(steps, tuple) and len(one) == len(steps)
+        assert one == steps if refused else all((p is None and q is None) or torch.equal(p, q) for p, q in zip(one, steps)), form
+    torch.cuda.synchronize()
