@@ -15,9 +15,15 @@
 // head's output: those stores are device-scope (the tiles sit on different XCDs) and complete before the ticket is drawn, and
 // the state's stores are issued behind it, so nobody waits for them.
 //
-// Bound by the launch and one trip through memory for small batches (one sequence x 16 heads, K = V = 128: 6 us on the GPU,
-// 11 us a step with the host's work, where the four launches took 86), by the state's bytes for large ones (200 sequences x 16
-// heads: 75 us for 422 MB = 5.6 TB/s).
+// Bound by the launch and one trip through memory for small batches (one sequence x 16 heads, K = V = 128: 11 us a step with the
+// host's work, where the four launches took 86), by the state's bytes for large ones.  The trip is one because everything is asked
+// for before anything is waited for: the convolution's operands four channels to a thread in wide loads, then the state, and no
+// branch stands between a load and the next one that holds its use.  Loaded one channel and tap at a time, each parameter converted
+// under the branch on its dtype, the kernel waited for memory about twenty times in a row before it asked for the state, and a
+// workgroup issued four times as many loads; the last tile of a head did the same with the norm's weight.  Steps with the state
+// read from and written to different memory, before and after: 53 sequences x 2 heads, K = 256, V = 512 29.3 -> 22.6 us (a copy of
+// as many bytes takes 21.7), 32 of them 18.1 -> 13.3, 128 of them 59.8 -> 51.7 (5.2 TB/s); x 16 heads, K = V = 128, 53 sequences
+// 26.1 -> 22.5, 128 of them 53.3 -> 46.4 (5.8 TB/s).
 
 #include <type_traits>
 
@@ -42,9 +48,41 @@ struct LayerStepParams {
     float beta_scale, scale, eps;
 };
 
-__device__ __forceinline__ float load_scalar(const void* p, int dtype, int64_t i) {
-    return dtype == GDN_BF16 ? (float)reinterpret_cast<const bf16_t*>(p)[i] : reinterpret_cast<const float*>(p)[i];
+// What a workgroup reads beside its state is loaded as it lies in memory and converted where it is used: a conversion that follows
+// its load under a branch (on a dtype, on an optional input) is a wait for memory each time, one after the other.
+__device__ __forceinline__ uint32_t load_bits(const void* p, int dtype, int64_t i) {
+    return dtype == GDN_BF16 ? reinterpret_cast<const uint16_t*>(p)[i] : reinterpret_cast<const uint32_t*>(p)[i];
 }
+__device__ __forceinline__ float float_of_bits(uint32_t x, int dtype) { return __builtin_bit_cast(float, dtype == GDN_BF16 ? x << 16 : x); }
+
+// N fours of parameters that follow each other, in either dtype: fp32 two to a pair of words, bf16 four to one, in the first N
+template <int N>
+struct Parameters {
+    typedef __attribute__((ext_vector_type(2))) uint32_t pair_t;
+    typedef __attribute__((ext_vector_type(2), aligned(2))) uint32_t unaligned_t;  // (an offset of one element is allowed)
+    pair_t pairs[2 * N];
+    __device__ __forceinline__ void clear() {
+#pragma unroll
+        for (int j = 0; j < 2 * N; j++) pairs[j] = pair_t{0, 0};
+    }
+    __device__ __forceinline__ void load(const void* p, bool bf16, int64_t at) {
+        const unaligned_t* from = reinterpret_cast<const unaligned_t*>(reinterpret_cast<const char*>(p) + at * (bf16 ? 2 : 4));
+#pragma unroll
+        for (int j = 0; j < N; j++) pairs[j] = from[j];
+        if (!bf16) {
+#pragma unroll
+            for (int j = N; j < 2 * N; j++) pairs[j] = from[j];
+        }
+    }
+    __device__ __forceinline__ float get(int i, bool bf16) const {
+        const uint32_t word = pairs[i / 4][i / 2 % 2];
+        return __builtin_bit_cast(float, bf16 ? (i % 2 == 0 ? word << 16 : word & 0xffff0000u) : pairs[i / 2][i % 2]);
+    }
+};
+
+// four activations; aligned as one is
+template <typename T>
+using Quad = __attribute__((ext_vector_type(4), aligned(sizeof(T)))) T;
 
 __device__ __forceinline__ float silu_of(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 
@@ -53,9 +91,9 @@ __global__ __launch_bounds__(4 * BV) void layer_step_kernel(const LayerStepParam
     typedef StepTile<K, BV> Tile;
     constexpr int RPT = Tile::RPT, KPL = K / WAVE, THREADS = Tile::THREADS;
     constexpr int CH = 2 * K + BV;                        // channels of the convolution: q | k | v
-    constexpr int PER = (CH + THREADS - 1) / THREADS;     // of them per thread
+    constexpr int PER = (CH / 4 + THREADS - 1) / THREADS;  // of them per thread, in fours
     __shared__ __attribute__((aligned(16))) float s_red[Tile::WAVES][2][BV];
-    __shared__ __attribute__((aligned(16))) float s_x[CH];
+    __shared__ __attribute__((aligned(16))) float s_x[CH], s_gate[BV], s_weight[BV];
     const Tile tile(s_red);
     const int tid = threadIdx.x;
     const int v0 = blockIdx.x * BV, h = blockIdx.y, hk = h / p.group;
@@ -63,56 +101,77 @@ __global__ __launch_bounds__(4 * BV) void layer_step_kernel(const LayerStepParam
 
     // ---- everything this token needs is asked for ahead of the state ----
     const T* x = reinterpret_cast<const T*>(p.qkv) + b * p.qkv_stride_b;
-    T cur[PER], hist[PER][KS - 1];
-    float w[PER][KS], bias[PER];
+    const bool w_bf16 = p.conv_w_dtype == GDN_BF16;
+    Quad<T> cur[PER], hist[PER][KS - 1];  // element (KS - 1) c + j of a thread's hist, KS c + j of its w: channel c, tap j
+    Parameters<KS> w[PER];
+    Parameters<1> bias[PER];
     int64_t channel[PER];
 #pragma unroll
     for (int i = 0; i < PER; i++) {
-        const int c = min(tid + i * THREADS, CH - 1);  // (the last round's spare threads repeat the last channel)
+        const int c = 4 * (tid + i * THREADS);
         channel[i] = c < K ? (int64_t)hk * K + c : c < 2 * K ? (int64_t)(p.HK + hk) * K + c - K : 2 * (int64_t)p.HK * K + (int64_t)h * p.V + v0 + c - 2 * K;
-        cur[i] = x[channel[i]];
+        cur[i] = Quad<T>{}, bias[i].clear(), w[i].clear();
 #pragma unroll
-        for (int j = 0; j < KS - 1; j++)
-            hist[i][j] = p.conv_state == nullptr ? (T)0.f : reinterpret_cast<const T*>(p.conv_state)[(b * C + channel[i]) * (KS - 1) + j];
+        for (int j = 0; j < KS - 1; j++) hist[i][j] = Quad<T>{};
+        if (c < CH) {
+            cur[i] = *reinterpret_cast<const Quad<T>*>(x + channel[i]);
+            if (p.conv_state != nullptr) {
+                const Quad<T>* from = reinterpret_cast<const Quad<T>*>(reinterpret_cast<const T*>(p.conv_state) + (b * C + channel[i]) * (KS - 1));
 #pragma unroll
-        for (int j = 0; j < KS; j++) w[i][j] = load_scalar(p.conv_weight, p.conv_w_dtype, channel[i] * KS + j);
-        bias[i] = p.conv_bias == nullptr ? 0.f : load_scalar(p.conv_bias, p.conv_w_dtype, channel[i]);
+                for (int j = 0; j < KS - 1; j++) hist[i][j] = from[j];
+            }
+            w[i].load(p.conv_weight, w_bf16, channel[i] * KS);
+            if (p.conv_bias != nullptr) bias[i].load(p.conv_bias, w_bf16, channel[i]);
+        }
     }
+    // the gate and the norm's weight of the tile's columns, one per thread; those that end up with the output take them out of LDS
+    const bool has_column = tid < BV;
     const bool writes_out = tile.rg == 0;  // the lanes that end up with the tile's output: the first BV / 4 of wave 0
-    float gate[4], norm_w[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        gate[e] = 0.f, norm_w[e] = 1.f;
-        if (writes_out && p.gate != nullptr) gate[e] = (float)reinterpret_cast<const T*>(p.gate)[b * p.gate_stride_b + (int64_t)h * p.V + v0 + 4 * tile.lv + e];
-        if (writes_out && p.norm_weight != nullptr) norm_w[e] = load_scalar(p.norm_weight, p.norm_w_dtype, v0 + 4 * tile.lv + e);
-    }
+    constexpr int DTYPE = std::is_same<T, bf16_t>::value ? GDN_BF16 : GDN_F32;
+    uint32_t gate_in = 0, weight_in = 0;
+    if (has_column && p.gate != nullptr) gate_in = load_bits(p.gate, DTYPE, b * p.gate_stride_b + (int64_t)h * p.V + v0 + tid);
+    if (has_column && p.norm_weight != nullptr) weight_in = load_bits(p.norm_weight, p.norm_w_dtype, v0 + tid);
     const float a_in = (float)reinterpret_cast<const T*>(p.a)[b * p.a_stride_b + h];
     const float b_in = (float)reinterpret_cast<const T*>(p.b)[b * p.b_stride_b + h];
     const float A_log = p.A_log[h], dt_bias = p.dt_bias[h];
 
     const int64_t state_off = (b * p.H + h) * K * p.V + v0;
     f32x4 S[RPT];
-    tile.load(S, p.h0 == nullptr ? nullptr : p.h0 + state_off, p.V);
+    tile.load_ahead(S, p.h0 == nullptr ? nullptr : p.h0 + state_off, p.V);
+
+    asm volatile("" : "+v"(gate_in), "+v"(weight_in));  // (or their conversion moves up behind their loads)
 
     // ---- convolution and gates ----
 #pragma unroll
     for (int i = 0; i < PER; i++) {
-        const int c = tid + i * THREADS;
-        float acc = bias[i] + w[i][KS - 1] * (float)cur[i];
+        const int c = 4 * (tid + i * THREADS);
+        if (c >= CH) continue;
+        f32x4 y;
 #pragma unroll
-        for (int j = 0; j < KS - 1; j++) acc += w[i][j] * (float)hist[i][j];
-        if (p.silu) acc = silu_of(acc);
+        for (int e = 0; e < 4; e++) {
+            float acc = bias[i].get(e, w_bf16) + w[i].get(KS * e + KS - 1, w_bf16) * (float)cur[i][e];
+#pragma unroll
+            for (int j = 0; j < KS - 1; j++) acc += w[i].get(KS * e + j, w_bf16) * (float)hist[i][((KS - 1) * e + j) / 4][((KS - 1) * e + j) % 4];
+            if (p.silu) acc = silu_of(acc);
+            y[e] = (float)(T)acc;
+        }
+        *reinterpret_cast<f32x4*>(&s_x[c]) = y;
         // q and k are written by one of the workgroups that compute them
-        if (c < CH) {
-            s_x[c] = (float)(T)acc;
-            if (c >= 2 * K || (blockIdx.x == 0 && h % p.group == 0)) {
-                T* out = reinterpret_cast<T*>(p.conv_state_out) + (b * C + channel[i]) * (KS - 1);
+        if (c >= 2 * K || (blockIdx.x == 0 && h % p.group == 0)) {
+            T* out = reinterpret_cast<T*>(p.conv_state_out) + (b * C + channel[i]) * (KS - 1);
 #pragma unroll
-                for (int j = 0; j + 1 < KS - 1; j++) out[j] = hist[i][j + 1];
-                out[KS - 2] = cur[i];
+            for (int n = 0; n < KS - 1; n++) {
+                Quad<T> taps;
+#pragma unroll
+                for (int m = 0; m < 4; m++) {
+                    const int e = (4 * n + m) / (KS - 1), j = (4 * n + m) % (KS - 1), from = (KS - 1) * e + j + 1;
+                    taps[m] = j == KS - 2 ? cur[i][e] : hist[i][from / 4][from % 4];
+                }
+                reinterpret_cast<Quad<T>*>(out)[n] = taps;
             }
         }
     }
+    if (has_column) s_gate[tid] = float_of_bits(gate_in, DTYPE), s_weight[tid] = p.norm_weight == nullptr ? 1.f : float_of_bits(weight_in, p.norm_w_dtype);
     const float z = a_in + dt_bias;
     const float eg = expf(-expf(A_log) * (z > 20.f ? z : log1pf(__expf(z))));
     const float beta = (float)(T)((float)(T)(1.f / (1.f + expf(-b_in))) * p.beta_scale);
@@ -132,6 +191,7 @@ __global__ __launch_bounds__(4 * BV) void layer_step_kernel(const LayerStepParam
     const f32x4 vt = *reinterpret_cast<const f32x4*>(&s_x[2 * K + 4 * tile.lv]);
     f32x4 sk, sq, r, y;
     tile.contract(S, k, q, sk, sq);
+    const f32x4 gate = *reinterpret_cast<const f32x4*>(&s_gate[4 * tile.lv]), norm_w = *reinterpret_cast<const f32x4*>(&s_weight[4 * tile.lv]);
 #pragma unroll
     for (int c = 0; c < 4; c++) {
         r[c] = token_residual(vt[c], sk[c], eg, beta);
@@ -153,6 +213,9 @@ __global__ __launch_bounds__(4 * BV) void layer_step_kernel(const LayerStepParam
 #pragma unroll
                 for (int e = 0; e < 4; e++) __hip_atomic_store(row + v0 + 4 * tile.lv + e, y[e], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
+            uint32_t weight[8];  // V <= 512; whoever draws the last ticket needs them, at once
+#pragma unroll
+            for (int i = 0; i < 8; i++) weight[i] = p.norm_weight == nullptr ? 0 : load_bits(p.norm_weight, p.norm_w_dtype, min(tile.lane + 64 * i, p.V - 1));
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             int drawn = 0;
             int32_t* const ticket = p.tickets + b * p.H + h;
@@ -161,16 +224,17 @@ __global__ __launch_bounds__(4 * BV) void layer_step_kernel(const LayerStepParam
             if (drawn == (int)gridDim.x - 1) {  // all other tiles of this head have stored their part
                 float ss = 0.f, part[8];
 #pragma unroll
-                for (int i = 0; i < 8; i++) {  // V <= 512
-                    const int c = tile.lane + 64 * i;
-                    part[i] = c < p.V ? __hip_atomic_load(row + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.f;
+                for (int i = 0; i < 8; i++) part[i] = __hip_atomic_load(row + min(tile.lane + 64 * i, p.V - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    if (tile.lane + 64 * i >= p.V) part[i] = 0.f;
                     ss += part[i] * part[i];
                 }
                 const float scale = rsqrtf(wave_total(ss) / (float)p.V + p.eps);
 #pragma unroll
                 for (int i = 0; i < 8; i++) {
                     const int c = tile.lane + 64 * i;
-                    if (c < p.V) out[c] = (T)(part[i] * scale * (p.norm_weight == nullptr ? 1.f : load_scalar(p.norm_weight, p.norm_w_dtype, c)));
+                    if (c < p.V) out[c] = (T)(part[i] * scale * (p.norm_weight == nullptr ? 1.f : float_of_bits(weight[i], p.norm_w_dtype)));
                 }
                 if (tile.lane == 0) __hip_atomic_store(ticket, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
             }
@@ -187,12 +251,14 @@ __global__ __launch_bounds__(4 * BV) void layer_step_kernel(const LayerStepParam
 namespace {
 
 // Columns per workgroup.  A head of at most 128 columns is one tile and needs no ticket (one sequence x 16 heads, K = V = 128:
-// 6.0 us a launch, 9.1 and 10.0 with 64 and 32 columns and tickets).  Wider ones: 128 columns while that leaves every CU a
-// workgroup, else 64 (K = 256, V = 512, 2 heads, 32 | 64 | 128 columns: 2 sequences 13.9 | 12.6 | 12.9 us, 53 sequences 36.2 | 32.0 |
-// 30.3 us; the narrower the tile, the more often the convolution of q and k is repeated).
+// 6.0 us a launch, 9.1 and 10.0 with 64 and 32 columns and tickets).  Wider ones: 64 columns while that is at most one workgroup per
+// CU, else 128: the narrower the tile, the more often the convolution of q and k is repeated, and a second workgroup on some of the
+// CUs takes longer than a larger one on each (K = 256, V = 512, 2 heads, 64 | 128 columns: 2 sequences 8.3 | 8.6 us, 16 of them 10.7
+// | 11.1, 20 13.7 | 11.8, 24 14.6 | 12.7, 32 15.0 | 14.8, 53 27.8 | 25.5; K = 128, V = 256, 4 heads: 2 sequences 7.5 | 7.8, 16 of
+// them 9.2 | 8.8, 64 17.9 | 15.3; back to back in a graph).
 int step_tile_columns(int B, int H, int V) {
     if (V == 32 || V == 64 || V == 128) return V;
-    if (V % 128 == 0 && (int64_t)B * H * (V / 128) >= 256) return 128;
+    if (V % 128 == 0 && (int64_t)B * H * (V / 64) > 256) return 128;
     return V % 64 == 0 ? 64 : 32;
 }
 

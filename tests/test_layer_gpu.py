@@ -190,6 +190,34 @@ def test_one_launch_step_matches_the_chain_of_kernels(B, HK, HV, DK, DV, dtype, 
                 assert torch.equal(x, y), name
 
 
+# every kernel size, parameters in either dtype, with and without a bias; a convolution's state at an odd element gives the bits
+# of the same state at an even one
+@pytest.mark.parametrize("dtype, w_dtype", [(BF16, BF16), (BF16, torch.float32), (torch.float32, torch.float32)])
+@pytest.mark.parametrize("kernel_size, bias, HK, HV, DK, DV", [(2, True, 1, 2, 64, 32), (3, False, 2, 2, 256, 96), (3, True, 1, 2, 128, 256),
+                                                               (4, False, 1, 1, 256, 512), (4, True, 1, 1, 64, 128)])  # fmt: skip
+def test_one_launch_step_takes_parameters_and_states_as_they_lie(kernel_size, bias, HK, HV, DK, DV, dtype, w_dtype, monkeypatch):
+    B = 3
+    qkv, ab, p, (conv, h) = _step_operands(B, HK, HV, DK, DV, dtype, seed=kernel_size + DK)
+    p["conv_weight"] = p["conv_weight"][..., :kernel_size].contiguous().to(w_dtype)
+    p["conv_bias"], p["norm_weight"] = p["conv_bias"].to(w_dtype) if bias else None, p["norm_weight"].to(w_dtype)
+    conv = conv[..., : kernel_size - 1].contiguous()
+    odd = torch.empty(conv.numel() + 1, dtype=dtype, device="cuda")[1:].view(conv.shape)
+    odd.copy_(conv)
+    results = []
+    for step, state in ((True, conv), (True, odd), (False, conv)):
+        with monkeypatch.context() as m:
+            answers = _watched_host(m, step=step)
+            out, c = _mix_step(qkv, ab, p, HK, HV, DK, DV, (state, h))
+        assert [x is not None for x in answers] == [step], "the kernel under test did not run"
+        results.append((out, *c))
+    for name, x, y, z in zip(("out", "conv", "h"), *results):
+        assert torch.equal(x, y), name
+        if name == "out":  # (the order of the norm's V squares, as above)
+            assert rel_l2(x, z) <= (1e-3 if dtype == BF16 else 1e-6), rel_l2(x, z)
+        else:
+            assert torch.equal(x, z), name
+
+
 def test_one_launch_step_under_graph_capture(monkeypatch):
     answers = _watched_host(monkeypatch, step=True)
     HK, HV, DK, DV = 2, 2, 128, 256  # several workgroups per head: tickets in memory of the graph's own
