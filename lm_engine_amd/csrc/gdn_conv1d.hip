@@ -5,12 +5,15 @@
 // Bound: HBM.  Algorithmic bytes per (token, channel): one read of x and one write of y, i.e.
 // 2 * sizeof(element); weights, bias, state and mask are negligible.
 //
-// A thread owns 16 bytes of channels (8 bf16 / 4 fp32) and walks TOKENS consecutive tokens with
-// the kernel_size - 1 previous rows in registers, so inside a block every row of x is read once;
-// neighbouring token blocks share kernel_size - 1 rows of halo and are walked in opposite directions, so
-// that both read them at the same moment.  Lanes cover consecutive channel
-// vectors: every load and store of a wave is one contiguous row segment; the four waves of a
-// workgroup take consecutive token blocks of the same channels.
+// A thread owns 16 bytes of channels (8 bf16 / 4 fp32) of TOKENS consecutive tokens and asks for its TOKENS + kernel_size - 1 rows
+// of x at once, before anything is converted; neighbouring token blocks share kernel_size - 1 rows of halo and read them at the
+// same moment, out of one cache.  Lanes cover consecutive channel vectors: every load and store of a wave is one contiguous row
+// segment; the four waves of a workgroup take consecutive token blocks of the same channels.
+//
+// Walked row by row, with the window in registers, 16 tokens a thread were 16 trips to memory one after the other (the branches on
+// the sequence's ends held the use of every row next to its load).  Before and after, bf16, inputs from memory: 8 x 4096 tokens,
+// 2048 channels 54.5 -> 48.5 us (5.5 TB/s), 2 x 4096 21.5 -> 15.9, 4 x 4096, 6144 channels 86.4 -> 75.5, 777 tokens, 2048 channels
+// 5.7 -> 5.1; 6 x 1500, 4096 channels 29.1 both, masked 31.8 -> 31.4; fp32, 4 x 4096, 2048 channels 45.9 -> 43.5, 1 x 4096 19.3 -> 14.3.
 
 #include <type_traits>
 
@@ -20,9 +23,8 @@
 namespace gdn {
 
 constexpr int CONV_THREADS = 256;
-constexpr int CONV_TOKENS = 16;  // tokens per thread of a large batch (measured: 16 beats 32, 64, 128; more workgroups in flight)
 constexpr int FRONT_MASK_ROWS = 64;  // of an integer mask in the layer's front
-constexpr int CONV_TOKENS_SHORT = 4;  // and of one whose waves would leave compute units idle (launch_conv)
+constexpr int CONV_TOKENS_SHORT = 4;  // tokens per thread of a batch whose waves would leave compute units idle (launch_conv_ks)
 
 struct ConvParams {
     const void* x;
@@ -44,16 +46,19 @@ struct ConvParams {
     MaskParams ints = {};
 };
 
+// TOKENS per thread of other batches: more are more registers and fewer waves, fewer read more of the halo twice.  4 x 4096 tokens,
+// 6144 channels, bf16, 5 | 6 | 8 | 12 | 16 tokens: 76.2 | 76.2 | 75.5 | 77.9 | 95.0 us; masked, 5 x 700 tokens: 8 | 12 | 16 22.4 | 21.4 | 25.4;
+// fp32, 4 x 4096 tokens, 2048 channels, 4 | 5 | 6 | 8 | 12 | 24: 43.5 | 44.2 | 45.8 | 47.5 | 48.3 | 60.0; 1 x 4096 14.3 | 15.3 at 4 | 5.
 template <typename T>
 struct ConvVec;
 template <>
 struct ConvVec<bf16_t> {
-    static constexpr int N = 8;
+    static constexpr int N = 8, TOKENS = 8, TOKENS_MASKED = 12;
     typedef bf16x8 type;
 };
 template <>
 struct ConvVec<float> {
-    static constexpr int N = 4;
+    static constexpr int N = 4, TOKENS = CONV_TOKENS_SHORT, TOKENS_MASKED = CONV_TOKENS_SHORT;
     typedef f32x4 type;
 };
 
@@ -73,11 +78,10 @@ __device__ __forceinline__ void load_contiguous(const void* base, int64_t first,
 }
 
 // MASK: the rows are multiplied by the padding mask on the way in and out.  A wave's TOKENS + KS - 1 mask values are one load, a
-// value per lane, read out per row: as a load for every row and every output row they stood between the loads of x (6 x 1500
-// tokens, 4096 channels, bf16: 33.7 -> 28.3 us a call, 29.3 without a mask; 8 x 4096 tokens, 2048 channels: 58.0 -> 54.3, 51.3).
-// Five waves per SIMD: at the 98 registers that the compiler takes unasked it is four (the masked convolution above 39.7 us).
+// value per lane, read out per row: as a load for every row and every output row they stood between the loads of x.
+// Four waves per SIMD: 112 registers at bf16 and 8 tokens.  Held to five it spills (8 x 4096 tokens, 2048 channels: 86.8 us).
 template <typename T, typename WT, int KS, bool SILU, int TOKENS, bool MASK>
-__global__ __launch_bounds__(CONV_THREADS, 5) void causal_conv1d_kernel(const ConvParams p) {
+__global__ __launch_bounds__(CONV_THREADS, 4) void causal_conv1d_kernel(const ConvParams p) {
     constexpr int VEC = ConvVec<T>::N;
     typedef typename ConvVec<T>::type vec_t;
     if ((int)blockIdx.z < p.front) {
@@ -94,7 +98,8 @@ __global__ __launch_bounds__(CONV_THREADS, 5) void causal_conv1d_kernel(const Co
 
     // a workgroup covers 64 channel vectors x (4 waves x TOKENS tokens): the halo rows of a wave are the
     // last rows of the wave before it, read on the same CU at about the same time
-    int c0 = (blockIdx.x * WAVE + threadIdx.x % WAVE) * VEC;
+    const unsigned groups = (p.C / VEC + WAVE - 1) / WAVE;
+    int c0 = (blockIdx.x % groups * WAVE + threadIdx.x % WAVE) * VEC;
     if constexpr (MASK) {
         c0 = min(c0, p.C - VEC);  // every lane stays, as a holder of mask values: spare ones repeat the last channels, with the same results
     } else {
@@ -102,15 +107,37 @@ __global__ __launch_bounds__(CONV_THREADS, 5) void causal_conv1d_kernel(const Co
     }
     const int b = (int)blockIdx.z - p.front;
     // (the same token in every lane of a wave)
-    const int s_begin = (blockIdx.y * (CONV_THREADS / WAVE) + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE)) * TOKENS;
-    if (s_begin >= p.S) return;
-    const int s_end = min(s_begin + TOKENS, p.S);
+    const int64_t first = (int64_t)(blockIdx.x / groups * (CONV_THREADS / WAVE) + __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE)) * TOKENS;
+    if (first >= p.S) return;
+    const int s_begin = (int)first, s_end = min(p.S - s_begin, TOKENS) + s_begin;
 
+    // ---- everything is asked for before anything is used; rows before the sequence and past the walk's end: its nearest one ----
     const T* xb = reinterpret_cast<const T*>(p.x) + (int64_t)b * p.x_stride_b + c0;
     T* yb = reinterpret_cast<T*>(p.y) + (int64_t)b * p.y_stride_b + c0;
-    // lane l: mask of token s_begin - (KS - 1) + l (the halo's and this walk's; others are not asked for)
+    float wflat[VEC * KS], bias[VEC];  // wflat[e * KS + j]: tap j of channel c0 + e
+    load_contiguous<WT, VEC * KS>(p.weight, (int64_t)c0 * KS, wflat);
+    vec_t rows[TOKENS + KS - 1];  // row i: token s_begin - (KS - 1) + i
+#pragma unroll
+    for (int i = 0; i < TOKENS + KS - 1; i++)
+        rows[i] = *reinterpret_cast<const vec_t*>(xb + (int64_t)min(max(s_begin - (KS - 1) + i, 0), s_end - 1) * p.x_stride_s);
+    const T* state = p.input_state == nullptr ? nullptr : reinterpret_cast<const T*>(p.input_state) + ((int64_t)b * p.C + c0) * (KS - 1);
+    // row s of the carried state or of zeros, for the kernel_size - 1 rows before the sequence
+    auto state_row = [&](int s) {
+        vec_t row;
+#pragma unroll
+        for (int e = 0; e < VEC; e++) row[e] = state == nullptr ? (T)0.f : state[e * (KS - 1) + (KS - 1) + s];
+        return row;
+    };
+    if (s_begin == 0) {
+#pragma unroll
+        for (int i = 0; i < KS - 1; i++) rows[i] = state_row(i - (KS - 1));
+    }
+#pragma unroll
+    for (int e = 0; e < VEC; e++) bias[e] = 0.f;
+    if (p.bias != nullptr) load_contiguous<WT, VEC>(p.bias, c0, bias);
+    // lane l: mask of token s_begin - (KS - 1) + l (the halo's and this walk's; others are not asked for); rows before the sequence are taken as they are
     static_assert(TOKENS + KS - 1 <= WAVE, "a lane per mask value");
-    float mask_of_lane = 0.f;
+    float mask_of_lane = 1.f;
     if constexpr (MASK) {
         const int s = s_begin - (KS - 1) + (int)(threadIdx.x % WAVE);
         if (s >= 0 && s < s_end) {
@@ -125,36 +152,19 @@ __global__ __launch_bounds__(CONV_THREADS, 5) void causal_conv1d_kernel(const Co
         return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mask_of_lane), s - s_begin + (KS - 1)));
     };
 
-    float wflat[VEC * KS], bias[VEC];  // wflat[e * KS + j]: tap j of channel c0 + e
-    load_contiguous<WT, VEC * KS>(p.weight, (int64_t)c0 * KS, wflat);
+    float hist[KS - 1][VEC];  // hist[j]: (masked) row s - (KS - 1) + j
+    auto masked_row = [&](const vec_t& v, int s, float (&row)[VEC]) {
+        const float m = MASK ? mask_at(s) : 1.f;
 #pragma unroll
-    for (int e = 0; e < VEC; e++) bias[e] = 0.f;
-    if (p.bias != nullptr) load_contiguous<WT, VEC>(p.bias, c0, bias);
-
-    auto load_row = [&](int s, float (&row)[VEC]) {
-        const vec_t v = *reinterpret_cast<const vec_t*>(xb + (int64_t)s * p.x_stride_s);
-#pragma unroll
-        for (int e = 0; e < VEC; e++) row[e] = (float)v[e];
-        if constexpr (MASK) {
-            const float m = mask_at(s);
-#pragma unroll
-            for (int e = 0; e < VEC; e++) row[e] *= m;
-        }
+        for (int e = 0; e < VEC; e++) row[e] = MASK ? (float)v[e] * m : (float)v[e];
     };
-
-    // row s of the (masked) input for s >= 0, the carried state or zeros for the kernel_size - 1 rows before the sequence
-    auto load_any = [&](int s, float (&row)[VEC]) {
-        if (s >= 0) {
-            load_row(s, row);
-        } else {
 #pragma unroll
-            for (int e = 0; e < VEC; e++)
-                row[e] = p.input_state == nullptr
-                             ? 0.f
-                             : (float)reinterpret_cast<const T*>(p.input_state)[((int64_t)b * p.C + c0 + e) * (KS - 1) + (KS - 1) + s];
-        }
-    };
-    auto emit = [&](int s, const float (&cur)[VEC], const float (&hist)[KS - 1][VEC]) {  // hist[j] = row s - (KS - 1) + j
+    for (int j = 0; j < KS - 1; j++) masked_row(rows[j], s_begin - (KS - 1) + j, hist[j]);
+#pragma unroll
+    for (int i = 0; i < TOKENS; i++) {
+        const int s = s_begin + i;
+        float cur[VEC];
+        masked_row(rows[i + KS - 1], s, cur);
         const float m = MASK ? mask_at(s) : 1.f;
         vec_t out;
 #pragma unroll
@@ -164,104 +174,58 @@ __global__ __launch_bounds__(CONV_THREADS, 5) void causal_conv1d_kernel(const Co
             for (int j = 0; j < KS - 1; j++) acc += wflat[e * KS + j] * hist[j][e];
             if (SILU) acc = acc * __builtin_amdgcn_rcpf(1.f + __expf(-acc));  // x * sigmoid(x)
             out[e] = (T)(MASK ? acc * m : acc);
+#pragma unroll
+            for (int j = 0; j + 1 < KS - 1; j++) hist[j][e] = hist[j + 1][e];
+            hist[KS - 2][e] = cur[e];
         }
-        *reinterpret_cast<vec_t*>(yb + (int64_t)s * p.y_stride_s) = out;
-    };
+        if (s < s_end) *reinterpret_cast<vec_t*>(yb + (int64_t)s * p.y_stride_s) = out;
+    }
 
-    // Token blocks are walked in alternating directions: an even block from its last token down, an odd one
-    // from its first token up.  The kernel_size - 1 rows two neighbouring blocks have in common are then read
-    // by both at the same moment - at the start of both walks or at the end of both - and come out of the
-    // cache; walked the same way, the second reader comes a whole walk later and fetches them from memory
-    // again (measured: 19 % more bytes fetched than the input holds, 5 % this way; the kernel time did not
-    // change, it streams at the rate of a plain copy either way).
-    const bool downward = ((s_begin / TOKENS) & 1) == 0;
-    float hist[KS - 1][VEC];
-    if (!downward) {
+    // the last kernel_size - 1 (masked) inputs, for the next call: read once more, so that no row is picked by a number known at run time
+    if (p.final_state != nullptr && s_end == p.S) {
+        T* fs = reinterpret_cast<T*>(p.final_state) + ((int64_t)b * p.C + c0) * (KS - 1);
 #pragma unroll
-        for (int j = 0; j < KS - 1; j++) load_any(s_begin - (KS - 1) + j, hist[j]);
-#pragma unroll 8
-        for (int s = s_begin; s < s_end; s++) {
-            float cur[VEC];
-            load_row(s, cur);
-            emit(s, cur, hist);
+        for (int j = 0; j < KS - 1; j++) {
+            const int s = p.S - (KS - 1) + j;
+            float row[VEC];
+            if (s >= 0) masked_row(*reinterpret_cast<const vec_t*>(xb + (int64_t)s * p.x_stride_s), s, row);
+            else masked_row(state_row(s), s, row);
 #pragma unroll
-            for (int e = 0; e < VEC; e++) {
-#pragma unroll
-                for (int j = 0; j + 1 < KS - 1; j++) hist[j][e] = hist[j + 1][e];
-                hist[KS - 2][e] = cur[e];
-            }
-        }
-        if (p.final_state != nullptr && s_end == p.S) {
-            T* fs = reinterpret_cast<T*>(p.final_state) + ((int64_t)b * p.C + c0) * (KS - 1);
-#pragma unroll
-            for (int e = 0; e < VEC; e++)
-#pragma unroll
-                for (int j = 0; j < KS - 1; j++) fs[e * (KS - 1) + j] = (T)hist[j][e];
-        }
-    } else {
-        // cur = row s, hist[j] = row s - (KS - 1) + j; stepping down shifts the window the other way
-        float cur[VEC];
-        load_row(s_end - 1, cur);
-#pragma unroll
-        for (int j = 0; j < KS - 1; j++) load_any(s_end - 1 - (KS - 1) + j, hist[j]);
-        if (p.final_state != nullptr && s_end == p.S) {  // the last kernel_size - 1 inputs: hist[1..], cur
-            T* fs = reinterpret_cast<T*>(p.final_state) + ((int64_t)b * p.C + c0) * (KS - 1);
-#pragma unroll
-            for (int e = 0; e < VEC; e++) {
-#pragma unroll
-                for (int j = 0; j + 1 < KS - 1; j++) fs[e * (KS - 1) + j] = (T)hist[j + 1][e];
-                fs[e * (KS - 1) + KS - 2] = (T)cur[e];
-            }
-        }
-#pragma unroll 8
-        for (int s = s_end - 1; s >= s_begin; s--) {
-            emit(s, cur, hist);
-            float next[VEC] = {};  // row s - KS, the new oldest row of the window around s - 1
-            if (s > s_begin) load_any(s - KS, next);
-#pragma unroll
-            for (int e = 0; e < VEC; e++) {
-                cur[e] = hist[KS - 2][e];
-#pragma unroll
-                for (int j = KS - 2; j > 0; j--) hist[j][e] = hist[j - 1][e];
-                hist[0][e] = next[e];
-            }
+            for (int e = 0; e < VEC; e++) fs[e * (KS - 1) + j] = (T)row[e];
         }
     }
 }
 
-template <typename T, typename WT, int KS, int TOKENS>
+template <typename T, typename WT, int KS>
 static void launch_conv_ks(const ConvParams& p, bool silu, hipStream_t stream) {
-    constexpr int SPAN = (CONV_THREADS / WAVE) * TOKENS;  // tokens per workgroup
-    const dim3 grid((p.C / ConvVec<T>::N + WAVE - 1) / WAVE, (p.S + SPAN - 1) / SPAN, p.B + p.front);
+    const int64_t groups = (p.C / ConvVec<T>::N + WAVE - 1) / WAVE;
     // the integer mask of a single row, or of single tokens, is for the prefix sums alone, as in the convolution by itself
     const bool masked = p.mask != nullptr || (p.mask_bytes != 0 && p.B > 1 && p.S > 1);
-    auto launch = [&](auto silu_tag, auto mask_tag) {
+    auto launch = [&](auto silu_tag, auto mask_tag, auto tokens_tag) {
+        constexpr int TOKENS = decltype(tokens_tag)::value, SPAN = (CONV_THREADS / WAVE) * TOKENS;  // tokens per workgroup
+        const dim3 grid((unsigned)(groups * ((p.S + SPAN - 1) / SPAN)), 1, p.B + p.front);
         hipLaunchKernelGGL((causal_conv1d_kernel<T, WT, KS, decltype(silu_tag)::value, TOKENS, decltype(mask_tag)::value>), grid, dim3(CONV_THREADS), 0, stream, p);
     };
-    if (silu && masked) launch(std::true_type{}, std::true_type{});
-    else if (silu) launch(std::true_type{}, std::false_type{});
-    else if (masked) launch(std::false_type{}, std::true_type{});
-    else launch(std::false_type{}, std::false_type{});
+    auto launch_with = [&](auto tokens_tag, auto mask_tag) {
+        if (silu) launch(std::true_type{}, mask_tag, tokens_tag);
+        else launch(std::false_type{}, mask_tag, tokens_tag);
+    };
+    typedef std::integral_constant<int, CONV_TOKENS_SHORT> few_tokens;
+    // Under 1792 waves of 16 tokens (7 per compute unit) more workgroups count for more than the halo.  4 | 8 tokens a thread, bf16,
+    // inputs from memory: 200 waves 5.3 | 6.1 us, 1024 9.7 | 9.8, 2000 16.3 | 15.6 (C = 2048), 2028 17.0 | 15.6 (C = 6144), 4096 28.5 | 28.2,
+    // 8192 50.6 | 48.2; masked, 4 | 12: 1584 16.3 | 17.0, 4056 31.2 | 29.9.
+    const bool few = groups * ((p.S + 15) / 16) * p.B < 1792;
+    if (masked && few) launch_with(few_tokens{}, std::true_type{});
+    else if (masked) launch_with(std::integral_constant<int, ConvVec<T>::TOKENS_MASKED>{}, std::true_type{});
+    else if (few) launch_with(few_tokens{}, std::false_type{});
+    else launch_with(std::integral_constant<int, ConvVec<T>::TOKENS>{}, std::false_type{});
 }
 
 template <typename T, typename WT>
 static int launch_conv(const ConvParams& p, int kernel_size, bool silu, hipStream_t stream) {
-    const int64_t groups = (p.C / ConvVec<T>::N + WAVE - 1) / WAVE;
-    const int64_t waves = groups * ((p.S + CONV_TOKENS - 1) / CONV_TOKENS) * p.B;
-    // Under 2048 waves (8 per compute unit) a walk of 16 tokens is one latency after another with little beside it; above, the
-    // halo of 3 rows per block counts.  4 | 16 tokens a thread, bf16, inputs from memory: C = 2048, 200 waves 5.9 | 12.1 us,
-    // 1024 11.5 | 18.1, 2000 19.9 | 22.3, 2100 21.9 | 23.4, 3072 28.4 | 27.5, 8192 71.5 | 59.7; C = 6144, 2000 waves
-    // 20.2 | 21.2, 2100 22.4 | 22.4, 3072 28.9 | 25.0.  fp32 crosses at about the same place: C = 2048, 2100 17.9 | 19.8,
-    // 4096 28.1 | 26.3.
-    if (waves < 2048) {
-        if (kernel_size == 2) launch_conv_ks<T, WT, 2, CONV_TOKENS_SHORT>(p, silu, stream);
-        else if (kernel_size == 3) launch_conv_ks<T, WT, 3, CONV_TOKENS_SHORT>(p, silu, stream);
-        else launch_conv_ks<T, WT, 4, CONV_TOKENS_SHORT>(p, silu, stream);
-    } else {
-        if (kernel_size == 2) launch_conv_ks<T, WT, 2, CONV_TOKENS>(p, silu, stream);
-        else if (kernel_size == 3) launch_conv_ks<T, WT, 3, CONV_TOKENS>(p, silu, stream);
-        else launch_conv_ks<T, WT, 4, CONV_TOKENS>(p, silu, stream);
-    }
+    if (kernel_size == 2) launch_conv_ks<T, WT, 2>(p, silu, stream);
+    else if (kernel_size == 3) launch_conv_ks<T, WT, 3>(p, silu, stream);
+    else launch_conv_ks<T, WT, 4>(p, silu, stream);
     return (int)hipGetLastError();
 }
 
@@ -277,7 +241,7 @@ int conv_args_status(const gdn_conv_args* a) {
     if (a->w_dtype != GDN_BF16 && a->w_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
     if (a->dtype == GDN_F32 && a->w_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;  // weights as wide as the data
     if (a->activation != GDN_ACT_NONE && a->activation != GDN_ACT_SILU) return GDN_ERR_UNSUPPORTED;
-    if (a->B > 65535 || a->S / (gdn::CONV_TOKENS * (gdn::CONV_THREADS / gdn::WAVE)) >= 65535) return GDN_ERR_UNSUPPORTED;
+    if (a->B > 65535 || a->S / 64 >= 65535) return GDN_ERR_UNSUPPORTED;
     const int64_t vec = (a->dtype == GDN_BF16) ? 8 : 4;
     if (a->C % vec != 0) return GDN_ERR_UNSUPPORTED;
     const int64_t strides[] = {a->x_stride_b, a->x_stride_s, a->y_stride_b, a->y_stride_s};

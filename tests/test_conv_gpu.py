@@ -151,6 +151,21 @@ def test_long_walks_match_short_ones(dtype, masked):
         assert torch.equal(y1[0, first:].cpu().to(F64), y[row, first:]) and torch.equal(s1[0].cpu().to(F64), s[row])
 
 
+# the ends of a walk of 4, 8 and 12 tokens and one past each; sequences shorter than the window
+@pytest.mark.parametrize("dtype, w_dtype", [(BF16, BF16), (BF16, F32), (F32, F32)])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("ks, S", [(4, 1), (4, 2), (4, 3), (3, 4), (2, 5), (4, 7), (4, 8), (3, 9), (4, 11), (4, 12), (4, 13), (2, 16), (4, 25)])
+def test_walks_of_any_length_end_where_the_sequence_does(ks, S, masked, dtype, w_dtype):
+    """Enough rows to fill the device take the longer walks, a few of them the short one: the same bits, the oracle's values."""
+    x, w, b, st, m = _inputs(1800, S, 24, ks, dtype, seed=S + ks, state=True, mask=masked)
+    w, b = w.to(w_dtype), b.to(w_dtype)
+    run = lambda n: lm_engine_amd.depthwise_causal_convolution(  # noqa: E731
+        x[:n].cuda(), w.cuda(), b.cuda(), st[:n].cuda(), None if m is None else m[:n].cuda(), output_state=True)
+    (y, s), (y1, s1) = run(1800), run(5)
+    assert torch.equal(y[:5], y1) and torch.equal(s[:5], s1)
+    _check(x[:5], w, b, st[:5], None if m is None else m[:5], "silu", f"walks ks={ks} S={S}")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("C", [8, 144, 152, 512, 520])
 @pytest.mark.parametrize("S", [1, 15, 16, 17, 61])
