@@ -141,7 +141,7 @@ def test_rejected_arguments():
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("masked", [False, True])
 def test_long_walks_match_short_ones(dtype, masked):
-    """A batch that fills the device takes 16 tokens a thread, its rows one by one take 4: the same bits, the oracle's values."""
+    """A batch that fills the device takes longer walks, its rows one by one 4 tokens a thread: the same bits, the oracle's values."""
     x, w, b, st, m = _inputs(8, 4099, 64, 4, dtype, seed=5, state=True, mask=masked)
     y, s = _check(x, w, b, st, m, "silu", "long walks")
     for row in (0, 7):
