@@ -48,6 +48,7 @@ import torch
 from . import _lib
 from ._autograd import kernel_rows
 from ._host import host, raw_stream
+from .kernels import Kernel, is_kernel_allowed
 
 
 CHUNK = 64
@@ -355,11 +356,12 @@ def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm
         NC = max(1, -(-max(lens + [1]) // CHUNK))
         covers = sum(lens) == B * T
         sequences = (*ops.upload_int32((starts, lens), q.device), NC)
-    flags = (_lib.GDN_FLAG_L2NORM if l2norm else 0) | (_lib.GDN_FLAG_LEFT_PADDED if left_padded else 0)
-    grads = host().delta_rule_bwd(raw_stream(q.get_device()), q, k, v, g, beta, initial_state, cu_seqlens, do, dht, scale, flags,
-                                  *(sequences or (None, None, 0)), covers, joined)  # fmt: skip
-    if grads is not None:
-        return grads
+    if is_kernel_allowed(Kernel.gated_delta_rule):  # (else ops.chunk_bwd_sweeps refuses the call)
+        flags = (_lib.GDN_FLAG_L2NORM if l2norm else 0) | (_lib.GDN_FLAG_LEFT_PADDED if left_padded else 0)
+        grads = host().delta_rule_bwd(raw_stream(q.get_device()), q, k, v, g, beta, initial_state, cu_seqlens, do, dht, scale, flags,
+                                      *(sequences or (None, None, 0)), covers, joined)  # fmt: skip
+        if grads is not None:
+            return grads
     if cu_seqlens is None:
         NC = -(-T // CHUNK)
         if T % CHUNK != 0:

@@ -13,6 +13,7 @@ import pytest
 import torch
 
 import lm_engine_amd
+from lm_engine_amd.kernels import enable_kernels
 from oracle.gdn_backward_oracle import gated_delta_rule_grads_autograd
 
 from .helpers import assert_parity, max_abs, random_inputs, rel_l2
@@ -217,6 +218,15 @@ def test_chunk_bf16_left_padded_batch():
         _assert_grads(got, want, torch.bfloat16)
         for x in ("q", "k", "v", "g", "beta"):
             assert not leaves[x].grad[b, : T - n].any(), f"gradient of {x} at the padding"
+
+
+@pytest.mark.parametrize("V", [64, 96])
+def test_a_backward_with_the_kernel_switched_off_is_refused(V):
+    x, v = (torch.randn(1, 70, 2, n, generator=torch.Generator().manual_seed(3)).bfloat16().cuda().requires_grad_(True) for n in (64, V))
+    print(f"case: backward with the kernel switched off, V={V}", flush=True)
+    o, _ = lm_engine_amd.chunk_gated_delta_rule(x, x, v)
+    with enable_kernels([], reset=True), pytest.raises(RuntimeError, match="no other implementation"):
+        o.sum().backward()
 
 
 def test_ungated_without_beta():

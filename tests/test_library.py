@@ -285,6 +285,26 @@ def test_kernel_flag_registry_follows_the_reference_convention():
     assert is_kernel_allowed(Kernel.gated_delta_rule)
 
 
+def test_a_backward_under_a_switched_off_kernel_is_refused(monkeypatch):
+    """Of the operator, the gates and the gated norm: ahead of anything that the native host path would launch."""
+    from lm_engine_amd import backward, layer_ops
+
+    class NotAsked:
+        def __getattr__(self, name):
+            raise AssertionError(f"{name} was called")
+
+    for module in (backward, layer_ops):
+        monkeypatch.setattr(module, "host", NotAsked)
+    x, h = torch.zeros(1, 64, 2, 64, dtype=torch.bfloat16), torch.zeros(2)
+    a = x[..., 0]
+    rule = lambda: backward._backward_on_kernels(x, x, x, None, None, x, None, 1.0, None, False, None, False, False)  # noqa: E731
+    with enable_kernels([], reset=True):
+        for call in (rule, lambda: layer_ops._delta_rule_gates_backward(a, a, h, h, a, a, False),
+                     lambda: layer_ops._gated_rmsnorm_backward(x, None, None, None, x)):  # fmt: skip
+            with pytest.raises(RuntimeError, match="no other implementation"):
+                call()
+
+
 def test_fused_launch_flag_is_on_by_default_and_can_be_switched_off():
     fused = Kernel.gated_delta_rule_fused_launch
     assert is_kernel_allowed(fused)
