@@ -292,22 +292,25 @@ int gdn_chunk_fwd_saving_is_staged(const gdn_args *args, const gdn_chunk_saves *
  *                   gdn_chunk_bwd_prepare (Y at its even chunks, tokens reversed); or NULL and
  *     y_chunks      bf16 [chunks][64][V]: Y of chunk (n, h, c) with its tokens in reverse order, from gdn_chunk_bwd_sweeps, or as
  *                   the V~ that the mirror scan saved at its even chunks (save_every = 2, save_reverse, bf16 saves, no output)
- *     q_raw, k_raw, v_raw, dout_raw   the caller's bf16 q, k, v, dO, [N, NC * 64, H, D] with element strides
- * Outputs, in the caller's layout, contiguous: dq_out, dk_out [N, NC * 64, H, K] and dv_out [N, NC * 64, H, V]
- * (bf16; the gradients with respect to q and k themselves, through the scale and the normalisation), dg_out and
- * dbeta_out fp32 [N, NC * 64, H] (dg_out is the gradient with respect to g: the reverse prefix sum of the gradient
- * with respect to gamma inside the chunk).
+ *     q_raw, k_raw, v_raw, dout_raw   the caller's bf16 q, k, v, dO, [N, T, H, D] with element strides (q and k: H / n heads with
+ *                   GDN_LOCAL_SHARED_HEADS(n)); T = NC * 64, or T_rows with seq_start or GDN_LOCAL_RAGGED_ROWS
+ * Outputs, in the caller's layout, contiguous (or column blocks of one array, out_stride_t): dq_out, dk_out [N, T, H, K] and dv_out
+ * [N, T, H, V] (bf16; the gradients with respect to q and k themselves, through the scale and the normalisation; one per head of v
+ * where value heads share those of q and k), dg_out fp32 and dbeta_out fp32, or bf16 with GDN_LOCAL_DBETA_BF16, [N, T, H] (dg_out is
+ * the gradient with respect to g: the reverse prefix sum of the gradient with respect to gamma inside the chunk).
  * K = 64, 128 or 256 and V a multiple of 64 (GDN_ERR_UNSUPPORTED otherwise).  Counterpart upstream: the chunk-local
  * kernels of fla's backward of chunk_gated_delta_rule, reached from gated_deltanet/module.py:197-209 under autograd.
  */
-#define GDN_LOCAL_DBETA_BF16 0x100 /* in saves_dtype: dbeta_out is bf16 */
-/* in saves_dtype: n heads of v share a head of q and k (n divides H): q_raw and k_raw have H / n heads; dq_out and dk_out keep a
- * gradient per head of v, [N, T, H, K] contiguous whatever out_stride_t, for gdn_fold_heads */
+/* Added to saves_dtype, where a caller that sets none of them gets what it always got: */
+#define GDN_LOCAL_DBETA_BF16 0x100  /* dbeta_out is bf16 */
+#define GDN_LOCAL_RAGGED_ROWS 0x200 /* seq_start NULL: the rows have T_rows tokens, (NC - 1) * 64 < T_rows <= NC * 64 (GDN_ERR_SHAPE otherwise) */
+/* n heads of v share a head of q and k (n divides H): q_raw and k_raw have H / n heads; dq_out and dk_out keep a gradient per head
+ * of v, [N, T, H, K] contiguous whatever out_stride_t, for gdn_fold_heads */
 #define GDN_LOCAL_SHARED_HEADS(n) ((n) << 16)
 typedef struct gdn_chunk_local_args {
     const void *v_new, *states, *dstates;
     const float *gamma, *beta, *rq, *rk;
-    int32_t saves_dtype; /* gdn_dtype of v_new and states, | GDN_LOCAL_DBETA_BF16 | GDN_LOCAL_SHARED_HEADS(n) */
+    int32_t saves_dtype; /* gdn_dtype of v_new and states, | GDN_LOCAL_.. */
     float scale;
     int64_t chunks;
     int32_t K, V;
@@ -322,8 +325,8 @@ typedef struct gdn_chunk_local_args {
     int64_t dout_stride_b, dout_stride_t, dout_stride_h;
     /* packed or left-padded batches: sequence n starts at token seq_start[n] (a flat index over the
      * rows of the caller's tensors, T_rows tokens per row) and has seq_len[n] tokens; its chunks c * 64 >= seq_len[n]
-     * are skipped, tokens past its end are not written.  NULL: sequence n is row n, of T_rows tokens where
-     * (NC - 1) * 64 < T_rows < NC * 64, else of NC * 64. */
+     * are skipped, tokens past its end are not written.  NULL: sequence n is row n, of NC * 64 tokens, or of T_rows with
+     * GDN_LOCAL_RAGGED_ROWS (T_rows is not read otherwise). */
     const int32_t *seq_start, *seq_len;
     int32_t T_rows;
     int32_t dstates_dtype; /* gdn_dtype of dstates */

@@ -233,7 +233,7 @@ int gdn_chunk_bwd_local(const gdn_chunk_local_args* a, void* stream) {
         if (x == nullptr) return GDN_ERR_NULL;
         else if (!aligned(x, 16)) return GDN_ERR_ALIGN;
     const int saves_dtype = a->saves_dtype & 0xff, group = a->saves_dtype >> 16;
-    if ((a->saves_dtype & 0xff00) != 0 && (a->saves_dtype & 0xff00) != GDN_LOCAL_DBETA_BF16) return GDN_ERR_UNSUPPORTED;
+    if ((a->saves_dtype & 0xff00 & ~(GDN_LOCAL_DBETA_BF16 | GDN_LOCAL_RAGGED_ROWS)) != 0) return GDN_ERR_UNSUPPORTED;
     if (group < 0 || (group > 0 && a->H % group != 0)) return GDN_ERR_SHAPE;
     if (saves_dtype != GDN_BF16 && saves_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
     if (a->dstates_dtype != GDN_BF16 && a->dstates_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
@@ -242,6 +242,7 @@ int gdn_chunk_bwd_local(const gdn_chunk_local_args* a, void* stream) {
     if (a->out_stride_t % 8 != 0) return GDN_ERR_ALIGN;
     if (a->H <= 0 || a->NC <= 0 || a->chunks % ((int64_t)a->H * a->NC) != 0) return GDN_ERR_SHAPE;
     if (a->seq_start != nullptr && (a->seq_len == nullptr || a->T_rows <= 0)) return GDN_ERR_SHAPE;
+    if ((a->saves_dtype & GDN_LOCAL_RAGGED_ROWS) != 0 && (a->seq_start != nullptr || a->T_rows <= 0 || (a->T_rows - 1) / 64 != a->NC - 1)) return GDN_ERR_SHAPE;
     const int64_t raw_strides[] = {a->q_stride_b, a->q_stride_t, a->q_stride_h, a->k_stride_b, a->k_stride_t, a->k_stride_h,
                                    a->v_stride_b, a->v_stride_t, a->v_stride_h, a->dout_stride_b, a->dout_stride_t, a->dout_stride_h};
     for (int64_t st : raw_strides)

@@ -1308,7 +1308,7 @@ int launch_chunk_bwd_local(const gdn_chunk_local_args& a, hipStream_t stream) {
     p.v_stride_b = a.v_stride_b, p.v_stride_t = a.v_stride_t, p.v_stride_h = a.v_stride_h;
     p.d_stride_b = a.dout_stride_b, p.d_stride_t = a.dout_stride_t, p.d_stride_h = a.dout_stride_h;
     p.seq_start = a.seq_start, p.seq_len = a.seq_len;
-    p.T_rows = a.seq_start != nullptr || (a.T_rows > (a.NC - 1) * C && a.T_rows < a.NC * C) ? a.T_rows : a.NC * C;
+    p.T_rows = a.seq_start != nullptr || (a.saves_dtype & GDN_LOCAL_RAGGED_ROWS) != 0 ? a.T_rows : a.NC * C;
     const dim3 grid((unsigned)a.chunks), block(BWD_THREADS);
     auto launch = [&](auto kc) {
         constexpr int KK = decltype(kc)::value;

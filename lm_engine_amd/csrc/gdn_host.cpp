@@ -591,6 +591,7 @@ PyObject* delta_rule_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
         l.dq_out = ptr(dq), l.dk_out = ptr(dk), l.dv_out = ptr(dv), l.dg_out = static_cast<float*>(ptr(dg)), l.dbeta_out = static_cast<float*>(ptr(dbeta));
         if (!(s.flags & GDN_FLAG_L2NORM)) l.rq = l.rk = nullptr;
         if (dbeta.scalar_type() == at::kBFloat16) l.saves_dtype |= GDN_LOCAL_DBETA_BF16;
+        if (seq_start == nullptr) l.saves_dtype |= GDN_LOCAL_RAGGED_ROWS;
         if (HK != H) l.saves_dtype |= GDN_LOCAL_SHARED_HEADS((int32_t)(H / HK)), l.dq_out = ptr(dq_each), l.dk_out = ptr(dk_each);
         return launch("gdn_chunk_bwd_local", pack_results({dq, dk, dv, g == nullptr ? at::Tensor() : dg, beta == nullptr ? at::Tensor() : dbeta, dh0}), [&] {
             const int status = local_fn(&l, stream);

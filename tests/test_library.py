@@ -103,6 +103,31 @@ def test_layer_ops_reject_bad_arguments_before_any_launch():
         assert lib.gdn_gated_rmsnorm_fwd(ctypes.byref(a), None) == status, over
 
 
+def test_flags_of_the_chunk_local_gradients_are_checked_before_any_launch():
+    lib = _lib.load_library()
+    flags = {name: int(value, 0) for name, value in re.findall(r"#define GDN_LOCAL_(\w+) (0x\w+)", open(HEADER).read())}
+    assert flags == {"DBETA_BF16": 0x100, "RAGGED_ROWS": 0x200}
+    ragged = flags["RAGGED_ROWS"]
+
+    def status(flag, **over):
+        a = _lib.GdnChunkLocalArgs()
+        for name, kind in a._fields_:
+            if kind is ctypes.c_void_p and name not in ("seq_start", "seq_len", "rk"):
+                setattr(a, name, 0x1000)  # never dereferenced: rq without rk is refused, behind the flags
+        a.saves_dtype, a.dstates_dtype, a.saves_sliced = _lib.GDN_BF16 | flag, _lib.GDN_BF16, 1
+        a.chunks, a.K, a.V, a.H, a.NC, a.scale = 6, 64, 64, 1, 3, 1.0
+        for name, value in over.items():
+            setattr(a, name, value)
+        return lib.gdn_chunk_bwd_local(ctypes.byref(a), None)
+
+    assert status(0x400) == status(ragged | 0x800) == -3
+    for T_rows in (0, 1, 64, 128, 193, -5):
+        assert status(ragged, T_rows=T_rows) == -2, T_rows
+    assert status(ragged, T_rows=150, seq_start=0x1000, seq_len=0x1000) == -2
+    for flag, T_rows in ((0, 0), (0, 150), (flags["DBETA_BF16"], -5), (ragged, 129), (ragged, 192), (ragged | 0x20000, 150)):
+        assert status(flag, T_rows=T_rows, H=2) == -1, (flag, T_rows)
+
+
 def test_convolution_rejects_bad_arguments_before_any_launch():
     lib = _lib.load_library()
 

@@ -159,6 +159,31 @@ def test_sweeps_in_one_launch_give_the_bits_of_smaller_batches(K, V, B, T):
 
 
 @pytest.mark.gpu
+def test_rows_of_whole_chunks_whatever_the_field_for_tokens_per_row_holds(monkeypatch):
+    """Without sequences and without the flag for ragged rows, ``T_rows`` is not read: the layout is that of NC * 64 tokens a row."""
+    from lm_engine_amd import _lib, ops
+
+    gen = torch.Generator().manual_seed(6)
+    q, k, v, do = (torch.randn(2, 128, 2, 64, generator=gen).bfloat16().cuda() for _ in range(4))
+    g, beta = -torch.rand(2, 128, 2, generator=gen).cuda(), torch.rand(2, 128, 2, generator=gen).bfloat16().cuda()
+    prep, S0, Vn, dS1, Y, _ = ops.chunk_bwd_sweeps(q, k, v, do, g, beta, 0.125, True, None, None, False, None, 2)
+    print("case: chunk-local gradients, T_rows without a meaning", flush=True)
+
+    def gradients(T_rows):
+        class Args(_lib.GdnChunkLocalArgs):
+            def __init__(self):
+                super().__init__()
+                self.T_rows = T_rows
+
+        with monkeypatch.context() as m:
+            m.setattr(_lib, "GdnChunkLocalArgs", Args)
+            return ops.chunk_local_grads(q, k, v, do, prep, Y, Vn, S0, dS1, 0.125, True, sliced=True)
+
+    for T_rows in (65, 100, 127):
+        assert all(torch.equal(x, y) for x, y in zip(gradients(T_rows), gradients(0))), T_rows
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("layout, lens, bad", [("packed", [100, 64, 0, 1, 133, 70], 1), ("packed", [100, 64, 0, 1, 133, 70], 4), ("padded", [200, 70, 1, 129], 1)])
 @pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (256, 512)])
 def test_nan_stays_in_its_sequence(layout, lens, bad, K, V):
