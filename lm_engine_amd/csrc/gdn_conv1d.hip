@@ -15,6 +15,7 @@
 // 2048 channels 54.5 -> 48.5 us (5.5 TB/s), 2 x 4096 21.5 -> 15.9, 4 x 4096, 6144 channels 86.4 -> 75.5, 777 tokens, 2048 channels
 // 5.7 -> 5.1; 6 x 1500, 4096 channels 29.1 both, masked 31.8 -> 31.4; fp32, 4 x 4096, 2048 channels 45.9 -> 43.5, 1 x 4096 19.3 -> 14.3.
 
+#include <algorithm>
 #include <type_traits>
 
 #include "gdn_common.h"
@@ -36,11 +37,11 @@ struct ConvParams {
     void* final_state;
     int64_t x_stride_b, x_stride_s, y_stride_b, y_stride_s;
     int B, S, C;
-    // The layer's front (gdn_layer_front): the launch's first plane of workgroups forms the gates, and its first workgroup the
+    // The layer's front (gdn_layer_front): the launch's first planes of workgroups form the gates, and its first workgroup the
     // prefix sums of an integer mask, which the convolution then reads itself.  As launches of their own, mask, convolution and
     // gates waited for each other: a padded prefill of 6 x 1500 tokens, 8 / 16 heads, K = V = 128 125.5 -> 116.8 us (6.5 + 33.4 + 4.2 |
     // 35.4 us of kernels), a prompt of 777 tokens, 2 heads, K = 256, V = 512 50.3 -> 47.9 (7.1 + 4.1 | 6.5).
-    int front = 0;         // 1: there is such a plane
+    int front = 0;         // such planes
     int mask_bytes = 0;    // element size of the integer mask; 0: `mask`, in the activations' type, if any
     GateParams gates = {};
     MaskParams ints = {};
@@ -86,11 +87,19 @@ __global__ __launch_bounds__(CONV_THREADS, 4) void causal_conv1d_kernel(const Co
     typedef typename ConvVec<T>::type vec_t;
     if ((int)blockIdx.z < p.front) {
         __shared__ int32_t s_sum[FRONT_MASK_ROWS];
-        const int64_t group = (int64_t)blockIdx.y * gridDim.x + blockIdx.x, groups = (int64_t)gridDim.x * gridDim.y;
-        if (group == 0 && p.mask_bytes != 0) {
-            if (p.mask_bytes == 8) padding_mask<CONV_THREADS, int64_t, void>(p.ints, s_sum);
-            else if (p.mask_bytes == 4) padding_mask<CONV_THREADS, int32_t, void>(p.ints, s_sum);
-            else padding_mask<CONV_THREADS, uint8_t, void>(p.ints, s_sum);
+        int64_t group = (int64_t)blockIdx.z * gridDim.x + blockIdx.x, groups = (int64_t)p.front * gridDim.x;
+        if (p.mask_bytes != 0) {
+            if (group == 0) {
+                if (threadIdx.x < FRONT_MASK_ROWS) s_sum[threadIdx.x] = 0;
+                __syncthreads();
+                if (p.mask_bytes == 8) mask_row_sums<CONV_THREADS, int64_t>(p.ints, s_sum);
+                else if (p.mask_bytes == 4) mask_row_sums<CONV_THREADS, int32_t>(p.ints, s_sum);
+                else mask_row_sums<CONV_THREADS, uint8_t>(p.ints, s_sum);
+                __syncthreads();
+                if (threadIdx.x < WAVE) mask_prefix_sums(p.ints, s_sum);
+                if (groups > 1) return;  // the others form the gates
+            }
+            if (groups > 1) group--, groups--;
         }
         for (int64_t i = group * CONV_THREADS + threadIdx.x; i < p.gates.tokens * p.gates.H; i += groups * CONV_THREADS) gates_at<T>(p.gates, i);
         return;
@@ -196,14 +205,27 @@ __global__ __launch_bounds__(CONV_THREADS, 4) void causal_conv1d_kernel(const Co
     }
 }
 
+// Planes of `workgroups` for the gates: as many as leave a thread at most FRONT_TRIPS of them.  One plane is sized by a row's share
+// of the convolution, the gates by the whole batch: with many short rows it was a tail of up to 128 trips on a few CUs.  One plane |
+// as many as needed, and the three launches beside them: 1024 x 16 tokens, 8 / 16 heads, K = V = 128 160.8 | 78.9 (82) us, 4096 x 4,
+// 4 heads, K = V = 64 125 | 53.0 (56), 1024 x 64 221 | 47.8 (50).  At 1, 2, 4 and 8 trips the same within 3 %, but for 64 x 16 tokens
+// with a mask at 8: 7.6 | 7.6 | 7.6 | 11.9.
+constexpr int FRONT_TRIPS = 4;
+static int front_planes(const ConvParams& p, int64_t workgroups) {
+    const int64_t per_plane = workgroups * CONV_THREADS * FRONT_TRIPS;
+    return (int)std::min<int64_t>((p.gates.tokens * p.gates.H + per_plane - 1) / per_plane, 65535 - p.B);
+}
+
 template <typename T, typename WT, int KS>
-static void launch_conv_ks(const ConvParams& p, bool silu, hipStream_t stream) {
+static void launch_conv_ks(ConvParams p, bool silu, hipStream_t stream) {
     const int64_t groups = (p.C / ConvVec<T>::N + WAVE - 1) / WAVE;
     // the integer mask of a single row, or of single tokens, is for the prefix sums alone, as in the convolution by itself
     const bool masked = p.mask != nullptr || (p.mask_bytes != 0 && p.B > 1 && p.S > 1);
     auto launch = [&](auto silu_tag, auto mask_tag, auto tokens_tag) {
         constexpr int TOKENS = decltype(tokens_tag)::value, SPAN = (CONV_THREADS / WAVE) * TOKENS;  // tokens per workgroup
-        const dim3 grid((unsigned)(groups * ((p.S + SPAN - 1) / SPAN)), 1, p.B + p.front);
+        const int64_t workgroups = groups * ((p.S + SPAN - 1) / SPAN);
+        if (p.front != 0) p.front = front_planes(p, workgroups);
+        const dim3 grid((unsigned)workgroups, 1, p.B + p.front);
         hipLaunchKernelGGL((causal_conv1d_kernel<T, WT, KS, decltype(silu_tag)::value, TOKENS, decltype(mask_tag)::value>), grid, dim3(CONV_THREADS), 0, stream, p);
     };
     auto launch_with = [&](auto tokens_tag, auto mask_tag) {

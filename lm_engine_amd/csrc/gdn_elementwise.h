@@ -1,8 +1,6 @@
 // Device helpers that the elementwise kernels (gdn_elementwise.hip) share with the layer's front (gdn_conv1d.hip).
 #pragma once
 
-#include <type_traits>
-
 #include "gdn_common.h"
 
 namespace gdn {
@@ -45,45 +43,60 @@ struct MaskParams {
     int B, S;
 };
 
-// Prefix sums of the mask's row sums, and the mask as T (void: not wanted), by one workgroup of THREADS; s_sum: LDS, a word per row.
-template <int THREADS, typename I, typename T>
-__device__ __forceinline__ void padding_mask(const MaskParams& p, int32_t* s_sum) {
-    constexpr int WAVES = THREADS / WAVE;
-    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
-    for (int b = threadIdx.x; b < p.B; b += THREADS) s_sum[b] = 0;
-    __syncthreads();
-    const int parts = p.B < WAVES ? WAVES / p.B : 1;  // waves per row
+// s_sum (LDS, cleared, a word per row) += the sums of the mask's rows, by one workgroup of THREADS.  A wave has four rows, or parts
+// of rows, at a time and two loads of each in flight: the few waves of the layer's front waited for one row after the other (64 x
+// 140 tokens, 4 heads, K = V = 64: 26.1 -> 14.8 us for the front, 21.4 as three launches; 64 x 1024 63.4 -> 43.5, 60.2; 32 x 512 23.7
+// -> 16.8, 24.6).  Four loads each were no faster and took 119 registers of the convolution, 63 without them.
+template <int THREADS, typename I>
+__device__ __forceinline__ void mask_row_sums(const MaskParams& p, int32_t* s_sum) {
+    constexpr int WAVES = THREADS / WAVE, ROWS = 4;
+    const int lane = threadIdx.x % WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int parts = p.B < WAVES * ROWS ? WAVES * ROWS / p.B : 1;  // of a row
     const int per = ((p.S + parts - 1) / parts + WAVE - 1) / WAVE * WAVE;
-    for (int unit = wave; unit < p.B * parts; unit += WAVES) {
-        const int b = unit / parts, begin = (unit % parts) * per, end = min(begin + per, p.S);
-        const I* const row = reinterpret_cast<const I*>(p.mask) + b * p.stride_b;
-        int32_t sum = 0;
-#pragma unroll 4
-        for (int s = begin + lane; s < end; s += WAVE) {
-            const I x = row[s * p.stride_s];
-            if constexpr (!std::is_void_v<T>) reinterpret_cast<T*>(p.out)[(int64_t)b * p.S + s] = (T)(float)x;
-            sum = (int32_t)((uint32_t)sum + (uint32_t)x);
+    for (int unit = wave * ROWS; unit < p.B * parts; unit += WAVES * ROWS) {
+        int b[ROWS], begin[ROWS], end[ROWS];
+        const I* row[ROWS];
+        int32_t sum[ROWS] = {};
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+            const int u = min(unit + r, p.B * parts - 1);
+            b[r] = u / parts, begin[r] = u % parts * per, end[r] = u == unit + r ? min(begin[r] + per, p.S) : 0;
+            row[r] = reinterpret_cast<const I*>(p.mask) + b[r] * p.stride_b;
         }
+#pragma unroll 2
+        for (int s = lane; s < per; s += WAVE) {
 #pragma unroll
-        for (int off = WAVE / 2; off >= 1; off >>= 1) sum = (int32_t)((uint32_t)sum + (uint32_t)__shfl_xor(sum, off, WAVE));
-        if (lane == 0) atomicAdd(&s_sum[b], sum);
-    }
-    __syncthreads();
-    if (wave == 0) {  // prefix sums, 64 rows at a time
-        int32_t before = 0;
-        for (int b0 = 0; b0 < p.B; b0 += WAVE) {
-            int32_t x = b0 + lane < p.B ? s_sum[b0 + lane] : 0;
-#pragma unroll
-            for (int off = 1; off < WAVE; off <<= 1) {
-                const int32_t y = __shfl_up(x, off, WAVE);
-                if (lane >= off) x = (int32_t)((uint32_t)x + (uint32_t)y);
+            for (int r = 0; r < ROWS; r++) {  // (no branch around a load: the row's last element stands in for one past its end)
+                const int at = begin[r] + s;
+                const uint32_t x = (uint32_t)row[r][min(at, p.S - 1) * p.stride_s];
+                sum[r] = (int32_t)((uint32_t)sum[r] + (at < end[r] ? x : 0u));
             }
-            x = (int32_t)((uint32_t)x + (uint32_t)before);
-            if (b0 + lane < p.B) p.prefix[b0 + lane + 1] = x;
-            before = __shfl(x, WAVE - 1, WAVE);
         }
-        if (lane == 0) p.prefix[0] = 0;
+#pragma unroll
+        for (int r = 0; r < ROWS; r++) {
+#pragma unroll
+            for (int off = WAVE / 2; off >= 1; off >>= 1) sum[r] = (int32_t)((uint32_t)sum[r] + (uint32_t)__shfl_xor(sum[r], off, WAVE));
+            if (lane == 0) atomicAdd(&s_sum[b[r]], sum[r]);
+        }
     }
+}
+
+// prefix[0 .. B] = 0 and the prefix sums of s_sum, by one wave
+__device__ __forceinline__ void mask_prefix_sums(const MaskParams& p, const int32_t* s_sum) {
+    const int lane = threadIdx.x % WAVE;
+    int32_t before = 0;
+    for (int b0 = 0; b0 < p.B; b0 += WAVE) {  // 64 rows at a time
+        int32_t x = b0 + lane < p.B ? s_sum[b0 + lane] : 0;
+#pragma unroll
+        for (int off = 1; off < WAVE; off <<= 1) {
+            const int32_t y = __shfl_up(x, off, WAVE);
+            if (lane >= off) x = (int32_t)((uint32_t)x + (uint32_t)y);
+        }
+        x = (int32_t)((uint32_t)x + (uint32_t)before);
+        if (b0 + lane < p.B) p.prefix[b0 + lane + 1] = x;
+        before = __shfl(x, WAVE - 1, WAVE);
+    }
+    if (lane == 0) p.prefix[0] = 0;
 }
 
 }  // namespace gdn

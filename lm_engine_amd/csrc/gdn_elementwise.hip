@@ -377,12 +377,33 @@ __global__ __launch_bounds__(256) void fold_heads_kernel(const FoldParams p) {
 // int32 prefix sums of its rows' sums [B + 1].  One workgroup, whose waves share the rows between them: bound by the launch and
 // one trip through memory.  As conversion, row sums, prefix sum, pad and copies it was six launches (6 x 1500 tokens, 8 / 16 heads,
 // K = V = 128: 145 -> 127 us for the layer's prefill); torch's kernels are the better ones where a workgroup would read for long.
-constexpr int MASK_THREADS = 1024;
+constexpr int MASK_THREADS = 1024, MASK_WAVES = MASK_THREADS / WAVE;
 
 template <typename I, typename T>
 __global__ __launch_bounds__(MASK_THREADS) void padding_mask_kernel(const MaskParams p) {
     __shared__ int32_t s_sum[GDN_MASK_MAX_ROWS];
-    padding_mask<MASK_THREADS, I, T>(p, s_sum);
+    const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
+    for (int b = threadIdx.x; b < p.B; b += MASK_THREADS) s_sum[b] = 0;
+    __syncthreads();
+    const int parts = p.B < MASK_WAVES ? MASK_WAVES / p.B : 1;  // waves per row
+    const int per = ((p.S + parts - 1) / parts + WAVE - 1) / WAVE * WAVE;
+    for (int unit = wave; unit < p.B * parts; unit += MASK_WAVES) {
+        const int b = unit / parts, begin = (unit % parts) * per, end = min(begin + per, p.S);
+        const I* const row = reinterpret_cast<const I*>(p.mask) + b * p.stride_b;
+        T* const out = reinterpret_cast<T*>(p.out) + (int64_t)b * p.S;
+        int32_t sum = 0;
+#pragma unroll 4
+        for (int s = begin + lane; s < end; s += WAVE) {
+            const I x = row[s * p.stride_s];
+            out[s] = (T)(float)x;
+            sum = (int32_t)((uint32_t)sum + (uint32_t)x);
+        }
+#pragma unroll
+        for (int off = WAVE / 2; off >= 1; off >>= 1) sum = (int32_t)((uint32_t)sum + (uint32_t)__shfl_xor(sum, off, WAVE));
+        if (lane == 0) atomicAdd(&s_sum[b], sum);
+    }
+    __syncthreads();
+    if (wave == 0) mask_prefix_sums(p, s_sum);
 }
 
 template <typename I>

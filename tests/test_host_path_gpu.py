@@ -428,3 +428,30 @@ def test_the_layers_front_in_one_launch_gives_the_bits_of_its_steps(B, S, dtype,
         assert refused == isinstance(steps, tuple) and len(one) == len(steps)
         assert one == steps if refused else all((p is None and q is None) or torch.equal(p, q) for p, q in zip(one, steps)), form
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize(
+    "B, S, HK, H, K, V, mask_dtype",
+    # many short rows: the gates on one plane of workgroups and on several; rows of a mask four to a wave, whole and cut, parts of rows
+    [(1024, 3, 4, 4, 64, 64, None), (300, 17, 2, 4, 64, 64, None), (64, 5, 4, 4, 64, 64, torch.int64), (64, 130, 4, 4, 64, 64, torch.bool), (17, 65, 2, 2, 64, 64, torch.int32),
+     (16, 1, 2, 2, 64, 64, torch.int64), (5, 300, 2, 2, 64, 64, torch.uint8), (2, 1000, 2, 2, 64, 64, torch.int64),
+     # walks of 8 and of 12 tokens that end within one, over several groups of channels, the last one whole and cut
+     (3, 4797, 5, 5, 64, 64, None), (3, 3201, 6, 6, 64, 128, None), (3, 4797, 5, 5, 64, 64, torch.int64), (3, 4797, 5, 5, 64, 64, torch.int32), (3, 4797, 5, 5, 64, 64, torch.bool), (3, 3201, 6, 6, 64, 128, torch.int64)],
+)  # fmt: skip
+def test_the_layers_front_of_many_rows_and_of_long_walks(B, S, HK, H, K, V, mask_dtype):
+    from lm_engine_amd.layer_ops import padding_mask
+
+    gen = torch.Generator("cuda").manual_seed(B + S)
+    r = lambda *shape: torch.randn(*shape, generator=gen, device="cuda").to(BF16)  # noqa: E731
+    C = 2 * HK * K + H * V
+    x, ab, w, bias, A, dt = r(B, S, C), r(B, S, 2 * H + 3), 0.3 * r(C, 1, 4), 0.1 * r(C), r(H).float(), r(H).float()
+    state, a, b, mask, stream, native = r(B, C, 3), ab[..., :H], ab[..., H : 2 * H], None, _host.raw_stream(0), _host.host()
+    if mask_dtype is not None:
+        lengths = torch.randint(0, S + 1, (B,), generator=torch.Generator().manual_seed(S))
+        mask = (torch.arange(S) >= S - lengths[:, None]).to(mask_dtype).cuda()
+    print(f"case: layer's front, {B} x {S} tokens, {C} channels, mask {mask_dtype}", flush=True)
+    *front, prefix = native.layer_front(stream, x, w, bias, state, mask, True, 1, a, b, A, dt, 1.0)
+    bits, wanted = (None, None) if mask is None else padding_mask(mask, BF16)
+    steps = [*native.conv(stream, x, w, bias, state, bits, True, 1), *native.gates(stream, a, b, A, dt, 1.0)]
+    assert all(torch.equal(p, q) for p, q in zip(front, steps)) and (mask is None) == (prefix is None)
+    assert mask is None or torch.equal(prefix, wanted) and torch.equal(wanted.cpu(), torch.nn.functional.pad(lengths.cumsum(0), (1, 0)).int())
