@@ -441,7 +441,7 @@ int gdn_chunk_fwd_profile(const gdn_args *args, void *stream, float *kernel_ms);
  *   final_state   [B, C, kernel_size - 1] contiguous in dtype, or NULL (not written)
  *
  * kernel_size 2..4, C a multiple of 8 (bf16) or 4 (fp32), rows, weight and bias 16-byte aligned;
- * w_dtype equals dtype or is fp32.
+ * w_dtype equals dtype or is fp32.  B at most 65535, S below 65535 * 64 (GDN_ERR_UNSUPPORTED otherwise).
  */
 typedef enum gdn_activation { GDN_ACT_NONE = 0, GDN_ACT_SILU = 1 } gdn_activation;
 

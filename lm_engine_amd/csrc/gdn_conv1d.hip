@@ -6,9 +6,10 @@
 // 2 * sizeof(element); weights, bias, state and mask are negligible.
 //
 // A thread owns 16 bytes of channels (8 bf16 / 4 fp32) of TOKENS consecutive tokens and asks for its TOKENS + kernel_size - 1 rows
-// of x at once, before anything is converted; neighbouring token blocks share kernel_size - 1 rows of halo and read them at the
-// same moment, out of one cache.  Lanes cover consecutive channel vectors: every load and store of a wave is one contiguous row
-// segment; the four waves of a workgroup take consecutive token blocks of the same channels.
+// of x at once, before anything is converted.  Lanes cover consecutive channel vectors: every load and store of a wave is one
+// contiguous row segment; the four waves of a workgroup take consecutive token blocks of the same channels, and read the
+// kernel_size - 1 rows of halo that they share at the same moment, out of one cache.  The next four blocks are another workgroup's,
+// as many ids away as there are groups of channels: on the same XCD only where these are a multiple of 8.
 //
 // Walked row by row, with the window in registers, 16 tokens a thread were 16 trips to memory one after the other (the branches on
 // the sequence's ends held the use of every row next to its load).  Before and after, bf16, inputs from memory: 8 x 4096 tokens,
@@ -24,6 +25,7 @@
 namespace gdn {
 
 constexpr int CONV_THREADS = 256;
+constexpr int CONV_MAX_TOKENS = 65535 * 64;  // of a row: longer ones have always been refused
 constexpr int FRONT_MASK_ROWS = 64;  // of an integer mask in the layer's front
 constexpr int CONV_TOKENS_SHORT = 4;  // tokens per thread of a batch whose waves would leave compute units idle (launch_conv_ks)
 
@@ -217,38 +219,38 @@ static int front_planes(const ConvParams& p, int64_t workgroups) {
 }
 
 template <typename T, typename WT, int KS>
-static void launch_conv_ks(ConvParams p, bool silu, hipStream_t stream) {
+static int launch_conv_ks(ConvParams p, bool silu, hipStream_t stream) {
     const int64_t groups = (p.C / ConvVec<T>::N + WAVE - 1) / WAVE;
     // the integer mask of a single row, or of single tokens, is for the prefix sums alone, as in the convolution by itself
     const bool masked = p.mask != nullptr || (p.mask_bytes != 0 && p.B > 1 && p.S > 1);
-    auto launch = [&](auto silu_tag, auto mask_tag, auto tokens_tag) {
+    auto launch = [&](auto silu_tag, auto mask_tag, auto tokens_tag) -> int {
         constexpr int TOKENS = decltype(tokens_tag)::value, SPAN = (CONV_THREADS / WAVE) * TOKENS;  // tokens per workgroup
         const int64_t workgroups = groups * ((p.S + SPAN - 1) / SPAN);
+        if (workgroups * CONV_THREADS > 0xffffffff) return GDN_ERR_UNSUPPORTED;  // (a grid's x holds at most 2^32 - 1 threads; x and y of more do not fit a GPU)
         if (p.front != 0) p.front = front_planes(p, workgroups);
         const dim3 grid((unsigned)workgroups, 1, p.B + p.front);
         hipLaunchKernelGGL((causal_conv1d_kernel<T, WT, KS, decltype(silu_tag)::value, TOKENS, decltype(mask_tag)::value>), grid, dim3(CONV_THREADS), 0, stream, p);
+        return (int)hipGetLastError();
     };
     auto launch_with = [&](auto tokens_tag, auto mask_tag) {
-        if (silu) launch(std::true_type{}, mask_tag, tokens_tag);
-        else launch(std::false_type{}, mask_tag, tokens_tag);
+        return silu ? launch(std::true_type{}, mask_tag, tokens_tag) : launch(std::false_type{}, mask_tag, tokens_tag);
     };
     typedef std::integral_constant<int, CONV_TOKENS_SHORT> few_tokens;
     // Under 1792 waves of 16 tokens (7 per compute unit) more workgroups count for more than the halo.  4 | 8 tokens a thread, bf16,
     // inputs from memory: 200 waves 5.3 | 6.1 us, 1024 9.7 | 9.8, 2000 16.3 | 15.6 (C = 2048), 2028 17.0 | 15.6 (C = 6144), 4096 28.5 | 28.2,
     // 8192 50.6 | 48.2; masked, 4 | 12: 1584 16.3 | 17.0, 4056 31.2 | 29.9.
     const bool few = groups * ((p.S + 15) / 16) * p.B < 1792;
-    if (masked && few) launch_with(few_tokens{}, std::true_type{});
-    else if (masked) launch_with(std::integral_constant<int, ConvVec<T>::TOKENS_MASKED>{}, std::true_type{});
-    else if (few) launch_with(few_tokens{}, std::false_type{});
-    else launch_with(std::integral_constant<int, ConvVec<T>::TOKENS>{}, std::false_type{});
+    if (masked && few) return launch_with(few_tokens{}, std::true_type{});
+    if (masked) return launch_with(std::integral_constant<int, ConvVec<T>::TOKENS_MASKED>{}, std::true_type{});
+    if (few) return launch_with(few_tokens{}, std::false_type{});
+    return launch_with(std::integral_constant<int, ConvVec<T>::TOKENS>{}, std::false_type{});
 }
 
 template <typename T, typename WT>
 static int launch_conv(const ConvParams& p, int kernel_size, bool silu, hipStream_t stream) {
-    if (kernel_size == 2) launch_conv_ks<T, WT, 2>(p, silu, stream);
-    else if (kernel_size == 3) launch_conv_ks<T, WT, 3>(p, silu, stream);
-    else launch_conv_ks<T, WT, 4>(p, silu, stream);
-    return (int)hipGetLastError();
+    if (kernel_size == 2) return launch_conv_ks<T, WT, 2>(p, silu, stream);
+    if (kernel_size == 3) return launch_conv_ks<T, WT, 3>(p, silu, stream);
+    return launch_conv_ks<T, WT, 4>(p, silu, stream);
 }
 
 }  // namespace gdn
@@ -263,7 +265,7 @@ int conv_args_status(const gdn_conv_args* a) {
     if (a->w_dtype != GDN_BF16 && a->w_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;
     if (a->dtype == GDN_F32 && a->w_dtype != GDN_F32) return GDN_ERR_UNSUPPORTED;  // weights as wide as the data
     if (a->activation != GDN_ACT_NONE && a->activation != GDN_ACT_SILU) return GDN_ERR_UNSUPPORTED;
-    if (a->B > 65535 || a->S / 64 >= 65535) return GDN_ERR_UNSUPPORTED;
+    if (a->B > 65535 || a->S >= gdn::CONV_MAX_TOKENS) return GDN_ERR_UNSUPPORTED;
     const int64_t vec = (a->dtype == GDN_BF16) ? 8 : 4;
     if (a->C % vec != 0) return GDN_ERR_UNSUPPORTED;
     const int64_t strides[] = {a->x_stride_b, a->x_stride_s, a->y_stride_b, a->y_stride_s};

@@ -153,6 +153,10 @@ def test_convolution_rejects_bad_arguments_before_any_launch():
         (dict(x=0x1008), -4),
         (dict(y=0x1000), -2),
         (dict(x_stride_s=8), -2),
+        (dict(S=65535 * 64), -3),
+        # more threads than a grid holds, in walks of 8 tokens (bf16) and of 4 (fp32)
+        (dict(S=65535 * 64 - 1, C=1 << 17, x_stride_s=1 << 17, y_stride_s=1 << 17), -3),
+        (dict(S=65535 * 64 - 1, C=1 << 15, x_stride_s=1 << 15, y_stride_s=1 << 15, dtype=_lib.GDN_F32, w_dtype=_lib.GDN_F32), -3),
     ]:
         assert lib.gdn_causal_conv1d_fwd(ctypes.byref(conv_args(**over)), None) == status, over
 
