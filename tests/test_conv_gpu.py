@@ -151,6 +151,24 @@ def test_long_walks_match_short_ones(dtype, masked):
         assert torch.equal(y1[0, first:].cpu().to(F64), y[row, first:]) and torch.equal(s1[0].cpu().to(F64), s[row])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype, C", [(BF16, 1024), (BF16, 1544), (F32, 1028)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_long_walks_over_several_groups_of_channels_match_short_ones(dtype, C, masked):
+    """A group is 64 threads' channels, 512 in bf16 and 256 in fp32: whole ones, and a last one cut to a single thread; tokens that are no multiple of a walk's."""
+    B, S = 7, 2053
+    x, w, b, st, m = _inputs(B, S, C, 4, dtype, seed=C, state=True, mask=masked)
+    run = lambda i, j, first=0, last=S: lm_engine_amd.depthwise_causal_convolution(  # noqa: E731
+        x[i:j, first:last].cuda(), w.cuda(), b.cuda(), st[i:j].cuda(), None if m is None else m[i:j, first:last].cuda(), output_state=True)
+    y, s = run(0, B)
+    for i in (0, 5):  # two rows, so that a mask counts: 2 x 330 tokens are walked four at a time
+        y1, _ = run(i, i + 2, 0, 330)
+        assert torch.equal(y[i : i + 2, :330], y1)
+    carried = x[5:, S - 203 : S - 200].transpose(1, 2).contiguous()  # (no padding that late)
+    tail = _check(x[5:, S - 200 :], w, b, carried, None if m is None else m[5:, S - 200 :], "silu", f"the end of long walks, C={C}")
+    assert torch.equal(tail[0], y[5:, S - 200 :].cpu().to(F64)) and torch.equal(tail[1], s[5:].cpu().to(F64))
+
+
 # the ends of a walk of 4, 8 and 12 tokens and one past each; sequences shorter than the window
 @pytest.mark.parametrize("dtype, w_dtype", [(BF16, BF16), (BF16, F32), (F32, F32)])
 @pytest.mark.parametrize("masked", [False, True])

@@ -355,9 +355,19 @@ def _training_forms():
         }  # fmt: skip
 
 
+# Which of the three gradients below the native path takes: not one value for all elements, in no case, nor rows that the norm
+# would have to copy, nor operands that need a conversion.  (): the Python code does not ask.
+_BACKWARD_TAKES = {"conv_bwd": (True, True, False), "gates_bwd": (True, True, False), "norm_bwd": (True, False, False), "delta_rule_bwd": (True, True, False)}
+_BACKWARD_TAKES_OF_FORM = {
+    ("conv_bwd", "state"): (), ("gates_bwd", "bf16 decay"): (False, False, False), ("gates_bwd", "one of two"): (True, False, False),
+    ("norm_bwd", "o strided"): (False, False, False), ("norm_bwd", "gate slice off its boundary"): (False, False, False),
+    ("delta_rule_bwd", "packed, int64 prefix"): (False, False, False), ("delta_rule_bwd", "fp32"): (), ("delta_rule_bwd", "V = 96"): (),
+}  # fmt: skip
+
+
 def test_backward_passes_end_as_they_do_without_the_native_path(monkeypatch):
     """The gradients of every form are the same bits with the native host path and without it, for a gradient that lies as
-    the output does, a column block of a wider one, and one value for all elements."""
+    the output does, a column block of a wider one, and one value for all elements; and every form takes the path it is meant to."""
     from lm_engine_amd import backward, conv, layer_ops, ops
 
     differ = []
@@ -378,7 +388,8 @@ def test_backward_passes_end_as_they_do_without_the_native_path(monkeypatch):
                     for d in (wide[..., : out.size(-1)].contiguous(), wide[..., 8 : 8 + out.size(-1)], torch.ones((), dtype=out.dtype).cuda().expand(out.shape)):
                         results += [x.clone() for x in torch.autograd.grad(out, leaves, d, retain_graph=True, allow_unused=True) if x is not None]
                 outcomes.append(results)
-                assert form != "plain" or path.took[0] == on, "the path under test was not the one taken"
+                takes = _BACKWARD_TAKES_OF_FORM.get((name, form), _BACKWARD_TAKES[name])
+                assert path.took == [on and x for x in takes], f"{name}, {form}: the path under test was not the one taken: {path.took}"
             if not all(x.dtype == y.dtype and x.shape == y.shape and torch.equal(x, y) for x, y in zip(*outcomes)) or len(outcomes[0]) != len(outcomes[1]):
                 differ.append((name, form))
     torch.cuda.synchronize()
@@ -388,8 +399,8 @@ def test_backward_passes_end_as_they_do_without_the_native_path(monkeypatch):
 @pytest.mark.parametrize("S, dtype", [(2, BF16), (70, BF16), (130, torch.float32), (1100, BF16)])
 @pytest.mark.parametrize("B", [1, 3])
 def test_the_layers_front_in_one_launch_gives_the_bits_of_its_steps(B, S, dtype, monkeypatch):
-    """Convolution, gates and the mask's prefix sums: short and long walks over the tokens, integer masks of every type and layout, a
-    single row (whose mask the convolution does not apply), rows without a token, and what is refused."""
+    """Convolution, gates and the mask's prefix sums: short walks over the tokens, integer masks of every type and layout, a single
+    row (whose mask the convolution does not apply), rows without a token, and what is refused."""
     from lm_engine_amd import layer
 
     x = _layer_operands(B, S)
