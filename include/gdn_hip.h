@@ -396,9 +396,10 @@ typedef struct gdn_chunk_bwd_prepare_args {
 int gdn_chunk_bwd_prepare(const gdn_chunk_bwd_prepare_args *args, void *stream);
 
 /*
- * Training support, fourth part: everything gdn_chunk_bwd_local needs from the states, in one call of three kernels - per-chunk
- * records, the forward sweep (the states the chunks start from, V~) and the reverse sweep (the gradients of the states they end
- * with, Y).  What gdn_chunk_bwd_prepare and two calls of gdn_chunk_fwd_saving arrive at through a mirror problem, in one step per
+ * Training support, fourth part: everything gdn_chunk_bwd_local needs from the states, in one call - per-chunk records, the forward
+ * sweep (the states the chunks start from, V~) and the reverse sweep (the gradients of the states they end with, Y).  Two launches:
+ * the records, and both sweeps in one; one more for the chunk offsets of packed sequences, and one more where K = 64 and a sweep
+ * of rows has more workgroups than the GPU compute units: the sweeps are a launch each then.  What gdn_chunk_bwd_prepare and two calls of gdn_chunk_fwd_saving arrive at through a mirror problem, in one step per
  * chunk, for every batch that gdn_chunk_fwd takes (fixed-length rows of any length, packed, left-padded; qk_heads as there):
  * bf16, K = 64, 128 or 256, V a multiple of 64 (GDN_ERR_UNSUPPORTED otherwise).
  *   args   as for gdn_chunk_fwd; h0, g, beta may be NULL; ht is not used and o not written (it must be a valid pointer and strides);

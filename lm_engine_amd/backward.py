@@ -6,8 +6,8 @@ the gradients of ``(o, final_state)`` with respect to ``(q, k, v, g, beta, initi
 
 Three ways through, same formulas:
 
-* bf16, K = 64, 128 or 256, V a multiple of 64 (whole rows, packed or left-padded batches): three kernel launches
-  (``_backward_on_kernels``) - ``gdn_chunk_bwd_sweeps`` (records, forward sweep, reverse sweep) and ``gdn_chunk_bwd_local``;
+* bf16, K = 64, 128 or 256, V a multiple of 64 (whole rows, packed or left-padded batches): three kernel launches, a few more
+  for some batches (``_backward_on_kernels``) - ``gdn_chunk_bwd_sweeps`` (records, both sweeps) and ``gdn_chunk_bwd_local``;
 * other bf16 shapes (V a multiple of 32 only): the two sweeps over the chunks of a chain on the scan kernel
   (``gdn_chunk_fwd_saving``: the forward's scan in a variant that also writes the chunk states and V~),
   everything chunk-local as batched library GEMMs (fp32, ``torch.bmm``) and elementwise torch operations on
@@ -341,8 +341,8 @@ def _chunk_local_grads(qs, kn, vc, doc, Y, Vn, S0, dS1, gam, bc):
 
 def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm, cu_seqlens, left_padded, joined):
     """The whole backward on three kernel launches (bf16; K = 64, 128 or 256; V a multiple of 64): ``gdn_chunk_bwd_sweeps``
-    (per-chunk records and scalars, both sweeps; one more launch for the chunk offsets of packed
-    sequences) and ``gdn_chunk_bwd_local`` writing the gradients in the caller's layout (one more launch, ``gdn_fold_heads``, where
+    (per-chunk records and scalars, both sweeps; one more launch for the chunk offsets of packed sequences, and one more at K = 64
+    for rows that fill the GPU with either sweep) and ``gdn_chunk_bwd_local`` writing the gradients in the caller's layout (one more launch, ``gdn_fold_heads``, where
     value heads share those of q and k).  Chunk states, V~ and Y pass between
     them as bf16, what the chunk-local products round them to anyway.  Batches that are not whole rows of whole chunks are laid
     out with the chunk count of their longest sequence."""

@@ -164,7 +164,8 @@ struct FindInRows {
     }
 };
 // Packed sequences.  Up to 63 of them keep their prefixes in the lanes of two registers, and a lookup is one comparison per lane; a
-// search waits for one load per step, seven of them in a row at 11 sequences (prepare, 32768 tokens, 16 heads, K = 128: 100 -> 92 us, in rows 92 -> 89).
+// search waits for one load per step, seven of them in a row at 11 sequences (prepare, 32768 tokens, 16 heads, K = 128, at steady
+// clocks: 91 - 95 -> 84 - 88 us; 40 sequences 103 -> 98; in rows, 8 x 4096 tokens, 82 -> 81).
 struct FindPacked {
     int off = 0, cu = 0;
 

@@ -624,8 +624,9 @@ __device__ __forceinline__ void Sweep<K, REV>::run(const SweepParams& p, int id,
 // reverse sweep comes first, its chunks are the longer ones.  `first`: the number of the launch's first workgroup.  Kernel times, two
 // launches | one: 4 x 4096 tokens, 16 heads, K = V = 128 (256 workgroups a sweep) 220 | 208 us, 2 x 4096 142 | 107, 2184 tokens 77 | 45;
 // 11 packed sequences, 32768 tokens 428 | 397; 9000 tokens, 3 heads, K = 256, V = 512 467 | 289.  Slower only where one launch takes
-// forward workgroups their place, see launch_sweeps, and by 3 % at 2 x 2048 tokens, 32 heads, V = 256 (196 | 202; the gap between
-// two launches is not in these figures).
+// forward workgroups their place, see launch_sweeps.  With many rounds of workgroups a sweep it is the gap between the launches that
+// goes: at 2 x 2048 tokens, 32 heads, V = 256 (512) the kernels alone take 196 | 202 us, calls of gdn_chunk_bwd_sweeps back to back 203
+// | 201; 8 x 2048, 16 heads, V = 128 265 | 256; 4 x 1024, 32 heads, V = 256 (1024) 187 | 186; 32 x 512, 16 heads (2048) 291 | 282.
 template <int K>
 __global__ __launch_bounds__(SWEEP_WAVES* WAVE) void chunk_sweeps_kernel(const SweepParams fwd, const SweepParams rev, unsigned groups, unsigned first) {
     constexpr int LDS = Sweep<K, true>::LDS_BYTES > Sweep<K, false>::LDS_BYTES ? Sweep<K, true>::LDS_BYTES : Sweep<K, false>::LDS_BYTES;

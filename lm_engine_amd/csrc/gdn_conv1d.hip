@@ -41,8 +41,9 @@ struct ConvParams {
     int B, S, C;
     // The layer's front (gdn_layer_front): the launch's first planes of workgroups form the gates, and its first workgroup the
     // prefix sums of an integer mask, which the convolution then reads itself.  As launches of their own, mask, convolution and
-    // gates waited for each other: a padded prefill of 6 x 1500 tokens, 8 / 16 heads, K = V = 128 125.5 -> 116.8 us (6.5 + 33.4 + 4.2 |
-    // 35.4 us of kernels), a prompt of 777 tokens, 2 heads, K = 256, V = 512 50.3 -> 47.9 (7.1 + 4.1 | 6.5).
+    // gates waited for each other: a padded prefill of 6 x 1500 tokens, 8 / 16 heads, K = V = 128 125.5 -> 116.8 us, a prompt of 777
+    // tokens, 2 heads, K = 256, V = 512 50.3 -> 47.9; back to back in a graph, three launches (two without a mask) | one: 37.5 | 30.0
+    // and 6.1 | 4.2, 64 x 512 tokens with a mask, 2 heads, K = 256, V = 512 64.3 | 51.6, 8 x 4096, 16 heads, K = V = 128 148.6 | 147.0.
     int front = 0;         // such planes
     int mask_bytes = 0;    // element size of the integer mask; 0: `mask`, in the activations' type, if any
     GateParams gates = {};

@@ -20,10 +20,11 @@
 // for before anything is waited for: the convolution's operands four channels to a thread in wide loads, then the state, and no
 // branch stands between a load and the next one that holds its use.  Loaded one channel and tap at a time, each parameter converted
 // under the branch on its dtype, the kernel waited for memory about twenty times in a row before it asked for the state, and a
-// workgroup issued four times as many loads; the last tile of a head did the same with the norm's weight.  Steps with the state
-// read from and written to different memory, before and after: 53 sequences x 2 heads, K = 256, V = 512 29.3 -> 22.6 us (a copy of
-// as many bytes takes 21.7), 32 of them 18.1 -> 13.3, 128 of them 59.8 -> 51.7 (5.2 TB/s); x 16 heads, K = V = 128, 53 sequences
-// 26.1 -> 22.5, 128 of them 53.3 -> 46.4 (5.8 TB/s).
+// workgroup issued four times as many loads; the last tile of a head did the same with the norm's weight.  Steps in a graph, each with
+// a state of its own and memory of its own for the new one, before and after: 53 sequences x 2 heads, K = 256, V = 512 32.5 -> 26.5 us,
+// 32 of them 21.1 -> 15.6, 128 of them 64.3 -> 54.3 (4.9 TB/s); x 16 heads, K = V = 128, 53 sequences 26.5 -> 22.8, 128 of them 55.0 ->
+// 47.7 (5.6 TB/s).  Where the new state takes the memory of the last step's, and so finds it in the caches: 53 sequences 28.5 -> 22.3
+// (a copy of as many bytes takes 21.7).
 
 #include <type_traits>
 
@@ -251,11 +252,11 @@ __global__ __launch_bounds__(4 * BV) void layer_step_kernel(const LayerStepParam
 namespace {
 
 // Columns per workgroup.  A head of at most 128 columns is one tile and needs no ticket (one sequence x 16 heads, K = V = 128:
-// 6.0 us a launch, 9.1 and 10.0 with 64 and 32 columns and tickets).  Wider ones: 64 columns while that is at most one workgroup per
+// 5.2 us a launch, 7.8 with 64 columns and tickets).  Wider ones: 64 columns while that is at most one workgroup per
 // CU, else 128: the narrower the tile, the more often the convolution of q and k is repeated, and a second workgroup on some of the
-// CUs takes longer than a larger one on each (K = 256, V = 512, 2 heads, 64 | 128 columns: 2 sequences 8.3 | 8.6 us, 16 of them 10.7
-// | 11.1, 20 13.7 | 11.8, 24 14.6 | 12.7, 32 15.0 | 14.8, 53 27.8 | 25.5; K = 128, V = 256, 4 heads: 2 sequences 7.5 | 7.8, 16 of
-// them 9.2 | 8.8, 64 17.9 | 15.3; back to back in a graph).
+// CUs takes longer than a larger one on each (K = 256, V = 512, 2 heads, 64 | 128 columns: 2 sequences 8.8 | 9.6 us, 16 of them 11.4
+// | 11.9, 20 14.3 | 12.5, 24 15.0 | 13.4, 32 16.0 | 15.9, 53 28.4 | 26.6; K = 128, V = 256, 4 heads: 2 sequences 7.9 | 8.3, 16 of
+// them 9.6 | 9.4, 64 18.4 | 16.2; measured as above, in a graph).
 int step_tile_columns(int B, int H, int V) {
     if (V == 32 || V == 64 || V == 128) return V;
     if (V % 128 == 0 && (int64_t)B * H * (V / 64) > 256) return 128;

@@ -7,8 +7,7 @@
   lm_engine/modeling_utils/normalization.py:69-124.
 
 Both take the (strided) slices of the layer's projections as they are; there is no torch fallback.
-Under autograd the gated norm's backward is one more HIP kernel (``gdn_gated_rmsnorm_bwd``); the gates'
-backward differentiates the same formula written in torch (``_autograd.py``).
+Under autograd the backward of either is one more HIP kernel (``gdn_gated_rmsnorm_bwd``, ``gdn_gates_bwd``).
 """
 
 from __future__ import annotations
