@@ -53,7 +53,7 @@ CYCLE_BUDGET_SOURCES = ("gdn_api.hip", "gdn_chunk.hip", "gdn_chunk_scan32_k64.hi
 
 
 def build_host_module() -> str:
-    """Compiles csrc/gdn_host.cpp, the host path of the inference entry points; always rebuilds."""
+    """Compiles csrc/gdn_host.cpp, the host path of the entry points; always rebuilds."""
     import sysconfig
 
     import torch

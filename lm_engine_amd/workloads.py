@@ -2,7 +2,7 @@
 
 Tensors are drawn on the CPU in fp32 from ``torch.Generator().manual_seed(1234 + index)`` in
 the fixed order q, k, v, b, g_raw, h0, (sequence lengths), then rounded to the configured
-dtype.  A CPU checker that consumes these (rounded) tensors sees bit-identical inputs to the
+dtype.  The oracle, which consumes these (rounded) tensors on the CPU, sees bit-identical inputs to the
 GPU path.  Shapes follow the operator contract at the reference call site
 lm_engine/modeling_utils/sequence_mixer_blocks/gated_deltanet/module.py:168-222:
 q, k ``[B, T, H, K]``, v ``[B, T, H, V]``, g fp32 ``[B, T, H]`` (log-decay <= 0),

@@ -3,7 +3,7 @@
 TEST INFRASTRUCTURE ONLY.  Nothing in the shipped package imports this
 directory: only ``tests/``, ``__graft_entry__.smoke()`` and the
 ``cpu_baseline`` leg of ``bench.py`` may call into it, and only as the
-checker, never as the thing measured or shipped.
+reference side of a comparison, never as the thing measured or shipped.
 """
 
 from .gdn_oracle import (  # noqa: F401

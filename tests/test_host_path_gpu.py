@@ -1,4 +1,4 @@
-"""The native host path of the inference entry points (csrc/gdn_host.cpp): what it hands on to the Python code, what it raises,
+"""The native host path of the entry points (csrc/gdn_host.cpp): what it hands on to the Python code, what it raises,
 and what it leaves behind.  The library's entry points are replaced by small stand-ins where a test needs a status or a look
 at the thread's state: nothing is launched then."""
 
