@@ -15,6 +15,14 @@
 // the sequence's ends held the use of every row next to its load).  Before and after, bf16, inputs from memory: 8 x 4096 tokens,
 // 2048 channels 54.5 -> 48.5 us (5.5 TB/s), 2 x 4096 21.5 -> 15.9, 4 x 4096, 6144 channels 86.4 -> 75.5, 777 tokens, 2048 channels
 // 5.7 -> 5.1; 6 x 1500, 4096 channels 29.1 both, masked 31.8 -> 31.4; fp32, 4 x 4096, 2048 channels 45.9 -> 43.5, 1 x 4096 19.3 -> 14.3.
+//
+// That way of asking had made calls of a few tokens on a carried state slower: the state came in element by element, twice (again for
+// the state that goes out), beside loads and results of tokens that were not there.  It goes in and out in 16-byte pieces now, the
+// state that goes out is picked from the registers where there are few to pick from (SHORT), and no conversion of the bias stands
+// under a branch in front of the rows' loads.  Row by row | element by element | now, back to back in a graph, bf16, 4 taps, SiLU: 256 x
+// 1 token, 6144 channels, with a state 12.0 | 27.5 | 8.0 us, without 5.3 | 6.8 | 5.2; 3000 x 1, 1024 channels 20.2 | 48.2 | 12.1; 3000 x 5, 512
+// channels 15.3 | 27.9 | 11.5; fp32, 256 x 1, 6144 channels 13.4 | 27.4 | 11.9; without a state 2 x 4096, 2048 channels, masked 22.8 |
+// 19.1 | 16.9, 4 x 1000, 2048 channels 10.8 | 9.6 | 9.4.
 
 #include <algorithm>
 #include <type_traits>
@@ -27,7 +35,7 @@ namespace gdn {
 constexpr int CONV_THREADS = 256;
 constexpr int CONV_MAX_TOKENS = 65535 * 64;  // of a row: longer ones have always been refused
 constexpr int FRONT_MASK_ROWS = 64;  // of an integer mask in the layer's front
-constexpr int CONV_TOKENS_SHORT = 4;  // tokens per thread of a batch whose waves would leave compute units idle (launch_conv_ks)
+constexpr int CONV_TOKENS_SHORT = 4;  // tokens per thread of short rows and of a batch whose waves would leave compute units idle (launch_conv_ks)
 
 struct ConvParams {
     const void* x;
@@ -51,20 +59,25 @@ struct ConvParams {
 };
 
 // TOKENS per thread of other batches: more are more registers and fewer waves, fewer read more of the halo twice.  4 x 4096 tokens,
-// 6144 channels, bf16, 5 | 6 | 8 | 12 | 16 tokens: 76.2 | 76.2 | 75.5 | 77.9 | 95.0 us; masked, 5 x 700 tokens: 8 | 12 | 16 22.4 | 21.4 | 25.4;
+// 6144 channels, bf16, 5 | 6 | 8 | 12 | 16 tokens: 76.2 | 76.2 | 75.5 | 77.9 | 95.0 us; masked, 8 | 10 | 12 (which spills): 2 x 4096, 2048
+// channels 16.9 | 18.3 | 18.3, 8 x 4096, 1024 channels 30.7 | 31.3 | 32.1, in the layer's front 6 x 1500, 4096 channels 28.6 | 28.9 | 30.2;
 // fp32, 4 x 4096 tokens, 2048 channels, 4 | 5 | 6 | 8 | 12 | 24: 43.5 | 44.2 | 45.8 | 47.5 | 48.3 | 60.0; 1 x 4096 14.3 | 15.3 at 4 | 5.
 template <typename T>
 struct ConvVec;
 template <>
 struct ConvVec<bf16_t> {
-    static constexpr int N = 8, TOKENS = 8, TOKENS_MASKED = 12;
+    static constexpr int N = 8, TOKENS = 8;
     typedef bf16x8 type;
 };
 template <>
 struct ConvVec<float> {
-    static constexpr int N = 4, TOKENS = CONV_TOKENS_SHORT, TOKENS_MASKED = CONV_TOKENS_SHORT;
+    static constexpr int N = 4, TOKENS = CONV_TOKENS_SHORT;
     typedef f32x4 type;
 };
+
+// 16 bytes of elements, aligned as one is
+template <typename T>
+using UnalignedVec = __attribute__((ext_vector_type(ConvVec<T>::N), aligned(sizeof(T)))) T;
 
 // VEC * KS weights of VEC consecutive channels are contiguous and 16-byte aligned: vector loads
 template <typename WT, int N>
@@ -83,8 +96,10 @@ __device__ __forceinline__ void load_contiguous(const void* base, int64_t first,
 
 // MASK: the rows are multiplied by the padding mask on the way in and out.  A wave's TOKENS + KS - 1 mask values are one load, a
 // value per lane, read out per row: as a load for every row and every output row they stood between the loads of x.
+// SHORT: rows behind the sequence's end are neither asked for nor formed, for calls of few tokens (an instance of its own also in fp32,
+// where the walks are as long: it takes 68 to 74 registers, the other 66 or fewer).
 // Four waves per SIMD: 112 registers at bf16 and 8 tokens.  Held to five it spills (8 x 4096 tokens, 2048 channels: 86.8 us).
-template <typename T, typename WT, int KS, bool SILU, int TOKENS, bool MASK>
+template <typename T, typename WT, int KS, bool SILU, int TOKENS, bool SHORT, bool MASK>
 __global__ __launch_bounds__(CONV_THREADS, 4) void causal_conv1d_kernel(const ConvParams p) {
     constexpr int VEC = ConvVec<T>::N;
     typedef typename ConvVec<T>::type vec_t;
@@ -128,25 +143,50 @@ __global__ __launch_bounds__(CONV_THREADS, 4) void causal_conv1d_kernel(const Co
     T* yb = reinterpret_cast<T*>(p.y) + (int64_t)b * p.y_stride_b + c0;
     float wflat[VEC * KS], bias[VEC];  // wflat[e * KS + j]: tap j of channel c0 + e
     load_contiguous<WT, VEC * KS>(p.weight, (int64_t)c0 * KS, wflat);
+    load_contiguous<WT, VEC>(p.bias == nullptr ? p.weight : p.bias, c0, bias);  // (no branch, in which its conversion would wait for it)
+#pragma unroll
+    for (int e = 0; e < VEC; e++) bias[e] = p.bias == nullptr ? 0.f : bias[e];
     vec_t rows[TOKENS + KS - 1];  // row i: token s_begin - (KS - 1) + i
+    // The carried state holds the kernel_size - 1 rows before the sequence: element e (KS - 1) + j is row j of channel c0 + e.
+    const int64_t state_at = ((int64_t)b * p.C + c0) * (KS - 1);
+    const bool carries = s_begin == 0 && p.input_state != nullptr;
+    const int tokens = s_end - s_begin;
+    auto load_state = [&]() {
 #pragma unroll
-    for (int i = 0; i < TOKENS + KS - 1; i++)
-        rows[i] = *reinterpret_cast<const vec_t*>(xb + (int64_t)min(max(s_begin - (KS - 1) + i, 0), s_end - 1) * p.x_stride_s);
-    const T* state = p.input_state == nullptr ? nullptr : reinterpret_cast<const T*>(p.input_state) + ((int64_t)b * p.C + c0) * (KS - 1);
-    // row s of the carried state or of zeros, for the kernel_size - 1 rows before the sequence
-    auto state_row = [&](int s) {
-        vec_t row;
-#pragma unroll
-        for (int e = 0; e < VEC; e++) row[e] = state == nullptr ? (T)0.f : state[e * (KS - 1) + (KS - 1) + s];
-        return row;
+        for (int i = 0; i < KS - 1; i++) rows[i] = reinterpret_cast<const UnalignedVec<T>*>(reinterpret_cast<const T*>(p.input_state) + state_at)[i];
     };
-    if (s_begin == 0) {
+    auto rows_of_state = [&]() {
+        vec_t carried[KS - 1];
 #pragma unroll
-        for (int i = 0; i < KS - 1; i++) rows[i] = state_row(i - (KS - 1));
+        for (int i = 0; i < KS - 1; i++) carried[i] = rows[i];
+#pragma unroll
+        for (int i = 0; i < KS - 1; i++)
+#pragma unroll
+            for (int e = 0; e < VEC; e++) rows[i][e] = carried[(e * (KS - 1) + i) / VEC][(e * (KS - 1) + i) % VEC];
+    };
+    auto load_row = [&](int i) { rows[i] = *reinterpret_cast<const vec_t*>(xb + (int64_t)min(max(s_begin - (KS - 1) + i, 0), s_end - 1) * p.x_stride_s); };
+    if constexpr (SHORT) {  // no load that is not needed, and the state's put in order behind all others
+#pragma unroll
+        for (int i = 0; i < KS - 1; i++) rows[i] = vec_t{};
+        if (carries) load_state();
+        if (s_begin > 0) {
+#pragma unroll
+            for (int i = 0; i < KS - 1; i++) load_row(i);
+        }
+        load_row(KS - 1);
+        if (tokens > 1) {
+#pragma unroll
+            for (int i = KS; i < TOKENS + KS - 1; i++) load_row(i);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < TOKENS + KS - 1; i++) load_row(i);
+        if (s_begin == 0) {
+#pragma unroll
+            for (int i = 0; i < KS - 1; i++) rows[i] = vec_t{};
+            if (carries) load_state(), rows_of_state();
+        }
     }
-#pragma unroll
-    for (int e = 0; e < VEC; e++) bias[e] = 0.f;
-    if (p.bias != nullptr) load_contiguous<WT, VEC>(p.bias, c0, bias);
     // lane l: mask of token s_begin - (KS - 1) + l (the halo's and this walk's; others are not asked for); rows before the sequence are taken as they are
     static_assert(TOKENS + KS - 1 <= WAVE, "a lane per mask value");
     float mask_of_lane = 1.f;
@@ -164,17 +204,49 @@ __global__ __launch_bounds__(CONV_THREADS, 4) void causal_conv1d_kernel(const Co
         return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mask_of_lane), s - s_begin + (KS - 1)));
     };
 
+    if constexpr (SHORT) {
+        if (carries) rows_of_state();
+    }
+
     float hist[KS - 1][VEC];  // hist[j]: (masked) row s - (KS - 1) + j
     auto masked_row = [&](const vec_t& v, int s, float (&row)[VEC]) {
         const float m = MASK ? mask_at(s) : 1.f;
 #pragma unroll
         for (int e = 0; e < VEC; e++) row[e] = MASK ? (float)v[e] * m : (float)v[e];
     };
+    // The last kernel_size - 1 (masked) inputs, for the next call: rows s_end - s_begin and up.  A row is picked by a number known at
+    // run time only where there are few to pick from; behind longer walks they are read once more, at the end.
+    const bool ends = p.final_state != nullptr && s_end == p.S;
+    auto store_state = [&](const vec_t (&row)[KS - 1]) {
+        UnalignedVec<T> out[KS - 1];
+#pragma unroll
+        for (int j = 0; j < KS - 1; j++) {
+            float x[VEC];
+            masked_row(row[j], p.S - (KS - 1) + j, x);
+#pragma unroll
+            for (int e = 0; e < VEC; e++) out[(e * (KS - 1) + j) / VEC][(e * (KS - 1) + j) % VEC] = (T)x[e];
+        }
+#pragma unroll
+        for (int n = 0; n < KS - 1; n++) reinterpret_cast<UnalignedVec<T>*>(reinterpret_cast<T*>(p.final_state) + state_at)[n] = out[n];
+    };
+    if constexpr (SHORT) {
+        if (ends) {
+            vec_t row[KS - 1];
+#pragma unroll
+            for (int j = 0; j < KS - 1; j++) {
+                row[j] = rows[1 + j];
+#pragma unroll
+                for (int t = 2; t <= TOKENS; t++) row[j] = tokens == t ? rows[t + j] : row[j];
+            }
+            store_state(row);
+        }
+    }
 #pragma unroll
     for (int j = 0; j < KS - 1; j++) masked_row(rows[j], s_begin - (KS - 1) + j, hist[j]);
 #pragma unroll
     for (int i = 0; i < TOKENS; i++) {
         const int s = s_begin + i;
+        if (SHORT && i >= tokens) break;
         float cur[VEC];
         masked_row(rows[i + KS - 1], s, cur);
         const float m = MASK ? mask_at(s) : 1.f;
@@ -190,20 +262,23 @@ __global__ __launch_bounds__(CONV_THREADS, 4) void causal_conv1d_kernel(const Co
             for (int j = 0; j + 1 < KS - 1; j++) hist[j][e] = hist[j + 1][e];
             hist[KS - 2][e] = cur[e];
         }
-        if (s < s_end) *reinterpret_cast<vec_t*>(yb + (int64_t)s * p.y_stride_s) = out;
+        if (SHORT || s < s_end) *reinterpret_cast<vec_t*>(yb + (int64_t)s * p.y_stride_s) = out;
     }
 
-    // the last kernel_size - 1 (masked) inputs, for the next call: read once more, so that no row is picked by a number known at run time
-    if (p.final_state != nullptr && s_end == p.S) {
-        T* fs = reinterpret_cast<T*>(p.final_state) + ((int64_t)b * p.C + c0) * (KS - 1);
+    if constexpr (!SHORT) {
+        if (ends) {
+            vec_t row[KS - 1];
 #pragma unroll
-        for (int j = 0; j < KS - 1; j++) {
-            const int s = p.S - (KS - 1) + j;
-            float row[VEC];
-            if (s >= 0) masked_row(*reinterpret_cast<const vec_t*>(xb + (int64_t)s * p.x_stride_s), s, row);
-            else masked_row(state_row(s), s, row);
+            for (int j = 0; j < KS - 1; j++) {
+                const int s = p.S - (KS - 1) + j;
+                if (s >= 0) {
+                    row[j] = *reinterpret_cast<const vec_t*>(xb + (int64_t)s * p.x_stride_s);
+                } else {
 #pragma unroll
-            for (int e = 0; e < VEC; e++) fs[e * (KS - 1) + j] = (T)row[e];
+                    for (int e = 0; e < VEC; e++) row[j][e] = carries ? reinterpret_cast<const T*>(p.input_state)[state_at + e * (KS - 1) + (KS - 1) + s] : (T)0.f;
+                }
+            }
+            store_state(row);
         }
     }
 }
@@ -224,27 +299,26 @@ static int launch_conv_ks(ConvParams p, bool silu, hipStream_t stream) {
     const int64_t groups = (p.C / ConvVec<T>::N + WAVE - 1) / WAVE;
     // the integer mask of a single row, or of single tokens, is for the prefix sums alone, as in the convolution by itself
     const bool masked = p.mask != nullptr || (p.mask_bytes != 0 && p.B > 1 && p.S > 1);
-    auto launch = [&](auto silu_tag, auto mask_tag, auto tokens_tag) -> int {
-        constexpr int TOKENS = decltype(tokens_tag)::value, SPAN = (CONV_THREADS / WAVE) * TOKENS;  // tokens per workgroup
+    auto launch = [&](auto silu_tag, auto mask_tag, auto short_tag) -> int {
+        constexpr bool SHORT = decltype(short_tag)::value, MASK = decltype(mask_tag)::value;
+        constexpr int TOKENS = SHORT ? CONV_TOKENS_SHORT : ConvVec<T>::TOKENS, SPAN = (CONV_THREADS / WAVE) * TOKENS;  // tokens per workgroup
         const int64_t workgroups = groups * ((p.S + SPAN - 1) / SPAN);
         if (workgroups * CONV_THREADS > 0xffffffff) return GDN_ERR_UNSUPPORTED;  // (a grid's x holds at most 2^32 - 1 threads; x and y of more do not fit a GPU)
         if (p.front != 0) p.front = front_planes(p, workgroups);
         const dim3 grid((unsigned)workgroups, 1, p.B + p.front);
-        hipLaunchKernelGGL((causal_conv1d_kernel<T, WT, KS, decltype(silu_tag)::value, TOKENS, decltype(mask_tag)::value>), grid, dim3(CONV_THREADS), 0, stream, p);
+        hipLaunchKernelGGL((causal_conv1d_kernel<T, WT, KS, decltype(silu_tag)::value, TOKENS, SHORT, MASK>), grid, dim3(CONV_THREADS), 0, stream, p);
         return (int)hipGetLastError();
     };
-    auto launch_with = [&](auto tokens_tag, auto mask_tag) {
-        return silu ? launch(std::true_type{}, mask_tag, tokens_tag) : launch(std::false_type{}, mask_tag, tokens_tag);
+    auto launch_with = [&](auto mask_tag, auto short_tag) {
+        return silu ? launch(std::true_type{}, mask_tag, short_tag) : launch(std::false_type{}, mask_tag, short_tag);
     };
-    typedef std::integral_constant<int, CONV_TOKENS_SHORT> few_tokens;
     // Under 1792 waves of 16 tokens (7 per compute unit) more workgroups count for more than the halo.  4 | 8 tokens a thread, bf16,
     // inputs from memory: 200 waves 5.3 | 6.1 us, 1024 9.7 | 9.8, 2000 16.3 | 15.6 (C = 2048), 2028 17.0 | 15.6 (C = 6144), 4096 28.5 | 28.2,
-    // 8192 50.6 | 48.2; masked, 4 | 12: 1584 16.3 | 17.0, 4056 31.2 | 29.9.
-    const bool few = groups * ((p.S + 15) / 16) * p.B < 1792;
-    if (masked && few) return launch_with(few_tokens{}, std::true_type{});
-    if (masked) return launch_with(std::integral_constant<int, ConvVec<T>::TOKENS_MASKED>{}, std::true_type{});
-    if (few) return launch_with(few_tokens{}, std::false_type{});
-    return launch_with(std::integral_constant<int, ConvVec<T>::TOKENS>{}, std::false_type{});
+    // 8192 50.6 | 48.2.  Rows of at most 4 tokens are one short walk however many they are: 256 x 1 token on a state, 6144 channels
+    // 8.0 | 10.9; rows of 7 are better off in one walk of 8 (3000, 512 channels, 4 taps, with a state 15.1 | 13.6).
+    const bool few = p.S <= CONV_TOKENS_SHORT || groups * ((p.S + 15) / 16) * p.B < 1792;
+    if (masked) return few ? launch_with(std::true_type{}, std::true_type{}) : launch_with(std::true_type{}, std::false_type{});
+    return few ? launch_with(std::false_type{}, std::true_type{}) : launch_with(std::false_type{}, std::false_type{});
 }
 
 template <typename T, typename WT>

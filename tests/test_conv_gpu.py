@@ -169,7 +169,32 @@ def test_long_walks_over_several_groups_of_channels_match_short_ones(dtype, C, m
     assert torch.equal(tail[0], y[5:, S - 200 :].cpu().to(F64)) and torch.equal(tail[1], s[5:].cpu().to(F64))
 
 
-# the ends of a walk of 4, 8 and 12 tokens and one past each; sequences shorter than the window
+# the state as it lies, in and out at any element, on short and on long walks, sequences shorter than the window among them
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("ks, B, S", [(2, 3, 1), (3, 3, 1), (4, 3, 1), (4, 3, 2), (3, 3, 2), (4, 3, 5), (4, 1800, 5), (3, 1800, 9)])
+def test_states_at_any_element(ks, B, S, dtype):
+    import ctypes
+
+    from lm_engine_amd import _lib
+
+    x, w, b, st, _ = (None if t is None else t.cuda() for t in _inputs(B, S, 24, ks, dtype, seed=ks + S, state=True))
+    y, s = lm_engine_amd.depthwise_causal_convolution(x, w, b, st, output_state=True)
+    moved, out = (torch.full((st.numel() + 2,), 7.0, dtype=dtype, device="cuda") for _ in range(2))
+    moved[1:-1] = st.flatten()
+    y1 = torch.empty_like(x)
+    a = _lib.GdnConvArgs()
+    a.x, a.weight, a.bias, a.y = x.data_ptr(), w.data_ptr(), b.data_ptr(), y1.data_ptr()
+    a.input_state, a.final_state = moved[1:].data_ptr(), out[1:].data_ptr()
+    a.x_stride_b, a.x_stride_s, a.y_stride_b, a.y_stride_s = S * 24, 24, S * 24, 24
+    a.B, a.S, a.C, a.kernel_size, a.activation = B, S, 24, ks, _lib.GDN_ACT_SILU
+    a.dtype = a.w_dtype = _lib.GDN_BF16 if dtype == BF16 else _lib.GDN_F32
+    print(f"case: conv states at an odd element, {B} x {S} ks={ks} {dtype}", flush=True)
+    assert _lib.load_library().gdn_causal_conv1d_fwd(ctypes.byref(a), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    assert torch.equal(y1, y) and torch.equal(out[1:-1].view(s.shape), s) and out[0] == out[-1] == 7.0
+
+
+# the ends of a walk of 4 and of 8 tokens and one past each; sequences shorter than the window
 @pytest.mark.parametrize("dtype, w_dtype", [(BF16, BF16), (BF16, F32), (F32, F32)])
 @pytest.mark.parametrize("masked", [False, True])
 @pytest.mark.parametrize("ks, S", [(4, 1), (4, 2), (4, 3), (3, 4), (2, 5), (4, 7), (4, 8), (3, 9), (4, 11), (4, 12), (4, 13), (2, 16), (4, 25)])

@@ -446,7 +446,7 @@ def test_the_layers_front_in_one_launch_gives_the_bits_of_its_steps(B, S, dtype,
     # many short rows: the gates on one plane of workgroups and on several; rows of a mask four to a wave, whole and cut, parts of rows
     [(1024, 3, 4, 4, 64, 64, None), (300, 17, 2, 4, 64, 64, None), (64, 5, 4, 4, 64, 64, torch.int64), (64, 130, 4, 4, 64, 64, torch.bool), (17, 65, 2, 2, 64, 64, torch.int32),
      (16, 1, 2, 2, 64, 64, torch.int64), (5, 300, 2, 2, 64, 64, torch.uint8), (2, 1000, 2, 2, 64, 64, torch.int64),
-     # walks of 8 and of 12 tokens that end within one, over several groups of channels, the last one whole and cut
+     # walks of 8 tokens that end within one, over several groups of channels, the last one whole and cut
      (3, 4797, 5, 5, 64, 64, None), (3, 3201, 6, 6, 64, 128, None), (3, 4797, 5, 5, 64, 64, torch.int64), (3, 4797, 5, 5, 64, 64, torch.int32), (3, 4797, 5, 5, 64, 64, torch.bool), (3, 3201, 6, 6, 64, 128, torch.int64)],
 )  # fmt: skip
 def test_the_layers_front_of_many_rows_and_of_long_walks(B, S, HK, H, K, V, mask_dtype):
