@@ -20,8 +20,11 @@
 // The workgroup is that of the half-slice scan (gdn_chunk_scan32.h): one (sequence, head) chain and one slice of 32 columns of V;
 // two compute waves with 16 columns of the state each in 16x16x32 accumulators, four loader waves that bring the next chunks
 // global -> registers -> LDS, a store wave that takes what is saved out of LDS.  What bounds it: the instruction stream of a
-// compute wave (K = 128: 38 and 60 MFMAs per chunk) and, with 256 workgroups, the memory (4 x 4096 tokens, 16 heads: 370 and 460 MB
-// that a sweep cannot do without, 3.9 and 3.8 TB/s).
+// compute wave (K = 128: 38 and 60 MFMAs per chunk), two of the four SIMDs carry none, and every slice of a chain loads the chunk's
+// records and rows of q and k again.  At K = 128, where the chains fill the chip, a workgroup therefore owns 64 columns (NC = 4):
+// a compute wave on every SIMD, one loader beside each, and the loaders also take out what is saved.  A step is then longer (2.7 us
+// loaded | 1.9 of the reverse sweep), but both sweeps of 4 x 4096 tokens, 16 heads fit the chip side by side: 206 -> 173 us, 817 MB
+// at 4.7 TB/s where a plain copy reaches 5.2; 11 packed sequences, 32768 tokens 402 -> 351.  K = 256 at 64 columns does not fit the LDS.
 
 #include <type_traits>
 
@@ -33,7 +36,7 @@ namespace gdn {
 
 namespace {
 
-constexpr int SWEEP_WAVES = 8;  // 0 1 compute | 2 3 loaders | 4 store | 5 exits at once | 6 7 loaders (as in the half-slice scan)
+constexpr int SWEEP_WAVES = 8;  // 0 1 compute | 2 3 loaders | 4 store | 5 exits at once | 6 7 loaders (as in the half-slice scan); NC = 4: 0 - 3 compute | 4 - 7 loaders
 constexpr int SWEEP_LOADERS = 4;
 
 // Order of the MFMAs of one chunk in a compute wave ("ops"), and where its side work goes; placement is the earliest-deadline
@@ -42,10 +45,11 @@ constexpr int SWEEP_LOADERS = 4;
 // Part A runs while X is formed and part B while Y is: neither depends on them.  The token tiles and slabs of the
 // triangular products are numbered in the order in which they become known: forwards in a forward sweep, backwards in a
 // reverse sweep (T^T is upper triangular), so "logical" tile t is tile 3 - t and slab s is slab 1 - s there.
-template <int K, bool REV>
+template <int K, bool REV, int NC>
 struct SweepRules {
     static constexpr int KS = K / 32, KT = K / 16;
-    static constexpr bool QS = REV && K > 128;  // rows of q in a single buffer, freed by a barrier behind part B (see the kernel)
+    static constexpr bool QS = REV && (K > 128 || (K == 128 && NC == 4));  // rows of q in a single buffer, freed by a barrier behind part B (see the kernel)
+    static constexpr bool ONE_STAGING = REV && K > 128;                     // and so are the staged saves
     static constexpr int NU = REV ? 6 : 0, NS = 4 * KS, NK = 2 * KT;
     static constexpr int NQA = !REV ? 0 : K > 128 ? 2 * KT - 8 : KT, NQB = REV ? 2 * KT - NQA : 0;
     static constexpr int OP_U = 0, OP_S = OP_U + NU, OP_QA = OP_S + NS, OP_T = OP_QA + NQA, OP_QB = OP_T + 6, OP_K = OP_QB + NQB, NOPS = OP_K + NK;
@@ -106,12 +110,12 @@ struct SweepRules {
             // reverse: ahead of this chunk's barrier, behind which the store wave takes it; forward: behind it (the store wave
             // takes it behind the next one), where a chunk of 38 MFMAs has the room
             const int t = pc - P_VST, first = OP_T + t_last(t) + DIST;
-            if (REV) return {QS && first < OP_K ? OP_K : first, OP_BAR};
+            if (REV) return {ONE_STAGING && first < OP_K ? OP_K : first, OP_BAR};
             return {first < OP_BAR + 1 ? OP_BAR + 1 : first, NOPS};
         }
         if (pc < P_SB) {
             const int s = pc - P_SST;
-            return {QS ? OP_K : OP_S + 2 * s + 1, lesser(OP_BAR, repack_first(s))};
+            return {ONE_STAGING ? OP_K : OP_S + 2 * s + 1, lesser(OP_BAR, repack_first(s))};
         }
         const int s = pc - P_SB;  // what no longer fits this chunk is packed at the start of the next (whose first chunk packs twice)
         if (repack_first(s) >= NOPS) return {lesser(repack_first(s) - NOPS, OP_S + 2 * s - 1), OP_S + 2 * s};
@@ -160,29 +164,32 @@ struct SweepRules {
     }
 };
 
-template <int K, bool REV>
-struct SweepSchedule : SweepRules<K, REV> {
-    static constexpr typename SweepRules<K, REV>::Table TABLE = SweepRules<K, REV>::make();
+template <int K, bool REV, int NC>
+struct SweepSchedule : SweepRules<K, REV, NC> {
+    static constexpr typename SweepRules<K, REV, NC>::Table TABLE = SweepRules<K, REV, NC>::make();
     static_assert(TABLE.ok, "no placement of the side work satisfies the windows");
     static constexpr int op_of(int pc) { return TABLE.op[pc]; }
 };
 
 // One workgroup of a sweep.
-template <int K, bool REV>
+template <int K, bool REV, int NC>
 struct Sweep {
-    typedef SweepSchedule<K, REV> SCH;
-    // K = 256, reverse: two stage halves with the rows of q and of k do not fit the LDS.  The rows of q, which a chunk needs for
-    // one group of MFMAs only, then get a single buffer and a second workgroup barrier per chunk ("barrier Q"), and so do
-    // the staged saves: they are written between that barrier and the chunk's own and taken out between the latter and
-    // the next barrier Q.
+    typedef SweepSchedule<K, REV, NC> SCH;
+    static_assert(NC == 2 || NC == 4, "compute waves of a workgroup");
+    static constexpr int NCOL = 16 * NC;  // columns of a workgroup
+    // K = 256, and K = 128 with four compute waves, reverse: two stage halves with the rows of q and of k do not fit the LDS.  The
+    // rows of q, which a chunk needs for one group of MFMAs only, then get a single buffer and a second workgroup barrier per chunk
+    // ("barrier Q"), and at K = 256 so do the staged saves: they are written between that barrier and the chunk's own and taken
+    // out between the latter and the next barrier Q.
     static constexpr bool QS = SCH::QS;
     static constexpr int NL = SWEEP_LOADERS;
     static constexpr int KS = SCH::KS, KT = SCH::KT;
-    // One half of the stage: fragments T' (forward: 6) or T^T | P^T (reverse: 12) | this workgroup's 32 columns of 64 rows of v or
+    // One half of the stage: fragments T' (forward: 6) or T^T | P^T (reverse: 12) | this workgroup's columns of 64 rows of v or
     // dO | rows of q (reverse) | of k | four vectors of 64 scales: ks | cs | e^{gamma_C} | - (forward), qs | ks | beta cs | e^{gamma_C}
     static constexpr int FRAGS = REV ? 12 : 6;
-    static constexpr int VLD = 64;                          // bytes per staged row of v / dO
-    static constexpr int V_UNITS = C * VLD / FRAG_BYTES;    // 1 KiB pieces: 16 rows each
+    static constexpr int VROW = 2 * NCOL;                   // bytes of a row of v / dO
+    static constexpr int VLD = NC == 2 ? VROW : VROW + 16;  // and per staged one: rows 128 bytes apart would start on two banks only
+    static constexpr int V_UNITS = C * VROW / FRAG_BYTES;   // 1 KiB pieces
     static constexpr int QLD = 2 * K + 16;                  // bytes per staged row of q / k (16 bytes of padding against bank conflicts)
     static constexpr int Q_UNITS = C * 2 * K / FRAG_BYTES;  // 1 KiB pieces of the rows of k; as many of q
     static constexpr int V_OFF = FRAGS * FRAG_BYTES;
@@ -199,30 +206,30 @@ struct Sweep {
     static constexpr int NQR = REV ? NKR : 0;
     static constexpr int NLOAD = NF + NV + NKR + NQR;
     static_assert(V_UNITS % NL == 0 && Q_UNITS % NL == 0, "the pieces must divide over the loader waves");
-    // the staged saves, transposed: [32 columns][K + 8 keys], [32 columns][64 + 8 tokens]; a compute-wave lane writes 8 consecutive
+    // the staged saves, transposed: [columns][K + 8 keys], [columns][64 + 8 tokens]; a compute-wave lane writes 8 consecutive
     // keys (its operand register as it is) or 4 consecutive tokens of one column, the store wave turns them back into rows
-    static constexpr int SCOL = (K + 8) * 2, VCOL = (C + 8) * 2, SBUFS = QS ? 1 : 2;
+    static constexpr int SCOL = (K + 8) * 2, VCOL = (C + 8) * 2, SBUFS = SCH::ONE_STAGING ? 1 : 2;
     // LDS: the stage halves | qstage | sstage | vstage
-    static constexpr int QSTAGE_OFF = 2 * STAGE_BYTES, SSTAGE_OFF = QSTAGE_OFF + (QS ? C * QLD : 0), VSTAGE_OFF = SSTAGE_OFF + SBUFS * 32 * SCOL;
-    static constexpr int LDS_BYTES = VSTAGE_OFF + SBUFS * 32 * VCOL;
+    static constexpr int QSTAGE_OFF = 2 * STAGE_BYTES, SSTAGE_OFF = QSTAGE_OFF + (QS ? C * QLD : 0), VSTAGE_OFF = SSTAGE_OFF + SBUFS * NCOL * SCOL;
+    static constexpr int LDS_BYTES = VSTAGE_OFF + SBUFS * NCOL * VCOL;
     static_assert(LDS_BYTES <= 160 * 1024 && STAGE_BYTES % 16 == 0, "stage exceeds LDS");
 
     static __device__ __forceinline__ void run(const SweepParams& p, int id, uint8_t* lds);
 };
 
-template <int K, bool REV>
-__device__ __forceinline__ void Sweep<K, REV>::run(const SweepParams& p, int id, uint8_t* const lds) {
+template <int K, bool REV, int NC>
+__device__ __forceinline__ void Sweep<K, REV, NC>::run(const SweepParams& p, int id, uint8_t* const lds) {
     uint8_t* const qstage = lds + QSTAGE_OFF;
     auto stage = [&](int i) { return lds + (i & 1) * STAGE_BYTES; };
-    auto sstage = [&](int i) { return lds + SSTAGE_OFF + (QS ? 0 : i & 1) * 32 * SCOL; };
-    auto vstage = [&](int i) { return lds + VSTAGE_OFF + (QS ? 0 : i & 1) * 32 * VCOL; };
+    auto sstage = [&](int i) { return lds + SSTAGE_OFF + (SBUFS == 1 ? 0 : i & 1) * NCOL * SCOL; };
+    auto vstage = [&](int i) { return lds + VSTAGE_OFF + (SBUFS == 1 ? 0 : i & 1) * NCOL * VCOL; };
     const int lane = threadIdx.x % WAVE;
     const int wave = threadIdx.x / WAVE;
 
     // workgroup -> (sequence-head chain, column slice), as in the scan of the forward: the slices of a chain on one XCD, the
     // chains of a packed batch dealt out longest first
     const int xcd = id % 8, rest = id / 8;
-    const int groups = p.V / 32;
+    const int groups = p.V / NCOL;
     const int vgroup = rest % groups;
     const int per_xcd = (p.N * p.H + 7) / 8;
     int n, h;
@@ -257,44 +264,46 @@ __device__ __forceinline__ void Sweep<K, REV>::run(const SweepParams& p, int id,
     // the chunk that step i of the sweep works on
     auto chunk_of = [&](int i) { return REV ? nchunks - 1 - i : i; };
 
-    const bool is_store = wave == 4;
-    const bool is_loader = wave == 2 || wave == 3 || wave >= 6;
-    if (wave == 5) return;
+    // The staged saves on their way out: rows of 32 columns (64 bytes) of one contiguous block per chunk and slice, [slice][rows][32].
+    // Lane group lane / 16 takes 8 columns of 16 consecutive rows through two transposing loads, 4 lanes per row; non-temporal, or
+    // the saves push the rows that the loaders share out of the L2.  Y goes out with its rows in reverse order, as
+    // gdn_chunk_bwd_local reads it.  Rows r0 .. r0 + 16 * COUNT - 1 of ROWS:
+    auto flush = [&](const uint8_t* staged, int ld, bf16_t* dst, int r0, auto countc, auto rowsc, auto reversec) {
+        constexpr int COUNT = decltype(countc)::value, ROWS = decltype(rowsc)::value;
+        constexpr bool REVERSE = decltype(reversec)::value;
+        const int l16 = lane % 16, piece = lane / 16;
+        const bf16_t* const m = reinterpret_cast<const bf16_t*>(staged);
+        bf16x8 x[COUNT];
+#pragma unroll
+        for (int i = 0; i < COUNT; i++) {
+            const bf16x4 lo = lds_read_tr4x16<false>(m, ld, 8 * piece, r0 + 16 * i, l16);
+            const bf16x4 hi = lds_read_tr4x16<false>(m, ld, 8 * piece + 4, r0 + 16 * i, l16);
+#pragma unroll
+            for (int e = 0; e < 4; e++) x[i][e] = lo[e], x[i][4 + e] = hi[e];
+        }
+#pragma unroll
+        for (int i = 0; i < COUNT; i++) {
+            const int row = r0 + 16 * i + l16;
+            __builtin_nontemporal_store(x[i], reinterpret_cast<bf16x8*>(dst + (REVERSE ? ROWS - 1 - row : row) * 32 + 8 * piece));
+        }
+    };
+    // slice `sl` of the workgroup's NC / 2
+    auto state_at = [&](int i, int sl) { return p.save_state + ((int64_t)chain * p.save_nc + chunk_of(i)) * K * p.V + K * 32 * (vgroup * (NC / 2) + sl); };
+    auto v_at_of = [&](int i, int sl) { return p.save_v + ((int64_t)chain * p.save_nc + chunk_of(i)) * C * p.V + C * 32 * (vgroup * (NC / 2) + sl); };
+    constexpr std::integral_constant<int, K> k_rows{};
+    constexpr std::integral_constant<int, C> c_rows{};
+    constexpr std::integral_constant<bool, REV> v_reversed{};
+    const bool is_store = NC == 2 && wave == 4;
+    const bool is_loader = NC == 2 ? (wave == 2 || wave == 3 || wave >= 6) : wave >= 4;
+    if (NC == 2 && wave == 5) return;
     if (is_store) {
         // ------------------------------ store ------------------------------
-        // rows of 32 columns (64 bytes) of one contiguous block per chunk, [slice][rows][32]: lane group lane / 16 takes 8 columns
-        // of 16 consecutive rows through two transposing loads, 4 lanes per row; non-temporal, or the saves push the rows
-        // that the loaders share out of the L2.  Y goes out with its rows in reverse order, as gdn_chunk_bwd_local reads it.
-        const int l16 = lane % 16, piece = lane / 16;
-        auto flush = [&](const uint8_t* staged, int ld, bf16_t* dst, auto rowsc, auto reversec) {
-            constexpr int ROWS = decltype(rowsc)::value;
-            constexpr bool REVERSE = decltype(reversec)::value;
-            const bf16_t* const m = reinterpret_cast<const bf16_t*>(staged);
-#pragma unroll 1
-            for (int r = 0; r < ROWS; r += 64) {
-                bf16x8 x[4];
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const bf16x4 lo = lds_read_tr4x16<false>(m, ld, 8 * piece, r + 16 * i, l16);
-                    const bf16x4 hi = lds_read_tr4x16<false>(m, ld, 8 * piece + 4, r + 16 * i, l16);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) x[i][e] = lo[e], x[i][4 + e] = hi[e];
-                }
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int row = r + 16 * i + l16;
-                    __builtin_nontemporal_store(x[i], reinterpret_cast<bf16x8*>(dst + (REVERSE ? ROWS - 1 - row : row) * 32 + 8 * piece));
-                }
-            }
-        };
+        constexpr std::integral_constant<int, 4> four{};
         auto flush_state = [&](int i) {
-            const int64_t at = ((int64_t)chain * p.save_nc + chunk_of(i)) * K * p.V + K * 32 * vgroup;
-            flush(sstage(i), SCOL / 2, p.save_state + at, std::integral_constant<int, K>{}, std::false_type{});
+#pragma unroll 1
+            for (int r = 0; r < K; r += 64) flush(sstage(i), SCOL / 2, state_at(i, 0), r, four, k_rows, std::false_type{});
         };
-        auto flush_v = [&](int i) {
-            const int64_t at = ((int64_t)chain * p.save_nc + chunk_of(i)) * C * p.V + C * 32 * vgroup;
-            flush(vstage(i), VCOL / 2, p.save_v + at, std::integral_constant<int, C>{}, std::integral_constant<bool, REV>{});
-        };
+        auto flush_v = [&](int i) { flush(vstage(i), VCOL / 2, v_at_of(i, 0), 0, four, c_rows, v_reversed); };
         __syncthreads();
         for (int i = 0; i < nchunks; i++) {
             if constexpr (QS) __syncthreads();  // barrier Q: what was staged for step i - 1 has been taken out
@@ -311,7 +320,7 @@ __device__ __forceinline__ void Sweep<K, REV>::run(const SweepParams& p, int id,
         // ------------------------------ loader ------------------------------
         // The kind of every slot is known at compile time: a branch in these loops makes the compiler wait for every load in
         // flight.  Addresses are a wave-uniform base of the chunk plus a 32-bit byte offset per lane.
-        const int lw = __builtin_amdgcn_readfirstlane(wave < 4 ? wave - 2 : wave - 4);
+        const int lw = __builtin_amdgcn_readfirstlane(NC == 2 && wave < 4 ? wave - 2 : wave - 4);
         // the slices of a chain ask for different lines at any one time (K = 256 has no registers for it)
         const int rot_f = vgroup % NF, rot_k = K > 128 ? 0 : vgroup % NKR;
         auto rotated = [](int i, int rot, int count) { return i + rot < count ? i + rot : i + rot - count; };
@@ -322,7 +331,7 @@ __device__ __forceinline__ void Sweep<K, REV>::run(const SweepParams& p, int id,
         const int hqk = qk_head_of(h, p.qk_div);
         const bf16_t* const qg = p.q + b * p.q_stride_b + seq_t0 * p.q_stride_t + (int64_t)hqk * p.q_stride_h;
         const bf16_t* const kg = p.k + b * p.k_stride_b + seq_t0 * p.k_stride_t + (int64_t)hqk * p.k_stride_h;
-        const bf16_t* const vg = p.v + b * p.v_stride_b + seq_t0 * p.v_stride_t + (int64_t)h * p.v_stride_h + 32 * vgroup;
+        const bf16_t* const vg = p.v + b * p.v_stride_b + seq_t0 * p.v_stride_t + (int64_t)h * p.v_stride_h + NCOL * vgroup;
         bf16x8 buf0[NLOAD], buf1[NLOAD];
         float sc0 = 0.f, sc1 = 0.f;  // this wave's scale vector, token `lane`
         // slots: NF fragments | NV pieces of v or dO | NKR of rows of k | NQR of rows of q
@@ -343,7 +352,7 @@ __device__ __forceinline__ void Sweep<K, REV>::run(const SweepParams& p, int id,
         };
         auto dst_of = [&](uint8_t* st, int i) -> uint8_t* {
             if (i < NF) return st + frag_of(i) * FRAG_BYTES + lane * 16;
-            if (i < NF + NV) return st + V_OFF + (lw * NV + i - NF) * FRAG_BYTES + lane * 16;
+            if (i < NF + NV) return st + V_OFF + ((lw * NV + i - NF) * V_ROWS + lane / V_PIECES) * VLD + v_piece * 16;
             const int unit = lw * NKR + rotated((i - NF - NV) % NKR, rot_k, NKR);
             const int at = (lane / Q_PIECES) * QLD + q_piece * 16 + unit * Q_ROWS * QLD;
             if (i < NF + NV + NKR) return st + K_OFF + at;
@@ -392,14 +401,38 @@ __device__ __forceinline__ void Sweep<K, REV>::run(const SweepParams& p, int id,
             else store_and_reload(buf0, sc0, 0, 0, no, no);
         }
         __syncthreads();  // stage[0] holds step 0
+        // Four compute waves leave no SIMD for a store wave: the loaders take out what is staged, each half of the rows of one slice.
+        auto flush_state = [&](int i) {
+            if constexpr (NC == 4) flush(sstage(i) + 32 * (lw / 2) * SCOL, SCOL / 2, state_at(i, lw / 2), K / 2 * (lw % 2), std::integral_constant<int, K / 32>{}, k_rows, std::false_type{});
+        };
+        auto flush_v = [&](int i) {
+            if constexpr (NC == 4) flush(vstage(i) + 32 * (lw / 2) * VCOL, VCOL / 2, v_at_of(i, lw / 2), C / 2 * (lw % 2), std::integral_constant<int, 2>{}, c_rows, v_reversed);
+        };
+        // what is complete behind the barrier of step i: the state of step i, Y of step i or V~ of step i - 1
+        auto flush_step = [&](int i, auto v_tag) {
+            flush_state(i);
+            if constexpr (REV) flush_v(i);
+            else if constexpr (decltype(v_tag)::value) flush_v(i - 1);
+        };
         // Barrier of step i: the compute waves are done with stage[i & 1] and step i + 1 is in the other half.  Before it: write
         // step i + 1 (its half was released by the barrier of step i - 1) and refill the freed registers with step i + 3.
         int i = 0;
+        if (NC == 4 && nchunks > 4) {  // two steps, the first of which has no V~ to take out yet
+            store_and_reload(buf1, sc1, 1, 3, yes, yes);
+            __syncthreads();
+            flush_step(0, no);
+            store_and_reload(buf0, sc0, 2, 4, yes, yes);
+            __syncthreads();
+            flush_step(1, yes);
+            i = 2;
+        }
         for (; i + 4 < nchunks; i += 2) {  // steady state: straight-line code, both reloads exist
             store_and_reload(buf1, sc1, i + 1, i + 3, yes, yes);
             __syncthreads();
+            flush_step(i, yes);
             store_and_reload(buf0, sc0, i + 2, i + 4, yes, yes);
             __syncthreads();
+            flush_step(i + 1, yes);
         }
         for (; i < nchunks; i += 2) {  // the last (at most four) steps; QS: each has its barrier Q
             if (i + 1 < nchunks) {
@@ -409,13 +442,17 @@ __device__ __forceinline__ void Sweep<K, REV>::run(const SweepParams& p, int id,
                 __syncthreads();
             }
             __syncthreads();
+            if (i == 0) flush_step(i, no);
+            else flush_step(i, yes);
             if (i + 1 < nchunks) {
                 if (i + 2 < nchunks) store_and_reload(buf0, sc0, i + 2, 0, no, yes);
                 else if constexpr (QS) __syncthreads();
                 __syncthreads();
+                flush_step(i + 1, yes);
             }
         }
         __syncthreads();  // the last staged V~
+        if (!REV && nchunks > 0) flush_v(nchunks - 1);
         return;
     }
 
@@ -426,8 +463,8 @@ __device__ __forceinline__ void Sweep<K, REV>::run(const SweepParams& p, int id,
     constexpr int NOPS = SCH::NOPS, OP_S = SCH::OP_S, OP_QA = SCH::OP_QA, OP_T = SCH::OP_T, OP_QB = SCH::OP_QB, OP_K = SCH::OP_K, OP_BAR = SCH::OP_BAR;
     constexpr int LA = SCH::LA;
     const int j16 = lane % 16, g = lane / 16;
-    const int half = wave;  // 0 or 1
-    const int c0 = 32 * vgroup + 16 * half;
+    const int half = wave;  // 0 .. NC - 1
+    const int c0 = NCOL * vgroup + 16 * half;
     f32x4 S[KT];
     const int64_t st_off = (int64_t)chain * K * p.V + c0 + j16;
     auto st_key = [&](int t, int r) { return 32 * (t / 2) + 8 * g + 4 * (t % 2) + r; };
@@ -627,43 +664,62 @@ __device__ __forceinline__ void Sweep<K, REV>::run(const SweepParams& p, int id,
 // forward workgroups their place, see launch_sweeps.  With many rounds of workgroups a sweep it is the gap between the launches that
 // goes: at 2 x 2048 tokens, 32 heads, V = 256 (512) the kernels alone take 196 | 202 us, calls of gdn_chunk_bwd_sweeps back to back 203
 // | 201; 8 x 2048, 16 heads, V = 128 265 | 256; 4 x 1024, 32 heads, V = 256 (1024) 187 | 186; 32 x 512, 16 heads (2048) 291 | 282.
-template <int K>
+template <int K, int NC>
 __global__ __launch_bounds__(SWEEP_WAVES* WAVE) void chunk_sweeps_kernel(const SweepParams fwd, const SweepParams rev, unsigned groups, unsigned first) {
-    constexpr int LDS = Sweep<K, true>::LDS_BYTES > Sweep<K, false>::LDS_BYTES ? Sweep<K, true>::LDS_BYTES : Sweep<K, false>::LDS_BYTES;
+    constexpr int LDS = Sweep<K, true, NC>::LDS_BYTES > Sweep<K, false, NC>::LDS_BYTES ? Sweep<K, true, NC>::LDS_BYTES : Sweep<K, false, NC>::LDS_BYTES;
     __shared__ __attribute__((aligned(16))) uint8_t lds[LDS];
     const unsigned id = blockIdx.x + first;
-    if (id < groups) Sweep<K, true>::run(rev, id, lds);
-    else Sweep<K, false>::run(fwd, id - groups, lds);
+    if (id < groups) Sweep<K, true, NC>::run(rev, id, lds);
+    else Sweep<K, false, NC>::run(fwd, id - groups, lds);
 }
 
 template <int K, bool REV>
 __global__ __launch_bounds__(SWEEP_WAVES* WAVE) void chunk_sweep_kernel(const SweepParams p) {
-    __shared__ __attribute__((aligned(16))) uint8_t lds[Sweep<K, REV>::LDS_BYTES];
-    Sweep<K, REV>::run(p, blockIdx.x, lds);
+    __shared__ __attribute__((aligned(16))) uint8_t lds[Sweep<K, REV, 2>::LDS_BYTES];
+    Sweep<K, REV, 2>::run(p, blockIdx.x, lds);
+}
+
+template <int K, int NC>
+int launch_both(const SweepParams& fwd, const SweepParams& rev, hipStream_t stream) {
+    const int64_t chains8 = ((int64_t)fwd.N * fwd.H + 7) / 8 * 8;
+    const unsigned groups = (unsigned)(chains8 * (fwd.V / (16 * NC)));
+    const dim3 block(SWEEP_WAVES * WAVE);
+    // (a launch holds at most 2^32 - 1 threads)
+    const int launches = (uint64_t)2 * groups * block.x >> 32 ? 2 : 1;
+    for (int i = 0; i < launches; i++) {
+        hipLaunchKernelGGL((chunk_sweeps_kernel<K, NC>), dim3(2 / launches * groups), block, 0, stream, fwd, rev, groups, i * groups);
+        if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
+    }
+    return GDN_OK;
 }
 
 template <int K>
 int launch_sweeps(const SweepParams& fwd, const SweepParams& rev, hipStream_t stream) {
     const int64_t chains8 = ((int64_t)fwd.N * fwd.H + 7) / 8 * 8;
     const unsigned groups = (unsigned)(chains8 * (fwd.V / 32));
-    const dim3 block(SWEEP_WAVES * WAVE);
     if constexpr (K == 64) {
         // Here two forward workgroups fit a compute unit (59 KB of LDS) and only one of both sweeps' (90 KB).  64 x 1024 tokens, 4
         // heads, two launches | one: 82 | 89 us; a packed batch, of uneven chains, gains all the same (30000 tokens, 16 heads 178 | 153).
         if (fwd.cu_seqlens == nullptr && groups > (unsigned)compute_units()) {
+            const dim3 block(SWEEP_WAVES * WAVE);
             hipLaunchKernelGGL((chunk_sweep_kernel<K, false>), dim3(groups), block, 0, stream, fwd);
             if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
             hipLaunchKernelGGL((chunk_sweep_kernel<K, true>), dim3(groups), block, 0, stream, rev);
             return (int)hipGetLastError();
         }
     }
-    // (a launch holds at most 2^32 - 1 threads)
-    const int launches = (uint64_t)2 * groups * block.x >> 32 ? 2 : 1;
-    for (int i = 0; i < launches; i++) {
-        hipLaunchKernelGGL((chunk_sweeps_kernel<K>), dim3(2 / launches * groups), block, 0, stream, fwd, rev, groups, i * groups);
-        if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
+    if constexpr (K == 128) {
+        // 64 columns to a workgroup: half as many workgroups whose step is about 1.45 times as long.  That pays unless the longest chain
+        // is what the launch waits for: its chunks against the chunks that a CU is given at 32 columns (of one sweep).  Records and
+        // sweeps at 32 | 64 columns, by that ratio.  Rows of one length: 2 x 2048 tokens, 16 heads (2.0) 63 | 82 us, 2048 tokens, 36
+        // heads (1.8) 90 | 88, 3 x 2048, 16 heads (1.3) 96 | 89, 5 x 2048 (0.8) 135 | 125, 8 x 2048 (0.5) 252 | 198, 128 x 128 (0.06) 407 |
+        // 283.  Uneven ones, longest first, which smaller workgroups fill up better: 3 sequences, 18000 tokens (2.1) 317 | 371, 6 of 11776
+        // (1.4) 160 | 174, 10 of 13312 (1.2) 201 | 193, 3 of 2548, 32 heads, V = 256 (0.8) 128 | 107, 24 of 20000 (0.4) 338 | 261.
+        const bool even = fwd.cu_seqlens == nullptr && fwd.pad_lens == nullptr;
+        const int64_t chunks = fwd.cu_seqlens == nullptr ? (int64_t)fwd.N * fwd.NT : fwd.T / C;
+        if (fwd.V % 64 == 0 && 4 * (int64_t)fwd.save_nc * compute_units() < (even ? 7 : 5) * chunks * fwd.H * (fwd.V / 32)) return launch_both<K, 4>(fwd, rev, stream);
     }
-    return GDN_OK;
+    return launch_both<K, 2>(fwd, rev, stream);
 }
 
 }  // namespace

@@ -56,6 +56,10 @@ CASES = [
     *(("rows", [T], K, 64, 2, 2) for K in (64, 128, 256) for T in (1, 63, 64, 65, 128, 192, 257, 384)),
     *(("packed", [100, 0, 64, 1, 333], K, V, 1, 2) for K, V in ((64, 64), (128, 128), (256, 64), (256, 512))),
     *(("padded", [200, 70, 0, 1], K, 128, 3, 3) for K in (64, 128, 256)),
+    # enough chains of about one length for workgroups of 64 columns (K = 128)
+    *(("rows", [T] * 5, 128, 128, 4, 8) for T in (1, 65, 192, 256, 257, 384, 449)),
+    ("packed", [100, 0, 64, 1, 333, 300, 257, 320, 130, 384], 128, 192, 4, 8),
+    ("padded", [200, 70, 0, 1], 128, 128, 7, 14),
 ]
 
 
