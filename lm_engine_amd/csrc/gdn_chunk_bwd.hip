@@ -33,6 +33,10 @@
 // K = 256 on sliced saves has one wave per SIMD and so 512 registers per lane: it asks for the
 // rows of the next slab, and of the next half of q and k, while the products of the current one run, and keeps them
 // in registers until their turn (PIPE below).
+// Bound: bytes and the trips through memory that stand in front of a barrier (882 MB at 4 x 4096 tokens, 16 heads, K = V = 128, 4.5 of
+// the 5.2 TB/s of a plain copy).  Nothing small is asked for where everybody waits for it: the tokens' scalars come while the first
+// slab's products are formed, the inverse norms of the end are kept in LDS, and at K <= 128 the rows of q and k are asked for ahead of the
+// sums behind phase 1: 204 -> 198 us; 11 packed sequences, 32768 tokens 408 -> 381.
 // K = 64, 128, 256; V a multiple of 64.
 #include <hip/hip_runtime.h>
 
@@ -200,7 +204,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
     constexpr int LDS_BYTES = cmax(PHASE1, PHASE2);
     __shared__ __attribute__((aligned(16))) uint8_t lds[LDS_BYTES];
     __shared__ __attribute__((aligned(16))) float s_gam[C], s_beta[C];  // (read 16 bytes at a time)
-    __shared__ float s_e[C], s_tail[C], s_fq[C], s_fk[C];
+    __shared__ float s_e[C], s_tail[C], s_fq[C], s_fk[C], s_rq[C];
     // Sums over waves: every wave leaves its part in a place of its own and they are added up in one order at the end (as LDS atomics
     // they stood in the waves' way - 653 -> 617 us per training step of 4 x 4096 tokens, 16 heads, K = V = 128 - and moved the
     // rounding of a few gradients from run to run).  Per token: <Y, V>; by 32 keys <dQs, Qs>, <dK, K> and the terms of dgamma and dbeta
@@ -256,15 +260,23 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 #pragma unroll
     for (int r = 0; r < 16; r++) zero[r] = 0.f;
 
-    if (t < C) {
-        const float g = p.gam[chunk * C + t];
-        s_gam[t] = g;
-        s_beta[t] = p.beta[chunk * C + t];
-        s_e[t] = __expf(g);
-        s_tail[t] = __expf(p.gam[chunk * C + C - 1] - g);
-        s_fq[t] = (p.rq != nullptr ? p.rq[chunk * C + t] : 1.f) * p.scale;  // q and k rows are scaled on their way into LDS
-        s_fk[t] = p.rk != nullptr ? p.rk[chunk * C + t] : 1.f;
-    }
+    // The tokens' scalars, by the wave that has no 64 x 64 product, while the others form the first slab's.  At the kernel's top the wave
+    // that brought them asked for its share of the slab only when they had arrived.
+    const bool norm = p.rq != nullptr;
+    auto put_scalars = [&]() {
+        int i = lane;
+        asm volatile("" : "+v"(i));  // the addresses are formed here, not ahead of phase 1 (where they would be spilled)
+        const float* const gam = p.gam + chunk * C;
+        const float gi = gam[i], last = gam[C - 1], beta = p.beta[chunk * C + i];
+        const float rq = norm ? p.rq[chunk * C + i] : 1.f, rk = norm ? p.rk[chunk * C + i] : 1.f;
+        s_gam[i] = gi;
+        s_beta[i] = beta;
+        s_e[i] = __expf(gi);
+        s_tail[i] = __expf(last - gi);
+        s_rq[i] = rq;
+        s_fq[i] = rq * p.scale;  // q and k rows are scaled on their way into LDS
+        s_fk[i] = rk;
+    };
 #ifdef GDN_CYCLE_BUDGET
     // Measurement build (python -m lm_engine_amd.build --cycle-budget): wave 0 reads the shader clock between the steps
     // of the kernel and adds the cycles of each up; sampled workgroups report at the end (the steps are named in bench.py's LOCAL_GROUPS).
@@ -521,6 +533,8 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
         if (wave != 1) {  // (the tile above the diagonal is not needed)
             DP = mma_nt(sDO + 32 * (wave / 2) * LDS64, LDS64, sVN + 32 * (wave % 2) * LDS64, LDS64, VW, DP, l32, lh);
             DA = mma_nt(sY + 32 * (wave / 2) * LDS64, LDS64, sVN + 32 * (wave % 2) * LDS64, LDS64, VW, DA, l32, lh);
+        } else if (hv == 0) {
+            put_scalars();
         }
         if constexpr (!PREFETCH && !ONE_TRIP) ask_ds1();
         LTICK(5);
@@ -557,8 +571,23 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
             for (int m = 0; m < NTW; m++)
                 dKdT[kh][m] = mma_nt(sS1 + 32 * (ktl + NKT * kh) * LDS64, LDS64, sVN + 32 * tt_of(m) * LDS64, LDS64, VW, dKdT[kh][m], l32, lh);
         LTICK(9);
+        if (ONE_TRIP && hv + 1 == V / VW) break;  // (the last barrier stands in front of phase 2)
         __syncthreads();  // the staged slab is free
         LTICK(10);
+    }
+    // K <= 128: the rows of q and k are asked for ahead of the sums and the barrier in front of phase 2
+    constexpr int CPR2 = KW / 8, RPP2 = BWD_THREADS / CPR2;
+    bf16x8 q_rows[ONE_TRIP ? C / RPP2 : 1], k_rows[ONE_TRIP ? C / RPP2 : 1];
+    if constexpr (ONE_TRIP) {
+        int tl = t;
+        asm volatile("" : "+v"(tl));  // the row addresses are formed here, not ahead of phase 1
+#pragma unroll
+        for (int it = 0; it < C / RPP2; it++) {
+            const int row = tl / CPR2 + RPP2 * it;
+            q_rows[it] = *reinterpret_cast<const bf16x8*>(qk_row_of(p.q_raw, p.q_stride_b, p.q_stride_t, p.q_stride_h, row) + 8 * (tl % CPR2));
+            k_rows[it] = *reinterpret_cast<const bf16x8*>(qk_row_of(p.k_raw, p.k_stride_b, p.k_stride_t, p.k_stride_h, row) + 8 * (tl % CPR2));
+        }
+        __builtin_amdgcn_sched_barrier(0);
     }
     dot = wave_sum(dot);
     if (lane == 0) s_red[0][wave] = dot;
@@ -568,6 +597,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
         if (t % 8 == 0) s_yv[t / 8 + 32 * it] = x;
     }
 
+    if constexpr (ONE_TRIP) __syncthreads();  // the last staged slab is free
     LTICK(11);
     // ---------------- phase 2: Q K^T, K K^T and the 64 x 64 stage ----------------
     // wave -> tile (ti, tj); rows i = 32 ti + 8 (r/4) + 4 h + r%4, column j = 32 tj + l32
@@ -588,8 +618,13 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 #pragma unroll
                 for (int it = 0; it < C / RPP; it++) {
                     const int row = t / CPR + RPP * it;
-                    bf16x8 qr = *reinterpret_cast<const bf16x8*>(qk_row_of(p.q_raw, p.q_stride_b, p.q_stride_t, p.q_stride_h, row) + KW * kh + 8 * p8);
-                    bf16x8 kr = *reinterpret_cast<const bf16x8*>(qk_row_of(p.k_raw, p.k_stride_b, p.k_stride_t, p.k_stride_h, row) + KW * kh + 8 * p8);
+                    bf16x8 qr, kr;
+                    if constexpr (ONE_TRIP) {
+                        qr = q_rows[it], kr = k_rows[it];
+                    } else {
+                        qr = *reinterpret_cast<const bf16x8*>(qk_row_of(p.q_raw, p.q_stride_b, p.q_stride_t, p.q_stride_h, row) + KW * kh + 8 * p8);
+                        kr = *reinterpret_cast<const bf16x8*>(qk_row_of(p.k_raw, p.k_stride_b, p.k_stride_t, p.k_stride_h, row) + KW * kh + 8 * p8);
+                    }
                     if (row >= valid) qr = zero8, kr = zero8;
                     const float fq = s_fq[row], fk = s_fk[row];
                     bf16x8 qb, kb;
@@ -719,7 +754,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                     acck[kh][m] = mfma32_bf16(kT[s], *reinterpret_cast<const bf16x8*>(sHT + i * LDS64 + 16 * s + 8 * lh), acck[kh][m]);
                 }
             }
-            if (p.rq != nullptr) {  // <dQs_i, Qs_i> and <dK_i, K_i> for the backward of the normalisation
+            if (norm) {  // <dQs_i, Qs_i> and <dK_i, K_i> for the backward of the normalisation
                 float dq_q = 0.f, dk_k = 0.f;
 #pragma unroll
                 for (int r = 0; r < 16; r++) {
@@ -743,8 +778,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 #pragma unroll
         for (int m = 0; m < NTW; m++) {
             const int i = 32 * tt_of(m) + l32;
-            const bool norm = p.rq != nullptr;
-            const float rq = norm ? p.rq[chunk * C + i] : 1.f, rk = norm ? p.rk[chunk * C + i] : 1.f;
+            const float rq = s_rq[i], rk = s_fk[i];
             float cq = 0.f, ck = 0.f;
             if (norm) {
 #pragma unroll
