@@ -64,7 +64,8 @@ uint64_t chunk_workspace_bytes(const gdn_args& a) {
 }
 
 // ------------------------------------------------------------------------------------------
-// chunk offsets of packed sequences: chunk_off[n] = sum_{m < n} ceil(len_m / C)
+// chunk offsets of packed sequences: chunk_off[n] = sum_{m < n} ceil(len_m / C), as a launch of their own for 64 sequences and more (and
+// for given records); the prepare step adds up fewer by itself (FindPacked)
 // ------------------------------------------------------------------------------------------
 // Lengths are taken through packed_bounds, and the running total is capped at the number of record slots
 // the workspace holds (`slots`): whatever cu_seqlens contains, no chunk gets a slot outside the workspace
@@ -239,7 +240,7 @@ int launch_chunk_fwd(const gdn_args& a, hipStream_t stream, hipEvent_t* events, 
         if (events != nullptr) (void)hipEventRecord(events[i], stream);
     };
     mark(0);
-    if (p.cu_seqlens != nullptr) {
+    if (p.cu_seqlens != nullptr && (p.records_given || !offsets_in_prepare(p.N))) {
         hipLaunchKernelGGL(chunk_offsets_kernel, dim3(1), dim3(256), 0, stream, p.cu_seqlens, p.chunk_off, p.seq_order, p.N, p.T, p.TC);
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
     }
@@ -283,7 +284,7 @@ int launch_chunk_bwd_sweeps(const gdn_args& a, const gdn_chunk_local_args& l, co
     r.v_stride_b = l.dout_stride_b, r.v_stride_t = l.dout_stride_t, r.v_stride_h = l.dout_stride_h;
     r.s_in = dht, r.s_out = dh0;
     r.save_state = static_cast<bf16_t*>(const_cast<void*>(l.dstates)), r.save_v = static_cast<bf16_t*>(const_cast<void*>(l.y_chunks));
-    if (p.cu_seqlens != nullptr) {
+    if (p.cu_seqlens != nullptr && !offsets_in_prepare(p.N)) {
         hipLaunchKernelGGL(chunk_offsets_kernel, dim3(1), dim3(256), 0, stream, p.cu_seqlens, p.chunk_off, p.seq_order, p.N, p.T, p.TC);
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
     }

@@ -165,16 +165,47 @@ struct FindInRows {
 };
 // Packed sequences.  Up to 63 of them keep their prefixes in the lanes of two registers, and a lookup is one comparison per lane; a
 // search waits for one load per step, seven of them in a row at 11 sequences (prepare, 32768 tokens, 16 heads, K = 128, at steady
-// clocks: 91 - 95 -> 84 - 88 us; 40 sequences 103 -> 98; in rows, 8 x 4096 tokens, 82 -> 81).
+// clocks: 91 - 95 -> 84 - 88 us; 40 sequences 103 -> 98; in rows, 8 x 4096 tokens, 82 -> 81).  Those few every wave adds up for itself
+// from the lengths, and one wave of the launch writes them down for the scan or the sweeps behind it (publish): a launch of its own in
+// front (chunk_offsets_kernel, which gives the same values) cost about 2 us of a forward: 3 sequences, 1000 tokens, 16 heads, K = V =
+// 128 25.2 -> 23.2 us, 5 of 2290 tokens, 3 heads, K = 256, V = 512 50.9 -> 48.6, 11 of 32768 tokens 248.6 -> 245.4.
+__host__ __device__ inline bool offsets_in_prepare(int N) { return N < WAVE; }
 struct FindPacked {
     int off = 0, cu = 0;
 
     __device__ __forceinline__ FindPacked(const ChunkParams& p, int lane) {
-        if (p.N < WAVE) off = p.chunk_off[min(lane, p.N)], cu = p.cu_seqlens[min(lane, p.N)];
+        if (!offsets_in_prepare(p.N)) return;
+        cu = p.cu_seqlens[min(lane, p.N)];
+        off = chunks(p, lane);
+        // inclusive prefix sums, capped at the record slots at every addition (as chunk_offsets_kernel's), then exclusive ones
+        off = min(off, p.TC);
+#pragma unroll
+        for (int d = 1; d < WAVE; d <<= 1) {
+            const int y = __shfl_up(off, d, WAVE);
+            if (lane >= d) off = min(off + y, p.TC);
+        }
+        off = __shfl_up(off, 1, WAVE);
+        if (lane == 0) off = 0;
+    }
+    __device__ __forceinline__ int chunks(const ChunkParams& p, int lane) const {  // of sequence `lane` (bounds as in packed_bounds)
+        const int next = __shfl_down(cu, 1, WAVE);
+        const int t0 = min(max(cu, 0), p.T), len = min(max(next, t0), p.T) - t0;
+        return lane < p.N ? (len + C - 1) / C : 0;
+    }
+    // one wave: the offsets, and the sequences by decreasing number of chunks (ties by index)
+    __device__ __forceinline__ void publish(const ChunkParams& p, int lane) const {
+        const int mine = chunks(p, lane);
+        int rank = 0;
+        for (int m = 0; m < p.N; m++) {
+            const int theirs = __builtin_amdgcn_readlane(mine, m);
+            rank += (theirs > mine || (theirs == mine && m < lane)) ? 1 : 0;
+        }
+        if (lane <= p.N) p.chunk_off[lane] = off;
+        if (lane < p.N) p.seq_order[rank] = lane;
     }
     __device__ __forceinline__ ChunkCoord operator()(const ChunkParams& p, int slot) const {
         if (slot >= p.TC) return no_chunk();
-        if (p.N < WAVE) {
+        if (offsets_in_prepare(p.N)) {
             // lanes N and up hold off[N]: bit N says that the slot lies past the last chunk, the bits below it how many sequences have begun
             const uint64_t begun = __builtin_amdgcn_ballot_w64(off <= slot);
             if (begun >> p.N & 1) return no_chunk();

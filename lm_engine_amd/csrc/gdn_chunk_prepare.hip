@@ -27,6 +27,9 @@ __global__ __launch_bounds__(PREP_THREADS, (K > 128 ? 1 : 3)) void chunk_prepare
         slot = (int)(jh * 8u + w % 8u);
     };
     const uint32_t rounds = (items - blockIdx.x + gridDim.x - 1) / gridDim.x;
+    if constexpr (std::is_same_v<Find, FindPacked>) {
+        if (offsets_in_prepare(p.N) && blockIdx.x == gridDim.x - 1 && threadIdx.x < WAVE) Find(p, threadIdx.x).publish(p, threadIdx.x);
+    }
     chunk_prepare32_body<K, 1, false, SWEEP, Find>(p, lds, item_of, items, blockIdx.x, gridDim.x, rounds, nullptr, 0, sw);
 }
 

@@ -170,6 +170,25 @@ def test_varlen_chunks_are_found_for_any_number_of_sequences(count):
     assert torch.equal(ht[lengths == 0].cpu(), inp["initial_state"][lengths == 0])
 
 
+@pytest.mark.parametrize("lengths, past", [([5], 0), ([64, 0, 64, 130], 0), ([100, 0, 65, 65, 200], 900), ([3] * 60 + [200, 0, 3], 0)])
+def test_offsets_of_few_sequences_are_those_of_many(lengths, past):
+    # Up to 63 sequences the prepare step forms the offsets and the scan's order, for more a kernel of its own: with empty sequences
+    # behind them, the same sequences take the other way.  Equal lengths, empty ones, an end past the batch (cut to it).
+    N, extra = len(lengths), 64 - len(lengths)
+    inp = _to_gpu(random_inputs(B=1, T=sum(lengths), H=2, K=64, V=64, dtype=BF16, seed=80, N=N))
+    cu = torch.tensor([0] + lengths).cumsum(0).to(torch.int32)
+    cu[-1] += past
+    h0, outcomes = inp.pop("initial_state"), []
+    for n in (0, extra):
+        leaves = {name: x.clone().requires_grad_(past == 0) for name, x in inp.items() if isinstance(x, torch.Tensor)}
+        state = torch.cat([h0, h0[:1].expand(n, -1, -1, -1)]) if n else h0
+        o, ht = lm_engine_amd.chunk_gated_delta_rule(**{**inp, **leaves}, initial_state=state, output_final_state=True, cu_seqlens=torch.cat([cu, cu[-1:].expand(n)]).cuda())
+        grads = torch.autograd.grad(o.float().square().sum() + ht[:N].sum(), list(leaves.values())) if past == 0 else ()  # (the backward refuses it)
+        outcomes.append([o, ht[:N], *grads])
+    torch.cuda.synchronize()
+    assert all(torch.equal(few, many) for few, many in zip(*outcomes))
+
+
 @pytest.mark.parametrize("K, V", [(128, 128), (64, 64), (256, 128)])
 def test_varlen_with_an_empty_sequence(K, V):
     # a sequence of length 0 has no chunk: its final state is its initial state, and its neighbours are untouched
