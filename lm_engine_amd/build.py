@@ -23,7 +23,7 @@ INCLUDE_DIR = os.path.join(os.path.dirname(PACKAGE_DIR), "include")
 LIBRARY_PATH = os.path.join(PACKAGE_DIR, "libgdn_hip.so")
 HOST_MODULE_PATH = os.path.join(PACKAGE_DIR, "gdn_host.so")
 
-SOURCES = ("gdn_api.hip", "gdn_recurrent.hip", "gdn_layer_step.hip", "gdn_chunk.hip", "gdn_chunk_prepare.hip", "gdn_chunk32.hip", "gdn_chunk_scan32_k64.hip", "gdn_chunk_scan32_k128.hip", "gdn_chunk_scan32_k256.hip", "gdn_chunk_fused.hip", "gdn_chunk_sweep.hip", "gdn_chunk_bwd.hip", "gdn_conv1d.hip", "gdn_conv1d_bwd.hip", "gdn_elementwise.hip")
+SOURCES = ("gdn_api.hip", "gdn_recurrent.hip", "gdn_layer_step.hip", "gdn_chunk.hip", "gdn_chunk_prepare.hip", "gdn_chunk32.hip", "gdn_chunk_scan32_k64.hip", "gdn_chunk_scan32_k128.hip", "gdn_chunk_scan32_k256.hip", "gdn_chunk_scan_keys.hip", "gdn_chunk_fused.hip", "gdn_chunk_sweep.hip", "gdn_chunk_bwd.hip", "gdn_conv1d.hip", "gdn_conv1d_bwd.hip", "gdn_elementwise.hip")
 
 HIPCC_FLAGS = (
     "--offload-arch=gfx950",
@@ -49,7 +49,7 @@ def _hipcc() -> str:
 
 
 CYCLE_BUDGET_LIBRARY_PATH = os.path.join(PACKAGE_DIR, "libgdn_hip_cycles.so")
-CYCLE_BUDGET_SOURCES = ("gdn_api.hip", "gdn_chunk.hip", "gdn_chunk_scan32_k64.hip", "gdn_chunk_scan32_k128.hip", "gdn_chunk_scan32_k256.hip", "gdn_chunk_bwd.hip")  # the sources that read GDN_CYCLE_BUDGET
+CYCLE_BUDGET_SOURCES = ("gdn_api.hip", "gdn_chunk.hip", "gdn_chunk_scan32_k64.hip", "gdn_chunk_scan32_k128.hip", "gdn_chunk_scan32_k256.hip", "gdn_chunk_scan_keys.hip", "gdn_chunk_bwd.hip")  # the sources that read GDN_CYCLE_BUDGET
 
 
 def build_host_module() -> str:

@@ -1,5 +1,5 @@
 // Chunked forward of the gated delta rule (K = 64, 128, 256): the choice of the scan kernel and the dispatch over the key dim.  The
-// kernels: gdn_chunk_scan32.h, a translation unit per key dim.
+// kernels: gdn_chunk_scan32.h, a translation unit per key dim, and gdn_chunk_scan_keys.hip.
 
 #include "gdn_chunk_common.h"
 #include "gdn_launch.h"
@@ -37,6 +37,10 @@ ScanPlan plan_scan(int K, int64_t chains, int V, bool packed, bool save, int rec
     plan.nw = nw;
     // a slice with a CU to itself is scanned by two waves of 16 columns each; the records are laid out for them
     plan.half = K > 128 || records_given == 2 || (nw == 1 && !records_given);
+    // K = 256, and twice as many workgroups still have a CU each: 16 columns to a workgroup and the keys over two waves, whose chunk step is a
+    // fifth shorter (forward of 4 x 777 tokens, 2 heads, V = 512, 256 workgroups 37.6 | 36.2 us; 30000 tokens, 3 heads 856 | 726).  More
+    // workgroups would run in rounds.
+    plan.split_keys = plan.half && !save && K == 256 && (chains + 7) / 8 * 8 * (V / 16) <= (int64_t)num_cus;
     // Saves go through LDS and the store wave in the half-slice scan: always at K <= 128; at K = 256 only in the scan
     // without output (no rows of q in LDS), with bf16 V~, and fp32 states at every second chunk at most (one buffer).
     plan.staged_saves = save && plan.half &&

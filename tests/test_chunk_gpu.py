@@ -367,6 +367,27 @@ def test_config4_long_context_full_size():
     assert torch.equal(h2, ht)
 
 
+# K = 256 with up to 256 workgroups of 16 columns: the scan whose keys are split over two waves.  One to seven chunks (its loaders' ring
+# fills and drains differently up to five), first and last token of a chunk, one to many column groups, shared heads of q and k
+@pytest.mark.parametrize("T, V, HK, H", [(1, 32, 1, 1), (63, 64, 1, 2), (64, 512, 2, 2), (65, 512, 3, 3), (129, 96, 2, 4), (192, 512, 2, 2), (257, 64, 4, 4), (321, 512, 1, 2), (448, 512, 2, 2)])
+def test_split_keys_at_the_edges_of_chunks(T, V, HK, H):
+    inp = random_inputs(B=2, T=T, H=H, K=256, V=V, dtype=BF16, seed=90 + T)
+    q, k = (inp[n][:, :, :HK] for n in ("q", "k"))
+    wide = dict(inp, q=q.repeat_interleave(H // HK, dim=2), k=k.repeat_interleave(H // HK, dim=2))
+    o_ref, h_ref = recurrent_gated_delta_rule_c(**wide, output_final_state=True)
+    gpu = _to_gpu(dict(inp, q=q.contiguous(), k=k.contiguous()))
+    print(f"case: split keys T={T} V={V} heads {HK} / {H}", flush=True)
+    o, ht = lm_engine_amd.chunk_gated_delta_rule(**gpu, output_final_state=True)
+    torch.cuda.synchronize()
+    assert_parity(o.float(), o_ref, BF16, "o")
+    assert_parity(ht, h_ref, BF16, "final_state")
+    if T > 64:  # a chunk's arithmetic does not depend on its place: a run cut behind the first chunk gives the same bits
+        part = lambda s: {n: (x[:, s] if n in ("q", "k", "v", "g", "beta") else x) for n, x in gpu.items()}  # noqa: E731
+        first, state = lm_engine_amd.chunk_gated_delta_rule(**part(slice(0, 64)), output_final_state=True)
+        second, end = lm_engine_amd.chunk_gated_delta_rule(**dict(part(slice(64, None)), initial_state=state), output_final_state=True)
+        assert torch.equal(torch.cat([first, second], dim=1), o) and torch.equal(end, ht)
+
+
 def test_shipped_head_shape_full_size():
     # the head shape of the reference's shipped configurations (k_head_dim 256, v_head_dim 512, 2 heads, micro-batch 8,
     # T = 4096; configs/research/m2rnn/400m-normal/gated-deltanet.yml:60-73): the half-slice scan with a single buffer
