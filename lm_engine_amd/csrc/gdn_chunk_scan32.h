@@ -496,22 +496,23 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
         // The compute waves leave the bf16 output tile of chunk c in LDS while they work on chunk c + 1; this
         // wave writes it out after the next barrier.  A store that waits for queue space then stalls here and
         // not in the wave that feeds the matrix pipe.
-        const int row0 = lane / 4, piece = lane % 4;
+        // All slices of a row together: with two of them whole 128-byte lines, 8 lanes a row and 8 rows a store.  Slice by slice, as
+        // halves of lines, the stores held up the loaders' reads beside them: 11 packed sequences, 32768 tokens, 16 heads, K = V = 128 245
+        // -> 231 us for the forward.  (One slice: its neighbour's workgroup writes the other half.)
+        constexpr int O_LANES = 4 * NW, O_ROWS = WAVE / O_LANES;  // lanes per row, rows per store
+        const int row0 = lane / O_LANES, piece = lane % O_LANES;
         bf16_t* og = p.o + b * p.o_stride_b + (seq_t0 + row0) * p.o_stride_t + (int64_t)h * p.o_stride_h +
                      32 * (vgroup * NW) + 8 * piece;
         auto flush = [&](int c) {  // output of chunk c
             const int valid = (int)min((int64_t)C, seq_len - (int64_t)c * C);
+            bf16x8 rows[C / O_ROWS];
 #pragma unroll
-            for (int w = 0; w < NW; w++) {
-                bf16x8 rows[4];
+            for (int i = 0; i < C / O_ROWS; i++)
+                rows[i] = *reinterpret_cast<const bf16x8*>(ostage_at(piece / 4, c & 1, row0 + O_ROWS * i, piece % 4));
 #pragma unroll
-                for (int i = 0; i < 4; i++)
-                    rows[i] = *reinterpret_cast<const bf16x8*>(ostage_at(w, c & 1, row0 + 16 * i, piece));
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    if (row0 + 16 * i < valid)
-                        __builtin_nontemporal_store(rows[i], reinterpret_cast<bf16x8*>(og + ((int64_t)c * C + 16 * i) * p.o_stride_t + 32 * w));
-            }
+            for (int i = 0; i < C / O_ROWS; i++)
+                if (row0 + O_ROWS * i < valid)
+                    __builtin_nontemporal_store(rows[i], reinterpret_cast<bf16x8*>(og + ((int64_t)c * C + O_ROWS * i) * p.o_stride_t));
         };
         // LSAVE, bf16 saves: staged as [32 columns][ld rows]; out as rows of 32 columns (64 bytes): lane group `piece`
         // (16 lanes) takes columns 8 piece .. + 7 of 16 consecutive rows through two transposing loads (4 columns x 16 rows
