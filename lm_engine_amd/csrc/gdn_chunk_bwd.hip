@@ -36,7 +36,7 @@
 // Bound: bytes and the trips through memory that stand in front of a barrier (882 MB at 4 x 4096 tokens, 16 heads, K = V = 128, 4.5 of
 // the 5.2 TB/s of a plain copy).  Nothing small is asked for where everybody waits for it: the tokens' scalars come while the first
 // slab's products are formed, the inverse norms of the end are kept in LDS, and at K <= 128 the rows of q and k are asked for ahead of the
-// sums behind phase 1: 204 -> 198 us; 11 packed sequences, 32768 tokens 408 -> 381.
+// sums behind phase 1: 204 -> 198 us; 11 packed sequences, 32768 tokens 408 -> 381.  dq and dk leave in whole rows: 198 -> 192, 381 -> 372.
 // K = 64, 128, 256; V a multiple of 64.
 #include <hip/hip_runtime.h>
 
@@ -773,8 +773,11 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 
     // With x = y / r the normalised row (y: input, r = |y|^-1 incl. epsilon): dy = r (dx - x <x, dx>); the scale of
     // q moves through: Qs = scale Qn, so dQn = scale dQs and Qn <Qn, dQn> = Qs <Qs, dQs> / scale.
+    // dq and dk go through LDS (the rows of q and k are no longer needed) and out as whole rows: a lane has 8 keys of one token, and stored from
+    // there an instruction wrote 32 bytes of each of 32 rows.
 #pragma unroll
-    for (int kh = 0; kh < KH; kh++)
+    for (int kh = 0; kh < KH; kh++) {
+        if (kh > 0) __syncthreads();  // the rows of the previous half are out
 #pragma unroll
         for (int m = 0; m < NTW; m++) {
             const int i = 32 * tt_of(m) + l32;
@@ -786,8 +789,6 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                 cq *= rq / p.scale, ck *= rk;
             }
             const float rqs = rq * p.scale;
-            bf16_t* const dq = p.dq_out + (tok0 + i) * p.dqk_stride_t + (int64_t)h * K + KW * kh + 32 * ktl + 8 * lh;
-            bf16_t* const dk = p.dk_out + (tok0 + i) * p.dqk_stride_t + (int64_t)h * K + KW * kh + 32 * ktl + 8 * lh;
 #pragma unroll
             for (int r8 = 0; r8 < 2; r8++) {  // registers 8 r8 + 4 x + e: keys 16 r8 + 8 x + 4 h + e
                 bf16x4 oq[2], ok[2];
@@ -799,13 +800,22 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                         oq[x][e] = (bf16_t)(accq[kh][m][r] * rqs - cq * (float)qv[kh][m][r8][r % 8]);
                         ok[x][e] = (bf16_t)(acck[kh][m][r] * rk - ck * (float)kv[kh][m][r8][r % 8]);
                     }
-                const bf16x8 q8 = eight_keys(oq[0], oq[1]), k8 = eight_keys(ok[0], ok[1]);
-                if (i < valid) {
-                    *reinterpret_cast<bf16x8*>(dq + 16 * r8) = q8;
-                    *reinterpret_cast<bf16x8*>(dk + 16 * r8) = k8;
-                }
+                *reinterpret_cast<bf16x8*>(sQ + i * LDK + 32 * ktl + 8 * lh + 16 * r8) = eight_keys(oq[0], oq[1]);
+                *reinterpret_cast<bf16x8*>(sK + i * LDK + 32 * ktl + 8 * lh + 16 * r8) = eight_keys(ok[0], ok[1]);
             }
         }
+        __syncthreads();
+        constexpr int CPR = KW / 8, RPP = BWD_THREADS / CPR;  // 16-byte pieces per row, rows per pass
+#pragma unroll
+        for (int it = 0; it < C / RPP; it++) {
+            const int row = t / CPR + RPP * it, at = row * LDK + 8 * (t % CPR);
+            if (row < valid) {
+                const int64_t to = (tok0 + row) * p.dqk_stride_t + (int64_t)h * K + KW * kh + 8 * (t % CPR);
+                *reinterpret_cast<bf16x8*>(p.dq_out + to) = *reinterpret_cast<const bf16x8*>(sQ + at);
+                *reinterpret_cast<bf16x8*>(p.dk_out + to) = *reinterpret_cast<const bf16x8*>(sK + at);
+            }
+        }
+    }
 
     if (t < C) {  // wave 0
         // (the tile above the diagonal has no sums)
