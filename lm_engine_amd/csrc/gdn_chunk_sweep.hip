@@ -658,8 +658,8 @@ __device__ __forceinline__ void Sweep<K, REV, NC>::run(const SweepParams& p, int
 
 // Both sweeps in one launch: neither needs anything of the other, so with fewer workgroups than compute units they run side by
 // side, and with more the forward sweep's first workgroups start on the units that the reverse sweep's last ones leave idle.  The
-// reverse sweep comes first, its chunks are the longer ones.  `first`: the number of the launch's first workgroup.  Kernel times, two
-// launches | one: 4 x 4096 tokens, 16 heads, K = V = 128 (256 workgroups a sweep) 220 | 208 us, 2 x 4096 142 | 107, 2184 tokens 77 | 45;
+// reverse sweep comes first, its chunks are the longer ones.  `first`: the number of the launch's first workgroup.  Kernel times at 32
+// columns to a workgroup, two launches | one: 4 x 4096 tokens, 16 heads, K = V = 128 (256 workgroups a sweep) 220 | 208 us, 2 x 4096 142 | 107, 2184 tokens 77 | 45;
 // 11 packed sequences, 32768 tokens 428 | 397; 9000 tokens, 3 heads, K = 256, V = 512 467 | 289.  Slower only where one launch takes
 // forward workgroups their place, see launch_sweeps.  With many rounds of workgroups a sweep it is the gap between the launches that
 // goes: at 2 x 2048 tokens, 32 heads, V = 256 (512) the kernels alone take 196 | 202 us, calls of gdn_chunk_bwd_sweeps back to back 203
