@@ -626,7 +626,7 @@ def bench_backward(w, inp, steps, warmup):
         "steps": steps,
         "ms_per_backward": round(ms, 3),
         "tokens_per_s": round(inp["q"].size(0) * inp["q"].size(1) / (ms * 1e-3), 1),
-        "composition": ("3 kernel launches (packed sequences: and their chunk offsets): per-chunk records, forward and reverse "
+        "composition": ("3 kernel launches (64 packed sequences or more: and their chunk offsets): per-chunk records, forward and reverse "
                         "sweep in one launch, chunk-local gradients; chunk states, V~ and Y pass between them as bf16"
                         if backward_kernels_apply(w.K, w.V) else
                         "2 saving scans + rocBLAS batched GEMMs + elementwise torch ops"),

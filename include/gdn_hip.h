@@ -398,7 +398,7 @@ int gdn_chunk_bwd_prepare(const gdn_chunk_bwd_prepare_args *args, void *stream);
 /*
  * Training support, fourth part: everything gdn_chunk_bwd_local needs from the states, in one call - per-chunk records, the forward
  * sweep (the states the chunks start from, V~) and the reverse sweep (the gradients of the states they end with, Y).  Two launches:
- * the records, and both sweeps in one; one more for the chunk offsets of packed sequences, and one more where K = 64 and a sweep
+ * the records, and both sweeps in one; one more for the chunk offsets of 64 packed sequences and more, and one more where K = 64 and a sweep
  * of rows has more workgroups than the GPU compute units: the sweeps are a launch each then.  What gdn_chunk_bwd_prepare and two calls of gdn_chunk_fwd_saving arrive at through a mirror problem, in one step per
  * chunk, for every batch that gdn_chunk_fwd takes (fixed-length rows of any length, packed, left-padded; qk_heads as there):
  * bf16, K = 64, 128 or 256, V a multiple of 64 (GDN_ERR_UNSUPPORTED otherwise).
@@ -417,7 +417,7 @@ uint64_t gdn_chunk_bwd_sweeps_workspace_bytes(const gdn_args *args);
  * Measurement aid, no counterpart in the reference: runs exactly what gdn_chunk_fwd runs, with a
  * HIP event recorded on `stream` before and after every kernel, waits for the last one and
  * returns each kernel's duration in milliseconds in kernel_ms[GDN_CHUNK_KERNELS], in launch
- * order: [0] chunk offsets of packed sequences (0 when cu_seqlens is NULL), [1] prepare, [2] scan.
+ * order: [0] chunk offsets of 64 packed sequences and more (else about 0), [1] prepare, [2] scan.
  * Unlike every other entry point it creates events and blocks the calling thread.
  */
 #define GDN_CHUNK_KERNELS 3
