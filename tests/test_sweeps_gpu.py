@@ -58,6 +58,7 @@ CASES = [
     *(("padded", [200, 70, 0, 1], K, 128, 3, 3) for K in (64, 128, 256)),
     # enough chains of about one length for workgroups of 64 columns (K = 128)
     *(("rows", [T] * 5, 128, 128, 4, 8) for T in (1, 65, 192, 256, 257, 384, 449)),
+    ("rows", [65] * 10, 128, 64, 4, 8),
     ("packed", [100, 0, 64, 1, 333, 300, 257, 320, 130, 384], 128, 192, 4, 8),
     ("padded", [200, 70, 0, 1], 128, 128, 7, 14),
 ]
