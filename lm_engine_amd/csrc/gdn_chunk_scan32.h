@@ -87,7 +87,7 @@ constexpr int SCAN_LOADERS = 4;
 // So with fewer than four compute waves the waves that land on their SIMDs get the light jobs:
 //   NW = 1:  0 compute | 1 2 3 loaders | 4 output store | 5 loader
 //   NW = 2:  0 1 compute | 2 3 loaders | 4 output store | 5 exits at once | 6 7 loaders
-//   NW = 4:  0..3 compute | 4..7 loaders (each compute wave shares with one loader; no output wave)
+//   NW = 4:  0..3 compute | 4..7 loaders (each compute wave shares with one loader), which also write the output
 //   NW = 1, HALF:  0 1 compute (16 columns each) | the rest as for NW = 2
 __host__ __device__ constexpr int scan_waves(int nw, bool half = false) { return nw == 1 && !half ? 6 : 8; }
 
@@ -340,8 +340,10 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
     constexpr bool QS = K > 128 && HASQ;
     static_assert(K <= 128 || HALF, "K = 256 runs as half slices");
     constexpr int NL = SCAN_LOADERS;
-    // a separate wave writes the output (see below); with four compute waves the LDS has no room for its staging
+    // The output goes through LDS and is written by a wave of its own (see below), with four compute waves by the loaders.  (A saving scan with
+    // four compute waves stores from these.)
     constexpr bool OS = NW < 4;
+    constexpr bool STAGED = OS || !SAVE;
     constexpr int KD = K / 32;    // 32-row tiles of the state
     constexpr int KS16 = K / 16;  // 16-wide slabs over the key dim
     // One half of the stage: [T diag(beta) 6 | P 6] (the head of the record) | the chunk's 64 rows of this
@@ -367,7 +369,7 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
     constexpr int NQ = (HASQ ? 2 : 1) * Q_UNITS / NL;   // q / k row slots per loader wave
     constexpr int NLOAD = NF + NV + NQ;    // 1 KiB moves per loader wave and chunk
     static_assert(SHARED_FRAGS % NL == 0 && V_UNITS % NL == 0 && (2 * Q_UNITS) % NL == 0, "the pieces must divide over the loader waves");
-    constexpr int OSTAGE_BYTES = (OS && !NOOUT) ? NW * 2 * C * 64 : 16;
+    constexpr int OSTAGE_BYTES = (STAGED && !NOOUT) ? NW * 2 * C * 64 : 16;
     static_assert(2 * STAGE_BYTES + (QS ? C * QLD : 0) + OSTAGE_BYTES <= 160 * 1024, "stage exceeds LDS");
 
     __shared__ __attribute__((aligned(16))) uint8_t stage[2][STAGE_BYTES];
@@ -757,13 +759,46 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
         // Barrier of iteration c: the compute waves are done with stage[c & 1] and chunk c + 1 is in the
         // other half.  Before it: write chunk c + 1 (its half was released by the barrier of iteration
         // c - 1) and refill the freed registers with chunk c + 3.
+        // Four compute waves: a loader writes tokens 16 lw .. 16 lw + 15 of the output, whole rows of the workgroup's 128 columns, 16 lanes a row.
+        // From the compute waves a store wrote 32 bytes of each of 32 rows, and waited for room in the memory queue where the products
+        // should be issued.  Forward, K = 128: 7 x 2048 tokens, 32 heads, V = 256
+        // 264 -> 253 us, 128 x 256, 16 heads, V = 128 265 -> 246, 16 x 2048 199 -> 196, 24 packed sequences, 32768 tokens 248 -> 227.
+        constexpr bool LOADERS_STORE = STAGED && !OS;
+        auto put_output = [&](int c, int valid) {
+            if constexpr (LOADERS_STORE) {
+                int l = lane;
+                asm volatile("" : "+v"(l));  // the addresses are formed here, not ahead of the loop (where they would be spilled)
+                bf16_t* const og = p.o + b * p.o_stride_b + (seq_t0 + (int64_t)c * C + 16 * lw) * p.o_stride_t + (int64_t)h * p.o_stride_h + 32 * (vgroup * NW);
+                const int64_t at = (int64_t)(l / 16) * p.o_stride_t + 8 * (l % 16);
+#pragma unroll
+                for (int i = 0; i < 4; i += 2) {
+                    bf16x8 rows[2];
+#pragma unroll
+                    for (int j = 0; j < 2; j++) rows[j] = *reinterpret_cast<const bf16x8*>(ostage_at(l / 4 % 4, c & 1, 16 * lw + 4 * (i + j) + l / 16, l % 4));
+#pragma unroll
+                    for (int j = 0; j < 2; j++)
+                        if (16 * lw + 4 * (i + j) + l / 16 < valid)
+                            __builtin_nontemporal_store(rows[j], reinterpret_cast<bf16x8*>(og + 4 * (i + j) * p.o_stride_t + at));
+                }
+            }
+        };
         int c = 0;
         // (QS: every iteration has barrier Q as well: inside store_and_reload, or on its own when nothing is left to write)
+        if (LOADERS_STORE && nchunks > 4) {  // two chunks, the first of which has no output to write
+            store_and_reload(buf1, sc1, 1, 3, yes, yes);
+            __syncthreads();
+            store_and_reload(buf0, sc0, 2, 4, yes, yes);
+            __syncthreads();
+            put_output(0, C);
+            c = 2;
+        }
         for (; c + 4 < nchunks; c += 2) {  // steady state: straight-line code, both reloads exist
             store_and_reload(buf1, sc1, c + 1, c + 3, yes, yes);
             __syncthreads();
+            put_output(c - 1, C);
             store_and_reload(buf0, sc0, c + 2, c + 4, yes, yes);
             __syncthreads();
+            put_output(c, C);
         }
         for (; c < nchunks; c += 2) {  // the last (at most four) chunks
             if (c + 1 < nchunks) {
@@ -773,13 +808,16 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
                 __syncthreads();
             }
             __syncthreads();
+            if (c > 0) put_output(c - 1, C);
             if (c + 1 < nchunks) {
                 if (c + 2 < nchunks) store_and_reload(buf0, sc0, c + 2, 0, no, yes);
                 else if constexpr (QS) __syncthreads();
                 __syncthreads();
+                put_output(c, C);
             }
         }
-        if (OS) __syncthreads();  // the hand-over of the last output tile
+        if (STAGED) __syncthreads();  // the hand-over of the last output tile
+        if (LOADERS_STORE && nchunks > 0) put_output(nchunks - 1, (int)(seq_len - (int64_t)(nchunks - 1) * C));
         return;
     }
 
@@ -1206,7 +1244,7 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
             } else if constexpr (pc >= SCH::P_OUT && pc < SCH::P_OUT + SCH::N_OUT) {
                 // output tile tt of the previous chunk, registers 8 half .. 8 half + 7
                 constexpr int i = pc - SCH::P_OUT, tt = i / 2, half = i % 2;
-                if (OS) {
+                if (STAGED) {
                     if (c > 0)
                         *reinterpret_cast<bf16x8*>(ostage_at(wave, (c - 1) & 1, 32 * tt + l32, 2 * half + lh)) =
                             pack8_16(acco[tt], half, 1.f);
@@ -1334,7 +1372,7 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
     for (int tt = 0; tt < 2; tt++)
 #pragma unroll
         for (int half = 0; half < 2; half++) {
-            if (OS) {
+            if (STAGED) {
                 if (nchunks > 0)
                     *reinterpret_cast<bf16x8*>(ostage_at(wave, (nchunks - 1) & 1, 32 * tt + l32, 2 * half + lh)) =
                         pack8_16(acco[tt], half, 1.f);
@@ -1343,7 +1381,7 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
                     pack8_16(acco[tt], half, 1.f);
             }
         }
-    if (OS) __syncthreads();
+    if (STAGED) __syncthreads();
 
     if (p.ht != nullptr) {
 #pragma unroll

@@ -367,6 +367,12 @@ def test_config4_long_context_full_size():
     assert torch.equal(h2, ht)
 
 
+# four slices to a workgroup, whose loaders write the output: one to eight chunks, first and last token of a chunk
+@pytest.mark.parametrize("T", [1, 63, 64, 65, 129, 192, 257, 321, 449])
+def test_four_slices_at_the_edges_of_chunks(T):
+    _check(random_inputs(B=9, T=T, H=16, K=64, V=128, dtype=BF16, seed=120 + T), "four slices")
+
+
 # K = 256 with up to 256 workgroups of 16 columns: the scan whose keys are split over two waves.  One to seven chunks (its loaders' ring
 # fills and drains differently up to five), first and last token of a chunk, one to many column groups, shared heads of q and k
 @pytest.mark.parametrize("T, V, HK, H", [(1, 32, 1, 1), (63, 64, 1, 2), (64, 512, 2, 2), (65, 512, 3, 3), (129, 96, 2, 4), (192, 512, 2, 2), (257, 64, 4, 4), (321, 512, 1, 2), (448, 512, 2, 2)])
