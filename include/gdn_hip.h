@@ -403,6 +403,7 @@ int gdn_chunk_bwd_prepare(const gdn_chunk_bwd_prepare_args *args, void *stream);
  * chunk, for every batch that gdn_chunk_fwd takes (fixed-length rows of any length, packed, left-padded; qk_heads as there):
  * bf16, K = 64, 128 or 256, V a multiple of 64 (GDN_ERR_UNSUPPORTED otherwise).
  *   args   as for gdn_chunk_fwd; h0, g, beta may be NULL; ht is not used and o not written (it must be a valid pointer and strides);
+ *          T of packed sequences is best the tokens that they hold: the width of a workgroup goes by the chunks of T;
  *          workspace of gdn_chunk_bwd_sweeps_workspace_bytes, 256-byte aligned, nothing in it has to be cleared
  *   local  the arrays that gdn_chunk_bwd_local will read are written here: v_new, states, dstates, y_chunks (bf16, saves_sliced),
  *          gamma, beta, rq, rk (all four; rq and rk are 1 without GDN_FLAG_L2NORM); H, K, V, NC, chunks = N H NC describe them, with

@@ -349,17 +349,17 @@ def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm
     from . import ops  # late: ops imports this module
 
     B, T = q.shape[:2]
-    covers = True  # every token belongs to a sequence
+    tokens = B * T  # that belong to a sequence
     sequences = None
     if cu_seqlens is not None:
         starts, lens = _chains(B, T, cu_seqlens, left_padded)
         NC = max(1, -(-max(lens + [1]) // CHUNK))
-        covers = sum(lens) == B * T
+        tokens = sum(lens)
         sequences = (*ops.upload_int32((starts, lens), q.device), NC)
     if is_kernel_allowed(Kernel.gated_delta_rule):  # (else ops.chunk_bwd_sweeps refuses the call)
         flags = (_lib.GDN_FLAG_L2NORM if l2norm else 0) | (_lib.GDN_FLAG_LEFT_PADDED if left_padded else 0)
         grads = host().delta_rule_bwd(raw_stream(q.get_device()), q, k, v, g, beta, initial_state, cu_seqlens, do, dht, scale, flags,
-                                      *(sequences or (None, None, 0)), covers, joined)  # fmt: skip
+                                      *(sequences or (None, None, 0)), tokens, joined)  # fmt: skip
         if grads is not None:
             return grads
     if cu_seqlens is None:
@@ -375,9 +375,10 @@ def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm
     do = kernel_rows(do.to(torch.bfloat16))
     if do.stride(1) > 1 << 24:  # the kernels count a chunk's rows in 32 bits; q, k and v were held to that by the forward
         do = do.contiguous()
-    prep, S0, Vn, dS1, Y, dh0 = ops.chunk_bwd_sweeps(q, k, v, do, g, beta, scale, l2norm, initial_state, cu_seqlens, left_padded, dht, NC)
+    prep, S0, Vn, dS1, Y, dh0 = ops.chunk_bwd_sweeps(q, k, v, do, g, beta, scale, l2norm, initial_state, cu_seqlens, left_padded, dht, NC,
+                                                  tokens=tokens)  # fmt: skip
     dq, dk, dv, dg, dbeta = ops.chunk_local_grads(q, k, v, do, prep, Y, Vn, S0, dS1, scale, l2norm, sequences, sliced=True,
-                                                  covers=covers, joined=joined)  # fmt: skip
+                                                  covers=tokens == B * T, joined=joined)  # fmt: skip
     if group > 1:
         dq, dk = (_fold(d, heads, group) for d in (dq, dk))
     return (

@@ -679,6 +679,37 @@ __global__ __launch_bounds__(SWEEP_WAVES* WAVE) void chunk_sweep_kernel(const Sw
     Sweep<K, REV, 2>::run(p, blockIdx.x, lds);
 }
 
+}  // namespace
+
+// Columns of a workgroup at K = 128; `longest`: chunks of the longest sequence, `chunks`: of all rows together.
+//
+// 64 columns are half as many workgroups whose step is about 1.45 times as long.  That pays unless the longest chain is what the launch waits
+// for: its chunks against the chunks that a CU is given at 32 columns (of one sweep).  Records and sweeps at 32 | 64 columns, by that ratio.
+// Rows of one length: 2 x 2048 tokens, 16 heads (2.0) 63 | 82 us, 2048 tokens, 36 heads (1.8) 90 | 88, 3 x 2048, 16 heads (1.3) 96 | 89, 5 x
+// 2048 (0.8) 135 | 125, 8 x 2048 (0.5) 252 | 198, 128 x 128 (0.06) 407 | 283.  Packed ones, dealt out longest first, which smaller workgroups
+// fill up better: 3 sequences, 18000 tokens (2.1) 317 | 371, 6 of 11776 (1.4) 160 | 174, 10 of 13312 (1.2) 201 | 193, 3 of 2548, 32 heads, V
+// = 256 (0.8) 128 | 107, 24 of 20000 (0.4) 338 | 261.  Tokens behind the last sequence are nobody's: the rows count for no more than
+// the sequences can have (one of 4000 tokens in a row of 32768: 97 | 140).
+//
+// Left-padded rows, whose lengths the host does not have here: one of them may be all there is, and the rows' chains go to the XCDs in the
+// order of the batch.  Where the chains of one row do not fit their XCD side by side at 32 columns, both sweeps of it, they queue for
+// its CUs and 64 columns win however the tokens lie: 26 x 2048, 5 heads, V = 128, one row full, the others 64 tokens 92 | 85, every length 189
+// | 169; 8 x 2048, 16 heads 168 | 135, V = 64 98 | 92; 43 x 2048, 3 heads, V = 256 109 | 96.  Where they fit, 32 columns are the
+// safe side: 32 x 2048, 4 heads, V = 128 86 | 102 and 189 | 159; 16 x 2048, 8 heads, V = 64 80 | 102 and 117 | 125; 48 x 2048, 2 heads, V =
+// 256 84 | 94 and 237 | 191.
+int sweep_columns_k128(int N, int H, int V, int longest, int64_t chunks, bool packed, bool padded, int num_cus) {
+    const int64_t slices = V / 32, possible = (int64_t)N * longest;
+    if (V % 64 != 0) return 32;
+    if (padded) {
+        const int64_t per_xcd = ((int64_t)N * H + 7) / 8, chains = H < per_xcd ? H : per_xcd;  // of one row, on one XCD
+        if (2 * chains * slices <= num_cus / 8) return 32;
+    }
+    if (chunks > possible) chunks = possible;
+    return 4 * (int64_t)longest * num_cus < (packed || padded ? 5 : 7) * chunks * H * slices ? 64 : 32;
+}
+
+namespace {
+
 template <int K, int NC>
 int launch_both(const SweepParams& fwd, const SweepParams& rev, hipStream_t stream) {
     const int64_t chains8 = ((int64_t)fwd.N * fwd.H + 7) / 8 * 8;
@@ -709,15 +740,9 @@ int launch_sweeps(const SweepParams& fwd, const SweepParams& rev, hipStream_t st
         }
     }
     if constexpr (K == 128) {
-        // 64 columns to a workgroup: half as many workgroups whose step is about 1.45 times as long.  That pays unless the longest chain
-        // is what the launch waits for: its chunks against the chunks that a CU is given at 32 columns (of one sweep).  Records and
-        // sweeps at 32 | 64 columns, by that ratio.  Rows of one length: 2 x 2048 tokens, 16 heads (2.0) 63 | 82 us, 2048 tokens, 36
-        // heads (1.8) 90 | 88, 3 x 2048, 16 heads (1.3) 96 | 89, 5 x 2048 (0.8) 135 | 125, 8 x 2048 (0.5) 252 | 198, 128 x 128 (0.06) 407 |
-        // 283.  Uneven ones, longest first, which smaller workgroups fill up better: 3 sequences, 18000 tokens (2.1) 317 | 371, 6 of 11776
-        // (1.4) 160 | 174, 10 of 13312 (1.2) 201 | 193, 3 of 2548, 32 heads, V = 256 (0.8) 128 | 107, 24 of 20000 (0.4) 338 | 261.
-        const bool even = fwd.cu_seqlens == nullptr && fwd.pad_lens == nullptr;
-        const int64_t chunks = fwd.cu_seqlens == nullptr ? (int64_t)fwd.N * fwd.NT : fwd.T / C;
-        if (fwd.V % 64 == 0 && 4 * (int64_t)fwd.save_nc * compute_units() < (even ? 7 : 5) * chunks * fwd.H * (fwd.V / 32)) return launch_both<K, 4>(fwd, rev, stream);
+        const bool packed = fwd.cu_seqlens != nullptr;
+        if (sweep_columns_k128(fwd.N, fwd.H, fwd.V, fwd.save_nc, packed ? fwd.T / C : (int64_t)fwd.N * fwd.NT, packed, fwd.pad_lens != nullptr, compute_units()) == 64)
+            return launch_both<K, 4>(fwd, rev, stream);
     }
     return launch_both<K, 2>(fwd, rev, stream);
 }

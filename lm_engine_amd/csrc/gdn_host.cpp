@@ -484,9 +484,9 @@ void need_rows(const at::Tensor& t, int64_t stride_elements, size_t address_byte
     for (int64_t i = 0; i + 1 < t.dim(); i++) need(t.stride(i) % stride_elements == 0);
 }
 
-// delta_rule_bwd(stream, q, k, v, g, beta, initial_state, cu_seqlens, do, dht, scale, flags, seq_start, seq_len, NC, covers, joined)
+// delta_rule_bwd(stream, q, k, v, g, beta, initial_state, cu_seqlens, do, dht, scale, flags, seq_start, seq_len, NC, tokens, joined)
 //   -> (dq, dk, dv, dg, dbeta, dh0)
-// Rows of a batch: without seq_start and seq_len.  Else NC chunks for the longest sequence; covers: every token belongs to one.
+// Rows of a batch: without seq_start and seq_len.  Else NC chunks for the longest sequence; tokens: how many belong to one.
 // joined: dq, dk and dv as column blocks of one tensor, where v has no more heads than q and k.
 PyObject* delta_rule_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return fast_path(n, 17, [&]() -> PyObject* {
@@ -495,7 +495,8 @@ PyObject* delta_rule_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const at::Tensor &q = operand(args[1]), &k = operand(args[2]), &v = operand(args[3]), &d = operand(args[8]);
         const at::Tensor *g = operand.optional(args[4]), *beta = operand.optional(args[5]), *h0 = operand.optional(args[6]), *cu = operand.optional(args[7]);
         const at::Tensor *dht = operand.optional(args[9]), *seq_start = operand.optional(args[12]), *seq_len = operand.optional(args[13]);
-        const bool covers = truth(args[15]), joined = truth(args[16]);
+        const int64_t tokens = integer(args[15]);
+        const bool joined = truth(args[16]);
         gdn_args s{};
         gdn_chunk_local_args l{};
         s.dtype = code_of(q), s.flags = (int32_t)integer(args[11]);
@@ -519,7 +520,8 @@ PyObject* delta_rule_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
         } else {
             need(!padded);
         }
-        need(NC > 0);
+        need(NC > 0 && tokens >= 0 && tokens <= B * T);
+        const bool covers = tokens == B * T;
         l.T_rows = size32(T);
         if (g != nullptr) need(g->scalar_type() == at::kFloat && g->sizes() == at::IntArrayRef({B, T, H}) && g->is_contiguous());
         s.beta_dtype = GDN_F32;
@@ -531,6 +533,7 @@ PyObject* delta_rule_bwd(PyObject*, PyObject* const* args, Py_ssize_t n) {
         for (const at::Tensor* t : states)
             if (t != nullptr) need(t->scalar_type() == at::kFloat && t->sizes() == at::IntArrayRef({N, H, K, V}) && t->is_contiguous() && aligned(ptr(t), 16));
         s.B = size32(B), s.T = size32(T), s.H = size32(H), s.K = (int32_t)K, s.V = size32(V), s.N = size32(N), s.chunk = 64;
+        if (cu != nullptr && !padded && !covers) s.T = std::max((int32_t)tokens, 1);  // (tokens behind the last sequence are no work to count on)
         s.qk_heads = HK == H ? 0 : (int32_t)HK;
         s.cu_seqlens = static_cast<const int32_t*>(ptr(cu));
         s.scale = (float)number(args[10]);

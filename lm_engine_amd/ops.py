@@ -595,9 +595,10 @@ def chunk_local_grads(q, k, v, dout, prep, y_mirror, v_new, states, dstates, sca
     return out["dq_out"], out["dk_out"], out["dv_out"], out["dg_out"], out["dbeta_out"]
 
 
-def chunk_bwd_sweeps(q, k, v, dout, g, beta, scale, l2norm, initial_state, cu_seqlens, left_padded, dht, chunks_per_chain):
+def chunk_bwd_sweeps(q, k, v, dout, g, beta, scale, l2norm, initial_state, cu_seqlens, left_padded, dht, chunks_per_chain, tokens=None):
     """``gdn_chunk_bwd_sweeps``: q, k, v, dout are the caller's bf16 ``[B, T, H, D]`` tensors (last dim contiguous), ``dht`` the
-    gradient of the final state or None, ``chunks_per_chain`` (NC) at least the chunks of the longest sequence.  Returns
+    gradient of the final state or None, ``chunks_per_chain`` (NC) at least the chunks of the longest sequence, ``tokens``
+    those that belong to a sequence where the caller knows (a packed row is walked no further).  Returns
     ``prep`` (``gamma, beta, rq, rk`` fp32 ``[N H, NC, 64]``) and, bf16 by 32-column slice, the states the chunks start from, V~, the
     gradients of the states they end with and Y with its tokens reversed - ``chunk_local_grads(..., sliced=True)`` takes them all -
     and the gradient of the initial state (None without one).  Chunks past the end of their sequence have no entries."""
@@ -617,6 +618,8 @@ def chunk_bwd_sweeps(q, k, v, dout, g, beta, scale, l2norm, initial_state, cu_se
     v_new, y = (torch.empty(N * H, NC, 64, V, dtype=torch.bfloat16, device=dev) for _ in range(2))
     dh0 = None if h0 is None else torch.empty(N, H, K, V, dtype=torch.float32, device=dev)
     args = _fill_args(q, k, v, g, beta, h0, None, v, cu_seqlens, scale, l2norm, False, dims, left_padded)  # (no output is written)
+    if cu_seqlens is not None and not left_padded and tokens is not None:
+        args.T = max(tokens, 1)
     workspace = torch.empty(int(lib.gdn_chunk_bwd_sweeps_workspace_bytes(ctypes.byref(args))), dtype=torch.uint8, device=dev)
     args.workspace, args.workspace_bytes = workspace.data_ptr(), workspace.numel()
     a = _lib.GdnChunkLocalArgs()

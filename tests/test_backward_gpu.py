@@ -624,3 +624,28 @@ def test_forward_records_are_exact_up_to_their_own_rounding(lens, K, l2norm):
         ratio = (error[name] / rounded[name]) ** 0.5
         print(f"   {name}: error / rounding {ratio:.3f}", flush=True)
         assert ratio <= 1.05, name
+
+
+@pytest.mark.parametrize("K, V", [(64, 64), (128, 128), (256, 64)])
+@pytest.mark.parametrize("lengths, rest", [([70, 0, 130], 500), ([64], 1), ([1, 0], 64), ([0, 0], 70)])
+@pytest.mark.parametrize("cu_dtype", [torch.int32, torch.int64])  # (int64: without the native host path)
+def test_tokens_behind_the_last_sequence_change_nothing(K, V, lengths, rest, cu_dtype):
+    # the sweeps walk the tokens of the sequences only: the same gradients as without the rest of the row, and zeros there
+    from lm_engine_amd.backward import gated_delta_rule_backward
+
+    gen = torch.Generator().manual_seed(K + rest)
+    live, H, N = sum(lengths), 2, len(lengths)
+    q, k, v, do = (torch.randn(1, live + rest, H, n, generator=gen).to(torch.bfloat16).cuda() for n in (K, K, V, V))
+    g, beta = -torch.rand(1, live + rest, H, generator=gen).cuda(), torch.rand(1, live + rest, H, generator=gen).to(torch.bfloat16).cuda()
+    h0, dht = torch.randn(N, H, K, V, generator=gen).cuda(), torch.randn(N, H, K, V, generator=gen).cuda()
+    cu = torch.tensor([0, *lengths]).cumsum(0).to(cu_dtype).cuda()
+    print(f"case: {rest} tokens behind {lengths}, K={K} V={V}", flush=True)
+
+    def grads(tokens):
+        cut = (x[:, :tokens] for x in (q, k, v, g, beta, do))
+        return gated_delta_rule_backward(*cut, dht, None, h0, cu, True)
+
+    for name, whole, cut in zip(("dq", "dk", "dv", "dg", "dbeta"), grads(live + rest), grads(max(live, 1))):
+        assert torch.equal(whole[:, :live], cut[:, :live]), name
+        assert (whole[:, live:] == 0).all(), f"{name} behind the last sequence"
+    assert torch.equal(grads(live + rest)[5], grads(max(live, 1))[5])

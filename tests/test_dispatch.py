@@ -1,0 +1,31 @@
+"""Which kernel a launch takes, at the places where both sides were measured (256 compute units)."""
+
+import pytest
+
+from tests.dispatch import sweep_columns
+
+
+@pytest.mark.parametrize(
+    "N, H, V, longest, chunks, layout, columns",
+    [
+        (4, 16, 128, 64, 256, "rows", 64),
+        (2, 16, 128, 32, 64, "rows", 32),
+        (11, 16, 128, 99, 512, "packed", 64),
+        (21, 16, 128, 32, 51, "packed", 32),   # one sequence of 2000 tokens, 20 of 64
+        (1, 16, 128, 63, 512, "packed", 32),   # one of 4000 tokens in a row of 32768: the rest of the row is nobody's
+        (2, 32, 128, 63, 78, "packed", 32),    # 4000 and 1000 tokens
+        # left-padded, only one row of them full as far as the host knows: whether its chains fit an XCD side by side
+        (6, 16, 128, 64, 6 * 64, "padded", 64),
+        (26, 5, 128, 32, 26 * 32, "padded", 64),
+        (32, 4, 128, 32, 32 * 32, "padded", 32),
+        (8, 16, 64, 32, 8 * 32, "padded", 64),
+        (16, 8, 64, 32, 16 * 32, "padded", 32),
+        (43, 3, 256, 32, 43 * 32, "padded", 64),
+        (48, 2, 256, 32, 48 * 32, "padded", 32),
+        (7, 14, 128, 4, 7 * 64, "padded", 64),  # rows of 4096 tokens, none of which uses more than 256
+        (2, 16, 128, 4, 2 * 64, "padded", 32),
+        (4, 16, 96, 64, 256, "rows", 32),      # whole slices of 64 columns only
+    ],
+)
+def test_width_of_the_sweeps(N, H, V, longest, chunks, layout, columns):
+    assert sweep_columns(N, H, V, longest, chunks, layout == "packed", layout == "padded") == columns
