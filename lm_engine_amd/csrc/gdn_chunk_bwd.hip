@@ -33,10 +33,13 @@
 // K = 256 on sliced saves has one wave per SIMD and so 512 registers per lane: it asks for the
 // rows of the next slab, and of the next half of q and k, while the products of the current one run, and keeps them
 // in registers until their turn (PIPE below).
-// Bound: bytes and the trips through memory that stand in front of a barrier (882 MB at 4 x 4096 tokens, 16 heads, K = V = 128, 4.5 of
-// the 5.2 TB/s of a plain copy).  Nothing small is asked for where everybody waits for it: the tokens' scalars come while the first
-// slab's products are formed, the inverse norms of the end are kept in LDS, and at K <= 128 the rows of q and k are asked for ahead of the
-// sums behind phase 1: 204 -> 198 us; 11 packed sequences, 32768 tokens 408 -> 381.  dq and dk leave in whole rows: 198 -> 192, 381 -> 372.
+// Bound: bytes and the trips through memory that stand in front of a barrier (882 MB at 4 x 4096 tokens, 16 heads, K = V = 128, 4.6 of
+// the 5.2 TB/s of a plain copy).  Nothing small is asked for where everybody waits for it: the tokens' scalars come at K <= 128 while the
+// first slab's products are formed, at K = 256 ahead of the prefetch (loads return in order), the inverse norms of the end are kept in
+// LDS, and at K <= 128 the rows of q and k are asked for ahead of the sums behind phase 1: 204 -> 198 us; 11 packed sequences, 32768 tokens
+// 408 -> 381.  There dq and dk also leave in whole rows: 198 -> 192, 381 -> 372 (K = 64, 4 x 4096 tokens, 16 heads, V = 128, both steps 140 -> 132).
+// At K = 256 their way through LDS costs more than it saves: 8 x 4096 tokens, 2 heads, V = 512 240 us through LDS, 237 without, V = 128, 4
+// heads 215 and 209, 4096 tokens, 3 heads, V = 512 48.1 and 47.2; the scalars behind the prefetch 242, 221 and 49.0 (through LDS).
 // K = 64, 128, 256; V a multiple of 64.
 #include <hip/hip_runtime.h>
 
@@ -260,8 +263,9 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 #pragma unroll
     for (int r = 0; r < 16; r++) zero[r] = 0.f;
 
-    // The tokens' scalars, by the wave that has no 64 x 64 product, while the others form the first slab's.  At the kernel's top the wave
-    // that brought them asked for its share of the slab only when they had arrived.
+    // The tokens' scalars, by the wave that has no 64 x 64 product: at K <= 128 while the others form the first slab's (at the kernel's top
+    // the wave that brought them asked for its share of the slab only when they had arrived), at K = 256, where by then the next slab is
+    // asked for and they would wait for it, at the top.
     const bool norm = p.rq != nullptr;
     auto put_scalars = [&]() {
         int i = lane;
@@ -358,6 +362,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
             *reinterpret_cast<bf16x8*>(sK + row * LDK + 8 * p8) = kb;
         }
     };
+    if (K > 128 && wave == 1) put_scalars();
     float yv[2] = {0.f, 0.f};  // this thread's part of <Y_i, V_i>, rows t / 8 and t / 8 + 32
     if constexpr (PIPE) ask_slab(0);
 #pragma unroll 1
@@ -533,7 +538,7 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
         if (wave != 1) {  // (the tile above the diagonal is not needed)
             DP = mma_nt(sDO + 32 * (wave / 2) * LDS64, LDS64, sVN + 32 * (wave % 2) * LDS64, LDS64, VW, DP, l32, lh);
             DA = mma_nt(sY + 32 * (wave / 2) * LDS64, LDS64, sVN + 32 * (wave % 2) * LDS64, LDS64, VW, DA, l32, lh);
-        } else if (hv == 0) {
+        } else if (K <= 128 && hv == 0) {
             put_scalars();
         }
         if constexpr (!PREFETCH && !ONE_TRIP) ask_ds1();
@@ -773,11 +778,10 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
 
     // With x = y / r the normalised row (y: input, r = |y|^-1 incl. epsilon): dy = r (dx - x <x, dx>); the scale of
     // q moves through: Qs = scale Qn, so dQn = scale dQs and Qn <Qn, dQn> = Qs <Qs, dQs> / scale.
-    // dq and dk go through LDS (the rows of q and k are no longer needed) and out as whole rows: a lane has 8 keys of one token, and stored from
-    // there an instruction wrote 32 bytes of each of 32 rows.
+    // K <= 128: dq and dk go through LDS (the rows of q and k are no longer needed) and out as whole rows: a lane has 8 keys of one token, and
+    // stored from there an instruction wrote 32 bytes of each of 32 rows.
 #pragma unroll
-    for (int kh = 0; kh < KH; kh++) {
-        if (kh > 0) __syncthreads();  // the rows of the previous half are out
+    for (int kh = 0; kh < KH; kh++)
 #pragma unroll
         for (int m = 0; m < NTW; m++) {
             const int i = 32 * tt_of(m) + l32;
@@ -800,17 +804,25 @@ __global__ __launch_bounds__(BWD_THREADS, (K <= 128 ? 2 : 1)) void chunk_local_g
                         oq[x][e] = (bf16_t)(accq[kh][m][r] * rqs - cq * (float)qv[kh][m][r8][r % 8]);
                         ok[x][e] = (bf16_t)(acck[kh][m][r] * rk - ck * (float)kv[kh][m][r8][r % 8]);
                     }
-                *reinterpret_cast<bf16x8*>(sQ + i * LDK + 32 * ktl + 8 * lh + 16 * r8) = eight_keys(oq[0], oq[1]);
-                *reinterpret_cast<bf16x8*>(sK + i * LDK + 32 * ktl + 8 * lh + 16 * r8) = eight_keys(ok[0], ok[1]);
+                const bf16x8 q8 = eight_keys(oq[0], oq[1]), k8 = eight_keys(ok[0], ok[1]);
+                if constexpr (K <= 128) {
+                    *reinterpret_cast<bf16x8*>(sQ + i * LDK + 32 * ktl + 8 * lh + 16 * r8) = q8;
+                    *reinterpret_cast<bf16x8*>(sK + i * LDK + 32 * ktl + 8 * lh + 16 * r8) = k8;
+                } else if (i < valid) {
+                    const int64_t to = (tok0 + i) * p.dqk_stride_t + (int64_t)h * K + KW * kh + 32 * ktl + 8 * lh + 16 * r8;
+                    *reinterpret_cast<bf16x8*>(p.dq_out + to) = q8;
+                    *reinterpret_cast<bf16x8*>(p.dk_out + to) = k8;
+                }
             }
         }
+    if constexpr (K <= 128) {
         __syncthreads();
-        constexpr int CPR = KW / 8, RPP = BWD_THREADS / CPR;  // 16-byte pieces per row, rows per pass
+        constexpr int CPR = K / 8, RPP = BWD_THREADS / CPR;  // 16-byte pieces per row, rows per pass
 #pragma unroll
         for (int it = 0; it < C / RPP; it++) {
             const int row = t / CPR + RPP * it, at = row * LDK + 8 * (t % CPR);
             if (row < valid) {
-                const int64_t to = (tok0 + row) * p.dqk_stride_t + (int64_t)h * K + KW * kh + 8 * (t % CPR);
+                const int64_t to = (tok0 + row) * p.dqk_stride_t + (int64_t)h * K + 8 * (t % CPR);
                 *reinterpret_cast<bf16x8*>(p.dq_out + to) = *reinterpret_cast<const bf16x8*>(sQ + at);
                 *reinterpret_cast<bf16x8*>(p.dk_out + to) = *reinterpret_cast<const bf16x8*>(sK + at);
             }
