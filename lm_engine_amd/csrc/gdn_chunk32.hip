@@ -14,7 +14,7 @@ extern template int launch32<256>(ChunkParams& p, hipStream_t stream, hipEvent_t
 
 // Which scan kernel a launch gets: compute waves (32-column slices) per workgroup, and whether a slice is split over
 // two half-slice waves.
-ScanPlan plan_scan(int K, int64_t chains, int V, bool packed, bool save, int records_given, int num_cus, const SaveRequest& req) {
+ScanPlan plan_scan(int K, int64_t chains, int T, int V, bool packed, bool save, int records_given, int num_cus, const SaveRequest& req) {
     // Slices per scan workgroup: one while that gives no more workgroups than CUs, so that every slice has a CU's load
     // bandwidth to itself; otherwise 2 or 4 slices of a chain share the records through one workgroup's LDS (they must
     // divide the V / 32 tiles).
@@ -41,6 +41,12 @@ ScanPlan plan_scan(int K, int64_t chains, int V, bool packed, bool save, int rec
     // fifth shorter (forward of 4 x 777 tokens, 2 heads, V = 512, 256 workgroups 37.6 | 36.2 us; 30000 tokens, 3 heads 856 | 726).  More
     // workgroups would run in rounds.
     plan.split_keys = plan.half && !save && K == 256 && (chains + 7) / 8 * 8 * (V / 16) <= (int64_t)num_cus;
+    // Four slices to a workgroup, rows of two to four chunks: what goes through LDS is stored a chunk later, with nothing left to compute beside
+    // it, and a short last chunk leaves the memory idle before.  Through LDS | from the compute waves, 16 heads, K = V = 128: 20 x 65 tokens 31.7 |
+    // 30.4 us, 20 x 160 43.1 | 41.0, 40 x 200 76.2 | 75.2, 100 x 65 105 | 100, 100 x 90 110 | 106, K = 64, 40 x 65 39.6 | 38.4.  The loaders
+    // are better where the chunks are full or many workgroups' stores crowd each other: 20 x 256 50.1 | 49.9, 40 x 256 79.0 | 79.5, 100 x 127 120 |
+    // 123, 100 x 200 177 | 182, K = 64, 100 x 127 89.4 | 90.5, 40 x 200 57.5 | 59.4; and with one chunk, 20 x 64 25.4 | 25.6.
+    plan.direct = nw == 4 && !save && !packed && T > C && (T <= 2 * C - C / 4 || (K == 128 && T < 4 * C && chains * (vtiles / nw) <= 3 * (int64_t)num_cus));
     // Saves go through LDS and the store wave in the half-slice scan: always at K <= 128; at K = 256 only in the scan
     // without output (no rows of q in LDS), with bf16 V~, and fp32 states at every second chunk at most (one buffer).
     plan.staged_saves = save && plan.half &&

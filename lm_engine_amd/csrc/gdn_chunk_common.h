@@ -93,6 +93,7 @@ struct ScanPlan {
     int nw;             // 32-column slices per workgroup
     bool half;          // a slice is scanned by two waves of 16 columns (records in the 16x16x32 fragment order)
     bool split_keys;    // ... and by two more for the other half of the keys, 16 columns to a workgroup (gdn_chunk_scan_keys.hip)
+    bool direct;        // four slices per workgroup: the compute waves store the output themselves
     bool staged_saves;  // a saving scan whose saves go through LDS and the store wave: only there bf16 saves exist
     bool no_output;     // the scan without output runs
 };
@@ -101,7 +102,7 @@ struct SaveRequest {
     bool no_output = false, has_state = true, has_vnew = true, state_bf16 = false, vnew_bf16 = false;
     int save_every = 1;
 };
-ScanPlan plan_scan(int K, int64_t chains, int V, bool packed, bool save, int records_given, int num_cus, const SaveRequest& req);
+ScanPlan plan_scan(int K, int64_t chains, int T, int V, bool packed, bool save, int records_given, int num_cus, const SaveRequest& req);
 
 struct RecordLayout {
     uint32_t off_p, off_qs, off_ks, off_cs, off_eg, bytes;

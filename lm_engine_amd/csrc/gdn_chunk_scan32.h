@@ -326,7 +326,9 @@ struct Scan16Schedule : Scan16Rules<K, NOOUT> {
 //
 // NOOUT (with SAVE and HALF, K <= 128): the scan writes no output and skips the products that form it; what it saves (the
 // state every chunk starts from, V~) is all it is run for.  The loaders still stage the whole record and the rows of q.
-template <int K, int NW, bool NT = false, bool SAVE = false, bool HALF = false, bool NOOUT = false>
+//
+// DIRECT (four compute waves): these store the output themselves (ScanPlan::direct).
+template <int K, int NW, bool NT = false, bool SAVE = false, bool HALF = false, bool NOOUT = false, bool DIRECT = SAVE && NW == 4>
 __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kernel(const ChunkParams p) {
     static_assert(!HALF || NW == 1, "the half-slice scan has one slice per workgroup");
     static_assert(!NOOUT || (SAVE && HALF && K >= 128), "the scan without output is the saving half-slice scan at K = 128 or 256");
@@ -341,9 +343,10 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
     static_assert(K <= 128 || HALF, "K = 256 runs as half slices");
     constexpr int NL = SCAN_LOADERS;
     // The output goes through LDS and is written by a wave of its own (see below), with four compute waves by the loaders.  (A saving scan with
-    // four compute waves stores from these.)
+    // four compute waves, and one of a few chunks, stores from these.)
+    static_assert(!DIRECT || NW == 4, "fewer compute waves have a store wave beside them");
     constexpr bool OS = NW < 4;
-    constexpr bool STAGED = OS || !SAVE;
+    constexpr bool STAGED = !DIRECT;
     constexpr int KD = K / 32;    // 32-row tiles of the state
     constexpr int KS16 = K / 16;  // 16-wide slabs over the key dim
     // One half of the stage: [T diag(beta) 6 | P 6] (the head of the record) | the chunk's 64 rows of this
@@ -1414,7 +1417,7 @@ int launch32(ChunkParams& p, hipStream_t stream, hipEvent_t* events, int num_cus
     SaveRequest req;
     req.no_output = p.no_output != 0, req.has_state = p.save_state != nullptr, req.has_vnew = p.save_vnew != nullptr;
     req.state_bf16 = p.save_state_bf16 != 0, req.vnew_bf16 = p.save_vnew_bf16 != 0, req.save_every = p.save_every;
-    const ScanPlan plan = plan_scan(K, chains, p.V, p.cu_seqlens != nullptr, save, p.records_given, num_cus, req);
+    const ScanPlan plan = plan_scan(K, chains, p.T, p.V, p.cu_seqlens != nullptr, save, p.records_given, num_cus, req);
     const int nw = plan.nw;
     const bool half = plan.half;
     if ((p.save_state_bf16 || p.save_vnew_bf16) && !plan.staged_saves) return GDN_ERR_UNSUPPORTED;  // (the C entry asks plan_scan first)
@@ -1441,7 +1444,9 @@ int launch32(ChunkParams& p, hipStream_t stream, hipEvent_t* events, int num_cus
         else hipLaunchKernelGGL((chunk_scan32_kernel<K, 1, false, true>), grid, dim3(scan_waves(1) * WAVE), 0, stream, p);
         return (int)hipGetLastError();
     }
-    if (nw == 4 && p.scan_groups == 1) hipLaunchKernelGGL((chunk_scan32_kernel<K, 4, true>), grid, dim3(scan_waves(4) * WAVE), 0, stream, p);
+    if (plan.direct && p.scan_groups == 1) hipLaunchKernelGGL((chunk_scan32_kernel<K, 4, true, false, false, false, true>), grid, dim3(scan_waves(4) * WAVE), 0, stream, p);
+    else if (plan.direct) hipLaunchKernelGGL((chunk_scan32_kernel<K, 4, false, false, false, false, true>), grid, dim3(scan_waves(4) * WAVE), 0, stream, p);
+    else if (nw == 4 && p.scan_groups == 1) hipLaunchKernelGGL((chunk_scan32_kernel<K, 4, true>), grid, dim3(scan_waves(4) * WAVE), 0, stream, p);
     else if (nw == 4) hipLaunchKernelGGL((chunk_scan32_kernel<K, 4>), grid, dim3(scan_waves(4) * WAVE), 0, stream, p);
     else if (nw == 2) hipLaunchKernelGGL((chunk_scan32_kernel<K, 2>), grid, dim3(scan_waves(2) * WAVE), 0, stream, p);
     else hipLaunchKernelGGL((chunk_scan32_kernel<K, 1, false, false, true>), grid, dim3(scan_waves(1, true) * WAVE), 0, stream, p);  // (a lone slice: two half-slice waves, plan_scan)

@@ -14,6 +14,7 @@ import lm_engine_amd
 from lm_engine_amd import _lib, ops
 from lm_engine_amd.workloads import get_workload, make_inputs
 from oracle.c_oracle import recurrent_gated_delta_rule_c
+from tests.dispatch import scan_plan
 from tests.helpers import assert_parity, max_abs, random_inputs, rel_l2
 
 
@@ -371,6 +372,30 @@ def test_config4_long_context_full_size():
 @pytest.mark.parametrize("T", [1, 63, 64, 65, 129, 192, 257, 321, 449])
 def test_four_slices_at_the_edges_of_chunks(T):
     _check(random_inputs(B=9, T=T, H=16, K=64, V=128, dtype=BF16, seed=120 + T), "four slices")
+
+
+# two to four chunks, where the compute waves of four slices store the output: with one workgroup to a chain and with two, left-padded rows with
+# zeros written at the padding; the loaders' kernel, which longer rows take, gives the same bits for the tokens it shares
+@pytest.mark.parametrize("K, B, H, V, T", [(64, 9, 16, 128, 65), (64, 9, 16, 128, 112), (128, 17, 16, 128, 65), (128, 17, 16, 128, 129), (128, 17, 16, 128, 255), (128, 9, 15, 256, 200)])
+def test_four_slices_of_few_chunks(K, B, H, V, T):
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert scan_plan(K, B * H, T, V).direct and not scan_plan(K, B * H, T + 256, V).direct
+    inp = random_inputs(B=B, T=T + 256, H=H, K=K, V=V, dtype=BF16, seed=140 + T)
+    first = {n: (x if n == "initial_state" else x[:, :T].contiguous()) for n, x in inp.items() if isinstance(x, torch.Tensor)}
+    o, _ = _check(first, "four slices, few chunks")
+    longer, _ = lm_engine_amd.chunk_gated_delta_rule(**_to_gpu(inp))
+    whole = T // 64 * 64
+    assert torch.equal(longer[:, :whole], o[:, :whole])
+    lengths = [T - 29 * b % T for b in range(B)]
+    cu = torch.tensor([0, *lengths]).cumsum(0).to(torch.int32).cuda()
+    gpu = _to_gpu(first)
+    padded, ht = lm_engine_amd.chunk_gated_delta_rule(**gpu, cu_seqlens=cu, output_final_state=True, left_padded=True)
+    for b in (0, 1, B - 1):
+        assert (padded[b, : T - lengths[b]] == 0).all(), f"row {b}: padding"
+        one = {n: (x[b : b + 1].cpu() if n == "initial_state" else x[b : b + 1, T - lengths[b] :].cpu()) for n, x in gpu.items()}
+        o_ref, h_ref = recurrent_gated_delta_rule_c(**one, output_final_state=True)
+        assert_parity(padded[b : b + 1, T - lengths[b] :].float(), o_ref, BF16, "o")
+        assert_parity(ht[b : b + 1], h_ref, BF16, "final_state")
 
 
 # K = 256 with up to 256 workgroups of 16 columns: the scan whose keys are split over two waves.  One to seven chunks (its loaders' ring

@@ -2,7 +2,7 @@
 
 import pytest
 
-from tests.dispatch import sweep_columns
+from tests.dispatch import scan_plan, sweep_columns
 
 
 @pytest.mark.parametrize(
@@ -29,3 +29,16 @@ from tests.dispatch import sweep_columns
 )
 def test_width_of_the_sweeps(N, H, V, longest, chunks, layout, columns):
     assert sweep_columns(N, H, V, longest, chunks, layout == "packed", layout == "padded") == columns
+
+
+@pytest.mark.parametrize(
+    "K, rows, H, T, V, packed, direct",
+    [
+        (128, 20, 16, 64, 128, False, False), (128, 20, 16, 65, 128, False, True), (128, 20, 16, 255, 128, False, True), (128, 20, 16, 256, 128, False, False),
+        (128, 12, 32, 200, 256, False, True), (128, 48, 16, 200, 128, False, True), (128, 49, 16, 200, 128, False, False), (128, 100, 16, 112, 128, False, True), (128, 100, 16, 113, 128, False, False),
+        (128, 100, 16, 128, 128, False, False), (64, 40, 16, 65, 128, False, True), (64, 40, 16, 128, 128, False, False), (128, 60, 16, 200, 128, True, False),
+        (128, 8, 16, 65, 128, False, False), (256, 40, 16, 65, 512, False, False),  # two slices, half slices
+    ],
+)  # fmt: skip
+def test_who_stores_the_output_of_four_slices(K, rows, H, T, V, packed, direct):
+    assert scan_plan(K, rows * H, T, V, packed).direct == direct
