@@ -1399,8 +1399,7 @@ __global__ __launch_bounds__(scan_waves(NW, HALF) * WAVE) void chunk_scan32_kern
 // ------------------------------------------------------------------------------------------
 int launch_chunk_fused(ChunkParams& p, int K, hipStream_t stream, int num_cus);        // gdn_chunk_fused.hip
 int launch_prepare32(const ChunkParams& p, int K, hipStream_t stream, int num_cus);  // gdn_chunk_prepare.hip
-template <int K>
-int launch_scan_keys(ChunkParams& p, hipStream_t stream);  // gdn_chunk_scan_keys.hip
+int launch_scan_keys(ChunkParams& p, hipStream_t stream);            // gdn_chunk_scan_keys.hip
 
 template <int K>
 int launch32(ChunkParams& p, hipStream_t stream, hipEvent_t* events, int num_cus) {
@@ -1427,7 +1426,7 @@ int launch32(ChunkParams& p, hipStream_t stream, hipEvent_t* events, int num_cus
     }
     if (events != nullptr) (void)hipEventRecord(events[2], stream);
     if constexpr (K == 256) {
-        if (plan.split_keys) return launch_scan_keys<K>(p, stream);
+        if (plan.split_keys) return launch_scan_keys(p, stream);
     }
     p.scan_groups = vtiles / nw;
     const dim3 grid((unsigned)(chains8 * p.scan_groups));

@@ -28,6 +28,7 @@ namespace gdn {
 
 namespace {
 
+constexpr int K = 256;
 constexpr int KEYS_WAVES = 8;  // 0 1 compute (a key half each) | 2 3 loaders | 4 output store | 5 exits at once | 6 7 loaders (as in the half-slice scan)
 constexpr int KEYS_LOADERS = 4;
 
@@ -36,7 +37,6 @@ constexpr int KEYS_LOADERS = 4;
 //     K S0 (4 token tiles x K/64 slabs) | S0^T q^T (as many; the other wave's two tiles first) | V~ = T' X (6) | S += k^T V~' (2 K/32) |
 //     O^T += V~^T P^T (this wave's two tiles x 2 slabs)
 // "Logical" output tiles: 0 and 1 are this wave's, 2 and 3 the other's.
-template <int K>
 struct KeysRules {
     static constexpr int KW = K / 2;  // keys of a wave
     static constexpr int KS = KW / 32, KT = KW / 16;
@@ -134,17 +134,14 @@ struct KeysRules {
     static_assert(OP_PUB_S < OP_GET_S && OP_GET_S < OP_PUB_Q && OP_PUB_Q < OP_GET_Q && OP_GET_Q + 2 < OP_P && OP_K < OP_BAR, "order of the hand-overs");
 };
 
-template <int K>
-struct KeysSchedule : KeysRules<K> {
-    static constexpr typename KeysRules<K>::Table TABLE = KeysRules<K>::make();
+struct KeysSchedule : KeysRules {
+    static constexpr KeysRules::Table TABLE = KeysRules::make();
     static_assert(TABLE.ok, "no placement of the side work satisfies the windows");
     static constexpr int op_of(int pc) { return TABLE.op[pc]; }
 };
 
-template <int K>
 __global__ __launch_bounds__(KEYS_WAVES* WAVE) void chunk_scan_keys_kernel(const ChunkParams p) {
-    typedef KeysSchedule<K> SCH;
-    static_assert(K == 256, "see above");
+    typedef KeysSchedule SCH;
     // the rows of q have a single buffer and the chunk a second workgroup barrier ("barrier Q", see the half-slice scan)
     constexpr int NL = KEYS_LOADERS;
     constexpr int KW = SCH::KW, KS = SCH::KS, KT = SCH::KT;
@@ -184,17 +181,16 @@ __global__ __launch_bounds__(KEYS_WAVES* WAVE) void chunk_scan_keys_kernel(const
     const int vgroup = rest % p.scan_groups;  // 16 columns
     const int per_xcd = (p.N * p.H + 7) / 8;
     int n, h;
-    const int32_t* const order = p.cu_seqlens != nullptr ? p.seq_order : p.row_order;  // (row_order: left-padded rows of given records)
     {
         const int i = rest / p.scan_groups;
-        if (order == nullptr) {
+        if (p.cu_seqlens == nullptr) {
             const int chain = xcd * per_xcd + i;
             if (i >= per_xcd || chain >= p.N * p.H) return;  // whole workgroup
             n = chain / p.H, h = chain % p.H;
         } else {
             const int rank = 8 * i + ((xcd - i) % 8 + 8) % 8;
             if (i >= per_xcd || rank >= p.N * p.H) return;  // whole workgroup
-            n = order[rank / p.H], h = rank % p.H;
+            n = p.seq_order[rank / p.H], h = rank % p.H;
         }
     }
     int slot_begin, nchunks;
@@ -209,8 +205,7 @@ __global__ __launch_bounds__(KEYS_WAVES* WAVE) void chunk_scan_keys_kernel(const
         packed_bounds(p.cu_seqlens, n, p.T, t0, len);
         b = 0, seq_t0 = t0, seq_len = min(len, nchunks * C);
     }
-    // (given records of a left-padded batch lie at the slots of the tokens they cover, the last ones of the row)
-    const uint8_t* const rec = p.rec + ((int64_t)h * p.TC + slot_begin + (p.records_given && p.pad_lens != nullptr ? p.NT - nchunks : 0)) * p.rec_bytes;
+    const uint8_t* const rec = p.rec + ((int64_t)h * p.TC + slot_begin) * p.rec_bytes;
 
     // Zeros at the padding rows of a left-padded batch, for a caller that asks for them, while the first chunk is on its way, by the two
     // waves that have nothing else to do: the workgroups of a chain together in whole rows, 16 bytes a lane (see the other scans).
@@ -612,13 +607,11 @@ __global__ __launch_bounds__(KEYS_WAVES* WAVE) void chunk_scan_keys_kernel(const
 
 }  // namespace
 
-template <int K>
 int launch_scan_keys(ChunkParams& p, hipStream_t stream) {
     p.scan_groups = p.V / 16;
     const unsigned chains8 = (unsigned)(((int64_t)p.N * p.H + 7) / 8 * 8);
-    hipLaunchKernelGGL(chunk_scan_keys_kernel<K>, dim3(chains8 * p.scan_groups), dim3(KEYS_WAVES * WAVE), 0, stream, p);
+    hipLaunchKernelGGL(chunk_scan_keys_kernel, dim3(chains8 * p.scan_groups), dim3(KEYS_WAVES * WAVE), 0, stream, p);
     return (int)hipGetLastError();
 }
-template int launch_scan_keys<256>(ChunkParams& p, hipStream_t stream);
 
 }  // namespace gdn
