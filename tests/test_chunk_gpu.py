@@ -398,6 +398,11 @@ def test_four_slices_of_few_chunks(K, B, H, V, T):
         assert_parity(ht[b : b + 1], h_ref, BF16, "final_state")
 
 
+@pytest.mark.parametrize("T", [113, 128])
+def test_four_slices_of_two_chunks_through_the_loaders(T):
+    _check(random_inputs(B=9, T=T, H=16, K=64, V=128, dtype=BF16, seed=160 + T), "four slices, two chunks")
+
+
 # K = 256 with up to 256 workgroups of 16 columns: the scan whose keys are split over two waves.  One to seven chunks (its loaders' ring
 # fills and drains differently up to five), first and last token of a chunk, one to many column groups, shared heads of q and k
 @pytest.mark.parametrize("T, V, HK, H", [(1, 32, 1, 1), (63, 64, 1, 2), (64, 512, 2, 2), (65, 512, 3, 3), (129, 96, 2, 4), (192, 512, 2, 2), (257, 64, 4, 4), (321, 512, 1, 2), (448, 512, 2, 2)])
@@ -417,6 +422,55 @@ def test_split_keys_at_the_edges_of_chunks(T, V, HK, H):
         first, state = lm_engine_amd.chunk_gated_delta_rule(**part(slice(0, 64)), output_final_state=True)
         second, end = lm_engine_amd.chunk_gated_delta_rule(**dict(part(slice(64, None)), initial_state=state), output_final_state=True)
         assert torch.equal(torch.cat([first, second], dim=1), o) and torch.equal(end, ht)
+
+
+def _half_slices(chains, T, V, packed=False):
+    """Past the line of the split keys: half slices, 32 columns to a workgroup."""
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        plan = scan_plan(256, chains, T, V, packed)
+        assert plan.half and not plan.split_keys
+
+
+# the same edges for launches with more workgroups, which keep the half-slice scan: its output, and shared heads of q and k
+@pytest.mark.parametrize("T, V, HK, H", [(1, 512, 2, 4), (63, 512, 4, 4), (64, 512, 2, 4), (65, 512, 1, 5), (129, 256, 3, 9), (192, 512, 2, 4), (257, 512, 4, 4), (321, 512, 2, 6), (448, 512, 4, 4)])
+def test_half_slices_of_256_keys_at_the_edges_of_chunks(T, V, HK, H):
+    _half_slices(4 * H, T, V)
+    inp = random_inputs(B=4, T=T, H=H, K=256, V=V, dtype=BF16, seed=170 + T)
+    q, k = (inp[n][:, :, :HK].contiguous() for n in ("q", "k"))
+    o_ref, h_ref = recurrent_gated_delta_rule_c(**dict(inp, q=q.repeat_interleave(H // HK, dim=2), k=k.repeat_interleave(H // HK, dim=2)), output_final_state=True)
+    print(f"case: half slices T={T} V={V} heads {HK} / {H}", flush=True)
+    o, ht = lm_engine_amd.chunk_gated_delta_rule(**_to_gpu(dict(inp, q=q, k=k)), output_final_state=True)
+    assert_parity(o.float(), o_ref, BF16, "o")
+    assert_parity(ht, h_ref, BF16, "final_state")
+
+
+@pytest.mark.parametrize("lengths", [[70, 0, 129, 0, 64, 65, 1, 200, 33, 128], [3] * 70])
+def test_half_slices_of_256_keys_on_packed_sequences(lengths):
+    V = 256
+    inp = random_inputs(B=1, T=sum(lengths), H=2, K=256, V=V, dtype=BF16, seed=180, N=len(lengths))
+    _half_slices(2 * len(lengths), sum(lengths), V, packed=True)
+    cu = torch.tensor([0] + lengths).cumsum(0).to(torch.int32)
+    _, ht = _check(dict(inp, cu_seqlens=cu), f"half slices, {len(lengths)} sequences")
+    empty = torch.tensor(lengths) == 0
+    assert torch.equal(ht[empty].cpu(), inp["initial_state"][empty])
+
+
+def test_half_slices_of_256_keys_on_left_padded_rows():
+    B, H, V = 8, 5, 128
+    _half_slices(B * H, 130, V)
+    test_padding_of_the_output_is_written_on_request_only(B, H, 256, V, 1)
+    lengths = [130, 0, 1, 129, 64, 66, 128, 65]
+    inp = random_inputs(B=B, T=130, H=H, K=256, V=V, dtype=BF16, seed=181)
+    gpu = _to_gpu(inp)
+    o, ht = lm_engine_amd.chunk_gated_delta_rule(**gpu, cu_seqlens=torch.tensor([0] + lengths).cumsum(0).to(torch.int32).cuda(), output_final_state=True, left_padded=True)
+    for b, n in enumerate(lengths):
+        if n == 0:
+            assert torch.equal(ht[b].cpu(), inp["initial_state"][b])
+            continue
+        row = {name: x[b : b + 1] if name == "initial_state" else x[b : b + 1, 130 - n :] for name, x in inp.items()}
+        o_ref, h_ref = recurrent_gated_delta_rule_c(**row, output_final_state=True)
+        assert_parity(o[b : b + 1, 130 - n :].float(), o_ref, BF16, f"o of row {b}")
+        assert_parity(ht[b : b + 1], h_ref, BF16, f"final state of row {b}")
 
 
 def test_shipped_head_shape_full_size():

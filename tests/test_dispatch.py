@@ -42,3 +42,37 @@ def test_width_of_the_sweeps(N, H, V, longest, chunks, layout, columns):
 )  # fmt: skip
 def test_who_stores_the_output_of_four_slices(K, rows, H, T, V, packed, direct):
     assert scan_plan(K, rows * H, T, V, packed).direct == direct
+
+
+def _cases_of(test):
+    return next(m for m in test.pytestmark if m.name == "parametrize").args[1]
+
+
+def test_the_cases_of_the_scans_take_the_scans_they_are_of():
+    """At 256 compute units: a rule that is moved moves no test to another kernel unnoticed."""
+    from tests import test_chunk_gpu as chunk
+
+    for T, V, _, H in _cases_of(chunk.test_split_keys_at_the_edges_of_chunks):
+        assert scan_plan(256, 2 * H, T, V).split_keys, (T, V, H)
+    for T, V, _, H in _cases_of(chunk.test_half_slices_of_256_keys_at_the_edges_of_chunks):
+        assert not scan_plan(256, 4 * H, T, V).split_keys, (T, V, H)
+    for T in _cases_of(chunk.test_four_slices_at_the_edges_of_chunks):
+        plan = scan_plan(64, 9 * 16, T, 128)
+        assert plan.nw == 4 and plan.direct == (T == 65), T
+    for T in _cases_of(chunk.test_four_slices_of_two_chunks_through_the_loaders):
+        plan = scan_plan(64, 9 * 16, T, 128)
+        assert plan.nw == 4 and not plan.direct, T
+
+
+def test_the_cases_of_the_sweeps_have_the_width_they_are_of():
+    from tests.test_sweeps_gpu import CASES
+
+    wide = 0
+    for layout, lens, K, V, _, H in CASES:
+        if K == 128:
+            rows, longest = len(lens), -(-max(lens) // 64)
+            chunks = sum(lens) // 64 if layout == "packed" else rows * longest
+            columns = sweep_columns(rows, H, V, longest, chunks, layout == "packed", layout == "padded")
+            assert columns == (64 if H >= 8 else 32), (layout, lens, H)
+            wide += columns == 64
+    assert wide == 10
