@@ -491,6 +491,8 @@ def cycle_budget(w):
         _lib.check_status(lib.gdn_cycle_budget_read(out, slots), "gdn_cycle_budget_read")
     rows = [[out[8 * i + j] for j in range(7)] for i in range(slots)]
     rows = [r for r in rows if r[6] > 0]
+    if not rows:
+        raise SystemExit(f"{w.name}: no half-slice scan in this launch")
     per_chunk = {n: round(sum(r[j] / r[6] for r in rows) / len(rows), 1) for j, n in enumerate(names)}
     scan_ms = sum(t["chunk_scan"] for t in times) / len(times)
     chunks = rows[0][6]

@@ -49,7 +49,7 @@ def _hipcc() -> str:
 
 
 CYCLE_BUDGET_LIBRARY_PATH = os.path.join(PACKAGE_DIR, "libgdn_hip_cycles.so")
-CYCLE_BUDGET_SOURCES = ("gdn_api.hip", "gdn_chunk.hip", "gdn_chunk_scan32_k64.hip", "gdn_chunk_scan32_k128.hip", "gdn_chunk_scan32_k256.hip", "gdn_chunk_scan_keys.hip", "gdn_chunk_bwd.hip")  # the sources that read GDN_CYCLE_BUDGET
+CYCLE_BUDGET_SOURCES = ("gdn_api.hip", "gdn_chunk.hip", "gdn_chunk_scan32_k64.hip", "gdn_chunk_scan32_k128.hip", "gdn_chunk_scan32_k256.hip", "gdn_chunk_bwd.hip")  # the sources that read GDN_CYCLE_BUDGET
 
 
 def build_host_module() -> str:

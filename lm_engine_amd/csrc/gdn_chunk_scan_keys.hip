@@ -446,17 +446,6 @@ __global__ __launch_bounds__(KEYS_WAVES* WAVE) void chunk_scan_keys_kernel(const
 #pragma unroll
     for (int s = 0; s < KS; s++) sb[s] = pack4x2(S[2 * s], S[2 * s + 1]);
 
-#ifdef GDN_CYCLE_BUDGET
-    // Measurement build: the shader clock between the groups of MFMAs, as in the half-slice scan
-    uint64_t cyc[6] = {0, 0, 0, 0, 0, 0};
-    uint64_t cyc_t0 = __builtin_readcyclecounter();
-    auto cyc_tick = [&](int group) {
-        const uint64_t t1 = __builtin_readcyclecounter();
-        cyc[group] += t1 - cyc_t0;
-        cyc_t0 = t1;
-        __builtin_amdgcn_sched_barrier(0);
-    };
-#endif
     for (int c = 0; c < nchunks; c++) {
         const uint8_t* const st = stage(c);
         const uint8_t* const stn = stage(c + 1);
@@ -507,13 +496,6 @@ __global__ __launch_bounds__(KEYS_WAVES* WAVE) void chunk_scan_keys_kernel(const
 
         static_for<0, NOPS>([&](auto opc) {
             constexpr int op = decltype(opc)::value;
-#ifdef GDN_CYCLE_BUDGET
-            if constexpr (op == 0) cyc_tick(5);
-            else if constexpr (op == OP_Q) cyc_tick(0);
-            else if constexpr (op == OP_T) cyc_tick(1);
-            else if constexpr (op == OP_K) cyc_tick(2);
-            else if constexpr (op == OP_P) cyc_tick(3);
-#endif
             if constexpr (op + LA < NOPS) fr[op + LA] = lds_frag(st, std::integral_constant<int, (op + LA < NOPS ? op + LA : 0)>{});
             if constexpr (op == OP_BAR) {
                 __syncthreads();  // this wave is done with chunk c's half; chunk c + 1 is in the other one
@@ -579,19 +561,7 @@ __global__ __launch_bounds__(KEYS_WAVES* WAVE) void chunk_scan_keys_kernel(const
             }
             __builtin_amdgcn_sched_barrier(0);
         });
-#ifdef GDN_CYCLE_BUDGET
-        cyc_tick(4);
-#endif
     }
-#ifdef GDN_CYCLE_BUDGET
-    // wave 0 of every 16th workgroup reports: [workgroup / 16][6 groups | chunks]
-    if (p.cycle_out != nullptr && wave == 0 && lane == 0 && blockIdx.x % 16 == 0 && blockIdx.x / 16 < GDN_CYCLE_BUDGET_SLOTS) {
-        uint64_t* out = p.cycle_out + (blockIdx.x / 16) * 8;
-#pragma unroll
-        for (int i = 0; i < 6; i++) out[i] = cyc[i];
-        out[6] = (uint64_t)nchunks;
-    }
-#endif
     if (nchunks > 0) {
 #pragma unroll
         for (int l = 0; l < 2; l++) out_tile(acco[l], (nchunks - 1) & 1, l);
