@@ -418,7 +418,7 @@ uint64_t gdn_chunk_bwd_sweeps_workspace_bytes(const gdn_args *args);
  * Measurement aid, no counterpart in the reference: runs exactly what gdn_chunk_fwd runs, with a
  * HIP event recorded on `stream` before and after every kernel, waits for the last one and
  * returns each kernel's duration in milliseconds in kernel_ms[GDN_CHUNK_KERNELS], in launch
- * order: [0] chunk offsets of 64 packed sequences and more (else about 0), [1] prepare, [2] scan.
+ * order: [0] chunk offsets of 64 packed sequences and more (else no kernel, the time between two events: some us), [1] prepare, [2] scan.
  * Unlike every other entry point it creates events and blocks the calling thread.
  */
 #define GDN_CHUNK_KERNELS 3

@@ -341,7 +341,7 @@ def _chunk_local_grads(qs, kn, vc, doc, Y, Vn, S0, dS1, gam, bc):
 
 def _backward_on_kernels(q, k, v, g, beta, do, dht, scale, initial_state, l2norm, cu_seqlens, left_padded, joined):
     """The whole backward on three kernel launches (bf16; K = 64, 128 or 256; V a multiple of 64): ``gdn_chunk_bwd_sweeps``
-    (per-chunk records and scalars, both sweeps; one more launch for the chunk offsets of packed sequences, and one more at K = 64
+    (per-chunk records and scalars, both sweeps; one more launch for the chunk offsets of 64 packed sequences or more, and one more at K = 64
     for rows that fill the GPU with either sweep) and ``gdn_chunk_bwd_local`` writing the gradients in the caller's layout (one more launch, ``gdn_fold_heads``, where
     value heads share those of q and k).  Chunk states, V~ and Y pass between
     them as bf16, what the chunk-local products round them to anyway.  Batches that are not whole rows of whole chunks are laid

@@ -31,15 +31,15 @@ ScanPlan plan_scan(int K, int64_t chains, int T, int V, bool packed, bool save, 
     // finishes a ragged batch sooner than four slices per workgroup storing from their compute waves (11 sequences of 202 .. 6350
     // tokens, H = 16, 2.75 workgroups per CU: 352 us against 575 us).
     if (save && packed && !records_given && K <= 128) nw = 1;
-    if (K > 128) nw = 1;  // K = 256 has the half-slice scan only, also as the saving variant and on given records
+    if (K > 128) nw = 1;  // K = 256 scans on half slices, also as the saving variant and on given records, or with the keys split (below)
     if (records_given == 2) nw = 1;  // records given in the half-slice scan's fragment order
     ScanPlan plan;
     plan.nw = nw;
     // a slice with a CU to itself is scanned by two waves of 16 columns each; the records are laid out for them
     plan.half = K > 128 || records_given == 2 || (nw == 1 && !records_given);
     // K = 256, and twice as many workgroups still have a CU each: 16 columns to a workgroup and the keys over two waves, whose chunk step is a
-    // fifth shorter (forward of 4 x 777 tokens, 2 heads, V = 512, 256 workgroups 37.6 | 36.2 us; 30000 tokens, 3 heads 856 | 726).  More
-    // workgroups would run in rounds.
+    // sixth shorter.  Forward, half slices | this, V = 512: 4 x 777 tokens, 2 heads, 256 workgroups 36.2 | 33.3 us, 4 x 64 14.5 | 14.5, 2000
+    // tokens 68.7 | 60.3.  More workgroups would run in rounds.
     plan.split_keys = plan.half && !save && K == 256 && (chains + 7) / 8 * 8 * (V / 16) <= (int64_t)num_cus;
     // Four slices to a workgroup, rows of two to four chunks: what goes through LDS is stored a chunk later, with nothing left to compute beside
     // it, and a short last chunk leaves the memory idle before.  Through LDS | from the compute waves, 16 heads, K = V = 128: 20 x 65 tokens 31.7 |

@@ -92,7 +92,7 @@ inline bool fused_launch_window(int64_t chains, int V, int num_cus) {
 struct ScanPlan {
     int nw;             // 32-column slices per workgroup
     bool half;          // a slice is scanned by two waves of 16 columns (records in the 16x16x32 fragment order)
-    bool split_keys;    // ... and by two more for the other half of the keys, 16 columns to a workgroup (gdn_chunk_scan_keys.hip)
+    bool split_keys;    // ... or: 16 columns to a workgroup, two waves with half of the keys each (gdn_chunk_scan_keys.hip)
     bool direct;        // four slices per workgroup: the compute waves store the output themselves
     bool staged_saves;  // a saving scan whose saves go through LDS and the store wave: only there bf16 saves exist
     bool no_output;     // the scan without output runs

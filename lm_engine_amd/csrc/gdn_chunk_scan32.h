@@ -1,6 +1,6 @@
 // Chunked forward of the gated delta rule (K = 64, 128, 256): the scan.  Whole-slice waves work on
 // v_mfma_f32_32x32x16_bf16 (K <= 128), half-slice waves on v_mfma_f32_16x16x32_bf16 (K <= 128 when a slice has a
-// CU to itself, and K = 256 always).
+// CU to itself, and K = 256 where the GPU is full; else gdn_chunk_scan_keys.hip).
 //
 // Two kernels (prepare: what does not depend on the state, written as MFMA operand fragments to a workspace
 // record per (head, chunk); scan: the serial pass over the chunks of a sequence with the state held in MFMA
@@ -87,7 +87,7 @@ constexpr int SCAN_LOADERS = 4;
 // So with fewer than four compute waves the waves that land on their SIMDs get the light jobs:
 //   NW = 1:  0 compute | 1 2 3 loaders | 4 output store | 5 loader
 //   NW = 2:  0 1 compute | 2 3 loaders | 4 output store | 5 exits at once | 6 7 loaders
-//   NW = 4:  0..3 compute | 4..7 loaders (each compute wave shares with one loader), which also write the output
+//   NW = 4:  0..3 compute | 4..7 loaders (each compute wave shares with one loader), which also write the output (or the compute waves, DIRECT)
 //   NW = 1, HALF:  0 1 compute (16 columns each) | the rest as for NW = 2
 __host__ __device__ constexpr int scan_waves(int nw, bool half = false) { return nw == 1 && !half ? 6 : 8; }
 

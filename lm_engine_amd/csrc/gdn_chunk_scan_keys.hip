@@ -10,8 +10,9 @@
 // 58 MFMAs a wave.  The waves hand over through an epoch word in LDS that the other polls (pair_publish, pair_wait): the products with q
 // stand between writing the halves of K S0 and needing the other's.
 //
-// Bound by the instruction stream of a compute wave, 1.4 us a chunk (1.75 in the half-slice scan).  Forward, half slices | this: 777
-// tokens, 2 heads, V = 512 37.5 | 36.0 us, 2000 tokens 69.5 | 61.5, 4 x 777 37.6 | 36.2, 30000 tokens, 3 heads 856 | 726.
+// Bound by the instruction stream of a compute wave: the kernel over 30000 tokens, 3 heads, V = 512 (469 chunks) 808 us in half slices, 680
+// here, 1.72 | 1.45 a chunk.  Forward, half slices | this: 64 tokens, 2 heads, V = 512 14.0 | 13.3 us, 777 tokens 36.1 | 33.1, 2000 68.7 |
+// 60.3, 4 x 777 36.2 | 33.3.
 // At K = 128, where 60 MFMAs become 34, what is duplicated and handed over eats what is saved: 4096 tokens, 16 heads, V = 128 87.0 | 88.8
 // us.  And with 32 columns, four compute waves beside four loaders, it is slower for every size (777 tokens 37.2 | 38.0; 65536 tokens, 32
 // heads, K = 128, V = 256 1572 | 1766).

@@ -13,7 +13,8 @@
 // The reverse sweep as a forward scan over a "mirror" problem (reversed rows, gdn_chunk_bwd_prepare) takes two chunk steps per chunk
 // and a kernel in front that forms P^T dO and its records; as one step it has 60 instead of 76 MFMAs per chunk (K = 128), none that
 // only pass through the pipeline, P^T dO is neither rounded nor stored, and the records come out of the forward's prepare step.
-// Kernel times, that kernel + forward sweep + reverse sweep against prepare + the two sweeps here: 4 x 4096 tokens, 16 heads,
+// Kernel times when the sweeps were launches of their own, 32 columns to a workgroup, that kernel + forward sweep + reverse sweep against
+// prepare + the two sweeps here: 4 x 4096 tokens, 16 heads,
 // K = V = 128: 148 + 106 + 160 | 53 + 95 + 122 us; 11 packed sequences of 32768 tokens together: 339 + 225 + 330 | 108 + 190 +
 // 243 us; 8 x 4096 tokens, 2 heads, K = 256, V = 512: 82 + 136 + 205 | 50 + 133 + 163 us.
 //
@@ -22,9 +23,9 @@
 // global -> registers -> LDS, a store wave that takes what is saved out of LDS.  What bounds it: the instruction stream of a
 // compute wave (K = 128: 38 and 60 MFMAs per chunk), two of the four SIMDs carry none, and every slice of a chain loads the chunk's
 // records and rows of q and k again.  At K = 128, where the chains fill the chip, a workgroup therefore owns 64 columns (NC = 4):
-// a compute wave on every SIMD, one loader beside each, and the loaders also take out what is saved.  A step is then longer (2.7 us
-// loaded | 1.9 of the reverse sweep), but both sweeps of 4 x 4096 tokens, 16 heads fit the chip side by side: 206 -> 173 us, 817 MB
-// at 4.7 TB/s where a plain copy reaches 5.2; 11 packed sequences, 32768 tokens 402 -> 351.  K = 256 at 64 columns does not fit the LDS.
+// a compute wave on every SIMD, one loader beside each, and the loaders also take out what is saved.  A step is then longer (one
+// sequence of 4000 tokens, 16 heads 1.9 us where 32 columns take 1.2), but both sweeps of 4 x 4096 tokens, 16 heads fit the chip side by
+// side: 205 -> 170 us, 817 MB at 4.8 TB/s where a plain copy reaches 5.2; 11 packed sequences, 32768 tokens 402 -> 348.  K = 256 at 64 columns does not fit the LDS.
 
 #include <type_traits>
 
